@@ -2,10 +2,10 @@
 
 The dense graph (Qwen3-0.6B and Qwen3-8B shapes) is driven through ModelRunner / BlockManager / Sequence (one model step and its sampled tokens) and
 through LLMEngine.generate (whole requests), a layer-list model through LLMEngine.generate.  Weights are synthetic: the framework's own seeded
-generator fills the matrices, and the norm gains are small, as a trained checkpoint's are not 1 either: the token's embedding then stands out of the
-residual stream and the greedy choice is as clear as a trained model's (with gains of 1 the two best of 150 thousand random logits lie closer
-together than 16-bit rounding in one row of a hundred).  float16 cases are the reference's graph (no head norms), bfloat16 ones the published
-checkpoints' (norms over the heads of q and k).
+generator fills the matrices, and the norm gains are chosen so that the token's embedding stands out of the residual stream behind the last layer: the
+greedy choice is then as clear as a trained model's usually is (with gains of 1 the two best of 150 thousand random logits lie closer together than
+16-bit rounding in some rows of a hundred, and an answer that takes the other one goes its own way from there on).  float16 cases are the reference's
+graph (no head norms), bfloat16 ones the published checkpoints' (norms over the heads of q and k).
 
 A case is a dict:
   path   "decode"   one step that extends `batch` sequences of `shortest` .. `longest` cached tokens (spread geometrically) by a token
@@ -22,8 +22,8 @@ import nvr_import
 
 BLOCK = 256
 MODELS = {  # the two shapes of nvr.ModelConfig's presets
-    "qwen3-0.6b": dict(V=151936, W=1024, F=3072, L=28, H=16, G=8, D=128, base=1e6, gain=0.10),
-    "qwen3-8b": dict(V=151936, W=4096, F=12288, L=36, H=32, G=8, D=128, base=1e6, gain=0.08),
+    "qwen3-0.6b": dict(V=151936, W=1024, F=3072, L=28, H=16, G=8, D=128, base=1e6, gains=(0.006, 0.06)),
+    "qwen3-8b": dict(V=151936, W=4096, F=12288, L=36, H=32, G=8, D=128, base=1e6, gains=(0.002, 0.024)),
 }
 LAYERS = dict(V=32768, W=1024, F=3072, L=4, H=16, G=8, D=128)  # the smallest size of the framework's own model comparison
 EPS, STD = 1e-6, 0.02
@@ -139,8 +139,8 @@ def _gains(case, seed):
     out = {"norm.weight": g(m["W"], 1.0)}
     for l in range(m["L"]):
         p = "layers.%d." % l
-        out[p + "input_layernorm.weight"] = g(m["W"], m["gain"])
-        out[p + "post_attention_layernorm.weight"] = g(m["W"], m["gain"])
+        out[p + "input_layernorm.weight"] = g(m["W"], m["gains"][0])
+        out[p + "post_attention_layernorm.weight"] = g(m["W"], m["gains"][1])
         if case["dtype"] == "bfloat16":
             out[p + "self_attn.q_norm.weight"] = g(m["D"], 1.0)
             out[p + "self_attn.k_norm.weight"] = g(m["D"], 1.0)
@@ -329,12 +329,12 @@ def work(case):
 
 
 def tolerance(case):
-    """About four times what the framework is off the values in 64 bits: 1.2e-3 in float16 and 1.0e-2 in bfloat16 after the 28 to 36 layers of a dense
+    """About four times what the framework is off the values in 64 bits (bfloat16: twice): 1.6e-3 in float16 and 1.3e-2 in bfloat16 after the 28 to 36 layers of a dense
     model (the last layer's keys and values included; two correct orders of the sums differ by about as much), 5e-3 after the 4 of the layer list, and 8e-7
     in float32 (1e-5: a sum over 3072 products may be taken in any order)."""
     if case["dtype"] == "float32":
         return {"rel": 1e-5, "max": 4e-4}
-    return {"rel": 5e-3, "max": 0.1} if case["dtype"] == "float16" else {"rel": 0.03, "max": 0.5}
+    return {"rel": 6e-3, "max": 0.1} if case["dtype"] == "float16" else {"rel": 0.03, "max": 0.5}
 
 
 # ---------------------------------------------------------------------------------------------------------------- the same in 64 bits
