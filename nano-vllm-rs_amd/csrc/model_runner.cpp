@@ -907,7 +907,7 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
 }
 
 // execute_model :105-128 with prepare_*_inputs :172-210 and create_*_context :222-300
-int nvr_model_runner::execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill) {
+int nvr_model_runner::execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill, bool logits_asked) {
     NVR_HIP_CHECK(hipSetDevice(device));
     if (layered) {                                                      // one step form for prompts, portions of prompts and decoded tokens
         facts_shown_valid = false; last_prefill = is_prefill; lm_parts = 0; logits_valid = true;
@@ -1104,9 +1104,10 @@ int nvr_model_runner::execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill
     // arg-max partials come with the logits when the whole batch goes through one lm_head launch (a pure function of
     // the shapes, so a replayed graph and this bookkeeping always agree)
     lm_parts = lm_fused ? KD(lm_head_parts((int64_t)nseq, Hd, Vl, Hd)) : 0;
-    // a batch that samples greedily everywhere takes its tokens from the arg-max partials: the f32 logits are then written
-    // only on demand (ensure_logits: execute_model callers that ask for them, copy_logits)
-    want_logits = !lazy_logits || lm_parts == 0;
+    // a batch that samples greedily everywhere takes its tokens from the arg-max partials: the f32 logits are then written only for a caller of
+    // execute_model that asks for them, by the step's own LM head (a second launch behind it streams the head's weights again: 63 us at 1 .. 32 rows
+    // of Qwen3-0.6B, 210 us of Qwen3-8B), or later on demand (ensure_logits: copy_logits behind an engine step)
+    want_logits = logits_asked || !lazy_logits || lm_parts == 0;
     for (size_t i = 0; i < nseq && !want_logits; ++i) want_logits = seqs[i]->sampling.temperature != 0.0f;
     logits_valid = want_logits;
     lm_input = is_prefill ? nlast : n;                                   // the rows the LM head reads this step (forward())

@@ -96,7 +96,7 @@ struct nvr_model_runner {
 
     ~nvr_model_runner();
     int init();
-    int execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill);
+    int execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill, bool logits_asked = false);   // logits_asked: the caller reads the f32 logits of every row
     // a full (un-sharded) checkpoint tensor by its HF / reference name -> this rank's slice of the packed
     // device weights (dtype 0 = f16, 1 = bf16, 2 = f32); copy_weight reads a local tensor back (tests)
     int load_tensor(const char *name, int dtype, const int64_t *shape, int ndim, const void *data);

@@ -209,7 +209,7 @@ int nvr_runner_execute_step(nvr_model_runner_t *r, nvr_seq_t *const *seqs, size_
 }
 int nvr_runner_execute_model(nvr_model_runner_t *r, nvr_seq_t *const *seqs, size_t n, int is_prefill, const float **logits_dev) {
     NVR_GUARD_BEGIN
-    int rc = r->execute(seqs, n, is_prefill != 0);
+    int rc = r->execute(seqs, n, is_prefill != 0, logits_dev != nullptr);
     if (rc == NVR_OK && logits_dev) { rc = r->ensure_logits(); *logits_dev = r->logits; }
     // a tensor-parallel step whose peer never arrived holds zeros in place of the peer's sums: never hand that out as a result
     if (rc == NVR_OK && logits_dev && r->tp > 1) rc = r->comm.p2p_check_error(r->stream);
