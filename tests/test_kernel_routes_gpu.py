@@ -58,3 +58,44 @@ def test_execute_model_stores_the_logits_with_the_step_as_on_demand(dtype, batch
         for s, t in zip(seqs, tokens):
             s.append_token(t)
             bm.may_append(s)
+
+
+@pytest.mark.parametrize("T,H,KVH,D,shift", [(1, 2, 2, 64, 0), (27, 16, 8, 128, 0), (65, 32, 8, 128, 0), (3, 3, 1, 256, 0), (5, 1, 1, 64, 0),    # the wide form: less than a round of lanes, several
+                                             (7, 4, 2, 96, 0), (7, 4, 2, 32, 0), (27, 16, 8, 128, 1)])                                         # the general form: other heads, unaligned weights
+def test_qk_norm_forms(T, H, KVH, D, shift):
+    """nvr_qk_norm_rope_store_kv on both of its kernels (16-byte pieces of a head by neighbouring lanes; a wave per head) against the oracle's ops with
+    their fp16 roundings: one rounding of each of n, the two products' difference and the store (3 ulps, as the operation's other test); slots, values."""
+    rng = np.random.default_rng(T + D)
+    N = (H + 2 * KVH) * D
+    xb = (rng.standard_normal((T, N)) * 1.5).astype(F16)
+    qw, kw = (1 + 0.3 * rng.standard_normal(D)).astype(F16), (1 + 0.3 * rng.standard_normal(D)).astype(F16)
+    pos = rng.integers(0, 400, T).astype(np.int64)
+    nslots = 2 * T + 4
+    slots = rng.permutation(nslots)[:T].astype(np.int32)
+    if T > 2:
+        slots[2] = -1
+    cos, sin = oracle.rope_table(D, 512, 1e6)
+    d_x, d_pos, d_slots, d_cos, d_sin = dev(xb), dev(pos), dev(slots), dev(cos), dev(sin)
+    d_qw, d_kw = dev(np.concatenate([np.zeros(shift, F16), qw])), dev(np.concatenate([np.zeros(shift, F16), kw]))
+    d_kc, d_vc = nvr.DeviceBuffer(nslots * KVH * D * 2), nvr.DeviceBuffer(nslots * KVH * D * 2)
+    d_kc.zero(); d_vc.zero()
+    nvr.check(nvr.lib().nvr_qk_norm_rope_store_kv(d_x.ptr, d_pos.ptr, d_slots.ptr, T, H, KVH, D, d_cos.ptr, d_sin.ptr, d_qw.ptr + 2 * shift, d_kw.ptr + 2 * shift, 1e-6,
+                                                  d_kc.ptr, d_vc.ptr, None))
+    nvr.check(nvr.lib().nvr_device_synchronize())
+    got = d_x.to_numpy((T, N), F16)
+    x = xb.astype(np.float32)
+    heads = []
+    for w, a, n in ((qw, 0, H), (kw, H, KVH)):
+        y = oracle.round_f16(oracle.rmsnorm(x[:, a * D:(a + n) * D].reshape(T * n, D), w.astype(np.float32), 1e-6)).reshape(T, n, D)
+        heads.append(oracle.round_f16(oracle.rope_apply(y, pos, cos, sin)).reshape(T, n * D))
+    ref = np.concatenate(heads + [x[:, (H + KVH) * D:]], 1)
+    assert np.all(np.abs(got.astype(np.float32) - ref) <= 2e-3 + 3 * 2.0 ** -10 * np.abs(ref))
+    kc, vc = d_kc.to_numpy((nslots, KVH * D), np.uint16), d_vc.to_numpy((nslots, KVH * D), np.uint16)
+    bits = got.view(np.uint16)
+    assert np.array_equal(bits[:, (H + KVH) * D:], xb.view(np.uint16)[:, (H + KVH) * D:])
+    seen = np.zeros(nslots, bool)
+    for t in range(T):
+        if slots[t] >= 0:
+            assert np.array_equal(kc[slots[t]], bits[t, H * D:(H + KVH) * D]) and np.array_equal(vc[slots[t]], bits[t, (H + KVH) * D:])
+            seen[slots[t]] = True
+    assert not kc[~seen].any() and not vc[~seen].any()
