@@ -114,6 +114,8 @@ int rmsnorm(const float *x, const float *w, float eps, int64_t T, int64_t Hd, fl
 }
 // tensor-parallel ranks: y = ((p_0 + p_1) + p_2) + ... over the ranks' partial sums parts[r * stride + ...] in rank order, then h <- h + y and
 // the norm, as rmsnorm_kernel<true>
+// NR > 0: that many parts, a column's all requested before the first add (NR = 0: nranks of them, one after the other)
+template <int NR>
 __global__ __launch_bounds__(256) void sum_ranks_rmsnorm_kernel(float *__restrict__ h, const float *__restrict__ parts, int nranks, int64_t stride,
                                                                 const float *__restrict__ w, float eps, int Hd, float *__restrict__ out) {
     __shared__ float sm[4];
@@ -122,7 +124,14 @@ __global__ __launch_bounds__(256) void sum_ranks_rmsnorm_kernel(float *__restric
     float ss = 0.f;
     for (int c = threadIdx.x; c < Hd; c += 256) {
         float y = pr[c];
-        for (int r = 1; r < nranks; ++r) y = y + pr[(int64_t)r * stride + c];
+        if (NR) {
+            float p[NR > 1 ? NR : 1];
+#pragma unroll
+            for (int r = 1; r < NR; ++r) p[r] = pr[r * stride + c];
+#pragma unroll
+            for (int r = 1; r < NR; ++r) y = y + p[r];
+        } else
+            for (int r = 1; r < nranks; ++r) y = y + pr[(int64_t)r * stride + c];
         const float v = hr[c] + y;
         hr[c] = v;
         ss = fmaf(v, v, ss);
@@ -133,7 +142,9 @@ __global__ __launch_bounds__(256) void sum_ranks_rmsnorm_kernel(float *__restric
 }
 int sum_ranks_add_rmsnorm(float *h, const float *parts, int nranks, int64_t stride, const float *w, float eps, int64_t T, int64_t Hd, float *out, hipStream_t s) {
     if (T == 0) return 0;
-    sum_ranks_rmsnorm_kernel<<<dim3((unsigned)T), dim3(256), 0, s>>>(h, parts, nranks, stride, w, eps, (int)Hd, out);
+#define NVR_SR(NR_) sum_ranks_rmsnorm_kernel<NR_><<<dim3((unsigned)T), dim3(256), 0, s>>>(h, parts, nranks, stride, w, eps, (int)Hd, out)
+    if (nranks == 2) NVR_SR(2); else if (nranks == 4) NVR_SR(4); else if (nranks == 8) NVR_SR(8); else NVR_SR(0);
+#undef NVR_SR
     F32_LAUNCH_CHECK("f32 sum_ranks_add_rmsnorm");
     return 0;
 }
@@ -193,8 +204,13 @@ __global__ __launch_bounds__(256) void linear_kernel(const float *__restrict__ x
 // tolerance, 2e-4, is for exactly that); bias as before.  C layout: lane (h, token t = lane % 32) holds features 8 b + 4 h + e (b = reg / 4, e = reg % 4).
 constexpr int MB = 64, MKT = 32, MLD = MKT + 4;
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-__global__ __launch_bounds__(256) void linear_mfma_kernel(const float *__restrict__ x, int64_t ldx, const float *__restrict__ W, int T, int K, int N,
-                                                          const float *__restrict__ bias, float *__restrict__ y) {
+// MPF K-tiles are requested ahead into registers (the weights of a short prompt come from HBM: with one tile ahead a K-step cost a round trip, 1.7 us).
+// Few output tiles (o / down projections of a short prompt: N = hidden) are split along k over blockIdx.z: part z writes the partial sums of its K-tiles to
+// y + z T N, and the launch that adds the residual and norms the row adds them up in order (sum_ranks_add_rmsnorm).  Qwen3-0.6B, 128 rows:
+// o / down 130 -> 10.4 us (8 parts), gate_up 55.7 -> 24.6, qkv 54.7 -> 23.5
+constexpr int MPF = 4;
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void linear_mfma_kernel(const float *__restrict__ x, int64_t ldx, const float *__restrict__ W, int T, int K, int N,
+                                                          const float *__restrict__ bias, float *__restrict__ y, int kslice) {
     __shared__ __attribute__((aligned(16))) float as[2][MB][MLD], bs[2][MB][MLD];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
     const int wn = wave >> 1, wm = wave & 1;                              // this wave: W rows n0 + 32 wn .., tokens t0 + 32 wm ..
@@ -204,36 +220,28 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(const float *__restric
     const float *wsrc[2], *xsrc[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        wsrc[i] = W + (int64_t)min(n0 + r + 32 * i, N - 1) * K + c * 4;
-        xsrc[i] = x + (int64_t)min(t0 + r + 32 * i, T - 1) * ldx + c * 4;
+        wsrc[i] = W + (int64_t)min(n0 + r + 32 * i, N - 1) * K + (int64_t)blockIdx.z * kslice + c * 4;
+        xsrc[i] = x + (int64_t)min(t0 + r + 32 * i, T - 1) * ldx + (int64_t)blockIdx.z * kslice + c * 4;
     }
-    float4 wv[2], xv[2];
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) { wv[i] = *reinterpret_cast<const float4 *>(wsrc[i] + k0); xv[i] = *reinterpret_cast<const float4 *>(xsrc[i] + k0); }
+    y += (int64_t)blockIdx.z * T * N;
+    struct Set { float4_t w0, w1, x0, x1; } s0, s1, s2, s3;               // (named sets of plain vectors: as arrays hipcc keeps them in LDS)
+    auto fetch = [&](Set &e, int k0) {
+        e.w0 = *reinterpret_cast<const float4_t *>(wsrc[0] + k0); e.x0 = *reinterpret_cast<const float4_t *>(xsrc[0] + k0);
+        e.w1 = *reinterpret_cast<const float4_t *>(wsrc[1] + k0); e.x1 = *reinterpret_cast<const float4_t *>(xsrc[1] + k0);
     };
-    auto stash = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            *reinterpret_cast<float4 *>(&as[buf][r + 32 * i][c * 4]) = wv[i];
-            *reinterpret_cast<float4 *>(&bs[buf][r + 32 * i][c * 4]) = xv[i];
-        }
+    auto stash = [&](int buf, const Set &e) {
+        *reinterpret_cast<float4_t *>(&as[buf][r][c * 4]) = e.w0; *reinterpret_cast<float4_t *>(&as[buf][r + 32][c * 4]) = e.w1;
+        *reinterpret_cast<float4_t *>(&bs[buf][r][c * 4]) = e.x0; *reinterpret_cast<float4_t *>(&bs[buf][r + 32][c * 4]) = e.x1;
     };
     f32x16 acc;
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-    const int KT = K / MKT;
-    fetch(0);
-    stash(0);
-    __syncthreads();
-    for (int kt = 0; kt < KT; ++kt) {
-        const int cur = kt & 1;
-        if (kt + 1 < KT) fetch((kt + 1) * MKT);
+    auto compute = [&](int buf) {
         float4 a4[4], b4[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            a4[j] = *reinterpret_cast<const float4 *>(&as[cur][wn * 32 + l32][h * 16 + j * 4]);
-            b4[j] = *reinterpret_cast<const float4 *>(&bs[cur][wm * 32 + l32][h * 16 + j * 4]);
+            a4[j] = *reinterpret_cast<const float4 *>(&as[buf][wn * 32 + l32][h * 16 + j * 4]);
+            b4[j] = *reinterpret_cast<const float4 *>(&bs[buf][wm * 32 + l32][h * 16 + j * 4]);
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -242,9 +250,24 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(const float *__restric
             acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4[j].z, b4[j].z, acc, 0, 0, 0);
             acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4[j].w, b4[j].w, acc, 0, 0, 0);
         }
-        if (kt + 1 < KT) stash(cur ^ 1);                                  // (the other buffer: last read in step kt - 1, before the barrier that ended it)
+    };
+    // (no condition around a request: behind the last K-tile the last one is read again and never used.  hipcc otherwise parks the requested registers in
+    //  accumulation registers at once, which waits for them)
+    const int KT = kslice / MKT, K4 = KT / MPF * MPF;
+    auto at = [&](int kt) { return min(kt, KT - 1) * MKT; };
+    fetch(s0, 0); fetch(s1, at(1)); fetch(s2, at(2)); fetch(s3, at(3));
+    stash(0, s0);
+    __syncthreads();
+    auto step = [&](int kt, int buf, Set &freed, const Set &next) {        // K-tile kt is in buffer buf; its set takes K-tile kt + MPF, the next one's is stashed
+        fetch(freed, at(kt + MPF));
+        compute(buf);
+        stash(buf ^ 1, next);                                             // (the other buffer: last read in the step before, in front of the barrier that ended it)
         __syncthreads();
-    }
+    };
+    for (int kt = 0; kt < K4; kt += MPF) { step(kt, 0, s0, s1); step(kt + 1, 1, s1, s2); step(kt + 2, 0, s2, s3); step(kt + 3, 1, s3, s0); }
+    if (K4 < KT) compute(0);                                              // the remainder: its K-tiles sit in buffer 0 and in sets 1, 2
+    if (K4 + 1 < KT) { __syncthreads(); stash(0, s1); __syncthreads(); compute(0); }
+    if (K4 + 2 < KT) { __syncthreads(); stash(0, s2); __syncthreads(); compute(0); }
     const int t = t0 + wm * 32 + l32;
     if (t < T) {
 #pragma unroll
@@ -427,12 +450,29 @@ int linear(const float *x, int64_t ldx, const float *W, int64_t T, int64_t K, in
         return 0;
     }
     if (K % MKT == 0 && ldx % 4 == 0 && N % 4 == 0 && ((uintptr_t)x | (uintptr_t)W | (uintptr_t)y) % 16 == 0) {     // matrix cores (r06)
-        linear_mfma_kernel<<<dim3((unsigned)((N + MB - 1) / MB), (unsigned)((T + MB - 1) / MB)), dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)N, bias, y);
+        linear_mfma_kernel<<<dim3((unsigned)((N + MB - 1) / MB), (unsigned)((T + MB - 1) / MB)), dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)N, bias, y, (int)K);
         F32_LAUNCH_CHECK("f32 linear (mfma)");
         return 0;
     }
     linear_kernel<<<dim3((unsigned)((N + LB - 1) / LB), (unsigned)((T + LB - 1) / LB)), dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)N, bias, y);
     F32_LAUNCH_CHECK("f32 linear");
+    return 0;
+}
+
+// parts of k for a product of few 64 x 64 tiles (1: none): doubled while the parts' workgroups still fit the 256 CUs once and a part keeps 8 K-tiles
+int linear_splitk_parts(int64_t T, int64_t K, int64_t N, int64_t ldx) {
+    if (T <= 8 || K % MKT || ldx % 4 || N % 4) return 1;
+    const int64_t tiles = ((N + MB - 1) / MB) * ((T + MB - 1) / MB);
+    int S = 1;
+    while (S < 8 && tiles * S * 2 <= 256 && K % (MKT * S * 2) == 0 && K / (S * 2) >= 8 * MKT) S *= 2;
+    return S;
+}
+int linear_splitk(const float *x, int64_t ldx, const float *W, int64_t T, int64_t K, int64_t N, int64_t S, float *parts, hipStream_t s) {
+    if (T < 1 || S < 1 || K % (MKT * S) || ldx % 4 || N % 4 || ((uintptr_t)x | (uintptr_t)W | (uintptr_t)parts) % 16)
+        return nvr::fail(NVR_ERR_UNSUPPORTED, "f32 linear_splitk: T=%ld K=%ld N=%ld in %ld parts", (long)T, (long)K, (long)N, (long)S);
+    linear_mfma_kernel<<<dim3((unsigned)((N + MB - 1) / MB), (unsigned)((T + MB - 1) / MB), (unsigned)S), dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)N, nullptr, parts,
+                                                                                                                       (int)(K / S));
+    F32_LAUNCH_CHECK("f32 linear_splitk (mfma)");
     return 0;
 }
 
@@ -746,6 +786,124 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnArgsF a, int paged) 
         a.out[((int64_t)t * a.H + hd) * D + d] = ctx > 0 ? o / sum : 0.f;
     }
 }
+// The same for head dims of 64, 128, 192 and 256 on 16-byte aligned rows: nothing but the last merge goes through LDS.  Sixteen lanes hold a key's row (and
+// the query's, and an output row): NF 16-byte pieces each, so a load of K or V touches whole lines, where a thread per key touched 64 lines per load and
+// paid for each; the score is summed over the sixteen lanes on DPP and every lane weighs its own piece of V with it.  A group of sixteen lanes walks keys
+// group, group + 4 NW, .. in batches of four with a running maximum of its own (K and V of the first batch are requested before anything is known but the
+// block table, those of the next batch before this one is used), the four groups of a wave meet in registers, the NW waves in LDS.  What bounds a decode
+// step's launch is that chain of round trips, not bytes: one sequence
+// of 128 .. 176 keys of Qwen3-0.6B 14.3 -> 8.0 us a launch, 128 prompt rows 38.6 -> 18.0
+template <int NF, int NW, bool PAGED>
+__global__ __launch_bounds__(64 * NW) void attention_rows_kernel(AttnArgsF a) {
+    constexpr int D = 64 * NF, KB = NF <= 2 ? 4 : 2;                     // keys a group requests at a time
+    constexpr int STEP = 4 * NW, ROUND = KB * STEP;                      // groups; keys of one round of all groups
+    __shared__ __attribute__((aligned(16))) float part[NW][D];
+    __shared__ float pm[NW], pl[NW];
+    const int t = blockIdx.x, hd = blockIdx.y, g = hd / (a.H / a.KVH);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, group = (int)threadIdx.x >> 4;
+    const int32_t *bt = PAGED ? a.block_tables + (int64_t)(a.seq_of_q ? a.seq_of_q[t] : t) * a.max_blocks : nullptr;
+    const int64_t base = PAGED ? 0 : (int64_t)a.kv_base[t];
+    // block of key j (any j >= 0: entries behind a sequence's blocks may be stale, and are never used: a key past the context reads key 0's row)
+    auto entry = [&](int j) -> int { return PAGED ? bt[min(j / a.block_size, a.max_blocks - 1)] : 0; };
+    auto row_of = [&](int e, int j) -> int64_t {                        // element offset of key j's row of this kv head
+        if (PAGED) return (((int64_t)max(e, 0) * a.block_size + j % a.block_size) * a.KVH + g) * D;
+        return (base + j) * a.ldkv + (int64_t)g * D;
+    };
+    int ea[KB], eb[KB];                                                  // the entries of two rounds: requested with the context length
+#pragma unroll
+    for (int u = 0; u < KB; ++u) { ea[u] = entry(group + u * STEP); eb[u] = entry(group + ROUND + u * STEP); }
+    const int64_t row0 = row_of(entry(0), 0);
+    float4_t q[NF];
+#pragma unroll
+    for (int i = 0; i < NF; ++i) q[i] = reinterpret_cast<const float4_t *>(a.q + (int64_t)t * a.ldq + (int64_t)hd * D)[l16 + 16 * i];
+    const int ctx = a.ctx_lens[t];
+    if (ctx <= 0) {                                                     // (uniform) no key: zeros
+        for (int d = threadIdx.x; d < D; d += 64 * NW) a.out[((int64_t)t * a.H + hd) * D + d] = 0.f;
+        return;
+    }
+    float4_t k[KB][NF], v[KB][NF], kn[KB][NF], vn[KB][NF];
+    auto request = [&](float4_t (&kk)[KB][NF], float4_t (&vv)[KB][NF], const int (&e)[KB], int j0) {
+#pragma unroll
+        for (int u = 0; u < KB; ++u) {
+            const int j = j0 + u * STEP;
+            const int64_t r = j < ctx ? row_of(e[u], j) : row0;
+            const float4_t *kr = reinterpret_cast<const float4_t *>(a.k + r), *vr = reinterpret_cast<const float4_t *>(a.v + r);
+#pragma unroll
+            for (int i = 0; i < NF; ++i) { kk[u][i] = kr[l16 + 16 * i]; vv[u][i] = vr[l16 + 16 * i]; }
+        }
+    };
+    float m = -INFINITY, l = 0.f;
+    float4_t o[NF];
+#pragma unroll
+    for (int i = 0; i < NF; ++i) o[i] = (float4_t){0.f, 0.f, 0.f, 0.f};
+    auto consume = [&](const float4_t (&kk)[KB][NF], const float4_t (&vv)[KB][NF], int j0) {
+        float s[KB], top = m;
+#pragma unroll
+        for (int u = 0; u < KB; ++u) {
+            float d = 0.f;
+#pragma unroll
+            for (int i = 0; i < NF; ++i)
+#pragma unroll
+                for (int c = 3; c >= 0; --c) d = fmaf(q[i][c], kk[u][i][c], d);
+            s[u] = j0 + u * STEP < ctx ? row_sum<16>(d) * a.scale : -INFINITY;
+            top = fmaxf(top, s[u]);
+        }
+        const float ref = top == -INFINITY ? 0.f : top;                  // (nothing seen yet, or scores of -inf alone: their weights are 0, not exp(-inf + inf))
+        const float keep = expf(m - ref);
+        m = top; l *= keep;
+#pragma unroll
+        for (int i = 0; i < NF; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) o[i][c] *= keep;
+#pragma unroll
+        for (int u = 0; u < KB; ++u) {
+            const bool live = j0 + u * STEP < ctx;
+            const float p = live ? expf(s[u] - ref) : 0.f;
+            l += p;
+#pragma unroll
+            for (int i = 0; i < NF; ++i)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) o[i][c] = fmaf(p, live ? vv[u][i][c] : 0.f, o[i][c]);
+        }
+    };
+    request(k, v, ea, group);
+    if (ROUND < ctx) request(kn, vn, eb, group + ROUND);                 // (uniform conditions from here on: the groups of a wave stay together)
+    for (int r0 = 0;; r0 += 2 * ROUND) {
+        const bool third = r0 + 2 * ROUND < ctx, fourth = r0 + 3 * ROUND < ctx;
+        if (third)
+#pragma unroll
+            for (int u = 0; u < KB; ++u) { ea[u] = entry(r0 + 2 * ROUND + group + u * STEP); eb[u] = entry(r0 + 3 * ROUND + group + u * STEP); }
+        consume(k, v, r0 + group);
+        if (third) request(k, v, ea, r0 + 2 * ROUND + group);
+        if (r0 + ROUND >= ctx) break;
+        consume(kn, vn, r0 + ROUND + group);
+        if (!third) break;
+        if (fourth) request(kn, vn, eb, r0 + 3 * ROUND + group);
+    }
+    // the four groups of the wave, then the waves
+    float top = fmaxf(m, __shfl_xor(m, 16, 64));
+    top = fmaxf(top, __shfl_xor(top, 32, 64));
+    const float w = expf(m - (top == -INFINITY ? 0.f : top));
+    l = xor16_partner_sum(xor32_partner_sum(l * w));
+#pragma unroll
+    for (int i = 0; i < NF; ++i) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) o[i][c] = xor16_partner_sum(xor32_partner_sum(o[i][c] * w));
+        if (lane < 16) reinterpret_cast<float4_t *>(part[wave])[l16 + 16 * i] = o[i];
+    }
+    if (lane == 0) { pm[wave] = top; pl[wave] = l; }
+    __syncthreads();
+    float mx = pm[0];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) mx = fmaxf(mx, pm[i]);
+    const float ref = mx == -INFINITY ? 0.f : mx;
+    for (int d = threadIdx.x; d < D; d += 64 * NW) {
+        float sum = 0.f, acc = 0.f;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) { const float e = expf(pm[i] - ref); sum = fmaf(e, pl[i], sum); acc = fmaf(e, part[i][d], acc); }
+        a.out[((int64_t)t * a.H + hd) * D + d] = acc / sum;
+    }
+}
 // opt the attention kernel in to > 64 KiB of dynamic LDS (runner init: never inside a stream capture)
 int prepare() {
     const void *fns[] = {reinterpret_cast<const void *>(&attention_kernel<1>), reinterpret_cast<const void *>(&attention_kernel<2>),
@@ -761,6 +919,20 @@ int attention(const AttnArgsF &a, bool paged, hipStream_t s) {
     const size_t lds = ((size_t)a.max_ctx + 5 * (size_t)a.D + 8) * 4;
     if (lds > 160 * 1024) return nvr::fail(NVR_ERR_UNSUPPORTED, "f32 attention: context %d does not fit the score buffer (%zu bytes of LDS)", a.max_ctx, lds);
     const dim3 grid((unsigned)a.nq, (unsigned)a.H);
+    // rows in 16-byte pieces: a multiple of 64 of them per head, everything aligned to them; eight waves share a query row's keys while the rows are few
+    // (a decode step), four from a CU's worth of rows on (a prompt: the rows themselves fill the chip)
+    const bool pieces = a.D % 64 == 0 && a.ldq % 4 == 0 && (paged || a.ldkv % 4 == 0) && (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) & 15) == 0;
+    if (pieces) {
+        const bool few = (int64_t)a.nq * a.H < 512;
+#define NVR_ARW(NF_, NW_) do { if (paged) attention_rows_kernel<NF_, NW_, true><<<grid, dim3(64 * NW_), 0, s>>>(a); \
+                               else attention_rows_kernel<NF_, NW_, false><<<grid, dim3(64 * NW_), 0, s>>>(a); } while (0)
+#define NVR_AR(NF_) do { if (few) NVR_ARW(NF_, 8); else NVR_ARW(NF_, 4); } while (0)
+        if (a.D == 64) NVR_AR(1); else if (a.D == 128) NVR_AR(2); else if (a.D == 192) NVR_AR(3); else NVR_AR(4);
+#undef NVR_AR
+#undef NVR_ARW
+        F32_LAUNCH_CHECK("f32 attention");
+        return 0;
+    }
     if (a.D <= 64) attention_kernel<1><<<grid, dim3(256), lds, s>>>(a, paged ? 1 : 0);
     else if (a.D <= 128) attention_kernel<2><<<grid, dim3(256), lds, s>>>(a, paged ? 1 : 0);
     else attention_kernel<4><<<grid, dim3(256), lds, s>>>(a, paged ? 1 : 0);

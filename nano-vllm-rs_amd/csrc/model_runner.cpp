@@ -288,9 +288,17 @@ int nvr_model_runner::gen_weights_f32() {
 // gathered (the communicator's all-gather: the one-shot arenas for decode-sized rows — bytes are moved, never summed there —, RCCL or the
 // in-process rendezvous otherwise), then summed in RANK ORDER in f32, added to the residual stream and normalised by one kernel: every rank holds
 // the same bits, equal to the f32 oracle's tensor-parallel sum.  One rank: the plain add + RMSNorm.
-int nvr_model_runner::row_parallel_norm_f32(int64_t T, const float *wn) {
+// parts of k of a row-parallel product of this step: what the kernel finds worth taking, as far as the slab buffer holds them
+int64_t nvr_model_runner::splitk_parts_f32(int64_t T, int64_t K) const {
+    int64_t S = nvr::kf::linear_splitk_parts(T, K, Hd, K);
+    while (S > 1 && S * T > 4 * slab_rows) S /= 2;
+    return S;
+}
+// parts > 1: the product left its partial sums in `slabs` (one rank): added up in their order like ranks' sums are
+int nvr_model_runner::row_parallel_norm_f32(int64_t T, const float *wn, int64_t parts) {
     namespace kf = nvr::kf;
     float *fh = reinterpret_cast<float *>(h), *fn = reinterpret_cast<float *>(n), *fp = reinterpret_cast<float *>(proj);
+    if (parts > 1) return kf::sum_ranks_add_rmsnorm(fh, slabs, (int)parts, T * Hd, wn, mc.rms_norm_eps, T, Hd, fn, stream);
     if (!comm.active()) return kf::add_rmsnorm(fh, fp, wn, mc.rms_norm_eps, T, Hd, fn, stream);
     if (!f32_gather) return nvr::fail(NVR_ERR_INVARIANT, "float32 tensor-parallel rank without its gather buffer");
     // in pieces of at most f32_gather_rows rows (the buffer holds tp x that many rows: sized for a decode batch and a few thousand prefill rows, not for
@@ -343,12 +351,16 @@ int nvr_model_runner::forward_f32(int64_t T, int64_t B, bool is_prefill, int64_t
             if (is_prefill) a.seq_of_q = d_kvbase;
         }
         RC(kf::attention(a, paged, st));
-        RC(kf::linear(fa, H * D, F(w.o), T, H * D, Hd, w.o_b ? F(w.o_b) : nullptr, fp, st));
+        // (a prompt on one rank, plain projections: few output tiles are split along k, and the add + norm behind them sums the parts: row_parallel_norm_f32)
+        const bool cut = !ride && !comm.active() && tp == 1 && !mc.use_bias;
+        int64_t S = cut ? splitk_parts_f32(T, H * D) : 1;
+        if (S > 1) RC(kf::linear_splitk(fa, H * D, F(w.o), T, H * D, Hd, S, slabs, st));
+        else RC(kf::linear(fa, H * D, F(w.o), T, H * D, Hd, w.o_b ? F(w.o_b) : nullptr, fp, st));
         if (ride) {                                                                                  // residual :382, norm :385, K12 + K13: one launch
             RC(kf::add_norm_linear_silu_mul(hc, fp, F(w.ln2), mc.rms_norm_eps, hn, F(w.gate_up), T, Hd, I, w.gate_up_b ? F(w.gate_up_b) : nullptr, fact, st));
             std::swap(hc, hn);
         } else {
-        RC(row_parallel_norm_f32(T, F(w.ln2)));                                                      // (exchange,) residual :382, norm :385
+        RC(row_parallel_norm_f32(T, F(w.ln2), S));                                                      // (exchange,) residual :382, norm :385
         if (kf::linear_silu_ok(T, Hd, Hd)) {                                                         // decode-sized: K12 + K13 in one launch
             RC(kf::linear_silu_mul(fn, Hd, F(w.gate_up), T, Hd, I, w.gate_up_b ? F(w.gate_up_b) : nullptr, fact, st));
         } else {
@@ -356,10 +368,12 @@ int nvr_model_runner::forward_f32(int64_t T, int64_t B, bool is_prefill, int64_t
             RC(kf::silu_and_mul(fg, T, I, fact, st));
         }
         }
-        RC(kf::linear(fact, I, F(w.down), T, I, Hd, w.down_b ? F(w.down_b) : nullptr, fp, st));
+        S = cut ? splitk_parts_f32(T, I) : 1;
+        if (S > 1) RC(kf::linear_splitk(fact, I, F(w.down), T, I, Hd, S, slabs, st));
+        else RC(kf::linear(fact, I, F(w.down), T, I, Hd, w.down_b ? F(w.down_b) : nullptr, fp, st));
         if (ride && l + 1 < L && !layers[l + 1].q_norm && !layers[l + 1].k_norm) owed = true;        // residual :389 + next norm :378: on the next layer's qkv launch
         else if (ride) RC(kf::add_rmsnorm(hc, fp, F(l + 1 < L ? layers[l + 1].ln1 : norm), mc.rms_norm_eps, T, Hd, fn, st));
-        else RC(row_parallel_norm_f32(T, F(l + 1 < L ? layers[l + 1].ln1 : norm)));                   // (exchange,) residual :389, next norm :378 / :501
+        else RC(row_parallel_norm_f32(T, F(l + 1 < L ? layers[l + 1].ln1 : norm), S));                   // (exchange,) residual :389, next norm :378 / :501
     }
     const float *hl = fn;
     if (is_prefill) { RC(kf::select_last_tokens(fn, d_cu, B, Hd, fnl, st)); hl = fnl; }

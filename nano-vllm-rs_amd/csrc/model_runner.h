@@ -142,7 +142,8 @@ private:
     int gen_weights();
     int gen_weights_f32();
     int forward_f32(int64_t T, int64_t B, bool is_prefill, int64_t max_ctx);
-    int row_parallel_norm_f32(int64_t T, const float *wn);
+    int row_parallel_norm_f32(int64_t T, const float *wn, int64_t parts = 1);
+    int64_t splitk_parts_f32(int64_t T, int64_t K) const;
     float *f32_h2 = nullptr;                             // float32, one rank: second residual-stream buffer [8][hidden] of the decode-sized steps whose add + norm
                                                          // rides on the consumer GEMV (the workgroups of that launch still read the first while one of them writes)
     float *f32_gather = nullptr; int64_t f32_gather_rows = 0;   // float32 tensor-parallel ranks: every rank's partial sums [tp][f32_gather_rows][hidden], a piece of the step's rows at a time

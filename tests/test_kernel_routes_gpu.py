@@ -99,3 +99,74 @@ def test_qk_norm_forms(T, H, KVH, D, shift):
             assert np.array_equal(kc[slots[t]], bits[t, H * D:(H + KVH) * D]) and np.array_equal(vc[slots[t]], bits[t, (H + KVH) * D:])
             seen[slots[t]] = True
     assert not kc[~seen].any() and not vc[~seen].any()
+
+
+def _attn_meta(ctx, tables=None, max_blocks=0):
+    m = nvr.AttnMetaC()
+    d_ctx = dev(np.asarray(ctx, np.int32))
+    m.context_lens, m.batch, m.max_context_len, m.max_blocks = d_ctx.ptr, len(ctx), max(ctx), max_blocks
+    d_bt = None
+    if tables is not None:
+        d_bt = dev(np.asarray(tables, np.int32))
+        m.block_tables = d_bt.ptr
+    return m, (d_ctx, d_bt)
+
+
+@pytest.mark.parametrize("H,KVH,D,ctx", [(2, 1, 64, [1, 127, 128, 129, 513]), (4, 4, 128, [1, 2, 128, 129, 256, 257, 700]), (2, 2, 192, [65, 64, 1]), (2, 1, 256, [63, 129, 300]),
+                                         (4, 2, 128, [5, 300] * 70),                                    # four waves per row: the rows fill the chip
+                                         (2, 1, 96, [1, 130])])                                         # the general form
+def test_float32_decode_attention_forms(H, KVH, D, ctx):
+    """The float32 paged decode attention at the edges of its rounds (4 keys x 32 or 16 groups, two rounds in flight) and in its general form, against the
+    oracle's softmax in float64; shuffled blocks, stale table entries behind a context."""
+    bs, B = 16, len(ctx)
+    rng = np.random.default_rng(D + B)
+    mb = max(-(-c // bs) for c in ctx) + 2
+    nb = B * mb
+    perm = rng.permutation(nb)
+    tables = perm.reshape(B, mb).astype(np.int32)
+    q = rng.standard_normal((B, H * D)).astype(np.float32)
+    k, v = rng.standard_normal((nb, bs, KVH, D)).astype(np.float32), rng.standard_normal((nb, bs, KVH, D)).astype(np.float32)
+    nvr.check(nvr.lib().nvr_ops_set_dtype(b"float32"))
+    try:
+        meta, keep = _attn_meta(ctx, tables, mb)
+        d_q, d_k, d_v, out = dev(q), dev(k), dev(v), nvr.DeviceBuffer(B * H * D * 4)
+        ws = nvr.DeviceBuffer(max(16, nvr.lib().nvr_paged_attn_workspace_bytes(B, H, D, max(ctx))))
+        scale = float(D ** -0.5)
+        nvr.check(nvr.lib().nvr_paged_attn_decode(d_q.ptr, H * D, d_k.ptr, d_v.ptr, C.byref(meta), H, KVH, D, bs, scale, out.ptr, ws.ptr, None))
+        nvr.check(nvr.lib().nvr_device_synchronize())
+        got = out.to_numpy((B, H, D), np.float32)
+    finally:
+        nvr.check(nvr.lib().nvr_ops_set_dtype(b"float16"))
+    for b in range(B):
+        kk = k[tables[b]].reshape(-1, KVH, D)[:ctx[b]].astype(np.float64)
+        vv = v[tables[b]].reshape(-1, KVH, D)[:ctx[b]].astype(np.float64)
+        for h in range(H):
+            g = h // (H // KVH)
+            s = kk[:, g] @ q[b, h * D:(h + 1) * D].astype(np.float64) * scale
+            p = np.exp(s - s.max())
+            ref = p @ vv[:, g] / p.sum()
+            # a score is a sum of D products (error about sqrt(D) eps |q||k| scale), a weight moves by that much of itself, and the output by the weights' shares of |v|
+            assert np.abs(got[b, h] - ref).max() <= 2e-5, (b, h)
+
+
+@pytest.mark.parametrize("T", [9, 64, 65, 128, 200])
+@pytest.mark.parametrize("hidden,inter", [(256, 512), (1024, 3072), (96, 160)])
+def test_float32_prompt_products_cut_along_k(T, hidden, inter):
+    """Prompts of the float32 path, whose o / down products are cut along k when their output tiles are few, against the oracle (f32): remainders of the
+    K-tiles a step requests ahead (160 = 5 of 32), tiles of one and more rows, one layer."""
+    heads = 1 if hidden == 96 else 2
+    m = mo.ModelConfig(vocab_size=256, hidden_size=hidden, intermediate_size=inter, num_hidden_layers=1, num_attention_heads=heads, num_key_value_heads=heads,
+                       head_dim=hidden // heads if hidden == 96 else 64, max_position_embeddings=256, rms_norm_eps=1e-6, rope_theta=1e4, tie_word_embeddings=True, init_std=0.05, seed=9)
+    from oracle import engine_oracle as eo
+    eo.reset_sequence_counter(); nvr.lib().nvr_seq_reset_id_counter()
+    ecfg = dict(max_num_seqs=1, max_num_batched_tokens=256, max_model_len=256, kvcache_block_size=16, num_kvcache_blocks=16)
+    model = nvr.ModelConfig(vocab_size=256, hidden_size=hidden, intermediate_size=inter, num_hidden_layers=1, num_attention_heads=heads, num_key_value_heads=heads,
+                            head_dim=m.head_dim, max_position_embeddings=256, rms_norm_eps=1e-6, rope_theta=1e4, tie_word_embeddings=1, init_std=0.05, seed=9)
+    o = mo.OracleEngine(m, eo.Config(**ecfg), fp16=False, bf16=False, max_pos=256)
+    p = nvr.LLMEngine(nvr.Config(skip_block_size_check=1, dtype="float32", **ecfg), model)
+    prompt = nvr.synthetic_tokens(T, 3, 1, 256).tolist()
+    o.add_request(prompt, eo.SamplingParams(temperature=0.0, max_tokens=1, ignore_eos=True))
+    p.add_request(prompt, nvr.SamplingParams(temperature=0.0, max_tokens=1, ignore_eos=True))
+    rec = p.step()
+    orec = o.step(forced_tokens=rec["tokens"])
+    assert np.abs(p.model_runner.logits(1) - orec["logits"]).max() < 2e-4
