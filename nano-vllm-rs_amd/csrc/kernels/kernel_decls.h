@@ -22,6 +22,9 @@ int rope_store_kv(half_bits *qkv, const int64_t *positions, const int32_t *slots
 // argmax over f32 rows; out_val (nullable) receives the row maxima, idx_offset is added to indices
 int argmax(const float *logits, int64_t B, int64_t V, int64_t *out_idx, float *out_val, int64_t idx_offset,
            hipStream_t s);
+// the same, few long rows cut into parts over the grid (ws: argmax_workspace_bytes(); null: argmax)
+size_t argmax_workspace_bytes();
+int argmax_parts(const float *logits, int64_t B, int64_t V, int64_t *out_idx, float *out_val, int64_t idx_offset, void *ws, hipStream_t s);
 int fill_weight(half_bits *dst, int64_t rows, int64_t cols, int64_t ld, int64_t global_cols, int64_t row0,
                 int64_t col0, uint64_t key, float scale, hipStream_t s);
 int fill_const(half_bits *dst, int64_t n, float v, hipStream_t s);

@@ -558,7 +558,10 @@ __global__ __launch_bounds__(kThreads) void sample_rows_kernel(const float *__re
 static size_t sample_header_bytes(int64_t B) { return (size_t)B * sizeof(RowHdr); }
 static size_t sample_header_offset(int64_t B, int64_t V) { return ((size_t)(B * V) * sizeof(float) + 255) / 256 * 256; }
 
-size_t sample_workspace_bytes(int64_t B, int64_t V) { return sample_header_offset(B, V) + 256 + sample_header_bytes(B); }
+size_t sample_workspace_bytes(int64_t B, int64_t V) {                   // (a runner's greedy batches use it too: argmax_parts)
+    const size_t n = sample_header_offset(B, V) + 256 + sample_header_bytes(B);
+    return n > argmax_workspace_bytes() ? n : argmax_workspace_bytes();
+}
 
 int sample(const float *logits, int64_t B, int64_t V, const float *temperature, const int64_t *top_k,
            const float *top_p, const uint64_t *keys, int64_t *out_ids, void *workspace, hipStream_t s, bool store_filtered) {

@@ -1443,11 +1443,11 @@ int nvr_model_runner::sample(nvr_seq *const *seqs, size_t nseq, int64_t *out) {
                 return NVR_OK;
             }
             if (lm_parts > 0) RC(KD(argmax_partials(d_lm_pval, d_lm_pidx, lm_parts, B, d_tok, nullptr, 0, stream)));
-            else RC(KD(argmax(logits, B, Vl, d_tok, nullptr, 0, stream)));
+            else RC(KD(argmax_parts(logits, B, Vl, d_tok, nullptr, 0, sample_ws, stream)));   // (sample_ws: nothing of a greedy batch is in it)
         } else {
             // vocab-sharded greedy (embed_head.rs:321-336): all-gather (max, argmax) pairs, then lowest index wins
             if (lm_parts > 0) RC(KD(argmax_partials(d_lm_pval, d_lm_pidx, lm_parts, B, d_tok, d_maxval, vocab_start, stream)));
-            else RC(KD(argmax(logits, B, Vl, d_tok, d_maxval, vocab_start, stream)));
+            else RC(KD(argmax_parts(logits, B, Vl, d_tok, d_maxval, vocab_start, sample_ws, stream)));
             RC(comm.all_gather_bytes(d_maxval, d_gather_val, (size_t)B * 4, stream));
             RC(comm.all_gather_bytes(d_tok, d_gather_idx, (size_t)B * 8, stream));
             std::vector<float> gv(tp * B); std::vector<int64_t> gi(tp * B);

@@ -101,6 +101,24 @@ def test_qk_norm_forms(T, H, KVH, D, shift):
     assert not kc[~seen].any() and not vc[~seen].any()
 
 
+@pytest.mark.parametrize("B,V", [(1, 65536), (1, 65535), (3, 151936), (1, 65539), (128, 65540), (129, 65540), (300, 64)])
+def test_greedy_rows_cut_into_parts(B, V):
+    """The greedy choice of f32 logits rows: cut into parts over the grid (few long rows) or one workgroup per row (short rows, or many of them), through a
+    float32 runner whose LM head leaves no arg-max partials — compared with the first maximum of the logits it returns, with ties planted by a zero head."""
+    for std in (0.02, 0.0):                                                # (0: every logit of a row is equal, the lowest index wins)
+        model = nvr.ModelConfig(vocab_size=V, hidden_size=64, intermediate_size=64, num_hidden_layers=1, num_attention_heads=1, num_key_value_heads=1, head_dim=64,
+                                max_position_embeddings=64, tie_word_embeddings=0, init_std=std, seed=3)
+        runner = nvr.ModelRunner(nvr.Config(skip_block_size_check=1, max_num_seqs=B, max_num_batched_tokens=4 * B, max_model_len=16, kvcache_block_size=16,
+                                            num_kvcache_blocks=B, dtype="float32"), model)
+        bm = nvr.BlockManager(B, 16)
+        seqs = [nvr.Sequence([(7 * i) % 64, i % 61], nvr.SamplingParams(temperature=0.0, ignore_eos=True), 16) for i in range(B)]
+        for s in seqs:
+            bm.allocate(s)
+        runner.execute_model(seqs, True)
+        tokens = runner.sample_tokens(seqs)
+        assert tokens == runner.logits(B).argmax(1).tolist()
+
+
 def _attn_meta(ctx, tables=None, max_blocks=0):
     m = nvr.AttnMetaC()
     d_ctx = dev(np.asarray(ctx, np.int32))
