@@ -117,6 +117,12 @@ int clamped_glu(const void *gu, int64_t T, int64_t F, float limit, float alpha, 
 
 // x += mult * y (x f32, y of the operand type, [n])
 int axpy(float *x, const void *y, bool bf16, float mult, int64_t n, hipStream_t s);
+// A join whose product comes as `parts` partial sums [parts][T][W] (added in their order, rounded to the operand type): alone, and in one launch with the norm_canon of the next
+// layer for steps of one row per sequence
+int axpy_parts(float *x, const float *parts, int nparts, bool bf16, float mult, int64_t n, hipStream_t s);
+bool join_norm_canon_ok(const Batch &b, int64_t W, int taps, const float *x, const float *parts, const float *hist);
+int join_norm_canon(float *x, const float *parts, int nparts, float mult, const Batch &b, int64_t W, float eps, int taps, float g1, const float *w1, void *out1, float g2, const float *w2,
+                    void *out2, bool bf16, float *hist, int64_t slots, hipStream_t s);
 
 // out[r] = x[rows[r]] / sqrt(mean^2 + eps) * g, in the operand type
 int norm_rows(const float *x, const int32_t *rows, int64_t R, int64_t W, float eps, float g, void *out, bool bf16, hipStream_t s);

@@ -192,6 +192,84 @@ __global__ __launch_bounds__(256) void norm_canon_rows_kernel(const float *__res
     }
 }
 
+// The join behind the last sublayer and norm_canon of one-row chunks (decode steps) in one launch: x <- x + mult * y where y is the operand type's rounding of the sum of
+// `parts` partial products [parts][T][W] (linear_splitk: added in their order), then the norm, the convolution over the slot's history and the history of the next step.  One
+// row per workgroup, NI 4-column pieces per thread, everything requested before the first sum: the launch is one trip to memory, as each of the two was (16 rows of 1024: 4.6 + 10.6 -> 8.0 us).
+template <class OT, int NI>
+__global__ __launch_bounds__(256) void join_norm_canon_kernel(float *__restrict__ x, const float *__restrict__ parts, int nparts, float mult, Batch b, int W, float eps, int taps, float g1,
+                                                              const float *__restrict__ w1, OT *__restrict__ out1, float g2, const float *__restrict__ w2, OT *__restrict__ out2,
+                                                              float *__restrict__ hist, int64_t slots) {
+    __shared__ float red[4];
+    const int t = blockIdx.x, st = b.start[t], hrows = taps - 1;               // (one row per sequence: row t is sequence t)
+    const int64_t slot = b.slot[t], stride = (int64_t)b.T * W; const int par = b.par[t];
+    const float *hin = hist + ((int64_t)par * slots + slot) * hrows * W;
+    float *hout = hist + ((int64_t)(par ^ 1) * slots + slot) * hrows * W;
+    float4 v[NI], h[NI][7];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int c = (threadIdx.x + i * 256) * 4;
+        if (c >= W) continue;
+        v[i] = *reinterpret_cast<const float4 *>(x + (int64_t)t * W + c);
+#pragma unroll
+        for (int d = 1; d < 8; ++d) {                                          // the row d back: history row hrows - d, or zero before position 0
+            h[i][d - 1] = float4{0.f, 0.f, 0.f, 0.f};
+            if (d <= hrows && st - d >= 0) h[i][d - 1] = *reinterpret_cast<const float4 *>(hin + (int64_t)(hrows - d) * W + c);
+        }
+        float4 y = *reinterpret_cast<const float4 *>(parts + (int64_t)t * W + c);
+        for (int z = 1; z < nparts; ++z) {
+            const float4 p = *reinterpret_cast<const float4 *>(parts + z * stride + (int64_t)t * W + c);
+            y.x += p.x; y.y += p.y; y.z += p.z; y.w += p.w;
+        }
+        float yr[4] = {y.x, y.y, y.z, y.w};
+        OT ro[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { st_f(ro, e, yr[e]); yr[e] = ld_f(ro, e); }
+        v[i].x += mult * yr[0]; v[i].y += mult * yr[1]; v[i].z += mult * yr[2]; v[i].w += mult * yr[3];
+        *reinterpret_cast<float4 *>(x + (int64_t)t * W + c) = v[i];
+        ss += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+    }
+    ss = block_sum<256>(ss, red);
+    const float r = 1.0f / sqrtf(ss / (float)W + eps);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int c = (threadIdx.x + i * 256) * 4;
+        if (c >= W) continue;
+        const float u0[4] = {v[i].x * r, v[i].y * r, v[i].z * r, v[i].w * r};
+        float a1[4] = {0.f, 0.f, 0.f, 0.f}, a2[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {                                          // tap j weighs the row taps - 1 - j back
+            if (j >= taps) break;
+            const int d = taps - 1 - j;
+            float uu[4] = {u0[0], u0[1], u0[2], u0[3]};
+#pragma unroll
+            for (int q = 1; q < 8; ++q) if (d == q) { uu[0] = h[i][q - 1].x; uu[1] = h[i][q - 1].y; uu[2] = h[i][q - 1].z; uu[3] = h[i][q - 1].w; }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                a1[e] += w1[(int64_t)(c + e) * taps + j] * (g1 * uu[e]);
+                if (out2) a2[e] += w2[(int64_t)(c + e) * taps + j] * (g2 * uu[e]);
+            }
+            if (d < hrows) *reinterpret_cast<float4 *>(hout + (int64_t)(hrows - 1 - d) * W + c) = float4{uu[0], uu[1], uu[2], uu[3]};
+        }
+        float o1[4], o2[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { o1[e] = g1 * u0[e] + a1[e]; o2[e] = g2 * u0[e] + a2[e]; }
+        st4_f(out1, (int64_t)t * W + c, o1);
+        if (out2) st4_f(out2, (int64_t)t * W + c, o2);
+    }
+}
+// the join alone (behind the last layer)
+template <class OT>
+__global__ __launch_bounds__(256) void axpy_parts_kernel(float *__restrict__ x, const float *__restrict__ parts, int nparts, int64_t n, float m) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    float y = parts[i];
+    for (int z = 1; z < nparts; ++z) y += parts[z * n + i];
+    OT r;
+    st_f(&r, 0, y);
+    x[i] += m * ld_f(&r, 0);
+}
+
 // ------------------------------------------------------------------------------------------------ K / V rows into the paged caches
 template <class CT>
 __global__ __launch_bounds__(256) void kv_store_kernel(const CT *__restrict__ proj, int64_t ld, int64_t kcol, int64_t vcol, Batch b, int G, int D, int Dv,
@@ -994,6 +1072,31 @@ int norm_canon(const float *x, const Batch &b, int64_t W, float eps, int taps, f
     if (bf16) norm_canon_kernel<bf16_t><<<dim3((unsigned)b.T), dim3(256), lds, s>>>(x, b, (int)W, eps, taps, g1, w1, (bf16_t *)out1, g2, w2, (bf16_t *)out2, hist, slots);
     else norm_canon_kernel<float><<<dim3((unsigned)b.T), dim3(256), lds, s>>>(x, b, (int)W, eps, taps, g1, w1, (float *)out1, g2, w2, (float *)out2, hist, slots);
     return launched("norm_canon");
+}
+
+bool join_norm_canon_ok(const Batch &b, int64_t W, int taps, const float *x, const float *parts, const float *hist) {
+    return b.T == b.B && b.max_rows == 1 && W % 4 == 0 && W <= 4096 && taps >= 1 && taps <= 8 && ((uintptr_t)x | (uintptr_t)parts | (uintptr_t)hist) % 16 == 0;
+}
+int join_norm_canon(float *x, const float *parts, int nparts, float mult, const Batch &b, int64_t W, float eps, int taps, float g1, const float *w1, void *out1, float g2, const float *w2,
+                    void *out2, bool bf16, float *hist, int64_t slots, hipStream_t s) {
+    if (b.T == 0) return 0;
+    if (!join_norm_canon_ok(b, W, taps, x, parts, hist) || nparts < 1) return nvr::fail(NVR_ERR_UNSUPPORTED, "join_norm_canon: %d rows of %d sequences, width %ld, %d taps", b.T, b.B, (long)W, taps);
+    const dim3 grid((unsigned)b.T);
+#define NVR_JNC(NI_)                                                                                                                                                                   \
+    do {                                                                                                                                                                               \
+        if (bf16) join_norm_canon_kernel<bf16_t, NI_><<<grid, dim3(256), 0, s>>>(x, parts, nparts, mult, b, (int)W, eps, taps, g1, w1, (bf16_t *)out1, g2, w2, (bf16_t *)out2, hist, slots); \
+        else join_norm_canon_kernel<float, NI_><<<grid, dim3(256), 0, s>>>(x, parts, nparts, mult, b, (int)W, eps, taps, g1, w1, (float *)out1, g2, w2, (float *)out2, hist, slots);       \
+    } while (0)
+    if (W <= 1024) NVR_JNC(1); else if (W <= 2048) NVR_JNC(2); else NVR_JNC(4);
+#undef NVR_JNC
+    return launched("join_norm_canon");
+}
+int axpy_parts(float *x, const float *parts, int nparts, bool bf16, float mult, int64_t n, hipStream_t s) {
+    if (n == 0) return 0;
+    const dim3 grid((unsigned)((n + 255) / 256));
+    if (bf16) axpy_parts_kernel<bf16_t><<<grid, dim3(256), 0, s>>>(x, parts, nparts, n, mult);
+    else axpy_parts_kernel<float><<<grid, dim3(256), 0, s>>>(x, parts, nparts, n, mult);
+    return launched("axpy_parts");
 }
 
 int kv_store(const void *proj, int64_t ld, int64_t kcol, int64_t vcol, const Batch &b, int64_t G, int64_t D, int64_t Dv, void *kc, void *vc, bool bf16,

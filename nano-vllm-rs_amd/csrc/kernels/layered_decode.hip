@@ -39,8 +39,8 @@ __device__ __forceinline__ bf16x4 read_tr(const char *p) { return __builtin_amdg
 // One build per size class C >= D, Dv, with no bound inside: a piece of a row past its end is read again from its last 16 bytes (the query's numbers there are zero, the output's are not stored).
 constexpr int image_stride(int C) { return C * 2 + 32; }             // bytes; an odd multiple of 32: the 8 rows 32 lanes read together sit on different banks
 
-// SHARED: the values are the first Dv numbers of the key rows.  bs_shift: log2 of the page size, or -1.  g: query rows per key/value head, in nrb groups of up to 16.  Grid: shares, groups, sequences.
-template <int C, bool DIFF, bool SHARED>
+// SHARED: the values are the first Dv numbers of the key rows.  PEN: a.pen, the penalty of every distance in the base-2 domain, is subtracted from a head's scores.  bs_shift: log2 of the page size, or -1.  g: query rows per key/value head, in nrb groups of up to 16.  Grid: shares, groups, sequences.
+template <int C, bool DIFF, bool SHARED, bool PEN = false>
 __global__ __launch_bounds__(256, 1) void attn_decode_kernel(SinkAttnArgs a, Batch b, int bs_shift, int g, int nsplit, int nrb, float *__restrict__ part_o,
                                                              float *__restrict__ part_ml, unsigned int *__restrict__ tickets) {
     constexpr int NKS = C / 32, NDT = C / 16, VS = image_stride(C), OS = C + 4;
@@ -55,6 +55,7 @@ __global__ __launch_bounds__(256, 1) void attn_decode_kernel(SinkAttnArgs a, Bat
     const bf16_t *kc = (const bf16_t *)a.kc, *vc = (const bf16_t *)a.vc;
     char *img = smem + wave * CH * VS;
     const float scale2 = a.scale * kLog2e;
+    const float *pen = PEN ? a.pen + (int64_t)(kvh * g + r0 + min(lm, nr - 1)) * a.pen_n : nullptr;
 
     bf16x8 qf[NKS];
     {
@@ -95,6 +96,12 @@ __global__ __launch_bounds__(256, 1) void attn_decode_kernel(SinkAttnArgs a, Bat
 #pragma unroll
                 for (int ks = 0; ks < NKS; ++ks) vf[mt][ks] = *reinterpret_cast<const bf16x8 *>(vp + min(ks * 32 + lq * 8, Dv - 8));
         }
+        f32x4 pn[2];
+        if constexpr (PEN)
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) pn[mt][e] = pen[max(pos - (base + mt * 16 + lq * 4 + e), 0)];
         f32x4 s[2];
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
@@ -118,7 +125,7 @@ __global__ __launch_bounds__(256, 1) void attn_decode_kernel(SinkAttnArgs a, Bat
             for (int e = 0; e < 4; ++e) {
                 const int j = base + mt * 16 + lq * 4 + e;
                 const bool out = j > pos || (a.window > 0 && pos - j >= a.window && j >= a.keep_first);
-                s[mt][e] = out ? -INFINITY : s[mt][e] * scale2;
+                s[mt][e] = out ? -INFINITY : PEN ? fmaf(s[mt][e], scale2, -pn[mt][e]) : s[mt][e] * scale2;
                 mx = fmaxf(mx, s[mt][e]);
             }
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64)); mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
@@ -241,7 +248,8 @@ int launch(const SinkAttnArgs &a, const Batch &b, int nsplit, int nrb, float *po
     const size_t lds = std::max((size_t)4 * CH * image_stride(C), (size_t)4 * 16 * (C + 4) * 4);
     const bool shared = a.vld != 0;
     const int bs_shift = (b.block_size & (b.block_size - 1)) == 0 ? __builtin_ctz((unsigned)b.block_size) : -1;
-    if (a.lambda) attn_decode_kernel<C, true, false><<<grid, blk, lds, s>>>(a, b, bs_shift, g, nsplit, nrb, po, pml, tickets);
+    if (a.pen) attn_decode_kernel<C, false, false, true><<<grid, blk, lds, s>>>(a, b, bs_shift, g, nsplit, nrb, po, pml, tickets);
+    else if (a.lambda) attn_decode_kernel<C, true, false><<<grid, blk, lds, s>>>(a, b, bs_shift, g, nsplit, nrb, po, pml, tickets);
     else if (shared) attn_decode_kernel<C, false, true><<<grid, blk, lds, s>>>(a, b, bs_shift, g, nsplit, nrb, po, pml, tickets);
     else attn_decode_kernel<C, false, false><<<grid, blk, lds, s>>>(a, b, bs_shift, g, nsplit, nrb, po, pml, tickets);
     hipError_t e = hipGetLastError();
@@ -254,16 +262,16 @@ int row_blocks(const SinkAttnArgs &a) { return (a.H * (a.lambda ? 2 : 1) / a.G +
 }  // namespace
 
 int prepare_decode() {
-    const void *fns[] = {(const void *)attn_decode_kernel<64, true, false>, (const void *)attn_decode_kernel<64, false, true>, (const void *)attn_decode_kernel<64, false, false>,
-                         (const void *)attn_decode_kernel<128, true, false>, (const void *)attn_decode_kernel<128, false, true>, (const void *)attn_decode_kernel<128, false, false>,
-                         (const void *)attn_decode_kernel<256, true, false>, (const void *)attn_decode_kernel<256, false, true>, (const void *)attn_decode_kernel<256, false, false>};
+    const void *fns[] = {(const void *)attn_decode_kernel<64, true, false>, (const void *)attn_decode_kernel<64, false, true>, (const void *)attn_decode_kernel<64, false, false>, (const void *)attn_decode_kernel<64, false, false, true>,
+                         (const void *)attn_decode_kernel<128, true, false>, (const void *)attn_decode_kernel<128, false, true>, (const void *)attn_decode_kernel<128, false, false>, (const void *)attn_decode_kernel<128, false, false, true>,
+                         (const void *)attn_decode_kernel<256, true, false>, (const void *)attn_decode_kernel<256, false, true>, (const void *)attn_decode_kernel<256, false, false>, (const void *)attn_decode_kernel<256, false, false, true>};
     for (const void *f : fns) NVR_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
     return 0;
 }
 
 bool attention_decode_ok(const SinkAttnArgs &a, bool bf16) {
     const bool shared = a.vld != 0;
-    return bf16 && !a.r1 && !a.r2 && !a.slope && !a.pen && !a.gate_bias && a.softcap == 0.f && a.chunk == 0 && !(a.lambda && a.sink) && a.G >= 1 && a.H % a.G == 0 && a.D % 32 == 0 && a.Dv % 16 == 0 &&
+    return bf16 && !a.r1 && !a.r2 && !a.slope && !(a.pen && (a.lambda || shared)) && !a.gate_bias && a.softcap == 0.f && a.chunk == 0 && !(a.lambda && a.sink) && a.G >= 1 && a.H % a.G == 0 && a.D % 32 == 0 && a.Dv % 16 == 0 &&
            a.D <= 256 && a.Dv <= 256 && !(a.v_grouped && !shared) && (!shared || (a.vc == a.kc && a.vld == a.D && a.Dv <= a.D && a.G == 1 && !a.lambda)) && a.ldq % 8 == 0 && a.ldo % 4 == 0 &&
            (((uintptr_t)a.q | (uintptr_t)a.kc | (uintptr_t)a.vc) & 15) == 0 && ((uintptr_t)a.out & 7) == 0;
 }
@@ -273,7 +281,7 @@ int attention_decode_groups(const SinkAttnArgs &a) { return a.G * row_blocks(a);
 int attention_decode(const SinkAttnArgs &a, const Batch &b, int max_splits, void *workspace, size_t workspace_bytes, unsigned int *tickets, int num_tickets, hipStream_t s) {
     if (b.B == 0) return 0;
     if (b.T != b.B || b.max_rows != 1) return nvr::fail(NVR_ERR_INVALID_ARG, "attention_decode: %d rows of %d sequences (one each)", b.T, b.B);
-    if (!attention_decode_ok(a, true)) return nvr::fail(NVR_ERR_UNSUPPORTED, "attention_decode: shape outside the kernel");
+    if (!attention_decode_ok(a, true) || (a.pen && a.pen_n < 1)) return nvr::fail(NVR_ERR_UNSUPPORTED, "attention_decode: shape outside the kernel");
     const int nrb = row_blocks(a);
     const int64_t pairs = (int64_t)b.B * a.G * nrb;
     if (b.B > 65535 || a.G * nrb > 65535) return nvr::fail(NVR_ERR_INVALID_ARG, "attention_decode: %d sequences of %d groups", b.B, a.G * nrb);

@@ -195,6 +195,13 @@ int LayeredModel::init(nvr_model_runner &r) {
     RC(dmalloc(&x, (size_t)(MT * W * 4))); RC(dmalloc(&tmp, (size_t)(MT * W * esz)));
     RC(dmalloc(&proj, (size_t)(MT * max_nmix * esz))); RC(dmalloc(&gu, (size_t)(MT * 2 * max_ff * esz))); RC(dmalloc(&ret_o, (size_t)(MT * max_hv * 4)));
     RC(dmalloc(&a1, (size_t)(MT * W * esz))); RC(dmalloc(&a2, (size_t)(MT * W * esz))); RC(dmalloc(&cat, (size_t)(MT * max_kcat * esz)));
+    if (bf16) {                                             // decode steps: the output product's partial sums, the counters of the attention's shares
+        parts_rows = std::min<int64_t>(r.max_seqs, 64);
+        RC(own(&parts, (size_t)(4 * parts_rows * W * 4)));
+        int64_t groups = 0;
+        for (const LayeredSpec::Layer &L : spec.layers) if (L.mixer == LayeredSpec::ATTENTION) groups = std::max(groups, L.kv_heads * ((L.heads / L.kv_heads + 15) / 16));
+        if (groups) { dec_tickets_n = r.max_seqs * groups; RC(own(&dec_tickets, (size_t)dec_tickets_n * 4)); }
+    }
     }
     const int64_t MT = r.max_tokens;
     logit_rows_cap = std::max<int64_t>(r.max_seqs, 64);
@@ -442,10 +449,17 @@ int LayeredModel::forward(nvr_model_runner &r, const StepPlan &p) {
     const int64_t W = spec.width;
     const float eps = (float)spec.eps;
     RC(kl::embed_scale(embed, bf16, b.ids, T, W, (float)spec.embedding_scale, x, s));
+    int64_t owed = 0;                                                               // partial sums of the last layer's output product that still have to join the stream
     for (size_t ri = 0; ri < spec.runs.size(); ++ri) {
         const size_t li = (size_t)spec.runs[ri];
         const LayeredSpec::Layer &L = spec.layers[li]; const LayerW &w = lw[li]; RunState &st = rs[ri];
-        RC(kl::norm_canon(x, b, W, eps, (int)spec.taps, w.g1, w.canon1, a1, w.g2, w.canon2, L.has_mlp ? a2 : nullptr, bf16, st.hist, slots, s));
+        if (owed && kl::join_norm_canon_ok(b, W, (int)spec.taps, x, parts, st.hist))
+            RC(kl::join_norm_canon(x, parts, (int)owed, (float)spec.residual_mult, b, W, eps, (int)spec.taps, w.g1, w.canon1, a1, w.g2, w.canon2, L.has_mlp ? a2 : nullptr, bf16, st.hist, slots, s));
+        else {
+            if (owed) RC(kl::axpy_parts(x, parts, (int)owed, bf16, (float)spec.residual_mult, T * W, s));
+            RC(kl::norm_canon(x, b, W, eps, (int)spec.taps, w.g1, w.canon1, a1, w.g2, w.canon2, L.has_mlp ? a2 : nullptr, bf16, st.hist, slots, s));
+        }
+        owed = 0;
         RC(gemm(r, a1, W, w.mix, T, W, w.nmix, proj));
         if (L.mixer == LayeredSpec::ATTENTION) {
             kl::SinkAttnArgs a{};
@@ -473,12 +487,17 @@ int LayeredModel::forward(nvr_model_runner &r, const StepPlan &p) {
                     wm.pen_dirty = false;
                 }
                 a.pen = wm.pen; a.pen_n = (int32_t)r.max_pos;
+                kl::SinkAttnArgs d = a;                                             // one position per sequence: the kernel for few query rows, with the table in the two factors' place (16 x 1040 keys of 8 heads: 40.2 + 5.5 us with the merge -> 25.0)
+                d.r1 = d.r2 = nullptr;
+                if (p.decode_sized && kl::attention_decode_ok(d, bf16)) RC(decode_attention(r, d, p));
+                else {
                 const size_t gi = (size_t)(std::find(attn_groups.begin(), attn_groups.end(), L.heads / L.kv_heads) - attn_groups.begin());
                 // decode-sized steps over long contexts: few tiles, many keys each — spread every tile's keys over several workgroups
                 const int64_t wgs = (int64_t)n_tiles[gi] * L.kv_heads;
                 int64_t nsplit = 1;
                 if (wgs < r.num_cus && max_ctx >= 512) nsplit = std::max<int64_t>(1, std::min<int64_t>({(2 * r.num_cus) / wgs, (max_ctx + 255) / 256, 16}));
                 RC(kl::sink_attention_tiled(a, b, (const kl::AttnTile *)(in_dev + o_tiles[gi]), n_tiles[gi], (int)nsplit, attn_ws, attn_ws_bytes, s));
+                }
             } else
                 RC(kl::sink_attention(a, b, bf16, s));
         } else {
@@ -493,9 +512,18 @@ int LayeredModel::forward(nvr_model_runner &r, const StepPlan &p) {
             RC(gemm(r, a2, W, w.gu, T, W, 2 * L.ff, gu));
             RC(kl::clamped_glu(gu, T, L.ff, (float)L.limit, 1.702f, (char *)cat + (size_t)(w.mixcols * esz), w.kcat, bf16, s));
         }
-        RC(gemm(r, cat, w.kcat, w.out, T, w.kcat, W, tmp));
-        RC(kl::axpy(x, tmp, bf16, (float)spec.residual_mult, T * W, s));
+        // decode steps: the product over mixer and feed-forward together is long and narrow (5120 x 1024 at the smallest size: 64 workgroups, 15.0 us; in 4 parts 5.9): cut along k, joined by the next
+        // launch that reads the stream
+        const int64_t S = (p.decode_sized && parts && T <= parts_rows && w.kcat % 32 == 0 && W % 16 == 0) ? nvr::kb::decode_splitk_slices(T, w.kcat, W) : 1;
+        if (S > 1 && w.kcat % (32 * S) == 0) {
+            RC(nvr::kb::linear_splitk((const uint16_t *)cat, w.kcat, (const uint16_t *)w.out, T, w.kcat, W, S, parts, s, nullptr));
+            owed = S;
+        } else {
+            RC(gemm(r, cat, w.kcat, w.out, T, w.kcat, W, tmp));
+            RC(kl::axpy(x, tmp, bf16, (float)spec.residual_mult, T * W, s));
+        }
     }
+    if (owed) RC(kl::axpy_parts(x, parts, (int)owed, bf16, (float)spec.residual_mult, T * W, s));
     RC(kl::norm_rows(x, d_want, (int64_t)R, W, eps, gfinal, xsel, bf16, s));
     return gemm(r, xsel, W, head, (int64_t)R, W, spec.vocab, r.logits, true);
 }

@@ -185,6 +185,7 @@ public:
     // streams layout
     void *v_first = nullptr;                                                // the step's values of the first layer that mixes: [max tokens][G Dv]
     void *dec_ws = nullptr; size_t dec_ws_bytes = 0; unsigned int *dec_tickets = nullptr; int64_t dec_tickets_n = 0;   // the dense graph's decode attention: split partials, arrival counters (zero between launches)
+    float *parts = nullptr; int64_t parts_rows = 0;                         // partial sums of a decode step's output product: [4][parts_rows][W]
     std::vector<void *> owned;                                              // device allocations of the sequential layout (freed with the model)
     // activations
     float *x = nullptr, *ret_o = nullptr;                                  // residual stream, retention outputs: f32
