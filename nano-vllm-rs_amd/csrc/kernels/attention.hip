@@ -804,13 +804,18 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
             part_size = (int)ps; np = (int)((mc + ps - 1) / ps);
         } else np = parts_for(a.nq, a.KVH, mc, waves, &part_size);
     }
+    // Few pairs over short contexts (a chat's first hundreds of tokens): the partitions' hand-off — partials out, a ticket, partials back — costs more than the keys: ONE workgroup of
+    // eight waves per pair, whose 128 keys per round need two rounds for the 256-token bucket, the second requested under the
+    // first.  Qwen3-0.6B at 128 keys, us a step: 903 -> 860 at 9 sequences, 948 -> 917 at 16
+    const bool brief = paged && a.workspace && !shared && mc <= 256 && pairs < 192;
+    if (brief) { np = 1; waves = 8; }
     // Work-balanced form (attn_share_kernel): a pair count whose last round of one-workgroup-per-pair launches would be mostly empty — 257..2047 pairs with
     // >= 15 % of the rounds' slots unused (33..37 and 65..74 sequences at 8 kv heads, ...), contexts long enough for the stream to matter — or a RAGGED batch
     // (balance_hint: the caller knows the sum of the contexts; per-pair launches size every pair's partitions by the LONGEST context and leave the short sequences'
     // workgroups idle, or — with several pairs per CU — end on the long sequences' workgroups: 32 sequences of 256..8192 keys 4.09 -> 2.43 ms per Qwen3-0.6B step,
     // 64 of 64..4096 keys 3.26 -> 2.78).  NVR_ATTN_SHARE=0: off.
     if constexpr (G * D <= 512)
-    if (!shared && paged && a.workspace && a.tickets && !a.seq_of_q && waves == 8 && p.bs_shift >= 0 && a.block_size >= 8 && a.nq <= 1024 && share_enabled()) {
+    if (!brief && !shared && paged && a.workspace && a.tickets && !a.seq_of_q && waves == 8 && p.bs_shift >= 0 && a.block_size >= 8 && a.nq <= 1024 && share_enabled()) {
         const int64_t cus = share_workgroups(), rounds = (pairs + cus - 1) / cus, units = (mc + 63) / 64;
         const int64_t cap = a.workspace_bytes ? (int64_t)(a.workspace_bytes / ((size_t)a.nq * a.H * (D + 2) * sizeof(float))) : units;
         const bool by_count = pairs > cus && rounds * cus * 100 >= pairs * 115 && mc >= 256;
@@ -849,7 +854,11 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
         if (int rc = flash_shared_prefix(a.q, a.ldq, a.k, a.v, a.block_tables, a.max_blocks, a.block_size, a.nq, a.H, a.KVH, a.D, a.scale,
                                          shared_part, sparts, np, p.part_o, p.part_ml, s, a.shared_rows, a.shared_count)) return rc;
     {
-        if (waves == 8) launch_cfg<D, G, DU / 2, 8, true>(p, paged, direct, nwg, s, fuse);  // K/V streamed once: nt loads
+        if (brief) {
+            const bool ub = p.block_size % (64 / (D / 8) * DU) == 0;
+            if (ub) attn_rows_kernel<D, G, true, true, DU, 8, true, true><<<dim3((unsigned)nwg), dim3(512), 0, s>>>(p);
+            else attn_rows_kernel<D, G, true, true, DU, 8, true, false><<<dim3((unsigned)nwg), dim3(512), 0, s>>>(p);
+        } else if (waves == 8) launch_cfg<D, G, DU / 2, 8, true>(p, paged, direct, nwg, s, fuse);  // K/V streamed once: nt loads
         else if (paged && waves == 1) { if constexpr (G * (D / 4) <= 64) launch_cfg<D, G, DU, 1, true>(p, paged, direct, nwg, s, fuse, shm); }   // (U = 2: 3.18-3.20 against 3.14-3.17 ms per configs[4] step)
         else if (paged && waves == 2) { if constexpr (G * (D / 4) <= 128) launch_cfg<D, G, DU, 2, true>(p, paged, direct, nwg, s, fuse, shm); }
         else if (paged) launch_cfg<D, G, DU, 4, true>(p, paged, direct, nwg, s, fuse, shm);
