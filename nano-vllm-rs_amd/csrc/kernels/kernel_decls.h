@@ -58,6 +58,15 @@ int64_t stream_row_limit();    // rows up to which the weight-streaming kernels 
 bool splitk_prefers_tiles(int64_t T, int64_t K, int64_t N);   // linear_splitk takes the LDS-tiled kernel (gemm_tiled_splitk) for this shape
 int linear_splitk(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, int64_t S,
                   float *slabs, hipStream_t s, const half_bits *Wt = nullptr);
+// Products of few rows that form their input, RMSNorm(h_in + sum_z slabs[z]) * w, themselves (linear.hip: NORM): S slabs, `stride` elements apart; h_out (another buffer than
+// h_in) receives the new residual rows.  *_ok: whether the shape takes the kernel
+bool norm_linear_plain_ok(int64_t T, int64_t K, int64_t N, int64_t S);
+bool norm_linear_silu_ok(int64_t T, int64_t K, int64_t I, int64_t S);
+bool norm_linear_rope_ok(int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D, int64_t S);
+int norm_linear(const NormIn &nm, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *y, hipStream_t s, const half_bits *Wt);
+int norm_linear_silu_mul(const NormIn &nm, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s, const half_bits *Wt);
+int norm_linear_qkv_rope_store(const NormIn &nm, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D, const int64_t *positions, const int32_t *slots,
+                               const float *cos_t, const float *sin_t, half_bits *qkv, half_bits *k_cache, half_bits *v_cache, hipStream_t s, const half_bits *Wt);
 // h = fp16(h + fp16(sum_z slabs[z])), out = rmsnorm(h)*w
 int add_rmsnorm_slabs(half_bits *h, const float *slabs, int64_t S, const half_bits *w, float eps, int64_t T, int64_t Hd,
                       half_bits *out, hipStream_t s);

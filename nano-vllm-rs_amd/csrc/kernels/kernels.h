@@ -17,6 +17,9 @@ constexpr int LM_HEAD_MAX_PARTS = 2048;
 
 struct TpArgmaxRec { float val; int32_t pad; int64_t idx; };           // 16 B: a rank's (max, global arg-max) of one row
 
+// the input of a product that forms RMSNorm(h_in + sum of S slabs, `stride` elements apart) * w itself (linear.hip: NORM); h_out receives the new residual rows
+struct NormIn { const half_bits *h_in; const float *slabs; int64_t stride; int32_t S; const half_bits *w; float eps; half_bits *h_out; };
+
 // Attention over rows of keys addressed either through a block table (paged) or contiguously.
 struct AttnArgs {
     const half_bits *q; int64_t ldq;          // q[t] at q + t*ldq, heads contiguous [H, D]

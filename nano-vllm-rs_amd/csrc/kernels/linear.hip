@@ -30,6 +30,9 @@
 namespace nvr { namespace NVR_DT_NS {
 
 enum { EPI_F16 = 0, EPI_F32 = 1, EPI_SILU = 2, EPI_ROPE = 3, EPI_SLAB = 4 };
+// rows up to which a decode step's add + norm rides on the product behind it: every workgroup reads every row's slabs again (16 KB a row at K = 1024), so the launch it saves pays for one
+// or two rows — Qwen3-0.6B at 300 keys, us a step apart / riding: 802 / 769 at one row, 822 / 800 at two, 851 / 890 at four
+constexpr int64_t NORM_ROWS = 2;
 
 struct LinEpi {
     // EPI_SILU: N is the intermediate size I; W holds gate rows [0,I) and up rows [I,2I)
@@ -42,6 +45,7 @@ struct LinEpi {
     // W is the TILED copy [N/16][K/32][16][32] (retile_weight): one wave-instruction reads 1 KiB contiguous
     int32_t tiled;
     int32_t gelu;                          // EPI_SILU: gelu (tanh form) instead of silu; EPI_F16: gelu (error function) of the product
+    NormIn norm;                           // NORM instances: x is formed by the workgroup itself
 };
 
 // W row handled by local row r (0..15) of n-tile i of workgroup bx
@@ -57,11 +61,16 @@ __device__ __forceinline__ int w_row(int bx, int i, int NT, int r, int N, const 
     return n < N ? n : N - 1;
 }
 
-template <int NT, int MT, int WAVES, int EPI>
+// NORM (MT = 1, T <= NORM_ROWS, T K <= NORM_ELEMS): the rows are RMSNorm(h + sum of the split-k slabs) (what add_rmsnorm_slabs leaves in memory, with its roundings: 16-bit sum of
+// the slabs, 16-bit residual add, 16-bit normalised row), formed by every workgroup in LDS while its first weight pieces are on the way, so that the add + norm launch in front of
+// the product disappears; workgroup 0 writes the new residual rows to norm.h_out, a second buffer, since the others still read the old ones.
+constexpr int NORM_ELEMS = 4096;
+template <int NT, int MT, int WAVES, int EPI, bool NORM = false>
 __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t *__restrict__ x, int64_t ldx,
                                                                    const half_t *__restrict__ W, int T, int K, int N,
                                                                    void *__restrict__ y, LinEpi epi) {
     constexpr int U = 4;                                    // k-steps in flight per wave
+    extern __shared__ __attribute__((aligned(16))) char norm_lds[];   // NORM: the normalised rows [T][K + 8]
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = lane & 15, q = lane >> 4;
     const int m0 = blockIdx.y * (16 * MT);
@@ -104,6 +113,67 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
         if (head >= epi.H && epi.slots && m < T) rope_slot = epi.slots[m];
     }
     constexpr int KS = 32 * WAVES;
+    half8_t a_first[U][NT];                                  // NORM: the first pieces of the weights, requested in front of the norm (they depend on nothing)
+    if constexpr (NORM) {
+        static_assert(MT == 1, "one row block");
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+                a_first[u][i] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(wrow[i] + (int64_t)min(wave * 32 + u * KS, K - 32) * kmul));
+        constexpr int NI = NORM_ELEMS / 4 / (WAVES * 64);     // 4-column pieces per thread
+        __shared__ float ss_w[NI * WAVES];                    // sums of squares of 64 neighbouring pieces (K is a multiple of 256: inside one row)
+        half_t *xs = reinterpret_cast<half_t *>(norm_lds);
+        const NormIn &nm = epi.norm;
+        const int per_row = K / 4, total = T * per_row;
+        half4_t hv[NI], gv[NI]; float4_t sv[NI][4];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int idx = i * (WAVES * 64) + (int)threadIdx.x;
+            if (idx < total) {
+                const int row = idx / per_row, c = (idx - row * per_row) * 4;
+                const int64_t o = (int64_t)row * K + c;
+                hv[i] = *reinterpret_cast<const half4_t *>((const half_t *)nm.h_in + o); gv[i] = *reinterpret_cast<const half4_t *>((const half_t *)nm.w + c);
+#pragma unroll
+                for (int z = 0; z < 4; ++z) sv[i][z] = z < nm.S ? *reinterpret_cast<const float4_t *>(nm.slabs + z * nm.stride + o) : (float4_t){0.f, 0.f, 0.f, 0.f};
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int idx = i * (WAVES * 64) + (int)threadIdx.x;
+            if (idx - lane < total) {                         // (wave-uniform: total is a multiple of 64)
+                float ss = 0.f;
+                float4_t a = sv[i][0];
+#pragma unroll
+                for (int z = 1; z < 4; ++z) a += sv[i][z];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    hv[i][e] = to_half_rn((float)hv[i][e] + (float)to_half_rn(a[e]));
+                    const float f = (float)hv[i][e]; ss += f * f;
+                }
+                ss = wave_sum(ss);
+                if (lane == 0) ss_w[i * WAVES + wave] = ss;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int idx = i * (WAVES * 64) + (int)threadIdx.x;
+            if (idx < total) {
+                const int row = idx / per_row, c = (idx - row * per_row) * 4;
+                float tot = 0.f;
+                for (int k = 0; k < per_row / 64; ++k) tot += ss_w[row * (per_row / 64) + k];
+                const float rms = sqrtf(tot / (float)K + nm.eps);
+                half4_t o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = to_half_rn(__fmul_rn(__fdiv_rn((float)hv[i][e], rms), (float)gv[i][e]));
+                *reinterpret_cast<half4_t *>(xs + row * (K + 8) + c) = o;
+                if (blockIdx.x == 0) *reinterpret_cast<half4_t *>((half_t *)nm.h_out + (int64_t)row * K + c) = hv[i];
+            }
+        }
+        __syncthreads();
+        xrow[0] = xs + (int64_t)min(r, T - 1) * (K + 8) + q * 8;
+    }
     constexpr bool SLABBED = EPI == EPI_SLAB;
     const int kbeg = SLABBED ? blockIdx.z * epi.kslice : 0;
     if (SLABBED) K = min(K, kbeg + epi.kslice);
@@ -114,7 +184,10 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
             const int kk = k + u * KS;
             if (kk < K) {
 #pragma unroll
-                for (int i = 0; i < NT; ++i) a[u][i] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(wrow[i] + (int64_t)kk * kmul));
+                for (int i = 0; i < NT; ++i) {
+                    if (NORM && k == kbeg + wave * 32) a[u][i] = a_first[u][i];
+                    else a[u][i] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(wrow[i] + (int64_t)kk * kmul));
+                }
 #pragma unroll
                 for (int j = 0; j < MT; ++j) b[u][j] = *reinterpret_cast<const half8_t *>(xrow[j] + kk);
             } else {
@@ -425,6 +498,34 @@ int linear_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, i
         else launch<1, 2, 4, EPI_ROPE>(xx, ldx, ww, (int)T, (int)K, N, qkv, e, gx, s);
     }
     return launch_check("linear_qkv_rope_store");
+}
+
+// ---- products of a decode step of few rows whose workgroups form RMSNorm(h + slabs) themselves (linear_skinny_kernel, NORM)
+bool norm_linear_ok(int64_t T, int64_t K, int64_t S) { return T >= 1 && T <= NORM_ROWS && K % 256 == 0 && T * K <= NORM_ELEMS && (S == 2 || S == 4); }
+template <int NT, int EPI>
+static int norm_launch(const NormIn &nm, const half_bits *W, int64_t T, int64_t K, int64_t N, void *y, LinEpi e, int64_t gx, bool tiled, hipStream_t s, const char *what) {
+    if (!norm_linear_ok(T, K, nm.S)) return nvr::fail(NVR_ERR_UNSUPPORTED, "%s: T=%ld K=%ld, %d slabs", what, (long)T, (long)K, nm.S);
+    e.norm = nm; e.tiled = tiled;
+    linear_skinny_kernel<NT, 1, 8, EPI, true><<<dim3((unsigned)gx), dim3(512), (size_t)(T * (K + 8) * 2), s>>>(nullptr, 0, (const half_t *)W, (int)T, (int)K, (int)N, y, e);
+    return launch_check(what);
+}
+// which products of these shapes take the weight-streaming kernel above at so few rows (large weights have a kernel of their own)
+bool norm_linear_plain_ok(int64_t T, int64_t K, int64_t N, int64_t S) { return norm_linear_ok(T, K, S) && N % 16 == 0 && !linear_stream_ok(T, K, N, K); }
+bool norm_linear_silu_ok(int64_t T, int64_t K, int64_t I, int64_t S) { return norm_linear_ok(T, K, S) && I % 16 == 0 && !linear_stream_silu_ok(T, K, I, K); }
+bool norm_linear_rope_ok(int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D, int64_t S) { return norm_linear_ok(T, K, S) && D % 16 == 0 && !linear_stream_rope_ok(T, K, H, KVH, D, K); }
+int norm_linear(const NormIn &nm, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *y, hipStream_t s, const half_bits *Wt) {
+    return norm_launch<1, EPI_F16>(nm, Wt ? Wt : W, T, K, N, y, LinEpi{}, N / 16, Wt != nullptr, s, "norm + linear");
+}
+int norm_linear_silu_mul(const NormIn &nm, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s, const half_bits *Wt) {
+    return norm_launch<2, EPI_SILU>(nm, Wt ? Wt : W, T, K, I, out, LinEpi{}, I / 16, Wt != nullptr, s, "norm + gate_up + silu");
+}
+int norm_linear_qkv_rope_store(const NormIn &nm, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D, const int64_t *positions, const int32_t *slots,
+                               const float *cos_t, const float *sin_t, half_bits *qkv, half_bits *k_cache, half_bits *v_cache, hipStream_t s, const half_bits *Wt) {
+    LinEpi e{};
+    e.pos = positions; e.slots = slots; e.cos_t = cos_t; e.sin_t = sin_t; e.kc = (half_t *)k_cache; e.vc = (half_t *)v_cache;
+    e.H = (int32_t)H; e.KVH = (int32_t)KVH; e.D = (int32_t)D;
+    const int64_t N = (H + 2 * KVH) * D;
+    return norm_launch<1, EPI_ROPE>(nm, Wt ? Wt : W, T, K, N, qkv, e, N / 16, Wt != nullptr, s, "norm + qkv + rope");
 }
 
 }}  // namespace nvr::k / nvr::kb (NVR_DT_NS)

@@ -881,13 +881,27 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
     const bool embed_norm = L > 0 && KD(embedding_rmsnorm_ok(T, Hd));                    // decode-sized: K1 + the first norm in one launch
     if (embed_norm) RC(KD(embedding_rmsnorm(ids, T, embed, layers[0].ln1, mc.rms_norm_eps, Hd, h, n, st)));
     else RC(KD(embedding(ids, T, embed, Hd, h, st)));
+    // Decode steps of few rows: the split-k slabs of o_proj and down_proj are added to the residual stream and normalised by the workgroups of the product behind them (linear.hip:
+    // NORM) instead of a launch of their own; the residual stream then alternates between h and proj (free in such a step: the slabs take proj's place).  `owed`: slabs of the
+    // down_proj in front of this layer
+    const int64_t S_o = KD(decode_splitk_slices(T, H * D, Hd)), S_d = KD(decode_splitk_slices(T, I, Hd));
+    const bool ride = !is_prefill && !comm.active() && tp == 1 && !mc.use_bias && Hd <= 2048 && KD(norm_linear_silu_ok(T, Hd, I, S_o)) && 
+                      (mc.qk_norm ? KD(norm_linear_plain_ok(T, Hd, QKV, S_d)) : KD(norm_linear_rope_ok(T, Hd, H, KVH, D, S_d)));
+    uint16_t *hc = h, *hn = proj;
+    int64_t owed = 0;
     for (int64_t l = 0; l < L; ++l) {
         const Layer &w = layers[l];
+        const uint16_t *const qkv_t = tl ? w.qkv_t : nullptr;
+        const k::NormIn before{hc, slabs, T * Hd, (int32_t)owed, w.ln1, mc.rms_norm_eps, hn};
         if (l == 0 && !embed_norm) RC(KD(rmsnorm(h, w.ln1, mc.rms_norm_eps, T, Hd, n, st)));   // later layers: see down_proj
         if (mc.qk_norm || mc.use_bias) {         // A-27: the head norms sit between the projection and RoPE: plain GEMM, then one
-            RC(KD(linear(n, Hd, w.qkv, T, Hd, QKV, qkv, false, st, tl ? w.qkv_t : nullptr)));      // norm + RoPE + KV-store launch
+            if (owed) { RC(KD(norm_linear(before, w.qkv, T, Hd, QKV, qkv, st, qkv_t))); std::swap(hc, hn); }
+            else RC(KD(linear(n, Hd, w.qkv, T, Hd, QKV, qkv, false, st, qkv_t)));                  // norm + RoPE + KV-store launch
             if (mc.use_bias) RC(KD(add_bias(qkv, w.qkv_b, T, QKV, st)));                            // A-30: the bias precedes the norms and RoPE (qwen3.rs:208-222)
             RC(KD(rope_store_kv(qkv, pos, slots, T, H, KVH, D, cos_t, sin_t, k_cache(l), v_cache(l), st, w.q_norm, w.k_norm, mc.rms_norm_eps)));
+        } else if (owed) {
+            RC(KD(norm_linear_qkv_rope_store(before, w.qkv, T, Hd, H, KVH, D, pos, slots, cos_t, sin_t, qkv, k_cache(l), v_cache(l), st, qkv_t)));
+            std::swap(hc, hn);
         } else {
             // qkv GEMM with the RoPE + KV-store epilogue (K3..K6 in one launch)
             RC(KD(linear_qkv_rope_store(n, Hd, w.qkv, T, Hd, H, KVH, D, pos, slots, cos_t, sin_t, qkv, k_cache(l), v_cache(l), st, tl ? w.qkv_t : nullptr,
@@ -922,6 +936,15 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
                 a.shared_count = (const int32_t *)(in_dev + off_dec + dof_scount);
             }
             RC(KD(attention(a, true, st)));
+        }
+        if (ride) {
+            RC(KD(linear_splitk(attn, H * D, w.o, T, H * D, Hd, S_o, slabs, st, tl ? w.o_t : nullptr)));
+            RC(KD(norm_linear_silu_mul(k::NormIn{hc, slabs, T * Hd, (int32_t)S_o, w.ln2, mc.rms_norm_eps, hn}, w.gate_up, T, Hd, I, act, st, tl ? w.gate_up_t : nullptr)));
+            std::swap(hc, hn);
+            RC(KD(linear_splitk(act, I, w.down, T, I, Hd, S_d, slabs, st, tl ? w.down_t : nullptr)));
+            owed = S_d;
+            if (l + 1 == L) RC(KD(add_rmsnorm_slabs(hc, slabs, S_d, norm, mc.rms_norm_eps, T, Hd, n, st)));
+            continue;
         }
         RC(row_parallel_norm(attn, H * D, w.o, tl ? w.o_t : nullptr, T, w.ln2, w.o_b));  // o_proj, residual :382, norm :385
         if (mc.use_bias) {                       // A-30: gate_up_proj, its bias, then SiluAndMul on the biased halves (qwen3.rs:305-314)

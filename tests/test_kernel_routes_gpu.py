@@ -260,3 +260,36 @@ def test_prompt_steps_run_their_last_layer_on_the_last_rows(dtype, qk_norm, kv_h
                 s.set_chunk(a, (L if b is None else b) - a)
             r.execute_model(seqs, True)
         assert np.abs(r.logits(n) - whole).max() < tol
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("hidden,inter,heads,kv,dim,qk_norm", [(256, 512, 4, 2, 64, 0), (1024, 1024, 8, 8, 128, 1), (2048, 512, 8, 4, 128, 0), (256, 512, 4, 1, 128, 1), (384, 512, 4, 2, 64, 0)])
+def test_decode_steps_of_one_and_two_rows_against_more(dtype, hidden, inter, heads, kv, dim, qk_norm):
+    """One or two sequences (add + norm inside the products behind them, where the width is a multiple of 256) give the logits that the same sequences give in a batch of three (launches of
+    their own): sums in another order, so within the 16-bit rounding of three layers; contexts on both sides of the 256 keys a single workgroup takes."""
+    model = nvr.ModelConfig(vocab_size=192, hidden_size=hidden, intermediate_size=inter, num_hidden_layers=3, num_attention_heads=heads, num_key_value_heads=kv, head_dim=dim,
+                            max_position_embeddings=512, rms_norm_eps=1e-6, rope_theta=1e4, tie_word_embeddings=0, init_std=hidden ** -0.5, seed=11, qk_norm=qk_norm)
+    sp = nvr.SamplingParams(temperature=0.0, ignore_eos=True)
+    lengths = [16, 127, 300]
+    prompts = [nvr.synthetic_tokens(L + 4, 4, i, 192) for i, L in enumerate(lengths)]
+
+    def steps(which):
+        r = nvr.ModelRunner(nvr.Config(skip_block_size_check=1, max_num_seqs=3, max_num_batched_tokens=512, max_model_len=512, kvcache_block_size=16, num_kvcache_blocks=64, dtype=dtype), model)
+        bm = nvr.BlockManager(64, 16)
+        seqs = [nvr.Sequence(prompts[i][:lengths[i]], sp, 16) for i in which]
+        for s in seqs:
+            bm.allocate(s)
+        r.execute_model(seqs, True)
+        out = []
+        for k in range(4):
+            for i, s in zip(which, seqs):
+                s.append_token(int(prompts[i][lengths[i] + k]))
+                bm.may_append(s)
+            r.execute_model(seqs, False)
+            out.append(r.logits(len(which)).copy())
+        return np.stack(out, 1)                                            # [sequence, step, vocabulary]
+    full = steps([0, 1, 2])
+    tol = 2.0 ** (-7 if dtype == "float16" else -4) * float(np.sqrt((full ** 2).mean())) * 4
+    for which in ([0], [1], [2], [0, 1], [1, 2]):
+        got = steps(which)
+        assert np.abs(got - full[which]).max() < tol, which
