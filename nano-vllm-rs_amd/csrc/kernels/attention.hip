@@ -443,19 +443,27 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float *__restrict
 
 // ---- work-balanced form (r06) ---------------------------------------------------------------------------------------
 // attn_rows_kernel gives every (query, kv head) pair its own workgroup(s): 264 pairs on 256 CUs (33 sequences x 8 kv heads) run as one full round and a tail,
-// 35.6 us per layer where 256 pairs take 24.5 (profiles/r06_priced_levers.txt 9.).  Here the launch is nw workgroups (one per CU) and the WORK is cut evenly: the
-// keys of all pairs, in units of CH = WAVES * TPI keys (one full round of a workgroup), pair after pair (query-major), form one line of U_tot units; workgroup w
-// walks the units [w * U_tot / nw, (w + 1) * U_tot / nw) — a suffix of one pair, whole pairs, a prefix of another.  A pair that lies inside one share is written
-// directly; a pair cut by share boundaries leaves one f32 partial per share (slot = share index - first share of the pair) and the LAST of its shares to finish
-// merges them (the ticket scheme of FUSE above: sc1 partials, one counter per pair, nobody polls; merge_partitions: the same arithmetic).
-// Paged K/V through block tables whose block size is a power of two >= TPI (the scalar block-table form), nt loads; per-segment arithmetic = attn_rows_kernel's.
+// 35.6 us per layer where 256 pairs take 24.5.  Here the launch is nw shares x KVH workgroups and the WORK is cut evenly: the keys of all queries, in units of
+// CH = WAVES * TPI keys (one full round of a workgroup), query after query, form one line of utot units; share w walks the units [w * utot / nw, (w + 1) * utot / nw)
+// — a suffix of one query's keys, whole queries, a prefix of another — once per kv head: the KVH workgroups of a share read the same cache rows at the same time.
+// A (query, kv head) pair that lies inside one share is written directly; a pair cut by share boundaries leaves one f32 partial per share (slot = share index -
+// first share of the pair) and the LAST of its shares to finish merges them (the ticket scheme of FUSE above: sc1 partials, one counter per pair, nobody polls;
+// merge_partitions: the same arithmetic).  Paged K/V through block tables whose block size is a power of two >= TPI (the scalar block-table form), nt loads.
+// What bounds it is the stream of K and V; what kept it from that, and what stands against it here:
+//  * a segment (one query's keys in one share) costs a start and a cross-wave merge of its own, about two units' time: every query is charged CHARGE units in
+//    front of its keys, so that a share of many short queries holds fewer keys (27 sequences of 64..8100 keys 40.9 -> 38.7 us, 64 of 64..4096 54.5 -> 49.1;
+//    one unit 39.1 / 51.9, four 39.0 / 50.7);
+//  * one wait per round: two rounds are in flight at any time (the block-table reload, which would make hipcc wait for everything at each round, waits for itself);
+//  * one share per CU: with those two, twice the shares only double the starts and merges (64 of 64..4096 keys: 49.1 us with one, 52.6 with two per CU).
+// Together 27 sequences of 64..8100 keys 41.8 -> 38.7 us a layer (184 MB: 4.4 -> 4.7 TB/s; 32 equal sequences of 4096 keys: 6.5).
 template <int D, int G, int U, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, int nq, int nw) {
     constexpr int LPR = D / 8, RPI = 64 / LPR, TPI = RPI * U, CH = TPI * WAVES;
     static_assert(G * D <= WAVES * 64 && G * (D / 4) <= WAVES * 64, "one pass over the (head, column) pairs");
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int dc = lane % LPR, tg = lane / LPR;
-    __shared__ int pre[1025];                               // pre[t] = units of the queries in front of t (a query's KVH pairs have the same count)
+    constexpr int CHARGE = 2;
+    __shared__ int pre[1025];                               // pre[t] = units of the queries in front of t, their charges included
     __shared__ int cx[1024];                                // ctx_lens[t]
     __shared__ float sm_acc[WAVES][G][D];
     __shared__ float sm_ml[WAVES][G][2];
@@ -465,7 +473,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
         for (int k = 0; k < nq; k += 64) {
             const int t = k + lane;
             const int c = t < nq ? p.ctx_lens[t] : 0;
-            int un = (c + CH - 1) / CH;
+            int un = c > 0 ? (c + CH - 1) / CH + CHARGE : 0;
 #pragma unroll
             for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(un, o, 64); if (lane >= o) un += v; }
             if (t < nq) { pre[t + 1] = base + un; cx[t] = c; }
@@ -474,66 +482,62 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
         if (lane == 0) pre[0] = 0;
     }
     __syncthreads();
-    const long long utot = (long long)p.KVH * pre[nq];
-    const long long ub = (long long)blockIdx.x * utot / nw, ue = (long long)(blockIdx.x + 1) * utot / nw;
+    const int g = blockIdx.x % p.KVH, ws = blockIdx.x / p.KVH;
+    const long long utot = pre[nq];
+    const long long ub = ws * utot / nw, ue = (ws + 1) * utot / nw;
     // a query without keys owns no unit: its output row is zero, as in attn_rows_kernel (L == 0)
-    for (int t0 = blockIdx.x; t0 < nq; t0 += nw)
+    for (int t0 = blockIdx.x; t0 < nq; t0 += gridDim.x)
         if (cx[t0] == 0)
             for (int x = threadIdx.x; x < p.H * D; x += WAVES * 64) p.out[(int64_t)t0 * p.H * D + x] = (half_t)0.f;
-    if (ub >= ue) return;                                   // (fewer units than workgroups: an empty share)
+    long long u = ub;
     const int row_elems = p.KVH * D;
 
     // ---- state of the segment being streamed (set by `open`, which also REQUESTS its first K/V rows: a segment is opened under the tail of the one in front) ----
-    int t = 0, g = 0, np = 1, slot = 0, p0 = 0, pend = 0, R = 0, ng = 0, gt0 = 0, bt_chunk = -1, bt_reg = 0;
+    int t = 0, np = 1, slot = 0, p0 = 0, pend = 0, R = 0, bt_chunk = -1, bt_reg = 0;
     const int32_t *bt = p.block_tables;
     half2_t qv[G][4];
-    half8_t k0[U], v0[U], kt[U], vt[U];                     // round 0 of the segment; its remainder groups
+    half8_t ka[U], va[U], kb[U], vb[U];                     // the wave's even / odd rounds: two are always requested ahead
     auto block_base = [&](int tb) -> int64_t {              // element offset of (scalar token tb, kv head g, d = 0)
         const int bi = tb >> p.bs_shift, bo = tb & (p.block_size - 1);
-        if ((bi >> 6) != bt_chunk) { bt_chunk = bi >> 6; const int idx = (bt_chunk << 6) + lane; bt_reg = idx < p.max_blocks ? bt[idx] : 0; }
+        if ((bi >> 6) != bt_chunk) {
+            bt_chunk = bi >> 6; const int idx = (bt_chunk << 6) + lane; bt_reg = idx < p.max_blocks ? bt[idx] : 0;
+            asm volatile("" : "+v"(bt_reg));                // waited for HERE: at the readlane below hipcc would wait for every K/V request in flight, on every round
+        }
         const int blk = __builtin_amdgcn_readlane(bt_reg, bi & 63);
         return (((int64_t)blk * p.block_size + bo) * p.KVH + g) * D;
     };
-    auto issue_remainder = [&]() {
-#pragma unroll
-        for (int x = 0; x < U; ++x) {
-            const int gt = gt0 + x * WAVES;
-            if (gt < ng) {
-                const int tb = p0 + gt * RPI;
-                const int64_t base = block_base(tb);
-                const unsigned off = (unsigned)(min(tg, pend - 1 - tb) * row_elems + dc * 8);
-                kt[x] = load_row16<true>(p.k + base + off); vt[x] = load_row16<true>(p.v + base + off);
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) { kt[x][j] = (half_t)0.f; vt[x][j] = (half_t)0.f; }
-            }
-        }
-    };
+    // round r of the wave.  No branch stands around a request (hipcc would then wait for all that is in flight): a round past the wave's last one asks for
+    // that one again, a wave without keys for the segment's first, and rows past the segment's end for its last row
     auto load_round = [&](int r, half8_t (&kk)[U], half8_t (&vv)[U]) {
-        const int64_t base = block_base(p0 + (r * WAVES + wave) * TPI);
+        const int tb = R > 0 ? p0 + (min(r, R - 1) * WAVES + wave) * TPI : p0;
+        const int64_t base = block_base(tb);
 #pragma unroll
         for (int x = 0; x < U; ++x) {
-            const unsigned off = (unsigned)((x * RPI + tg) * row_elems + dc * 8);
+            const unsigned off = (unsigned)(min(x * RPI + tg, pend - 1 - tb) * row_elems + dc * 8);
             kk[x] = load_row16<true>(p.k + base + off); vv[x] = load_row16<true>(p.v + base + off);
         }
     };
-    // opens the segment that starts at unit u (u < ue); returns its length in units
-    auto open = [&](long long u) -> int {
-        int lo = 0, hi = nq;                                // the query of unit u: the last t with KVH * pre[t] <= u (queries without keys own no unit)
-        while (hi - lo > 1) { const int mid = (lo + hi) >> 1; if ((long long)p.KVH * pre[mid] <= u) lo = mid; else hi = mid; }
-        t = lo;
-        const int ut = pre[t + 1] - pre[t], rem = (int)(u - (long long)p.KVH * pre[t]);
-        g = rem / ut;
-        const int lu = rem - g * ut, seg = (int)min((long long)(ut - lu), ue - u);
-        // shares that touch this pair: unit x belongs to share floor(((x + 1) * nw - 1) / utot)
-        const long long S = (long long)p.KVH * pre[t] + (long long)g * ut, E = S + ut - 1;
-        const int wf = (int)(((S + 1) * nw - 1) / utot), wl = (int)(((E + 1) * nw - 1) / utot);
-        np = wl - wf + 1; slot = (int)blockIdx.x - wf;
+    // opens the next segment of the share, if there is one: the rest of a query's units, or as many as the share still holds
+    auto open = [&]() -> bool {
+        int lu = 0, seg = 0;
+        for (;;) {
+            if (u >= ue) return false;
+            int lo = 0, hi = nq;                            // the query of unit u: the last t with pre[t] <= u (queries without keys own no unit)
+            while (hi - lo > 1) { const int mid = (lo + hi) >> 1; if (pre[mid] <= u) lo = mid; else hi = mid; }
+            t = lo;
+            const int e = (int)min((long long)pre[t + 1], ue) - pre[t];
+            lu = max((int)(u - pre[t]) - CHARGE, 0); seg = e - CHARGE - lu;
+            u = pre[t] + e;
+            if (seg > 0) break;                             // (else the share ends inside the query's charge)
+        }
+        // shares that touch this query's keys: unit x belongs to share floor(((x + 1) * nw - 1) / utot)
+        const int wf = (int)(((pre[t] + CHARGE + 1ll) * nw - 1) / utot), wl = (int)(((long long)pre[t + 1] * nw - 1) / utot);
+        np = wl - wf + 1; slot = ws - wf;
         p0 = lu * CH; pend = min(cx[t], (lu + seg) * CH);
-        ng = (pend - p0 + RPI - 1) / RPI; R = (pend - p0) / CH; gt0 = R * (WAVES * U) + wave;
+        R = max(pend - p0 - wave * TPI + CH - 1, 0) / CH;   // rounds in which this wave has a key
         bt = p.block_tables + (int64_t)t * p.max_blocks;
         bt_chunk = (p0 >> p.bs_shift) >> 6;
-        { const int idx = (bt_chunk << 6) + lane; bt_reg = idx < p.max_blocks ? bt[idx] : 0; }
+        { const int idx = (bt_chunk << 6) + lane; bt_reg = idx < p.max_blocks ? bt[idx] : 0; asm volatile("" : "+v"(bt_reg)); }
         const half_t *qrow = p.q + (int64_t)t * p.ldq + (int64_t)g * G * D + dc * 8;
 #pragma unroll
         for (int i = 0; i < G; ++i) {
@@ -541,15 +545,13 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
 #pragma unroll
             for (int j = 0; j < 4; ++j) qv[i][j] = (half2_t){h[2 * j], h[2 * j + 1]};
         }
-        if (R >= 1) load_round(0, k0, v0);
-        if (R <= 1) issue_remainder();                      // (requested before the arithmetic of the last full round, as in attn_rows_kernel)
+        load_round(0, ka, va); load_round(1, kb, vb);
         asm volatile("" ::: "memory");                      // the requests stay HERE: hipcc would sink them to their first use, behind the tail of the segment in front
-        return seg;
+        return true;
     };
 
-    long long u = ub;
-    u += open(u);
-    for (;;) {
+    bool more = open();
+    while (more) {
         float m[G], l[G], acc[G][8];
 #pragma unroll
         for (int i = 0; i < G; ++i) {
@@ -557,12 +559,12 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
 #pragma unroll
             for (int j = 0; j < 8; ++j) acc[i][j] = 0.f;
         }
-        auto process = [&](auto check, const half8_t (&kk)[U], const half8_t (&vv)[U], int tok0) {
-            constexpr bool CHECK = decltype(check)::value;
+        auto process = [&](const half8_t (&kk)[U], const half8_t (&vv)[U], int r) {
+            const int left = pend - p0 - (r * WAVES + wave) * TPI;      // keys of the segment from the round's first one on
             float sc[U][G];
 #pragma unroll
             for (int x = 0; x < U; ++x) {
-                const bool valid = !CHECK || tok0 + x * (WAVES * RPI) + tg < pend;
+                const bool valid = x * RPI + tg < left;
 #pragma unroll
                 for (int i = 0; i < G; ++i) {
                     float d = 0.f;
@@ -578,7 +580,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
 #pragma unroll
                 for (int x = 1; x < U; ++x) mx = fmaxf(mx, sc[x][i]);
                 const float mn = fmaxf(m[i], mx);
-                const float ms = (CHECK && mn == -INFINITY) ? 0.f : mn;
+                const float ms = (mn == -INFINITY) ? 0.f : mn;
                 const float alpha = __expf(m[i] - ms);
                 m[i] = mn;
                 float ps = 0.f;
@@ -594,20 +596,22 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
                 l[i] = __fmaf_rn(l[i], alpha, ps);
             }
         };
-        if (R >= 1) process(std::false_type{}, k0, v0, 0);
-        for (int r = 1; r < R; ++r) {
-            half8_t kk[U], vv[U];
-            load_round(r, kk, vv);
-            if (r == R - 1) issue_remainder();
-            process(std::false_type{}, kk, vv, 0);
+        for (int r = 0; r < R; r += 2) {
+            process(ka, va, r);
+            if (r + 1 >= R) break;
+            load_round(r + 2, ka, va);
+            asm volatile("" ::: "memory");                  // the requests stay in front of the other round's arithmetic
+            __builtin_amdgcn_sched_barrier(0);
+            process(kb, vb, r + 1);
+            load_round(r + 3, kb, vb);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if (gt0 < ng) process(std::true_type{}, kt, vt, p0 + gt0 * RPI);
 
         // the segment is in the accumulators: what its tail needs of the state, then the NEXT segment is opened (its query, block table and first K/V rows
         // are on their way while this one is merged and handed over)
-        const int st = t, sg = g, snp = np, sslot = slot;
-        const bool more = u < ue;
-        if (more) u += open(u);
+        const int st = t, snp = np, sslot = slot;
+        more = open();
 
         // row-group slots of the wave -> the wave's sums; waves -> the segment's partial (attn_rows_kernel's arithmetic)
 #pragma unroll
@@ -624,7 +628,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
             }
         }
         __syncthreads();
-        const int64_t pair0 = ((int64_t)st * p.H + (int64_t)sg * G) * p.num_parts;
+        const int64_t pair0 = ((int64_t)st * p.H + (int64_t)g * G) * p.num_parts;
         const auto rs_o = __builtin_amdgcn_make_buffer_rsrc(p.part_o + pair0 * D, 0, (int)(G * p.num_parts * D * 4), 0x00020000);
         const auto rs_ml = __builtin_amdgcn_make_buffer_rsrc(p.part_ml + pair0 * 2, 0, (int)(G * p.num_parts * 2 * 4), 0x00020000);
         if (threadIdx.x < G * D) {
@@ -641,7 +645,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
                 L = mul_then_add(wgt, sm_ml[w2][i][1], L);
             }
             if (snp == 1) {
-                p.out[((int64_t)st * p.H + sg * G + i) * D + d] = (half_t)(L > 0.f ? o / L : 0.f);
+                p.out[((int64_t)st * p.H + g * G + i) * D + d] = (half_t)(L > 0.f ? o / L : 0.f);
             } else {
                 const int sl = i * p.num_parts + sslot;
                 __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o), rs_o, (sl * D + d) * 4, 0, 16);
@@ -653,7 +657,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
             constexpr int TPH = D / 4;
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                  // every storing wave drains its stores (and the next segment's first rows land) ...
             __syncthreads();
-            unsigned int *cnt = p.tickets + (int64_t)st * p.KVH + sg;
+            unsigned int *cnt = p.tickets + (int64_t)st * p.KVH + g;
             if (threadIdx.x == 0) ticket_s = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ... one ticket
             __syncthreads();
             if (ticket_s == (unsigned)(snp - 1)) {                            // the last of the pair's shares to finish merges it
@@ -663,12 +667,11 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
                     const half4_t hv = merge_partitions(snp,
                         [&](int pi) { return __builtin_bit_cast(float2_t, __builtin_amdgcn_raw_buffer_load_b64(rs_ml, (i * p.num_parts + pi) * 8, 0, 16)); },
                         [&](int pi) { return __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(rs_o, ((i * p.num_parts + pi) * D + d) * 4, 0, 16)); });
-                    *reinterpret_cast<half4_t *>(p.out + ((int64_t)st * p.H + sg * G + i) * D + d) = hv;
+                    *reinterpret_cast<half4_t *>(p.out + ((int64_t)st * p.H + g * G + i) * D + d) = hv;
                 }
                 if (threadIdx.x == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // re-arm for the next launch
             }
         }
-        if (!more) break;
         __syncthreads();                                                      // sm_acc / sm_ml / ticket_s are the next segment's too
     }
 }
@@ -819,15 +822,14 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
         const int64_t cus = share_workgroups(), rounds = (pairs + cus - 1) / cus, units = (mc + 63) / 64;
         const int64_t cap = a.workspace_bytes ? (int64_t)(a.workspace_bytes / ((size_t)a.nq * a.H * (D + 2) * sizeof(float))) : units;
         const bool by_count = pairs > cus && rounds * cus * 100 >= pairs * 115 && mc >= 256;
-        // shares: one per CU for the pair-count case (uniform contexts: a second segment per share buys nothing); for ragged batches the caller's count — two per CU
-        // (co-resident: twice the rows in flight, and the dispatcher evens out what the static cut leaves), three from 2 pairs per CU on, fewer while a share would
-        // hold less than four 64-key units (measured: profiles/r06_priced_levers.txt 14.)
-        const int64_t nw = a.balance_hint > 0 ? a.balance_hint : share_mode() == 2 ? cus * (pairs <= 2 * cus ? 2 : 3) : cus;
+        // workgroups: one per CU, or the caller's count for ragged batches (fewer, where a share would hold less than four 64-key units)
+        const int64_t nw = a.balance_hint > 0 ? a.balance_hint : cus;
         if ((by_count || a.balance_hint || share_mode() == 2) && pairs < 2048 && cap >= units) {
             p.part_size = 64; p.num_parts = (int32_t)cap;
             p.part_o = (float *)a.workspace; p.part_ml = p.part_o + (int64_t)a.nq * a.H * cap * D;
             p.part0 = 0; p.kv0 = 0; p.kv0_rows = nullptr; p.tickets = a.tickets;
-            attn_share_kernel<D, G, DU / 2, 8><<<dim3((unsigned)nw), dim3(512), 0, s>>>(p, (int)a.nq, (int)nw);
+            const int shares = (int)std::max<int64_t>(1, nw / a.KVH);
+            attn_share_kernel<D, G, DU / 2, 8><<<dim3((unsigned)(shares * a.KVH)), dim3(512), 0, s>>>(p, (int)a.nq, shares);
             hipError_t e = hipGetLastError();
             if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "attention (work-balanced) launch failed: %s", hipGetErrorString(e));
             return 0;

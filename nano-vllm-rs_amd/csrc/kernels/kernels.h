@@ -47,7 +47,7 @@ struct AttnArgs {
     // own partition per pair, that partition's workgroup merges the pair (it is the last arriver by stream order; no counter is touched)
     unsigned int *tickets;
     // paged decode with `tickets`: > 0 = the caller knows the contexts are RAGGED (their sum is well below nq * max_ctx) and asks for the work-balanced form
-    // (attn_share_kernel) with this many equal shares of all pairs' keys, wherever it can run — not only where the pair count asks for it
+    // (attn_share_kernel) with this many workgroups over equal shares of all keys, wherever it can run — not only where the pair count asks for it
     int32_t balance_hint;
 };
 

@@ -749,9 +749,9 @@ static inline uint64_t graph_key(bool want_logits, size_t nseq, int64_t bucket, 
 bool nvr_model_runner::ragged_batch(size_t nseq, int64_t sum_ctx, int64_t max_ctx) {
     if (f32 || nseq == 0 || decode_shared_len > 0) return false;
     const int64_t pairs = (int64_t)nseq * KVH, units = sum_ctx * KVH / 64, cus = num_cus;
-    // shares: two per CU (three from 2 pairs per CU on), but none of less than four units (a tensor-parallel rank with one kv head: 32 sequences of 256..8192
+    // workgroups: one per CU, but none with a share of less than four units (a tensor-parallel rank with one kv head: 32 sequences of 256..8192
     // keys are 1176 units — 512 shares of 2.3 units lost 2-5 % to the per-pair launch)
-    decode_shares = (int32_t)std::max<int64_t>(64, std::min<int64_t>(cus * (pairs <= 2 * cus ? 2 : 3), units / 4));
+    decode_shares = (int32_t)std::max<int64_t>(64, std::min<int64_t>(cus, units / 4));
     // ... and not below six units per CU in all: the step is then launch-bound and the per-pair launch's shorter ramp wins (12 sequences of 20..1500 keys: 1.08
     // against 1.24 ms per step; 8 of 64..8192 keys — 2040 units — 1.65 -> 1.33 the other way)
     return pairs <= 1024 && max_ctx * (int64_t)nseq * 100 >= sum_ctx * 130 && units >= 6 * cus;

@@ -293,3 +293,36 @@ def test_decode_steps_of_one_and_two_rows_against_more(dtype, hidden, inter, hea
     for which in ([0], [1], [2], [0, 1], [1, 2]):
         got = steps(which)
         assert np.abs(got - full[which]).max() < tol, which
+
+
+@pytest.mark.parametrize("B,G,KVH,D,bs,ctx", [
+    (40, 2, 8, 128, 256, [1 + (577 * i) % 1900 for i in range(40)]),                       # ragged: many queries to a share, long ones cut
+    (300, 1, 1, 64, 8, [1, 63, 64, 65, 300] * 60),                                         # one kv head, the smallest block, shares of one or two units
+    (130, 8, 2, 64, 16, [1 + 2 * i for i in range(130)]),                                  # the widest group
+    (90, 4, 3, 128, 64, [0 if i % 7 == 3 else 1 + (311 * i) % 700 for i in range(90)]),    # 3 kv heads do not divide the CUs; queries without keys
+    (33, 2, 8, 128, 16, [5000] + [1] * 32),                                                # one long query: shares that end inside the charge of a short one
+])
+def test_work_balanced_attention_against_the_per_pair_form(B, G, KVH, D, bs, ctx):
+    """Equal shares of all queries' keys (each query charged two units for its start) against a workgroup per pair, over the same cache: both keep f32 scores,
+    weights and sums and round once, so their outputs differ by one rounding of the result and the order of f32 sums of up to 5000 terms — 2 ulps of float16."""
+    l = nvr.lib()
+    rng = np.random.default_rng(B + D)
+    H, blocks = G * KVH, [(c + bs - 1) // bs for c in ctx]
+    mb, perm, o = max(blocks) + 1, rng.permutation(sum(blocks)), 0
+    bt = np.full((B, mb), -1, np.int32)
+    for b, n in enumerate(blocks):
+        bt[b, :n] = perm[o:o + n]; o += n
+    k, v = (dev(rng.standard_normal((sum(blocks), bs, KVH, D)).astype(F16).view(np.uint16)) for _ in range(2))
+    q = dev(rng.standard_normal((B, H, D)).astype(F16).view(np.uint16))
+    d_ctx, d_bt, tickets = dev(np.asarray(ctx, np.int32)), dev(bt), dev(np.zeros(B * KVH, np.uint32))
+    meta = nvr.AttnMetaC()
+    meta.context_lens, meta.block_tables, meta.max_blocks, meta.batch, meta.max_context_len = d_ctx.ptr, d_bt.ptr, mb, B, max(ctx)
+    ws = nvr.DeviceBuffer(l.nvr_paged_attn_workspace_bytes(B, H, D, max(ctx)))
+    ref, got = nvr.DeviceBuffer(B * H * D * 2), nvr.DeviceBuffer(B * H * D * 2)
+    nvr.check(l.nvr_fill_const(got.ptr, B * H * D, C.c_float(float("nan")), None))
+    args = (q.ptr, H * D, k.ptr, v.ptr, C.byref(meta), H, KVH, D, bs, D ** -0.5)
+    nvr.check(l.nvr_paged_attn_decode(*args, ref.ptr, ws.ptr, None))
+    nvr.check(l.nvr_paged_attn_decode_fused(*args, got.ptr, ws.ptr, tickets.ptr, None))
+    a, b = ref.to_numpy((B, H, D), F16).astype(np.float32), got.to_numpy((B, H, D), F16).astype(np.float32)
+    assert np.all(np.abs(a - b) <= 2 * np.maximum(np.spacing(np.abs(a).astype(F16)).astype(np.float32), 2.0 ** -14 / 8)), np.abs(a - b).max()
+    assert not tickets.to_numpy((B * KVH,), np.uint32).any()
