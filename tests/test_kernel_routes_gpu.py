@@ -326,3 +326,20 @@ def test_work_balanced_attention_against_the_per_pair_form(B, G, KVH, D, bs, ctx
     a, b = ref.to_numpy((B, H, D), F16).astype(np.float32), got.to_numpy((B, H, D), F16).astype(np.float32)
     assert np.all(np.abs(a - b) <= 2 * np.maximum(np.spacing(np.abs(a).astype(F16)).astype(np.float32), 2.0 ** -14 / 8)), np.abs(a - b).max()
     assert not tickets.to_numpy((B * KVH,), np.uint32).any()
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("heads,vdim,ff,batch", [(1, 30, 48, 1), (3, 32, 48, 16), (5, 4, 64, 17), (2, 64, 2064, 32), (4, 96, 40, 33)])
+def test_layer_list_gated_head_norm_and_clamped_unit(dtype, heads, vdim, ff, batch):
+    """A retention layer's gated head norm by a wave per head (head widths that are multiples of 4, head counts that leave waves without a head) and by the general form, and the clamped unit in
+    its product's epilogue (up to 32 rows: one and two blocks of 16, few and many column tiles) or behind it, against the float64 restatement; bounds as in the test of the decode steps above."""
+    import rugudra_util as u
+    cfg = u.make_config([u.retention_layer(heads, 32, vdim, ff=ff), u.attention_layer(2, 1, 64, 64, ff=ff)], width=64, taps=4)
+    w = u.make_weights(cfg, seed=heads + vdim)
+    d = u.Driver(cfg, w, dtype=dtype, slots=batch, pages=batch * 2, max_tokens=max(64, 9 * batch), max_len=64)
+    rng = np.random.default_rng(ff)
+    tokens = [rng.integers(0, 97, 8 + i % 3) for i in range(batch)]
+    d.step([("s%d" % i, t[:-2]) for i, t in enumerate(tokens)])
+    got = [d.step([("s%d" % i, t[len(t) - 2 + k:len(t) - 1 + k]) for i, t in enumerate(tokens)]) for k in range(2)]
+    err = [u.row_errors(np.concatenate([g["s%d" % i] for g in got]), u.expected_logits(cfg, w, tokens[i])[-2:]) for i in range(0, batch, 5)]
+    assert np.median(err) < u.TOL[dtype] / 2 and np.max(err) < (0.5 if dtype == "bfloat16" else 1e-2)
