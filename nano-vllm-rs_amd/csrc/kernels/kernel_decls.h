@@ -79,6 +79,9 @@ int linear_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t
 int linear_gelu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *y, bool *applied, hipStream_t s);
 // gate / up products with gelu (tanh form) in silu's place
 int linear_gelu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s);
+// gate_up with the clamped gated unit of a layer list in the epilogue, rows of out ldo apart (few rows)
+bool linear_clamped_glu_ok(const half_bits *x, int64_t ldx, int64_t T, int64_t K, int64_t I, const half_bits *out, int64_t ldo);
+int linear_clamped_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, float limit, float alpha, half_bits *out, int64_t ldo, hipStream_t s);
 int linear_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H,
                           int64_t KVH, int64_t D, const int64_t *positions, const int32_t *slots, const float *cos_t,
                           const float *sin_t, half_bits *qkv, half_bits *k_cache, half_bits *v_cache, hipStream_t s,

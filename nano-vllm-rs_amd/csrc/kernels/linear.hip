@@ -44,7 +44,8 @@ struct LinEpi {
     int32_t kslice; int64_t slab_stride;
     // W is the TILED copy [N/16][K/32][16][32] (retile_weight): one wave-instruction reads 1 KiB contiguous
     int32_t tiled;
-    int32_t gelu;                          // EPI_SILU: gelu (tanh form) instead of silu; EPI_F16: gelu (error function) of the product
+    int32_t gelu;                          // EPI_SILU: 1 gelu (tanh form) instead of silu, 2 the clamped unit below; EPI_F16: gelu (error function) of the product
+    float limit, alpha; int64_t ldy;       // EPI_SILU with gelu == 2: min(g, limit) sigmoid(alpha min(g, limit)) (clamp(u, +-limit) + 1); row stride of y (0: I)
     NormIn norm;                           // NORM instances: x is formed by the workgroup itself
 };
 
@@ -250,10 +251,15 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float gf = (float)to_half_rn(g4[e]), uf = (float)to_half_rn(u4[e]);
-                    const float sg = gate_factor(gf, epi.gelu);
-                    h[e] = to_half_rn(__fmul_rn(__fmul_rn(gf, sg), uf));
+                    if (epi.gelu == 2) {
+                        const float g = fminf(gf, epi.limit), u = fminf(fmaxf(uf, -epi.limit), epi.limit);
+                        h[e] = to_half_rn(g / (1.0f + expf(-epi.alpha * g)) * (u + 1.0f));
+                    } else {
+                        const float sg = gate_factor(gf, epi.gelu);
+                        h[e] = to_half_rn(__fmul_rn(__fmul_rn(gf, sg), uf));
+                    }
                 }
-                *reinterpret_cast<half4_t *>(reinterpret_cast<half_t *>(y) + (int64_t)m * N + n) = h;
+                *reinterpret_cast<half4_t *>(reinterpret_cast<half_t *>(y) + (int64_t)m * (epi.ldy ? epi.ldy : N) + n) = h;
             }
         }
     } else {   // EPI_ROPE: NT == 1
@@ -463,6 +469,30 @@ int linear_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t
 // the same with gelu (tanh form) in silu's place
 int linear_gelu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s) {
     return linear_glu(x, ldx, W, T, K, I, out, s, nullptr, true);
+}
+
+// gate_up GEMM + the clamped gated unit of a layer list: W [2I, K] (gate rows, then up rows), out [T, ldo].  Few rows, whose product the weight-row kernel takes: the unit
+// is a launch of its own otherwise, and a launch behind a launch is about 5 us whatever it holds (16 rows of 1024, I = 3072: 11.3 -> 6.3 us together).  More rows run the tiles' kernels, which
+// store each product once and whose 16384-row unit is a copy at the memory's rate.
+bool linear_clamped_glu_ok(const half_bits *x, int64_t ldx, int64_t T, int64_t K, int64_t I, const half_bits *out, int64_t ldo) {
+    return T <= 32 && K % 32 == 0 && I % 16 == 0 && ldx % 8 == 0 && ldo % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)out % 8 == 0 && !linear_stream_silu_ok(T, K, I, ldx);
+}
+int linear_clamped_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, float limit, float alpha, half_bits *out, int64_t ldo, hipStream_t s) {
+    if (!linear_clamped_glu_ok(x, ldx, T, K, I, out, ldo)) return nvr::fail(NVR_ERR_UNSUPPORTED, "linear_clamped_glu: T=%ld K=%ld I=%ld", (long)T, (long)K, (long)I);
+    if (T == 0) return 0;
+    LinEpi e{};
+    e.gelu = 2; e.limit = limit; e.alpha = alpha; e.ldy = ldo;
+    const unsigned gx = (unsigned)(I / 16);
+    const half_t *xx = (const half_t *)x, *ww = (const half_t *)W;
+    const int wv = waves_for(K);
+    if (T <= 16 || I / 16 < 128) {
+        if (wv >= 8) launch<2, 1, 8, EPI_SILU>(xx, ldx, ww, (int)T, (int)K, (int)I, out, e, gx, s);
+        else launch<2, 1, 4, EPI_SILU>(xx, ldx, ww, (int)T, (int)K, (int)I, out, e, gx, s);
+    } else {
+        if (wv >= 8) launch<2, 2, 8, EPI_SILU>(xx, ldx, ww, (int)T, (int)K, (int)I, out, e, gx, s);
+        else launch<2, 2, 4, EPI_SILU>(xx, ldx, ww, (int)T, (int)K, (int)I, out, e, gx, s);
+    }
+    return launch_check("linear_clamped_glu");
 }
 
 // qkv GEMM + RoPE on q,k heads + store of k,v rows into the paged caches

@@ -325,8 +325,12 @@ int LayeredModel::forward_joint(nvr_model_runner &r, const StepPlan &p) {
                 RC(kl::grouped_linear(d, bf16, s));
             }
             if (fs) {
-                RC(gemm(r, a2, W, w.sgu, T, W, 2 * fs, gu));
-                RC(kl::clamped_glu(gu, T, fs, (float)L.shared_limit, 1.702f, act, fs, bf16, s));
+                if (bf16 && nvr::kb::linear_clamped_glu_ok((const uint16_t *)a2, W, T, W, fs, (uint16_t *)act, fs))
+                    RC(nvr::kb::linear_clamped_glu((const uint16_t *)a2, W, (const uint16_t *)w.sgu, T, W, fs, (float)L.shared_limit, 1.702f, (uint16_t *)act, fs, s));
+                else {
+                    RC(gemm(r, a2, W, w.sgu, T, W, 2 * fs, gu));
+                    RC(kl::clamped_glu(gu, T, fs, (float)L.shared_limit, 1.702f, act, fs, bf16, s));
+                }
                 RC(gemm(r, act, fs, w.sdown, T, fs, W, shared_y));
             }
             RC(kl::moe_combine(e_y, place_of, T, L.top, fs ? shared_y : nullptr, W, a2, bf16, s, moe_score, fs ? shared_g : nullptr, 1));

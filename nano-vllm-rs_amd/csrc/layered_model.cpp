@@ -509,8 +509,13 @@ int LayeredModel::forward(nvr_model_runner &r, const StepPlan &p) {
             RC(kl::head_norm_gate(ret_o, proj, w.nmix, w.gcol, T, L.heads, L.vdim, eps, nullptr, cat, w.kcat, bf16, s));
         }
         if (L.has_mlp) {
-            RC(gemm(r, a2, W, w.gu, T, W, 2 * L.ff, gu));
-            RC(kl::clamped_glu(gu, T, L.ff, (float)L.limit, 1.702f, (char *)cat + (size_t)(w.mixcols * esz), w.kcat, bf16, s));
+            uint16_t *const glu = (uint16_t *)((char *)cat + (size_t)(w.mixcols * esz));
+            if (bf16 && nvr::kb::linear_clamped_glu_ok((const uint16_t *)a2, W, T, W, L.ff, glu, w.kcat))
+                RC(nvr::kb::linear_clamped_glu((const uint16_t *)a2, W, (const uint16_t *)w.gu, T, W, L.ff, (float)L.limit, 1.702f, glu, w.kcat, s));
+            else {
+                RC(gemm(r, a2, W, w.gu, T, W, 2 * L.ff, gu));
+                RC(kl::clamped_glu(gu, T, L.ff, (float)L.limit, 1.702f, glu, w.kcat, bf16, s));
+            }
         }
         // decode steps: the product over mixer and feed-forward together is long and narrow (5120 x 1024 at the smallest size: 64 workgroups, 15.0 us; in 4 parts 5.9): cut along k, joined by the next
         // launch that reads the stream
