@@ -8,9 +8,10 @@
 // decode attention: one workgroup per CU slot keeps the T x K activation block in LDS (XOR-swizzled 16-byte
 // chunks: ds_read_b128 of 16 rows at one k offset is conflict-free) for its whole life; each WAVE owns whole
 // 16-row weight tiles (tile j -> wave j % all_waves: neighbouring waves stream neighbouring 16·K·2-byte regions) and
-// runs the full k loop alone: U row-chunk loads of 1 KiB in flight per wave (A operand straight from HBM to VGPRs,
-// non-temporal), B operand from LDS, one v_mfma_f32_16x16x32_f16 per 16 tokens and k-step, no cross-wave
-// reduction and no barrier inside the stream.
+// runs the full k loop alone: two sets of U row-chunk loads of 1 KiB in flight per wave, the stream running on across the
+// tiles' ends (A operand straight from HBM to VGPRs, non-temporal), B operand from LDS, one v_mfma_f32_16x16x32_f16 per 16
+// tokens and k-step, no cross-wave reduction and no barrier inside the stream.  151 936 x 1024 weights: one set at a time
+// 62 us for up to 16 rows (5.0 TB/s), two 52 us (6.0); 17..32 rows 62 us either way.
 // Greedy arg-max: every lane keeps (best value, lowest index) of the logits it produced for its token; lanes, waves and
 // finally workgroups are merged with "greater value, else lower index", the workgroup results go to a small
 // partials array and argmax_partials finishes the job, instead of re-reading all 4·T·N logit bytes.
@@ -33,31 +34,47 @@ __global__ __launch_bounds__(WAVES * 64) void lm_head_kernel(const half_t *__res
                                                              int32_t *__restrict__ pidx, int flags) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int ROWS = MT * 16;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 15, q = lane >> 4;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, q = lane >> 4;
     const int cpr = K / 8;                                       // 16-byte chunks per activation row
+    const int ntiles = N / 16, nw = gridDim.x * WAVES, tile0 = blockIdx.x * WAVES + wave;
+    // flags bit 1: W is the tiled copy [N/16][K/32][16][32] (retile_weight): 1 KiB contiguous per wave-instruction
+    const bool tiled = flags & 2;
+    const int64_t tile_step = tiled ? (int64_t)(K / 32) * 512 : (int64_t)16 * K;
+    const half_t *wl = W + (tiled ? r * 32 + q * 8 : (int64_t)r * K + q * 8);
+    const int kmul = tiled ? 16 : 1;
+    // the wave's weights are one stream of U-piece sets over all its tiles, two sets requested ahead at any time, across the tiles' ends and in front of the activations
+    // (behind its last set the wave asks for that one again: no branch around a request)
+    const int last = tile0 < ntiles ? tile0 + (ntiles - 1 - tile0) / nw * nw : ntiles - 1;
+    int lt = min(tile0, last), lk = 0;
+    half8_t wa[U], wb[U];
+    auto request = [&](half8_t (&a)[U]) {
+        const half_t *wr = wl + lt * tile_step;
+#pragma unroll
+        for (int u = 0; u < U; ++u) a[u] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(wr + (int64_t)(lk + u * 32) * kmul));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        const bool end = lk + 32 * U >= K, more = lt + nw <= last;
+        if (!end) lk += 32 * U;
+        else if (more) { lk = 0; lt += nw; }
+    };
+    request(wa);
+    request(wb);
     fill_x_image<ROWS, WAVES * 64, 8>(smem, x, ldx, 0, cpr, T, tid);
     __syncthreads();
+    __builtin_amdgcn_s_waitcnt(0x0f70);                          // vmcnt(0), here and known to hipcc: it would find the activations' (guarded) loads pending in every turn of the loop below
 
-    const int ntiles = N / 16, nw = gridDim.x * WAVES;
     float best[MT]; int besti[MT];
 #pragma unroll
     for (int j = 0; j < MT; ++j) { best[j] = -INFINITY; besti[j] = 0x7fffffff; }
-
-    for (int tile = blockIdx.x * WAVES + wave; tile < ntiles; tile += nw) {
-        // flags bit 1: W is the tiled copy [N/16][K/32][16][32] (retile_weight): 1 KiB contiguous per wave-instruction
-        const bool tiled = flags & 2;
-        const half_t *wr = tiled ? W + (int64_t)tile * (K / 32) * 512 + r * 32 + q * 8 : W + ((int64_t)tile * 16 + r) * K + q * 8;
-        const int kmul = tiled ? 16 : 1;
-        float4_t acc[MT];
+    // one loop over the whole stream, tile ends included: at the head of a loop of its own per tile hipcc would wait for all that is in flight
+    float4_t acc[MT];
 #pragma unroll
-        for (int j = 0; j < MT; ++j) acc[j] = (float4_t){0.f, 0.f, 0.f, 0.f};
-        for (int k0 = 0; k0 < K; k0 += 32 * U) {
-            half8_t a[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) a[u] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(wr + (int64_t)(k0 + u * 32) * kmul));
+    for (int j = 0; j < MT; ++j) acc[j] = (float4_t){0.f, 0.f, 0.f, 0.f};
+    for (int tile = tile0, k0 = 0; tile < ntiles;) {
+        auto use = [&](const half8_t (&a)[U], int k) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int ch = (k0 >> 3) + u * 4 + q;
+                const int ch = (k >> 3) + u * 4 + q;
 #pragma unroll
                 for (int j = 0; j < MT; ++j) {
                     const int row = j * 16 + r;
@@ -65,7 +82,14 @@ __global__ __launch_bounds__(WAVES * 64) void lm_head_kernel(const half_t *__res
                     acc[j] = mfma16(a[u], b, acc[j]);
                 }
             }
-        }
+        };
+        use(wa, k0);
+        request(wa);
+        use(wb, k0 + 32 * U);
+        request(wb);
+        k0 += 64 * U;                                             // (64 * U divides K: lm_head_ok)
+        if (k0 < K) continue;
+        k0 = 0;
         // C layout: rows n = q*4 + e (4 consecutive vocabulary entries), column = token r
         const int n0 = tile * 16 + q * 4;
 #pragma unroll
@@ -75,7 +99,9 @@ __global__ __launch_bounds__(WAVES * 64) void lm_head_kernel(const half_t *__res
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 if (acc[j][e] > best[j]) { best[j] = acc[j][e]; besti[j] = n0 + e; }     // tiles ascend: first maximum kept
+            acc[j] = (float4_t){0.f, 0.f, 0.f, 0.f};
         }
+        tile += nw;
     }
 
     // lanes r, r+16, r+32, r+48 hold the same token; then the waves through LDS (the activation image is dead)
