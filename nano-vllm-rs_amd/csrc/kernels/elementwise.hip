@@ -457,7 +457,7 @@ __global__ __launch_bounds__(256) void rope_store_kernel(half_t *__restrict__ qk
     }
 }
 // The same with an RMSNorm over head_dim on every q and k head in front of the rotation (real Qwen3 checkpoints:
-// self_attn.q_norm / k_norm; an extension of the reference graph): n = fp16((x / rms) * w) with the arithmetic of
+// self_attn.q_norm / k_norm; an extension of the reference graph, DESIGN A-27): n = fp16((x / rms) * w) with the arithmetic of
 // rmsnorm_kernel (RMSNorm::forward_simple, layernorm.rs:58-75), then RoPE on n.  A head belongs to LPH = D / 16 neighbouring lanes, each with 8
 // elements of either half in 16-byte pieces (the pairs it rotates), and one workgroup walks a token's heads and value rows together, so that every load
 // of the row is in flight at once.  Bound by the latency of one trip to memory at few rows, by the bytes of the rows at many: against a wave per head and

@@ -569,8 +569,7 @@ int flash_prefill(const FlashArgs &a, bool paged, hipStream_t s) {
     // at most one workgroup per CU and more than five steps: two groups of waves share a tile's steps (with more workgroups the second one of a CU fills the SIMDs as the second group
     // would; over fewer steps the meeting costs what it saves).  Qwen3-0.6B prompt steps, us with one / two groups: 64 tokens 1320 / 1353, 4 x 200..300 2843 / 2849, 509 2027 / 1998,
     // 1024 3285 / 3172, 1900 4331 / 4145, 510 behind 1530 cached 2923 / 2727, 800 behind 7200 cached 6765 / 5959
-    // (by the whole step's tiles: a step in parts has the bits of the step in one)
-    const bool few = (int64_t)std::max(a.step_tiles, a.ntiles) * a.KVH <= 256 && a.max_keys > 5 * NVR_FLASH_KT;
+    const bool few = grid.x <= 256 && a.max_keys > 5 * NVR_FLASH_KT;
 #define NVR_FLASH(DD, GG)                                                                             \
     if (a.D == DD && G == GG) {                                                                       \
         if (diff && ub) flash_prefill_kernel<DD, GG, true, true, false, false, false, true><<<grid, block, 0, s>>>(p);   \
@@ -581,7 +580,6 @@ int flash_prefill(const FlashArgs &a, bool paged, hipStream_t s) {
         else if (pen) flash_prefill_kernel<DD, GG, true, false, false, true><<<grid, block, 0, s>>>(p);   \
         else if (few && ub) flash_prefill_kernel<DD, GG, true, true, false, false, false, false, 2><<<grid, dim3(128 * FLASH_WAVES), 0, s>>>(p);    \
         else if (few && !paged) flash_prefill_kernel<DD, GG, false, false, false, false, false, false, 2><<<grid, dim3(128 * FLASH_WAVES), 0, s>>>(p);  \
-        else if (few && paged) flash_prefill_kernel<DD, GG, true, false, false, false, false, false, 2><<<grid, dim3(128 * FLASH_WAVES), 0, s>>>(p);  \
         else if (ub) flash_prefill_kernel<DD, GG, true, true><<<grid, block, 0, s>>>(p);              \
         else if (paged) flash_prefill_kernel<DD, GG, true><<<grid, block, 0, s>>>(p);                 \
         else flash_prefill_kernel<DD, GG, false><<<grid, block, 0, s>>>(p);                           \

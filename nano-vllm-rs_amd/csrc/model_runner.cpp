@@ -768,7 +768,7 @@ bool nvr_model_runner::ragged_batch(size_t nseq, int64_t sum_ctx, int64_t max_ct
 // Every op is a row-wise kernel, a 256-row-tile GEMM (each part is big enough to take the same kernel as the whole step) or attention
 // over whole sequences, so the bits are those of the serial form.  Host order keeps one segment queued ahead of every reduce (a backend
 // that blocks the host inside the reduce still finds work queued).
-int nvr_model_runner::forward_prefill_two(int64_t T, int64_t B, int64_t max_ctx) {
+int nvr_model_runner::forward_prefill_two(int64_t T, int64_t B) {
     hipStream_t st = stream;
     const int64_t r0s[2] = {0, mb_rows}, nrs[2] = {mb_rows, T - mb_rows};
     const int64_t t0s[2] = {0, mb_tiles}, nts[2] = {mb_tiles, n_tiles - mb_tiles};
@@ -786,7 +786,7 @@ int nvr_model_runner::forward_prefill_two(int64_t T, int64_t B, int64_t max_ctx)
             f.k = k_cache(l); f.v = v_cache(l); f.block_tables = dd_bt; f.max_blocks = (int32_t)max_blocks_per_seq; f.block_size = (int32_t)block_size;
         } else if (prefill_kv_cache) { f.k = k_cache(l); f.v = v_cache(l); f.ldkv = KVH * D; }
         else { f.k = qkv + H * D; f.v = qkv + (H + KVH) * D; f.ldkv = QKV; }
-        f.tiles = (const k::FlashTile *)(in_dev + off_tiles) + t0s[m]; f.ntiles = (int32_t)nts[m]; f.max_keys = (int32_t)max_ctx; f.step_tiles = (int32_t)n_tiles;
+        f.tiles = (const k::FlashTile *)(in_dev + off_tiles) + t0s[m]; f.ntiles = (int32_t)nts[m];
         f.H = (int32_t)H; f.KVH = (int32_t)KVH; f.D = (int32_t)D; f.scale = scale; f.out = attn;
         RC(KD(flash_prefill(f, prefill_paged, st)));
         return mb_route[1] == 0 ? KD(gemm256(attn + r0 * H * D, H * D, w.o, nr, H * D, Hd, proj + r0 * Hd, st))
@@ -876,7 +876,7 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
     const int32_t *slots = is_prefill ? d_slots : dd_slots, *ctx = is_prefill ? d_ctx : dd_ctx;
     const int32_t *bt = dd_bt;
     if (f32) return forward_f32(T, B, is_prefill, max_ctx);
-    if (is_prefill && tp_overlap == 2 && mb_rows > 0) return forward_prefill_two(T, B, max_ctx);
+    if (is_prefill && tp_overlap == 2 && mb_rows > 0) return forward_prefill_two(T, B);
     const bool tl = tiled_weights && T <= 64;                            // decode-sized steps stream the tiled weight copies
     const bool embed_norm = L > 0 && KD(embedding_rmsnorm_ok(T, Hd));                    // decode-sized: K1 + the first norm in one launch
     if (embed_norm) RC(KD(embedding_rmsnorm(ids, T, embed, layers[0].ln1, mc.rms_norm_eps, Hd, h, n, st)));

@@ -359,7 +359,7 @@ def test_prompt_attention_by_two_groups_of_waves(paged, G, KVH, D, cases):
     rng = np.random.default_rng(G * D + len(cases))
     if not paged:
         cases = [(n, n) for _, n in cases]
-    H, bs, l = G * KVH, 48 if G == 1 else 64, nvr.lib()                   # (48: steps that cross block ends)
+    H, bs, l = G * KVH, 64, nvr.lib()
     blocks = [(c + bs - 1) // bs for c, _ in cases]
     T, mb = sum(n for _, n in cases), max(blocks) + 1
     cu = np.concatenate([[0], np.cumsum([n for _, n in cases])]).astype(np.int32)
