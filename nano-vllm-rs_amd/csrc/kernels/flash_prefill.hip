@@ -130,20 +130,16 @@ constexpr int FLASH_WAVES = NVR_FLASH_WAVES;     // waves per workgroup: 32 quer
 // DIFF: differential attention.  A wave's two query tiles are the two maps of ONE head at the same 16 positions: map t multiplies its half of the K fragments, both use
 // every V fragment, and the difference, its norm and the gate are formed from the accumulators (the maps' outputs of a query sit in the same lanes).
 // A window with kept first keys (PEN, DIFF): the steps over the kept keys come first, then those from the window's first key on.
-// KS (plain form): KS groups of FLASH_WAVES waves hold the same queries and take the steps in turn (step it * KS + group), each with a ring of its own; the groups' maxima, sums and outputs
-// meet in LDS behind the last step.  A launch of few tiles leaves CUs idle and lasts as long as its longest chain of steps, one wave per SIMD: that chain is KS times shorter.
-template <int D, int G, bool PAGED, bool UB = false, bool SHARED = false, bool PEN = false, bool GATE = false, bool DIFF = false, int KS = 1>
-__global__ __launch_bounds__(64 * FLASH_WAVES * KS, 8 / FLASH_WAVES / KS) void flash_prefill_kernel(FlashParams p) {   // 2 waves per SIMD: <= 256 registers per lane
-    constexpr int NT = 64 * FLASH_WAVES;         // threads of a group
-    static_assert(KS == 1 || (NVR_FLASH_NBUF == 2 && !SHARED && !PEN && !GATE && !DIFF), "groups: the plain form, which waits for all of a ring");
-    const int grp = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT), tid = KS == 1 ? (int)threadIdx.x : (int)threadIdx.x % NT;
+template <int D, int G, bool PAGED, bool UB = false, bool SHARED = false, bool PEN = false, bool GATE = false, bool DIFF = false>
+__global__ __launch_bounds__(64 * FLASH_WAVES, 8 / FLASH_WAVES) void flash_prefill_kernel(FlashParams p) {   // 2 waves per SIMD: <= 256 registers per lane
+    constexpr int NT = 64 * FLASH_WAVES;         // threads
     constexpr int KT = NVR_FLASH_KT;             // keys per step
     constexpr int NBUF = NVR_FLASH_NBUF;         // K/V tiles in the LDS ring: NBUF-1 in flight ahead of the one in use
     constexpr int CPR = D / 8;                   // 16-byte chunks per K/V row
     constexpr int PIECES = KT * CPR / NT;        // 16-byte pieces per thread and operand
     constexpr int NKS = D / 32, NDT = D / 16, NQT = 2, NMT = KT / 16, NK2 = KT / 32;
     constexpr int STAGE = 2 * KT * D * 2;        // bytes of one ring slot [K | V]
-    __shared__ __attribute__((aligned(16))) char smem[KS * NBUF * STAGE];
+    __shared__ __attribute__((aligned(16))) char smem[NBUF * STAGE];
 
     const int g = blockIdx.x % p.KVH;
     FlashTile tile;
@@ -154,7 +150,7 @@ __global__ __launch_bounds__(64 * FLASH_WAVES * KS, 8 / FLASH_WAVES / KS) void f
         if (tile.nq <= 0) return;                                     // (workgroup-uniform: the launch is sized for the whole batch)
         tile.pos0 = 0x3fffffff; tile.kv_ref = p.srows ? p.srows[0] : 0;
     } else tile = p.tiles[blockIdx.x / p.KVH];
-    const int wave = tid >> 6, lane = tid & 63;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = lane & 15, g4 = lane >> 4;
     // SHARED: blockIdx.y cuts the shared keys into partitions of shared_len tokens (more workgroups than 8 per kv head at 512 sequences)
     // (a window: the first step is the one that holds the first key the tile's first query sees)
@@ -162,7 +158,7 @@ __global__ __launch_bounds__(64 * FLASH_WAVES * KS, 8 / FLASH_WAVES / KS) void f
                                                                     (GATE && p.chunk > 0) ? tile.pos0 / p.chunk * p.chunk / KT * KT : 0);
     const int kv_end = SHARED ? kv_start + p.shared_len : tile.pos0 + tile.nq;
     const int nkept = ((PEN || DIFF) && p.window > 0) ? min((p.keep_first + KT - 1) / KT, kv_start / KT) : 0;      // steps over the kept first keys
-    auto first_key = [&](int it) { return ((PEN || DIFF) && it < nkept) ? it * KT : kv_start + ((KS == 1 ? it : it * KS + grp) - nkept) * KT; };
+    auto first_key = [&](int it) { return ((PEN || DIFF) && it < nkept) ? it * KT : kv_start + (it - nkept) * KT; };
 
     // the wave's two query tiles: head and position block
     int qi[NQT], head[NQT], qpos[NQT], qrow[NQT]; bool qvalid[NQT];
@@ -208,12 +204,12 @@ __global__ __launch_bounds__(64 * FLASH_WAVES * KS, 8 / FLASH_WAVES / KS) void f
     // instructions per step next to 68 MFMAs).  Keys beyond the last visible one (the final step of a tile) are clamped to it.
     constexpr int V_OFF = KT * D * 2;            // V image behind the K image of a ring slot
     static_assert(V_OFF == PIECES * NT * 16, "glds_pieces walks the pieces of the K image, then of the V image, NT * 16 bytes apart");
-    const unsigned lds_ring = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem + grp * NBUF * STAGE;
+    const unsigned lds_ring = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem;
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     int64_t kconst[PIECES], vconst[PIECES];      // element offsets of this thread's pieces inside a step
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
-        const int idx = i * NT + tid, row = idx / CPR, c = idx % CPR;
+        const int idx = i * NT + threadIdx.x, row = idx / CPR, c = idx % CPR;
         const int vsw = D == 128 ? ((row & 7) << 1) : (((row >> 1) & 3) << 1);      // = v_swz<D>(row), spelled out: a call here makes hipcc drop the host stub
         const int64_t rowoff = (PAGED && UB) ? ((int64_t)row * p.KVH + g) * D : (int64_t)row * p.ldkv + (int64_t)g * D;
         kconst[i] = rowoff + (c ^ (row & (CPR - 1))) * 8;
@@ -246,7 +242,7 @@ __global__ __launch_bounds__(64 * FLASH_WAVES * KS, 8 / FLASH_WAVES / KS) void f
             }
 #pragma unroll
             for (int i = 0; i < PIECES; ++i) {
-                const int idx = i * NT + tid, row = idx / CPR, c = idx % CPR;
+                const int idx = i * NT + threadIdx.x, row = idx / CPR, c = idx % CPR;
                 int key = kt + row; if (key > kv_end - 1) key = kv_end - 1;
                 int64_t off;
                 if (PAGED && UB) {
@@ -276,7 +272,7 @@ __global__ __launch_bounds__(64 * FLASH_WAVES * KS, 8 / FLASH_WAVES / KS) void f
     float m[NQT];
 #pragma unroll
     for (int t = 0; t < NQT; ++t) {
-        m[t] = grp ? -1e30f : -INFINITY; ol[t] = (float4_t){0.f, 0.f, 0.f, 0.f};      // (the second group's first step may hold no visible key of a query: a finite maximum keeps the differences finite)
+        m[t] = -INFINITY; ol[t] = (float4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < NDT; ++i) o[t][i] = (float4_t){0.f, 0.f, 0.f, 0.f};
     }
@@ -290,7 +286,7 @@ __global__ __launch_bounds__(64 * FLASH_WAVES * KS, 8 / FLASH_WAVES / KS) void f
     for (int t = 0; t < NQT; ++t) {
         pr1[t] = (PEN && p.r1) ? p.r1[head[t]] * (lin ? 1.44269504088896340736f : 1.0f) : 0.f; pr2[t] = (PEN && p.r2) ? p.r2[head[t]] : 0.f;
         if (PEN && p.sink) { m[t] = p.sink[head[t]] * 1.44269504088896340736f; ol[t] = (float4_t){1.f, 1.f, 1.f, 1.f}; }
-        else if (!GATE && !DIFF && p.sink && grp == 0) { m[t] = p.sink[head[t]] / p.scale; ol[t] = (float4_t){1.f, 1.f, 1.f, 1.f}; }      // (raw scores: the sink in their unit)
+        else if (!GATE && !DIFF && p.sink) { m[t] = p.sink[head[t]] / p.scale; ol[t] = (float4_t){1.f, 1.f, 1.f, 1.f}; }      // (raw scores: the sink in their unit)
         if (DIFF) m[t] = -1e30f;                                // (a step of a window may hold no visible key of a query: a finite maximum keeps the differences finite)
     }
     half8_t ones;
@@ -301,8 +297,7 @@ __global__ __launch_bounds__(64 * FLASH_WAVES * KS, 8 / FLASH_WAVES / KS) void f
     for (int t = 0; t < NQT; ++t) { gbias[t] = GATE ? p.gate_bias[head[t]] : 0.f; qcs[t] = (GATE && p.chunk > 0) ? qpos[t] / p.chunk * p.chunk : 0; }
     if (GATE && p.softcap > 0.f) gcap2 = 2.0f * 1.44269504088896340736f / p.softcap;
 
-    const int all_steps = nkept + (kv_end - kv_start + KT - 1) / KT, nsteps = (all_steps + KS - 1) / KS;
-    auto has_step = [&](int it) { return KS == 1 || it * KS + grp < all_steps; };             // (the groups walk the same number of steps, for their barriers)
+    const int nsteps = nkept + (kv_end - kv_start + KT - 1) / KT;
     // step `it` computes on ring slot it % NBUF while tile it+NBUF-1 is requested into the slot step it-1 just released;
     // before its closing barrier every wave waits until only the loads of tiles it+2.. are outstanding, so tile it+1 has
     // landed for all waves after the barrier and the global loads never drain inside the stream.
@@ -310,8 +305,8 @@ __global__ __launch_bounds__(64 * FLASH_WAVES * KS, 8 / FLASH_WAVES / KS) void f
         constexpr int cur = decltype(cur_c)::value;
         const int kt = first_key(it);
         const bool more = it + NBUF - 1 < nsteps;
-        if (more && has_step(it + NBUF - 1)) stage((cur + NBUF - 1) % NBUF, first_key(it + NBUF - 1));
-        const char *kl = smem + (grp * NBUF + cur) * STAGE, *vl = kl + KT * D * 2;
+        if (more) stage((cur + NBUF - 1) % NBUF, first_key(it + NBUF - 1));
+        const char *kl = smem + cur * STAGE, *vl = kl + KT * D * 2;
         if (kt <= wave_last) {
 
         // Sᵀ tiles: NMT x (16 keys x 16 queries) per query tile; one K fragment read feeds both
@@ -449,7 +444,7 @@ __global__ __launch_bounds__(64 * FLASH_WAVES * KS, 8 / FLASH_WAVES / KS) void f
 
 #pragma unroll
     for (int b = 0; b < NBUF - 1; ++b)
-        if (b < nsteps && has_step(b)) stage(b, first_key(b));
+        if (b < nsteps) stage(b, first_key(b));
     if (NBUF - 1 < nsteps) {
         if (NBUF == 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         else if (NBUF == 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(1 * 2 * PIECES) : "memory");
@@ -496,28 +491,6 @@ __global__ __launch_bounds__(64 * FLASH_WAVES * KS, 8 / FLASH_WAVES / KS) void f
             }
         }
         return;
-    }
-    if constexpr (KS > 1) {                                     // (the last step's barrier has freed the rings)
-        constexpr int PER = NDT + 1;
-        float4_t *po = reinterpret_cast<float4_t *>(smem) + (int64_t)wave * (NQT * PER * 64) + lane;
-        if (grp == 1) {
-#pragma unroll
-            for (int t = 0; t < NQT; ++t) {
-#pragma unroll
-                for (int dt = 0; dt < NDT; ++dt) po[(t * PER + dt) * 64] = o[t][dt];
-                po[(t * PER + NDT) * 64] = (float4_t){m[t], ol[t][0], 0.f, 0.f};
-            }
-        }
-        __syncthreads();
-        if (grp == 1) return;
-#pragma unroll
-        for (int t = 0; t < NQT; ++t) {
-            const float4_t ml = po[(t * PER + NDT) * 64];
-            const float mn = fmaxf(m[t], ml[0]), a0 = __builtin_amdgcn_exp2f((m[t] - mn) * cs), a1 = __builtin_amdgcn_exp2f((ml[0] - mn) * cs);   // (group 0 has seen key 0: mn is finite)
-            ol[t][0] = ol[t][0] * a0 + ml[1] * a1;
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) o[t][dt] = o[t][dt] * a0 + po[(t * PER + dt) * 64] * a1;
-        }
     }
 #pragma unroll
     for (int t = 0; t < NQT; ++t) {
@@ -566,10 +539,6 @@ int flash_prefill(const FlashArgs &a, bool paged, hipStream_t s) {
     const int G = a.H / a.KVH;
     dim3 grid((unsigned)((int64_t)a.ntiles * a.KVH)), block(64 * FLASH_WAVES);
     const bool ub = paged && p.bs_shift >= 0 && a.block_size % NVR_FLASH_KT == 0;
-    // at most one workgroup per CU and more than five steps: two groups of waves share a tile's steps (with more workgroups the second one of a CU fills the SIMDs as the second group
-    // would; over fewer steps the meeting costs what it saves).  Qwen3-0.6B prompt steps, us with one / two groups: 64 tokens 1320 / 1353, 4 x 200..300 2843 / 2849, 509 2027 / 1998,
-    // 1024 3285 / 3172, 1900 4331 / 4145, 510 behind 1530 cached 2923 / 2727, 800 behind 7200 cached 6765 / 5959
-    const bool few = grid.x <= 256 && a.max_keys > 5 * NVR_FLASH_KT;
 #define NVR_FLASH(DD, GG)                                                                             \
     if (a.D == DD && G == GG) {                                                                       \
         if (diff && ub) flash_prefill_kernel<DD, GG, true, true, false, false, false, true><<<grid, block, 0, s>>>(p);   \
@@ -578,8 +547,6 @@ int flash_prefill(const FlashArgs &a, bool paged, hipStream_t s) {
         else if (gate) flash_prefill_kernel<DD, GG, true, false, false, false, true><<<grid, block, 0, s>>>(p);   \
         else if (pen && ub) flash_prefill_kernel<DD, GG, true, true, false, true><<<grid, block, 0, s>>>(p);   \
         else if (pen) flash_prefill_kernel<DD, GG, true, false, false, true><<<grid, block, 0, s>>>(p);   \
-        else if (few && ub) flash_prefill_kernel<DD, GG, true, true, false, false, false, false, 2><<<grid, dim3(128 * FLASH_WAVES), 0, s>>>(p);    \
-        else if (few && !paged) flash_prefill_kernel<DD, GG, false, false, false, false, false, false, 2><<<grid, dim3(128 * FLASH_WAVES), 0, s>>>(p);  \
         else if (ub) flash_prefill_kernel<DD, GG, true, true><<<grid, block, 0, s>>>(p);              \
         else if (paged) flash_prefill_kernel<DD, GG, true><<<grid, block, 0, s>>>(p);                 \
         else flash_prefill_kernel<DD, GG, false><<<grid, block, 0, s>>>(p);                           \

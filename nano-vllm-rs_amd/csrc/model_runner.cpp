@@ -920,7 +920,7 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
             } else if (prefill_kv_cache) {                          // every sequence's blocks are consecutive: its K/V rows are contiguous IN the cache
                 f.k = k_cache(l); f.v = v_cache(l); f.ldkv = KVH * D;
             } else { f.k = qkv + H * D; f.v = qkv + (H + KVH) * D; f.ldkv = QKV; }
-            f.tiles = (const k::FlashTile *)(in_dev + off_tiles); f.ntiles = (int32_t)n_tiles; f.max_keys = (int32_t)max_ctx;
+            f.tiles = (const k::FlashTile *)(in_dev + off_tiles); f.ntiles = (int32_t)n_tiles;
             f.H = (int32_t)H; f.KVH = (int32_t)KVH; f.D = (int32_t)D; f.scale = scale; f.out = attn;
             RC(KD(flash_prefill(f, prefill_paged, st)));
         } else if (is_prefill) {                                     // head shapes outside the MFMA kernel: row kernel

@@ -729,7 +729,6 @@ static int run_prefill_attn(const nvr_half *q, int64_t ldq, const nvr_half *kk, 
         f.q = q; f.ldq = ldq; f.k = kk; f.v = v; f.ldkv = ldkv; f.block_tables = m->block_tables; f.max_blocks = m->max_blocks;
         f.block_size = (int32_t)bs; f.tiles = d; f.ntiles = (int32_t)tiles.size(); f.H = (int32_t)H; f.KVH = (int32_t)KVH; f.D = (int32_t)D;
         f.scale = scale; f.out = out;
-        for (const k::FlashTile &t : tiles) f.max_keys = std::max(f.max_keys, t.pos0 + t.nq);
         rc = KO(flash_prefill(f, paged, st));
         hipStreamSynchronize(st);
         hipFree(d);

@@ -343,46 +343,3 @@ def test_layer_list_gated_head_norm_and_clamped_unit(dtype, heads, vdim, ff, bat
     got = [d.step([("s%d" % i, t[len(t) - 2 + k:len(t) - 1 + k]) for i, t in enumerate(tokens)]) for k in range(2)]
     err = [u.row_errors(np.concatenate([g["s%d" % i] for g in got]), u.expected_logits(cfg, w, tokens[i])[-2:]) for i in range(0, batch, 5)]
     assert np.median(err) < u.TOL[dtype] / 2 and np.max(err) < (0.5 if dtype == "bfloat16" else 1e-2)
-
-
-@pytest.mark.parametrize("paged", [False, True])
-@pytest.mark.parametrize("G,KVH,D,cases", [
-    (2, 8, 128, [(321, 321), (449, 449)]),               # six and eight steps, the last of one key: the groups end on different steps
-    (1, 2, 64, [(700, 40), (65, 65), (1, 1)]),           # (keys, new rows): tiles of one step beside tiles of eleven
-    (4, 2, 128, [(385, 385), (2049, 7)]),
-    (1, 1, 128, [(640, 640)]),
-    (4, 1, 64, [(1000, 33), (512, 512)]),
-])
-def test_prompt_attention_by_two_groups_of_waves(paged, G, KVH, D, cases):
-    """Few tiles over more than five 64-key steps: two groups of waves take a tile's steps in turn and meet at the end, contiguous rows and cache blocks, against the oracle.  P is rounded to
-    float16 before P V (2^-11 relative per term) and the meeting adds f32 roundings only: the bounds of the one-group form's tests, 2 ulps and 2e-3 on outputs of order 1."""
-    rng = np.random.default_rng(G * D + len(cases))
-    if not paged:
-        cases = [(n, n) for _, n in cases]
-    H, bs, l = G * KVH, 64, nvr.lib()
-    blocks = [(c + bs - 1) // bs for c, _ in cases]
-    T, mb = sum(n for _, n in cases), max(blocks) + 1
-    cu = np.concatenate([[0], np.cumsum([n for _, n in cases])]).astype(np.int32)
-    ctx, scale = np.asarray([c for c, _ in cases], np.int32), float(D ** -0.5)
-    q = rng.standard_normal((T, H, D)).astype(F16)
-    meta = nvr.AttnMetaC()
-    d_cu, d_ctx, out = dev(cu), dev(ctx), nvr.DeviceBuffer(T * H * D * 2)
-    meta.is_prefill, meta.cu_seqlens_q, meta.cu_seqlens_k, meta.batch = 1, d_cu.ptr, d_cu.ptr, len(cases)
-    meta.max_seqlen_q = meta.max_seqlen_k = meta.max_context_len = int(ctx.max())
-    if paged:
-        kc, vc = (rng.standard_normal((sum(blocks), bs, KVH, D)).astype(F16) for _ in range(2))
-        bt = np.full((len(cases), mb), -1, np.int32)
-        perm, o = rng.permutation(sum(blocks)), 0
-        for b, n in enumerate(blocks):
-            bt[b, :n] = perm[o:o + n]; o += n
-        d_bt, d_q, d_k, d_v = dev(bt), dev(q.view(np.uint16)), dev(kc.view(np.uint16)), dev(vc.view(np.uint16))
-        meta.context_lens, meta.block_tables, meta.max_blocks = d_ctx.ptr, d_bt.ptr, mb
-        nvr.check(l.nvr_attn_prefill_paged(d_q.ptr, H * D, d_k.ptr, d_v.ptr, C.byref(meta), T, H, KVH, D, bs, scale, out.ptr, None))
-        ref = oracle.attn_paged(q.astype(np.float32), cu, kc.astype(np.float32), vc.astype(np.float32), bt, ctx, scale)
-    else:
-        k, v = (rng.standard_normal((T, KVH, D)).astype(F16) for _ in range(2))
-        d = dev(np.concatenate([q.reshape(T, -1), k.reshape(T, -1), v.reshape(T, -1)], 1).view(np.uint16))
-        nvr.check(l.nvr_attn_prefill_varlen(d.ptr, d.ptr + H * D * 2, d.ptr + (H + KVH) * D * 2, (H + 2 * KVH) * D, C.byref(meta), T, H, KVH, D, scale, out.ptr, None))
-        ref = oracle.attn_prefill_varlen(q.astype(np.float32), k.astype(np.float32), v.astype(np.float32), cu, scale)
-    got = out.to_numpy((T, H, D), F16).astype(np.float32)
-    assert np.all(np.abs(got - ref) <= 2 * np.spacing(np.abs(ref).astype(F16)).astype(np.float32) + 2e-3), np.abs(got - ref).max()
