@@ -842,33 +842,6 @@ int nvr_model_runner::forward_prefill_two(int64_t T, int64_t B) {
     return NVR_OK;
 }
 
-// The last layer of a prefill step behind its qkv product: nothing reads the other rows' hidden states any more (their keys and values are in the caches; the LM head takes
-// every sequence's last row, embed_head.rs:272-289), so attention, o_proj and the MLP run on the B last rows alone, as a decode step would run them: one query row per sequence over
-// the cached keys.  What is left out of a layer is its attention over the prompt, three of its four products and both norms: Qwen3-0.6B, 32 x 1024 tokens
-// 34.9 -> 34.0 ms a step, 509 tokens 2.10 -> 2.08 ms.
-// The rows end in n[0 .. B), normalised by the final norm.
-int nvr_model_runner::last_layer_rows(int64_t B, int64_t max_ctx) {
-    hipStream_t st = stream;
-    const Layer &w = layers[L - 1];
-    const bool tl = tiled_weights && B <= 64;
-    uint16_t *qr = gu, *hr = gu + B * QKV;                               // (gu: nothing of this layer; B (QKV + Hd) <= max_tokens 2 I elements: execute())
-    RC(KD(select_last_tokens(qkv, d_cu, B, QKV, qr, st)));
-    RC(KD(select_last_tokens(h, d_cu, B, Hd, hr, st)));
-    k::AttnArgs a{};
-    a.q = qr; a.ldq = QKV; a.ctx_lens = dd_ctx; a.nq = (int32_t)B; a.H = (int32_t)H; a.KVH = (int32_t)KVH; a.D = (int32_t)D;
-    a.scale = scale; a.max_ctx = (int32_t)max_ctx; a.out = attn;
-    a.k = k_cache(L - 1); a.v = v_cache(L - 1); a.block_tables = dd_bt; a.max_blocks = (int32_t)max_blocks_per_seq;
-    a.block_size = (int32_t)block_size; a.workspace = attn_ws; a.workspace_bytes = attn_ws_bytes; a.tickets = attn_tickets;
-    RC(KD(attention(a, true, st)));
-    uint16_t *const whole = h;
-    h = hr;                                                              // (the residual rows row_parallel_norm adds to)
-    int rc = row_parallel_norm(attn, H * D, w.o, tl ? w.o_t : nullptr, B, w.ln2);
-    if (!rc) rc = KD(linear_silu_mul(n, Hd, w.gate_up, B, Hd, I, act, st, tl ? w.gate_up_t : nullptr));
-    if (!rc) rc = row_parallel_norm(act, I, w.down, tl ? w.down_t : nullptr, B, norm);
-    h = whole;
-    return rc;
-}
-
 // Qwen3Model::forward, src/models/qwen3.rs:487-505; layer wiring :372-392; attention :208-240; MLP :305-314.
 int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max_ctx) {
     hipStream_t st = stream;
@@ -907,7 +880,6 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
             RC(KD(linear_qkv_rope_store(n, Hd, w.qkv, T, Hd, H, KVH, D, pos, slots, cos_t, sin_t, qkv, k_cache(l), v_cache(l), st, tl ? w.qkv_t : nullptr,
                                         is_prefill && n_tiles > 0 && (prefill_paged || prefill_kv_cache))));
         }
-        if (is_prefill && prefill_last_rows && l == L - 1) { RC(last_layer_rows(B, max_ctx)); break; }
         k::AttnArgs a{};
         a.q = qkv; a.ldq = QKV; a.ctx_lens = ctx; a.nq = (int32_t)T; a.H = (int32_t)H; a.KVH = (int32_t)KVH; a.D = (int32_t)D;
         a.scale = scale; a.max_ctx = (int32_t)max_ctx; a.out = attn;
@@ -960,7 +932,7 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
     }
     if (L == 0) RC(KD(rmsnorm(h, norm, mc.rms_norm_eps, T, Hd, n, st)));                  // final norm :501
     const uint16_t *hl = n;
-    if (is_prefill && !prefill_last_rows) { RC(KD(select_last_tokens(n, d_cu, B, Hd, nlast, st))); hl = nlast; }      // embed_head.rs:272-289
+    if (is_prefill) { RC(KD(select_last_tokens(n, d_cu, B, Hd, nlast, st))); hl = nlast; }      // embed_head.rs:272-289
     if (lm_parts > 0) {                                                                        // f32 logits (A-21) + arg-max partials
         int32_t np = 0;
         RC(KD(lm_head(hl, Hd, lm_head, B, Hd, Vl, logits, d_lm_pval, d_lm_pidx, &np, st, want_logits, (tiled_weights && B <= 32) ? lm_head_t : nullptr)));
@@ -1021,17 +993,11 @@ int nvr_model_runner::execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill
         mb_rows = mb_tiles = 0;
         tp_overlap_chunks = 0;
         int64_t total = 0;
-        bool tables_fit = true;
         for (size_t b = 0; b < nseq; ++b) {
             int64_t lo, hi; range_of(*seqs[b], &lo, &hi);
             prefill_paged |= lo > 0;
             total += hi - lo;
-            tables_fit &= (int64_t)seqs[b]->block_table.size() <= max_blocks_per_seq;
         }
-        // the last layer on the last rows alone (last_layer_rows): one rank, the plain graph's projections, and few enough last rows that a decode-sized layer is the smaller one
-        // (from a quarter of the step's rows on it is not worth its launches)
-        prefill_last_rows = flash_ok && tables_fit && tp == 1 && !comm.active() && !mc.use_bias && L > 0 && total >= 4 * (int64_t)nseq &&
-                            (int64_t)nseq * (QKV + Hd) <= max_tokens * 2 * I;
         if (total > max_tokens) return nvr::fail(NVR_ERR_INVALID_ARG, "prefill of %ld tokens exceeds max_num_batched_tokens %ld", (long)total, (long)max_tokens);
         // Whole prompts: the flash kernel reads K / V from the caches, never from the step's qkv buffer, so the qkv GEMM writes them once
         // (gemm256 skips the k / v columns of the qkv buffer: -9 % on that GEMM).  If every sequence's blocks are consecutive (blocks come off
@@ -1094,13 +1060,9 @@ int nvr_model_runner::execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill
             }
             cu[b + 1] = (int32_t)T;
             max_ctx = std::max(max_ctx, end);
-            if (prefill_paged || prefill_last_rows) {
+            if (prefill_paged) {
                 if ((int64_t)s.block_table.size() > max_blocks_per_seq) return nvr::fail(NVR_ERR_INVARIANT, "block table longer than max_model_len allows");
                 std::memcpy(bt + b * max_blocks_per_seq, s.block_table.data(), s.block_table.size() * 4);
-                if (prefill_last_rows) {                                  // what a decode step's attention reads
-                    for (int64_t j = (int64_t)s.block_table.size(); j < max_blocks_per_seq; ++j) bt[b * max_blocks_per_seq + j] = -1;
-                    ((int32_t *)(hd + dof_ctx))[b] = (int32_t)end;
-                }
             }
             if (flash_ok) {                                              // longest-context tiles of a sequence first
                 const int64_t nq = end - c0;
@@ -1172,8 +1134,7 @@ int nvr_model_runner::execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill
     auto up = [&](size_t off, size_t bytes) { return hipMemcpyAsync(in_dev + off, in_host + off, bytes, hipMemcpyHostToDevice, stream); };
     if (is_prefill) {
         NVR_HIP_CHECK(up(0, n_tiles ? off_tiles + (size_t)n_tiles * sizeof(k::FlashTile) : prefill_bytes));   // ids | pos | slots | ctx | kv base | cu | tiles
-        if (prefill_last_rows) NVR_HIP_CHECK(up(off_dec + dof_ctx, dof_bt - dof_ctx + nseq * max_blocks_per_seq * 4));
-        else if (prefill_paged) NVR_HIP_CHECK(up(off_dec + dof_bt, nseq * max_blocks_per_seq * 4));
+        if (prefill_paged) NVR_HIP_CHECK(up(off_dec + dof_bt, nseq * max_blocks_per_seq * 4));
     } else NVR_HIP_CHECK(up(off_dec, dof_bt + nseq * max_blocks_per_seq * 4));
 
     last_rows = nseq; last_prefill = is_prefill; last_tokens = T;
@@ -1186,7 +1147,7 @@ int nvr_model_runner::execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill
     want_logits = logits_asked || !lazy_logits || lm_parts == 0;
     for (size_t i = 0; i < nseq && !want_logits; ++i) want_logits = seqs[i]->sampling.temperature != 0.0f;
     logits_valid = want_logits;
-    lm_input = is_prefill && !prefill_last_rows ? nlast : n;             // the rows the LM head reads this step (forward())
+    lm_input = is_prefill ? nlast : n;                                   // the rows the LM head reads this step (forward())
     if (is_prefill || cfg.enforce_eager || graphs_disabled) {
         const int rc = forward(T, (int64_t)nseq, is_prefill, max_ctx);
         if (rc && comm_stream) {

@@ -211,58 +211,6 @@ def test_layer_list_decode_steps(W, taps, heads, kv, dim, lengths):
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
-@pytest.mark.parametrize("qk_norm,kv_heads,head_dim,lengths", [(0, 2, 64, [4]), (0, 2, 64, [3]), (1, 2, 64, [5, 90, 17, 4]), (0, 1, 128, [63, 64, 65, 200]), (1, 2, 128, [8] * 65), (0, 2, 64, [3, 5, 4])])
-def test_prompt_steps_run_their_last_layer_on_the_last_rows(dtype, qk_norm, kv_heads, head_dim, lengths):
-    """A prompt step (last layer on the sequences' last rows: a quarter of the step's rows or fewer) against the same prompts without their last token and a decode step behind them:
-    logits of the two within the rounding of the 16-bit type over two layers, last layer's keys and values of every row there (a decode step reads them), portions too."""
-    model = nvr.ModelConfig(vocab_size=160, hidden_size=128, intermediate_size=256, num_hidden_layers=2, num_attention_heads=2, num_key_value_heads=kv_heads, head_dim=head_dim,
-                            max_position_embeddings=512, rms_norm_eps=1e-6, rope_theta=1e4, tie_word_embeddings=0, init_std=0.08, seed=5, qk_norm=qk_norm)
-    n = len(lengths)
-    blocks = sum(-(-(L + 1) // 16) for L in lengths)
-    prompts = [nvr.synthetic_tokens(L + 1, 8, i, 160) for i, L in enumerate(lengths)]
-    sp = nvr.SamplingParams(temperature=0.0, ignore_eos=True)
-
-    def engine(chunked):
-        r = nvr.ModelRunner(nvr.Config(skip_block_size_check=1, max_num_seqs=n, max_num_batched_tokens=max(64, sum(lengths)), max_model_len=512, kvcache_block_size=16, num_kvcache_blocks=blocks,
-                                       dtype=dtype, enable_chunked_prefill=chunked), model)
-        bm = nvr.BlockManager(blocks, 16)
-        return r, bm
-
-    def begin(bm, cut):
-        seqs = [nvr.Sequence(p[:L - cut], sp, 16) for p, L in zip(prompts, lengths)]
-        for s in seqs:
-            bm.allocate(s)
-        return seqs
-
-    def decode(r, bm, seqs, at):
-        for s, p, L in zip(seqs, prompts, lengths):
-            s.append_token(int(p[L + at]))
-            bm.may_append(s)
-        r.execute_model(seqs, False)
-        return r.logits(n).copy()
-    r, bm = engine(0)
-    seqs = begin(bm, 0)
-    r.execute_model(seqs, True)
-    whole = r.logits(n).copy()
-    after = decode(r, bm, seqs, 0)
-    r, bm = engine(0)
-    seqs = begin(bm, 1)
-    r.execute_model(seqs, True)
-    step = decode(r, bm, seqs, -1)
-    tol = 2.0 ** (-8 if dtype == "float16" else -5) * float(np.abs(step).max())      # a few dozen roundings of 2^-11 (2^-8) through two layers, at the logits' scale
-    assert np.abs(whole - step).max() < tol
-    assert np.abs(after - decode(r, bm, seqs, 0)).max() < tol
-    if min(lengths) >= 8:                                                              # in two portions: the second behind the first one's cached rows
-        r, bm = engine(1)
-        seqs = begin(bm, 0)
-        for a, b in ((0, 3), (3, None)):
-            for s, L in zip(seqs, lengths):
-                s.set_chunk(a, (L if b is None else b) - a)
-            r.execute_model(seqs, True)
-        assert np.abs(r.logits(n) - whole).max() < tol
-
-
-@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("hidden,inter,heads,kv,dim,qk_norm", [(256, 512, 4, 2, 64, 0), (1024, 1024, 8, 8, 128, 1), (2048, 512, 8, 4, 128, 0), (256, 512, 4, 1, 128, 1), (384, 512, 4, 2, 64, 0)])
 def test_decode_steps_of_one_and_two_rows_against_more(dtype, hidden, inter, heads, kv, dim, qk_norm):
     """One or two sequences (add + norm inside the products behind them, where the width is a multiple of 256) give the logits that the same sequences give in a batch of three (launches of
