@@ -441,7 +441,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float *__restrict
     *reinterpret_cast<half4_t *>(out + pair * D + d) = hv;
 }
 
-// ---- work-balanced form (r06) ---------------------------------------------------------------------------------------
+// ---- work-balanced form ---------------------------------------------------------------------------------------
 // attn_rows_kernel gives every (query, kv head) pair its own workgroup(s): 264 pairs on 256 CUs (33 sequences x 8 kv heads) run as one full round and a tail,
 // 35.6 us per layer where 256 pairs take 24.5.  Here the launch is nw shares x KVH workgroups and the WORK is cut evenly: the keys of all queries, in units of
 // CH = WAVES * TPI keys (one full round of a workgroup), query after query, form one line of utot units; share w walks the units [w * utot / nw, (w + 1) * utot / nw)
