@@ -484,7 +484,9 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
     __syncthreads();
     const int g = blockIdx.x % p.KVH, ws = blockIdx.x / p.KVH;
     const long long utot = pre[nq];
-    const long long ub = ws * utot / nw, ue = (ws + 1) * utot / nw;
+    // no more shares than units: behind a share without a unit the slots of a cut query would count a share that never draws its ticket (few queries with keys, many without)
+    nw = (int)min((long long)nw, max(utot, 1ll));
+    const long long ub = min(ws * utot / nw, utot), ue = min((ws + 1) * utot / nw, utot);
     // a query without keys owns no unit: its output row is zero, as in attn_rows_kernel (L == 0)
     for (int t0 = blockIdx.x; t0 < nq; t0 += gridDim.x)
         if (cx[t0] == 0)

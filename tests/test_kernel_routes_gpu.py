@@ -253,27 +253,46 @@ def test_decode_steps_of_one_and_two_rows_against_more(dtype, hidden, inter, hea
 def test_work_balanced_attention_against_the_per_pair_form(B, G, KVH, D, bs, ctx):
     """Equal shares of all queries' keys (each query charged two units for its start) against a workgroup per pair, over the same cache: both keep f32 scores,
     weights and sums and round once, so their outputs differ by one rounding of the result and the order of f32 sums of up to 5000 terms — 2 ulps of float16."""
+    _work_balanced_against_per_pair(B, G, KVH, D, bs, ctx, max(ctx), 1)
+
+
+@pytest.mark.parametrize("B,G,KVH,D,bs,ctx", [
+    (300, 2, 1, 64, 8, [128 if i % 30 == 0 else 0 for i in range(300)]),                   # 40 units, 256 shares: a cut query's units lay in shares 19 and 25
+    (300, 1, 1, 128, 16, [[0, 256, 1, 129, 192][i % 97 % 5] if i % 97 < 5 else 0 for i in range(300)]),
+    (270, 4, 1, 64, 16, [0] * 269 + [256]),                                                # one query: all units are its own
+    (100, 2, 3, 64, 8, [65 if i == 50 else 0 for i in range(100)]),
+    (260, 2, 1, 64, 8, [0] * 260),
+])
+def test_work_balanced_attention_of_few_queries_with_keys(B, G, KVH, D, bs, ctx):
+    """Fewer units of keys than shares: every cut query is merged by its last share and its counter returns to zero, so that a second launch over the same counters does the same."""
+    _work_balanced_against_per_pair(B, G, KVH, D, bs, ctx, 256, 2)
+
+
+def _work_balanced_against_per_pair(B, G, KVH, D, bs, ctx, bound, launches):
     l = nvr.lib()
     rng = np.random.default_rng(B + D)
     H, blocks = G * KVH, [(c + bs - 1) // bs for c in ctx]
-    mb, perm, o = max(blocks) + 1, rng.permutation(sum(blocks)), 0
+    mb, nb, o = max(blocks) + 1, max(sum(blocks), 1), 0
+    perm = rng.permutation(nb)
     bt = np.full((B, mb), -1, np.int32)
     for b, n in enumerate(blocks):
         bt[b, :n] = perm[o:o + n]; o += n
-    k, v = (dev(rng.standard_normal((sum(blocks), bs, KVH, D)).astype(F16).view(np.uint16)) for _ in range(2))
+    k, v = (dev(rng.standard_normal((nb, bs, KVH, D)).astype(F16).view(np.uint16)) for _ in range(2))
     q = dev(rng.standard_normal((B, H, D)).astype(F16).view(np.uint16))
     d_ctx, d_bt, tickets = dev(np.asarray(ctx, np.int32)), dev(bt), dev(np.zeros(B * KVH, np.uint32))
     meta = nvr.AttnMetaC()
-    meta.context_lens, meta.block_tables, meta.max_blocks, meta.batch, meta.max_context_len = d_ctx.ptr, d_bt.ptr, mb, B, max(ctx)
-    ws = nvr.DeviceBuffer(l.nvr_paged_attn_workspace_bytes(B, H, D, max(ctx)))
+    meta.context_lens, meta.block_tables, meta.max_blocks, meta.batch, meta.max_context_len = d_ctx.ptr, d_bt.ptr, mb, B, bound
+    ws = nvr.DeviceBuffer(l.nvr_paged_attn_workspace_bytes(B, H, D, bound))
     ref, got = nvr.DeviceBuffer(B * H * D * 2), nvr.DeviceBuffer(B * H * D * 2)
-    nvr.check(l.nvr_fill_const(got.ptr, B * H * D, C.c_float(float("nan")), None))
     args = (q.ptr, H * D, k.ptr, v.ptr, C.byref(meta), H, KVH, D, bs, D ** -0.5)
     nvr.check(l.nvr_paged_attn_decode(*args, ref.ptr, ws.ptr, None))
-    nvr.check(l.nvr_paged_attn_decode_fused(*args, got.ptr, ws.ptr, tickets.ptr, None))
-    a, b = ref.to_numpy((B, H, D), F16).astype(np.float32), got.to_numpy((B, H, D), F16).astype(np.float32)
-    assert np.all(np.abs(a - b) <= 2 * np.maximum(np.spacing(np.abs(a).astype(F16)).astype(np.float32), 2.0 ** -14 / 8)), np.abs(a - b).max()
-    assert not tickets.to_numpy((B * KVH,), np.uint32).any()
+    a = ref.to_numpy((B, H, D), F16).astype(np.float32)
+    for _ in range(launches):
+        nvr.check(l.nvr_fill_const(got.ptr, B * H * D, C.c_float(float("nan")), None))
+        nvr.check(l.nvr_paged_attn_decode_fused(*args, got.ptr, ws.ptr, tickets.ptr, None))
+        b = got.to_numpy((B, H, D), F16).astype(np.float32)
+        assert np.all(np.abs(a - b) <= 2 * np.maximum(np.spacing(np.abs(a).astype(F16)).astype(np.float32), 2.0 ** -14 / 8)), np.abs(a - b).max()
+        assert not tickets.to_numpy((B * KVH,), np.uint32).any()
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
