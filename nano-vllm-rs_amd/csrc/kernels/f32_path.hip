@@ -205,12 +205,15 @@ __global__ __launch_bounds__(256) void linear_kernel(const float *__restrict__ x
 constexpr int MB = 64, MKT = 32, MLD = MKT + 4;
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 // MPF K-tiles are requested ahead into registers (the weights of a short prompt come from HBM: with one tile ahead a K-step cost a round trip, 1.7 us).
-// Few output tiles (o / down projections of a short prompt: N = hidden) are split along k over blockIdx.z: part z writes the partial sums of its K-tiles to
-// y + z T N, and the launch that adds the residual and norms the row adds them up in order (sum_ranks_add_rmsnorm).  Qwen3-0.6B, 128 rows:
-// o / down 130 -> 10.4 us (8 parts), gate_up 55.7 -> 24.6, qkv 54.7 -> 23.5
+// A row-parallel product (o / down projections: N = hidden, few output tiles) sums k in segments whose number follows from K and N alone (linear_segments), added up in their
+// order: a row of a prompt has the same bits whatever else is in its step.  Where the step's tiles are few, blockIdx.z = one segment each: segment z writes its partial sums to
+// y + z T N, and the launch that adds the residual and norms the row adds them up (sum_ranks_add_rmsnorm).  Where the tiles fill the chip, or the slabs would not hold the sums, a
+// workgroup walks the segments (SEG) of `seg` K-tiles, a multiple of MPF, and adds them up itself.  Qwen3-0.6B, us a launch with one segment and one tile ahead / now: o / down 131 / 10.0
+// at 128 rows, 130 / 28.9 at 509, 132 / 53.3 (SEG) at 1024; gate_up 55.6 / 23.4, 116 / 59.6, 221 / 112; qkv 54.6 / 22.8, 76 / 40, 150 / 75
 constexpr int MPF = 4;
+template <bool SEG>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void linear_mfma_kernel(const float *__restrict__ x, int64_t ldx, const float *__restrict__ W, int T, int K, int N,
-                                                          const float *__restrict__ bias, float *__restrict__ y, int kslice) {
+                                                          const float *__restrict__ bias, float *__restrict__ y, int kslice, int seg) {
     __shared__ __attribute__((aligned(16))) float as[2][MB][MLD], bs[2][MB][MLD];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
     const int wn = wave >> 1, wm = wave & 1;                              // this wave: W rows n0 + 32 wn .., tokens t0 + 32 wm ..
@@ -233,9 +236,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
         *reinterpret_cast<float4_t *>(&as[buf][r][c * 4]) = e.w0; *reinterpret_cast<float4_t *>(&as[buf][r + 32][c * 4]) = e.w1;
         *reinterpret_cast<float4_t *>(&bs[buf][r][c * 4]) = e.x0; *reinterpret_cast<float4_t *>(&bs[buf][r + 32][c * 4]) = e.x1;
     };
-    f32x16 acc;
+    f32x16 acc, tot;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    for (int i = 0; i < 16; ++i) { acc[i] = 0.f; tot[i] = -0.f; }          // (-0 + a = a for every a)
     auto compute = [&](int buf) {
         float4 a4[4], b4[4];
 #pragma unroll
@@ -264,7 +267,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
         stash(buf ^ 1, next);                                             // (the other buffer: last read in the step before, in front of the barrier that ended it)
         __syncthreads();
     };
-    for (int kt = 0; kt < K4; kt += MPF) { step(kt, 0, s0, s1); step(kt + 1, 1, s1, s2); step(kt + 2, 0, s2, s3); step(kt + 3, 1, s3, s0); }
+    for (int kt = 0, end = seg; kt < K4; kt += MPF) {
+        step(kt, 0, s0, s1); step(kt + 1, 1, s1, s2); step(kt + 2, 0, s2, s3); step(kt + 3, 1, s3, s0);
+        if (SEG && kt + MPF == end) {
+            end += seg;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) { tot[i] += acc[i]; acc[i] = 0.f; }
+        }
+    }
+    if (SEG) acc = tot;                                                   // (whole segments: no remainder below)
     if (K4 < KT) compute(0);                                              // the remainder: its K-tiles sit in buffer 0 and in sets 1, 2
     if (K4 + 1 < KT) { __syncthreads(); stash(0, s1); __syncthreads(); compute(0); }
     if (K4 + 2 < KT) { __syncthreads(); stash(0, s2); __syncthreads(); compute(0); }
@@ -450,7 +461,7 @@ int linear(const float *x, int64_t ldx, const float *W, int64_t T, int64_t K, in
         return 0;
     }
     if (K % MKT == 0 && ldx % 4 == 0 && N % 4 == 0 && ((uintptr_t)x | (uintptr_t)W | (uintptr_t)y) % 16 == 0) {     // matrix cores (r06)
-        linear_mfma_kernel<<<dim3((unsigned)((N + MB - 1) / MB), (unsigned)((T + MB - 1) / MB)), dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)N, bias, y, (int)K);
+        linear_mfma_kernel<false><<<dim3((unsigned)((N + MB - 1) / MB), (unsigned)((T + MB - 1) / MB)), dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)N, bias, y, (int)K, 0);
         F32_LAUNCH_CHECK("f32 linear (mfma)");
         return 0;
     }
@@ -459,20 +470,23 @@ int linear(const float *x, int64_t ldx, const float *W, int64_t T, int64_t K, in
     return 0;
 }
 
-// parts of k for a product of few 64 x 64 tiles (1: none): doubled while the parts' workgroups still fit the 256 CUs once and a part keeps 8 K-tiles
-int linear_splitk_parts(int64_t T, int64_t K, int64_t N, int64_t ldx) {
-    if (T <= 8 || K % MKT || ldx % 4 || N % 4) return 1;
-    const int64_t tiles = ((N + MB - 1) / MB) * ((T + MB - 1) / MB);
+// segments of k of a row-parallel product of more than 8 rows (1: none), from K and N alone: doubled while the workgroups of one 64-row tile still fit the 256 CUs once and a segment keeps 8 K-tiles
+int linear_segments(int64_t K, int64_t N, int64_t ldx) {
+    if (K % MKT || ldx % 4 || N % 4) return 1;
     int S = 1;
-    while (S < 8 && tiles * S * 2 <= 256 && K % (MKT * S * 2) == 0 && K / (S * 2) >= 8 * MKT) S *= 2;
+    while (S < 8 && (N + MB - 1) / MB * S * 2 <= 256 && K % (MKT * MPF * S * 2) == 0 && K / (S * 2) >= 8 * MKT) S *= 2;
     return S;
 }
-int linear_splitk(const float *x, int64_t ldx, const float *W, int64_t T, int64_t K, int64_t N, int64_t S, float *parts, hipStream_t s) {
-    if (T < 1 || S < 1 || K % (MKT * S) || ldx % 4 || N % 4 || ((uintptr_t)x | (uintptr_t)W | (uintptr_t)parts) % 16)
-        return nvr::fail(NVR_ERR_UNSUPPORTED, "f32 linear_splitk: T=%ld K=%ld N=%ld in %ld parts", (long)T, (long)K, (long)N, (long)S);
-    linear_mfma_kernel<<<dim3((unsigned)((N + MB - 1) / MB), (unsigned)((T + MB - 1) / MB), (unsigned)S), dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)N, nullptr, parts,
-                                                                                                                       (int)(K / S));
-    F32_LAUNCH_CHECK("f32 linear_splitk (mfma)");
+// up to 6 workgroups per CU the segments run apart; beyond, the slabs' bytes cost more than the rounds they fill (Qwen3-0.6B, ms a prompt, one after the other / apart: 550 tokens 11.45 / 10.46, 700
+// 13.89 / 13.32, 768 14.83 / 14.32, 1024 20.17 / 20.37)
+bool linear_segments_apart(int64_t T, int64_t N, int64_t S) { return (N + MB - 1) / MB * ((T + MB - 1) / MB) * S <= 1536; }
+int linear_segmented(const float *x, int64_t ldx, const float *W, int64_t T, int64_t K, int64_t N, int64_t S, bool apart, float *y, hipStream_t s) {
+    if (T < 1 || S < 1 || K % (MKT * MPF * S) || ldx % 4 || N % 4 || ((uintptr_t)x | (uintptr_t)W | (uintptr_t)y) % 16)
+        return nvr::fail(NVR_ERR_UNSUPPORTED, "f32 linear_segmented: T=%ld K=%ld N=%ld in %ld segments", (long)T, (long)K, (long)N, (long)S);
+    const dim3 grid((unsigned)((N + MB - 1) / MB), (unsigned)((T + MB - 1) / MB), apart ? (unsigned)S : 1u);
+    if (apart) linear_mfma_kernel<false><<<grid, dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)N, nullptr, y, (int)(K / S), 0);
+    else linear_mfma_kernel<true><<<grid, dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)N, nullptr, y, (int)K, (int)(K / S / MKT));
+    F32_LAUNCH_CHECK("f32 linear_segmented (mfma)");
     return 0;
 }
 
@@ -788,19 +802,21 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnArgsF a, int paged) 
 }
 // The same for head dims of 64, 128, 192 and 256 on 16-byte aligned rows: nothing but the last merge goes through LDS.  Sixteen lanes hold a key's row (and
 // the query's, and an output row): NF 16-byte pieces each, so a load of K or V touches whole lines, where a thread per key touched 64 lines per load and
-// paid for each; the score is summed over the sixteen lanes on DPP and every lane weighs its own piece of V with it.  A group of sixteen lanes walks keys
-// group, group + 4 NW, .. in batches of four with a running maximum of its own (K and V of the first batch are requested before anything is known but the
-// block table, those of the next batch before this one is used), the four groups of a wave meet in registers, the NW waves in LDS.  What bounds a decode
-// step's launch is that chain of round trips, not bytes: one sequence
-// of 128 .. 176 keys of Qwen3-0.6B 14.3 -> 8.0 us a launch, 128 prompt rows 38.6 -> 18.0
+// paid for each; the score is summed over the sixteen lanes on DPP and every lane weighs its own piece of V with it.  Sixteen groups share a round of 64 keys (32 for wide heads), a group
+// taking keys group, group + 16, .. with a running maximum of its own; a row's even and its odd rounds are summed apart.  Eight waves take them side by side (a decode step: the keys have to
+// fill the chip), four waves in turn (a prompt: the rows do) — the same sums in the same order, so that a row's bits do not depend on how many rows are in its step.  K and V of the first
+// round are requested before anything is known but the block table, those of the next round before this one is used; the four groups of a wave meet in registers, the eight sums of the row
+// in LDS.  What bounds a decode step's launch is that chain of round trips, not bytes.  Qwen3-0.6B, us a launch, the general form / this one: one sequence of 150 keys 14.3 / 7.3, of 4096 keys
+// 195 / 78; prompts of 128 rows 38 / 19, 509 268 / 129, 1024 873 / 401
 template <int NF, int NW, bool PAGED>
 __global__ __launch_bounds__(64 * NW) void attention_rows_kernel(AttnArgsF a) {
     constexpr int D = 64 * NF, KB = NF <= 2 ? 4 : 2;                     // keys a group requests at a time
-    constexpr int STEP = 4 * NW, ROUND = KB * STEP;                      // groups; keys of one round of all groups
-    __shared__ __attribute__((aligned(16))) float part[NW][D];
-    __shared__ float pm[NW], pl[NW];
+    constexpr int STEP = 16, ROUND = KB * STEP, NEXT = NW == 8 ? 2 * ROUND : ROUND;   // groups of four waves; keys of their round; from a wave's round to its next one
+    __shared__ __attribute__((aligned(16))) float part[8][D];
+    __shared__ float pm[8], pl[8];
     const int t = blockIdx.x, hd = blockIdx.y, g = hd / (a.H / a.KVH);
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, group = (int)threadIdx.x >> 4;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, group = (wave & 3) * 4 + (lane >> 4);
+    const int first = NW == 8 ? (wave >> 2) * ROUND : 0;                 // the wave's first round
     const int32_t *bt = PAGED ? a.block_tables + (int64_t)(a.seq_of_q ? a.seq_of_q[t] : t) * a.max_blocks : nullptr;
     const int64_t base = PAGED ? 0 : (int64_t)a.kv_base[t];
     // block of key j (any j >= 0: entries behind a sequence's blocks may be stale, and are never used: a key past the context reads key 0's row)
@@ -811,7 +827,7 @@ __global__ __launch_bounds__(64 * NW) void attention_rows_kernel(AttnArgsF a) {
     };
     int ea[KB], eb[KB];                                                  // the entries of two rounds: requested with the context length
 #pragma unroll
-    for (int u = 0; u < KB; ++u) { ea[u] = entry(group + u * STEP); eb[u] = entry(group + ROUND + u * STEP); }
+    for (int u = 0; u < KB; ++u) { ea[u] = entry(first + group + u * STEP); eb[u] = entry(first + NEXT + group + u * STEP); }
     const int64_t row0 = row_of(entry(0), 0);
     float4_t q[NF];
 #pragma unroll
@@ -832,12 +848,15 @@ __global__ __launch_bounds__(64 * NW) void attention_rows_kernel(AttnArgsF a) {
             for (int i = 0; i < NF; ++i) { kk[u][i] = kr[l16 + 16 * i]; vv[u][i] = vr[l16 + 16 * i]; }
         }
     };
-    float m = -INFINITY, l = 0.f;
-    float4_t o[NF];
+    struct Sums { float m, l; float4_t o[NF]; } even, odd;
+    auto clear = [&](Sums &e) {
+        e.m = -INFINITY; e.l = 0.f;
 #pragma unroll
-    for (int i = 0; i < NF; ++i) o[i] = (float4_t){0.f, 0.f, 0.f, 0.f};
-    auto consume = [&](const float4_t (&kk)[KB][NF], const float4_t (&vv)[KB][NF], int j0) {
-        float s[KB], top = m;
+        for (int i = 0; i < NF; ++i) e.o[i] = (float4_t){0.f, 0.f, 0.f, 0.f};
+    };
+    clear(even); clear(odd);
+    auto consume = [&](Sums &e, const float4_t (&kk)[KB][NF], const float4_t (&vv)[KB][NF], int j0) {
+        float s[KB], top = e.m;
 #pragma unroll
         for (int u = 0; u < KB; ++u) {
             float d = 0.f;
@@ -849,58 +868,62 @@ __global__ __launch_bounds__(64 * NW) void attention_rows_kernel(AttnArgsF a) {
             top = fmaxf(top, s[u]);
         }
         const float ref = top == -INFINITY ? 0.f : top;                  // (nothing seen yet, or scores of -inf alone: their weights are 0, not exp(-inf + inf))
-        const float keep = expf(m - ref);
-        m = top; l *= keep;
+        const float keep = expf(e.m - ref);
+        e.m = top; e.l *= keep;
 #pragma unroll
         for (int i = 0; i < NF; ++i)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) o[i][c] *= keep;
+            for (int c = 0; c < 4; ++c) e.o[i][c] *= keep;
 #pragma unroll
         for (int u = 0; u < KB; ++u) {
             const bool live = j0 + u * STEP < ctx;
             const float p = live ? expf(s[u] - ref) : 0.f;
-            l += p;
+            e.l += p;
 #pragma unroll
             for (int i = 0; i < NF; ++i)
 #pragma unroll
-                for (int c = 0; c < 4; ++c) o[i][c] = fmaf(p, live ? vv[u][i][c] : 0.f, o[i][c]);
+                for (int c = 0; c < 4; ++c) e.o[i][c] = fmaf(p, live ? vv[u][i][c] : 0.f, e.o[i][c]);
         }
     };
-    request(k, v, ea, group);
-    if (ROUND < ctx) request(kn, vn, eb, group + ROUND);                 // (uniform conditions from here on: the groups of a wave stay together)
-    for (int r0 = 0;; r0 += 2 * ROUND) {
-        const bool third = r0 + 2 * ROUND < ctx, fourth = r0 + 3 * ROUND < ctx;
+    request(k, v, ea, first + group);
+    if (first + NEXT < ctx) request(kn, vn, eb, first + NEXT + group);   // (conditions of the wave from here on: its groups stay together)
+    for (int r0 = first;; r0 += 2 * NEXT) {
+        const bool third = r0 + 2 * NEXT < ctx, fourth = r0 + 3 * NEXT < ctx;
         if (third)
 #pragma unroll
-            for (int u = 0; u < KB; ++u) { ea[u] = entry(r0 + 2 * ROUND + group + u * STEP); eb[u] = entry(r0 + 3 * ROUND + group + u * STEP); }
-        consume(k, v, r0 + group);
-        if (third) request(k, v, ea, r0 + 2 * ROUND + group);
-        if (r0 + ROUND >= ctx) break;
-        consume(kn, vn, r0 + ROUND + group);
+            for (int u = 0; u < KB; ++u) { ea[u] = entry(r0 + 2 * NEXT + group + u * STEP); eb[u] = entry(r0 + 3 * NEXT + group + u * STEP); }
+        consume(even, k, v, r0 + group);
+        if (third) request(k, v, ea, r0 + 2 * NEXT + group);
+        if (r0 + NEXT >= ctx) break;
+        consume(NW == 8 ? even : odd, kn, vn, r0 + NEXT + group);
         if (!third) break;
-        if (fourth) request(kn, vn, eb, r0 + 3 * ROUND + group);
+        if (fourth) request(kn, vn, eb, r0 + 3 * NEXT + group);
     }
     // the four groups of the wave, then the waves
-    float top = fmaxf(m, __shfl_xor(m, 16, 64));
-    top = fmaxf(top, __shfl_xor(top, 32, 64));
-    const float w = expf(m - (top == -INFINITY ? 0.f : top));
-    l = xor16_partner_sum(xor32_partner_sum(l * w));
+    auto merge = [&](Sums &e, int w8) {
+        float top = fmaxf(e.m, __shfl_xor(e.m, 16, 64));
+        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        const float w = expf(e.m - (top == -INFINITY ? 0.f : top));
+        e.l = xor16_partner_sum(xor32_partner_sum(e.l * w));
 #pragma unroll
-    for (int i = 0; i < NF; ++i) {
+        for (int i = 0; i < NF; ++i) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) o[i][c] = xor16_partner_sum(xor32_partner_sum(o[i][c] * w));
-        if (lane < 16) reinterpret_cast<float4_t *>(part[wave])[l16 + 16 * i] = o[i];
-    }
-    if (lane == 0) { pm[wave] = top; pl[wave] = l; }
+            for (int c = 0; c < 4; ++c) e.o[i][c] = xor16_partner_sum(xor32_partner_sum(e.o[i][c] * w));
+            if (lane < 16) reinterpret_cast<float4_t *>(part[w8])[l16 + 16 * i] = e.o[i];
+        }
+        if (lane == 0) { pm[w8] = top; pl[w8] = e.l; }
+    };
+    merge(even, wave);
+    if (NW == 4) merge(odd, wave + 4);
     __syncthreads();
     float mx = pm[0];
 #pragma unroll
-    for (int i = 1; i < NW; ++i) mx = fmaxf(mx, pm[i]);
+    for (int i = 1; i < 8; ++i) mx = fmaxf(mx, pm[i]);
     const float ref = mx == -INFINITY ? 0.f : mx;
     for (int d = threadIdx.x; d < D; d += 64 * NW) {
         float sum = 0.f, acc = 0.f;
 #pragma unroll
-        for (int i = 0; i < NW; ++i) { const float e = expf(pm[i] - ref); sum = fmaf(e, pl[i], sum); acc = fmaf(e, part[i][d], acc); }
+        for (int i = 0; i < 8; ++i) { const float e = expf(pm[i] - ref); sum = fmaf(e, pl[i], sum); acc = fmaf(e, part[i][d], acc); }
         a.out[((int64_t)t * a.H + hd) * D + d] = acc / sum;
     }
 }
@@ -919,8 +942,8 @@ int attention(const AttnArgsF &a, bool paged, hipStream_t s) {
     const size_t lds = ((size_t)a.max_ctx + 5 * (size_t)a.D + 8) * 4;
     if (lds > 160 * 1024) return nvr::fail(NVR_ERR_UNSUPPORTED, "f32 attention: context %d does not fit the score buffer (%zu bytes of LDS)", a.max_ctx, lds);
     const dim3 grid((unsigned)a.nq, (unsigned)a.H);
-    // rows in 16-byte pieces: a multiple of 64 of them per head, everything aligned to them; eight waves share a query row's keys while the rows are few
-    // (a decode step), four from a CU's worth of rows on (a prompt: the rows themselves fill the chip)
+    // rows in 16-byte pieces: a multiple of 16 of them per head, everything aligned to them; eight waves share a query row's keys while there are less than two rows of workgroups per CU (eight
+    // waves in place of four cost a step of 64 prompt rows 2.76 against 2.61 ms, four in place of eight a sequence of 4096 keys 3.62 against 3.04); the same bits either way
     const bool pieces = a.D % 64 == 0 && a.ldq % 4 == 0 && (paged || a.ldkv % 4 == 0) && (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) & 15) == 0;
     if (pieces) {
         const bool few = (int64_t)a.nq * a.H < 512;

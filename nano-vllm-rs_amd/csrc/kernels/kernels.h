@@ -100,8 +100,9 @@ int rmsnorm(const float *x, const float *w, float eps, int64_t T, int64_t Hd, fl
 int add_rmsnorm(float *h, const float *y, const float *w, float eps, int64_t T, int64_t Hd, float *out, hipStream_t s);
 int sum_ranks_add_rmsnorm(float *h, const float *parts, int nranks, int64_t stride, const float *w, float eps, int64_t T, int64_t Hd, float *out, hipStream_t s);
 int linear(const float *x, int64_t ldx, const float *W, int64_t T, int64_t K, int64_t N, const float *bias, float *y, hipStream_t s);
-int linear_splitk_parts(int64_t T, int64_t K, int64_t N, int64_t ldx);   // parts of k worth taking (1: none)
-int linear_splitk(const float *x, int64_t ldx, const float *W, int64_t T, int64_t K, int64_t N, int64_t S, float *parts, hipStream_t s);   // parts [S][T][N]
+int linear_segments(int64_t K, int64_t N, int64_t ldx);   // segments of k a row-parallel product of more than 8 rows is summed in (1: none)
+bool linear_segments_apart(int64_t T, int64_t N, int64_t S);   // whether a step of T rows runs them in workgroups of their own, as far as [S][T][N] fits the caller's slabs
+int linear_segmented(const float *x, int64_t ldx, const float *W, int64_t T, int64_t K, int64_t N, int64_t S, bool apart, float *y, hipStream_t s);   // y: [T][N], apart: [S][T][N], to be added up in their order
 int rope_store_kv(float *qkv, const int64_t *pos, const int32_t *slots, int64_t T, int64_t H, int64_t KVH, int64_t D, const float *cos_t,
                   const float *sin_t, float *kc, float *vc, const float *q_norm, const float *k_norm, float eps, hipStream_t s);
 int silu_and_mul(const float *gu, int64_t T, int64_t I, float *out, hipStream_t s);

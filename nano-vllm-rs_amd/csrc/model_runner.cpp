@@ -131,7 +131,7 @@ int nvr_model_runner::init() {                                       // ModelRun
     // (rows of a STEP, prefill steps included: sized by max_seqs alone, a prefill of 257..1024 tokens on an engine of few sequences lost the split-k route
     //  and fell to 9-12 row blocks of the streaming kernel — Qwen3-0.6B, 8 sequences: 257 tokens 2.38 ms against 1.49 ms for 256; scratch/prefill_scan.py)
     slab_rows = std::max<int64_t>(64, std::min<int64_t>(1024, std::max<int64_t>({max_seqs, max_tokens, 256})));
-    RC(dmalloc(&slabs, 4 * slab_rows * Hd));
+    RC(dmalloc(&slabs, (f32 ? 8 : 4) * slab_rows * Hd));
     { int v = 0; if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && v > 0) num_cus = v; }
     allow_missing_comm = env.tp_no_comm;                                               // compute-only profiling of one rank
     if (!env.tp_graph && tp > 1) graphs_disabled = true;
@@ -284,16 +284,20 @@ int nvr_model_runner::gen_weights_f32() {
     return NVR_OK;
 }
 
+// a row-parallel product of more than 8 rows on one rank without biases: its segments of k (from the shape alone), in `slabs` where they run apart (returns their number) or added up in
+// `proj` (returns 1): the same bits either way
+int nvr_model_runner::row_parallel_f32(const float *x, int64_t K, const float *W, const float *bias, int64_t T, bool cut, int64_t *parts) {
+    namespace kf = nvr::kf;
+    const int64_t S = cut && T > 8 ? kf::linear_segments(K, Hd, K) : 1;
+    const bool apart = S > 1 && S * T <= 8 * slab_rows && kf::linear_segments_apart(T, Hd, S);
+    *parts = apart ? S : 1;
+    if (S == 1) return kf::linear(x, K, W, T, K, Hd, bias, reinterpret_cast<float *>(proj), stream);
+    return kf::linear_segmented(x, K, W, T, K, Hd, S, apart, apart ? slabs : reinterpret_cast<float *>(proj), stream);
+}
 // RowParallelLinear's exchange on the float32 path (linear.rs:236-238) + residual + RMSNorm: every rank's f32 partial sums [T, hidden] are
 // gathered (the communicator's all-gather: the one-shot arenas for decode-sized rows — bytes are moved, never summed there —, RCCL or the
 // in-process rendezvous otherwise), then summed in RANK ORDER in f32, added to the residual stream and normalised by one kernel: every rank holds
 // the same bits, equal to the f32 oracle's tensor-parallel sum.  One rank: the plain add + RMSNorm.
-// parts of k of a row-parallel product of this step: what the kernel finds worth taking, as far as the slab buffer holds them
-int64_t nvr_model_runner::splitk_parts_f32(int64_t T, int64_t K) const {
-    int64_t S = nvr::kf::linear_splitk_parts(T, K, Hd, K);
-    while (S > 1 && S * T > 4 * slab_rows) S /= 2;
-    return S;
-}
 // parts > 1: the product left its partial sums in `slabs` (one rank): added up in their order like ranks' sums are
 int nvr_model_runner::row_parallel_norm_f32(int64_t T, const float *wn, int64_t parts) {
     namespace kf = nvr::kf;
@@ -351,11 +355,9 @@ int nvr_model_runner::forward_f32(int64_t T, int64_t B, bool is_prefill, int64_t
             if (is_prefill) a.seq_of_q = d_kvbase;
         }
         RC(kf::attention(a, paged, st));
-        // (a prompt on one rank, plain projections: few output tiles are split along k, and the add + norm behind them sums the parts: row_parallel_norm_f32)
         const bool cut = !ride && !comm.active() && tp == 1 && !mc.use_bias;
-        int64_t S = cut ? splitk_parts_f32(T, H * D) : 1;
-        if (S > 1) RC(kf::linear_splitk(fa, H * D, F(w.o), T, H * D, Hd, S, slabs, st));
-        else RC(kf::linear(fa, H * D, F(w.o), T, H * D, Hd, w.o_b ? F(w.o_b) : nullptr, fp, st));
+        int64_t S;
+        RC(row_parallel_f32(fa, H * D, F(w.o), w.o_b ? F(w.o_b) : nullptr, T, cut, &S));
         if (ride) {                                                                                  // residual :382, norm :385, K12 + K13: one launch
             RC(kf::add_norm_linear_silu_mul(hc, fp, F(w.ln2), mc.rms_norm_eps, hn, F(w.gate_up), T, Hd, I, w.gate_up_b ? F(w.gate_up_b) : nullptr, fact, st));
             std::swap(hc, hn);
@@ -368,9 +370,7 @@ int nvr_model_runner::forward_f32(int64_t T, int64_t B, bool is_prefill, int64_t
             RC(kf::silu_and_mul(fg, T, I, fact, st));
         }
         }
-        S = cut ? splitk_parts_f32(T, I) : 1;
-        if (S > 1) RC(kf::linear_splitk(fact, I, F(w.down), T, I, Hd, S, slabs, st));
-        else RC(kf::linear(fact, I, F(w.down), T, I, Hd, w.down_b ? F(w.down_b) : nullptr, fp, st));
+        RC(row_parallel_f32(fact, I, F(w.down), w.down_b ? F(w.down_b) : nullptr, T, cut, &S));
         if (ride && l + 1 < L && !layers[l + 1].q_norm && !layers[l + 1].k_norm) owed = true;        // residual :389 + next norm :378: on the next layer's qkv launch
         else if (ride) RC(kf::add_rmsnorm(hc, fp, F(l + 1 < L ? layers[l + 1].ln1 : norm), mc.rms_norm_eps, T, Hd, fn, st));
         else RC(row_parallel_norm_f32(T, F(l + 1 < L ? layers[l + 1].ln1 : norm), S));                   // (exchange,) residual :389, next norm :378 / :501

@@ -58,7 +58,7 @@ struct nvr_model_runner {
              *nlast = nullptr;
     float *logits = nullptr; void *attn_ws = nullptr; size_t attn_ws_bytes = 0;
     unsigned int *attn_tickets = nullptr;  // [max_seqs * KVH] arrival counters of the split-KV decode attention (fused merge; zero between launches)
-    float *slabs = nullptr;                // split-k partials of o_proj / down_proj: [S][T][Hd] f32, S * T <= 4 * slab_rows
+    float *slabs = nullptr;                // split-k partials of o_proj / down_proj: [S][T][Hd] f32, S * T <= 4 * slab_rows (float32 runners: 8 * slab_rows)
     // step inputs: one pinned host arena mirrored by one device arena
     char *in_host = nullptr, *in_dev = nullptr; size_t in_bytes = 0;
     int64_t *d_ids = nullptr, *d_pos = nullptr; int32_t *d_slots = nullptr, *d_cu = nullptr, *d_ctx = nullptr,
@@ -143,7 +143,7 @@ private:
     int gen_weights_f32();
     int forward_f32(int64_t T, int64_t B, bool is_prefill, int64_t max_ctx);
     int row_parallel_norm_f32(int64_t T, const float *wn, int64_t parts = 1);
-    int64_t splitk_parts_f32(int64_t T, int64_t K) const;
+    int row_parallel_f32(const float *x, int64_t K, const float *W, const float *bias, int64_t T, bool cut, int64_t *parts);
     float *f32_h2 = nullptr;                             // float32, one rank: second residual-stream buffer [8][hidden] of the decode-sized steps whose add + norm
                                                          // rides on the consumer GEMV (the workgroups of that launch still read the first while one of them writes)
     float *f32_gather = nullptr; int64_t f32_gather_rows = 0;   // float32 tensor-parallel ranks: every rank's partial sums [tp][f32_gather_rows][hidden], a piece of the step's rows at a time

@@ -190,6 +190,40 @@ def test_float32_prompt_products_cut_along_k(T, hidden, inter):
     assert np.abs(p.model_runner.logits(1) - orec["logits"]).max() < 2e-4
 
 
+@pytest.mark.parametrize("hidden,inter,heads,kv,dim", [(1024, 3072, 16, 8, 128),       # o / down in 8 segments of k
+                                                       (512, 1024, 4, 2, 64),          # in 1 and 4
+                                                       (768, 2560, 4, 1, 192)])        # in 2 and 4; heads of three pieces
+def test_float32_prompt_rows_have_the_same_bits_in_every_step(hidden, inter, heads, kv, dim):
+    """A float32 prompt alone, in portions, beside another prompt and in engines of other sizes: steps of few and many rows, whose products' segments run apart or one after the other and whose
+    rows' keys are shared by eight waves or four.  The last row's logits have the same bits (portions of more than 8 rows: fewer run the decode step's products)."""
+    model = nvr.ModelConfig(vocab_size=256, hidden_size=hidden, intermediate_size=inter, num_hidden_layers=2, num_attention_heads=heads, num_key_value_heads=kv, head_dim=dim,
+                            max_position_embeddings=2048, rms_norm_eps=1e-6, rope_theta=1e4, tie_word_embeddings=0, init_std=hidden ** -0.5, seed=5)
+    sp = nvr.SamplingParams(temperature=0.0, ignore_eos=True)
+
+    def last_row(lengths, cuts=(), budget=4096, seqs=2):
+        r = nvr.ModelRunner(nvr.Config(skip_block_size_check=1, max_num_seqs=seqs, max_num_batched_tokens=budget, max_model_len=2048, kvcache_block_size=16, num_kvcache_blocks=256,
+                                       dtype="float32", enable_chunked_prefill=1), model)
+        bm = nvr.BlockManager(256, 16)
+        group = [nvr.Sequence(nvr.synthetic_tokens(L, 6, i, 256), sp, 16) for i, L in enumerate(lengths)]
+        for s in group:
+            bm.allocate(s)
+        done = 0
+        for c in cuts:                                                       # portions of the first prompt, alone
+            group[0].set_chunk(done, c - done)
+            r.execute_model(group[:1], True)
+            done = c
+        if cuts:
+            group[0].set_chunk(done, lengths[0] - done)
+        r.execute_model(group, True)
+        return r.logits(len(group))[0].copy()
+    for T in (33, 200, 700):
+        whole = last_row([T])
+        assert np.isfinite(whole).all() and whole.std() > 0
+        for other in (dict(lengths=[T], cuts=[9]), dict(lengths=[T], cuts=[T - 20]), dict(lengths=[T], cuts=[T // 3, 2 * T // 3]), dict(lengths=[T, 300]), dict(lengths=[T, 900], cuts=[T - 9]),
+                      dict(lengths=[T], budget=max(T, 64), seqs=1)):
+            assert np.array_equal(last_row(**other), whole), (T, other)
+
+
 @pytest.mark.parametrize("W,taps,heads,kv,dim,lengths", [(64, 1, 4, 2, 64, [1, 31, 32]), (1024, 4, 2, 1, 64, [33, 127]), (1040, 4, 4, 1, 128, [30, 255, 256]), (2080, 8, 4, 4, 64, [3, 129]),
                                                          (4160, 3, 4, 2, 64, [5]), (96, 9, 2, 2, 64, [40, 7]), (256, 4, 4, 2, 64, [20] * 66)])
 def test_layer_list_decode_steps(W, taps, heads, kv, dim, lengths):
