@@ -29,13 +29,13 @@
 
 namespace nvr { namespace NVR_DT_NS {
 
-enum { EPI_F16 = 0, EPI_F32 = 1, EPI_SILU = 2, EPI_ROPE = 3, EPI_SLAB = 4 };
+enum { EPI_F16 = 0, EPI_F32 = 1, EPI_SILU = 2, EPI_ROPE = 3, EPI_SLAB = 4, EPI_CLAMP = 5 };
 // rows up to which a decode step's add + norm rides on the product behind it: every workgroup reads every row's slabs again (16 KB a row at K = 1024), so the launch it saves pays for one
 // or two rows — Qwen3-0.6B at 300 keys, us a step apart / riding: 802 / 769 at one row, 822 / 800 at two, 851 / 890 at four
 constexpr int64_t NORM_ROWS = 2;
 
 struct LinEpi {
-    // EPI_SILU: N is the intermediate size I; W holds gate rows [0,I) and up rows [I,2I)
+    // EPI_SILU, EPI_CLAMP: N is the intermediate size I; W holds gate rows [0,I) and up rows [I,2I)
     // EPI_ROPE: qkv output [T, (H+2KVH)*D] + caches
     const int64_t *pos; const int32_t *slots; const float *cos_t, *sin_t;
     half_t *kc, *vc;
@@ -44,15 +44,19 @@ struct LinEpi {
     int32_t kslice; int64_t slab_stride;
     // W is the TILED copy [N/16][K/32][16][32] (retile_weight): one wave-instruction reads 1 KiB contiguous
     int32_t tiled;
-    int32_t gelu;                          // EPI_SILU: 1 gelu (tanh form) instead of silu, 2 the clamped unit below; EPI_F16: gelu (error function) of the product
-    float limit, alpha; int64_t ldy;       // EPI_SILU with gelu == 2: min(g, limit) sigmoid(alpha min(g, limit)) (clamp(u, +-limit) + 1); row stride of y (0: I)
-    NormIn norm;                           // NORM instances: x is formed by the workgroup itself
+    int32_t gelu;                          // EPI_SILU: gelu (tanh form) instead of silu; EPI_F16: gelu (error function) of the product
 };
+// What single instances need beyond it stays out of the others' arguments
+struct LinEpiNorm : LinEpi { NormIn norm; };                       // NORM instances: x is formed by the workgroup itself
+struct LinEpiClamp : LinEpi { float limit, alpha; int64_t ldy; };  // EPI_CLAMP: min(g, limit) sigmoid(alpha min(g, limit)) (clamp(u, +-limit) + 1); row stride of y
+template <int EPI, bool NORM> struct LinArgs { using type = LinEpi; };
+template <int EPI> struct LinArgs<EPI, true> { using type = LinEpiNorm; };
+template <> struct LinArgs<EPI_CLAMP, false> { using type = LinEpiClamp; };
 
 // W row handled by local row r (0..15) of n-tile i of workgroup bx
 template <int EPI>
 __device__ __forceinline__ int w_row(int bx, int i, int NT, int r, int N, const LinEpi &e) {
-    if (EPI == EPI_SILU) return (i == 0 ? 0 : N) + bx * 16 + r;             // N == I here
+    if (EPI == EPI_SILU || EPI == EPI_CLAMP) return (i == 0 ? 0 : N) + bx * 16 + r;             // N == I here
     if (EPI == EPI_ROPE) {
         const int tph = e.D / 16, head = bx / tph, c = bx % tph;            // tiles per head
         if (head < e.H + e.KVH) return head * e.D + (r < 8 ? c * 8 + r : e.D / 2 + c * 8 + (r - 8));
@@ -69,7 +73,7 @@ constexpr int NORM_ELEMS = 4096;
 template <int NT, int MT, int WAVES, int EPI, bool NORM = false>
 __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t *__restrict__ x, int64_t ldx,
                                                                    const half_t *__restrict__ W, int T, int K, int N,
-                                                                   void *__restrict__ y, LinEpi epi) {
+                                                                   void *__restrict__ y, typename LinArgs<EPI, NORM>::type epi) {
     constexpr int U = 4;                                    // k-steps in flight per wave
     extern __shared__ __attribute__((aligned(16))) char norm_lds[];   // NORM: the normalised rows [T][K + 8]
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -83,8 +87,8 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
         if (epi.tiled) {
             // tile index in the tiled copy: SiLU — gate tile bx, up tile I/16 + bx; RoPE — tile bx of the permuted row order;
             // else tile bx*NT + i (clamped like w_row clamps its rows)
-            int64_t tile = EPI == EPI_SILU ? (i == 0 ? (int64_t)blockIdx.x : (int64_t)(N / 16) + blockIdx.x) : (int64_t)blockIdx.x * NT + i;
-            if (EPI != EPI_SILU && EPI != EPI_ROPE && tile > N / 16 - 1) tile = N / 16 - 1;
+            int64_t tile = EPI == EPI_SILU || EPI == EPI_CLAMP ? (i == 0 ? (int64_t)blockIdx.x : (int64_t)(N / 16) + blockIdx.x) : (int64_t)blockIdx.x * NT + i;
+            if (EPI != EPI_SILU && EPI != EPI_CLAMP && EPI != EPI_ROPE && tile > N / 16 - 1) tile = N / 16 - 1;
             wrow[i] = W + tile * (int64_t)(K / 32) * 512 + r * 32 + q * 8;
         } else wrow[i] = W + (int64_t)w_row<EPI>(blockIdx.x, i, NT, r, N, epi) * K + q * 8;
     }
@@ -241,7 +245,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
                 }
             }
         }
-    } else if (EPI == EPI_SILU) {
+    } else if (EPI == EPI_SILU || EPI == EPI_CLAMP) {
         // tiles (0,j) = gate, (1,j) = up for the same 16 columns: act = fp16(silu(fp16 g) * fp16 u)
         for (int j = wave; j < MT; j += WAVES) {
             const float4_t g4 = reduce(j), u4 = reduce(MT + j);
@@ -251,7 +255,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float gf = (float)to_half_rn(g4[e]), uf = (float)to_half_rn(u4[e]);
-                    if (epi.gelu == 2) {
+                    if constexpr (EPI == EPI_CLAMP) {
                         const float g = fminf(gf, epi.limit), u = fminf(fmaxf(uf, -epi.limit), epi.limit);
                         h[e] = to_half_rn(g / (1.0f + expf(-epi.alpha * g)) * (u + 1.0f));
                     } else {
@@ -259,7 +263,8 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
                         h[e] = to_half_rn(__fmul_rn(__fmul_rn(gf, sg), uf));
                     }
                 }
-                *reinterpret_cast<half4_t *>(reinterpret_cast<half_t *>(y) + (int64_t)m * (epi.ldy ? epi.ldy : N) + n) = h;
+                if constexpr (EPI == EPI_CLAMP) *reinterpret_cast<half4_t *>(reinterpret_cast<half_t *>(y) + (int64_t)m * epi.ldy + n) = h;
+                else *reinterpret_cast<half4_t *>(reinterpret_cast<half_t *>(y) + (int64_t)m * N + n) = h;
             }
         }
     } else {   // EPI_ROPE: NT == 1
@@ -308,7 +313,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
 }
 
 template <int NT, int MT, int WAVES, int EPI>
-static void launch(const half_t *x, int64_t ldx, const half_t *W, int T, int K, int N, void *y, const LinEpi &e,
+static void launch(const half_t *x, int64_t ldx, const half_t *W, int T, int K, int N, void *y, const typename LinArgs<EPI, false>::type &e,
                    unsigned gx, hipStream_t s, unsigned gz = 1) {
     dim3 grid(gx, (unsigned)((T + 16 * MT - 1) / (16 * MT)), gz);
     linear_skinny_kernel<NT, MT, WAVES, EPI><<<grid, dim3(WAVES * 64), 0, s>>>(x, ldx, W, T, K, N, y, e);
@@ -480,17 +485,17 @@ bool linear_clamped_glu_ok(const half_bits *x, int64_t ldx, int64_t T, int64_t K
 int linear_clamped_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, float limit, float alpha, half_bits *out, int64_t ldo, hipStream_t s) {
     if (!linear_clamped_glu_ok(x, ldx, T, K, I, out, ldo)) return nvr::fail(NVR_ERR_UNSUPPORTED, "linear_clamped_glu: T=%ld K=%ld I=%ld", (long)T, (long)K, (long)I);
     if (T == 0) return 0;
-    LinEpi e{};
-    e.gelu = 2; e.limit = limit; e.alpha = alpha; e.ldy = ldo;
+    LinEpiClamp e{};
+    e.limit = limit; e.alpha = alpha; e.ldy = ldo;
     const unsigned gx = (unsigned)(I / 16);
     const half_t *xx = (const half_t *)x, *ww = (const half_t *)W;
     const int wv = waves_for(K);
     if (T <= 16 || I / 16 < 128) {
-        if (wv >= 8) launch<2, 1, 8, EPI_SILU>(xx, ldx, ww, (int)T, (int)K, (int)I, out, e, gx, s);
-        else launch<2, 1, 4, EPI_SILU>(xx, ldx, ww, (int)T, (int)K, (int)I, out, e, gx, s);
+        if (wv >= 8) launch<2, 1, 8, EPI_CLAMP>(xx, ldx, ww, (int)T, (int)K, (int)I, out, e, gx, s);
+        else launch<2, 1, 4, EPI_CLAMP>(xx, ldx, ww, (int)T, (int)K, (int)I, out, e, gx, s);
     } else {
-        if (wv >= 8) launch<2, 2, 8, EPI_SILU>(xx, ldx, ww, (int)T, (int)K, (int)I, out, e, gx, s);
-        else launch<2, 2, 4, EPI_SILU>(xx, ldx, ww, (int)T, (int)K, (int)I, out, e, gx, s);
+        if (wv >= 8) launch<2, 2, 8, EPI_CLAMP>(xx, ldx, ww, (int)T, (int)K, (int)I, out, e, gx, s);
+        else launch<2, 2, 4, EPI_CLAMP>(xx, ldx, ww, (int)T, (int)K, (int)I, out, e, gx, s);
     }
     return launch_check("linear_clamped_glu");
 }
@@ -533,8 +538,10 @@ int linear_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, i
 // ---- products of a decode step of few rows whose workgroups form RMSNorm(h + slabs) themselves (linear_skinny_kernel, NORM)
 bool norm_linear_ok(int64_t T, int64_t K, int64_t S) { return T >= 1 && T <= NORM_ROWS && K % 256 == 0 && T * K <= NORM_ELEMS && (S == 2 || S == 4); }
 template <int NT, int EPI>
-static int norm_launch(const NormIn &nm, const half_bits *W, int64_t T, int64_t K, int64_t N, void *y, LinEpi e, int64_t gx, bool tiled, hipStream_t s, const char *what) {
+static int norm_launch(const NormIn &nm, const half_bits *W, int64_t T, int64_t K, int64_t N, void *y, const LinEpi &le, int64_t gx, bool tiled, hipStream_t s, const char *what) {
     if (!norm_linear_ok(T, K, nm.S)) return nvr::fail(NVR_ERR_UNSUPPORTED, "%s: T=%ld K=%ld, %d slabs", what, (long)T, (long)K, nm.S);
+    LinEpiNorm e{};
+    static_cast<LinEpi &>(e) = le;
     e.norm = nm; e.tiled = tiled;
     linear_skinny_kernel<NT, 1, 8, EPI, true><<<dim3((unsigned)gx), dim3(512), (size_t)(T * (K + 8) * 2), s>>>(nullptr, 0, (const half_t *)W, (int)T, (int)K, (int)N, y, e);
     return launch_check(what);
