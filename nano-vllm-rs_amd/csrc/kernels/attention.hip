@@ -698,6 +698,13 @@ static inline int parts_for(int64_t nq, int64_t KVH, int64_t max_ctx, int waves,
     return (int)((max_ctx + ps - 1) / ps);
 }
 
+// Longest context of up to 128 pairs that one workgroup per pair takes without partitions: a round of 128 keys and half a chunk.  A second round costs more than the partitions' hand-off
+// does from about 144 keys on while there are enough CUs for the partitions; from 129 pairs on the partitions fill the chip more than once and it pays up to 256 keys.  Groups of 8 merge
+// for longer than they stream.  Qwen3-0.6B (8 kv heads), us a step in partitions / without: 1 sequence of 128 keys 728 / 716, 136 735 / 734, 144 741 / 739, 152 740 / 754, 201 736 / 778;
+// 4 sequences of 128 816 / 786, 201 822 / 853; 16 of 128 932 / 881, 251 952 / 973; 17 of 251 1026 / 995, 23 1080 / 1044.  8 groups of 4 heads, us a launch: 128 keys 6.3 / 6.1, 140 6.7 / 6.9;
+// of 8 heads: 128 keys 9.0 / 10.1
+int64_t attn_brief_context(int64_t nq, int64_t H, int64_t KVH) { return nq * KVH <= 128 && H <= 4 * KVH ? 136 : 0; }
+
 size_t attn_workspace_bytes(int64_t nq, int64_t H, int64_t D, int64_t max_ctx) {
     int64_t max_parts = (max_ctx + 63) / 64;
     if (max_parts > 1024) max_parts = 1024;
@@ -809,10 +816,9 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
             part_size = (int)ps; np = (int)((mc + ps - 1) / ps);
         } else np = parts_for(a.nq, a.KVH, mc, waves, &part_size);
     }
-    // Few pairs over short contexts (a chat's first hundreds of tokens): the partitions' hand-off — partials out, a ticket, partials back — costs more than the keys: ONE workgroup of
-    // eight waves per pair, whose 128 keys per round need two rounds for the 256-token bucket, the second requested under the
-    // first.  Qwen3-0.6B at 128 keys, us a step: 903 -> 860 at 9 sequences, 948 -> 917 at 16
-    const bool brief = paged && a.workspace && !shared && mc <= 256 && pairs < 192;
+    // Few pairs over short contexts (a chat's first hundred tokens): the partitions' hand-off — partials out, a ticket, partials back — costs more than the keys: ONE workgroup of
+    // eight waves per pair, whose round is 128 keys (attn_brief_context).
+    const bool brief = paged && a.workspace && !shared && mc <= (pairs <= 128 ? attn_brief_context(a.nq, a.H, a.KVH) : pairs < 192 ? 256 : 0);
     if (brief) { np = 1; waves = 8; }
     // Work-balanced form (attn_share_kernel): a pair count whose last round of one-workgroup-per-pair launches would be mostly empty — 257..2047 pairs with
     // >= 15 % of the rounds' slots unused (33..37 and 65..74 sequences at 8 kv heads, ...), contexts long enough for the stream to matter — or a RAGGED batch

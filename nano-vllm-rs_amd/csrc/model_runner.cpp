@@ -740,7 +740,12 @@ int64_t nvr_model_runner::shared_prefix_plan(nvr_seq *const *seqs, size_t nseq, 
 
 // a captured decode step is a function of (batch size, context bucket, shared-prefix length, whole batch or a group of it, logits wanted)
 static inline uint64_t graph_key(bool want_logits, size_t nseq, int64_t bucket, int64_t shared_len, bool group, bool ragged) {
-    return ((uint64_t)want_logits << 63) | ((uint64_t)group << 62) | ((uint64_t)ragged << 61) | ((uint64_t)nseq << 44) | ((uint64_t)(shared_len / 64) << 24) | (uint64_t)(bucket / 256);
+    return ((uint64_t)want_logits << 63) | ((uint64_t)group << 62) | ((uint64_t)ragged << 61) | ((uint64_t)nseq << 44) | ((uint64_t)(shared_len / 64) << 24) | (uint64_t)(bucket / 256);   // (0: the brief contexts in front of the first 256)
+}
+// the bound on the contexts a decode step is captured for: multiples of 256, and the brief contexts of few sequences, whose attention takes another form
+int64_t nvr_model_runner::context_bucket(size_t nseq, int64_t max_ctx) const {
+    const int64_t brief = f32 || decode_shared_len > 0 ? 0 : KD(attn_brief_context((int64_t)nseq, H, KVH));
+    return max_ctx <= brief ? brief : (max_ctx + 255) / 256 * 256;
 }
 // A decode batch whose contexts are ragged: the attention launch sizes every (sequence, kv head) pair's partitions by the LONGEST context of the step (its bucket, under
 // a captured graph): the short sequences' workgroups idle (or finish early) while the long ones stream — the work-balanced launch (attn_share_kernel) cuts the keys
@@ -1163,7 +1168,7 @@ int nvr_model_runner::execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill
     }
 
     // decode: replay a hipGraph captured per (batch size, context bucket) — execute_with_cuda_graph :303-326
-    const int64_t bucket = (max_ctx + 255) / 256 * 256;
+    const int64_t bucket = context_bucket(nseq, max_ctx);
     const uint64_t key = graph_key(want_logits, nseq, bucket, decode_shared_len, decode_shared_len > 0 && decode_shared_rows < (int64_t)nseq, decode_ragged);
     auto it = graphs.find(key);
     if (it == graphs.end()) {
@@ -1231,7 +1236,7 @@ int nvr_model_runner::execute_decode_ahead(nvr_seq *const *seqs, size_t nseq, in
     want_logits = !lazy_logits; logits_valid = want_logits; lm_input = n;
     const int64_t T = (int64_t)nseq;
     if (cfg.enforce_eager || graphs_disabled) return forward(T, T, false, max_ctx);
-    const int64_t bucket = (max_ctx + 255) / 256 * 256;
+    const int64_t bucket = context_bucket(nseq, max_ctx);
     const uint64_t key = graph_key(want_logits, nseq, bucket, decode_shared_len, decode_shared_len > 0 && decode_shared_rows < (int64_t)nseq, decode_ragged);
     auto it = graphs.find(key);
     if (it == graphs.end()) {

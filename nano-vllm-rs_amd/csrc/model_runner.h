@@ -142,6 +142,7 @@ private:
     int gen_weights();
     int gen_weights_f32();
     int forward_f32(int64_t T, int64_t B, bool is_prefill, int64_t max_ctx);
+    int64_t context_bucket(size_t nseq, int64_t max_ctx) const;
     int row_parallel_norm_f32(int64_t T, const float *wn, int64_t parts = 1);
     int row_parallel_f32(const float *x, int64_t K, const float *W, const float *bias, int64_t T, bool cut, int64_t *parts);
     float *f32_h2 = nullptr;                             // float32, one rank: second residual-stream buffer [8][hidden] of the decode-sized steps whose add + norm

@@ -329,6 +329,45 @@ def _work_balanced_against_per_pair(B, G, KVH, D, bs, ctx, bound, launches):
         assert not tickets.to_numpy((B * KVH,), np.uint32).any()
 
 
+@pytest.mark.parametrize("B,G,KVH,D,bs,ctx,bound", [
+    (1, 2, 8, 128, 256, [136], 136),
+    (5, 1, 2, 64, 16, [1, 15, 128, 129, 136], 136),
+    (6, 4, 2, 128, 24, [127, 24, 136, 130, 48, 2], 136),                                   # blocks that are no multiple of a chunk's 16 keys
+    (9, 2, 3, 64, 5, [136, 7, 129, 128, 64, 65, 10, 113, 1], 136),
+    (16, 2, 8, 128, 48, [100 + i for i in range(16)], 130),                                # the most pairs of a round's contexts
+    (17, 2, 8, 128, 16, [240 + i % 17 for i in range(17)], 256),                           # from here on whole buckets
+    (23, 8, 8, 64, 24, [1 + 11 * i for i in range(23)], 256),
+    (191, 8, 1, 128, 32, [1 + (37 * i) % 256 for i in range(191)], 256),
+    (16, 2, 8, 128, 16, [137 + i for i in range(16)], 256),                                # beside the rule: longer contexts of few pairs, groups of 8, more pairs
+    (2, 8, 2, 64, 16, [100, 136], 136),
+    (24, 1, 8, 64, 16, [130] * 24, 136),
+])
+def test_brief_decode_attention_against_partitions(B, G, KVH, D, bs, ctx, bound):
+    """Contexts that one workgroup per pair takes without partitions, and their neighbours, against the same call with a bound that cuts them into partitions: f32 sums in another order and one
+    rounding, 2 ulps of float16 as above."""
+    l = nvr.lib()
+    rng = np.random.default_rng(B + D)
+    H, blocks = G * KVH, [(c + bs - 1) // bs for c in ctx]
+    mb, perm, o = max(blocks) + 1, rng.permutation(sum(blocks)), 0
+    bt = np.full((B, mb), -1, np.int32)
+    for b, n in enumerate(blocks):
+        bt[b, :n] = perm[o:o + n]; o += n
+    k, v = (dev(rng.standard_normal((sum(blocks), bs, KVH, D)).astype(F16).view(np.uint16)) for _ in range(2))
+    q = dev(rng.standard_normal((B, H, D)).astype(F16).view(np.uint16))
+    d_ctx, d_bt, tickets = dev(np.asarray(ctx, np.int32)), dev(bt), dev(np.zeros(B * KVH, np.uint32))
+    out = []
+    for most in (bound, 2048):
+        meta = nvr.AttnMetaC()
+        meta.context_lens, meta.block_tables, meta.max_blocks, meta.batch, meta.max_context_len = d_ctx.ptr, d_bt.ptr, mb, B, most
+        ws, got = nvr.DeviceBuffer(l.nvr_paged_attn_workspace_bytes(B, H, D, most)), nvr.DeviceBuffer(B * H * D * 2)
+        nvr.check(l.nvr_fill_const(got.ptr, B * H * D, C.c_float(float("nan")), None))
+        nvr.check(l.nvr_paged_attn_decode_fused(q.ptr, H * D, k.ptr, v.ptr, C.byref(meta), H, KVH, D, bs, D ** -0.5, got.ptr, ws.ptr, tickets.ptr, None))
+        out.append(got.to_numpy((B, H, D), F16).astype(np.float32))
+        assert not tickets.to_numpy((B * KVH,), np.uint32).any()
+    a, b = out
+    assert np.all(np.abs(a - b) <= 2 * np.maximum(np.spacing(np.abs(b).astype(F16)).astype(np.float32), 2.0 ** -14 / 8)), np.abs(a - b).max()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("heads,vdim,ff,batch", [(1, 30, 48, 1), (3, 32, 48, 16), (5, 4, 64, 17), (2, 64, 2064, 32), (4, 96, 40, 33)])
 def test_layer_list_gated_head_norm_and_clamped_unit(dtype, heads, vdim, ff, batch):
