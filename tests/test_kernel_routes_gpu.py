@@ -225,23 +225,43 @@ def test_float32_prompt_rows_have_the_same_bits_in_every_step(hidden, inter, hea
 
 
 @pytest.mark.parametrize("W,taps,heads,kv,dim,lengths", [(64, 1, 4, 2, 64, [1, 31, 32]), (1024, 4, 2, 1, 64, [33, 127]), (1040, 4, 4, 1, 128, [30, 255, 256]), (2080, 8, 4, 4, 64, [3, 129]),
-                                                         (4160, 3, 4, 2, 64, [5]), (96, 9, 2, 2, 64, [40, 7]), (256, 4, 4, 2, 64, [20] * 66)])
+                                                         (4160, 3, 4, 2, 64, [5]), (96, 9, 2, 2, 64, [40, 7]), (256, 4, 4, 2, 64, [20] * 64), (256, 4, 4, 2, 64, [20] * 66)])
 def test_layer_list_decode_steps(W, taps, heads, kv, dim, lengths):
     """Decode steps of the distance-penalty design in bfloat16: the output product cut along k, the join with the next norm and convolution in one launch (widths of one piece per thread to
-    four, one tap to eight) or apart (beyond), attention with the penalty table over few query rows at the edges of its chunks, batches above the parts' rows — against the float64 restatement."""
+    four, one tap to eight) or apart (beyond), attention with the penalty table over few query rows at the edges of its chunks, batches of the parts' rows and above them — against the float64 restatement; every row is looked at."""
     import rugudra_util as u
     cfg = u.make_config([u.attention_layer(heads, kv, dim, dim, ff=256), u.retention_layer(2, 32, 32, ff=None), u.attention_layer(heads, kv, dim, dim, ff=64)], width=W, taps=taps)
     w = u.make_weights(cfg, seed=W + taps)
     n = len(lengths)
     d = u.Driver(cfg, w, dtype="bfloat16", slots=n, pages=n * 20, max_tokens=max(512, sum(lengths)), max_len=512)
     rng = np.random.default_rng(taps)
-    tokens = [rng.integers(0, 97, L + 3) for L in lengths]
+    base = [rng.integers(0, 97, L + 3) for L in lengths[:3]]
+    tokens = [base[i % 3] for i in range(n)]
     d.step([("s%d" % i, t[:L]) for i, (t, L) in enumerate(zip(tokens, lengths))])
     got = [d.step([("s%d" % i, t[L + k:L + k + 1]) for i, (t, L) in enumerate(zip(tokens, lengths))]) for k in range(3)]
-    err = [u.row_errors(np.concatenate([g["s%d" % i] for g in got]), u.expected_logits(cfg, w, tokens[i])[lengths[i]:]) for i in range(min(n, 4))]
-    # (the middle row and not the worst: where a retention head's output nearly cancels, its norm magnifies bfloat16's rounding — a prompt's rows of such a model are 0.008 off on
-    #  average and 0.43 at the worst, decode steps 0.006 and 0.042; a wrong key, row or part shows in every row at the order of 1)
-    assert np.median(err) < u.TOL["bfloat16"] / 2 and np.max(err) < 0.5
+    _compare_layer_rows(cfg, w, "bfloat16", base, [np.concatenate([g["s%d" % i] for g in got]) for i in range(n)])
+
+
+def _compare_layer_rows(cfg, w, dtype, base, rows):
+    """rows[i]: a request's last logits, its tokens base[i % 3].  The first three against the float64 restatement, row by row; every further row has the bits of the request it repeats (a row's
+    sums do not depend on its place in the batch).  bfloat16: a row may be three times as far off as the worst of four draws in which every weight moves by a rounding of its own size — where a
+    retention head's output nearly cancels, its norm magnifies both alike (measured: 0.5 of it in the middle, 1.07 at the worst; a wrong key, row or part is off at the order of 1)."""
+    import rugudra_util as u
+    for i, t in enumerate(base):
+        n = len(rows[i])
+        want = u.expected_logits(cfg, w, t)
+        err = u.row_errors(rows[i], want[-n:])
+        bound = u.TOL["float32"] / 2
+        if dtype == "bfloat16":
+            moved = []
+            for seed in range(4):
+                rng = np.random.default_rng(100 + seed)
+                v = {k: np.asarray(x, np.float64) * (1 + 2.0 ** -9 * rng.standard_normal(np.shape(x))) for k, x in w.items()}
+                moved.append(u.row_errors(u.expected_logits(cfg, v, t)[-n:], want[-n:]))
+            bound = 3 * np.max(moved, axis=0)
+        assert np.all(err < bound), (i, err, bound)
+    for i in range(3, len(rows)):
+        assert np.array_equal(rows[i], rows[i % 3]), i
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
@@ -372,14 +392,14 @@ def test_brief_decode_attention_against_partitions(B, G, KVH, D, bs, ctx, bound)
 @pytest.mark.parametrize("heads,vdim,ff,batch", [(1, 30, 48, 1), (3, 32, 48, 16), (5, 4, 64, 17), (2, 64, 2064, 32), (4, 96, 40, 33)])
 def test_layer_list_gated_head_norm_and_clamped_unit(dtype, heads, vdim, ff, batch):
     """A retention layer's gated head norm by a wave per head (head widths that are multiples of 4, head counts that leave waves without a head) and by the general form, and the clamped unit in
-    its product's epilogue (up to 32 rows: one and two blocks of 16, few and many column tiles) or behind it, against the float64 restatement; bounds as in the test of the decode steps above."""
+    its product's epilogue (up to 32 rows: one and two blocks of 16, few and many column tiles) or behind it, against the float64 restatement; every row is looked at."""
     import rugudra_util as u
     cfg = u.make_config([u.retention_layer(heads, 32, vdim, ff=ff), u.attention_layer(2, 1, 64, 64, ff=ff)], width=64, taps=4)
     w = u.make_weights(cfg, seed=heads + vdim)
     d = u.Driver(cfg, w, dtype=dtype, slots=batch, pages=batch * 2, max_tokens=max(64, 9 * batch), max_len=64)
     rng = np.random.default_rng(ff)
-    tokens = [rng.integers(0, 97, 8 + i % 3) for i in range(batch)]
+    base = [rng.integers(0, 97, 8 + i) for i in range(min(batch, 3))]
+    tokens = [base[i % 3] for i in range(batch)]
     d.step([("s%d" % i, t[:-2]) for i, t in enumerate(tokens)])
     got = [d.step([("s%d" % i, t[len(t) - 2 + k:len(t) - 1 + k]) for i, t in enumerate(tokens)]) for k in range(2)]
-    err = [u.row_errors(np.concatenate([g["s%d" % i] for g in got]), u.expected_logits(cfg, w, tokens[i])[-2:]) for i in range(0, batch, 5)]
-    assert np.median(err) < u.TOL[dtype] / 2 and np.max(err) < (0.5 if dtype == "bfloat16" else 1e-2)
+    _compare_layer_rows(cfg, w, dtype, base, [np.concatenate([g["s%d" % i] for g in got]) for i in range(batch)])
