@@ -291,10 +291,13 @@ def test_decode_steps_of_one_and_two_rows_against_more(dtype, hidden, inter, hea
             out.append(r.logits(len(which)).copy())
         return np.stack(out, 1)                                            # [sequence, step, vocabulary]
     full = steps([0, 1, 2])
-    tol = 2.0 ** (-7 if dtype == "float16" else -4) * float(np.sqrt((full ** 2).mean())) * 4
+    # a sum in another order crosses a rounding of half an ulp here and there, eight places a layer on the residual stream: sqrt(24) * 2^-12 / sqrt(3) relative (float16) if all of them did;
+    # three times that for a row's norm, and for its largest of 192 logits four times its norm (measured, float16: 0.0012 and 0.0038; bfloat16, eight times as coarse: 0.0094 and 0.030)
+    row = 3 * 24 ** 0.5 * 2.0 ** (-12 if dtype == "float16" else -9) / 3 ** 0.5
+    rms = np.sqrt((full ** 2).mean(-1, keepdims=True))
     for which in ([0], [1], [2], [0, 1], [1, 2]):
-        got = steps(which)
-        assert np.abs(got - full[which]).max() < tol, which
+        d = (steps(which) - full[which]) / rms[which]
+        assert np.sqrt((d ** 2).mean(-1)).max() < row and np.abs(d).max() < 4 * row, which
 
 
 @pytest.mark.parametrize("B,G,KVH,D,bs,ctx", [
