@@ -822,7 +822,7 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
     if (brief) { np = 1; waves = 8; }
     // Work-balanced form (attn_share_kernel): a pair count whose last round of one-workgroup-per-pair launches would be mostly empty — 257..2047 pairs with
     // >= 15 % of the rounds' slots unused (33..37 and 65..74 sequences at 8 kv heads, ...), contexts long enough for the stream to matter — or a RAGGED batch
-    // (balance_hint: the caller knows the sum of the contexts; per-pair launches size every pair's partitions by the LONGEST context and leave the short sequences'
+    // (ragged: the caller knows the sum of the contexts; per-pair launches size every pair's partitions by the LONGEST context and leave the short sequences'
     // workgroups idle, or — with several pairs per CU — end on the long sequences' workgroups: 32 sequences of 256..8192 keys 4.09 -> 2.43 ms per Qwen3-0.6B step,
     // 64 of 64..4096 keys 3.26 -> 2.78).  NVR_ATTN_SHARE=0: off.
     if constexpr (G * D <= 512)
@@ -830,13 +830,11 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
         const int64_t cus = share_workgroups(), rounds = (pairs + cus - 1) / cus, units = (mc + 63) / 64;
         const int64_t cap = a.workspace_bytes ? (int64_t)(a.workspace_bytes / ((size_t)a.nq * a.H * (D + 2) * sizeof(float))) : units;
         const bool by_count = pairs > cus && rounds * cus * 100 >= pairs * 115 && mc >= 256;
-        // workgroups: one per CU, or the caller's count for ragged batches (fewer, where a share would hold less than four 64-key units)
-        const int64_t nw = a.balance_hint > 0 ? a.balance_hint : cus;
-        if ((by_count || a.balance_hint || share_mode() == 2) && pairs < 2048 && cap >= units) {
+        if ((by_count || a.ragged || share_mode() == 2) && pairs < 2048 && cap >= units) {
             p.part_size = 64; p.num_parts = (int32_t)cap;
             p.part_o = (float *)a.workspace; p.part_ml = p.part_o + (int64_t)a.nq * a.H * cap * D;
             p.part0 = 0; p.kv0 = 0; p.kv0_rows = nullptr; p.tickets = a.tickets;
-            const int shares = (int)std::max<int64_t>(1, nw / a.KVH);
+            const int shares = (int)std::max<int64_t>(1, cus / a.KVH);                      // one workgroup per CU
             attn_share_kernel<D, G, DU / 2, 8><<<dim3((unsigned)(shares * a.KVH)), dim3(512), 0, s>>>(p, (int)a.nq, shares);
             hipError_t e = hipGetLastError();
             if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "attention (work-balanced) launch failed: %s", hipGetErrorString(e));
