@@ -453,9 +453,14 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float *__restrict
 //  * a segment (one query's keys in one share) costs a start and a cross-wave merge of its own, about two units' time: every query is charged CHARGE units in
 //    front of its keys, so that a share of many short queries holds fewer keys (27 sequences of 64..8100 keys 40.9 -> 38.7 us, 64 of 64..4096 54.5 -> 49.1;
 //    one unit 39.1 / 51.9, four 39.0 / 50.7);
-//  * one wait per round: two rounds are in flight at any time (the block-table reload, which would make hipcc wait for everything at each round, waits for itself);
+//  * one trip per round: a segment starts with two rounds requested and asks for the next one behind each (the block-table reload, which would make hipcc wait for everything at each
+//    round, waits for itself).  For groups of 4 and 8 heads, whose arithmetic fills the time of a round, and heads of 64, whose rows are short, the requests are held in front of it (AHEAD); the
+//    waves of smaller groups of 128 are at the memory's rate without, and requests held cost them 6 % of it;
 //  * one share per CU: with those two, twice the shares only double the starts and merges (64 of 64..4096 keys: 49.1 us with one, 52.6 with two per CU).
-// Together 27 sequences of 64..8100 keys 41.8 -> 38.7 us a layer (184 MB: 4.4 -> 4.7 TB/s; 32 equal sequences of 4096 keys: 6.5).
+// us a launch of 8 kv heads of 128, before these (one or two shares per CU, whichever is less) / with requests past a segment's end / now: 27 sequences of 64..8100 keys 43.3 / 35.9 / 35.1, 64 of
+// 64..4096 59.7 / 47.4 / 45.0, 40 of 32..2000 28.0 / 21.0 / 21.0, 33 of 4000 84.9 / 90.8 / 83.6-86.5 (6.3 TB/s), 48 of 4000 117.4 / 124.6 / 117.9, 65 of 4000 159 / 172 / 160, 74 of 1500
+// 74.2 / 79.8 / 75.5, 48 of 1500 50.2 / 50.4 / 48.9, 33 of 700 23.6 / 21.7 / 22.2.  Groups of 4, not AHEAD / AHEAD: 40 of 1500 keys 55.1 / 49.5, 33 of 4000 102.6 / 91.7, 27 of 64..8100
+// 44.5 / 39.8; heads of 64, 4 kv heads, 66 of 4000 keys: groups of 8 111.4 / 98.3, of 4 74.1 / 60.5, of 2 63.0 / 45.4.
 template <int D, int G, int U, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, int nq, int nw) {
     constexpr int LPR = D / 8, RPI = 64 / LPR, TPI = RPI * U, CH = TPI * WAVES;
@@ -463,6 +468,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int dc = lane % LPR, tg = lane / LPR;
     constexpr int CHARGE = 2;
+    constexpr bool AHEAD = D == 64 || G >= 4;
     __shared__ int pre[1025];                               // pre[t] = units of the queries in front of t, their charges included
     __shared__ int cx[1024];                                // ctx_lens[t]
     __shared__ float sm_acc[WAVES][G][D];
@@ -508,14 +514,15 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
         const int blk = __builtin_amdgcn_readlane(bt_reg, bi & 63);
         return (((int64_t)blk * p.block_size + bo) * p.KVH + g) * D;
     };
-    // round r of the wave.  No branch stands around a request (hipcc would then wait for all that is in flight): a round past the wave's last one asks for
-    // that one again, a wave without keys for the segment's first, and rows past the segment's end for its last row
+    // round r of the wave: a wave without keys asks for the segment's first row, and rows past the segment's end are its last row.  No branch stands around an AHEAD request (hipcc would then wait
+    // for all that is in flight): past the wave's last round all its lanes ask for one 16-byte piece of that round, for all of it again they read 4 rounds too many per 66 of 4000 keys
     auto load_round = [&](int r, half8_t (&kk)[U], half8_t (&vv)[U]) {
         const int tb = R > 0 ? p0 + (min(r, R - 1) * WAVES + wave) * TPI : p0;
         const int64_t base = block_base(tb);
 #pragma unroll
         for (int x = 0; x < U; ++x) {
-            const unsigned off = (unsigned)(min(x * RPI + tg, pend - 1 - tb) * row_elems + dc * 8);
+            unsigned off = (unsigned)(min(x * RPI + tg, pend - 1 - tb) * row_elems + dc * 8);
+            if (AHEAD) off &= r < R ? ~0u : 0u;
             kk[x] = load_row16<true>(p.k + base + off); vv[x] = load_row16<true>(p.v + base + off);
         }
     };
@@ -601,13 +608,11 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
         for (int r = 0; r < R; r += 2) {
             process(ka, va, r);
             if (r + 1 >= R) break;
-            load_round(r + 2, ka, va);
-            asm volatile("" ::: "memory");                  // the requests stay in front of the other round's arithmetic
-            __builtin_amdgcn_sched_barrier(0);
+            if (AHEAD || r + 2 < R) load_round(r + 2, ka, va);
+            if (AHEAD) { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); }   // the requests stay in front of the other round's arithmetic
             process(kb, vb, r + 1);
-            load_round(r + 3, kb, vb);
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
+            if (AHEAD || r + 3 < R) load_round(r + 3, kb, vb);
+            if (AHEAD) { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); }
         }
 
         // the segment is in the accumulators: what its tail needs of the state, then the NEXT segment is opened (its query, block table and first K/V rows
