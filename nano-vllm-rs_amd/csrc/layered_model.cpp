@@ -353,6 +353,7 @@ int LayeredModel::execute(nvr_model_runner &r, nvr_seq *const *seqs, size_t nseq
         o_ftiles[k] = carve(cnt * sizeof(nvr::kt::FlashTile)); n_ftiles[k] = (int32_t)cnt;
     }
     if (off > in_bytes) return fail(NVR_ERR_INVARIANT, "execute_model: step inputs of %zu bytes exceed the arena", off);
+    NVR_HIP_CHECK(hipStreamSynchronize(r.stream));                       // in_host is written again: the upload of a step whose results nobody has read may still wait behind the step in front of it
     for (size_t k = 0; k < flash_kinds.size(); ++k) {
         const int64_t pw = flash_kinds[k].positions;
         nvr::kt::FlashTile *tl = (nvr::kt::FlashTile *)(in_host + o_ftiles[k]);

@@ -311,3 +311,28 @@ def test_greedy_generation_through_the_scheduler(dtype, chunked):
             row = lg[k]
             spread = np.sqrt(((row - row.mean()) ** 2).mean())
             assert row.max() - row[full[k + 1]] <= 3 * TOL[dtype] * spread, f"request {sid}: token {k + 1} is not the greedy choice"
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_steps_queued_one_behind_the_other(dtype):
+    """Steps whose results nobody reads in between — portions of a prompt, then single tokens — give the bits of the same steps read one by one: a step's inputs are not written over those of
+    the step in front while their upload still waits."""
+    cfg = make_config([attention_layer(4, 2, 64, 64, ff=1024), retention_layer(4, 64, 64, ff=1024)], width=512, taps=4)
+    w = make_weights(cfg, seed=3)
+    tokens = np.random.default_rng(8).integers(0, 97, 1900)
+    cuts = [(0, 900), (900, 1800), (1800, 1897), (1897, 1898), (1898, 1899), (1899, 1900)]
+    got = []
+    for read in (True, False):
+        d = Driver(cfg, w, dtype=dtype, slots=1, pages=128, max_tokens=1024, max_len=2048)
+        s = d.nvr.Sequence(tokens[:900].tolist(), d.nvr.SamplingParams(temperature=0.0, max_tokens=1 << 20, ignore_eos=True), block_size=d.page)
+        d.bm.allocate(s)
+        for a, b in cuts:
+            if a:
+                s.extend(tokens[a:b].tolist())
+                d.bm.extend(s)
+            s.set_chunk(a, b - a)
+            d.runner.execute_step([s])
+            if read:
+                d.runner.logits(1, cfg["vocab"])
+        got.append(d.runner.logits(1, cfg["vocab"]).copy())
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1])
