@@ -1,7 +1,7 @@
 // f32_path.hip — Config.dtype = "float32" (reference src/config.rs:51,113-116; the reference's own CPU path computes in f32): every op of the
-// Qwen3 graph on 4-byte storage, as plain FMA kernels.  This is the REFERENCE-PRECISION path of the product — outputs comparable with the
-// reference's f32 CPU path at 1e-3 instead of through 16-bit rounding — a parity vehicle first: FMA kernels for the decode-sized steps, the f32
-// matrix cores (v_mfma_f32_32x32x2_f32, 1/16 of the fp16 rate) for the GEMMs of prefill-sized steps since r06.  Each kernel cites the reference op it restates, like its 16-bit twin:
+// Qwen3 graph on 4-byte storage and sums.  This is the REFERENCE-PRECISION path of the product — outputs comparable with the
+// reference's f32 CPU path at 1e-3 instead of through 16-bit rounding: FMA kernels for the decode-sized steps and attention, the f32
+// matrix cores (v_mfma_f32_32x32x2_f32, 1/16 of the fp16 rate) for the GEMMs of steps of more than 8 rows.  Each kernel cites the reference op it restates, like its 16-bit twin:
 //   embedding   VocabParallelEmbedding::forward, src/layers/embed_head.rs:77-97
 //   rmsnorm     RMSNorm::forward_simple, src/layers/layernorm.rs:58-75; add_rmsnorm: forward_with_residual :170-176
 //   linear      Linear::forward x·Wᵀ(+b), src/layers/linear.rs:12-24
@@ -688,7 +688,7 @@ int activation(int kind, const float *x, int64_t T, int64_t cols, float *out, hi
 
 // ---------------------------------------------------------------- attention: one workgroup per (query row, head).  Keys of the row: ctx_lens[t] of them,
 // either rows kv_base[t] + j of a contiguous K / V (stride ldkv; the prefill step's own qkv buffer) or cache rows through block table seq_of_q[t]
-// (paged decode).  Scores of all keys in LDS (two-pass softmax as compute_attention writes it), then out[d] = sum_j p_j v_j[d] / sum.
+// (paged decode).  Scores of all keys in LDS (two-pass softmax as compute_attention writes it), then out[d] = sum_j p_j v_j[d] / sum.  The general form: head dims that are no multiple of 64, unaligned rows.
 template <int NV>   // output columns per lane: head_dim <= 64 * NV
 __global__ __launch_bounds__(256) void attention_kernel(AttnArgsF a, int paged) {
     extern __shared__ float sc[];                                       // [max_ctx] scores, then probabilities | q [D] | partial outputs [4][D] | 8 of reduction scratch
@@ -807,7 +807,8 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnArgsF a, int paged) 
 // fill the chip), four waves in turn (a prompt: the rows do) — the same sums in the same order, so that a row's bits do not depend on how many rows are in its step.  K and V of the first
 // round are requested before anything is known but the block table, those of the next round before this one is used; the four groups of a wave meet in registers, the eight sums of the row
 // in LDS.  What bounds a decode step's launch is that chain of round trips, not bytes.  Qwen3-0.6B, us a launch, the general form / this one: one sequence of 150 keys 14.3 / 7.3, of 4096 keys
-// 195 / 78; prompts of 128 rows 38 / 19, 509 268 / 129, 1024 873 / 401
+// 195 / 78 (a decode step of one sequence, 128 / 512 / 1024 / 2048 / 4096 / 8000 keys: 1230 / 1798 / 2467 / 3752 / 6293 / 11132 us before it and the other changes beside it, 1021 / 1247 / 1504 /
+// 2002 / 3000 / 4922 now); prompts of 128 rows 38 / 19, 509 268 / 129, 1024 873 / 401
 template <int NF, int NW, bool PAGED>
 __global__ __launch_bounds__(64 * NW) void attention_rows_kernel(AttnArgsF a) {
     constexpr int D = 64 * NF, KB = NF <= 2 ? 4 : 2;                     // keys a group requests at a time
