@@ -822,9 +822,8 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
         } else np = parts_for(a.nq, a.KVH, mc, waves, &part_size);
     }
     // Few pairs over short contexts (a chat's first hundred tokens): the partitions' hand-off — partials out, a ticket, partials back — costs more than the keys: ONE workgroup of
-    // eight waves per pair, whose round is 128 keys (attn_brief_context).  Up to 64 keys there is one partition anyway, and its four waves end sooner (184 pairs of 60 keys, groups of 4 and 8: 5.8 and
-    // 6.8 us against 6.8 and 9.2; 136 keys 12.4 and 20.0 in partitions against 7.6 and 10.0).
-    const bool brief = paged && a.workspace && !shared && mc > 64 && mc <= (pairs <= 128 ? attn_brief_context(a.nq, a.H, a.KVH) : pairs < 192 ? 256 : 0);
+    // eight waves per pair, whose round is 128 keys (attn_brief_context).
+    const bool brief = paged && a.workspace && !shared && mc <= (pairs <= 128 ? attn_brief_context(a.nq, a.H, a.KVH) : pairs < 192 ? 256 : 0);
     if (brief) { np = 1; waves = 8; }
     // Work-balanced form (attn_share_kernel): a pair count whose last round of one-workgroup-per-pair launches would be mostly empty — 257..2047 pairs with
     // >= 15 % of the rounds' slots unused (33..37 and 65..74 sequences at 8 kv heads, ...), contexts long enough for the stream to matter — or a RAGGED batch

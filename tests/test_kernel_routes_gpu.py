@@ -364,8 +364,6 @@ def _work_balanced_against_per_pair(B, G, KVH, D, bs, ctx, bound, launches):
     (16, 2, 8, 128, 16, [137 + i for i in range(16)], 256),                                # beside the rule: longer contexts of few pairs, groups of 8, more pairs
     (2, 8, 2, 64, 16, [100, 136], 136),
     (24, 1, 8, 64, 16, [130] * 24, 136),
-    (23, 8, 8, 64, 24, [1 + (7 * i) % 64 for i in range(23)], 64),                         # up to 64 keys, and from there on
-    (5, 4, 2, 128, 16, [65, 64, 1, 33, 65], 65),
 ])
 def test_brief_decode_attention_against_partitions(B, G, KVH, D, bs, ctx, bound):
     """Contexts that one workgroup per pair takes without partitions, and their neighbours, against the same call with a bound that cuts them into partitions: f32 sums in another order and one
