@@ -550,8 +550,8 @@ NVR_API int nvr_add_rmsnorm_slabs(nvr_half *h, const float *slabs, int64_t S, co
  * rows 16t..16t+15; mode 1: the qkv row order of the RoPE epilogue (rotation partners of a q / k head in one tile; needs H, KVH, D). */
 NVR_API int nvr_retile_weight(const nvr_half *src, nvr_half *dst, int64_t N, int64_t K, int mode, int64_t H, int64_t KVH, int64_t D,
                               void *stream);
-/* The same ops reading a tiled copy: W stays the row-major weight (taken when the shape routes to a tile GEMM, T > 64), Wt is its
- * nvr_retile_weight copy (mode 1 for qkv, mode 0 otherwise) and is what the weight-streaming decode kernels read.  Results are
+/* The same ops reading a tiled copy: W stays the row-major weight (taken when the shape routes to the 256-row tile GEMM), Wt is its
+ * nvr_retile_weight copy (mode 1 for qkv, mode 0 otherwise) and is what the weight-streaming decode kernels and the 128-row tiles read.  Results are
  * bit-identical to the row-major entry points (tests/test_kernels_gpu.py::test_tiled_entry_points_match_row_major). */
 NVR_API int nvr_linear_tiled(const nvr_half *x, int64_t ldx, const nvr_half *W, const nvr_half *Wt, int64_t T, int64_t K, int64_t N,
                              void *y, int y_is_f32, void *stream);

@@ -4,18 +4,24 @@
 // rotary_embedding.rs:23-48; attention.rs:150-174).  Bound: MFMA (dense contraction, SURVEY §8d:
 // 880.8 MFLOP per prefill token for Qwen3-0.6B).
 //
-// Structure (cdna_hip_programming.md §5 "standard MFMA GEMM main loop", the 128x128 two-barrier form):
-//   workgroup = 4 waves = 128 (n) x 128 (m) output tile, BK = 64; wave (wn, wm) owns 64 x 64 = 4x4 MFMA tiles
-//   of v_mfma_f32_16x16x32_f16 (A = W rows, B = x rows, both K-contiguous in memory);
-//   both operand tiles are staged global -> LDS by global_load_lds_dwordx4 (16 B per lane, no VGPR round
-//   trip) into two buffers, the load of K-tile t+1 overlapping the MFMAs on tile t;
+// Structure:
+//   workgroup = 4 waves = 128 (n) x 128 / 64 / 32 (m) output tile, BK = 64; wave (wn, wm) owns 64 x 64 / 32 / 16, MFMA tiles of v_mfma_f32_16x16x32_f16 (A = W rows, B = x rows, both
+//   K-contiguous in memory);
+//   both operand tiles are staged global -> LDS by global_load_lds_dwordx4 (16 B per lane, no VGPR round trip) into a ring of 2..4 K-tiles behind counted waits, and the fragments of a
+//   k-step of 32 are read from LDS while the k-step in front of it is multiplied, so that one wave per SIMD keeps requests, LDS reads and products going at once (with the reads of a
+//   K-tile in front of its products: K = 2048, N = 1024, 3814 tokens 24.3 us, this way 21.8, 2048 / 1000 tokens as two slices 11.1 / 9.4);
+//   the tiles of a launch are dealt to the XCDs in compact blocks (TileMap: the same product 18.9);
+//   what bounds it: a CU takes operand bytes in at 80-87 GB/s (loads alone take 22.4 us of K = 3072's 26.3, products and reads alone 20.1).
 //   LDS image = [row][8 chunks of 16 B] with chunk' = chunk ^ (row & 7): the swizzle is applied to the per-lane
 //   SOURCE address (the LDS destination of glds is lane-linear) and again on the ds_read_b128 address, so a
 //   16-lane fragment read touches 8 distinct 16-B slots (2-way instead of 16-way conflicts).
+//   A tiled copy of W (retile_weight) is read where there is one: a K-tile of 16 rows is then 2 KiB in a row in memory instead of 16 pieces of 128 B, 3-6 % of a launch whose weights come from
+//   HBM (509 tokens, us: qkv 9.9 -> 9.5, down_proj in 4 slices 9.5 -> 9.2; 3814 tokens down_proj 32.4 -> 30.0).
 // Row mapping of the A operand lets one lane hold what its epilogue needs: for SiluAndMul a wave's 4 n-tiles are
 // [gate c, gate c+16, up c, up c+16]; for RoPE an n-tile is 8 columns of the first half of a head and their 8
 // partners of the second half (the partner of lane l sits in lane l^32).
 #include <cstdlib>
+#include <type_traits>
 #include "kernels.h"
 #include "device_utils.h"
 #include "../common.h"
@@ -24,45 +30,55 @@ namespace nvr { namespace NVR_DT_NS {
 
 enum { TEPI_F16 = 0, TEPI_SILU = 2, TEPI_ROPE = 3, TEPI_LMHEAD = 4, TEPI_SLAB = 5 };
 
+// Where a launch's tiles lie: nx column tiles (W rows) x ny token tiles x nz k-slices, numbered slice by slice, within a slice in strips of `width` column tiles, within a strip
+// token tile by token tile.  Workgroups are dealt to the 8 XCDs in turn and each XCD has an L2 of its own, so XCD c takes the c-th eighth of that line: a compact block of tiles,
+// whose rows of W and x it fetches once.
+struct TileMap { int32_t nx, ny, width; };
+struct TileAt { int32_t x, y, z; };
+__device__ __forceinline__ TileAt tile_of(const TileMap &m) {
+    const unsigned n = gridDim.x, xcd = blockIdx.x & 7, rem = n & 7;
+    unsigned t = xcd * (n >> 3) + min(xcd, rem) + (blockIdx.x >> 3);
+    TileAt at;
+    const unsigned slice = (unsigned)m.nx * m.ny;
+    at.z = t / slice; t -= at.z * slice;
+    const unsigned strip = t / ((unsigned)m.width * m.ny), first = strip * m.width;
+    t -= first * m.ny;
+    const unsigned w = min((unsigned)m.width, m.nx - first);
+    at.y = t / w; at.x = first + (t - at.y * w);
+    return at;
+}
+
 struct TileEpi {
     const int64_t *pos; const int32_t *slots; const float *cos_t, *sin_t;
     half_t *kc, *vc;
-    int32_t H, KVH, D;
+    int32_t H, KVH, D, kv_cache_only;      // kv_cache_only: k and v go to the caches alone
     // TEPI_LMHEAD: f32 logits [T, N] (nullable) and the greedy arg-max of every row over this workgroup's 128 columns:
     // pval / pidx [column tile][T] (maximum, lowest index), merged by argmax_partials
     float *logits; float *pval; int32_t *pidx;
-    // TEPI_SLAB: blockIdx.z owns k in [z*kslice, (z+1)*kslice) and writes its f32 partial tile to slabs[z][T][N]
+    // TEPI_SLAB: k-slice z owns k in [z*kslice, (z+1)*kslice) and writes its f32 partial tile to slabs[z][T][N]
     float *slabs; int64_t slab_stride; int32_t kslice;
     int32_t gelu;                          // TEPI_SILU: gelu (tanh form) instead of silu
+    TileMap map;
+    int32_t tiled;                         // W is the copy [rows/16][K/32][16][32] (retile_weight; TEPI_ROPE: its 16-row tiles are the n-tiles)
 };
 
 constexpr int BM = 128, BN = 128, BK = 64;
-// ring depths of the mid-batch instances (one workgroup per CU): K-tiles in flight = depth - 1.  r04 read the launches of these GEMMs as "3.4 us + the
-// workgroup's operand bytes at 50-56 GB/s per CU"; that rate is bytes in flight over the L2 round trip (3 K-tiles x 24 KiB per CU in the 4-deep ring)
-#ifndef NVR_RING64
-#define NVR_RING64 4
-#endif
-#ifndef NVR_RING32
-#define NVR_RING32 4
-#endif
-#ifndef NVR_RING96
-#define NVR_RING96 4
-#endif
-constexpr int RING64 = NVR_RING64, RING32 = NVR_RING32, RING96 = NVR_RING96;
+constexpr int RING96 = 3;                                                 // K-tiles in the LDS ring of the 96-row kernel
 
-// s_waitcnt vmcnt(younger x PER + EXTRA): K-tile kt has landed once at most the PER requests per thread of each of the `younger` K-tiles behind it (and EXTRA
-// requests issued after them) are outstanding
-template <int PER, int EXTRA = 0>
+// s_waitcnt vmcnt(N)
+template <int N>
+__device__ __forceinline__ void wait_requests() {
+    static_assert(N <= 63, "vmcnt is a 6-bit count");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// K-tile kt has landed once at most the PER requests per thread of each of the `younger` (0..3) K-tiles behind it are outstanding
+template <int PER>
 __device__ __forceinline__ void wait_ring(int younger) {
-    static_assert(6 * PER + EXTRA <= 63, "vmcnt is a 6-bit count");
     switch (younger) {
-    case 0: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(EXTRA) : "memory"); break;
-    case 1: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER + EXTRA) : "memory"); break;
-    case 2: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER + EXTRA) : "memory"); break;
-    case 3: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * PER + EXTRA) : "memory"); break;
-    case 4: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * PER + EXTRA) : "memory"); break;
-    case 5: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(5 * PER + EXTRA) : "memory"); break;
-    default: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(6 * PER + EXTRA) : "memory"); break;
+    case 0: wait_requests<0>(); break;
+    case 1: wait_requests<PER>(); break;
+    case 2: wait_requests<2 * PER>(); break;
+    default: wait_requests<3 * PER>(); break;
     }
 }
 
@@ -81,45 +97,50 @@ __device__ __forceinline__ int tile_w_row(int bx, int t, int r, int N, const Til
     return bx * BN + t * 16 + r;
 }
 
-// NS = 2: two LDS buffers (64 KiB, two workgroups per CU), the load of K-tile t+1 overlaps the MFMAs on tile t and is waited
-// for in full at the end of the step — right when tiles outnumber the CUs.  NS = 4: a ring of four buffers (128 KiB, one
-// workgroup per CU) with three K-tiles in flight and counted s_waitcnt vmcnt: when there are fewer tiles than CUs (decode
-// batches of 129..~1000 rows, short prefills) a workgroup is alone on its CU and every K-step of the NS = 2 form costs one
-// full memory latency (21 us for a K = 1024 tile); the ring hides it.
-// MT: 16-token m-tiles per wave.  4 = the 128-token tile; 2 / 1 = a 64- / 32-token tile for batches of 65..~1000 rows, where 128 x 128 tiles
-// leave half the CUs without a workgroup (T = 512: 128 / 96 / 128 workgroups for qkv / gate_up / the split-k GEMMs; 23 / 16 / 12 us):
-// twice the workgroups, each with the same 128 W rows and half the tokens.
+// the same n-tile in the tiled copy
+template <int EPI>
+__device__ __forceinline__ int tile_w_block(int bx, int t, int N) {
+    if (EPI == TEPI_SILU) return ((t & 3) >> 1) * (N >> 4) + bx * 4 + (t >> 2) * 2 + (t & 1);
+    return bx * 8 + t;
+}
+
+// NS: K-tiles in the LDS ring (tiled_launch).  MT: 16-token m-tiles per wave, 4 = the 128-token tile, 2 / 1 = a 64- / 32-token tile for batches of 65..~1000 rows, where 128 x 128 tiles
+// leave half the CUs without a workgroup.
 template <int EPI, int NS, int MT = 4>
-__global__ __launch_bounds__(256) void gemm_tiled_kernel(const half_t *__restrict__ x, int64_t ldx,
+__global__ __launch_bounds__(256, 2) void gemm_tiled_kernel(const half_t *__restrict__ x, int64_t ldx,
                                                          const half_t *__restrict__ W, int T, int K, int N, int NW,
                                                          half_t *__restrict__ y, TileEpi epi) {
     // one LDS array (cdna guide §5 item 4a): [NS buffers][A 16 KiB | B 16 or 8 KiB]
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int BMt = 32 * MT;                                          // tokens per workgroup
     constexpr int BUF = (BN + BMt) * BK * 2;                              // bytes of one LDS buffer
+    const TileAt at = tile_of(epi.map);
+    static_assert(NS >= 2 && NS <= 4, "wait_ring counts up to three younger K-tiles");
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = lane & 15, q = lane >> 4;
     const int wn = wave >> 1, wm = wave & 1;
-    const int m0 = blockIdx.y * BMt;
+    const int m0 = at.y * BMt;
 
     // staging: thread t copies 16-byte piece idx = i*256 + t (row = idx/8, LDS chunk c' = idx%8) of each operand tile
+    const int kmul = epi.tiled ? 16 : 1;                                  // k -> element offset: (k / 32) * 512 in the tiled copy
     const half_t *asrc[4], *bsrc[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int idx = i * 256 + threadIdx.x, row = idx >> 3, c = (idx & 7) ^ (row & 7);
-        int wr = tile_w_row<EPI>(blockIdx.x, row >> 4, row & 15, N, epi);
+        int wr = tile_w_row<EPI>(at.x, row >> 4, row & 15, N, epi);
         if (wr > NW - 1) wr = NW - 1;
         int xr = m0 + row; if (xr > T - 1) xr = T - 1;
-        asrc[i] = W + (int64_t)wr * K + c * 8;
+        if (epi.tiled) asrc[i] = W + ((int64_t)min(tile_w_block<EPI>(at.x, row >> 4, N), NW / 16 - 1) * (K / 32) + (c >> 2)) * 512 + (row & 15) * 32 + (c & 3) * 8;
+        else asrc[i] = W + (int64_t)wr * K + c * 8;
         bsrc[i] = x + (int64_t)xr * ldx + c * 8;                          // (rows >= BMt: unused)
-        if (EPI == TEPI_SLAB) { asrc[i] += (int64_t)blockIdx.z * epi.kslice; bsrc[i] += (int64_t)blockIdx.z * epi.kslice; }
+        if (EPI == TEPI_SLAB) { asrc[i] += (int64_t)at.z * epi.kslice * kmul; bsrc[i] += (int64_t)at.z * epi.kslice; }
     }
     auto stage = [&](int buf, int k0) {
         char *a_dst = smem + buf * BUF, *b_dst = a_dst + BN * BK * 2;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int piece = (i * 256 + wave * 64) * 16;               // wave-uniform LDS base; hardware adds lane*16
-            __builtin_amdgcn_global_load_lds(asrc[i] + k0, (__attribute__((address_space(3))) void *)(a_dst + piece), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds(asrc[i] + k0 * kmul, (__attribute__((address_space(3))) void *)(a_dst + piece), 16, 0, 0);
             if (i < MT) __builtin_amdgcn_global_load_lds(bsrc[i] + k0, (__attribute__((address_space(3))) void *)(b_dst + piece), 16, 0, 0);
         }
     };
@@ -130,99 +151,129 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const half_t *__restric
 #pragma unroll
         for (int j = 0; j < MT; ++j) acc[i][j] = (float4_t){0.f, 0.f, 0.f, 0.f};
 
-    // TEPI_ROPE on the 32- / 64-token tiles (decode batches of 65..~1000 rows: one wave of workgroups, every microsecond of the tile is a
-    // microsecond of the launch): the epilogue's inputs arrive UNDER the K loop instead of as three dependent round trips behind it
-    // (position -> cos / sin row -> rotate; cache slot -> store: 15.9 us against 10.95 for the same GEMM with a plain epilogue, T = 512,
-    // profiles/r04_mid_batch_gemm.txt).  Positions and slots are requested here, in front of the first operand tile; the cos / sin
-    // pieces in K-step 0, once the positions are in (they are older than the tile that step has just waited for).
-    constexpr bool PRE = EPI == TEPI_ROPE && MT <= 2;
-    constexpr int NWO = (BMt * 16) / 256;                                 // write-out rounds of the epilogue: round i stores row i*16 + tid/16
-    int64_t pre_pos[MT];
-    int pre_slot[NWO];
-    float4_t pre_cs[MT][4], pre_sn[MT][4];
-    const int rope_head = PRE ? (int)(blockIdx.x * 8 + wn * 4) / (epi.D / 16) : 0;    // the head of this wave's four n-tiles (16 | D)
-    const bool rope_rot = PRE && rope_head < epi.H + epi.KVH;
-    if (PRE) {
+    // TEPI_ROPE: the epilogue's inputs arrive UNDER the K loop instead of as three dependent round trips behind it (position -> cos / sin row -> rotate; cache
+    // slot -> store).  Positions and slots are requested here, in front of the first operand tile, the cos / sin pieces once the positions are in.  A wave's four
+    // n-tiles need 128 consecutive bytes of each table per token; lanes q and q + 2 need the same ones, so each requests two n-tiles' pieces and they trade them.
+    constexpr bool ROPE = EPI == TEPI_ROPE;
+    int64_t rope_pos[MT];
+    int rope_slot[MT];
+    float4_t pre_cs[MT][2], pre_sn[MT][2];
+    const int tph = ROPE ? epi.D / 16 : 1, tsh = 31 - __clz(tph), heads = epi.H + 2 * epi.KVH;      // n-tiles per head: 1, 2, 4 or 8
+    const int rope_head = ROPE ? (at.x * 8 + wn * 4) >> tsh : 0;          // the head of the first of this wave's four n-tiles
+    const bool rope_rot = ROPE && rope_head < epi.H + epi.KVH;
+    if (ROPE) {
 #pragma unroll
         for (int j = 0; j < MT; ++j) {
-            // (as inline asm: a compiler-visible load whose first use sits in the K loop makes hipcc drain vmcnt(0) there, operand tiles in
-            //  flight included; the value is complete once K-step 0 has waited for its tile, which is younger — see the pin there)
-            const int m = m0 + wm * (16 * MT) + j * 16 + r;
-            const int64_t *src = epi.pos + (m < T ? m : T - 1);
-            asm volatile("global_load_dwordx2 %0, %1, off" : "=v"(pre_pos[j]) : "v"(src) : "memory");
+            // (as inline asm: a compiler-visible load makes hipcc drain vmcnt(0) at its first use, operand tiles in flight included; the values are complete
+            //  once the first operand tile is, which is younger — see the pin there)
+            const int m = m0 + wm * (16 * MT) + j * 16 + r, mc = m < T ? m : T - 1;
+            const int64_t *src = epi.pos + mc;
+            asm volatile("global_load_dwordx2 %0, %1, off" : "=v"(rope_pos[j]) : "v"(src) : "memory");
+            const int32_t *ss = epi.slots ? epi.slots + mc : reinterpret_cast<const int32_t *>(src);      // (no branch: a value in flight would be copied at its end)
+            asm volatile("global_load_dword %0, %1, off" : "=v"(rope_slot[j]) : "v"(ss) : "memory");
         }
-#pragma unroll
-        for (int i = 0; i < NWO; ++i) { const int m = m0 + i * 16 + (int)(threadIdx.x >> 4); pre_slot[i] = (epi.slots && m < T) ? epi.slots[m] : -1; }
     }
 
     const int KT = (EPI == TEPI_SLAB ? epi.kslice : K) / BK;
-    if (NS == 2) {
-        stage(0, 0);
-        __syncthreads();                                                  // includes s_waitcnt vmcnt(0)
-    } else {
+    auto read_a = [&](const char *buf, int ks, int i) {
+        const int arow = wn * 64 + i * 16 + r;
+        return *reinterpret_cast<const half8_t *>(buf + (arow * 8 + ((ks * 4 + q) ^ (arow & 7))) * 16);
+    };
+    auto read_b = [&](const char *buf, int ks, int j) {
+        const int brow = wm * (16 * MT) + j * 16 + r;
+        return *reinterpret_cast<const half8_t *>(buf + BN * BK * 2 + (brow * 8 + ((ks * 4 + q) ^ (brow & 7))) * 16);
+    };
+    // A K-tile is two k-steps of 32, each with its fragments in registers.  While one k-step is multiplied the fragments of the next are read from LDS, so that with one
+    // wave per SIMD neither the LDS reads nor the requests for later K-tiles stand in front of the matrix cores.
+    half8_t fa[2][4], fb[2][MT];
+    auto read_frag = [&](int slot, int ks) {
+        const char *buf = smem + slot * BUF;
 #pragma unroll
-        for (int st = 0; st < NS - 1; ++st) if (st < KT) stage(st, st * BK);
-    }
-    for (int kt = 0; kt < KT; ++kt) {
-        int cur = kt & 1;
-        if (NS == 2) {
-            if (kt + 1 < KT) stage(cur ^ 1, (kt + 1) * BK);
-        } else {
-            // K-tile kt has landed once at most the 4 + MT loads per thread of each younger K-tile in flight are outstanding
-            const int younger = min(NS - 2, KT - 1 - kt);
-            // (K-step 1 of a rotating TEPI_ROPE wave: the 8 * MT cos / sin requests of K-step 0 are younger than the two tiles that may stay in
-            //  flight and may stay in flight with them; later steps find them landed)
-            if (PRE && kt == 1 && rope_rot) wait_ring<4 + MT, (PRE ? 8 * MT : 0)>(younger);
-            else wait_ring<4 + MT>(younger);
-            __builtin_amdgcn_s_barrier();                                 // every thread's pieces are in; buffer (kt-1) % NS is free
-            cur = kt % NS;
-            if (kt + NS - 1 < KT) stage((kt + NS - 1) % NS, (kt + NS - 1) * BK);
-        }
-        if (PRE && kt == 0 && rope_rot) {
-            const int tph = epi.D / 16, half_d = epi.D / 2;
+        for (int i = 0; i < 4; ++i) fa[ks][i] = read_a(buf, ks, i);
 #pragma unroll
-            for (int j = 0; j < MT; ++j) asm volatile("" : "+v"(pre_pos[j]));   // uses stay behind this step's counted wait (volatile asm keeps its order)
+        for (int j = 0; j < MT; ++j) fb[ks][j] = read_b(buf, ks, j);
+    };
+    auto multiply = [&](int ks, bool reads) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int j = 0; j < MT; ++j)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int jj = ((int)(blockIdx.x * 8 + wn * 4 + i) % tph) * 8 + (q & 1) * 4;
-                    pre_cs[j][i] = *reinterpret_cast<const float4_t *>(epi.cos_t + pre_pos[j] * half_d + jj);
-                    pre_sn[j][i] = *reinterpret_cast<const float4_t *>(epi.sin_t + pre_pos[j] * half_d + jj);
-                }
+                acc[i][j] = mfma16(fa[ks][i], fb[ks][j], acc[i][j]);
+        if (reads) {                                                      // the reads between the first products, so that they land under the later ones
+            constexpr int P = MT > 1 ? MT / 2 : 1;
+            __builtin_amdgcn_sched_group_barrier(0x8, P, 0); __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, P, 0); __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, P, 0); __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, P, 0); __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 4 * MT - 4 * P, 0);
         }
-        const char *a_lds = smem + cur * BUF, *b_lds = a_lds + BN * BK * 2;
+    };
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            half8_t a[4], b[MT];
+    for (int st = 0; st < NS; ++st) if (st < KT) stage(st, st * BK);
+    wait_ring<4 + MT>(min(NS - 1, KT - 1));
+    if (ROPE) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int arow = wn * 64 + i * 16 + r;
-                a[i] = *reinterpret_cast<const half8_t *>(a_lds + (arow * 8 + ((ks * 4 + q) ^ (arow & 7))) * 16);
-            }
-#pragma unroll
-            for (int j = 0; j < MT; ++j) {
-                const int brow = wm * (16 * MT) + j * 16 + r;
-                b[j] = *reinterpret_cast<const half8_t *>(b_lds + (brow * 8 + ((ks * 4 + q) ^ (brow & 7))) * 16);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < MT; ++j)
-                    acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
+        for (int j = 0; j < MT; ++j) {
+            asm volatile("" : "+v"(rope_pos[j]), "+v"(rope_slot[j]));     // uses stay behind the counted wait (volatile asm keeps its order)
+            if (!epi.slots) rope_slot[j] = -1;
         }
-        if (NS == 2) __syncthreads();
     }
-    if (NS != 2) __syncthreads();                                         // the epilogue reuses the operand buffers
-
+    if (rope_rot) {
+        const int half_d = epi.D / 2;
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int jj = ((at.x * 8 + wn * 4 + (q >> 1) * 2 + u) & (tph - 1)) * 8 + (q & 1) * 4;
+                pre_cs[j][u] = *reinterpret_cast<const float4_t *>(epi.cos_t + rope_pos[j] * half_d + jj);
+                pre_sn[j][u] = *reinterpret_cast<const float4_t *>(epi.sin_t + rope_pos[j] * half_d + jj);
+            }
+    }
+    __builtin_amdgcn_s_barrier();
+    read_frag(0, 0);
+    int slot = 0;
+    // first k-step of a K-tile; behind it this wave has read the whole tile
+    auto first_half = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        read_frag(slot, 1);
+        multiply(0, true);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0xC07F);                               // lgkmcnt(0)
+    };
+    auto second_half = [&](int next) {
+        read_frag(next, 0);
+        multiply(1, true);
+        slot = next;
+    };
+    int kt = 0;
+    for (; kt + NS < KT; ++kt) {
+        first_half();
+        // K-tile kt + 1 has landed once at most the 4 + MT requests per thread of each of the NS - 2 younger K-tiles are outstanding (the cos / sin requests of a rotating
+        // TEPI_ROPE wave are younger than K-tiles 1 .. NS - 1 and may stay in flight with them)
+        if (rope_rot && kt + 1 < NS) wait_requests<(NS - 2) * (4 + MT) + 4 * MT>();
+        else wait_requests<(NS - 2) * (4 + MT)>();
+        __builtin_amdgcn_s_barrier();                                     // every thread's pieces of K-tile kt + 1 are in, and every wave has read K-tile kt: its slot is free
+        __builtin_amdgcn_sched_barrier(0);
+        stage(slot, (kt + NS) * BK);
+        second_half(slot + 1 == NS ? 0 : slot + 1);
+    }
+    for (; kt + 1 < KT; ++kt) {                                           // the last NS - 1 K-tiles but one: nothing left to request
+        first_half();
+        wait_ring<4 + MT>(KT - 2 - kt);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        second_half(slot + 1 == NS ? 0 : slot + 1);
+    }
+    first_half();
+    multiply(1, false);
     if (EPI == TEPI_SLAB) {                                                // f32 partial sums, C layout: 4 consecutive columns of token r
-        float *sl = epi.slabs + (int64_t)blockIdx.z * epi.slab_stride;
+        float *sl = epi.slabs + (int64_t)at.z * epi.slab_stride;
 #pragma unroll
         for (int j = 0; j < MT; ++j) {
             const int m = m0 + wm * (16 * MT) + j * 16 + r;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int n = blockIdx.x * BN + wn * 64 + i * 16 + q * 4;
+                const int n = at.x * BN + wn * 64 + i * 16 + q * 4;
                 if (m < T && n < N) *reinterpret_cast<float4_t *>(sl + (int64_t)m * N + n) = acc[i][j];
             }
         }
@@ -233,13 +284,14 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const half_t *__restric
         // row maxima are taken over the f32 accumulators in increasing column order (ties keep the lowest index, A-12)
         float *sv = reinterpret_cast<float *>(smem);                      // [2 (wn)][BMt tokens]
         int *si = reinterpret_cast<int *>(smem + 2 * BMt * 4);
+        __syncthreads();                                                  // (the operand buffers are read by every wave)
 #pragma unroll
         for (int j = 0; j < MT; ++j) {
             const int ml = wm * (16 * MT) + j * 16 + r, m = m0 + ml;
             float bv = -INFINITY; int bi = 0x7fffffff;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int n = blockIdx.x * BN + wn * 64 + i * 16 + q * 4;
+                const int n = at.x * BN + wn * 64 + i * 16 + q * 4;
                 if (epi.logits && m < T && n < N) *reinterpret_cast<float4_t *>(epi.logits + (int64_t)m * N + n) = acc[i][j];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -259,90 +311,93 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const half_t *__restric
             float bv = sv[threadIdx.x]; int bi = si[threadIdx.x];
             const float v = sv[BMt + threadIdx.x]; const int i2 = si[BMt + threadIdx.x];
             if (v > bv || (v == bv && i2 < bi)) { bv = v; bi = i2; }
-            epi.pval[(int64_t)blockIdx.x * T + m0 + threadIdx.x] = bv;
-            epi.pidx[(int64_t)blockIdx.x * T + m0 + threadIdx.x] = bi;
+            epi.pval[(int64_t)at.x * T + m0 + threadIdx.x] = bv;
+            epi.pidx[(int64_t)at.x * T + m0 + threadIdx.x] = bi;
         }
         return;
     }
-    // epilogue: C layout row (n) = q*4 + reg, col (token) = r.  Each lane produces 4 consecutive output columns of one
-    // token; they are staged in LDS (the operand buffers are free now; row stride 272 B keeps ds_read_b128 aligned)
-    // and written out as full 16-byte pieces of contiguous rows (a lane-per-row 8-byte store pattern is issue-bound).
-    constexpr int OST = 272;                                              // bytes per staged row (128 fp16 + pad)
-    constexpr int OUTC = (EPI == TEPI_SILU) ? 64 : 128;                   // output columns of this workgroup
-    char *ot = smem;
-    auto stash = [&](int ml, int lc, half4_t hv) { *reinterpret_cast<half4_t *>(ot + ml * OST + lc * 2) = hv; };
+    // epilogue: C layout row (n) = q*4 + reg, col (token) = r: a lane holds 4 consecutive columns of one token in each n-tile.  Two neighbouring n-tiles trade the
+    // odd 16-lane rows of one for the even rows of the other (v_permlane16_swap), after which a lane holds 8 consecutive columns of one of them: 16-byte stores,
+    // 64 consecutive bytes of a token row per instruction, without a pass through LDS (3814 tokens, us: gate_up 52.0 -> 50.3, qkv 35.3 -> 34.8; 4672 tokens with the rotation 68.0 -> 60.0).
+    auto pair8 = [&](half4_t x, half4_t y) -> half8_t {
+        union { half4_t h; unsigned u[2]; } a, b;
+        union { half8_t h; unsigned u[4]; } o;
+        a.h = x; b.h = y;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const auto t = __builtin_amdgcn_permlane16_swap(a.u[e], b.u[e], false, false);
+            o.u[e] = t[0]; o.u[2 + e] = t[1];
+        }
+        return o.h;
+    };
+    const int col_in_pair = (q & 1) * 16 + (q >> 1) * 8;                  // first column a lane holds of a pair of n-tiles whose 32 columns are consecutive
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
-        const int ml = wm * (16 * MT) + j * 16 + r;
-        const int m = m0 + ml;
-        const int mc = m < T ? m : T - 1;
+        const int m = m0 + wm * (16 * MT) + j * 16 + r;
         if (EPI == TEPI_F16) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                half4_t h = {(half_t)acc[i][j][0], (half_t)acc[i][j][1], (half_t)acc[i][j][2], (half_t)acc[i][j][3]};
-                stash(ml, wn * 64 + i * 16 + q * 4, h);
+            for (int i = 0; i < 4; i += 2) {
+                half4_t h[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) h[u] = (half4_t){(half_t)acc[i + u][j][0], (half_t)acc[i + u][j][1], (half_t)acc[i + u][j][2], (half_t)acc[i + u][j][3]};
+                const half8_t v8 = pair8(h[0], h[1]);
+                const int n = at.x * BN + wn * 64 + i * 16 + col_in_pair;
+                if (m < T && n < N) *reinterpret_cast<half8_t *>(y + (int64_t)m * N + n) = v8;
             }
         } else if (EPI == TEPI_SILU) {
+            half4_t h[2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {                                 // tiles i (gate) and i+2 (up), same 16 columns
-                half4_t h;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float gf = (float)to_half_rn(acc[i][j][e]), uf = (float)to_half_rn(acc[i + 2][j][e]);
                     const float sg = gate_factor(gf, epi.gelu);
-                    h[e] = to_half_rn(__fmul_rn(__fmul_rn(gf, sg), uf));
+                    h[i][e] = to_half_rn(__fmul_rn(__fmul_rn(gf, sg), uf));
                 }
-                stash(ml, wn * 32 + i * 16 + q * 4, h);
             }
+            const half8_t v8 = pair8(h[0], h[1]);
+            const int n = at.x * 64 + wn * 32 + col_in_pair;
+            if (m < T && n < N) *reinterpret_cast<half8_t *>(y + (int64_t)m * N + n) = v8;
         } else {                                                          // TEPI_ROPE
-            const int tph = epi.D / 16, half_d = epi.D / 2;
-            const int64_t p = PRE ? pre_pos[j] : epi.pos[mc];
+            const int half_d = epi.D / 2;
+            const int64_t ldy = (int64_t)heads * epi.D;
+            float4_t cs[4], sn[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int g = blockIdx.x * 8 + wn * 4 + i, head = g / tph, c = g % tph;
-                if (head >= epi.H + 2 * epi.KVH) continue;
-                float v[4], pv[4];
+            for (int u = 0; u < 2; ++u)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) { v[e] = (float)to_half_rn(acc[i][j][e]); pv[e] = __shfl_xor(v[e], 32, 64); }
-                half4_t h; int col;
-                if (head < epi.H + epi.KVH) {
-                    const int jj = c * 8 + (q & 1) * 4;
-                    const float4_t cs = PRE ? pre_cs[j][i] : *reinterpret_cast<const float4_t *>(epi.cos_t + p * half_d + jj);
-                    const float4_t sn = PRE ? pre_sn[j][i] : *reinterpret_cast<const float4_t *>(epi.sin_t + p * half_d + jj);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        h[e] = (q < 2) ? to_half_rn(mul_sub_unfused(v[e], cs[e], pv[e], sn[e]))
-                                       : to_half_rn(mul_add_unfused(v[e], cs[e], pv[e], sn[e]));
-                    col = (q < 2) ? jj : half_d + jj;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) h[e] = to_half_rn(acc[i][j][e]);
-                    col = c * 16 + q * 4;
+                for (int e = 0; e < 4; ++e) {
+                    const auto tc = __builtin_amdgcn_permlane32_swap(__float_as_uint(pre_cs[j][u][e]), __float_as_uint(pre_cs[j][u][e]), false, false);
+                    const auto ts = __builtin_amdgcn_permlane32_swap(__float_as_uint(pre_sn[j][u][e]), __float_as_uint(pre_sn[j][u][e]), false, false);
+                    cs[u][e] = __uint_as_float(tc[0]); cs[2 + u][e] = __uint_as_float(tc[1]);
+                    sn[u][e] = __uint_as_float(ts[0]); sn[2 + u][e] = __uint_as_float(ts[1]);
                 }
-                stash(ml, head * epi.D + col - blockIdx.x * 128, h);       // the 8 n-tiles cover 128 consecutive columns
-            }
-        }
-    }
-    __syncthreads();
-    // cooperative write-out: 16-byte pieces, consecutive threads -> consecutive pieces of a row
-    const int64_t ldy = (EPI == TEPI_ROPE) ? (int64_t)(epi.H + 2 * epi.KVH) * epi.D : (int64_t)N;
-    const int ncols = (EPI == TEPI_ROPE) ? (int)ldy : N;
-    constexpr int CPR = OUTC / 8;                                         // pieces per row
 #pragma unroll
-    for (int i = 0; i < (BMt * CPR) / 256; ++i) {
-        const int pidx = i * 256 + threadIdx.x, row = pidx / CPR, ch = pidx % CPR;
-        const int m = m0 + row, col = blockIdx.x * OUTC + ch * 8;
-        if (m >= T || col >= ncols) continue;
-        const half8_t v8 = *reinterpret_cast<const half8_t *>(ot + row * OST + ch * 16);
-        *reinterpret_cast<half8_t *>(y + (int64_t)m * ldy + col) = v8;
-        if (EPI == TEPI_ROPE) {
-            const int head = col / epi.D;
-            if (head >= epi.H) {
-                const int slot = PRE ? pre_slot[i] : (epi.slots ? epi.slots[m] : -1);
-                if (slot >= 0) {
-                    const bool is_k = head < epi.H + epi.KVH;
-                    const int kvh = is_k ? head - epi.H : head - epi.H - epi.KVH;
-                    *reinterpret_cast<half8_t *>((is_k ? epi.kc : epi.vc) + ((int64_t)slot * epi.KVH + kvh) * epi.D + (col - head * epi.D)) = v8;
+            for (int i = 0; i < 4; i += 2) {
+                half4_t h[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const bool rot = ((at.x * 8 + wn * 4 + i + u) >> tsh) < epi.H + epi.KVH;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float v = (float)to_half_rn(acc[i + u][j][e]);
+                        const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+                        const float pv = __uint_as_float(q < 2 ? t[1] : t[0]);                        // the partner column: the same register of lane ^ 32
+                        // rotary_embedding.rs:36-44: out1 = x1*c - x2*s ; out2 = x2*c + x1*s
+                        const float f = !rot ? v : (q < 2) ? mul_sub_unfused(v, cs[i + u][e], pv, sn[i + u][e]) : mul_add_unfused(v, cs[i + u][e], pv, sn[i + u][e]);
+                        h[u][e] = to_half_rn(f);
+                    }
+                }
+                const half8_t v8 = pair8(h[0], h[1]);
+                const int g = at.x * 8 + wn * 4 + i + (q & 1), head = g >> tsh, c = g & (tph - 1);    // of the n-tile whose columns the lane now holds
+                const bool rot = head < epi.H + epi.KVH;
+                // rotated heads: an n-tile is 8 columns of the first half of the head (lanes q < 2) and their 8 partners
+                const int col = rot ? c * 8 + (q >> 1) * half_d : c * 16 + (q >> 1) * 8;
+                if (m < T && head < heads) {
+                    if (head < epi.H || !epi.kv_cache_only) *reinterpret_cast<half8_t *>(y + (int64_t)m * ldy + head * epi.D + col) = v8;
+                    if (head >= epi.H && rope_slot[j] >= 0) {
+                        const int kvh = rot ? head - epi.H : head - epi.H - epi.KVH;
+                        *reinterpret_cast<half8_t *>((rot ? epi.kc : epi.vc) + ((int64_t)rope_slot[j] * epi.KVH + kvh) * epi.D + col) = v8;
+                    }
                 }
             }
         }
@@ -356,21 +411,22 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const half_t *__restric
 // 12 MFMA tiles per wave and k-step), the four-buffer ring with counted waits of gemm_tiled_kernel<.., 4, ..>, the same K order per output as
 // every other tiling of this file (same bits as the 128-row tiles and as the unfused GEMM + SiluAndMul).
 constexpr int S96_A = 96 * BK * 2, S96_BUF = S96_A + BM * BK * 2;        // bytes of the A image / of one ring buffer
-__global__ __launch_bounds__(256) void gemm_tiled_silu96_kernel(const half_t *__restrict__ x, int64_t ldx, const half_t *__restrict__ W, int T, int K, int I,
-                                                                half_t *__restrict__ y) {
+__global__ __launch_bounds__(256, 2) void gemm_tiled_silu96_kernel(const half_t *__restrict__ x, int64_t ldx, const half_t *__restrict__ W, int T, int K, int I,
+                                                                half_t *__restrict__ y, int tiled) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int NS = RING96;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = lane & 15, q = lane >> 4;
     const int m0 = blockIdx.y * BM;
+    const int kmul = tiled ? 16 : 1;
     const half_t *asrc[3], *bsrc[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int idx = i * 256 + threadIdx.x, row = idx >> 3, c = (idx & 7) ^ (row & 7);
         if (i < 3) {                                                      // A: local row = 16 t + rr, t = 0..2 gate tiles, 3..5 up tiles of the same columns
             const int t = row >> 4, rr = row & 15;
-            const int wr = (t < 3 ? 0 : I) + (int)blockIdx.x * 48 + (t % 3) * 16 + rr;
-            asrc[i] = W + (int64_t)wr * K + c * 8;
+            const int blk = (t < 3 ? 0 : I / 16) + (int)blockIdx.x * 3 + t % 3;
+            asrc[i] = W + (tiled ? ((int64_t)blk * (K / 32) + (c >> 2)) * 512 + rr * 32 + (c & 3) * 8 : (int64_t)(blk * 16 + rr) * K + c * 8);
         }
         int xr = m0 + row; if (xr > T - 1) xr = T - 1;
         bsrc[i] = x + (int64_t)xr * ldx + c * 8;
@@ -380,7 +436,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_silu96_kernel(const half_t *__
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int piece = (i * 256 + wave * 64) * 16;               // wave-uniform LDS base; hardware adds lane*16
-            if (i < 3) __builtin_amdgcn_global_load_lds(asrc[i] + k0, (__attribute__((address_space(3))) void *)(a_dst + piece), 16, 0, 0);
+            if (i < 3) __builtin_amdgcn_global_load_lds(asrc[i] + k0 * kmul, (__attribute__((address_space(3))) void *)(a_dst + piece), 16, 0, 0);
             __builtin_amdgcn_global_load_lds(bsrc[i] + k0, (__attribute__((address_space(3))) void *)(b_dst + piece), 16, 0, 0);
         }
     };
@@ -390,35 +446,54 @@ __global__ __launch_bounds__(256) void gemm_tiled_silu96_kernel(const half_t *__
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = (float4_t){0.f, 0.f, 0.f, 0.f};
     const int KT = K / BK;
+    half8_t fa[2][6], fb[2][2];                                           // fragments of the two k-steps of a K-tile: one multiplied, the other being read, as in gemm_tiled_kernel
+    auto read_frag = [&](int slot, int ks) {
+        const char *a_lds = smem + slot * S96_BUF, *b_lds = a_lds + S96_A;
 #pragma unroll
-    for (int st = 0; st < NS - 1; ++st) if (st < KT) stage(st, st * BK);
-    for (int kt = 0; kt < KT; ++kt) {
-        // K-tile kt has landed once at most the 7 loads per thread of each younger K-tile in flight are outstanding
-        const int younger = min(NS - 2, KT - 1 - kt);
-        wait_ring<7>(younger);
-        __builtin_amdgcn_s_barrier();                                     // every thread's pieces are in; buffer (kt-1) % NS is free
-        const int cur = kt % NS;
-        if (kt + NS - 1 < KT) stage((kt + NS - 1) % NS, (kt + NS - 1) * BK);
-        const char *a_lds = smem + cur * S96_BUF, *b_lds = a_lds + S96_A;
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            half8_t a[6], b[2];
-#pragma unroll
-            for (int i = 0; i < 6; ++i) {
-                const int arow = i * 16 + r;
-                a[i] = *reinterpret_cast<const half8_t *>(a_lds + (arow * 8 + ((ks * 4 + q) ^ (arow & 7))) * 16);
-            }
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int brow = wave * 32 + j * 16 + r;
-                b[j] = *reinterpret_cast<const half8_t *>(b_lds + (brow * 8 + ((ks * 4 + q) ^ (brow & 7))) * 16);
-            }
-#pragma unroll
-            for (int i = 0; i < 6; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
+        for (int i = 0; i < 6; ++i) {
+            const int arow = i * 16 + r;
+            fa[ks][i] = *reinterpret_cast<const half8_t *>(a_lds + (arow * 8 + ((ks * 4 + q) ^ (arow & 7))) * 16);
         }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int brow = wave * 32 + j * 16 + r;
+            fb[ks][j] = *reinterpret_cast<const half8_t *>(b_lds + (brow * 8 + ((ks * 4 + q) ^ (brow & 7))) * 16);
+        }
+    };
+    auto multiply = [&](int ks, bool reads) {
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = mfma16(fa[ks][i], fb[ks][j], acc[i][j]);
+        if (reads) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 2, 0); __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 2, 0); __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 2, 0); __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 6, 0);
+        }
+    };
+#pragma unroll
+    for (int st = 0; st < NS; ++st) if (st < KT) stage(st, st * BK);
+    wait_ring<7>(min(NS - 1, KT - 1));
+    __builtin_amdgcn_s_barrier();
+    read_frag(0, 0);
+    int slot = 0;
+    for (int kt = 0; kt < KT; ++kt) {
+        __builtin_amdgcn_sched_barrier(0);
+        read_frag(slot, 1);
+        multiply(0, true);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0xC07F);                               // lgkmcnt(0)
+        if (kt + 1 == KT) break;
+        wait_ring<7>(min(NS - 2, KT - 2 - kt));
+        __builtin_amdgcn_s_barrier();                                     // K-tile kt + 1 is in, and every wave has read K-tile kt
+        __builtin_amdgcn_sched_barrier(0);
+        if (kt + NS < KT) stage(slot, (kt + NS) * BK);
+        slot = slot + 1 == NS ? 0 : slot + 1;
+        read_frag(slot, 0);
+        multiply(1, true);
     }
+    multiply(1, false);
     __syncthreads();                                                      // the epilogue reuses the operand buffers
     // act = fp16(silu(fp16 g) * fp16 u) (activation.rs:46-63; the rounding points of the unfused graph), staged in LDS and written as 16-byte pieces
     constexpr int OST = 112;                                              // bytes per staged row (48 fp16 + pad)
@@ -453,57 +528,58 @@ static int tiled_check(const char *what) {
     return 0;
 }
 
-// ring (NS = 4) when the grid leaves CUs idle anyway
-static bool tiled_ring(unsigned tiles) { return tiles < 256; }
-// 64- or 32-token tiles when 128-token tiles would leave CUs without a workgroup: the largest tile that reaches ~192 workgroups — unless that count
-// needs a second, mostly empty round: with the 4-buffer ring a 64-token workgroup is alone on its CU (96 KB of LDS), so 257..511 of them run as one full
-// round + a tail while half as many tiles of twice the height finish in one (scratch/route_scan.py: Qwen3-0.6B bs 384 -> 385 got FASTER, 3.87 -> 3.67
-// ms/step; r06: bs 321..384 -3..5 %, bs 513 -4 %).  Returns the m-tiles per wave (4, 2, 1).
-static int tiled_mt(int64_t T, int64_t nx_nz) {
-    int mt = 1;
-    if (T > 64 && nx_nz * ((T + 127) / 128) >= 192) mt = 4;       // (192 workgroups of 128 tokens beat 384 of 64: 15.6 vs 19.3 us, gate_up at T = 512)
-    else if (nx_nz * ((T + 63) / 64) >= 192) mt = 2;              // (33..64 rows never take a 128-token tile: half of it would be masked rows)
-    if (mt == 2 && T > 64) {
-        const int64_t wgs = nx_nz * ((T + 63) / 64), taller = nx_nz * ((T + 127) / 128);
-        if (wgs > 256 && wgs < 512 && taller >= 128) mt = 4;      // (< 512: NVR_TILED_LAUNCH gives them the ring, one workgroup per CU)
-    }
+// Token tile of a launch with `cols` = column tiles x k-slices: 128, 64 or 32 tokens (4, 2, 1 m-tiles per wave).  A CU is fed through its L2 -> LDS path at 80-87 GB/s whatever the
+// tile (loads alone, no products: 0.25 / 0.30 / 0.375 us per K-tile of 20 / 24 / 32 KiB), so a launch costs its fullest CU's workgroups times that.  Measured, us: 200 tokens x 4096
+// columns, K = 1024 6.8 on 224 tiles of 32 tokens / 7.7 on 128 of 64; 300 tokens 8.4 on 320 of 32 / 7.6 on 160 of 64; 1000 tokens 12.5 on 512 of 64 / 11.6 on 256 of 128; 509 tokens of
+// gate_up (48 column tiles) 13.3 on 384 of 64 or 192 of 128, 15.9 on 768 of 32.
+static int tiled_mt(int64_t T, int64_t cols) {
+    auto cost = [&](int mt, int us) { return (cols * ((T + 32 * mt - 1) / (32 * mt)) + 255) / 256 * us; };
+    int mt = 4;
+    if (cost(2, 300) < cost(mt, 375)) mt = 2;
+    if (cost(1, 250) < cost(mt, mt == 4 ? 375 : 300)) mt = 1;
     return mt;
+}
+// Strips of a launch's tiles (TileMap): as many as keep the rows of W and x that one XCD reads fewest.  3814 tokens, us in 1 / 2 / 4 / 8 strips: o_proj (8 column tiles) 19.0 / 18.9 /
+// 19.0 / 21.8, qkv (32) 35.2 / 33.0 / 33.2 / 33.3, gate_up (48) 56.4 / 51.4 / 50.5 / 50.3; in the order of a 2-d grid, 8 token tiles apart on one XCD, o_proj 21.8.
+static TileMap tile_map(int64_t nx, int64_t ny, int64_t nz, int64_t tokens) {
+    const int64_t xcds = nz >= 8 ? 1 : 8 / nz;                            // XCDs of a k-slice
+    int64_t strips = 1, best = INT64_MAX;
+    for (int64_t a = 1; a <= xcds && a <= nx; a *= 2) {
+        const int64_t rows = (nx + a - 1) / a * BN + (ny * a + xcds - 1) / xcds * tokens;
+        if (rows < best) { best = rows; strips = a; }
+    }
+    return TileMap{(int32_t)nx, (int32_t)ny, (int32_t)((nx + strips - 1) / strips)};
 }
 constexpr size_t kStageBytes = 2 * BM * BK * 2;                          // MT = 4
 constexpr size_t kStageBytes64 = (BN + 64) * BK * 2;                     // MT = 2
 constexpr size_t kStageBytes32 = (BN + 32) * BK * 2;                     // MT = 1
-// grid: x = column tiles, y is filled in here (token tiles of 128, 64 or 32), z = k slices; the 4-buffer ring whenever a
-// workgroup is alone on its CU (the smaller tiles fit two workgroups per CU even with the ring)
-#define NVR_TILED_LAUNCH(EPI_, grid, T_, ...)                                                                      \
-    do {                                                                                                           \
-        const int mt_ = tiled_mt((T_), (int64_t)(grid).x * (grid).z);                                              \
-        (grid).y = (unsigned)(((T_) + 32 * mt_ - 1) / (32 * mt_));                                                 \
-        const unsigned wgs_ = (grid).x * (grid).y * (grid).z;                                                      \
-        if (mt_ == 1) {                                                                                            \
-            if (tiled_ring(wgs_ / 2)) gemm_tiled_kernel<EPI_, RING32, 1><<<grid, dim3(256), RING32 * kStageBytes32, s>>>(__VA_ARGS__); \
-            else gemm_tiled_kernel<EPI_, 2, 1><<<grid, dim3(256), 2 * kStageBytes32, s>>>(__VA_ARGS__);           \
-        } else if (mt_ == 2) {                                                                                     \
-            if (tiled_ring(wgs_ / 2)) gemm_tiled_kernel<EPI_, RING64, 2><<<grid, dim3(256), RING64 * kStageBytes64, s>>>(__VA_ARGS__); \
-            else gemm_tiled_kernel<EPI_, 2, 2><<<grid, dim3(256), 2 * kStageBytes64, s>>>(__VA_ARGS__);           \
-        } else {                                                                                                   \
-            if (tiled_ring(wgs_)) gemm_tiled_kernel<EPI_, 4><<<grid, dim3(256), 4 * kStageBytes, s>>>(__VA_ARGS__); \
-            else gemm_tiled_kernel<EPI_, 2><<<grid, dim3(256), 2 * kStageBytes, s>>>(__VA_ARGS__);                 \
-        }                                                                                                          \
-    } while (0)
+// K-tiles in flight: two of the 128-token tiles when two workgroups share a CU (64 KiB each), three when one is alone on it; three or (a long K loop, one workgroup per CU) four of the 64-token
+// tiles, four of the 32-token tiles.  More are slower: 512 tokens x 4096 columns 8.2 us with three, 8.3 with four, 8.7 with six (a launch's LDS takes time to be given out).
+template <int EPI>
+static void tiled_launch(int64_t nx, int64_t nz, const half_bits *x_, int64_t ldx, const half_bits *W_, const half_bits *Wt, int64_t T, int64_t K, int64_t N, int64_t NW, half_t *y, TileEpi e, hipStream_t s) {
+    const half_t *x = (const half_t *)x_, *W = (const half_t *)(Wt ? Wt : W_);
+    e.tiled = Wt != nullptr;
+    const int mt = tiled_mt(T, nx * nz);
+    const int64_t ny = (T + 32 * mt - 1) / (32 * mt), wgs = nx * ny * nz;
+    e.map = tile_map(nx, ny, nz, 32 * mt);
+    const dim3 grid((unsigned)wgs), block(256);
+#define NVR_TILED(NS_, MT_, BYTES_) gemm_tiled_kernel<EPI, NS_, MT_><<<grid, block, (NS_) * (BYTES_), s>>>(x, ldx, W, (int)T, (int)K, (int)N, (int)NW, y, e)
+    if (mt == 4) { if (wgs <= 256) NVR_TILED(3, 4, kStageBytes); else NVR_TILED(2, 4, kStageBytes); }
+    else if (mt == 2) { if (wgs <= 256) NVR_TILED(4, 2, kStageBytes64); else NVR_TILED(3, 2, kStageBytes64); }
+    else NVR_TILED(4, 1, kStageBytes32);
+#undef NVR_TILED
+}
 // > 64 KiB of dynamic LDS needs an opt-in per kernel instance; called at runner creation (never inside a stream capture)
 int gemm_tiled_prepare() {
     static bool done = false;
     if (done) return 0;
-#define NVR_TILED_ATTR(EPI_)                                                                                          \
-    { hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tiled_kernel<EPI_, 4>), hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                         (int)(4 * kStageBytes));                                                    \
-      if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tiled_kernel<EPI_, RING64, 2>),   \
-                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(RING64 * kStageBytes64)); \
-      if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tiled_kernel<EPI_, RING32, 1>),   \
-                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(RING32 * kStageBytes32)); \
+#define NVR_TILED_ATTR1(EPI_, NS_, MT_, BYTES_)                                                                                                                   \
+    { hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tiled_kernel<EPI_, NS_, MT_>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(NS_ * BYTES_)); \
       if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "gemm_tiled: LDS opt-in failed: %s", hipGetErrorString(e)); }
+#define NVR_TILED_ATTR(EPI_) NVR_TILED_ATTR1(EPI_, 3, 4, kStageBytes) NVR_TILED_ATTR1(EPI_, 4, 2, kStageBytes64) NVR_TILED_ATTR1(EPI_, 3, 2, kStageBytes64) NVR_TILED_ATTR1(EPI_, 4, 1, kStageBytes32)
     NVR_TILED_ATTR(TEPI_F16) NVR_TILED_ATTR(TEPI_SILU) NVR_TILED_ATTR(TEPI_ROPE) NVR_TILED_ATTR(TEPI_LMHEAD) NVR_TILED_ATTR(TEPI_SLAB)
 #undef NVR_TILED_ATTR
+#undef NVR_TILED_ATTR1
     if (hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tiled_silu96_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, RING96 * S96_BUF) != hipSuccess)
         return nvr::fail(NVR_ERR_HIP, "gemm_tiled: LDS opt-in failed (96-row SiLU tiles)");
     done = true;
@@ -517,14 +593,13 @@ bool gemm_tiled_lm_head_ok(int64_t T, int64_t K, int64_t N, int64_t ldx) {
            N < (1ll << 31);
 }
 int gemm_tiled_lm_head(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, float *logits,
-                       float *part_val, int32_t *part_idx, int32_t *nparts, hipStream_t s) {
+                       float *part_val, int32_t *part_idx, int32_t *nparts, hipStream_t s, const half_bits *Wt) {
     if (!gemm_tiled_lm_head_ok(T, K, N, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_lm_head: T=%ld K=%ld N=%ld", (long)T, (long)K, (long)N);
     TileEpi e{};
     e.logits = logits; e.pval = part_val; e.pidx = part_idx;
-    dim3 grid((unsigned)((N + BN - 1) / BN), (unsigned)((T + BM - 1) / BM));
-    *nparts = (int32_t)grid.x;
+    *nparts = (int32_t)((N + BN - 1) / BN);
     if (int rc = gemm_tiled_prepare()) return rc;
-    NVR_TILED_LAUNCH(TEPI_LMHEAD, grid, T, (const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K, (int)N, (int)N, nullptr, e);
+    tiled_launch<TEPI_LMHEAD>(*nparts, 1, x, ldx, W, Wt, T, K, N, N, nullptr, e, s);
     return tiled_check("gemm_tiled_lm_head");
 }
 
@@ -532,52 +607,48 @@ int gemm_tiled_lm_head(const half_bits *x, int64_t ldx, const half_bits *W, int6
 bool gemm_tiled_splitk_ok(int64_t T, int64_t K, int64_t N, int64_t S, int64_t ldx) {
     return tiled_enabled() && T > 32 && S >= 1 && K % (S * BK) == 0 && N % 16 == 0 && ldx % 8 == 0;
 }
-int gemm_tiled_splitk(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, int64_t S, float *slabs, hipStream_t s) {
+int gemm_tiled_splitk(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, int64_t S, float *slabs, hipStream_t s, const half_bits *Wt) {
     if (!gemm_tiled_splitk_ok(T, K, N, S, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_splitk: T=%ld K=%ld N=%ld S=%ld", (long)T, (long)K, (long)N, (long)S);
     if (int rc = gemm_tiled_prepare()) return rc;
     TileEpi e{};
     e.slabs = slabs; e.slab_stride = T * N; e.kslice = (int32_t)(K / S);
-    dim3 grid((unsigned)((N + BN - 1) / BN), (unsigned)((T + BM - 1) / BM), (unsigned)S);
-    NVR_TILED_LAUNCH(TEPI_SLAB, grid, T, (const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K, (int)N, (int)N, nullptr, e);
+    tiled_launch<TEPI_SLAB>((N + BN - 1) / BN, S, x, ldx, W, Wt, T, K, N, N, nullptr, e, s);
     return tiled_check("gemm_tiled_splitk");
 }
 
 bool gemm_tiled_ok(int64_t T, int64_t K, int64_t N, int64_t ldx) { return tiled_enabled() && T > 32 && K % BK == 0 && N % 16 == 0 && ldx % 8 == 0; }
 
-int gemm_tiled(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *y, hipStream_t s) {
+int gemm_tiled(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *y, hipStream_t s, const half_bits *Wt) {
     if (!gemm_tiled_ok(T, K, N, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled: T=%ld K=%ld N=%ld", (long)T, (long)K, (long)N);
-    dim3 grid((unsigned)((N + BN - 1) / BN), (unsigned)((T + BM - 1) / BM));
     if (int rc = gemm_tiled_prepare()) return rc;
-    NVR_TILED_LAUNCH(TEPI_F16, grid, T, (const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K, (int)N, (int)N, (half_t *)y, TileEpi{});
+    tiled_launch<TEPI_F16>((N + BN - 1) / BN, 1, x, ldx, W, Wt, T, K, N, N, (half_t *)y, TileEpi{}, s);
     return tiled_check("gemm_tiled");
 }
-int gemm_tiled_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s, bool gelu) {
+int gemm_tiled_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s, bool gelu, const half_bits *Wt) {
     if (!gemm_tiled_ok(T, K, I, ldx) || I % 64) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_silu_mul: T=%ld K=%ld I=%ld", (long)T, (long)K, (long)I);
-    dim3 grid((unsigned)(I / 64), (unsigned)((T + BM - 1) / BM));
     if (int rc = gemm_tiled_prepare()) return rc;
     {   // 96-row tiles when they put a workgroup on (nearly) every CU where the 128-row tiles leave a quarter of them idle (T = 512, I = 3072: 256 against 192;
         // T = 321..384: 192 against 144)
         const int64_t ty = (T + BM - 1) / BM, w128 = (I / 64) * ty, w96 = (I / 48) * ty;
-        if (!gelu && I % 48 == 0 && tiled_mt(T, I / 64) == 4 && tiled_ring((unsigned)w128) && w96 <= 256 && w96 > w128 && w128 * 8 <= w96 * 7) {
-            gemm_tiled_silu96_kernel<<<dim3((unsigned)(I / 48), (unsigned)ty), dim3(256), RING96 * S96_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K, (int)I, (half_t *)out);
+        if (!gelu && I % 48 == 0 && tiled_mt(T, I / 64) == 4 && w96 <= 256 && w96 > w128 && w128 * 8 <= w96 * 7) {
+            gemm_tiled_silu96_kernel<<<dim3((unsigned)(I / 48), (unsigned)ty), dim3(256), RING96 * S96_BUF, s>>>((const half_t *)x, ldx, (const half_t *)(Wt ? Wt : W), (int)T, (int)K, (int)I, (half_t *)out, Wt != nullptr);
             return tiled_check("gemm_tiled_silu_mul (96-row tiles)");
         }
     }
     TileEpi e{}; e.gelu = gelu ? 1 : 0;
-    NVR_TILED_LAUNCH(TEPI_SILU, grid, T, (const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K, (int)I, (int)(2 * I), (half_t *)out, e);
+    tiled_launch<TEPI_SILU>(I / 64, 1, x, ldx, W, Wt, T, K, I, 2 * I, (half_t *)out, e, s);
     return tiled_check("gemm_tiled_silu_mul");
 }
 int gemm_tiled_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D,
                               const int64_t *positions, const int32_t *slots, const float *cos_t, const float *sin_t, half_bits *qkv,
-                              half_bits *k_cache, half_bits *v_cache, hipStream_t s) {
+                              half_bits *k_cache, half_bits *v_cache, hipStream_t s, const half_bits *Wt, bool kv_cache_only) {
     const int64_t N = (H + 2 * KVH) * D;
     if (!gemm_tiled_ok(T, K, N, ldx) || D % 16 || 128 % D) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_qkv_rope_store: T=%ld K=%ld D=%ld", (long)T, (long)K, (long)D);
     TileEpi e{};
     e.pos = positions; e.slots = slots; e.cos_t = cos_t; e.sin_t = sin_t; e.kc = (half_t *)k_cache; e.vc = (half_t *)v_cache;
-    e.H = (int32_t)H; e.KVH = (int32_t)KVH; e.D = (int32_t)D;
-    dim3 grid((unsigned)((N / 16 + 7) / 8), (unsigned)((T + BM - 1) / BM));
+    e.H = (int32_t)H; e.KVH = (int32_t)KVH; e.D = (int32_t)D; e.kv_cache_only = kv_cache_only;
     if (int rc = gemm_tiled_prepare()) return rc;
-    NVR_TILED_LAUNCH(TEPI_ROPE, grid, T, (const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K, (int)N, (int)N, (half_t *)qkv, e);
+    tiled_launch<TEPI_ROPE>((N / 16 + 7) / 8, 1, x, ldx, W, Wt, T, K, N, N, (half_t *)qkv, e, s);
     return tiled_check("gemm_tiled_qkv_rope_store");
 }
 

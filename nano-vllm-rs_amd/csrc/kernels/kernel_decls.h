@@ -107,20 +107,21 @@ int linear_stream_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bit
 
 // LM head over more than 32 rows: the 128x128 kernel with the logits / arg-max epilogue (one partial per 128-column tile)
 bool gemm_tiled_splitk_ok(int64_t T, int64_t K, int64_t N, int64_t S, int64_t ldx);
-int gemm_tiled_splitk(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, int64_t S, float *slabs, hipStream_t s);
+// Wt (here and below): the tiled copy of W (retile_weight), read in its place
+int gemm_tiled_splitk(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, int64_t S, float *slabs, hipStream_t s, const half_bits *Wt = nullptr);
 int gemm_tiled_prepare();                                                   // LDS opt-in of the ring instances (call outside captures)
 bool gemm_tiled_lm_head_ok(int64_t T, int64_t K, int64_t N, int64_t ldx);
 int gemm_tiled_lm_head(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, float *logits,
-                       float *part_val, int32_t *part_idx, int32_t *nparts, hipStream_t s);
+                       float *part_val, int32_t *part_idx, int32_t *nparts, hipStream_t s, const half_bits *Wt = nullptr);
 
 // LDS-tiled MFMA GEMM for the prefill regime (T >= 128): same results layout and epilogues as the kernels above
 bool gemm_tiled_ok(int64_t T, int64_t K, int64_t N, int64_t ldx);
-int gemm_tiled(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *y, hipStream_t s);
+int gemm_tiled(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *y, hipStream_t s, const half_bits *Wt = nullptr);
 int gemm_tiled_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out,
-                        hipStream_t s, bool gelu = false);
+                        hipStream_t s, bool gelu = false, const half_bits *Wt = nullptr);
 int gemm_tiled_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH,
                               int64_t D, const int64_t *positions, const int32_t *slots, const float *cos_t, const float *sin_t,
-                              half_bits *qkv, half_bits *k_cache, half_bits *v_cache, hipStream_t s);
+                              half_bits *qkv, half_bits *k_cache, half_bits *v_cache, hipStream_t s, const half_bits *Wt = nullptr, bool kv_cache_only = false);
 
 // 256x256x64 eight-wave MFMA GEMM (T >= 256, N % 256 == 0 / I % 128 == 0 / whole heads per 256 rows): same results
 // layout and epilogues; preferred over gemm_tiled when its shape test passes

@@ -319,14 +319,15 @@ static void launch(const half_t *x, int64_t ldx, const half_t *W, int T, int K, 
     linear_skinny_kernel<NT, MT, WAVES, EPI><<<grid, dim3(WAVES * 64), 0, s>>>(x, ldx, W, T, K, N, y, e);
 }
 
-// 256x256 kernel or 128x128 kernel?  Fitted to the sweep (us, profiles/r01_gemm_ablation.txt): a wave of <= 256 tiles costs
-// 17*K/1024 + 20 on the 256x256 kernel (long single-tile latency); the 128x128 kernel costs 15*K/1024 while its tiles fit one per
-// CU and 21*K/1024 per wave of 512 (two workgroups per CU) beyond that, + 5 per launch.  N = W rows
+// 256x256 kernel or 128x128 kernel?  Fitted to both over 22 token counts (100..8192) x the projections of Qwen3-0.6B and Qwen3-8B, weights from HBM.  A round of <= 256 tiles of the
+// 256x256 kernel takes 18.5 K/1024 + 8 us however few there are (K = 1024 25 us, 2048 39, 4096 81, 12288 235).  The 128x128 kernel takes 9.4 K/1024 + 3.5 us while its tiles fit one per CU
+// (13.3 / 22 / 42 / 118), beyond that 8 K/1024 + 1.2 per 256 tiles, a last part of a round counted half (768 tiles 31, 1152 45, 2048 73 at K = 1024).  us of both, 256 / 128: qkv of 0.6B 27.1 /
+// 20.4 at 2048 tokens, 27.4 / 29.4 at 2560, 49.8 / 45.6 at 4672; o_proj 44.8 / 34.4 at 8192; 8B qkv 84.6 / 64.7 at 1280, 82.9 / 100.1 at 1536, 166 / 153 at 3062.  N = W rows
 static inline bool prefer_256(int64_t T, int64_t K, int64_t N) {
     const int64_t t256 = ((N + 255) / 256) * ((T + 255) / 256), t128 = ((N + 127) / 128) * ((T + 127) / 128);
-    const double kk = (double)K / 1024.0;
-    const double c256 = (double)((t256 + 255) / 256) * (17.0 * kk + 20.0);
-    const double c128 = (t128 <= 256 ? 15.0 * kk : (double)((t128 + 511) / 512) * 21.0 * kk) + 5.0;
+    const double kk = (double)K / 1024.0, rounds = (double)t128 / 256.0;
+    const double c256 = (double)((t256 + 255) / 256) * (18.5 * kk + 8.0);
+    const double c128 = t128 <= 256 ? 9.4 * kk + 3.5 : 0.5 * (rounds + (double)((t128 + 255) / 256)) * (8.0 * kk + 1.2) + 2.0;
     return c256 < c128;
 }
 // one rule for the plain and the fused launchers (N = output features), so that a fused GEMM and its unfused twin run the same kernel
@@ -368,7 +369,7 @@ static int linear_routed(const half_bits *x, int64_t ldx, const half_bits *W, in
     // own single-tile latency (21-31 us) loses to the weight-streaming kernel run over 32-token blocks while T or T*N is small
     if (!y_f32 && gemm256_ok(T, K, N, ldx) && prefer_256(T, K, N)) return act ? gemm256_gelu(x, ldx, W, T, K, N, (half_bits *)y, s) : gemm256(x, ldx, W, T, K, N, (half_bits *)y, s);   // prefill regime
     if (gelu) *gelu = false;                               // (the tiled and the streaming kernel have no such epilogue)
-    if (!y_f32 && gemm_tiled_ok(T, K, N, ldx) && !prefer_stream(T, N)) return gemm_tiled(x, ldx, W, T, K, N, (half_bits *)y, s);
+    if (!y_f32 && gemm_tiled_ok(T, K, N, ldx) && !prefer_stream(T, N)) return gemm_tiled(x, ldx, W, T, K, N, (half_bits *)y, s, Wt);
     if (!y_f32 && linear_stream_ok(T, K, N, ldx)) return linear_stream(x, ldx, W, T, K, N, (half_bits *)y, s, Wt);   // large weights
     const half_t *xx = (const half_t *)x, *ww = (const half_t *)(Wt ? Wt : W);
     const int t = (int)T, k = (int)K, n = (int)N;
@@ -422,7 +423,7 @@ int linear_splitk(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T
     if (K % (32 * S) || N % 16 || ldx % 8 || S < 1)
         return nvr::fail(NVR_ERR_UNSUPPORTED, "linear_splitk: K=%ld must be a multiple of 32*S (S=%ld), N=%ld of 16", (long)K, (long)S, (long)N);
     if (T == 0) return 0;
-    if (splitk_prefers_tiles(T, K, N) && gemm_tiled_splitk_ok(T, K, N, S, ldx)) return gemm_tiled_splitk(x, ldx, W, T, K, N, S, slabs, s);   // LDS tiles
+    if (splitk_prefers_tiles(T, K, N) && gemm_tiled_splitk_ok(T, K, N, S, ldx)) return gemm_tiled_splitk(x, ldx, W, T, K, N, S, slabs, s, Wt);   // LDS tiles
     LinEpi e{};
     e.kslice = (int32_t)(K / S); e.slab_stride = T * N;
     if (Wt) { W = Wt; e.tiled = 1; }
@@ -447,7 +448,7 @@ static int linear_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64
         return nvr::fail(NVR_ERR_UNSUPPORTED, "linear_silu_mul: K=%ld must be a multiple of 32, I=%ld of 16", (long)K, (long)I);
     if (T == 0) return 0;
     if (gemm256_silu_ok(T, K, I, ldx) && prefer_256(T, K, 2 * I)) return gelu ? gemm256_gelu_mul(x, ldx, W, T, K, I, out, s) : gemm256_silu_mul(x, ldx, W, T, K, I, out, s);   // see linear()
-    if (gemm_tiled_ok(T, K, I, ldx) && I % 64 == 0 && !prefer_stream(T, 2 * I)) return gemm_tiled_silu_mul(x, ldx, W, T, K, I, out, s, gelu);
+    if (gemm_tiled_ok(T, K, I, ldx) && I % 64 == 0 && !prefer_stream(T, 2 * I)) return gemm_tiled_silu_mul(x, ldx, W, T, K, I, out, s, gelu, Wt);
     if (linear_stream_silu_ok(T, K, I, ldx)) return linear_stream_silu_mul(x, ldx, W, T, K, I, out, s, Wt, gelu);              // large weights
     const half_t *xx = (const half_t *)x, *ww = (const half_t *)(Wt ? Wt : W);
     LinEpi e{};
@@ -511,7 +512,7 @@ int linear_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, i
     if (gemm256_rope_ok(T, K, H, KVH, D, ldx) && prefer_256(T, K, (H + 2 * KVH) * D))                                  // see linear()
         return gemm256_qkv_rope_store(x, ldx, W, T, K, H, KVH, D, positions, slots, cos_t, sin_t, qkv, k_cache, v_cache, s, kv_cache_only);
     if (gemm_tiled_ok(T, K, (H + 2 * KVH) * D, ldx) && 128 % D == 0 && !prefer_stream(T, (H + 2 * KVH) * D))
-        return gemm_tiled_qkv_rope_store(x, ldx, W, T, K, H, KVH, D, positions, slots, cos_t, sin_t, qkv, k_cache, v_cache, s);
+        return gemm_tiled_qkv_rope_store(x, ldx, W, T, K, H, KVH, D, positions, slots, cos_t, sin_t, qkv, k_cache, v_cache, s, Wt, kv_cache_only);
     if (linear_stream_rope_ok(T, K, H, KVH, D, ldx))                                                                  // large weights
         return linear_stream_qkv_rope_store(x, ldx, W, T, K, H, KVH, D, positions, slots, cos_t, sin_t, qkv, k_cache, v_cache, s, Wt);
     const half_t *xx = (const half_t *)x, *ww = (const half_t *)(Wt ? Wt : W);

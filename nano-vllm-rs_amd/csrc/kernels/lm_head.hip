@@ -341,7 +341,7 @@ int lm_head(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int6
         if (gemm256_lm_head_ok(T, K, N, ldx))                          // >= 256 rows: 256x256 tiles (r06), same outputs
             return gemm256_lm_head(x, ldx, W, T, K, N, store_logits ? logits : nullptr, part_val, part_idx, nparts, s);
         if (gemm_tiled_lm_head_ok(T, K, N, ldx))                       // more than 32 rows: 128x128 tiles, same outputs
-            return gemm_tiled_lm_head(x, ldx, W, T, K, N, store_logits ? logits : nullptr, part_val, part_idx, nparts, s);
+            return gemm_tiled_lm_head(x, ldx, W, T, K, N, store_logits ? logits : nullptr, part_val, part_idx, nparts, s, Wt);
         return nvr::fail(NVR_ERR_UNSUPPORTED, "lm_head: T=%ld K=%ld N=%ld (T <= 32: K multiple of 256 (above 2048: in equal chunks of <= 2048 that are multiples of 256); T > 32: K multiple of 64, "
                          "N <= 128 * %d; N multiple of 16)", (long)T, (long)K, (long)N, LM_HEAD_MAX_PARTS);
     }

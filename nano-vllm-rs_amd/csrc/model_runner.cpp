@@ -836,7 +836,7 @@ int nvr_model_runner::forward_prefill_two(int64_t T, int64_t B) {
     RC(KD(select_last_tokens(n, d_cu, B, Hd, nlast, st)));                                       // embed_head.rs:272-289
     if (lm_parts > 0) {
         int32_t np = 0;
-        RC(KD(lm_head(nlast, Hd, lm_head, B, Hd, Vl, logits, d_lm_pval, d_lm_pidx, &np, st, want_logits, (tiled_weights && B <= 32) ? lm_head_t : nullptr)));
+        RC(KD(lm_head(nlast, Hd, lm_head, B, Hd, Vl, logits, d_lm_pval, d_lm_pidx, &np, st, want_logits, tiled_weights ? lm_head_t : nullptr)));
         if (np != lm_parts) return nvr::fail(NVR_ERR_INVARIANT, "lm_head produced %d partials, planned %d", np, lm_parts);
     } else {
         RC(KD(linear(nlast, Hd, lm_head, B, Hd, Vl, logits, true, st)));
@@ -852,7 +852,7 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
     const int32_t *bt = dd_bt;
     if (f32) return forward_f32(T, B, is_prefill, max_ctx);
     if (is_prefill && tp_overlap == 2 && mb_rows > 0) return forward_prefill_two(T, B);
-    const bool tl = tiled_weights && T <= 64;                            // decode-sized steps stream the tiled weight copies
+    const bool tl = tiled_weights;                                       // (the 256-row tiles take the weights as they are: their W comes from L2)
     const bool embed_norm = L > 0 && KD(embedding_rmsnorm_ok(T, Hd));                    // decode-sized: K1 + the first norm in one launch
     if (embed_norm) RC(KD(embedding_rmsnorm(ids, T, embed, layers[0].ln1, mc.rms_norm_eps, Hd, h, n, st)));
     else RC(KD(embedding(ids, T, embed, Hd, h, st)));
@@ -937,7 +937,7 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
     if (is_prefill) { RC(KD(select_last_tokens(n, d_cu, B, Hd, nlast, st))); hl = nlast; }      // embed_head.rs:272-289
     if (lm_parts > 0) {                                                                        // f32 logits (A-21) + arg-max partials
         int32_t np = 0;
-        RC(KD(lm_head(hl, Hd, lm_head, B, Hd, Vl, logits, d_lm_pval, d_lm_pidx, &np, st, want_logits, (tiled_weights && B <= 32) ? lm_head_t : nullptr)));
+        RC(KD(lm_head(hl, Hd, lm_head, B, Hd, Vl, logits, d_lm_pval, d_lm_pidx, &np, st, want_logits, tiled_weights ? lm_head_t : nullptr)));
         if (np != lm_parts) return nvr::fail(NVR_ERR_INVARIANT, "lm_head produced %d partials, planned %d", np, lm_parts);
     } else {
         RC(KD(linear(hl, Hd, lm_head, B, Hd, Vl, logits, true, st)));
@@ -1446,7 +1446,7 @@ int nvr_model_runner::ensure_logits() {
     NVR_HIP_CHECK(hipSetDevice(device));
     int32_t np = 0;
     RC(KD(lm_head(lm_input, Hd, lm_head, (int64_t)last_rows, Hd, Vl, logits, d_lm_pval, d_lm_pidx, &np, stream, true,
-                  (tiled_weights && last_rows <= 32) ? lm_head_t : nullptr)));
+                  tiled_weights ? lm_head_t : nullptr)));
     logits_valid = true;
     return NVR_OK;
 }

@@ -406,3 +406,93 @@ def test_layer_list_gated_head_norm_and_clamped_unit(dtype, heads, vdim, ff, bat
     d.step([("s%d" % i, t[:-2]) for i, t in enumerate(tokens)])
     got = [d.step([("s%d" % i, t[len(t) - 2 + k:len(t) - 1 + k]) for i, t in enumerate(tokens)]) for k in range(2)]
     _compare_layer_rows(cfg, w, dtype, base, [np.concatenate([g["s%d" % i] for g in got]) for i in range(batch)])
+
+
+def _bits(rng, shape, std):
+    """float16 numbers of a deviation."""
+    return (rng.standard_normal(shape) * std).astype(F16)
+
+
+def _copy_of(d_W, N, K, mode=0, H=0, KVH=0, D=0):
+    d_T = nvr.DeviceBuffer(N * K * 2)
+    nvr.check(nvr.lib().nvr_retile_weight(d_W.ptr, d_T.ptr, N, K, mode, H, KVH, D, None))
+    return d_T
+
+
+def _product_bound(x, W):
+    """|x . W^T rounded to float16 - exact|: K roundings to 24 bits of a sum of products, and one to 11 bits."""
+    ref = x.astype(np.float64) @ W.astype(np.float64).T
+    room = x.shape[1] * 2.0 ** -24 * (np.abs(x.astype(np.float64)) @ np.abs(W.astype(np.float64)).T)
+    return ref, np.abs(ref) * 2.0 ** -11 + room + 2.0 ** -25
+
+
+@pytest.mark.parametrize("T,K,N", [(97, 64, 4112), (129, 128, 4112), (255, 192, 2064), (200, 320, 4112), (301, 576, 4112), (700, 256, 1040), (1030, 1088, 4112)])
+def test_tile_products_of_few_k_tiles_and_ragged_edges(T, K, N):
+    """Products on 32-, 64- and 128-token tiles with fewer K-tiles than the ring holds, a column tile that is mostly past the edge and tiles that do not fill the XCDs' shares evenly: against
+    64 bits, and the tiled copy of the weights against the weights, bit for bit."""
+    rng, l = np.random.default_rng(T + K), nvr.lib()
+    x, W = _bits(rng, (T, K), 0.5), _bits(rng, (N, K), 0.1)
+    d_x, d_W = dev(x), dev(W)
+    d_T, ya, yb = _copy_of(d_W, N, K), nvr.DeviceBuffer(T * N * 2), nvr.DeviceBuffer(T * N * 2)
+    nvr.check(l.nvr_linear(d_x.ptr, K, d_W.ptr, T, K, N, ya.ptr, 0, None))
+    nvr.check(l.nvr_linear_tiled(d_x.ptr, K, d_W.ptr, d_T.ptr, T, K, N, yb.ptr, 0, None))
+    a, b = ya.to_numpy((T, N), F16), yb.to_numpy((T, N), F16)
+    assert np.array_equal(a.view(np.uint16), b.view(np.uint16))
+    ref, bound = _product_bound(x, W)
+    assert np.all(np.abs(a - ref) <= bound)
+    S = 2
+    if K % (64 * S) == 0:
+        sa, sb = nvr.DeviceBuffer(S * T * N * 4), nvr.DeviceBuffer(S * T * N * 4)
+        nvr.check(l.nvr_linear_splitk(d_x.ptr, K, d_W.ptr, T, K, N, S, sa.ptr, None))
+        nvr.check(l.nvr_linear_splitk_tiled(d_x.ptr, K, d_W.ptr, d_T.ptr, T, K, N, S, sb.ptr, None))
+        s = sa.to_numpy((S, T, N), np.float32)
+        assert np.array_equal(s, sb.to_numpy((S, T, N), np.float32))
+        assert np.all(np.abs(s.astype(np.float64).sum(0) - ref) <= bound)
+
+
+@pytest.mark.parametrize("T,K,I", [(97, 128, 3072), (200, 64, 4160), (509, 1024, 3072), (384, 192, 3072), (700, 320, 2112)])
+def test_tile_gate_up_forms(T, K, I):
+    """gate_up + SiLU on the tiles (128-row and 96-row ones): the tiled copy's bits, and every element within two roundings of the unit of the rounded products."""
+    rng, l = np.random.default_rng(T + I), nvr.lib()
+    x, W = _bits(rng, (T, K), 0.5), _bits(rng, (2 * I, K), 0.1)
+    d_x, d_W = dev(x), dev(W)
+    d_T, oa, ob, d_y = _copy_of(d_W, 2 * I, K), nvr.DeviceBuffer(T * I * 2), nvr.DeviceBuffer(T * I * 2), nvr.DeviceBuffer(T * 2 * I * 2)
+    nvr.check(l.nvr_linear_silu_mul(d_x.ptr, K, d_W.ptr, T, K, I, oa.ptr, None))
+    nvr.check(l.nvr_linear_silu_mul_tiled(d_x.ptr, K, d_W.ptr, d_T.ptr, T, K, I, ob.ptr, None))
+    nvr.check(l.nvr_linear(d_x.ptr, K, d_W.ptr, T, K, 2 * I, d_y.ptr, 0, None))           # the unfused product: the same sums
+    a = oa.to_numpy((T, I), F16)
+    assert np.array_equal(a.view(np.uint16), ob.to_numpy((T, I), F16).view(np.uint16))
+    y = d_y.to_numpy((T, 2 * I), F16).astype(np.float64)
+    want = y[:, :I] / (1 + np.exp(-y[:, :I])) * y[:, I:]
+    assert np.all(np.abs(a - want) <= np.abs(want) * 2.0 ** -10 + 2.0 ** -24)
+
+
+@pytest.mark.parametrize("T,K,H,KVH,D", [(200, 128, 30, 3, 64), (129, 64, 20, 6, 128), (333, 256, 41, 5, 32), (260, 64, 66, 3, 16), (700, 320, 8, 4, 128)])
+def test_tile_qkv_rope_store_forms(T, K, H, KVH, D):
+    """qkv + RoPE + store on the tiles: heads of 16..128 whose boundaries lie inside a wave's columns, tokens without a slot; the rotation of the product's own rounded values with every
+    operation rounded apart is exact, and so are the cache rows and the tiled copy."""
+    rng, l = np.random.default_rng(T + D), nvr.lib()
+    N, heads = (H + 2 * KVH) * D, H + KVH
+    x, W = _bits(rng, (T, K), 0.5), _bits(rng, (N, K), 0.1)
+    d_x, d_W = dev(x), dev(W)
+    d_T, d_y = _copy_of(d_W, N, K, 1, H, KVH, D), nvr.DeviceBuffer(T * N * 2)
+    nvr.check(l.nvr_linear(d_x.ptr, K, d_W.ptr, T, K, N, d_y.ptr, 0, None))
+    pos = rng.integers(0, 512, T).astype(np.int64)
+    slots = rng.permutation(1024)[:T].astype(np.int32)
+    slots[::7] = -1
+    cos, sin = oracle.rope_table(D, 512, 1e6)
+    d_pos, d_slots, d_cos, d_sin = dev(pos), dev(slots), dev(cos), dev(sin)
+    y = d_y.to_numpy((T, N), F16).reshape(T, H + 2 * KVH, D)
+    u, v = y[:, :heads, :D // 2].astype(np.float32), y[:, :heads, D // 2:].astype(np.float32)
+    c, s = np.asarray(cos, np.float32)[pos][:, None], np.asarray(sin, np.float32)[pos][:, None]
+    want = y.copy()
+    want[:, :heads, :D // 2], want[:, :heads, D // 2:] = (u * c - v * s).astype(F16), (v * c + u * s).astype(F16)
+    kept = slots >= 0
+    for fn, extra in ((l.nvr_linear_qkv_rope_store, ()), (l.nvr_linear_qkv_rope_store_tiled, (d_T.ptr,))):
+        q, kc, vc = nvr.DeviceBuffer(T * N * 2), dev(np.zeros((1024, KVH, D), F16)), dev(np.zeros((1024, KVH, D), F16))
+        nvr.check(fn(d_x.ptr, K, d_W.ptr, *extra, T, K, H, KVH, D, d_pos.ptr, d_slots.ptr, d_cos.ptr, d_sin.ptr, q.ptr, kc.ptr, vc.ptr, None))
+        assert np.array_equal(q.to_numpy((T, N), np.uint16), want.reshape(T, N).view(np.uint16))
+        for cache, first in ((kc, H), (vc, H + KVH)):
+            full = np.zeros((1024, KVH, D), F16)
+            full[slots[kept]] = want[kept, first:first + KVH]
+            assert np.array_equal(cache.to_numpy((1024, KVH, D), np.uint16), full.view(np.uint16))

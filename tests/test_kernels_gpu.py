@@ -979,8 +979,8 @@ def test_retile_weight_layout(N, K, mode, H, KVH, D):
 @pytest.mark.parametrize("T", [1, 32, 64, 200])
 def test_tiled_entry_points_match_row_major(T):
     """Every *_tiled entry point against its row-major twin on the Qwen3-0.6B shapes: identical bits (the tiled copy changes where
-    a weight byte lives, never which bytes meet in an MFMA or in which order they are summed); T = 200 takes the tile GEMMs, which
-    read the row-major W and ignore Wt."""
+    a weight byte lives, never which bytes meet in an MFMA or in which order they are summed); T = 200 takes the 128-row tile
+    GEMMs."""
     rng = np.random.default_rng(17 + T)
     l = nvr.lib()
     Hd, H, KVH, D, I = 1024, 16, 8, 128, 3072
