@@ -36,6 +36,14 @@ __device__ __forceinline__ float4_t mfma16(half8_t a, half8_t b, float4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 #endif
 }
+// D = A(32 x 16) . B(16 x 32) + C (v_mfma_f32_32x32x16_f16 / _bf16): lane l holds row / column l & 31 of A / B at k = 8 (l >> 5) .., and of D column l & 31 at rows 8 (e >> 2) + 4 (l >> 5) + (e & 3)
+__device__ __forceinline__ float16_t mfma32(half8_t a, half8_t b, float16_t c) {
+#ifdef NVR_BF16
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+#else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+#endif
+}
 // c + a.x * b.x + a.y * b.y in f32 (v_dot2_f32_f16 / v_dot2c_f32_bf16)
 __device__ __forceinline__ float dot2(half2_t a, half2_t b, float c) {
 #ifdef NVR_BF16

@@ -507,6 +507,262 @@ __global__ __launch_bounds__(64 * FLASH_WAVES, 8 / FLASH_WAVES) void flash_prefi
     }
 }
 
+// The plain causal form of heads of 128 (no penalty, window, gate or second map), the one that prompts of the dense graph take.  Same tiles, same 64-key steps, on 32 x 32 x 16 products:
+//   Sᵀ[32 keys, 32 queries]  A = K rows, B = the wave's 32 query rows (lane & 31; G = 2: two heads of 16 positions), 16 scores of one query per lane and 32-key tile;
+//   Oᵀ[32 d, 32 queries]     B = the exponentials of 16 keys as they lie in the score registers (k-slot (h, j) <-> key 8 (j / 4) + 4 h + j % 4, h = lane / 32), A = Vᵀ by
+//                            ds_read_b64_tr_b16 in the same key order.
+// What bounds it: the matrix cores and the exponentials (1024 + 512 cycles of a wave and step) as far as they run side by side.  A product of 16 x 16 x 32 holds its wave's issue for as long as
+// it takes; one of 32 x 32 x 16 leaves half of its 32 cycles to the wave's vector instructions, so a step is laid out as two blocks of 16 products with vector work of their own between them:
+//   block 1: Sᵀ of step i + 1 | the exponentials of step i's first 32 keys       block 2: Oᵀ of step i | the exponentials of its second 32 keys, the maxima of step i + 1
+// (K runs one step ahead of V through the LDS ring).  The running maximum of a query is raised only when a step exceeds it by 2^8 in the exponentials' unit: the rescaling of the
+// accumulators, 64 multiplications a step while maxima still move, then happens once or twice a tile; a query's decision does not depend on its wave's other queries, so its bits do not either.
+// bfloat16, G = 2, us before (16 x 16 x 32 products, a maximum per step) / now: 32 prompts of 1024 tokens 204 / 177 a layer, one of 509 15.8 / 12.9, of 2048 47.5 / 40.9, of 8192 330 / 301; 3814
+// tokens behind 11440 cached ones 191 / 172; 100 steps of one workgroup per CU 138 / 123, of two 214 / 201 (1.07 PFLOP/s: cycles fall by 23 %, the clock from 2.1 to 1.75 GHz).  Without the K reads
+// 171, without the V reads 188, without the exponentials 185, without the LDS-DMA 183, products and the rest of the vector work alone 127.
+constexpr float FLASH_SLACK = 8.0f;                             // log2 of what an exponential may exceed 1 by
+// N products, each followed by READS LDS reads (those of the product AHEAD products later) and VALU vector instructions
+template <int N, int READS, int AHEAD, int VALU>
+__device__ __forceinline__ void sched_pattern() {
+    __builtin_amdgcn_sched_group_barrier(0x100, READS * AHEAD, 0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        if (i < N - AHEAD) __builtin_amdgcn_sched_group_barrier(0x100, READS, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, VALU, 0);
+    }
+}
+template <int G, bool PAGED, bool UB>
+__global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
+    constexpr int D = 128, NT = 256, KT = 64, CPR = D / 8, PIECES = KT * CPR / NT, IMG = KT * D * 2;      // IMG: bytes of a K or V image of one step
+    static_assert(FLASH_WAVES == 4, "four waves share a tile");
+    __shared__ __attribute__((aligned(16))) char smem[4 * IMG];           // K of even / odd steps, V of even / odd steps
+    const int g = blockIdx.x % p.KVH;
+    const FlashTile tile = p.tiles[blockIdx.x / p.KVH];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, t = (lane >> 4) & 1, h = lane >> 5;
+    const int kv_end = tile.pos0 + tile.nq, nsteps = (kv_end + KT - 1) / KT;
+    // the lane's query: head and position
+    const int head = g * G + (G == 1 ? 0 : G == 2 ? t : (wave & 1) * 2 + t), pblk = G == 1 ? wave * 2 + t : G == 2 ? wave : (wave >> 1);
+    const int qi = pblk * 16 + r;
+    const bool qvalid = qi < tile.nq;
+    const int qc = qvalid ? qi : tile.nq - 1, qpos = tile.pos0 + qc, qrow = tile.q_row0 + qc;
+    half8_t qf[8];
+    const half_t *qptr = p.q + (int64_t)qrow * p.ldq + (int64_t)head * D + h * 8;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) qf[ks] = *reinterpret_cast<const half8_t *>(qptr + ks * 16);
+    // steps that hold a key for any query of this wave
+    const int mysteps = __builtin_amdgcn_readfirstlane((tile.pos0 + min(tile.nq - 1, (G == 1 ? wave * 2 + 1 : G == 2 ? wave : (wave >> 1)) * 16 + 15)) / KT + 1);
+
+    int bt_reg = 0, bt_chunk = -1;                                        // UB: register copy of 64 block-table entries (an asm load that waits for itself: see flash_prefill_kernel)
+    auto load_bt_chunk = [&](int c) {
+        bt_chunk = c;
+        const int32_t *src = p.block_tables + (int64_t)tile.kv_ref * p.max_blocks + min((c << 6) + lane, p.max_blocks - 1);
+        asm volatile("global_load_dword %0, %1, off\n\ts_waitcnt vmcnt(0)" : "=v"(bt_reg) : "v"(src) : "memory");
+    };
+    if (PAGED && UB) load_bt_chunk(0);
+    const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) char *)smem;
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    // images: [key][16-byte chunks]; K chunk ^ (key & 15): 16 keys of one chunk lie in 16 slots of a 256-byte bank row; V chunk ^ (key & 3) << 2: the 4 keys x 64 bytes that 32 lanes read
+    // transposed lie in the four quarters of one
+    // A thread's PIECES pieces of an image are one chunk of rows 16 apart: one offset in bytes per operand, the rest of the address is uniform.
+    const int srow = threadIdx.x / CPR, sc = threadIdx.x % CPR;
+    const int64_t row_elems = PAGED ? (int64_t)p.KVH * D : p.ldkv;        // cache / tensor row to row
+    const int32_t koff = (int32_t)(((int64_t)srow * row_elems + (int64_t)g * D + (sc ^ srow) * 8) * 2), voff = (int32_t)(((int64_t)srow * row_elems + (int64_t)g * D + (sc ^ ((srow & 3) << 2)) * 8) * 2);
+    static_assert(NT / CPR == 16 && PIECES == 4, "a piece's row is srow + 16 i");
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) asm volatile("" :: "v"(qf[ks]));       // landed before the first LDS-DMA goes out (see flash_prefill_kernel)
+    // K (v = 0) or V (v = 1) of step `it` into its image
+    auto stage = [&](int v, int it) {
+        const int kt = it * KT;
+        const half_t *base = v ? p.v : p.k;
+        const unsigned lds = (unsigned)__builtin_amdgcn_readfirstlane((int)(lds_base + (v * 2 + (it & 1)) * IMG + wave_u * 1024));
+        int64_t row0 = 0;                                                 // UB: cache row of the step's block's first key
+        if (PAGED && UB) {                                                // (every key of the step is in one block)
+            const int bi = kt >> p.bs_shift;
+            if ((bi >> 6) != bt_chunk) load_bt_chunk(bi >> 6);
+            row0 = (int64_t)__builtin_amdgcn_readlane(bt_reg, bi & 63) * p.block_size;
+        }
+        if ((!PAGED || UB) && kt + KT <= kv_end) {
+            const half_t *b0 = base + (PAGED ? row0 + (kt & (p.block_size - 1)) : (int64_t)(tile.kv_ref + kt)) * row_elems;
+            const half_t *b1 = b0 + 16 * row_elems, *b2 = b1 + 16 * row_elems, *b3 = b2 + 16 * row_elems;
+            unsigned keep;
+            asm volatile("s_mov_b32 %0, m0\n\t"
+                         "s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %3\n\t"
+                         "s_add_u32 m0, m0, %[st]\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %4\n\t"
+                         "s_add_u32 m0, m0, %[st]\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %5\n\t"
+                         "s_add_u32 m0, m0, %[st]\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %6\n\t"
+                         "s_mov_b32 m0, %0"
+                         : "=&s"(keep)
+                         : "v"(v ? voff : koff), "s"(lds), "s"(b0), "s"(b1), "s"(b2), "s"(b3), [st] "n"(NT * 16)
+                         : "memory", "scc");
+        } else {
+            int row_o = srow, chunk_o = sc;                               // (opaque: hipcc would keep every piece's address in registers over the whole loop)
+            asm volatile("" : "+v"(row_o), "+v"(chunk_o));
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i) {
+                const int row = row_o + 16 * i;
+                const int key = min(kt + row, kv_end - 1);                // keys beyond the last visible one are clamped to it (and masked)
+                int64_t at;
+                if (PAGED && UB) at = row0 + (key & (p.block_size - 1));
+                else if (PAGED) {
+                    int bi, bo;
+                    if (p.bs_shift >= 0) { bi = key >> p.bs_shift; bo = key & (p.block_size - 1); }
+                    else { bi = key / p.block_size; bo = key - bi * p.block_size; }
+                    at = (int64_t)p.block_tables[(int64_t)tile.kv_ref * p.max_blocks + bi] * p.block_size + bo;
+                } else at = tile.kv_ref + key;
+                const half_t *src = base + at * row_elems + (int64_t)g * D + (chunk_o ^ (v ? (row & 3) << 2 : row & 15)) * 8;
+                unsigned keep;
+                asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(src), "s"(lds + i * NT * 16) : "memory");
+            }
+        }
+    };
+    // LDS addresses: K fragment (32-key tile mt, k-step ks): key mt 32 + (lane & 31), chunk 2 ks + h; V fragment (16 keys k, 32 columns dt): keys k 16 + 4 h + r / 4 and 8 behind
+    const int krow = lane & 31;
+    unsigned ka = (krow * CPR + (h ^ (krow & 15))) * 16, va = 2 * IMG + (h * 4 + (r >> 2)) * (D * 2) + (((t * 2 + ((r & 3) >> 1)) ^ ((r >> 2) << 2)) << 4) + ((r & 1) << 3);
+    // (both move between the images of even and odd steps; the 12 addresses formed from them are formed anew in each step: registers are short)
+    unsigned kas[8], vas[4];
+    auto addresses = [&]() {
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) { kas[ks] = ka ^ (ks << 5); asm volatile("" : "+v"(kas[ks])); }
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) { vas[dt] = va ^ (dt << 6); asm volatile("" : "+v"(vas[dt])); }
+    };
+    auto read_k = [&](int mt, int ks) { return *reinterpret_cast<const half8_t *>(smem + kas[ks] + mt * 32 * D * 2); };
+    auto read_v = [&](int k, int dt) {
+        const half4_t a0 = lds_read_tr16(smem + vas[dt] + k * 16 * D * 2), a1 = lds_read_tr16(smem + vas[dt] + (k * 16 + 8) * D * 2);
+        return __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+
+    float16_t o[4], s0, s1;                                               // s0, s1: scores of a step's first and second 32 keys
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) o[dt] = (float16_t)(0.f);
+    const float cs = p.scale * 1.44269504088896340736f, slack = FLASH_SLACK / cs;      // the softmax runs on raw scores: p = 2^((s - m) cs)
+    float m = -INFINITY, l = 0.f;
+    if (p.sink) { m = p.sink[head] / p.scale; l = h == 0 ? 1.f : 0.f; }   // (l: this half wave's keys)
+    half2_t one2;
+    one2[0] = one2[1] = (half_t)1.0f;
+
+    auto scores = [&](float16_t &c, float16_t &d) {
+        c = (float16_t)(0.f); d = (float16_t)(0.f);
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) { c = mfma32(read_k(0, ks), qf[ks], c); d = mfma32(read_k(1, ks), qf[ks], d); }
+    };
+    auto mask = [&](int kt, float16_t &d) {                               // 32 keys from kt on
+        const int room = qpos - kt - 4 * h;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)                                      // (written out: hipcc keeps the conditions in scalar registers, and other values leave those for memory)
+            asm("v_cmp_gt_i32 vcc, %1, %2\n\tv_cndmask_b32 %0, %0, %3, vcc" : "+v"(d[e]) : "n"((e >> 2) * 8 + (e & 3)), "v"(room), "v"(-INFINITY) : "vcc");
+    };
+    auto maximum = [&](const float16_t &c, const float16_t &d) {
+        float a = fmaxf(c[0], c[1]), b = fmaxf(d[0], d[1]);
+#pragma unroll
+        for (int e = 2; e < 16; e += 2) { a = fmaxf(fmaxf(a, c[e]), c[e + 1]); b = fmaxf(fmaxf(b, d[e]), d[e + 1]); }
+        return xor32_partner_max(fmaxf(a, b));
+    };
+    auto raise = [&](float mx) {
+        const bool up = mx > m + slack;                                   // (finite from the first step on: key 0 <= qpos)
+        if (__any(up)) {
+            const float mn = up ? mx : m, alpha = __builtin_amdgcn_exp2f((m - mn) * cs);
+            m = mn; l *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
+        }
+    };
+    // exponentials of 16 keys of a step, and their sum as the products see them
+    auto exponentials = [&](const float16_t &d, int k, float mc) {        // keys 16 k .. of the 32
+        half8_t pf;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) pf[j] = (half_t)__builtin_amdgcn_exp2f(fmaf(d[k * 8 + j], cs, mc));
+        return pf;
+    };
+    auto add_up = [&](half8_t pf) {
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) l = dot2((half2_t){pf[j], pf[j + 1]}, one2, l);
+    };
+    auto values = [&](int k, half8_t pf) {
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) o[dt] = mfma32(read_v(k, dt), pf, o[dt]);
+    };
+    auto request = [&](int it) {
+        if (it + 2 < nsteps) stage(0, it + 2);
+        if (it + 1 < nsteps) stage(1, it + 1);
+    };
+    auto close = [&]() {                                                  // what was requested at the start of the step has landed for every wave, and every wave has read its images
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+    };
+
+    stage(0, 0); stage(1, 0);
+    if (nsteps > 1) stage(0, 1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    addresses();
+    scores(s0, s1);
+    if (KT - 1 > tile.pos0) { mask(0, s0); mask(32, s1); }
+    raise(maximum(s0, s1));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();                                         // (K of step 2 takes the place of K of step 0)
+    int it = 0;
+    for (; it + 1 < mysteps; ++it) {                                      // a step and the scores of the one behind it
+        request(it);
+        ka ^= IMG;
+        addresses();
+        const float mc = -m * cs;
+        half8_t pf[4];
+        float16_t n0, n1;
+        __builtin_amdgcn_sched_barrier(0);
+        scores(n0, n1);
+        pf[0] = exponentials(s0, 0, mc); pf[1] = exponentials(s0, 1, mc);
+        sched_pattern<16, 1, 4, 3>();
+        asm volatile("" : "+v"(pf[0]), "+v"(pf[1]));                      // (hipcc would move the exponentials behind the branch, to their uses)
+        __builtin_amdgcn_sched_barrier(0);
+        if ((it + 2) * KT - 1 > tile.pos0) { mask((it + 1) * KT, n0); mask((it + 1) * KT + 32, n1); }      // a step that reaches past the tile's first query
+        __builtin_amdgcn_sched_barrier(0);
+        values(0, pf[0]); values(1, pf[1]);
+        pf[2] = exponentials(s1, 0, mc); pf[3] = exponentials(s1, 1, mc);
+        values(2, pf[2]); values(3, pf[3]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) add_up(pf[k]);
+        const float mx = maximum(n0, n1);
+        s0 = n0; s1 = n1;
+        sched_pattern<16, 2, 2, 5>();
+        __builtin_amdgcn_sched_barrier(0);
+        raise(mx);
+        va ^= IMG;
+        close();
+    }
+    {                                                                     // the wave's last step
+        request(it);
+        addresses();
+        const float mc = -m * cs;
+        half8_t pf[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) { pf[k] = exponentials(k < 2 ? s0 : s1, k & 1, mc); add_up(pf[k]); }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) values(k, pf[k]);
+        close();
+    }
+    for (++it; it < nsteps; ++it) { request(it); close(); }               // steps of the tile's later queries
+    l = xor32_partner_sum(l);
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    half_t *orow = p.out + (int64_t)qrow * p.ldo + (int64_t)head * D + h * 8;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; e += 8) {
+            // columns e + 4 h .. and e + 8 + 4 h ..: the half waves trade, and each holds 8 consecutive columns
+            union { half_t v[8]; unsigned u[4]; } x;
+            union { half8_t v; unsigned u[4]; } y;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x.v[j] = (half_t)(o[dt][e + j] * inv);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const auto sw = __builtin_amdgcn_permlane32_swap(x.u[j], x.u[2 + j], false, false);
+                y.u[j] = sw[0]; y.u[2 + j] = sw[1];
+            }
+            if (qvalid) *reinterpret_cast<half8_t *>(orow + dt * 32 + e * 2) = y.v;
+        }
+}
+
 bool flash_prefill_ok(int D, int H, int KVH) {
     if (KVH <= 0 || H % KVH) return false;
     const int G = H / KVH;
@@ -539,6 +795,19 @@ int flash_prefill(const FlashArgs &a, bool paged, hipStream_t s) {
     const int G = a.H / a.KVH;
     dim3 grid((unsigned)((int64_t)a.ntiles * a.KVH)), block(64 * FLASH_WAVES);
     const bool ub = paged && p.bs_shift >= 0 && a.block_size % NVR_FLASH_KT == 0;
+    if (a.D == 128 && !diff && !gate && !pen) {
+#define NVR_FLASH_PLAIN(GG)                                                                           \
+    if (G == GG) {                                                                                    \
+        if (ub) flash_plain_kernel<GG, true, true><<<grid, block, 0, s>>>(p);                         \
+        else if (paged) flash_plain_kernel<GG, true, false><<<grid, block, 0, s>>>(p);                \
+        else flash_plain_kernel<GG, false, false><<<grid, block, 0, s>>>(p);                          \
+    }
+        NVR_FLASH_PLAIN(1) NVR_FLASH_PLAIN(2) NVR_FLASH_PLAIN(4)
+#undef NVR_FLASH_PLAIN
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "flash_prefill launch failed: %s", hipGetErrorString(e));
+        return 0;
+    }
 #define NVR_FLASH(DD, GG)                                                                             \
     if (a.D == DD && G == GG) {                                                                       \
         if (diff && ub) flash_prefill_kernel<DD, GG, true, true, false, false, false, true><<<grid, block, 0, s>>>(p);   \
@@ -547,9 +816,11 @@ int flash_prefill(const FlashArgs &a, bool paged, hipStream_t s) {
         else if (gate) flash_prefill_kernel<DD, GG, true, false, false, false, true><<<grid, block, 0, s>>>(p);   \
         else if (pen && ub) flash_prefill_kernel<DD, GG, true, true, false, true><<<grid, block, 0, s>>>(p);   \
         else if (pen) flash_prefill_kernel<DD, GG, true, false, false, true><<<grid, block, 0, s>>>(p);   \
-        else if (ub) flash_prefill_kernel<DD, GG, true, true><<<grid, block, 0, s>>>(p);              \
-        else if (paged) flash_prefill_kernel<DD, GG, true><<<grid, block, 0, s>>>(p);                 \
-        else flash_prefill_kernel<DD, GG, false><<<grid, block, 0, s>>>(p);                           \
+        else if constexpr (DD == 64) {                                                                \
+            if (ub) flash_prefill_kernel<DD, GG, true, true><<<grid, block, 0, s>>>(p);               \
+            else if (paged) flash_prefill_kernel<DD, GG, true><<<grid, block, 0, s>>>(p);             \
+            else flash_prefill_kernel<DD, GG, false><<<grid, block, 0, s>>>(p);                       \
+        }                                                                                             \
     }
     NVR_FLASH(128, 1) NVR_FLASH(128, 2) NVR_FLASH(128, 4) NVR_FLASH(64, 1) NVR_FLASH(64, 2) NVR_FLASH(64, 4)
 #undef NVR_FLASH

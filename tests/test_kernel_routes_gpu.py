@@ -496,3 +496,60 @@ def test_tile_qkv_rope_store_forms(T, K, H, KVH, D):
             full = np.zeros((1024, KVH, D), F16)
             full[slots[kept]] = want[kept, first:first + KVH]
             assert np.array_equal(cache.to_numpy((1024, KVH, D), np.uint16), full.view(np.uint16))
+
+
+def _prefill(q, ctx, nq, k, v, tables, H, KVH, D, bs):
+    """nvr_attn_prefill_paged of sequences of ctx tokens whose last nq are queries."""
+    T, B = int(sum(nq)), len(nq)
+    cu = np.concatenate([[0], np.cumsum(nq)]).astype(np.int32)
+    bt = np.zeros((B, max(len(t) for t in tables)), np.int32)
+    for b, t in enumerate(tables):
+        bt[b, :len(t)] = t
+    d_cu, d_ctx, d_bt, d_out, d_q, d_k, d_v = dev(cu), dev(np.asarray(ctx, np.int32)), dev(bt), nvr.DeviceBuffer(T * H * D * 2), dev(q), dev(k), dev(v)
+    meta = nvr.AttnMetaC()
+    meta.is_prefill, meta.cu_seqlens_q, meta.context_lens, meta.block_tables = 1, d_cu.ptr, d_ctx.ptr, d_bt.ptr
+    meta.max_blocks, meta.batch, meta.max_context_len = bt.shape[1], B, int(max(ctx))
+    nvr.check(nvr.lib().nvr_attn_prefill_paged(d_q.ptr, H * D, d_k.ptr, d_v.ptr, C.byref(meta), T, H, KVH, D, bs, float(D ** -0.5), d_out.ptr, None))
+    return d_out.to_numpy((T, H, D), F16)
+
+
+@pytest.mark.parametrize("G,KVH,bs,ctx,growth", [
+    (2, 2, 64, [1, 63, 64, 65, 129], 0.0), (1, 3, 128, [127, 128, 200], 0.0), (4, 1, 64, [33, 97, 320], 0.0),
+    (2, 1, 64, [700], 9.0), (1, 2, 48, [391, 70], 9.0), (4, 2, 256, [513], -9.0),      # scores that outgrow the running maximum again and again, and that fall off; a block size without a power of two
+    (2, 1, 64, [4400], 3.0),                                                          # more blocks than the register copy of a table holds
+])
+def test_prompt_attention_of_heads_of_128(G, KVH, bs, ctx, growth):
+    """The plain prompt attention against 64 bits at the edges of its tiles and steps, and the bits of a prompt in portions against the prompt whole."""
+    rng, D, H = np.random.default_rng(sum(ctx)), 128, G * KVH
+    NB = sum(-(-c // bs) for c in ctx)
+    order, tables, at = rng.permutation(NB), [], 0
+    k, v = np.zeros((NB * bs, KVH, D), F16), _bits(rng, (NB * bs, KVH, D), 1.0)
+    q, want = [], []
+    for c in ctx:
+        t = order[at:at + -(-c // bs)]
+        at += len(t)
+        rows = (t[:, None] * bs + np.arange(bs)[None]).reshape(-1)[:c]
+        ramp = np.linspace(0.1, abs(growth), c)[::1 if growth > 0 else -1] if growth else np.ones(c)
+        qs = _bits(rng, (c, H, D), 1.0)
+        if growth:                                                                    # keys near one direction that every query has: the score follows the ramp
+            axis = np.ones(D) / np.sqrt(D)
+            k[rows] = (rng.standard_normal((c, KVH, D)) * 0.3 + axis * ramp[:, None, None] * 4).astype(F16)
+            qs = (qs.astype(np.float64) + axis * 4).astype(F16)
+        else:
+            k[rows] = _bits(rng, (c, KVH, D), 1.0)
+        tables.append(t.astype(np.int32))
+        q.append(qs)
+        kk, vv, qq = (np.repeat(a[rows].astype(np.float64), G, 1) if a is not None else qs.astype(np.float64) for a in (k, v, None))
+        s = np.einsum("ihd,jhd->hij", qq, kk) * D ** -0.5
+        s[:, np.arange(c)[None, :] > np.arange(c)[:, None]] = -np.inf
+        p = np.exp(s - s.max(2, keepdims=True))
+        want.append(np.einsum("hij,jhd->ihd", p / p.sum(2, keepdims=True), vv))
+    whole = _prefill(np.concatenate(q), ctx, ctx, k, v, tables, H, KVH, D, bs)
+    # a weight is rounded to 11 bits before it meets its value, and so is the result: 2^-11 of the sum of |weight x value| (at most the largest |value|, about 4.5) each, and the sums' 24 bits
+    assert np.max(np.abs(whole - np.concatenate(want))) <= 2 * 4.5 * 2.0 ** -11
+    at = 0
+    for i, c in enumerate(ctx):
+        for n in {1, min(c, 17), min(c, 70), c}:                                      # its last n tokens alone
+            part = _prefill(q[i][c - n:], [c], [n], k, v, [tables[i]], H, KVH, D, bs)
+            assert np.array_equal(part.view(np.uint16), whole[at + c - n:at + c].view(np.uint16)), (c, n)
+        at += c
