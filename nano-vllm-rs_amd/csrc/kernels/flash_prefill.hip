@@ -514,12 +514,12 @@ __global__ __launch_bounds__(64 * FLASH_WAVES, 8 / FLASH_WAVES) void flash_prefi
 // What bounds it: the matrix cores and the exponentials (1024 + 512 cycles of a wave and step) as far as they run side by side.  A product of 16 x 16 x 32 holds its wave's issue for as long as
 // it takes; one of 32 x 32 x 16 leaves half of its 32 cycles to the wave's vector instructions, so a step is laid out as two blocks of 16 products with vector work of their own between them:
 //   block 1: Sᵀ of step i + 1 | the exponentials of step i's first 32 keys       block 2: Oᵀ of step i | the exponentials of its second 32 keys, the maxima of step i + 1
-// (K runs one step ahead of V through the LDS ring).  The running maximum of a query is raised only when a step exceeds it by 2^8 in the exponentials' unit: the rescaling of the
-// accumulators, 64 multiplications a step while maxima still move, then happens once or twice a tile; a query's decision does not depend on its wave's other queries, so its bits do not either.
-// bfloat16, G = 2, us before (16 x 16 x 32 products, a maximum per step) / now: 32 prompts of 1024 tokens 204 / 177 a layer, one of 509 15.8 / 12.9, of 2048 47.5 / 40.9, of 8192 330 / 301; 3814
-// tokens behind 11440 cached ones 191 / 172; 100 steps of one workgroup per CU 138 / 123, of two 214 / 201 (1.07 PFLOP/s: cycles fall by 23 %, the clock from 2.1 to 1.75 GHz).  Without the K reads
-// 171, without the V reads 188, without the exponentials 185, without the LDS-DMA 183, products and the rest of the vector work alone 127.
-constexpr float FLASH_SLACK = 8.0f;                             // log2 of what an exponential may exceed 1 by
+// (K runs one step ahead of V through the LDS ring).  The accumulators are rescaled at a step's start, behind the barrier, where the products on them have long ended, and only if a query of the
+// wave met a larger score.  Raising the maximum only past a margin (2^8 in the exponentials' unit) takes another 7 % off, but the largest weight is then no longer the 1 that has no rounding:
+// the attention's error against 64 bits grew by 2.5 %.
+// bfloat16, G = 2, us before (16 x 16 x 32 products, one after the other) / now: 32 prompts of 1024 tokens 201 / 184 a layer, one of 509 16.2 / 15.1, of 2048 49.0 / 45.5, of 8192 334 / 325; 100
+// steps of one workgroup per CU 143 / 134, of two 212 / 212: cycles fall, and with the matrix cores' load the clock, from 2.1 to 1.75 GHz.  Of 202 us of two per CU without rescaling: without the K
+// reads 171, the V reads 188, the exponentials 185, the LDS-DMA 183, products and the rest of the vector work alone 127.
 // N products, each followed by READS LDS reads (those of the product AHEAD products later) and VALU vector instructions
 template <int N, int READS, int AHEAD, int VALU>
 __device__ __forceinline__ void sched_pattern() {
@@ -635,7 +635,7 @@ __global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
     float16_t o[4], s0, s1;                                               // s0, s1: scores of a step's first and second 32 keys
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) o[dt] = (float16_t)(0.f);
-    const float cs = p.scale * 1.44269504088896340736f, slack = FLASH_SLACK / cs;      // the softmax runs on raw scores: p = 2^((s - m) cs)
+    const float cs = p.scale * 1.44269504088896340736f;      // the softmax runs on raw scores: p = 2^((s - m) cs)
     float m = -INFINITY, l = 0.f;
     if (p.sink) { m = p.sink[head] / p.scale; l = h == 0 ? 1.f : 0.f; }   // (l: this half wave's keys)
     half2_t one2;
@@ -658,14 +658,15 @@ __global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
         for (int e = 2; e < 16; e += 2) { a = fmaxf(fmaxf(a, c[e]), c[e + 1]); b = fmaxf(fmaxf(b, d[e]), d[e + 1]); }
         return xor32_partner_max(fmaxf(a, b));
     };
+    // the running maximum takes in a step's; alpha: what the accumulators are multiplied by (1 for a query whose maximum stays)
     auto raise = [&](float mx) {
-        const bool up = mx > m + slack;                                   // (finite from the first step on: key 0 <= qpos)
-        if (__any(up)) {
-            const float mn = up ? mx : m, alpha = __builtin_amdgcn_exp2f((m - mn) * cs);
-            m = mn; l *= alpha;
+        const float mn = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f((m - mn) * cs);      // (finite from the first step on: key 0 <= qpos)
+        m = mn; l *= alpha;
+        return alpha;
+    };
+    auto rescale = [&](float alpha) {
 #pragma unroll
-            for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
-        }
+        for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
     };
     // exponentials of 16 keys of a step, and their sum as the products see them
     auto exponentials = [&](const float16_t &d, int k, float mc) {        // keys 16 k .. of the 32
@@ -698,7 +699,7 @@ __global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
     addresses();
     scores(s0, s1);
     if (KT - 1 > tile.pos0) { mask(0, s0); mask(32, s1); }
-    raise(maximum(s0, s1));
+    float mx = maximum(s0, s1);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();                                         // (K of step 2 takes the place of K of step 0)
     int it = 0;
@@ -706,9 +707,10 @@ __global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
         request(it);
         ka ^= IMG;
         addresses();
-        const float mc = -m * cs;
         half8_t pf[4];
         float16_t n0, n1;
+        if (__any(mx > m)) rescale(raise(mx));
+        const float mc = -m * cs;
         __builtin_amdgcn_sched_barrier(0);
         scores(n0, n1);
         pf[0] = exponentials(s0, 0, mc); pf[1] = exponentials(s0, 1, mc);
@@ -722,17 +724,17 @@ __global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
         values(2, pf[2]); values(3, pf[3]);
 #pragma unroll
         for (int k = 0; k < 4; ++k) add_up(pf[k]);
-        const float mx = maximum(n0, n1);
+        mx = maximum(n0, n1);
         s0 = n0; s1 = n1;
         sched_pattern<16, 2, 2, 5>();
         __builtin_amdgcn_sched_barrier(0);
-        raise(mx);
         va ^= IMG;
         close();
     }
     {                                                                     // the wave's last step
         request(it);
         addresses();
+        if (__any(mx > m)) rescale(raise(mx));
         const float mc = -m * cs;
         half8_t pf[4];
 #pragma unroll

@@ -1092,8 +1092,8 @@ int nvr_model_runner::execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill
                     }
                 }
                 // A step whose workgroups are all resident at once, one or two per CU (two are worth 1.6 of one): the CUs take one each, longest first, and then the rest in turn — shortest
-                // first, so that the longest of the first share a CU with the shortest of the rest.  us a layer, longest first all through / so: one prompt of 3000 tokens 62.0 / 58.7, of 4096
-                // 91.3 / 84.8, 3814 behind 11440 cached 176.8 / 168.7; beyond two per CU (4600 107.0 / 105.5, 5500 136.9 / 133.9) freed slots level the rest.
+                // first, so that the longest of the first share a CU with the shortest of the rest.  us a layer, longest first all through / so: one prompt of 3000 tokens 66.2 / 64.3, of 4096
+                // 96.5 / 92.6, 3814 behind 11440 cached 185.1 / 179.7; beyond two per CU freed slots level the rest (4600 112.7 / 111.6, 5500 143.8 / 152.3).
                 const int64_t round = std::max<int64_t>(1, num_cus / KVH);
                 if (tp == 1 && n_tiles > round && n_tiles <= 2 * round) {
                     std::stable_sort(tl, tl + n_tiles, [](const k::FlashTile &a, const k::FlashTile &b) { return a.pos0 + a.nq > b.pos0 + b.nq; });
