@@ -28,7 +28,7 @@
 
 namespace nvr { namespace NVR_DT_NS {
 
-enum { TEPI_F16 = 0, TEPI_SILU = 2, TEPI_ROPE = 3, TEPI_LMHEAD = 4, TEPI_SLAB = 5 };
+enum { TEPI_F16 = 0, TEPI_SILU = 2, TEPI_ROPE = 3, TEPI_LMHEAD = 4, TEPI_SLAB = 5, TEPI_RESID = 6 };     // RESID: y <- y + x.W^T, the product rounded first
 
 // Where a launch's tiles lie: nx column tiles (W rows) x ny token tiles x nz k-slices, numbered slice by slice, within a slice in strips of `width` column tiles, within a strip
 // token tile by token tile.  Workgroups are dealt to the 8 XCDs in turn and each XCD has an L2 of its own, so XCD c takes the c-th eighth of that line: a compact block of tiles,
@@ -331,17 +331,29 @@ __global__ __launch_bounds__(256, 2) void gemm_tiled_kernel(const half_t *__rest
         return o.h;
     };
     const int col_in_pair = (q & 1) * 16 + (q >> 1) * 8;                  // first column a lane holds of a pair of n-tiles whose 32 columns are consecutive
+    half8_t resid[MT][2];                                                 // TEPI_RESID: what the products are added to, all of it requested at once
+    if (EPI == TEPI_RESID) {
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                resid[j][i] = *reinterpret_cast<const half8_t *>(y + (int64_t)min(m0 + wm * (16 * MT) + j * 16 + r, T - 1) * N + min(at.x * BN + wn * 64 + i * 32 + col_in_pair, N - 8));
+    }
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
         const int m = m0 + wm * (16 * MT) + j * 16 + r;
-        if (EPI == TEPI_F16) {
+        if (EPI == TEPI_F16 || EPI == TEPI_RESID) {
 #pragma unroll
             for (int i = 0; i < 4; i += 2) {
                 half4_t h[2];
 #pragma unroll
                 for (int u = 0; u < 2; ++u) h[u] = (half4_t){(half_t)acc[i + u][j][0], (half_t)acc[i + u][j][1], (half_t)acc[i + u][j][2], (half_t)acc[i + u][j][3]};
-                const half8_t v8 = pair8(h[0], h[1]);
+                half8_t v8 = pair8(h[0], h[1]);
                 const int n = at.x * BN + wn * 64 + i * 16 + col_in_pair;
+                if (EPI == TEPI_RESID) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v8[e] = to_half_rn((float)resid[j][i >> 1][e] + (float)v8[e]);
+                }
                 if (m < T && n < N) *reinterpret_cast<half8_t *>(y + (int64_t)m * N + n) = v8;
             }
         } else if (EPI == TEPI_SILU) {
@@ -577,7 +589,7 @@ int gemm_tiled_prepare() {
     { hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tiled_kernel<EPI_, NS_, MT_>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(NS_ * BYTES_)); \
       if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "gemm_tiled: LDS opt-in failed: %s", hipGetErrorString(e)); }
 #define NVR_TILED_ATTR(EPI_) NVR_TILED_ATTR1(EPI_, 3, 4, kStageBytes) NVR_TILED_ATTR1(EPI_, 4, 2, kStageBytes64) NVR_TILED_ATTR1(EPI_, 3, 2, kStageBytes64) NVR_TILED_ATTR1(EPI_, 4, 1, kStageBytes32)
-    NVR_TILED_ATTR(TEPI_F16) NVR_TILED_ATTR(TEPI_SILU) NVR_TILED_ATTR(TEPI_ROPE) NVR_TILED_ATTR(TEPI_LMHEAD) NVR_TILED_ATTR(TEPI_SLAB)
+    NVR_TILED_ATTR(TEPI_F16) NVR_TILED_ATTR(TEPI_SILU) NVR_TILED_ATTR(TEPI_ROPE) NVR_TILED_ATTR(TEPI_LMHEAD) NVR_TILED_ATTR(TEPI_SLAB) NVR_TILED_ATTR(TEPI_RESID)
 #undef NVR_TILED_ATTR
 #undef NVR_TILED_ATTR1
     if (hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tiled_silu96_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, RING96 * S96_BUF) != hipSuccess)
@@ -623,6 +635,12 @@ int gemm_tiled(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, i
     if (int rc = gemm_tiled_prepare()) return rc;
     tiled_launch<TEPI_F16>((N + BN - 1) / BN, 1, x, ldx, W, Wt, T, K, N, N, (half_t *)y, TileEpi{}, s);
     return tiled_check("gemm_tiled");
+}
+int gemm_tiled_resid(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *h, hipStream_t s, const half_bits *Wt) {
+    if (!gemm_tiled_ok(T, K, N, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_resid: T=%ld K=%ld N=%ld", (long)T, (long)K, (long)N);
+    if (int rc = gemm_tiled_prepare()) return rc;
+    tiled_launch<TEPI_RESID>((N + BN - 1) / BN, 1, x, ldx, W, Wt, T, K, N, N, (half_t *)h, TileEpi{}, s);
+    return tiled_check("gemm_tiled_resid");
 }
 int gemm_tiled_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s, bool gelu, const half_bits *Wt) {
     if (!gemm_tiled_ok(T, K, I, ldx) || I % 64) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_silu_mul: T=%ld K=%ld I=%ld", (long)T, (long)K, (long)I);

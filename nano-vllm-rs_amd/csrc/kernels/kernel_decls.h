@@ -117,6 +117,7 @@ int gemm_tiled_lm_head(const half_bits *x, int64_t ldx, const half_bits *W, int6
 // LDS-tiled MFMA GEMM for the prefill regime (T >= 128): same results layout and epilogues as the kernels above
 bool gemm_tiled_ok(int64_t T, int64_t K, int64_t N, int64_t ldx);
 int gemm_tiled(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *y, hipStream_t s, const half_bits *Wt = nullptr);
+int gemm_tiled_resid(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *h, hipStream_t s, const half_bits *Wt = nullptr);   // h <- h + x.W^T, the product rounded first
 int gemm_tiled_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out,
                         hipStream_t s, bool gelu = false, const half_bits *Wt = nullptr);
 int gemm_tiled_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH,
@@ -138,7 +139,11 @@ int gemm256_resid(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T
 bool gemm256_lm_head_ok(int64_t T, int64_t K, int64_t N, int64_t ldx);
 int gemm256_lm_head(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, float *logits, float *part_val,
                     int32_t *part_idx, int32_t *nparts, hipStream_t s);
-bool gemm256_preferred(int64_t T, int64_t K, int64_t N, int64_t ldx);     // linear() would take the 256x256 kernel for this shape
+bool gemm256_preferred(int64_t T, int64_t K, int64_t N, int64_t ldx);     // the 256x256 kernel is the faster one of the two for the whole shape
+bool linear_add_residual_ok(int64_t T, int64_t K, int64_t N, int64_t ldx);   // the shapes nvr_linear_add_residual takes
+// h <- h + x.W^T (the product rounded first) of a prompt-sized step on the tiles that the shape takes
+bool linear_resid_ok(int64_t T, int64_t K, int64_t N, int64_t ldx);
+int linear_resid(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *h, hipStream_t s, const half_bits *Wt = nullptr);
 int gemm256_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s);
 int gemm256_gelu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s);
 int gemm256_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D,

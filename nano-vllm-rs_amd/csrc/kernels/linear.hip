@@ -22,6 +22,7 @@
 // Rounding points mirror the oracle (oracle/model_oracle.py): the f32 accumulator is rounded to fp16
 // where the unfused graph stores an fp16 tensor (qkv, gate_up), then the epilogue math runs in f32
 // without FMA contraction and is rounded again.
+#include <algorithm>
 #include <cstdlib>
 #include "kernels.h"
 #include "device_utils.h"
@@ -323,20 +324,46 @@ static void launch(const half_t *x, int64_t ldx, const half_t *W, int T, int K, 
 // 256x256 kernel takes 18.5 K/1024 + 8 us however few there are (K = 1024 25 us, 2048 39, 4096 81, 12288 235).  The 128x128 kernel takes 9.4 K/1024 + 3.5 us while its tiles fit one per CU
 // (13.3 / 22 / 42 / 118), beyond that 8 K/1024 + 1.2 per 256 tiles, a last part of a round counted half (768 tiles 31, 1152 45, 2048 73 at K = 1024).  us of both, 256 / 128: qkv of 0.6B 27.1 /
 // 20.4 at 2048 tokens, 27.4 / 29.4 at 2560, 49.8 / 45.6 at 4672; o_proj 44.8 / 34.4 at 8192; 8B qkv 84.6 / 64.7 at 1280, 82.9 / 100.1 at 1536, 166 / 153 at 3062.  N = W rows
-static inline bool prefer_256(int64_t T, int64_t K, int64_t N) {
-    const int64_t t256 = ((N + 255) / 256) * ((T + 255) / 256), t128 = ((N + 127) / 128) * ((T + 127) / 128);
-    const double kk = (double)K / 1024.0, rounds = (double)t128 / 256.0;
-    const double c256 = (double)((t256 + 255) / 256) * (18.5 * kk + 8.0);
-    const double c128 = t128 <= 256 ? 9.4 * kk + 3.5 : 0.5 * (rounds + (double)((t128 + 255) / 256)) * (8.0 * kk + 1.2) + 2.0;
-    return c256 < c128;
+static double cost_256(int64_t T, int64_t K, int64_t N) {
+    const int64_t tiles = ((N + 255) / 256) * ((T + 255) / 256);
+    return (double)((tiles + 255) / 256) * (18.5 * (double)K / 1024.0 + 8.0);
 }
-// one rule for the plain and the fused launchers (N = output features), so that a fused GEMM and its unfused twin run the same kernel
+static double cost_128(int64_t T, int64_t K, int64_t N) {
+    const int64_t tiles = ((N + 127) / 128) * ((T + 127) / 128);
+    const double kk = (double)K / 1024.0, rounds = (double)tiles / 256.0;
+    return tiles <= 256 ? 9.4 * kk + 3.5 : 0.5 * (rounds + (double)((tiles + 255) / 256)) * (8.0 * kk + 1.2) + 2.0;
+}
+static inline bool prefer_256(int64_t T, int64_t K, int64_t N) { return cost_256(T, K, N) < cost_128(T, K, N); }
 bool gemm256_preferred(int64_t T, int64_t K, int64_t N, int64_t ldx) { return gemm256_ok(T, K, N, ldx) && prefer_256(T, K, N); }
+// Rows [0, r) of a product on 256x256 tiles and the others on 128x128 ones (0: all on the latter, T: all on the former).  A last round of 256x256 tiles costs as much as a full one however few
+// they are, so the rows that do not fill one go to the small tiles where that is estimated 4 % cheaper: both kernels sum a row's products in the same order, and a row has the same bits on either.
+// us, the better kernel for all rows / split: 8B qkv 154.9 / 130.3 at 3062 rows, o_proj 154.1 / 134.4 at 4672, down_proj 453.7 / 377.2 at 4672, 484.6 / 393.1 at 5120; 0.6B gate_up 45.9 / 42.2 at
+// 3062, qkv 43.1 / 38.8 at 4300, 44.7 / 43.5 at 4672, o_proj 76.5 / 64.8 at 17000.
+static int64_t rows_on_256(int64_t T, int64_t K, int64_t N) {
+    const double c256 = cost_256(T, K, N), c128 = cost_128(T, K, N);
+    int64_t best = c256 < c128 ? T : 0;
+    double least = 0.96 * std::min(c256, c128);
+    const int64_t tn = (N + 255) / 256;
+    for (int64_t rounds = 1; rounds * 256 / tn * 256 <= T - 65; ++rounds) {
+        const int64_t r = rounds * 256 / tn * 256;
+        const double c = r > 0 ? cost_256(r, K, N) + cost_128(T - r, K, N) : 1e30;
+        if (c < least) { least = c; best = r; }
+    }
+    return best;
+}
+// the shapes for which the 256x256 kernel was estimated the faster one when nvr_linear_add_residual was added: what it takes does not move with the tiles' speed
+bool linear_add_residual_ok(int64_t T, int64_t K, int64_t N, int64_t ldx) {
+    const int64_t t256 = ((N + 255) / 256) * ((T + 255) / 256), t128 = ((N + 127) / 128) * ((T + 127) / 128);
+    const double kk = (double)K / 1024.0, c128 = (t128 <= 256 ? 15.0 * kk : (double)((t128 + 511) / 512) * 21.0 * kk) + 5.0;
+    return gemm256_ok(T, K, N, ldx) && (double)((t256 + 255) / 256) * (17.0 * kk + 20.0) < c128;
+}
 int64_t stream_row_limit() { return 64; }
 // split-k GEMMs of the N = hidden projections: LDS tiles beyond the streaming kernels' rows — and from 33 rows on over large weights, where the
 // streaming split-k kernel walks the weights once per 32-row block (Qwen3-8B bs 64: o + down 92 us per layer against 46 us at bs 128 on the tiles;
 // up to 32 rows the streaming kernel stays ahead: Qwen3-8B bs 32 / 16 5.00 / 4.20 ms per step against 5.10 / 4.38 on 32-token tiles, 8 slices)
 bool splitk_prefers_tiles(int64_t T, int64_t K, int64_t N) { return T > stream_row_limit() || (T > 32 && N * K * 2 >= (24ll << 20)); }
+// ... and with 8 slices whatever the weights: 64 rows, N = 1024, K = 2048 / 3072 5.0 / 6.3 us as two blocks and 2 slices, 4.3 / 5.0 on the tiles
+constexpr int64_t TILE_SLICES = 8;
 // k-slices of the N = hidden GEMMs of a decode-sized step (linear_splitk): reach ~256 workgroups with slices of >= 256 columns that are
 // multiples of 64
 int decode_splitk_slices(int64_t T, int64_t K, int64_t N) {
@@ -348,7 +375,7 @@ int decode_splitk_slices(int64_t T, int64_t K, int64_t N) {
 static inline bool prefer_stream(int64_t T, int64_t N) {
     // up to 64 rows the weight-streaming kernel; beyond, the LDS-tiled kernel with 32- / 64-token tiles and the 4-buffer ring (r02,
     // ctx 256: bs 66 2.20 -> 1.83 ms/step, bs 96 2.48 -> 2.15, bs 128 2.82 -> 2.23).
-    return T <= stream_row_limit() || T * N <= 384 * 1024;
+    return T <= stream_row_limit() || T * N <= 256 * 1024;       // (qkv of 0.6B, 80 rows 9.1 / 7.9, 96 rows 10.0 / 7.9)
 }
 static inline int waves_for(int64_t K) { return K >= 2048 ? 16 : (K >= 1024 ? 8 : 4); }
 
@@ -365,9 +392,14 @@ static int linear_routed(const half_bits *x, int64_t ldx, const half_bits *W, in
         return nvr::fail(NVR_ERR_UNSUPPORTED, "linear: K=%ld must be a multiple of 32, N=%ld of 16, ldx=%ld of 8",
                          (long)K, (long)N, (long)ldx);
     if (T == 0) return 0;
-    // Routing by measured crossovers (scratch/gemm_route_sweep.py, profiles/r01_gemm_ablation.txt): prefer_256 above; the 128x128 kernel's
-    // own single-tile latency (21-31 us) loses to the weight-streaming kernel run over 32-token blocks while T or T*N is small
-    if (!y_f32 && gemm256_ok(T, K, N, ldx) && prefer_256(T, K, N)) return act ? gemm256_gelu(x, ldx, W, T, K, N, (half_bits *)y, s) : gemm256(x, ldx, W, T, K, N, (half_bits *)y, s);   // prefill regime
+    // prompts: rows_on_256; up to 64 rows and for small T * N the weight-streaming kernel over blocks of 32 rows
+    if (!y_f32 && gemm256_ok(T, K, N, ldx)) {
+        if (act) { if (prefer_256(T, K, N)) return gemm256_gelu(x, ldx, W, T, K, N, (half_bits *)y, s); }
+        else if (const int64_t r = rows_on_256(T, K, N)) {
+            if (int rc = gemm256(x, ldx, W, r, K, N, (half_bits *)y, s)) return rc;
+            return r == T ? 0 : gemm_tiled(x + r * ldx, ldx, W, T - r, K, N, (half_bits *)y + r * N, s, Wt);
+        }
+    }
     if (gelu) *gelu = false;                               // (the tiled and the streaming kernel have no such epilogue)
     if (!y_f32 && gemm_tiled_ok(T, K, N, ldx) && !prefer_stream(T, N)) return gemm_tiled(x, ldx, W, T, K, N, (half_bits *)y, s, Wt);
     if (!y_f32 && linear_stream_ok(T, K, N, ldx)) return linear_stream(x, ldx, W, T, K, N, (half_bits *)y, s, Wt);   // large weights
@@ -416,6 +448,14 @@ int linear_gelu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, 
     return linear_routed(x, ldx, W, T, K, N, y, false, s, nullptr, applied);
 }
 
+bool linear_resid_ok(int64_t T, int64_t K, int64_t N, int64_t ldx) { return gemm_tiled_ok(T, K, N, ldx) && !prefer_stream(T, N) && N % 8 == 0; }
+int linear_resid(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *h, hipStream_t s, const half_bits *Wt) {
+    if (!linear_resid_ok(T, K, N, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "linear_resid: T=%ld K=%ld N=%ld", (long)T, (long)K, (long)N);
+    const int64_t r = gemm256_ok(T, K, N, ldx) ? rows_on_256(T, K, N) : 0;
+    if (r > 0) if (int rc = gemm256_resid(x, ldx, W, r, K, N, h, s)) return rc;
+    return r == T ? 0 : gemm_tiled_resid(x + r * ldx, ldx, W, T - r, K, N, h + r * N, s, Wt);
+}
+
 // split-k over S workgroups per tile: slabs[z][T][N] f32 partial sums (summed by add_rmsnorm_slabs); the narrow
 // row-parallel GEMMs of the decode step (o_proj, down_proj: N = hidden) reach all 256 CUs this way
 int linear_splitk(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, int64_t S,
@@ -423,7 +463,7 @@ int linear_splitk(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T
     if (K % (32 * S) || N % 16 || ldx % 8 || S < 1)
         return nvr::fail(NVR_ERR_UNSUPPORTED, "linear_splitk: K=%ld must be a multiple of 32*S (S=%ld), N=%ld of 16", (long)K, (long)S, (long)N);
     if (T == 0) return 0;
-    if (splitk_prefers_tiles(T, K, N) && gemm_tiled_splitk_ok(T, K, N, S, ldx)) return gemm_tiled_splitk(x, ldx, W, T, K, N, S, slabs, s, Wt);   // LDS tiles
+    if ((splitk_prefers_tiles(T, K, N) || (T > 32 && S >= TILE_SLICES)) && gemm_tiled_splitk_ok(T, K, N, S, ldx)) return gemm_tiled_splitk(x, ldx, W, T, K, N, S, slabs, s, Wt);   // LDS tiles
     LinEpi e{};
     e.kslice = (int32_t)(K / S); e.slab_stride = T * N;
     if (Wt) { W = Wt; e.tiled = 1; }
@@ -447,8 +487,12 @@ static int linear_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64
     if (K % 32 || I % 16 || ldx % 8)
         return nvr::fail(NVR_ERR_UNSUPPORTED, "linear_silu_mul: K=%ld must be a multiple of 32, I=%ld of 16", (long)K, (long)I);
     if (T == 0) return 0;
-    if (gemm256_silu_ok(T, K, I, ldx) && prefer_256(T, K, 2 * I)) return gelu ? gemm256_gelu_mul(x, ldx, W, T, K, I, out, s) : gemm256_silu_mul(x, ldx, W, T, K, I, out, s);   // see linear()
-    if (gemm_tiled_ok(T, K, I, ldx) && I % 64 == 0 && !prefer_stream(T, 2 * I)) return gemm_tiled_silu_mul(x, ldx, W, T, K, I, out, s, gelu, Wt);
+    if (const int64_t r = gemm256_silu_ok(T, K, I, ldx) ? rows_on_256(T, K, 2 * I) : 0) {
+        if (int rc = gelu ? gemm256_gelu_mul(x, ldx, W, r, K, I, out, s) : gemm256_silu_mul(x, ldx, W, r, K, I, out, s)) return rc;
+        return r == T ? 0 : gemm_tiled_silu_mul(x + r * ldx, ldx, W, T - r, K, I, out + r * I, s, gelu, Wt);
+    }
+    // (56 rows and more of weights that the large-weight kernel does not take: the two blocks of 32 rows each read x for every 16 columns; 64 rows, K = 1024, I = 3072 9.1 / 8.2, 48 rows 8.2 / 8.2)
+    if (gemm_tiled_ok(T, K, I, ldx) && I % 64 == 0 && (!prefer_stream(T, 2 * I) || (T >= 56 && T * I > 128 * 1024 && !linear_stream_silu_ok(T, K, I, ldx)))) return gemm_tiled_silu_mul(x, ldx, W, T, K, I, out, s, gelu, Wt);
     if (linear_stream_silu_ok(T, K, I, ldx)) return linear_stream_silu_mul(x, ldx, W, T, K, I, out, s, Wt, gelu);              // large weights
     const half_t *xx = (const half_t *)x, *ww = (const half_t *)(Wt ? Wt : W);
     LinEpi e{};
@@ -509,8 +553,10 @@ int linear_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, i
     if (K % 32 || D % 16 || ldx % 8)
         return nvr::fail(NVR_ERR_UNSUPPORTED, "linear_qkv_rope_store: K=%ld must be a multiple of 32, D=%ld of 16", (long)K, (long)D);
     if (T == 0) return 0;
-    if (gemm256_rope_ok(T, K, H, KVH, D, ldx) && prefer_256(T, K, (H + 2 * KVH) * D))                                  // see linear()
-        return gemm256_qkv_rope_store(x, ldx, W, T, K, H, KVH, D, positions, slots, cos_t, sin_t, qkv, k_cache, v_cache, s, kv_cache_only);
+    if (const int64_t r = gemm256_rope_ok(T, K, H, KVH, D, ldx) ? rows_on_256(T, K, (H + 2 * KVH) * D) : 0) {
+        if (int rc = gemm256_qkv_rope_store(x, ldx, W, r, K, H, KVH, D, positions, slots, cos_t, sin_t, qkv, k_cache, v_cache, s, kv_cache_only)) return rc;
+        return r == T ? 0 : gemm_tiled_qkv_rope_store(x + r * ldx, ldx, W, T - r, K, H, KVH, D, positions + r, slots ? slots + r : nullptr, cos_t, sin_t, qkv + r * (H + 2 * KVH) * D, k_cache, v_cache, s, Wt, kv_cache_only);
+    }
     if (gemm_tiled_ok(T, K, (H + 2 * KVH) * D, ldx) && 128 % D == 0 && !prefer_stream(T, (H + 2 * KVH) * D))
         return gemm_tiled_qkv_rope_store(x, ldx, W, T, K, H, KVH, D, positions, slots, cos_t, sin_t, qkv, k_cache, v_cache, s, Wt, kv_cache_only);
     if (linear_stream_rope_ok(T, K, H, KVH, D, ldx))                                                                  // large weights

@@ -610,7 +610,7 @@ int nvr_model_runner::row_parallel_norm(const uint16_t *x, int64_t K, const uint
     }
     int64_t S = 1;
     if (!comm.active() && tp == 1 && T <= 64 && T <= KD(stream_row_limit()) && Hd <= 2048) {
-        S = KD(decode_splitk_slices(T, K, Hd));
+        S = T > 32 && 8 * T <= 4 * slab_rows && KD(gemm_tiled_splitk_ok(T, K, Hd, 8, K)) ? 8 : KD(decode_splitk_slices(T, K, Hd));
     } else if (!comm.active() && tp == 1 && T > 32 && T <= 64 && Hd <= 8192 && KD(splitk_prefers_tiles(T, K, Hd)) && 8 * T <= 4 * slab_rows &&
                KD(gemm_tiled_splitk_ok(T, K, Hd, 4, K))) {
         // 33..64 rows over large weights (Qwen3-8B bs 64): one 64-token tile per 128 weight rows, k split until ~256 workgroups stream the
@@ -628,10 +628,10 @@ int nvr_model_runner::row_parallel_norm(const uint16_t *x, int64_t K, const uint
         RC(KD(linear_splitk(x, K, W, T, K, Hd, S, slabs, stream, Wt)));
         return KD(add_rmsnorm_slabs(h, slabs, S, wn, mc.rms_norm_eps, T, Hd, n, stream));
     }
-    if (!comm.active() && tp == 1 && KD(gemm256_preferred(T, K, Hd, K))) {
-        // prefill-sized steps on one rank: the residual add rides in the 256x256 GEMM's epilogue (h <- fp16(h + fp16(x W^T)), the same
+    if (!comm.active() && tp == 1 && KD(linear_resid_ok(T, K, Hd, K))) {
+        // prefill-sized steps on one rank: the residual add rides in the product's epilogue (h <- fp16(h + fp16(x W^T)), the same
         // rounding points), and the norm reads one tensor instead of h and the projection (r02: 41.6 -> ~21 us per norm at 32 x 1024)
-        RC(KD(gemm256_resid(x, K, W, T, K, Hd, h, stream)));
+        RC(KD(linear_resid(x, K, W, T, K, Hd, h, stream, Wt)));
         return KD(rmsnorm(h, wn, mc.rms_norm_eps, T, Hd, n, stream));
     }
     // (the step's GEMM kernel by linear.hip's routing: 256-row tiles when its cost rule prefers them, else the 128-row kernel; the chunks call THAT kernel)

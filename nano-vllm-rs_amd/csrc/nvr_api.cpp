@@ -620,7 +620,7 @@ int nvr_retile_weight(const nvr_half *src, nvr_half *dst, int64_t N, int64_t K, 
 }
 int nvr_linear_add_residual(const nvr_half *x, int64_t ldx, const nvr_half *W, int64_t T, int64_t K, int64_t N, nvr_half *h, void *s) {
     NO_F32("nvr_linear_add_residual");
-    if (!k::gemm256_preferred(T, K, N, ldx))
+    if (!k::linear_add_residual_ok(T, K, N, ldx))
         return nvr::fail(NVR_ERR_UNSUPPORTED, "nvr_linear_add_residual: T=%ld K=%ld N=%ld is not a shape of the 256x256 prefill GEMM", (long)T, (long)K, (long)N);
     return KO(gemm256_resid(x, ldx, W, T, K, N, h, (hipStream_t)s));
 }

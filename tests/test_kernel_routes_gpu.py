@@ -553,3 +553,51 @@ def test_prompt_attention_of_heads_of_128(G, KVH, bs, ctx, growth):
             part = _prefill(q[i][c - n:], [c], [n], k, v, [tables[i]], H, KVH, D, bs)
             assert np.array_equal(part.view(np.uint16), whole[at + c - n:at + c].view(np.uint16)), (c, n)
         at += c
+
+
+@pytest.mark.parametrize("kind,T,K,N", [("plain", 4200, 1024, 4096), ("silu", 3062, 1024, 3072), ("rope", 4300, 1024, 4096)])
+def test_products_whose_rows_are_split_over_two_kernels(kind, T, K, N):
+    """Prompt products whose last rows go to smaller tiles: the rows around the line have the bits of the same rows in a call of their own."""
+    rng, l = np.random.default_rng(T), nvr.lib()
+    rows, H, KVH, D = (2 * N if kind == "silu" else N), 16, 8, 128
+    x, W = _bits(rng, (T, K), 0.5), _bits(rng, (rows, K), 0.1)
+    d_W, pos = dev(W), rng.integers(0, 512, T).astype(np.int64)
+    slots = np.arange(T, dtype=np.int32)
+    cos, sin = oracle.rope_table(D, 512, 1e6)
+    d_cos, d_sin = dev(cos), dev(sin)
+
+    def run(a, b):
+        n, d_x, y = b - a, dev(x[a:b]), nvr.DeviceBuffer((b - a) * N * 2)
+        if kind == "plain":
+            nvr.check(l.nvr_linear(d_x.ptr, K, d_W.ptr, n, K, N, y.ptr, 0, None))
+        elif kind == "silu":
+            nvr.check(l.nvr_linear_silu_mul(d_x.ptr, K, d_W.ptr, n, K, N, y.ptr, None))
+        else:
+            kc, vc, d_pos, d_slots = dev(np.zeros((n, KVH, D), F16)), dev(np.zeros((n, KVH, D), F16)), dev(pos[a:b]), dev(slots[:n])
+            nvr.check(l.nvr_linear_qkv_rope_store(d_x.ptr, K, d_W.ptr, n, K, H, KVH, D, d_pos.ptr, d_slots.ptr, d_cos.ptr, d_sin.ptr, y.ptr, kc.ptr, vc.ptr, None))
+            out = y.to_numpy((n, N), np.uint16)
+            assert np.array_equal(kc.to_numpy((n, KVH * D), np.uint16), out[:, H * D:(H + KVH) * D]) and np.array_equal(vc.to_numpy((n, KVH * D), np.uint16), out[:, (H + KVH) * D:])
+            return out
+        return y.to_numpy((n, N), np.uint16)
+    whole = run(0, T)
+    for a, b in ((0, 130), (2500, 2700), (4030, 4160), (T - 140, T)):
+        if b <= T:
+            assert np.array_equal(run(a, b), whole[a:b]), (a, b)
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("tokens", [2200, 3300, 4400])
+def test_prompt_steps_add_products_to_the_residual_rows_in_place(dtype, tokens):
+    """Steps whose o / down products are added where the residual rows lie (tiles of both kernels, a last tile that is partly past the end): the logits of a prompt of more tokens than split-k
+    slabs hold against the same prompt in portions of 1100 tokens, which take other tiles, bit for bit."""
+    model = nvr.ModelConfig(vocab_size=512, hidden_size=1024, intermediate_size=1536, num_hidden_layers=2, num_attention_heads=8, num_key_value_heads=4, head_dim=128,
+                            max_position_embeddings=8192, tie_word_embeddings=1, seed=7)
+    prompt, got = nvr.synthetic_tokens(tokens, 3, 0, 512), []
+    sp = nvr.SamplingParams(temperature=0.0, max_tokens=1, ignore_eos=True)
+    for kw in (dict(max_num_batched_tokens=tokens + 64), dict(max_num_batched_tokens=1100, enable_chunked_prefill=1)):
+        eng = nvr.LLMEngine(nvr.Config(max_num_seqs=1, max_model_len=tokens + 8, kvcache_block_size=256, num_kvcache_blocks=tokens // 256 + 2, dtype=dtype, **kw), model)
+        eng.add_request(prompt, sp)
+        while not eng.is_finished():
+            rec = eng.step()
+        got.append(eng.model_runner.logits(1).copy())
+    assert np.array_equal(got[0], got[1])                                             # (portions of more than 1024 tokens: none sums k in slices)
