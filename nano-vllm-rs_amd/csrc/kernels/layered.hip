@@ -943,6 +943,172 @@ __global__ __launch_bounds__(256) void retention_block_kernel(RetentionArgs a, B
     if (nown) S[(int64_t)dn * Dv + Dv - 1] = sn;
 }
 
+// Retention over prompts in chunks of 16 tokens on the f32 matrix instructions (key sizes 64 and 128, one decay per head, fully rotated bf16 rows): with S the state before the chunk and
+// decay d, token i of the chunk reads  o_i = d^(i+1) S^T q_i + sum_(j <= i) d^(i-j) (q_i . k_j) v_j  and the chunk leaves  S <- d^n S + sum_j d^(n-1-j) k_j v_j^T.
+// The recurrence token by token (retention_block_kernel) is bound by the vector units: 3 instructions per number of the state and token, without packed f32.  Here these are two products of
+// 16 tokens with f32 operands and sums (v_mfma_f32_16x16x4_f32, twice the vector units' rate), and the state is rounded once in 16 tokens by the decay.
+// A workgroup holds D x 64 of a head's state, wave w columns 16 w .. + 15 of all D rows, as accumulators: lane l, register r of tile t is row 16 t + 4 (l >> 4) + r, column l & 15.  With the
+// inner index of step r taken as 4 (l >> 4) + r the same registers are the B operand of S^T q, and the transposed scores (k q^T: row j, column i) are the A operand of their product with v:
+// neither passes through LDS.  The scores' sums over D are shared by the waves (D / 4 coordinates each, added in the order of the waves).  The next chunk's rows lie
+// in LDS, and the one after is requested, before this one's last barrier: one barrier per chunk.  Powers of the decay: products in f64, rounded once, that of the
+// state's own as two f32 numbers.  A chunk's k v^T is summed before it joins the state, whose error against 64 bits is thereby
+// below the token-by-token sum's (1024 tokens of a unit normal: output 1.7e-7 of its size against 4.6e-7, state 1.6e-7 against 5.5e-7; 16 tokens 1.16e-7 against 1.24e-7).
+// 16 x 1024 tokens, 16 heads of 128 x 128: 266 us against 686 of the recurrence (150 us of matrix instructions; the rest is LDS, rotation and the waits of a chunk at two waves a SIMD);
+// one prompt of 1024: 163 against 352; 2 x 16 tokens, 64 heads of 128 x 64: 6.9 against 11.0.  Not a bit-for-bit cut: where a prompt's portions end moves the chunks' limits.
+template <int D>
+__global__ __launch_bounds__(256, 2) void retention_chunk_kernel(RetentionArgs a, Batch b) {
+    constexpr int ND = D / 16, QS = D + 4, KS = 20, HALF = D / 2, PT = D / 8;      // (row strides: the 16 lanes of a b128 read touch every bank once)
+    constexpr int BUF = 2 * 16 * QS + D * KS + 64 * KS;
+    extern __shared__ __attribute__((aligned(16))) float rsm[];                     // two chunks' q, k, k^T and v^T; two chunks' scores [4][64][4]; the powers
+    float *const pw = rsm + 2 * BUF + 2 * 1024, *const pl = pw + 20;
+    const int sq = blockIdx.x, h = blockIdx.y, cb = blockIdx.z * 64, Dv = a.Dv;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, m = lane & 15, g = lane >> 4;
+    const int hq = a.qk_share > 1 ? h / a.qk_share : h;
+    const int r0 = b.cu[sq], n = b.cu[sq + 1] - r0, st = b.start[sq];
+    if (tid == 0) { double p = 1.0; const double dd = a.decay[h]; for (int i = 0; i < 17; ++i) { pw[i] = (float)p; pl[i] = (float)(p - (double)pw[i]); p *= dd; } }
+    float *S = a.state + (((int64_t)b.slot[sq] * a.H + h) * D) * Dv + cb + w * 16 + m;
+    f32x4 sa[ND];
+#pragma unroll
+    for (int t = 0; t < ND; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sa[t][r] = st > 0 ? S[(int64_t)(16 * t + 4 * g + r) * Dv] : 0.f;
+#pragma unroll
+    for (int t = 0; t < ND; ++t) asm volatile("" : "+v"(sa[t]));                   // (waited for here, not in the loop)
+    // staged: 4 coordinates of the lower half and their partners of one token's q and k, 4 value columns of a token
+    const int ti = tid / PT & 15, d0 = (tid % PT) * 4, vi = tid >> 4, vc = (tid & 15) * 4;
+    const bool rot = D == 128 || tid < 16 * PT;
+    uint2 ql, qh, kl, kh, vv;
+    f32x4 cs, sn;
+    const bf16_t *pq = (const bf16_t *)a.proj + (int64_t)r0 * a.ld + hq * D + d0, *pv = (const bf16_t *)a.proj + (int64_t)r0 * a.ld + a.vcol + (int64_t)h * Dv + cb + vc;
+    const float *cp = a.cos_t + (int64_t)st * HALF + d0, *sp = a.sin_t + (int64_t)st * HALF + d0;
+    // (no branch around the loads, which would bring their wait up to it: tokens past the end read the last one's row, and put() leaves zeros for them)
+    auto request = [&](int i0) {
+        const int64_t i = min(i0 + ti, n - 1);
+        const bf16_t *pr = pq + i * a.ld;
+        ql = *reinterpret_cast<const uint2 *>(pr + a.qcol); qh = *reinterpret_cast<const uint2 *>(pr + a.qcol + HALF);
+        kl = *reinterpret_cast<const uint2 *>(pr + a.kcol); kh = *reinterpret_cast<const uint2 *>(pr + a.kcol + HALF);
+        cs = *reinterpret_cast<const f32x4 *>(cp + i * HALF); sn = *reinterpret_cast<const f32x4 *>(sp + i * HALF);
+        vv = *reinterpret_cast<const uint2 *>(pv + (int64_t)min(i0 + vi, n - 1) * a.ld);
+    };
+    auto put = [&](float *buf, int i0) {
+        float *qs = buf, *ks = qs + 16 * QS, *kt = ks + 16 * QS, *vt = kt + D * KS;
+        asm volatile("" : "+v"(ql), "+v"(qh), "+v"(kl), "+v"(kh), "+v"(cs), "+v"(sn), "+v"(vv));
+        const uint32_t mk = i0 + ti < n ? 0xffffffffu : 0u, mv = i0 + vi < n ? 0xffffffffu : 0u;
+        kl.x &= mk; kl.y &= mk; kh.x &= mk; kh.y &= mk; vv.x &= mv; vv.y &= mv;
+        const bf16_t *e0 = reinterpret_cast<const bf16_t *>(&ql), *e1 = reinterpret_cast<const bf16_t *>(&qh), *f0 = reinterpret_cast<const bf16_t *>(&kl), *f1 = reinterpret_cast<const bf16_t *>(&kh);
+        const bf16_t *ve = reinterpret_cast<const bf16_t *>(&vv);
+        f32x4 q0, q1, k0, k1;
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            const float qu = ld_f(e0, y), qv = ld_f(e1, y), ku = ld_f(f0, y), kv = ld_f(f1, y);
+            q0[y] = qu * cs[y] - qv * sn[y]; q1[y] = qv * cs[y] + qu * sn[y];
+            k0[y] = (ku * cs[y] - kv * sn[y]) * a.kscale; k1[y] = (kv * cs[y] + ku * sn[y]) * a.kscale;
+        }
+        if (rot) {
+#pragma unroll
+            for (int y = 0; y < 4; ++y) { kt[(d0 + y) * KS + ti] = k0[y]; kt[(HALF + d0 + y) * KS + ti] = k1[y]; }
+            *reinterpret_cast<f32x4 *>(qs + ti * QS + d0) = q0; *reinterpret_cast<f32x4 *>(qs + ti * QS + HALF + d0) = q1;
+            *reinterpret_cast<f32x4 *>(ks + ti * QS + d0) = k0; *reinterpret_cast<f32x4 *>(ks + ti * QS + HALF + d0) = k1;
+        }
+#pragma unroll
+        for (int y = 0; y < 4; ++y) vt[(vc + y) * KS + vi] = ld_f(ve, y);
+    };
+    if (n > 0) {
+        request(0);
+        put(rsm, 0);
+        request(16);
+    }
+    __syncthreads();
+    float wp[4], wo[4], wv[4], dh = pw[16], dl = pl[16];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) { const int j = 4 * g + r; wp[r] = pw[max(m - j, 0)]; wo[r] = pw[j + 1]; wv[r] = pw[15 - j]; }
+    for (int i0 = 0; i0 < n; i0 += 16) {
+        // one barrier per chunk: everything of this chunk's buffer is read, and the next one's is written, before it
+        const int nb = min(16, n - i0), par = (i0 >> 4) & 1;
+        const float *qs = rsm + par * BUF, *ks = qs + 16 * QS, *kt = ks + 16 * QS, *vt = kt + D * KS;
+        float *ps = rsm + 2 * BUF + par * 1024;
+        f32x4 pp = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < ND / 4; ++t) {
+            f32x4 pt = {0.f, 0.f, 0.f, 0.f};
+            const int c = w * (D / 4) + 16 * t + 4 * g;
+            const f32x4 kf = *reinterpret_cast<const f32x4 *>(ks + m * QS + c), qf = *reinterpret_cast<const f32x4 *>(qs + m * QS + c);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) pt = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[r], qf[r], pt, 0, 0, 0);
+            pp = t ? pp + pt : pt;
+        }
+        *reinterpret_cast<f32x4 *>(ps + (w * 64 + lane) * 4) = pp;
+        f32x4 o[ND];                                                               // (a sum per tile: 16 products each, then over the tiles)
+#pragma unroll
+        for (int t = 0; t < ND; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < ND; t += 2) {
+            const f32x4 qa = *reinterpret_cast<const f32x4 *>(qs + m * QS + 16 * t + 4 * g), qb = *reinterpret_cast<const f32x4 *>(qs + m * QS + 16 * t + 16 + 4 * g);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[r], sa[t][r], o[t], 0, 0, 0);
+                o[t + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(qb[r], sa[t + 1][r], o[t + 1], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int d = ND / 2; d; d >>= 1)
+#pragma unroll
+            for (int t = 0; t < d; ++t) o[t] = o[t] + o[t + d];
+        put(rsm + (par ^ 1) * BUF, i0 + 16);
+        request(i0 + 32);
+        const f32x4 vf = *reinterpret_cast<const f32x4 *>(vt + (w * 16 + m) * KS + 4 * g);
+        f32x4 vw;
+        if (nb < 16) {                                                             // the last chunk of a prompt
+            dh = pw[nb]; dl = pl[nb];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) wv[r] = pw[max(nb - 1 - (4 * g + r), 0)];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vw[r] = vf[r] * wv[r];
+#pragma unroll
+        for (int t = 0; t < ND; t += 2) {                                          // the chunk's own sum first, then one rounding of the state
+            const f32x4 ka = *reinterpret_cast<const f32x4 *>(kt + (16 * t + m) * KS + 4 * g), kb = *reinterpret_cast<const f32x4 *>(kt + (16 * t + 16 + m) * KS + 4 * g);
+            f32x4 ua = {0.f, 0.f, 0.f, 0.f}, ub = ua, uc = ua, ud = ua;
+#pragma unroll
+            for (int r = 0; r < 4; r += 2) {
+                ua = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[r], vw[r], ua, 0, 0, 0);
+                ub = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[r], vw[r], ub, 0, 0, 0);
+                uc = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[r + 1], vw[r + 1], uc, 0, 0, 0);
+                ud = __builtin_amdgcn_mfma_f32_16x16x4f32(kb[r + 1], vw[r + 1], ud, 0, 0, 0);
+            }
+            ua = ua + uc; ub = ub + ud;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                sa[t][r] = fmaf(sa[t][r], dh, fmaf(sa[t][r], dl, ua[r]));
+                sa[t + 1][r] = fmaf(sa[t + 1][r], dh, fmaf(sa[t + 1][r], dl, ub[r]));
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            const f32x4 px = *reinterpret_cast<const f32x4 *>(ps + (y * 64 + lane) * 4);
+            pp = y ? pp + px : px;
+        }
+        f32x4 oc = {0.f, 0.f, 0.f, 0.f}, od = oc;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            pp[r] = m >= 4 * g + r ? pp[r] * wp[r] : 0.f;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {
+            oc = __builtin_amdgcn_mfma_f32_16x16x4f32(pp[r], vf[r], oc, 0, 0, 0);
+            od = __builtin_amdgcn_mfma_f32_16x16x4f32(pp[r + 1], vf[r + 1], od, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (4 * g + r < nb) a.o[(int64_t)(r0 + i0 + 4 * g + r) * a.H * Dv + (int64_t)h * Dv + cb + w * 16 + m] = fmaf(o[0][r], wo[r], oc[r] + od[r]);
+    }
+#pragma unroll
+    for (int t = 0; t < ND; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[(int64_t)(16 * t + 4 * g + r) * Dv] = sa[t][r];
+}
+
 template <class OT>
 __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float *__restrict__ o, const OT *__restrict__ gate, int64_t ldg, int64_t gcol, int H, int Dv,
                                                              float eps, const float *__restrict__ w, OT *__restrict__ out, int64_t ldo, int w_heads) {
@@ -1070,6 +1236,7 @@ static const size_t kMaxLds = 160 * 1024 - 2048;
 int prepare() {
     NVR_HIP_CHECK(hipFuncSetAttribute((const void *)sink_attn_rows_kernel<float>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
     NVR_HIP_CHECK(hipFuncSetAttribute((const void *)sink_attn_rows_kernel<bf16_t>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
+    NVR_HIP_CHECK(hipFuncSetAttribute((const void *)retention_chunk_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
     NVR_HIP_CHECK(hipFuncSetAttribute((const void *)sink_attn_mfma_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
     NVR_HIP_CHECK(hipFuncSetAttribute((const void *)sink_attn_mfma_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
     NVR_HIP_CHECK(hipFuncSetAttribute((const void *)sink_attn_mfma_kernel<256>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
@@ -1247,6 +1414,16 @@ int retention(const RetentionArgs &a, const Batch &b, bool bf16, hipStream_t s) 
         else if (bf16) retention_seq_kernel<R_, bf16_t, 0><<<grid, dim3(256), 0, s>>>(a, b);     \
         else retention_seq_kernel<R_, float, 0><<<grid, dim3(256), 0, s>>>(a, b);                \
     } while (0)
+    // steps that hold a prompt of a whole chunk or more (from 16 rows the chunk form is the faster one at every size measured: 4.8 us against 7.9 at 2 x 16 tokens, 2 heads of 64 x 64; single
+    // tokens keep the recurrence, which the state's bytes bound)
+    if (bf16 && !gated && !a.tok_gate && a.v_ones == 0 && (a.D == 64 || a.D == 128) && a.rot_dims == a.D && a.Dv % 64 == 0 && b.max_rows >= 16 && ((a.ld | a.qcol | a.kcol | a.vcol) & 3) == 0 &&
+        ((uintptr_t)a.proj & 7) == 0 && (((uintptr_t)a.cos_t | (uintptr_t)a.sin_t) & 15) == 0) {
+        const dim3 g((unsigned)b.B, (unsigned)a.H, (unsigned)(a.Dv / 64));
+        const size_t lds = (2 * (32 * ((size_t)a.D + 4) + (a.D + 64) * 20) + 2 * 1024 + 40) * 4;
+        if (a.D == 64) retention_chunk_kernel<64><<<g, dim3(256), lds, s>>>(a, b);
+        else retention_chunk_kernel<128><<<g, dim3(256), lds, s>>>(a, b);
+        return launched("retention");
+    }
     const size_t lds = ((size_t)(gated ? 3 : 2) * 16 * a.D + 16 * 32 + 16 * 8 * 32 + 32 + 128) * 4;
     if (a.D <= 256 && lds <= 64 * 1024) {                 // (beyond: the token-by-token form, whose LDS does not grow with the key size)
         const dim3 grid((unsigned)b.B, (unsigned)a.H, (unsigned)(((a.tok_gate && a.v_ones == 1 ? a.Dv - 1 : a.Dv) + 31) / 32));   // (a single column of ones rides in the first block)

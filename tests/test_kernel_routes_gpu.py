@@ -601,3 +601,24 @@ def test_prompt_steps_add_products_to_the_residual_rows_in_place(dtype, tokens):
             rec = eng.step()
         got.append(eng.model_runner.logits(1).copy())
     assert np.array_equal(got[0], got[1])                                             # (portions of more than 1024 tokens: none sums k in slices)
+
+
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (64, 192), (128, 64), (128, 128)])
+@pytest.mark.parametrize("lens", [(16, 1, 17), (31, 33, 15), (48, 50, 3)])
+def test_retention_prompts_in_chunks_of_16_tokens(dim, vdim, lens):
+    """The prompt form of retention (key sizes 64 and 128, bfloat16): whole chunks, one token over and one short, sequences of less than a chunk beside longer ones, a second portion that starts from
+    the state the first one left, then two single tokens through the recurrence; quick, slow and nearly no decay.  Row by row against the float64 restatement."""
+    import rugudra_util as u
+    cfg = u.make_config([u.retention_layer(3, dim, vdim, decay=[0.3, 0.95, 0.9995], ff=None)], width=128, taps=3)
+    w = u.make_weights(cfg, seed=dim + vdim)
+    d = u.Driver(cfg, w, dtype="bfloat16", slots=3, pages=48, max_tokens=256, max_len=256)
+    rng = np.random.default_rng(lens[0])
+    toks = [rng.integers(0, 97, n + 2 * lens[0] + 2) for n in lens]
+    at, rows = [0, 0, 0], [[], [], []]
+    for step in (lens, (lens[0], lens[0] + 1, lens[0] - 1), (1, 1, 1), (1, 1, 1)):
+        out = d.step([("s%d" % i, toks[i][at[i]:at[i] + n]) for i, n in enumerate(step)])
+        for i, n in enumerate(step):
+            at[i] += n
+            rows[i].append(out["s%d" % i])
+    for i in range(3):
+        _compare_layer_rows(cfg, w, "bfloat16", [toks[i][:at[i]]], [np.concatenate(rows[i])[-4:]])
