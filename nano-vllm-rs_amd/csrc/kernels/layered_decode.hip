@@ -97,11 +97,20 @@ __global__ __launch_bounds__(256, 1) void attn_decode_kernel(SinkAttnArgs a, Bat
                 for (int ks = 0; ks < NKS; ++ks) vf[mt][ks] = *reinterpret_cast<const bf16x8 *>(vp + min(ks * 32 + lq * 8, Dv - 8));
         }
         f32x4 pn[2];
-        if constexpr (PEN)
+        if constexpr (PEN) {
+            if (base + CH - 1 <= pos) {                 // four neighbours of the table in one request (their distance falls as the key rises)
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt)
+                for (int mt = 0; mt < 2; ++mt) {
+                    f32x4 r;
+                    __builtin_memcpy(&r, pen + (pos - (base + mt * 16 + lq * 4 + 3)), 16);
+                    pn[mt] = f32x4{r[3], r[2], r[1], r[0]};
+                }
+            } else
 #pragma unroll
-                for (int e = 0; e < 4; ++e) pn[mt][e] = pen[max(pos - (base + mt * 16 + lq * 4 + e), 0)];
+                for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) pn[mt][e] = pen[max(pos - (base + mt * 16 + lq * 4 + e), 0)];
+        }
         f32x4 s[2];
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {

@@ -701,8 +701,10 @@ kl::SinkAttnArgs LayeredModel::diff_args(const LayerW &w, const LayeredSpec::Lay
 
 // One position per sequence: up to four workgroups per compute unit share the keys.
 int LayeredModel::decode_attention(nvr_model_runner &r, const kl::SinkAttnArgs &a, const StepPlan &p) {
+    // shares of the keys: at most two workgroups on a compute unit, all resident at once.  More shares leave some units with three of them and most with two, and merge more partial rows (16
+    // sequences of 1040 keys, 8 key/value heads: 4 shares 20.0 us, 5 26.3; of 2048 keys: 4 32.9, 8 40.6; 64 of 1040: 1 56.9, 2 64.7; 8 of 8192, 4 heads: 16 37, 32 47)
     const int64_t pairs = (int64_t)p.b.B * kl::attention_decode_groups(a);
-    return kl::attention_decode(a, p.b, (int)std::max<int64_t>(1, 4 * (int64_t)r.num_cus / std::max<int64_t>(pairs, 1)), attn_ws, attn_ws_bytes, dec_tickets, (int)dec_tickets_n, r.stream);
+    return kl::attention_decode(a, p.b, (int)std::max<int64_t>(1, 2 * (int64_t)r.num_cus / std::max<int64_t>(pairs, 1)), attn_ws, attn_ws_bytes, dec_tickets, (int)dec_tickets_n, r.stream);
 }
 
 // Tensors by the names of the checkpoint: "embed", "head", "final.norm" [W], "pos" [positions][W], "side.embed" [vocab][layers * side]; per layer i "l<i>.norm1" / "norm1b" / "norm2" / "norm2b" [W],
