@@ -62,6 +62,8 @@ struct SinkAttnArgs {
     // softmax attention of its own over the same values, and out = f (a1 - lambda a2) / sqrt(mean^2 + eps) over the head's Dv numbers, f = out_scale * sigmoid(head_gate[t * ldhg + h])
     // (head_gate rows of the operand type; null: no gate).  General form: the maps' outputs pass through maps_o ([T][H][2][Dv] f32).  Not together with penalties, sinks or gate_bias
     const float *lambda; float out_scale, eps; const void *head_gate; int64_t ldhg; float *maps_o;
+    // attention_decode: not null: the step's own key and value rows (sequence s: nk + s * ldn, [G][D], and nv, [G][Dv]; 16-byte aligned) are not in the pages yet: they are read here and stored there
+    const void *nk, *nv; int64_t ldn;
 };
 int sink_attention(const SinkAttnArgs &a, const Batch &b, bool bf16, hipStream_t s);     // any shape; a context that fits the LDS score buffer
 // The same on the matrix cores (bf16 operands, D % 32 == 0 and Dv % 16 == 0, with two maps D % 16 == 0 and Dv % 8 == 0, both <= 256, at most 16 query heads per key/value head — a head with

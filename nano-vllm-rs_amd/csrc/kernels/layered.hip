@@ -194,39 +194,62 @@ __global__ __launch_bounds__(256) void norm_canon_rows_kernel(const float *__res
 
 // The join behind the last sublayer and norm_canon of one-row chunks (decode steps) in one launch: x <- x + mult * y where y is the operand type's rounding of the sum of
 // `parts` partial products [parts][T][W] (linear_splitk: added in their order), then the norm, the convolution over the slot's history and the history of the next step.  One
-// row per workgroup, NI 4-column pieces per thread, everything requested before the first sum: the launch is one trip to memory, as each of the two was (16 rows of 1024: 4.6 + 10.6 -> 8.0 us).
-template <class OT, int NI>
-__global__ __launch_bounds__(256) void join_norm_canon_kernel(float *__restrict__ x, const float *__restrict__ parts, int nparts, float mult, Batch b, int W, float eps, int taps, float g1,
+// row per workgroup, NI 4-column pieces per thread, everything requested before the first sum: the launch is one trip to memory, as each of the two was (16 rows of 1024: 4.6 + 10.6 -> 5.0 us).
+// TAPS: the taps where they are 2, 3 or 4 — a thread's weights are then TAPS 16-byte pieces of its four columns, requested with the rest (a general number, TAPS 0, reads them one by one behind the
+// norm: 8.1 us).  parts null: no join, the norm and convolution of one-row chunks alone (10.9 -> 5.0 us).
+template <class OT, int NI, int TAPS>
+__global__ __launch_bounds__(256) void join_norm_canon_kernel(float *__restrict__ x, const float *__restrict__ parts, int nparts, float mult, Batch b, int W, float eps, int taps_rt, float g1,
                                                               const float *__restrict__ w1, OT *__restrict__ out1, float g2, const float *__restrict__ w2, OT *__restrict__ out2,
                                                               float *__restrict__ hist, int64_t slots) {
     __shared__ float red[4];
+    constexpr int MT = TAPS ? TAPS : 8;
+    const int taps = TAPS ? TAPS : taps_rt;
     const int t = blockIdx.x, st = b.start[t], hrows = taps - 1;               // (one row per sequence: row t is sequence t)
     const int64_t slot = b.slot[t], stride = (int64_t)b.T * W; const int par = b.par[t];
     const float *hin = hist + ((int64_t)par * slots + slot) * hrows * W;
     float *hout = hist + ((int64_t)(par ^ 1) * slots + slot) * hrows * W;
-    float4 v[NI], h[NI][7];
-    float ss = 0.f;
+    float4 v[NI], h[NI][MT > 1 ? MT - 1 : 1], p[NI][8];
+    float k1[NI][TAPS ? TAPS * 4 : 1], k2[NI][TAPS ? TAPS * 4 : 1];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int c = (threadIdx.x + i * 256) * 4;
         if (c >= W) continue;
         v[i] = *reinterpret_cast<const float4 *>(x + (int64_t)t * W + c);
+        if (parts)
 #pragma unroll
-        for (int d = 1; d < 8; ++d) {                                          // the row d back: history row hrows - d, or zero before position 0
+            for (int z = 0; z < 8; ++z) if (z < nparts) p[i][z] = *reinterpret_cast<const float4 *>(parts + z * stride + (int64_t)t * W + c);
+        if constexpr (TAPS != 0)
+#pragma unroll
+            for (int j = 0; j < TAPS; ++j) {
+                *reinterpret_cast<float4 *>(&k1[i][j * 4]) = *reinterpret_cast<const float4 *>(w1 + (int64_t)c * TAPS + j * 4);
+                if (out2) *reinterpret_cast<float4 *>(&k2[i][j * 4]) = *reinterpret_cast<const float4 *>(w2 + (int64_t)c * TAPS + j * 4);
+            }
+#pragma unroll
+        for (int d = 1; d < MT; ++d) {                                         // the row d back: history row hrows - d, or zero before position 0
             h[i][d - 1] = float4{0.f, 0.f, 0.f, 0.f};
             if (d <= hrows && st - d >= 0) h[i][d - 1] = *reinterpret_cast<const float4 *>(hin + (int64_t)(hrows - d) * W + c);
         }
-        float4 y = *reinterpret_cast<const float4 *>(parts + (int64_t)t * W + c);
-        for (int z = 1; z < nparts; ++z) {
-            const float4 p = *reinterpret_cast<const float4 *>(parts + z * stride + (int64_t)t * W + c);
-            y.x += p.x; y.y += p.y; y.z += p.z; y.w += p.w;
-        }
-        float yr[4] = {y.x, y.y, y.z, y.w};
-        OT ro[4];
+    }
+    float ss = 0.f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) { st_f(ro, e, yr[e]); yr[e] = ld_f(ro, e); }
-        v[i].x += mult * yr[0]; v[i].y += mult * yr[1]; v[i].z += mult * yr[2]; v[i].w += mult * yr[3];
-        *reinterpret_cast<float4 *>(x + (int64_t)t * W + c) = v[i];
+    for (int i = 0; i < NI; ++i) {
+        const int c = (threadIdx.x + i * 256) * 4;
+        if (c >= W) continue;
+        if (parts) {
+            float4 y = p[i][0];
+#pragma unroll
+            for (int z = 1; z < 8; ++z) if (z < nparts) { y.x += p[i][z].x; y.y += p[i][z].y; y.z += p[i][z].z; y.w += p[i][z].w; }
+            for (int z = 8; z < nparts; ++z) {
+                const float4 q = *reinterpret_cast<const float4 *>(parts + z * stride + (int64_t)t * W + c);
+                y.x += q.x; y.y += q.y; y.z += q.z; y.w += q.w;
+            }
+            float yr[4] = {y.x, y.y, y.z, y.w};
+            OT ro[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { st_f(ro, e, yr[e]); yr[e] = ld_f(ro, e); }
+            v[i].x += mult * yr[0]; v[i].y += mult * yr[1]; v[i].z += mult * yr[2]; v[i].w += mult * yr[3];
+            *reinterpret_cast<float4 *>(x + (int64_t)t * W + c) = v[i];
+        }
         ss += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
     }
     ss = block_sum<256>(ss, red);
@@ -238,16 +261,16 @@ __global__ __launch_bounds__(256) void join_norm_canon_kernel(float *__restrict_
         const float u0[4] = {v[i].x * r, v[i].y * r, v[i].z * r, v[i].w * r};
         float a1[4] = {0.f, 0.f, 0.f, 0.f}, a2[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {                                          // tap j weighs the row taps - 1 - j back
+        for (int j = 0; j < MT; ++j) {                                         // tap j weighs the row taps - 1 - j back
             if (j >= taps) break;
             const int d = taps - 1 - j;
             float uu[4] = {u0[0], u0[1], u0[2], u0[3]};
 #pragma unroll
-            for (int q = 1; q < 8; ++q) if (d == q) { uu[0] = h[i][q - 1].x; uu[1] = h[i][q - 1].y; uu[2] = h[i][q - 1].z; uu[3] = h[i][q - 1].w; }
+            for (int q = 1; q < MT; ++q) if (d == q) { uu[0] = h[i][q - 1].x; uu[1] = h[i][q - 1].y; uu[2] = h[i][q - 1].z; uu[3] = h[i][q - 1].w; }
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                a1[e] += w1[(int64_t)(c + e) * taps + j] * (g1 * uu[e]);
-                if (out2) a2[e] += w2[(int64_t)(c + e) * taps + j] * (g2 * uu[e]);
+                a1[e] += (TAPS ? k1[i][TAPS ? e * TAPS + j : 0] : w1[(int64_t)(c + e) * taps + j]) * (g1 * uu[e]);
+                if (out2) a2[e] += (TAPS ? k2[i][TAPS ? e * TAPS + j : 0] : w2[(int64_t)(c + e) * taps + j]) * (g2 * uu[e]);
             }
             if (d < hrows) *reinterpret_cast<float4 *>(hout + (int64_t)(hrows - 1 - d) * W + c) = float4{uu[0], uu[1], uu[2], uu[3]};
         }
@@ -257,6 +280,14 @@ __global__ __launch_bounds__(256) void join_norm_canon_kernel(float *__restrict_
         st4_f(out1, (int64_t)t * W + c, o1);
         if (out2) st4_f(out2, (int64_t)t * W + c, o2);
     }
+}
+template <class OT, int NI>
+void join_norm_canon_launch(float *x, const float *parts, int nparts, float mult, const Batch &b, int W, float eps, int taps, float g1, const float *w1, void *out1, float g2, const float *w2,
+                            void *out2, float *hist, int64_t slots, hipStream_t s) {
+    const bool al = ((uintptr_t)w1 | (uintptr_t)w2) % 16 == 0;
+    auto k = !al ? join_norm_canon_kernel<OT, NI, 0> : taps == 2 ? join_norm_canon_kernel<OT, NI, 2> : taps == 3 ? join_norm_canon_kernel<OT, NI, 3> : taps == 4 ? join_norm_canon_kernel<OT, NI, 4>
+                 : join_norm_canon_kernel<OT, NI, 0>;
+    k<<<dim3((unsigned)b.T), dim3(256), 0, s>>>(x, parts, nparts, mult, b, W, eps, taps, g1, w1, (OT *)out1, g2, w2, (OT *)out2, hist, slots);
 }
 // the join alone (behind the last layer)
 template <class OT>
@@ -1262,6 +1293,7 @@ int norm_canon(const float *x, const Batch &b, int64_t W, float eps, int taps, f
                bool bf16, float *hist, int64_t slots, hipStream_t s) {
     if (b.T == 0) return 0;
     if (taps < 1) return nvr::fail(NVR_ERR_INVALID_ARG, "norm_canon: taps %d (at least 1)", taps);
+    if (join_norm_canon_ok(b, W, taps, x, nullptr, hist)) return join_norm_canon(const_cast<float *>(x), nullptr, 0, 0.f, b, W, eps, taps, g1, w1, out1, g2, w2, out2, bf16, hist, slots, s);
     if (W % 4 == 0 && taps <= 8 && ((uintptr_t)x | (uintptr_t)hist) % 16 == 0) {
         // rows per workgroup: many for prompts (the convolution weights of a column are read once per workgroup), few for decode-sized steps (more workgroups)
 #define NVR_NC(RB_)                                                                                                                                       \
@@ -1287,12 +1319,11 @@ bool join_norm_canon_ok(const Batch &b, int64_t W, int taps, const float *x, con
 int join_norm_canon(float *x, const float *parts, int nparts, float mult, const Batch &b, int64_t W, float eps, int taps, float g1, const float *w1, void *out1, float g2, const float *w2,
                     void *out2, bool bf16, float *hist, int64_t slots, hipStream_t s) {
     if (b.T == 0) return 0;
-    if (!join_norm_canon_ok(b, W, taps, x, parts, hist) || nparts < 1) return nvr::fail(NVR_ERR_UNSUPPORTED, "join_norm_canon: %d rows of %d sequences, width %ld, %d taps", b.T, b.B, (long)W, taps);
-    const dim3 grid((unsigned)b.T);
-#define NVR_JNC(NI_)                                                                                                                                                                   \
-    do {                                                                                                                                                                               \
-        if (bf16) join_norm_canon_kernel<bf16_t, NI_><<<grid, dim3(256), 0, s>>>(x, parts, nparts, mult, b, (int)W, eps, taps, g1, w1, (bf16_t *)out1, g2, w2, (bf16_t *)out2, hist, slots); \
-        else join_norm_canon_kernel<float, NI_><<<grid, dim3(256), 0, s>>>(x, parts, nparts, mult, b, (int)W, eps, taps, g1, w1, (float *)out1, g2, w2, (float *)out2, hist, slots);       \
+    if (!join_norm_canon_ok(b, W, taps, x, parts, hist) || (parts && nparts < 1)) return nvr::fail(NVR_ERR_UNSUPPORTED, "join_norm_canon: %d rows of %d sequences, width %ld, %d taps", b.T, b.B, (long)W, taps);
+#define NVR_JNC(NI_)                                                                                                                                                   \
+    do {                                                                                                                                                               \
+        if (bf16) join_norm_canon_launch<bf16_t, NI_>(x, parts, nparts, mult, b, (int)W, eps, taps, g1, w1, out1, g2, w2, out2, hist, slots, s);                      \
+        else join_norm_canon_launch<float, NI_>(x, parts, nparts, mult, b, (int)W, eps, taps, g1, w1, out1, g2, w2, out2, hist, slots, s);                             \
     } while (0)
     if (W <= 1024) NVR_JNC(1); else if (W <= 2048) NVR_JNC(2); else NVR_JNC(4);
 #undef NVR_JNC

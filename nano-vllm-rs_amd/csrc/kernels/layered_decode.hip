@@ -82,14 +82,17 @@ __global__ __launch_bounds__(256, 1) void attn_decode_kernel(SinkAttnArgs a, Bat
         const int base = x < kept ? x * CH : j0 + (x - kept) * CH;
         bf16x8 kf[2][NKS], vf[2][NKS];
         int64_t row[2];
+        bool own[2];                                    // the lane's row is the step's own one and lies outside the pages
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
             const int j = min(base + mt * 16 + lm, ctx - 1), pg = bs_shift >= 0 ? j >> bs_shift : j / bs;
             row[mt] = ((int64_t)bt[pg] * bs + (j - pg * bs)) * a.G + kvh;
+            own[mt] = !SHARED && a.nk != nullptr && j == pos;
         }
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
-            const bf16_t *kp = kc + row[mt] * D, *vp = vc + row[mt] * Dv;
+            const bf16_t *kp = own[mt] ? (const bf16_t *)a.nk + (int64_t)sq * a.ldn + (int64_t)kvh * D : kc + row[mt] * D;
+            const bf16_t *vp = own[mt] ? (const bf16_t *)a.nv + (int64_t)sq * a.ldn + (int64_t)kvh * Dv : vc + row[mt] * Dv;
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks) kf[mt][ks] = *reinterpret_cast<const bf16x8 *>(kp + min(ks * 32 + lq * 8, D - 8));
             if constexpr (!SHARED)
@@ -111,6 +114,17 @@ __global__ __launch_bounds__(256, 1) void attn_decode_kernel(SinkAttnArgs a, Bat
 #pragma unroll
                     for (int e = 0; e < 4; ++e) pn[mt][e] = pen[max(pos - (base + mt * 16 + lq * 4 + e), 0)];
         }
+        if (!SHARED && a.nk && base + CH > pos)         // the chunk that ends with it: its lanes (several, with the same bytes) leave it in the pages
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt)
+                if (own[mt]) {
+                    bf16_t *kd = (bf16_t *)a.kc + row[mt] * D, *vd = (bf16_t *)a.vc + row[mt] * Dv;
+#pragma unroll
+                    for (int ks = 0; ks < NKS; ++ks) {
+                        *reinterpret_cast<bf16x8 *>(kd + min(ks * 32 + lq * 8, D - 8)) = kf[mt][ks];
+                        *reinterpret_cast<bf16x8 *>(vd + min(ks * 32 + lq * 8, Dv - 8)) = vf[mt][ks];
+                    }
+                }
         f32x4 s[2];
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
@@ -281,7 +295,7 @@ int prepare_decode() {
 bool attention_decode_ok(const SinkAttnArgs &a, bool bf16) {
     const bool shared = a.vld != 0;
     return bf16 && !a.r1 && !a.r2 && !a.slope && !(a.pen && (a.lambda || shared)) && !a.gate_bias && a.softcap == 0.f && a.chunk == 0 && !(a.lambda && a.sink) && a.G >= 1 && a.H % a.G == 0 && a.D % 32 == 0 && a.Dv % 16 == 0 &&
-           a.D <= 256 && a.Dv <= 256 && !(a.v_grouped && !shared) && (!shared || (a.vc == a.kc && a.vld == a.D && a.Dv <= a.D && a.G == 1 && !a.lambda)) && a.ldq % 8 == 0 && a.ldo % 4 == 0 &&
+           a.D <= 256 && a.Dv <= 256 && !(a.v_grouped && !shared) && (!shared || (a.vc == a.kc && a.vld == a.D && a.Dv <= a.D && a.G == 1 && !a.lambda)) && a.ldq % 8 == 0 && a.ldo % 4 == 0 && (!a.nk || (!shared && a.ldn % 8 == 0 && (((uintptr_t)a.nk | (uintptr_t)a.nv) & 15) == 0)) &&
            (((uintptr_t)a.q | (uintptr_t)a.kc | (uintptr_t)a.vc) & 15) == 0 && ((uintptr_t)a.out & 7) == 0;
 }
 

@@ -469,7 +469,13 @@ int LayeredModel::forward(nvr_model_runner &r, const StepPlan &p) {
             a.out = cat; a.ldo = w.kcat;
             a.v_grouped = w.flash ? 0 : 1;                                          // (a property of the layer: the pages keep one layout)
             const bool tiled = kl::sink_attention_tiled_ok(a, bf16, (int)r.block_size);   // (a property of the layer's shape: the same answer every step)
-            RC(kl::kv_store(proj, w.nmix, w.kcol, w.vcol, b, L.kv_heads, L.dim, L.vdim, st.kc, st.vc, bf16, tiled && !w.flash, s));
+            // one position per sequence: the kernel for few query rows, with the table in the two factors' place (16 x 1040 keys of 8 heads: 40.2 + 5.5 us with the merge -> 25.0); it also puts the
+            // step's own key and value rows into the pages
+            kl::SinkAttnArgs d = a;
+            d.r1 = d.r2 = nullptr;
+            d.nk = (const char *)proj + (size_t)(w.kcol * esz); d.nv = (const char *)proj + (size_t)(w.vcol * esz); d.ldn = w.nmix;
+            const bool few = tiled && p.decode_sized && kl::attention_decode_ok(d, bf16);
+            if (!few) RC(kl::kv_store(proj, w.nmix, w.kcol, w.vcol, b, L.kv_heads, L.dim, L.vdim, st.kc, st.vc, bf16, tiled && !w.flash, s));
             if (w.flash && !p.decode_sized) {
                 // prompts and portions: the dense graph's flash kernel in its penalty / sink form (K and V through the block tables, the step's own rows included)
                 const size_t gi = flash_kind(nvr::kb::flash_tile_positions((int)L.heads, (int)L.kv_heads));
@@ -488,9 +494,8 @@ int LayeredModel::forward(nvr_model_runner &r, const StepPlan &p) {
                     wm.pen_dirty = false;
                 }
                 a.pen = wm.pen; a.pen_n = (int32_t)r.max_pos;
-                kl::SinkAttnArgs d = a;                                             // one position per sequence: the kernel for few query rows, with the table in the two factors' place (16 x 1040 keys of 8 heads: 40.2 + 5.5 us with the merge -> 25.0)
-                d.r1 = d.r2 = nullptr;
-                if (p.decode_sized && kl::attention_decode_ok(d, bf16)) RC(decode_attention(r, d, p));
+                d.pen = wm.pen; d.pen_n = (int32_t)r.max_pos;
+                if (few) RC(decode_attention(r, d, p));
                 else {
                 const size_t gi = (size_t)(std::find(attn_groups.begin(), attn_groups.end(), L.heads / L.kv_heads) - attn_groups.begin());
                 // decode-sized steps over long contexts: few tiles, many keys each — spread every tile's keys over several workgroups

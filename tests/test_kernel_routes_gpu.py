@@ -622,3 +622,21 @@ def test_retention_prompts_in_chunks_of_16_tokens(dim, vdim, lens):
             rows[i].append(out["s%d" % i])
     for i in range(3):
         _compare_layer_rows(cfg, w, "bfloat16", [toks[i][:at[i]]], [np.concatenate(rows[i])[-4:]])
+
+
+@pytest.mark.parametrize("taps", [2, 3, 4, 5])
+@pytest.mark.parametrize("dim,width", [(64, 132), (128, 1028)])
+def test_layer_list_single_tokens_across_pages(taps, dim, width):
+    """Single tokens of a layer-list model: the norm and convolution with their weights in registers (2 to 4 taps, one of several 4-column pieces of a row left over) and read one by one (5), the
+    decode attention that puts the step's own key and value rows into the pages itself — first and last row of a page, a page just begun — with chunks of keys that end at, before and behind the
+    position.  Against the float64 restatement, row by row."""
+    import rugudra_util as u
+    cfg = u.make_config([u.attention_layer(4, 2, dim, dim, ff=None), u.attention_layer(2, 1, dim, dim, ff=None)], width=width, taps=taps)
+    w = u.make_weights(cfg, seed=taps)
+    d = u.Driver(cfg, w, dtype="bfloat16", slots=3, pages=24, max_tokens=128, max_len=96)
+    rng = np.random.default_rng(dim)
+    toks = [rng.integers(0, 97, n) for n in (20, 36, 70)]
+    first = [n - 6 for n in (20, 36, 70)]                                    # positions 14 .. 19, 30 .. 35 and 64 .. 69 of pages of 16
+    d.step([("s%d" % i, t[:f]) for i, (t, f) in enumerate(zip(toks, first))])
+    out = [d.step([("s%d" % i, t[f + k:f + k + 1]) for i, (t, f) in enumerate(zip(toks, first))]) for k in range(6)]
+    _compare_layer_rows(cfg, w, "bfloat16", toks, [np.concatenate([o["s%d" % i] for o in out]) for i in range(3)])
