@@ -17,11 +17,8 @@ namespace nvr { namespace kf {
 #define F32_LAUNCH_CHECK(what)                                                                                          \
     do { hipError_t e_ = hipGetLastError(); if (e_ != hipSuccess) return nvr::fail(NVR_ERR_HIP, what " launch failed: %s", hipGetErrorString(e_)); } while (0)
 
-__device__ __forceinline__ float wsum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
+// (the pairs of a 32, 16, 8, 4, 2, 1 butterfly, on the lane swaps and DPP: six round trips through LDS less at the end of every output column)
+__device__ __forceinline__ float wsum(float v) { return wave_sum(v); }
 __device__ __forceinline__ float wmax(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
@@ -299,19 +296,48 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 // arithmetic (a thread's columns c = tid, tid + 256, ..; fma chain of squares; wave sums, then the four waves in order; v / rms * w): the same bits.
 // Every workgroup of a consumer GEMV does this for itself (K floats per row: nothing beside the weight rows it streams), so the add + norm launch in
 // front of the GEMV disappears; h_out (given to ONE workgroup) receives the new residual stream — a second buffer, the others are still reading h_in.
+// NormRows: a thread's first four columns (all of them up to K = 1024), requested IN FRONT of the weight pieces — loads come back in order, and behind the weights the norm would start only
+// when those have arrived (qkv of K = 1024 / N = 4096: 8.1 -> 5.0 us, gate_up of 3072: 8.2 -> 6.2 us).
 template <int TT>
-__device__ __forceinline__ void add_norm_rows_to_lds(const float *__restrict__ h_in, const float *__restrict__ y, const float *__restrict__ nw, float eps, int T,
+struct NormRows {
+    float h[TT][4], y[TT][4], w[4];
+    __device__ __forceinline__ void request(const float *__restrict__ h_in, const float *__restrict__ yp, const float *__restrict__ nw, int T, int K) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int c = min((int)threadIdx.x + 256 * u, K - 1);
+#pragma unroll
+            for (int t = 0; t < TT; ++t) { const int64_t o = (int64_t)(t < T ? t : 0) * K + c; h[t][u] = h_in[o]; y[t][u] = yp[o]; }
+            w[u] = nw[c];
+        }
+        asm volatile("" ::: "memory");
+    }
+};
+template <int TT>
+__device__ __forceinline__ void add_norm_rows_to_lds(NormRows<TT> &n, const float *__restrict__ h_in, const float *__restrict__ y, const float *__restrict__ nw, float eps, int T,
                                                      int K, float *__restrict__ h_out, float *xs, float *sm) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     float ss[TT];
 #pragma unroll
     for (int t = 0; t < TT; ++t) ss[t] = 0.f;
-    for (int c = tid; c < K; c += 256) {
-        float hv[TT], yv[TT];
 #pragma unroll
-        for (int t = 0; t < TT; ++t) { const int64_t o = (int64_t)(t < T ? t : 0) * K + c; hv[t] = h_in[o]; yv[t] = y[o]; }
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int t = 0; t < TT; ++t) { const float v = hv[t] + yv[t]; xs[t * K + c] = v; ss[t] = fmaf(v, v, ss[t]); }
+        for (int t = 0; t < TT; ++t) { n.h[t][u] = tid + 256 * u < K ? n.h[t][u] + n.y[t][u] : 0.f; ss[t] = fmaf(n.h[t][u], n.h[t][u], ss[t]); }
+    for (int c0 = tid + 1024; c0 < K; c0 += 1024) {
+        float hv[TT][4], yv[TT][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int c = min(c0 + 256 * u, K - 1);
+#pragma unroll
+            for (int t = 0; t < TT; ++t) { const int64_t o = (int64_t)(t < T ? t : 0) * K + c; hv[t][u] = h_in[o]; yv[t][u] = y[o]; }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int c = c0 + 256 * u;
+            if (c < K)
+#pragma unroll
+                for (int t = 0; t < TT; ++t) { const float v = hv[t][u] + yv[t][u]; xs[t * K + c] = v; ss[t] = fmaf(v, v, ss[t]); }
+        }
     }
 #pragma unroll
     for (int t = 0; t < TT; ++t) { const float v = wsum(ss[t]); if (lane == 0) sm[t * 4 + wave] = v; }
@@ -323,7 +349,21 @@ __device__ __forceinline__ void add_norm_rows_to_lds(const float *__restrict__ h
         for (int i = 1; i < 4; ++i) r = r + sm[t * 4 + i];
         rms[t] = sqrtf(r / (float)K + eps);
     }
-    for (int c = tid; c < K; c += 256) {
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+        if (t < T) {
+            float o[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) o[u] = n.h[t][u] / rms[t] * n.w[u];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (tid + 256 * u < K) xs[t * K + tid + 256 * u] = o[u];
+            if (h_out)
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (tid + 256 * u < K) h_out[(int64_t)t * K + tid + 256 * u] = n.h[t][u];
+        }
+    for (int c = tid + 1024; c < K; c += 256) {
         const float w = nw[c];
 #pragma unroll
         for (int t = 0; t < TT; ++t)
@@ -388,10 +428,12 @@ __global__ __launch_bounds__(256) void gemv_silu_kernel(const float *__restrict_
     const float4 *g4 = reinterpret_cast<const float4 *>(W + (int64_t)n * K), *u4 = reinterpret_cast<const float4 *>(W + (int64_t)(I + n) * K);
     const int n4 = K / 4;
     float4 wg0[4], wu0[4];                                              // NORM: the first weight pieces are requested in front of the norm (they depend on nothing)
-    if (NORM) {
+    if constexpr (NORM) {
+        NormRows<TT> nr;
+        nr.request(h_in, y, nw, T, K);
 #pragma unroll
         for (int u = 0; u < 4; ++u) { const int k4 = min(lane + 64 * u, n4 - 1); wg0[u] = g4[k4]; wu0[u] = u4[k4]; }
-        add_norm_rows_to_lds<TT>(h_in, y, nw, eps, T, K, blockIdx.x == 0 ? h_out : nullptr, xs, xs + TT * K); x = xs; ldx = K;
+        add_norm_rows_to_lds<TT>(nr, h_in, y, nw, eps, T, K, blockIdx.x == 0 ? h_out : nullptr, xs, xs + TT * K); x = xs; ldx = K;
     }
     if (n_ >= I) return;
     float ag[TT], au[TT];
@@ -431,13 +473,14 @@ int linear_silu_mul(const float *x, int64_t ldx, const float *W, int64_t T, int6
     if (!linear_silu_ok(T, K, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "f32 linear_silu_mul: T=%ld K=%ld (decode-sized steps)", (long)T, (long)K);
     const dim3 grid((unsigned)((I + 3) / 4));
     if (T == 1) gemv_silu_kernel<1><<<grid, dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)I, bias, act);
+    else if (T == 2) gemv_silu_kernel<2><<<grid, dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)I, bias, act);
     else if (T <= 4) gemv_silu_kernel<4><<<grid, dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)I, bias, act);
     else gemv_silu_kernel<8><<<grid, dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)I, bias, act);
     F32_LAUNCH_CHECK("f32 gemv + silu");
     return 0;
 }
-// rows of the launch's template instance (1 / 4 / 8) and whether their normalised image fits the LDS a kernel gets without an opt-in
-static int gemv_rows(int64_t T) { return T == 1 ? 1 : T <= 4 ? 4 : 8; }
+// rows of the launch's template instance (1 / 2 / 4 / 8) and whether their normalised image fits the LDS a kernel gets without an opt-in
+static int gemv_rows(int64_t T) { return T <= 2 ? (int)T : T <= 4 ? 4 : 8; }
 bool fused_norm_ok(int64_t T, int64_t K) { return T >= 1 && T <= 8 && K % 4 == 0 && (size_t)gemv_rows(T) * (K + 4) * 4 <= 48 * 1024; }
 int add_norm_linear_silu_mul(const float *h_in, const float *y, const float *nw, float eps, float *h_out, const float *W, int64_t T, int64_t K, int64_t I,
                              const float *bias, float *act, hipStream_t s) {
@@ -445,7 +488,7 @@ int add_norm_linear_silu_mul(const float *h_in, const float *y, const float *nw,
     const dim3 grid((unsigned)((I + 3) / 4));
     const size_t lds = (size_t)gemv_rows(T) * (K + 4) * 4;
 #define NVR_GS(TT_) gemv_silu_kernel<TT_, true><<<grid, dim3(256), lds, s>>>(nullptr, 0, W, (int)T, (int)K, (int)I, bias, act, h_in, y, nw, eps, h_out)
-    if (T == 1) NVR_GS(1); else if (T <= 4) NVR_GS(4); else NVR_GS(8);
+    if (T == 1) NVR_GS(1); else if (T == 2) NVR_GS(2); else if (T <= 4) NVR_GS(4); else NVR_GS(8);
 #undef NVR_GS
     F32_LAUNCH_CHECK("f32 add + norm + gemv + silu");
     return 0;
@@ -455,6 +498,7 @@ int linear(const float *x, int64_t ldx, const float *W, int64_t T, int64_t K, in
     if (T <= 8 && K % 4 == 0 && ldx % 4 == 0) {
         const dim3 grid((unsigned)((N + 3) / 4));
         if (T == 1) gemv_kernel<1><<<grid, dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)N, bias, y);
+        else if (T == 2) gemv_kernel<2><<<grid, dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)N, bias, y);
         else if (T <= 4) gemv_kernel<4><<<grid, dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)N, bias, y);
         else gemv_kernel<8><<<grid, dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)N, bias, y);
         F32_LAUNCH_CHECK("f32 gemv");
@@ -525,11 +569,14 @@ __global__ __launch_bounds__(256) void gemv_rope_kernel(const float *__restrict_
     const float4 *g4 = reinterpret_cast<const float4 *>(W + (int64_t)n1 * K), *u4 = reinterpret_cast<const float4 *>(W + (int64_t)n2 * K);
     const int n4 = K / 4;
     float4 w10[4], w20[4];
-    if (NORM) {
+    NormRows<NORM ? TT : 1> nr;
+    if constexpr (NORM) nr.request(h_in, y, nw, T, K);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) { const int k4 = min(lane + 64 * u, n4 - 1); w10[u] = g4[k4]; w20[u] = u4[k4]; }
-        add_norm_rows_to_lds<TT>(h_in, y, nw, eps, T, K, blockIdx.x == 0 ? h_out : nullptr, xs, xs + TT * K); x = xs; ldx = K;
-    }
+    for (int u = 0; u < 4; ++u) { const int k4 = min(lane + 64 * u, n4 - 1); w10[u] = g4[k4]; w20[u] = u4[k4]; }
+    float cs[TT], sn[TT];                                               // (behind the reduction they would be a round trip of their own; the weights do not wait for the positions)
+#pragma unroll
+    for (int t = 0; t < TT; ++t) { cs[t] = cos_t[p[t] * half + j]; sn[t] = sin_t[p[t] * half + j]; }
+    if constexpr (NORM) { add_norm_rows_to_lds<TT>(nr, h_in, y, nw, eps, T, K, blockIdx.x == 0 ? h_out : nullptr, xs, xs + TT * K); x = xs; ldx = K; }
     if (pair_ >= N / 2) return;
     float a1[TT], a2[TT];
 #pragma unroll
@@ -539,7 +586,7 @@ __global__ __launch_bounds__(256) void gemv_rope_kernel(const float *__restrict_
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int k4 = min(k0 + 64 * u, n4 - 1);
-            if (NORM && k0 == lane) { w1[u] = w10[u]; w2[u] = w20[u]; } else { w1[u] = g4[k4]; w2[u] = u4[k4]; }
+            if (k0 == lane) { w1[u] = w10[u]; w2[u] = w20[u]; } else { w1[u] = g4[k4]; w2[u] = u4[k4]; }
 #pragma unroll
             for (int t = 0; t < TT; ++t) a[t][u] = reinterpret_cast<const float4 *>(x + (int64_t)(t < T ? t : 0) * ldx)[k4];
         }
@@ -562,8 +609,7 @@ __global__ __launch_bounds__(256) void gemv_rope_kernel(const float *__restrict_
             if (bias) { x1 = x1 + bias[n1]; x2 = x2 + bias[n2]; }
             float o1 = x1, o2 = x2;
             if (!is_v) {
-                const float c = cos_t[p[t] * half + j], sn = sin_t[p[t] * half + j];
-                o1 = rot_sub(x1, c, x2, sn); o2 = rot_add(x2, c, x1, sn);
+                o1 = rot_sub(x1, cs[t], x2, sn[t]); o2 = rot_add(x2, cs[t], x1, sn[t]);
             }
             float *row = qkv + (int64_t)t * N;
             row[n1] = o1; row[n2] = o2;
@@ -581,7 +627,7 @@ int linear_qkv_rope_store(const float *x, int64_t ldx, const float *W, int64_t T
     const int64_t pairs = (H + 2 * KVH) * D / 2;
     const dim3 grid((unsigned)((pairs + 3) / 4));
 #define NVR_GR(TT_) gemv_rope_kernel<TT_><<<grid, dim3(256), 0, s>>>(x, ldx, W, (int)T, (int)K, (int)H, (int)KVH, (int)D, bias, pos, slots, cos_t, sin_t, qkv, kc, vc)
-    if (T == 1) NVR_GR(1); else if (T <= 4) NVR_GR(4); else NVR_GR(8);
+    if (T == 1) NVR_GR(1); else if (T == 2) NVR_GR(2); else if (T <= 4) NVR_GR(4); else NVR_GR(8);
 #undef NVR_GR
     F32_LAUNCH_CHECK("f32 gemv + rope + store");
     return 0;
@@ -596,7 +642,7 @@ int add_norm_linear_qkv_rope_store(const float *h_in, const float *y, const floa
     const size_t lds = (size_t)gemv_rows(T) * (K + 4) * 4;
 #define NVR_GR(TT_) gemv_rope_kernel<TT_, true><<<grid, dim3(256), lds, s>>>(nullptr, 0, W, (int)T, (int)K, (int)H, (int)KVH, (int)D, bias, pos, slots, cos_t, sin_t, \
                                                                             qkv, kc, vc, h_in, y, nw, eps, h_out)
-    if (T == 1) NVR_GR(1); else if (T <= 4) NVR_GR(4); else NVR_GR(8);
+    if (T == 1) NVR_GR(1); else if (T == 2) NVR_GR(2); else if (T <= 4) NVR_GR(4); else NVR_GR(8);
 #undef NVR_GR
     F32_LAUNCH_CHECK("f32 add + norm + gemv + rope + store");
     return 0;
@@ -809,8 +855,10 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnArgsF a, int paged) 
 // in LDS.  What bounds a decode step's launch is that chain of round trips, not bytes.  Qwen3-0.6B, us a launch, the general form / this one: one sequence of 150 keys 14.3 / 7.3, of 4096 keys
 // 195 / 78 (a decode step of one sequence, 128 / 512 / 1024 / 2048 / 4096 / 8000 keys: 1230 / 1798 / 2467 / 3752 / 6293 / 11132 us before it and the other changes beside it, 1021 / 1247 / 1504 /
 // 2002 / 3000 / 4922 now); prompts of 128 rows 38 / 19, 509 268 / 129, 1024 873 / 401
-template <int NF, int NW, bool PAGED>
-__global__ __launch_bounds__(64 * NW) void attention_rows_kernel(AttnArgsF a) {
+// PAGED 2: pages of a power of two tokens (1 << shift): a shift and a mask per key where the general form divides twice, some 40 instructions each in front of every request
+// (one sequence of 150 keys 7.4 -> 7.0 us a launch)
+template <int NF, int NW, int PAGED>
+__global__ __launch_bounds__(64 * NW) void attention_rows_kernel(AttnArgsF a, int shift) {
     constexpr int D = 64 * NF, KB = NF <= 2 ? 4 : 2;                     // keys a group requests at a time
     constexpr int STEP = 16, ROUND = KB * STEP, NEXT = NW == 8 ? 2 * ROUND : ROUND;   // groups of four waves; keys of their round; from a wave's round to its next one
     __shared__ __attribute__((aligned(16))) float part[8][D];
@@ -821,8 +869,9 @@ __global__ __launch_bounds__(64 * NW) void attention_rows_kernel(AttnArgsF a) {
     const int32_t *bt = PAGED ? a.block_tables + (int64_t)(a.seq_of_q ? a.seq_of_q[t] : t) * a.max_blocks : nullptr;
     const int64_t base = PAGED ? 0 : (int64_t)a.kv_base[t];
     // block of key j (any j >= 0: entries behind a sequence's blocks may be stale, and are never used: a key past the context reads key 0's row)
-    auto entry = [&](int j) -> int { return PAGED ? bt[min(j / a.block_size, a.max_blocks - 1)] : 0; };
+    auto entry = [&](int j) -> int { return PAGED ? bt[min(PAGED == 2 ? j >> shift : j / a.block_size, a.max_blocks - 1)] : 0; };
     auto row_of = [&](int e, int j) -> int64_t {                        // element offset of key j's row of this kv head
+        if (PAGED == 2) return ((((int64_t)max(e, 0) << shift) + (j & ((1 << shift) - 1))) * a.KVH + g) * D;
         if (PAGED) return (((int64_t)max(e, 0) * a.block_size + j % a.block_size) * a.KVH + g) * D;
         return (base + j) * a.ldkv + (int64_t)g * D;
     };
@@ -948,8 +997,10 @@ int attention(const AttnArgsF &a, bool paged, hipStream_t s) {
     const bool pieces = a.D % 64 == 0 && a.ldq % 4 == 0 && (paged || a.ldkv % 4 == 0) && (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) & 15) == 0;
     if (pieces) {
         const bool few = (int64_t)a.nq * a.H < 512;
-#define NVR_ARW(NF_, NW_) do { if (paged) attention_rows_kernel<NF_, NW_, true><<<grid, dim3(64 * NW_), 0, s>>>(a); \
-                               else attention_rows_kernel<NF_, NW_, false><<<grid, dim3(64 * NW_), 0, s>>>(a); } while (0)
+        const int shift = paged && (a.block_size & (a.block_size - 1)) == 0 ? __builtin_ctz((unsigned)a.block_size) : -1;
+#define NVR_ARW(NF_, NW_) do { if (shift >= 0) attention_rows_kernel<NF_, NW_, 2><<<grid, dim3(64 * NW_), 0, s>>>(a, shift); \
+                               else if (paged) attention_rows_kernel<NF_, NW_, 1><<<grid, dim3(64 * NW_), 0, s>>>(a, 0); \
+                               else attention_rows_kernel<NF_, NW_, 0><<<grid, dim3(64 * NW_), 0, s>>>(a, 0); } while (0)
 #define NVR_AR(NF_) do { if (few) NVR_ARW(NF_, 8); else NVR_ARW(NF_, 4); } while (0)
         if (a.D == 64) NVR_AR(1); else if (a.D == 128) NVR_AR(2); else if (a.D == 192) NVR_AR(3); else NVR_AR(4);
 #undef NVR_AR

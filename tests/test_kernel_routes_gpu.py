@@ -640,3 +640,33 @@ def test_layer_list_single_tokens_across_pages(taps, dim, width):
     d.step([("s%d" % i, t[:f]) for i, (t, f) in enumerate(zip(toks, first))])
     out = [d.step([("s%d" % i, t[f + k:f + k + 1]) for i, (t, f) in enumerate(zip(toks, first))]) for k in range(6)]
     _compare_layer_rows(cfg, w, "bfloat16", toks, [np.concatenate([o["s%d" % i] for o in out]) for i in range(3)])
+
+
+@pytest.mark.parametrize("hidden", [72, 1020, 1284, 3072])
+def test_float32_decode_rows_form_their_norm_from_columns_in_registers(hidden):
+    """float32 decode steps of 5, 2 and 1 rows whose add + norm rides in the consuming products: rows of less than a thread's first four columns, a few short of them, and beyond them (ragged and
+    whole) — the logits of the runner that keeps the launches apart, bit for bit; pages of 24 tokens (no power of two) beside pages of 16."""
+    import os
+    model = nvr.ModelConfig(vocab_size=400, hidden_size=hidden, intermediate_size=96, num_hidden_layers=2, num_attention_heads=2, num_key_value_heads=1, head_dim=64, max_position_embeddings=128,
+                            tie_word_embeddings=1, seed=hidden)
+    prompts = [nvr.synthetic_tokens(11 + 9 * i, 5, i, 400) for i in range(5)]
+    got = []
+    for fused, page in (("0", 16), ("1", 16), ("1", 24)):
+        os.environ["NVR_F32_FUSED_NORM"] = fused
+        try:
+            eng = nvr.LLMEngine(nvr.Config(skip_block_size_check=1, dtype="float32", max_num_seqs=5, max_num_batched_tokens=256, max_model_len=96, kvcache_block_size=page, num_kvcache_blocks=40), model)
+        finally:
+            os.environ.pop("NVR_F32_FUSED_NORM", None)
+        for i, p in enumerate(prompts):
+            eng.add_request(p, nvr.SamplingParams(temperature=0.0, max_tokens=(9, 6, 3, 3, 3)[i], ignore_eos=True))
+        out, rows = [], set()
+        while not eng.is_finished():
+            rec = eng.step()
+            rows.add(rec["num_seqs"])
+            out.append((rec["tokens"], eng.model_runner.logits(rec["num_seqs"]).copy().view(np.uint32)))
+        assert {1, 2, 5} <= rows
+        got.append(out)
+    for other in got[1:]:
+        assert len(other) == len(got[0])
+        for (ta, la), (tb, lb) in zip(got[0], other):
+            assert ta == tb and np.array_equal(la, lb)
