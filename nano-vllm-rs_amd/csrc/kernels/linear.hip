@@ -31,9 +31,9 @@
 namespace nvr { namespace NVR_DT_NS {
 
 enum { EPI_F16 = 0, EPI_F32 = 1, EPI_SILU = 2, EPI_ROPE = 3, EPI_SLAB = 4, EPI_CLAMP = 5 };
-// rows up to which a decode step's add + norm rides on the product behind it: every workgroup reads every row's slabs again (16 KB a row at K = 1024), so the launch it saves pays for one
-// or two rows — Qwen3-0.6B at 300 keys, us a step apart / riding: 802 / 769 at one row, 822 / 800 at two, 851 / 890 at four
-constexpr int64_t NORM_ROWS = 2;
+// rows up to which a decode step's add + norm rides on the product behind it: every workgroup reads every row's slabs again (16 KB a row at K = 1024), so the launch it saves pays for a few
+// rows — Qwen3-0.6B at 300 keys, us a step apart / riding: 802 / 727 at one row, 822 / 760 at two, 840 / 792 at three, 863 / 826 at four (as many as NORM_ELEMS holds of that width)
+constexpr int64_t NORM_ROWS = 4;
 
 struct LinEpi {
     // EPI_SILU, EPI_CLAMP: N is the intermediate size I; W holds gate rows [0,I) and up rows [I,2I)
@@ -103,30 +103,42 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
 #pragma unroll
         for (int j = 0; j < MT; ++j) acc[i][j] = (float4_t){0.f, 0.f, 0.f, 0.f};
 
-    // EPI_ROPE: the epilogue of token tile j runs on wave j; its position / slot / cos / sin loads are issued here, ahead of the
-    // weight stream, instead of as a chain of dependent global loads (pos -> cos,sin) after the reduction barrier
+    // Loads come back in the order they were requested.  EPI_ROPE: the epilogue of token tile j runs on wave j; its position and slot are requested first, its cosines and sines (which wait for the
+    // position) behind the first weight pieces, all ahead of their use after the reduction barrier.
     float4_t rope_cs = (float4_t){0.f, 0.f, 0.f, 0.f}, rope_sn = rope_cs;
     int rope_slot = -1;
+    int64_t rope_p = 0;
+    const int rope_tph = EPI == EPI_ROPE ? epi.D / 16 : 1, rope_head = blockIdx.x / rope_tph;
     if (EPI == EPI_ROPE && wave < MT) {
-        const int m = m0 + wave * 16 + r, mc = m < T ? m : T - 1;
-        const int tph = epi.D / 16, head = blockIdx.x / tph, c = blockIdx.x % tph, half_d = epi.D / 2;
-        if (head < epi.H + epi.KVH) {
-            const int jj = c * 8 + (q & 1) * 4;
-            const int64_t p = epi.pos[mc];
-            rope_cs = *reinterpret_cast<const float4_t *>(epi.cos_t + p * half_d + jj);
-            rope_sn = *reinterpret_cast<const float4_t *>(epi.sin_t + p * half_d + jj);
-        }
-        if (head >= epi.H && epi.slots && m < T) rope_slot = epi.slots[m];
+        const int m = m0 + wave * 16 + r;
+        rope_p = epi.pos[m < T ? m : T - 1];
+        if (rope_head >= epi.H && epi.slots && m < T) rope_slot = epi.slots[m];
     }
+    auto rope_request = [&]() {
+        if (EPI == EPI_ROPE && wave < MT && rope_head < epi.H + epi.KVH) {
+            const int64_t at = rope_p * (epi.D / 2) + (blockIdx.x % rope_tph) * 8 + (q & 1) * 4;
+            rope_cs = *reinterpret_cast<const float4_t *>(epi.cos_t + at);
+            rope_sn = *reinterpret_cast<const float4_t *>(epi.sin_t + at);
+        }
+    };
     constexpr int KS = 32 * WAVES;
-    half8_t a_first[U][NT];                                  // NORM: the first pieces of the weights, requested in front of the norm (they depend on nothing)
+    constexpr bool AHEAD = NORM || EPI == EPI_ROPE;
+    half8_t a_first[U][NT], b_first[U][MT];                  // AHEAD: the first pieces of the weights (and rows)
+    auto first_request = [&]() {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int kk = min(wave * 32 + u * KS, K - 32);
+#pragma unroll
+            for (int i = 0; i < NT; ++i) a_first[u][i] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(wrow[i] + (int64_t)kk * kmul));
+            if constexpr (!NORM)
+#pragma unroll
+                for (int j = 0; j < MT; ++j) b_first[u][j] = *reinterpret_cast<const half8_t *>(xrow[j] + kk);
+        }
+        asm volatile("" ::: "memory");
+    };
+    if constexpr (AHEAD && !NORM) { first_request(); rope_request(); }
     if constexpr (NORM) {
         static_assert(MT == 1, "one row block");
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int i = 0; i < NT; ++i)
-                a_first[u][i] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(wrow[i] + (int64_t)min(wave * 32 + u * KS, K - 32) * kmul));
         constexpr int NI = NORM_ELEMS / 4 / (WAVES * 64);     // 4-column pieces per thread
         __shared__ float ss_w[NI * WAVES];                    // sums of squares of 64 neighbouring pieces (K is a multiple of 256: inside one row)
         half_t *xs = reinterpret_cast<half_t *>(norm_lds);
@@ -144,6 +156,9 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
                 for (int z = 0; z < 4; ++z) sv[i][z] = z < nm.S ? *reinterpret_cast<const float4_t *>(nm.slabs + z * nm.stride + o) : (float4_t){0.f, 0.f, 0.f, 0.f};
             }
         }
+        asm volatile("" ::: "memory");
+        first_request();                                      // the weights behind the rows: in front of them, the norm would start when they
+                                                              // have arrived (one row: qkv of 4096 columns 6.5 -> 5.5 us, gate_up of 3072 6.6 -> 5.8)
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const int idx = i * (WAVES * 64) + (int)threadIdx.x;
@@ -161,6 +176,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
                 if (lane == 0) ss_w[i * WAVES + wave] = ss;
             }
         }
+        rope_request();
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
@@ -168,7 +184,14 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
             if (idx < total) {
                 const int row = idx / per_row, c = (idx - row * per_row) * 4;
                 float tot = 0.f;
-                for (int k = 0; k < per_row / 64; ++k) tot += ss_w[row * (per_row / 64) + k];
+                const int np = per_row / 64;
+                for (int k0 = 0; k0 < np; k0 += 4) {           // (four requested together, added in their order)
+                    float p[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) p[k] = ss_w[row * np + min(k0 + k, np - 1)];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) if (k0 + k < np) tot += p[k];
+                }
                 const float rms = sqrtf(tot / (float)K + nm.eps);
                 half4_t o;
 #pragma unroll
@@ -191,11 +214,14 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
             if (kk < K) {
 #pragma unroll
                 for (int i = 0; i < NT; ++i) {
-                    if (NORM && k == kbeg + wave * 32) a[u][i] = a_first[u][i];
+                    if (AHEAD && k == kbeg + wave * 32) a[u][i] = a_first[u][i];
                     else a[u][i] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(wrow[i] + (int64_t)kk * kmul));
                 }
 #pragma unroll
-                for (int j = 0; j < MT; ++j) b[u][j] = *reinterpret_cast<const half8_t *>(xrow[j] + kk);
+                for (int j = 0; j < MT; ++j) {
+                    if (AHEAD && !NORM && k == kbeg + wave * 32) b[u][j] = b_first[u][j];
+                    else b[u][j] = *reinterpret_cast<const half8_t *>(xrow[j] + kk);
+                }
             } else {
 #pragma unroll
                 for (int i = 0; i < NT; ++i) a[u][i] = (half8_t)(half_t)0;

@@ -670,3 +670,19 @@ def test_float32_decode_rows_form_their_norm_from_columns_in_registers(hidden):
         assert len(other) == len(got[0])
         for (ta, la), (tb, lb) in zip(got[0], other):
             assert ta == tb and np.array_equal(la, lb)
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("hidden,qk_norm", [(256, False), (768, True), (1024, False), (1280, False)])
+def test_decode_steps_of_one_to_five_rows(hidden, qk_norm, dtype):
+    """A batch that shrinks from five rows to one: the add + norm formed by the consuming products (up to four rows of 1024 numbers, three of 1280; a wave count of row pieces that is and is not a
+    multiple of four) and by its own launch, the rotation's sines requested behind the first weights (key heads, value heads, with and without q / k norms) — logits against the oracle, step by
+    step, at the engine's tolerance for the type."""
+    from oracle import model_oracle as mo
+    from test_engine_gpu import _run_pair
+    mcfg = mo.small(hidden_size=hidden, num_hidden_layers=2, intermediate_size=512, head_dim=128, num_attention_heads=4, num_key_value_heads=2, qk_norm=qk_norm, seed=hidden, init_std=0.02)
+    ecfg = dict(max_num_seqs=5, max_num_batched_tokens=256, max_model_len=128, kvcache_block_size=16, num_kvcache_blocks=40)
+    prompts = [oracle.fill_tokens(6 + 5 * i, 3, i, mcfg.vocab_size).tolist() for i in range(5)]
+    sps = [dict(temperature=0.0, max_tokens=3 + 2 * i, ignore_eos=True) for i in range(5)]
+    r = _run_pair(mcfg, ecfg, prompts, sps, dtype=dtype)
+    assert r["decode_steps"] >= 10
