@@ -462,8 +462,22 @@ __global__ __launch_bounds__(256) void rope_store_kernel(half_t *__restrict__ qk
 // elements of either half in 16-byte pieces (the pairs it rotates), and one workgroup walks a token's heads and value rows together, so that every load
 // of the row is in flight at once.  Bound by the latency of one trip to memory at few rows, by the bytes of the rows at many: against a wave per head and
 // 2-byte pieces (the general form below) 27 rows of 16 + 8 heads of 128 8.0 -> 4.6 us, 509 rows 10.3 -> 4.7, 3062 rows of 32 + 8 heads 39.7 -> 17.3 (4.3 TB/s)
+// A workgroup has a thread for every piece up to 1024 (a second pass over the value rows was a second trip), a head's sum goes over its lanes on DPP in the pairs of a LPH / 2, .., 1 butterfly
+// (27 rows of 16 + 8 heads: 0.4 us of 4.6 a launch in a step)
 template <int LPH>
-__global__ __launch_bounds__(256) void qknorm_rope_store_kernel(half_t *__restrict__ qkv, const int64_t *__restrict__ pos,
+__device__ __forceinline__ float head_sum(float x) {
+    static_assert(LPH == 2 || LPH == 4 || LPH == 8 || LPH == 16, "lanes of a head");
+    if constexpr (LPH == 16) return row_sum<16>(x);
+    if constexpr (LPH >= 8) {                                                 // the lane 4 away inside 8: banks of 4 lanes 0 and 2 take the next bank's, 1 and 3 the one before
+        int y = __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x104, 0xF, 0x5, false);
+        y = __builtin_amdgcn_update_dpp(y, __float_as_int(x), 0x114, 0xF, 0xA, false);
+        x += __int_as_float(y);
+    }
+    if constexpr (LPH >= 4) x = dpp_add<0x4E>(x);
+    return dpp_add<0xB1>(x);
+}
+template <int LPH>
+__global__ __launch_bounds__(1024) void qknorm_rope_store_kernel(half_t *__restrict__ qkv, const int64_t *__restrict__ pos,
                                                                 const int32_t *__restrict__ slots, int H, int KVH,
                                                                 const float *__restrict__ cos_t, const float *__restrict__ sin_t,
                                                                 const half_t *__restrict__ qw, const half_t *__restrict__ kw, float eps,
@@ -474,7 +488,7 @@ __global__ __launch_bounds__(256) void qknorm_rope_store_kernel(half_t *__restri
     const int n_rot = (H + KVH) * LPH, n_v = KVH * LPH * 2;                    // lanes of the rotated heads, then 16-byte pieces of the value rows
     const int slot = slots ? slots[t] : -1;
     const float *c = cos_t + pos[t] * half_d, *sn = sin_t + pos[t] * half_d;
-    for (int i = threadIdx.x; i < n_rot + n_v; i += 256) {                    // (n_rot and 256 are multiples of LPH: a head's lanes take the branch together)
+    for (int i = threadIdx.x; i < n_rot + n_v; i += blockDim.x) {             // (n_rot and whole waves are multiples of LPH: a head's lanes take the branch together)
         if (i >= n_rot) {
             const int e = (i - n_rot) * 8;
             if (slot >= 0) *reinterpret_cast<half8_t *>(vc + (int64_t)slot * KVH * D + e) = *reinterpret_cast<const half8_t *>(row + (int64_t)(H + KVH) * D + e);
@@ -491,8 +505,7 @@ __global__ __launch_bounds__(256) void qknorm_rope_store_kernel(half_t *__restri
         float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) { const float a = (float)x1[e], b = (float)x2[e]; ss += a * a + b * b; }
-#pragma unroll
-        for (int o = LPH / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+        ss = head_sum<LPH>(ss);
         const float rms = sqrtf(ss / (float)D + eps);
         half8_t o1, o2;
 #pragma unroll
@@ -557,7 +570,9 @@ int rope_store_kv(half_bits *qkv, const int64_t *positions, const int32_t *slots
         if (!q_norm_w || !k_norm_w) return nvr::fail(NVR_ERR_INVALID_ARG, "rope_store_kv: q and k norm weights come together");
         // the wide form: heads of a power-of-two number of 16-byte pairs of pieces, everything it reads in 16-byte pieces aligned to them
         const bool wide = (((uintptr_t)qkv | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)q_norm_w | (uintptr_t)k_norm_w | (uintptr_t)cos_t | (uintptr_t)sin_t) & 15) == 0;
-#define NVR_QKN(LPH_) qknorm_rope_store_kernel<LPH_><<<dim3((unsigned)T), dim3(256), 0, s>>>((half_t *)qkv, positions, slots, (int)H, (int)KVH, cos_t, sin_t, \
+        const int64_t pieces = (H + KVH) * (D / 16) + KVH * (D / 8);
+        const unsigned threads = (unsigned)std::min<int64_t>(1024, (pieces + 63) / 64 * 64);
+#define NVR_QKN(LPH_) qknorm_rope_store_kernel<LPH_><<<dim3((unsigned)T), dim3(threads), 0, s>>>((half_t *)qkv, positions, slots, (int)H, (int)KVH, cos_t, sin_t, \
                                                                      (const half_t *)q_norm_w, (const half_t *)k_norm_w, eps, (half_t *)k_cache, (half_t *)v_cache)
         if (wide && D == 128) NVR_QKN(8);
         else if (wide && D == 64) NVR_QKN(4);
