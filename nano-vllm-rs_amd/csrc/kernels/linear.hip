@@ -401,7 +401,7 @@ int decode_splitk_slices(int64_t T, int64_t K, int64_t N) {
 static inline bool prefer_stream(int64_t T, int64_t N) {
     // up to 64 rows the weight-streaming kernel; beyond, the LDS-tiled kernel with 32- / 64-token tiles and the 4-buffer ring (r02,
     // ctx 256: bs 66 2.20 -> 1.83 ms/step, bs 96 2.48 -> 2.15, bs 128 2.82 -> 2.23).
-    return T <= stream_row_limit() || T * N <= 256 * 1024;       // (qkv of 0.6B, 80 rows 9.1 / 7.9, 96 rows 10.0 / 7.9)
+    return T <= stream_row_limit() || T * N <= 192 * 1024;       // (qkv of 0.6B, 80 rows 9.1 / 7.9, 96 rows 10.0 / 7.9)
 }
 static inline int waves_for(int64_t K) { return K >= 2048 ? 16 : (K >= 1024 ? 8 : 4); }
 
@@ -609,7 +609,8 @@ int linear_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, i
 }
 
 // ---- products of a decode step of few rows whose workgroups form RMSNorm(h + slabs) themselves (linear_skinny_kernel, NORM)
-bool norm_linear_ok(int64_t T, int64_t K, int64_t S) { return T >= 1 && T <= NORM_ROWS && K % 256 == 0 && T * K <= NORM_ELEMS && (S == 2 || S == 4); }
+// (three and four rows: from the width on at which the products behind a launch of its own split k over the same eight waves, so that the step's bits are theirs)
+bool norm_linear_ok(int64_t T, int64_t K, int64_t S) { return T >= 1 && T <= NORM_ROWS && (T <= 2 || waves_for(K) == 8) && K % 256 == 0 && T * K <= NORM_ELEMS && (S == 2 || S == 4); }
 template <int NT, int EPI>
 static int norm_launch(const NormIn &nm, const half_bits *W, int64_t T, int64_t K, int64_t N, void *y, const LinEpi &le, int64_t gx, bool tiled, hipStream_t s, const char *what) {
     if (!norm_linear_ok(T, K, nm.S)) return nvr::fail(NVR_ERR_UNSUPPORTED, "%s: T=%ld K=%ld, %d slabs", what, (long)T, (long)K, nm.S);
