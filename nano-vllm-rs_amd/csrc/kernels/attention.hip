@@ -40,7 +40,40 @@ struct AttnParams {
     float *part_o; float *part_ml;     // [nq, H, num_parts, D], [nq, H, num_parts, 2]
     half_t *out;                       // [nq, H, D]
     unsigned int *tickets;             // FUSE: one arrival counter per (query, kv head), zero between launches (the last arriver re-arms it)
+    const half_t *qn_w, *kn_w; float qk_eps; const int64_t *pos; const int32_t *slots; const float *cos_t, *sin_t;   // QKN (AttnArgs)
 };
+
+// One 8-element piece of a head of 128 held by 16 lanes (dc = lane % 16, elements dc * 8 ..): RMSNorm over the head and rotation as qknorm_rope_store_kernel does them — its sums' pairs, its
+// roundings, nothing contracted: the same bits.  g: the norm's weights of the piece, c / s: cosines and sines of pairs (dc % 8) * 8 ..
+__device__ __forceinline__ half8_t norm_rotate_piece(half8_t x, half8_t g, const float4_t (&c)[2], const float4_t (&s)[2], float eps, int dc) {
+#pragma clang fp contract(off)
+    auto partner = [](half8_t v) {                      // the other half's piece, 8 lanes away inside the row of 16
+        int4 w = __builtin_bit_cast(int4, v);
+        w.x = __builtin_amdgcn_update_dpp(0, w.x, 0x128, 0xF, 0xF, false); w.y = __builtin_amdgcn_update_dpp(0, w.y, 0x128, 0xF, 0xF, false);
+        w.z = __builtin_amdgcn_update_dpp(0, w.z, 0x128, 0xF, 0xF, false); w.w = __builtin_amdgcn_update_dpp(0, w.w, 0x128, 0xF, 0xF, false);
+        return __builtin_bit_cast(half8_t, w);
+    };
+    const bool low = dc < 8;
+    const half8_t px = partner(x);
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float a = (float)(low ? x[e] : px[e]), b = (float)(low ? px[e] : x[e]), aa = a * a, bb = b * b, ab = aa + bb;
+        ss = ss + ab;
+    }
+    ss = head_sum<8>(ss);
+    const float rms = sqrtf(ss / 128.0f + eps);
+    half8_t n, o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) n[e] = to_half_rn(__fmul_rn(__fdiv_rn((float)x[e], rms), (float)g[e]));
+    const half8_t pn = partner(n);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float cc = c[e >> 2][e & 3], sn = s[e >> 2][e & 3];
+        o[e] = low ? to_half_rn(mul_sub_unfused((float)n[e], cc, (float)pn[e], sn)) : to_half_rn(mul_add_unfused((float)n[e], cc, (float)pn[e], sn));
+    }
+    return o;
+}
 
 // a * b rounded, then + c rounded: never contracted into an fma, whatever kernel this is inlined into
 __device__ __forceinline__ float mul_then_add(float a, float b, float c) {
@@ -125,8 +158,12 @@ __device__ __forceinline__ half4_t merge_partitions(int np, LoadML load_ml, Load
 // SHM (shared-prefix decode where EVERY query shares the prefix and its own keys fit one partition): the partials of the shared
 // partitions [0, part0) were written by the launch in front of this one (flash_shared_prefix), so the single own-partition workgroup of a (query, kv head) IS
 // the last arriver by stream order: it merges the pair itself (own partial through LDS, the same merge_partitions: the merge launch's bits) — no merge launch.
-template <int D, int G, bool PAGED, bool DIRECT_OUT, int U, int WAVES, bool NT, bool UB, bool FUSE = false, bool SHM = false>
+// QKN (heads of 128, UB): the step's own rows come raw — RMSNorm over q and k heads, rotation and the store of the new key and value row ride here instead of a launch of their own in front
+// (4.6 us a layer at a few rows, as much as this whole kernel over short contexts): the first waves form the G query heads and the key row, 16 lanes a head, while every wave's first keys are on
+// their way; all read them back from LDS.  The row of the last key is taken from there, not from the cache; the workgroup whose keys end with it stores it.
+template <int D, int G, bool PAGED, bool DIRECT_OUT, int U, int WAVES, bool NT, bool UB, bool FUSE = false, bool SHM = false, bool QKN = false>
 __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(AttnParams p) {
+    static_assert(!QKN || (D == 128 && PAGED && UB && !SHM && G < 4 * WAVES), "QKN: paged heads of 128");
     constexpr int LPR = D / 8;          // lanes per K/V row
     constexpr int RPI = 64 / LPR;       // rows per wave-instruction (= tokens per row group)
     constexpr int TPI = RPI * U;        // tokens per chunk
@@ -173,9 +210,26 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(AttnParams p) {
                                              (__attribute__((address_space(3))) void *)shm_pml, 4, 0, 0);
         }
     }
+    // QKN: head item wave * 4 + tg (G query heads, then the key head) of the step's row, and the value row's piece
+    const half_t *own_row = QKN ? p.q + (int64_t)t * p.ldq : nullptr;
+    const int hi = wave * 4 + tg, own_slot = QKN && p.slots ? p.slots[t] : -1;
+    const bool forms = QKN && wave * 4 <= G;                              // (uniform)
+    half8_t hx, hg, own_k, own_v; float4_t hc[2], hs[2];
+    __shared__ half8_t own_lds[QKN ? (G + 1) * 16 : 1];
+    if constexpr (QKN) {
+        const int64_t at = p.pos[t] * (D / 2) + (dc & 7) * 8;
+        if (forms) {
+            const int hh = min(hi, G);
+            hx = *reinterpret_cast<const half8_t *>(own_row + (hh < G ? g * G + hh : p.H + g) * D + dc * 8);
+            hg = *reinterpret_cast<const half8_t *>((hh < G ? p.qn_w : p.kn_w) + dc * 8);
+#pragma unroll
+            for (int x = 0; x < 2; ++x) { hc[x] = *reinterpret_cast<const float4_t *>(p.cos_t + at + 4 * x); hs[x] = *reinterpret_cast<const float4_t *>(p.sin_t + at + 4 * x); }
+        }
+        own_v = *reinterpret_cast<const half8_t *>(own_row + (p.H + p.KVH + g) * D + dc * 8);
+    }
     // q slice of this lane for the G heads of kv head g (fp16 pairs for v_dot2); requested in front of ctx's first use
     half2_t qv[G][4];
-    {
+    if constexpr (!QKN) {
         const half_t *qrow = p.q + (int64_t)t * p.ldq + (int64_t)g * G * D + dc * 8;
 #pragma unroll
         for (int i = 0; i < G; ++i) {
@@ -284,11 +338,8 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(AttnParams p) {
         }
     };
 
-    half8_t kt[U], vt[U];
-    if (R == 0) issue_remainder(kt, vt);
-    for (int r = 0; r < R; ++r) {
-        const int tb = p0 + (r * WAVES + wave) * TPI;
-        half8_t kk[U], vv[U];
+    half8_t kt[U], vt[U], kk[U], vv[U];
+    auto issue_round = [&](int tb) {
         if (PAGED && UB) {
             const int64_t base = block_base(tb);
 #pragma unroll
@@ -303,10 +354,49 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(AttnParams p) {
 #pragma unroll
             for (int u = 0; u < U; ++u) { kk[u] = load_row16<NT>(p.k + off[u]); vv[u] = load_row16<NT>(p.v + off[u]); }
         }
+    };
+    if (R == 0) issue_remainder(kt, vt);
+    if constexpr (QKN) {
+        if (R > 0) issue_round(p0 + wave * TPI);
+        asm volatile("" ::: "memory");                                    // the requests stay in front of the norm
+        if (forms) {
+            const half8_t o = norm_rotate_piece(hx, hg, hc, hs, p.qk_eps, dc);
+            if (hi <= G) own_lds[hi * 16 + dc] = o;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                // (LDS alone: __syncthreads may wait for the keys as well)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            const half8_t h = own_lds[i * 16 + dc];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) qv[i][j] = (half2_t){h[2 * j], h[2 * j + 1]};
+        }
+        own_k = own_lds[G * 16 + dc];
+        if (wave == WAVES - 1 && tg == 0 && own_slot >= 0 && pend == ctx && p0 < ctx) {
+            const int64_t dst = ((int64_t)own_slot * p.KVH + g) * D + dc * 8;
+            *reinterpret_cast<half8_t *>(const_cast<half_t *>(p.k) + dst) = own_k;
+            *reinterpret_cast<half8_t *>(const_cast<half_t *>(p.v) + dst) = own_v;
+        }
+    }
+    // QKN: the pieces of token ctx - 1 among rows tb + step * u + tg (clamped to the partition's last one: those lanes' weights are 0, but what they are multiplied with has to be a number)
+    auto take_own = [&](half8_t (&ka)[U], half8_t (&va)[U], int tb, int step) {
+        if (QKN && own_slot >= 0)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (min(tb + step * u + tg, pend - 1) == ctx - 1) { ka[u] = own_k; va[u] = own_v; }
+    };
+    for (int r = 0; r < R; ++r) {
+        const int tb = p0 + (r * WAVES + wave) * TPI;
+        if (!QKN || r > 0) issue_round(tb);
         if (r == R - 1) issue_remainder(kt, vt);
+        if (QKN && tb + TPI >= ctx) take_own(kk, vv, tb, RPI);
         process(std::false_type{}, kk, vv, 0);
     }
-    if (gt0 < ng) process(std::true_type{}, kt, vt, p0 + gt0 * RPI);
+    if (gt0 < ng) {
+        if (QKN && p0 + (gt0 + (U - 1) * WAVES + 1) * RPI >= ctx) take_own(kt, vt, p0 + gt0 * RPI, WAVES * RPI);
+        process(std::true_type{}, kt, vt, p0 + gt0 * RPI);
+    }
 
     // bring the row-group slots of the wave to their common max and sum them, then merge the waves through LDS
     constexpr bool ONE = SHM && WAVES == 1;                               // one wave per workgroup: its sums ARE the partition's partial (the cross-wave
@@ -718,8 +808,14 @@ size_t attn_workspace_bytes(int64_t nq, int64_t H, int64_t D, int64_t max_ctx) {
 }
 
 template <int D, int G, int U, int WAVES, bool NT>
-static void launch_cfg(const AttnParams &p, bool paged, bool direct, int64_t nwg, hipStream_t s, bool fuse = false, bool shm = false) {
+static void launch_cfg(const AttnParams &p, bool paged, bool direct, int64_t nwg, hipStream_t s, bool fuse = false, bool shm = false, bool qkn = false) {
     dim3 grid((unsigned)nwg), block(WAVES * 64);
+    if constexpr (D == 128 && G <= 4 && WAVES >= 4 && NT)
+        if (qkn) {
+            if (direct) attn_rows_kernel<D, G, true, true, U, WAVES, NT, true, false, false, true><<<grid, block, 0, s>>>(p);
+            else attn_rows_kernel<D, G, true, false, U, WAVES, NT, true, true, false, true><<<grid, block, 0, s>>>(p);
+            return;
+        }
     constexpr int TPI = 64 / (D / 8) * U;
     const bool ub = paged && p.block_size % TPI == 0 && (p.num_parts == 1 || p.part_size % TPI == 0);
     if constexpr (WAVES <= 4 && NT) {                                     // (only instantiated where launch_attn can ask for it)
@@ -743,6 +839,11 @@ static void launch_cfg(const AttnParams &p, bool paged, bool direct, int64_t nwg
         if (direct) attn_rows_kernel<D, G, false, true, U, WAVES, NT, false><<<grid, block, 0, s>>>(p);
         else attn_rows_kernel<D, G, false, false, U, WAVES, NT, false><<<grid, block, 0, s>>>(p);
     }
+}
+
+static int own_rows(const AttnArgs &a, hipStream_t s) {                    // what QKN does inside the attention, by the launch of its own
+    if (!a.qn_w) return 0;
+    return rope_store_kv(const_cast<half_bits *>(a.q), a.pos, a.slots, a.nq, a.H, a.KVH, a.D, a.cos_t, a.sin_t, const_cast<half_bits *>(a.k), const_cast<half_bits *>(a.v), s, a.qn_w, a.kn_w, a.qk_eps);
 }
 
 template <int D, int G>
@@ -839,6 +940,7 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
             p.part_size = 64; p.num_parts = (int32_t)cap;
             p.part_o = (float *)a.workspace; p.part_ml = p.part_o + (int64_t)a.nq * a.H * cap * D;
             p.part0 = 0; p.kv0 = 0; p.kv0_rows = nullptr; p.tickets = a.tickets;
+            if (int rc = own_rows(a, s)) return rc;
             const int shares = (int)std::max<int64_t>(1, cus / a.KVH);                      // one workgroup per CU
             attn_share_kernel<D, G, DU / 2, 8><<<dim3((unsigned)(shares * a.KVH)), dim3(512), 0, s>>>(p, (int)a.nq, shares);
             hipError_t e = hipGetLastError();
@@ -863,18 +965,27 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
     p.tickets = a.tickets;
     // ... and with a shared-prefix pass in front whose group is the whole batch, one own partition per pair: that workgroup merges (SHM)
     const bool shm = shared && paged && !a.shared_rows && np - sparts == 1 && a.tickets != nullptr;
+    // the step's own rows (QKN): in this launch where four or eight waves walk a pair's keys in blocks of whole chunks and there is a CU for every pair (beyond, the start of every pair's workgroup
+    // pays for it again: Qwen3-0.6B with norms at 300 keys, us a step by a launch in front / here: 1 sequence 764 / 721, 2 833 / 784, 4 896 / 826, 8 975 / 912, 16 1062 / 998, 32 1159 / 1115,
+    // 64 1674 / 1677, 128 2243 / 2249; 256 of 1024 keys 6069 / 6090)
+    const int tpi = 64 / (D / 8) * (brief || waves == 4 ? DU : DU / 2);
+    const bool qkn = a.qn_w && D == 128 && G <= 4 && !shared && paged && pairs <= share_workgroups() && (waves == 8 || waves == 4) && (direct || fuse) && p.block_size % tpi == 0 && (p.num_parts == 1 || p.part_size % tpi == 0) && a.ldq % 8 == 0 &&
+                     (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.qn_w | (uintptr_t)a.kn_w | (uintptr_t)a.cos_t | (uintptr_t)a.sin_t) & 15) == 0;
+    if (qkn) { p.qn_w = (const half_t *)a.qn_w; p.kn_w = (const half_t *)a.kn_w; p.qk_eps = a.qk_eps; p.pos = a.pos; p.slots = a.slots; p.cos_t = a.cos_t; p.sin_t = a.sin_t; }
+    else if (int rc = own_rows(a, s)) return rc;
     if (shared)
         if (int rc = flash_shared_prefix(a.q, a.ldq, a.k, a.v, a.block_tables, a.max_blocks, a.block_size, a.nq, a.H, a.KVH, a.D, a.scale,
                                          shared_part, sparts, np, p.part_o, p.part_ml, s, a.shared_rows, a.shared_count)) return rc;
     {
         if (brief) {
             const bool ub = p.block_size % (64 / (D / 8) * DU) == 0;
-            if (ub) attn_rows_kernel<D, G, true, true, DU, 8, true, true><<<dim3((unsigned)nwg), dim3(512), 0, s>>>(p);
+            if (qkn) launch_cfg<D, G, DU, 8, true>(p, true, true, nwg, s, false, false, true);
+            else if (ub) attn_rows_kernel<D, G, true, true, DU, 8, true, true><<<dim3((unsigned)nwg), dim3(512), 0, s>>>(p);
             else attn_rows_kernel<D, G, true, true, DU, 8, true, false><<<dim3((unsigned)nwg), dim3(512), 0, s>>>(p);
-        } else if (waves == 8) launch_cfg<D, G, DU / 2, 8, true>(p, paged, direct, nwg, s, fuse);  // K/V streamed once: nt loads
+        } else if (waves == 8) launch_cfg<D, G, DU / 2, 8, true>(p, paged, direct, nwg, s, fuse, false, qkn);  // K/V streamed once: nt loads
         else if (paged && waves == 1) { if constexpr (G * (D / 4) <= 64) launch_cfg<D, G, DU, 1, true>(p, paged, direct, nwg, s, fuse, shm); }   // (U = 2: 3.18-3.20 against 3.14-3.17 ms per configs[4] step)
         else if (paged && waves == 2) { if constexpr (G * (D / 4) <= 128) launch_cfg<D, G, DU, 2, true>(p, paged, direct, nwg, s, fuse, shm); }
-        else if (paged) launch_cfg<D, G, DU, 4, true>(p, paged, direct, nwg, s, fuse, shm);
+        else if (paged) launch_cfg<D, G, DU, 4, true>(p, paged, direct, nwg, s, fuse, shm, qkn);
         else launch_cfg<D, G, DU, 4, false>(p, paged, direct, nwg, s);                     // prefill: rows re-read from L2
     }
     if (!direct && !fuse && !shm)

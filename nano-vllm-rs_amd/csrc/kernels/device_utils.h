@@ -141,6 +141,20 @@ __device__ __forceinline__ float row_sum(float x) {
     return x;
 }
 
+// sum over LPH consecutive lanes in the pairs of a LPH / 2, .., 2, 1 xor butterfly (row_sum<8> pairs lane i with 7 - i)
+template <int LPH>
+__device__ __forceinline__ float head_sum(float x) {
+    static_assert(LPH == 2 || LPH == 4 || LPH == 8 || LPH == 16, "lanes of a head");
+    if constexpr (LPH == 16) return row_sum<16>(x);
+    if constexpr (LPH >= 8) {                                                 // the lane 4 away inside 8: banks of 4 lanes 0 and 2 take the next bank's, 1 and 3 the one before
+        int y = __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x104, 0xF, 0x5, false);
+        y = __builtin_amdgcn_update_dpp(y, __float_as_int(x), 0x114, 0xF, 0xA, false);
+        x += __int_as_float(y);
+    }
+    if constexpr (LPH >= 4) x = dpp_add<0x4E>(x);
+    return dpp_add<0xB1>(x);
+}
+
 // lane-wise butterflies across the 16-lane rows of a wave on the gfx950 lane-swap instructions (no LDS traffic):
 // v_permlane16_swap exchanges the odd rows of one register with the even rows of another, v_permlane32_swap the
 // upper half of one with the lower half of the other; fed the same value twice, the two results are x and its

@@ -465,18 +465,6 @@ __global__ __launch_bounds__(256) void rope_store_kernel(half_t *__restrict__ qk
 // A workgroup has a thread for every piece up to 1024 (a second pass over the value rows was a second trip), a head's sum goes over its lanes on DPP in the pairs of a LPH / 2, .., 1 butterfly
 // (27 rows of 16 + 8 heads: 0.4 us of 4.6 a launch in a step)
 template <int LPH>
-__device__ __forceinline__ float head_sum(float x) {
-    static_assert(LPH == 2 || LPH == 4 || LPH == 8 || LPH == 16, "lanes of a head");
-    if constexpr (LPH == 16) return row_sum<16>(x);
-    if constexpr (LPH >= 8) {                                                 // the lane 4 away inside 8: banks of 4 lanes 0 and 2 take the next bank's, 1 and 3 the one before
-        int y = __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x104, 0xF, 0x5, false);
-        y = __builtin_amdgcn_update_dpp(y, __float_as_int(x), 0x114, 0xF, 0xA, false);
-        x += __int_as_float(y);
-    }
-    if constexpr (LPH >= 4) x = dpp_add<0x4E>(x);
-    return dpp_add<0xB1>(x);
-}
-template <int LPH>
 __global__ __launch_bounds__(1024) void qknorm_rope_store_kernel(half_t *__restrict__ qkv, const int64_t *__restrict__ pos,
                                                                 const int32_t *__restrict__ slots, int H, int KVH,
                                                                 const float *__restrict__ cos_t, const float *__restrict__ sin_t,

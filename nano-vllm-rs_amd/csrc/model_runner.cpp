@@ -873,7 +873,8 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
             if (owed) { RC(KD(norm_linear(before, w.qkv, T, Hd, QKV, qkv, st, qkv_t))); std::swap(hc, hn); }
             else RC(KD(linear(n, Hd, w.qkv, T, Hd, QKV, qkv, false, st, qkv_t)));                  // norm + RoPE + KV-store launch
             if (mc.use_bias) RC(KD(add_bias(qkv, w.qkv_b, T, QKV, st)));                            // A-30: the bias precedes the norms and RoPE (qwen3.rs:208-222)
-            RC(KD(rope_store_kv(qkv, pos, slots, T, H, KVH, D, cos_t, sin_t, k_cache(l), v_cache(l), st, w.q_norm, w.k_norm, mc.rms_norm_eps)));
+            if (is_prefill || !mc.qk_norm)                                                          // (a decode step's rows are normed, rotated and stored by its attention)
+                RC(KD(rope_store_kv(qkv, pos, slots, T, H, KVH, D, cos_t, sin_t, k_cache(l), v_cache(l), st, w.q_norm, w.k_norm, mc.rms_norm_eps)));
         } else if (owed) {
             RC(KD(norm_linear_qkv_rope_store(before, w.qkv, T, Hd, H, KVH, D, pos, slots, cos_t, sin_t, qkv, k_cache(l), v_cache(l), st, qkv_t)));
             std::swap(hc, hn);
@@ -905,6 +906,7 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
             a.block_size = (int32_t)block_size; a.workspace = attn_ws; a.workspace_bytes = attn_ws_bytes; a.tickets = attn_tickets;
             a.shared_len = (int32_t)decode_shared_len;
             a.ragged = decode_ragged;
+            if (mc.qk_norm) { a.qn_w = w.q_norm; a.kn_w = w.k_norm; a.qk_eps = mc.rms_norm_eps; a.pos = pos; a.slots = slots; a.cos_t = cos_t; a.sin_t = sin_t; }
             if (decode_shared_len > 0 && decode_shared_rows < T) {     // a group inside the batch: per-row kv0, member rows, member count
                 a.shared_kv0 = (const int32_t *)(in_dev + off_dec + dof_skv0); a.shared_rows = (const int32_t *)(in_dev + off_dec + dof_srows);
                 a.shared_count = (const int32_t *)(in_dev + off_dec + dof_scount);

@@ -686,3 +686,29 @@ def test_decode_steps_of_one_to_five_rows(hidden, qk_norm, dtype):
     sps = [dict(temperature=0.0, max_tokens=3 + 2 * i, ignore_eos=True) for i in range(5)]
     r = _run_pair(mcfg, ecfg, prompts, sps, dtype=dtype)
     assert r["decode_steps"] >= 10
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("heads,kv", [(2, 2), (4, 2), (4, 1)])
+def test_decode_attention_forms_norms_and_stores_its_own_rows(heads, kv, dtype):
+    """Models with q / k norms on heads of 128: a decode step whose attention norms, rotates and stores the step's rows itself (pages of 16 tokens; four and eight waves, one workgroup
+    per sequence and head, and several with a last one that merges) against the same step with that launch in front (pages of 20 tokens, no whole chunks): logits bit for bit, step by step, over contexts that end at, before and behind
+    a round of keys and a page, and as graph replays and eagerly."""
+    model = nvr.ModelConfig(vocab_size=512, hidden_size=256, intermediate_size=256, num_hidden_layers=2, num_attention_heads=heads, num_key_value_heads=kv, head_dim=128,
+                            max_position_embeddings=1024, tie_word_embeddings=1, seed=heads, qk_norm=1)
+    for lens in ([126, 30, 5, 8], [700], [255, 120, 640], [640, 7, 321, 64] * 5, [260] * (97 if heads == kv else 1)):
+        got = []
+        for page, eager in ((20, 1), (16, 1), (16, 0)):
+            eng = nvr.LLMEngine(nvr.Config(skip_block_size_check=1, max_num_seqs=len(lens), max_num_batched_tokens=2048, max_model_len=960, kvcache_block_size=page, num_kvcache_blocks=2000, dtype=dtype,
+                                           enforce_eager=eager), model)
+            for i, n in enumerate(lens):
+                eng.add_request(nvr.synthetic_tokens(n, 9, i, 512), nvr.SamplingParams(temperature=0.0, max_tokens=6, ignore_eos=True))
+            out = []
+            while not eng.is_finished():
+                rec = eng.step()
+                out.append((rec["tokens"], eng.model_runner.logits(rec["num_seqs"]).copy().view(np.uint32)))
+            got.append(out)
+        for other in got[1:]:
+            assert len(other) == len(got[0])
+            for (ta, la), (tb, lb) in zip(got[0], other):
+                assert ta == tb and np.array_equal(la, lb), lens
