@@ -551,8 +551,10 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float *__restrict
 // 64..4096 59.7 / 47.4 / 45.0, 40 of 32..2000 28.0 / 21.0 / 21.0, 33 of 4000 84.9 / 90.8 / 83.6-86.5 (6.3 TB/s), 48 of 4000 117.4 / 124.6 / 117.9, 65 of 4000 159 / 172 / 160, 74 of 1500
 // 74.2 / 79.8 / 75.5, 48 of 1500 50.2 / 50.4 / 48.9, 33 of 700 23.6 / 21.7 / 22.2.  Groups of 4, not AHEAD / AHEAD: 40 of 1500 keys 55.1 / 49.5, 33 of 4000 102.6 / 91.7, 27 of 64..8100
 // 44.5 / 39.8; heads of 64, 4 kv heads, 66 of 4000 keys: groups of 8 111.4 / 98.3, of 4 74.1 / 60.5, of 2 63.0 / 45.4.
-template <int D, int G, int U, int WAVES>
+// QKN (27 sequences of 64 .. 8100 keys: a step of Qwen3-0.6B 1950 -> 1922 us): as in attn_rows_kernel, the step's own rows come raw; a segment's query heads (and key row, where it holds the query's last key) are formed when it is opened, behind its first requests.
+template <int D, int G, int U, int WAVES, bool QKN = false>
 __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, int nq, int nw) {
+    static_assert(!QKN || (D == 128 && G < 4 * WAVES), "QKN: heads of 128");
     constexpr int LPR = D / 8, RPI = 64 / LPR, TPI = RPI * U, CH = TPI * WAVES;
     static_assert(G * D <= WAVES * 64 && G * (D / 4) <= WAVES * 64, "one pass over the (head, column) pairs");
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -595,6 +597,9 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
     const int32_t *bt = p.block_tables;
     half2_t qv[G][4];
     half8_t ka[U], va[U], kb[U], vb[U];                     // the wave's even / odd rounds: two are always requested ahead
+    __shared__ half8_t own_lds[2][QKN ? (G + 1) * 16 : 1];  // (two: a wave may open the second segment while another still reads the first one's; behind it the tails' barriers stand between)
+    half8_t own_k, own_v;
+    int own_j = -1, opened = 0;                             // own_j: the segment's last key where it is the step's own row and has a slot
     auto block_base = [&](int tb) -> int64_t {              // element offset of (scalar token tb, kv head g, d = 0)
         const int bi = tb >> p.bs_shift, bo = tb & (p.block_size - 1);
         if ((bi >> 6) != bt_chunk) {
@@ -636,15 +641,56 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
         R = max(pend - p0 - wave * TPI + CH - 1, 0) / CH;   // rounds in which this wave has a key
         bt = p.block_tables + (int64_t)t * p.max_blocks;
         bt_chunk = (p0 >> p.bs_shift) >> 6;
+        int64_t own_pos = 0; int own_slot = -1;
+        if constexpr (QKN) { own_pos = p.pos[t]; own_slot = p.slots ? p.slots[t] : -1; }
         { const int idx = (bt_chunk << 6) + lane; bt_reg = idx < p.max_blocks ? bt[idx] : 0; asm volatile("" : "+v"(bt_reg)); }
-        const half_t *qrow = p.q + (int64_t)t * p.ldq + (int64_t)g * G * D + dc * 8;
+        half8_t hx, hg; float4_t hc[2], hs[2];
+        if constexpr (QKN) {
+            const half_t *row = p.q + (int64_t)t * p.ldq;
+            if (wave * 4 <= G) {
+                const int hh = min(wave * 4 + tg, G);
+                const int64_t at = own_pos * (D / 2) + (dc & 7) * 8;
+                hx = *reinterpret_cast<const half8_t *>(row + (hh < G ? g * G + hh : p.H + g) * D + dc * 8);
+                hg = *reinterpret_cast<const half8_t *>((hh < G ? p.qn_w : p.kn_w) + dc * 8);
 #pragma unroll
-        for (int i = 0; i < G; ++i) {
-            const half8_t h = *reinterpret_cast<const half8_t *>(qrow + i * D);
+                for (int x = 0; x < 2; ++x) { hc[x] = *reinterpret_cast<const float4_t *>(p.cos_t + at + 4 * x); hs[x] = *reinterpret_cast<const float4_t *>(p.sin_t + at + 4 * x); }
+            }
+            own_v = *reinterpret_cast<const half8_t *>(row + (p.H + p.KVH + g) * D + dc * 8);
+        } else {
+            const half_t *qrow = p.q + (int64_t)t * p.ldq + (int64_t)g * G * D + dc * 8;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) qv[i][j] = (half2_t){h[2 * j], h[2 * j + 1]};
+            for (int i = 0; i < G; ++i) {
+                const half8_t h = *reinterpret_cast<const half8_t *>(qrow + i * D);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) qv[i][j] = (half2_t){h[2 * j], h[2 * j + 1]};
+            }
         }
         load_round(0, ka, va); load_round(1, kb, vb);
+        if constexpr (QKN) {
+            asm volatile("" ::: "memory");
+            half8_t *lds = own_lds[opened & 1];
+            if (wave * 4 <= G) {
+                const half8_t o = norm_rotate_piece(hx, hg, hc, hs, p.qk_eps, dc);
+                if (wave * 4 + tg <= G) lds[(wave * 4 + tg) * 16 + dc] = o;
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int i = 0; i < G; ++i) {
+                const half8_t h = lds[i * 16 + dc];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) qv[i][j] = (half2_t){h[2 * j], h[2 * j + 1]};
+            }
+            own_k = lds[G * 16 + dc];
+            own_j = own_slot >= 0 && pend == cx[t] ? pend - 1 : -1;
+            if (wave == WAVES - 1 && tg == 0 && own_j >= 0) {
+                const int64_t dst = ((int64_t)own_slot * p.KVH + g) * D + dc * 8;
+                *reinterpret_cast<half8_t *>(const_cast<half_t *>(p.k) + dst) = own_k;
+                *reinterpret_cast<half8_t *>(const_cast<half_t *>(p.v) + dst) = own_v;
+            }
+            ++opened;
+        }
         asm volatile("" ::: "memory");                      // the requests stay HERE: hipcc would sink them to their first use, behind the tail of the segment in front
         return true;
     };
@@ -658,8 +704,12 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
 #pragma unroll
             for (int j = 0; j < 8; ++j) acc[i][j] = 0.f;
         }
-        auto process = [&](const half8_t (&kk)[U], const half8_t (&vv)[U], int r) {
+        auto process = [&](half8_t (&kk)[U], half8_t (&vv)[U], int r) {
             const int left = pend - p0 - (r * WAVES + wave) * TPI;      // keys of the segment from the round's first one on
+            if (QKN && own_j >= 0 && left <= TPI)                       // the round that holds the step's own row (and, clamped to it, rows past the segment's end)
+#pragma unroll
+                for (int x = 0; x < U; ++x)
+                    if (x * RPI + tg >= left - 1) { kk[x] = own_k; vv[x] = own_v; }
             float sc[U][G];
 #pragma unroll
             for (int x = 0; x < U; ++x) {
@@ -846,6 +896,13 @@ static int own_rows(const AttnArgs &a, hipStream_t s) {                    // wh
     return rope_store_kv(const_cast<half_bits *>(a.q), a.pos, a.slots, a.nq, a.H, a.KVH, a.D, a.cos_t, a.sin_t, const_cast<half_bits *>(a.k), const_cast<half_bits *>(a.v), s, a.qn_w, a.kn_w, a.qk_eps);
 }
 
+static bool own_rows_aligned(const AttnArgs &a) {
+    return a.qn_w && a.ldq % 8 == 0 && (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.qn_w | (uintptr_t)a.kn_w | (uintptr_t)a.cos_t | (uintptr_t)a.sin_t) & 15) == 0;
+}
+static void own_rows_params(AttnParams &p, const AttnArgs &a) {
+    p.qn_w = (const half_t *)a.qn_w; p.kn_w = (const half_t *)a.kn_w; p.qk_eps = a.qk_eps; p.pos = a.pos; p.slots = a.slots; p.cos_t = a.cos_t; p.sin_t = a.sin_t;
+}
+
 template <int D, int G>
 static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
     AttnParams p{};
@@ -940,9 +997,18 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
             p.part_size = 64; p.num_parts = (int32_t)cap;
             p.part_o = (float *)a.workspace; p.part_ml = p.part_o + (int64_t)a.nq * a.H * cap * D;
             p.part0 = 0; p.kv0 = 0; p.kv0_rows = nullptr; p.tickets = a.tickets;
-            if (int rc = own_rows(a, s)) return rc;
             const int shares = (int)std::max<int64_t>(1, cus / a.KVH);                      // one workgroup per CU
-            attn_share_kernel<D, G, DU / 2, 8><<<dim3((unsigned)(shares * a.KVH)), dim3(512), 0, s>>>(p, (int)a.nq, shares);
+            bool in_it = false;
+            if constexpr (D == 128 && G <= 4)
+                if (own_rows_aligned(a)) {
+                    own_rows_params(p, a);
+                    attn_share_kernel<D, G, DU / 2, 8, true><<<dim3((unsigned)(shares * a.KVH)), dim3(512), 0, s>>>(p, (int)a.nq, shares);
+                    in_it = true;
+                }
+            if (!in_it) {
+                if (int rc = own_rows(a, s)) return rc;
+                attn_share_kernel<D, G, DU / 2, 8><<<dim3((unsigned)(shares * a.KVH)), dim3(512), 0, s>>>(p, (int)a.nq, shares);
+            }
             hipError_t e = hipGetLastError();
             if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "attention (work-balanced) launch failed: %s", hipGetErrorString(e));
             return 0;
@@ -969,9 +1035,8 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
     // pays for it again: Qwen3-0.6B with norms at 300 keys, us a step by a launch in front / here: 1 sequence 764 / 721, 2 833 / 784, 4 896 / 826, 8 975 / 912, 16 1062 / 998, 32 1159 / 1115,
     // 64 1674 / 1677, 128 2243 / 2249; 256 of 1024 keys 6069 / 6090)
     const int tpi = 64 / (D / 8) * (brief || waves == 4 ? DU : DU / 2);
-    const bool qkn = a.qn_w && D == 128 && G <= 4 && !shared && paged && pairs <= share_workgroups() && (waves == 8 || waves == 4) && (direct || fuse) && p.block_size % tpi == 0 && (p.num_parts == 1 || p.part_size % tpi == 0) && a.ldq % 8 == 0 &&
-                     (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.qn_w | (uintptr_t)a.kn_w | (uintptr_t)a.cos_t | (uintptr_t)a.sin_t) & 15) == 0;
-    if (qkn) { p.qn_w = (const half_t *)a.qn_w; p.kn_w = (const half_t *)a.kn_w; p.qk_eps = a.qk_eps; p.pos = a.pos; p.slots = a.slots; p.cos_t = a.cos_t; p.sin_t = a.sin_t; }
+    const bool qkn = D == 128 && G <= 4 && !shared && paged && pairs <= share_workgroups() && (waves == 8 || waves == 4) && (direct || fuse) && p.block_size % tpi == 0 && (p.num_parts == 1 || p.part_size % tpi == 0) && own_rows_aligned(a);
+    if (qkn) own_rows_params(p, a);
     else if (int rc = own_rows(a, s)) return rc;
     if (shared)
         if (int rc = flash_shared_prefix(a.q, a.ldq, a.k, a.v, a.block_tables, a.max_blocks, a.block_size, a.nq, a.H, a.KVH, a.D, a.scale,

@@ -712,3 +712,17 @@ def test_decode_attention_forms_norms_and_stores_its_own_rows(heads, kv, dtype):
             assert len(other) == len(got[0])
             for (ta, la), (tb, lb) in zip(got[0], other):
                 assert ta == tb and np.array_equal(la, lb), lens
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("heads", [8, 16])
+def test_work_balanced_decode_attention_forms_its_own_rows(heads, dtype):
+    """The work-balanced decode attention (34 sequences of 8 kv heads) where it norms, rotates and stores the step's rows itself: segments that hold a query's last key and segments that do not,
+    queries cut by shares — logits against the oracle step by step, at the engine's tolerance for the type."""
+    from oracle import model_oracle as mo
+    from test_engine_gpu import _run_pair
+    mcfg = mo.small(hidden_size=256, num_hidden_layers=1, intermediate_size=256, head_dim=128, num_attention_heads=heads, num_key_value_heads=8, qk_norm=True, seed=heads, init_std=0.02)
+    ecfg = dict(max_num_seqs=34, max_num_batched_tokens=8192, max_model_len=512, kvcache_block_size=16, num_kvcache_blocks=700)
+    prompts = [oracle.fill_tokens(250 + i if i % 3 else 12 + 7 * i, 3, i, mcfg.vocab_size).tolist() for i in range(34)]
+    r = _run_pair(mcfg, ecfg, prompts, [dict(temperature=0.0, max_tokens=4, ignore_eos=True)] * 34, dtype=dtype)
+    assert r["decode_steps"] >= 3
