@@ -755,7 +755,10 @@ __global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
             union { half_t v[8]; unsigned u[4]; } x;
             union { half8_t v; unsigned u[4]; } y;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) x.v[j] = (half_t)(o[dt][e + j] * inv);
+            for (int j = 0; j < 8; ++j) {                                  // (the quotient, corrected once: within half a unit of f32; an infinite one stays)
+                const float w = o[dt][e + j], d = w * inv, c = fmaf(fmaf(-d, l, w), inv, d);
+                x.v[j] = (half_t)(fabsf(d) < INFINITY ? c : d);
+            }
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const auto sw = __builtin_amdgcn_permlane32_swap(x.u[j], x.u[2 + j], false, false);
