@@ -646,11 +646,17 @@ __global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
 #pragma unroll
         for (int ks = 0; ks < 8; ++ks) { c = mfma32(read_k(0, ks), qf[ks], c); d = mfma32(read_k(1, ks), qf[ks], d); }
     };
-    auto mask = [&](int kt, float16_t &d) {                               // 32 keys from kt on
-        const int room = qpos - kt - 4 * h;
+    // 32 keys from kt on: key kt + i is hidden where i > qpos - kt, bit i - 4 h of a word of the lane's; two instructions a score, a bit spread over a word and a choice of bits by it (compares
+    // would each hold a pair of scalar registers or wait for vcc; 32 prompts of 1024 tokens and one of 509: the time of compares and selects).  The scores are read by the compiler's own instructions: it knows how long a matrix result takes.
+    auto mask = [&](int kt, float16_t &d) {
+        unsigned hidden = 0xffffffffu << min(max(qpos - kt - 4 * h + 1, 0), 31), minus_inf = 0xff800000u;
+        asm("" : "+v"(hidden), "+v"(minus_inf));                          // (opaque, as the words below: hipcc would turn all of it into compares and selects)
 #pragma unroll
-        for (int e = 0; e < 16; ++e)                                      // (written out: hipcc keeps the conditions in scalar registers, and other values leave those for memory)
-            asm("v_cmp_gt_i32 vcc, %1, %2\n\tv_cndmask_b32 %0, %0, %3, vcc" : "+v"(d[e]) : "n"((e >> 2) * 8 + (e & 3)), "v"(room), "v"(-INFINITY) : "vcc");
+        for (int e = 0; e < 16; ++e) {
+            unsigned w = (unsigned)__builtin_amdgcn_sbfe((int)hidden, (e >> 2) * 8 + (e & 3), 1);
+            asm("" : "+v"(w));
+            d[e] = __uint_as_float((w & minus_inf) | (~w & __float_as_uint(d[e])));
+        }
     };
     auto maximum = [&](const float16_t &c, const float16_t &d) {
         float a = fmaxf(c[0], c[1]), b = fmaxf(d[0], d[1]);
