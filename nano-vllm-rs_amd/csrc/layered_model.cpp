@@ -308,7 +308,7 @@ int LayeredModel::execute(nvr_model_runner &r, nvr_seq *const *seqs, size_t nseq
     NVR_HIP_CHECK(hipSetDevice(r.device));
     if (nseq == 0) return fail(NVR_ERR_INVALID_ARG, "execute_model: empty batch");
     if ((int64_t)nseq > r.max_seqs) return fail(NVR_ERR_INVALID_ARG, "execute_model: %zu sequences exceed max_num_seqs %ld", nseq, (long)r.max_seqs);
-    int64_t T = 0, max_ctx = 0, max_rows = 0;
+    int64_t T = 0, max_ctx = 0, max_rows = 0, min_rows = INT32_MAX;
     for (size_t i = 0; i < nseq; ++i) {
         const nvr_seq *s = seqs[i];
         if (s->chunk_len == 0 || s->chunk_start + s->chunk_len > s->num_tokens)
@@ -318,7 +318,7 @@ int LayeredModel::execute(nvr_model_runner &r, nvr_seq *const *seqs, size_t nseq
         if (end > r.max_pos) return fail(NVR_ERR_INVALID_ARG, "execute_model: sequence %lu reaches position %ld (max_model_len %ld)", (unsigned long)s->seq_id, (long)end, (long)r.max_pos);
         if ((int64_t)s->block_table.size() * r.block_size < end) return fail(NVR_ERR_NOT_ALLOCATED, "execute_model: sequence %lu has blocks for %zu tokens, needs %ld", (unsigned long)s->seq_id, s->block_table.size() * (size_t)r.block_size, (long)end);
         for (size_t j = 0; j < nseq; ++j) if (j != i && seqs[j]->state_slot == s->state_slot) return fail(NVR_ERR_INVARIANT, "execute_model: two sequences of the batch share state slot %d", s->state_slot);
-        T += (int64_t)s->chunk_len; max_ctx = std::max(max_ctx, end); max_rows = std::max<int64_t>(max_rows, (int64_t)s->chunk_len);
+        T += (int64_t)s->chunk_len; max_ctx = std::max(max_ctx, end); max_rows = std::max<int64_t>(max_rows, (int64_t)s->chunk_len); min_rows = std::min<int64_t>(min_rows, (int64_t)s->chunk_len);
     }
     if (T > r.max_tokens) return fail(NVR_ERR_INVALID_ARG, "execute_model: %ld tokens exceed max_num_batched_tokens %ld", (long)T, (long)r.max_tokens);
     const size_t R = want ? nwant : nseq;
@@ -393,7 +393,7 @@ int LayeredModel::execute(nvr_model_runner &r, nvr_seq *const *seqs, size_t nseq
     b.ids = (const int64_t *)(in_dev + o_ids); b.row_seq = (const int32_t *)(in_dev + o_rs); b.cu = (const int32_t *)(in_dev + o_cu);
     b.start = (const int32_t *)(in_dev + o_st); b.slot = (const int32_t *)(in_dev + o_sl); b.par = (const int32_t *)(in_dev + o_par);
     b.block_tables = (const int32_t *)(in_dev + o_bt); b.max_blocks = (int32_t)MB; b.block_size = (int32_t)r.block_size;
-    b.T = (int32_t)T; b.B = (int32_t)nseq; b.max_ctx = (int32_t)max_ctx; b.max_rows = (int32_t)max_rows;
+    b.T = (int32_t)T; b.B = (int32_t)nseq; b.max_ctx = (int32_t)max_ctx; b.max_rows = (int32_t)max_rows; b.min_rows = (int32_t)min_rows;
     const int32_t *d_want = (const int32_t *)(in_dev + o_want);
 
     bool decode_sized = true;

@@ -624,6 +624,30 @@ def test_retention_prompts_in_chunks_of_16_tokens(dim, vdim, lens):
         _compare_layer_rows(cfg, w, "bfloat16", [toks[i][:at[i]]], [np.concatenate(rows[i])[-4:]])
 
 
+@pytest.mark.parametrize("dim,vdim", [(64, 128), (128, 64)])
+@pytest.mark.parametrize("n", [1, 7, 15])
+def test_retention_of_a_short_portion_does_not_depend_on_its_neighbours(dim, vdim, n):
+    """A sequence of less than a chunk of rows, in a step of the same size beside one long portion and beside several short ones, first and behind other tokens: the bits of its logits, and of
+    those of the single token behind it (its state)."""
+    import rugudra_util as u
+    cfg = u.make_config([u.retention_layer(3, dim, vdim, decay=[0.3, 0.95, 0.9995], ff=None)], width=128, taps=3)
+    w = u.make_weights(cfg, seed=n)
+    d = u.Driver(cfg, w, dtype="bfloat16", slots=8, pages=48, max_tokens=256, max_len=256)
+    rng = np.random.default_rng(n)
+    toks, other = rng.integers(0, 97, 2 * n + 2), rng.integers(0, 97, 45)
+    got = []
+    for parts in ((45,), (15, 15, 15), (30, 15)):
+        rows = []
+        for a, b in ((0, n), (n, 2 * n)):
+            rows.append(d.step([("s", toks[a:b])] + [("o%d" % i, other[:k]) for i, k in enumerate(parts)])["s"])
+            for i in range(len(parts)):
+                d.end("o%d" % i)
+        rows += [d.step([("s", toks[k:k + 1])])["s"] for k in (2 * n, 2 * n + 1)]
+        d.end("s")
+        got.append(np.concatenate(rows).view(np.uint32))
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
 @pytest.mark.parametrize("taps", [2, 3, 4, 5])
 @pytest.mark.parametrize("dim,width", [(64, 132), (128, 1028)])
 def test_layer_list_single_tokens_across_pages(taps, dim, width):
