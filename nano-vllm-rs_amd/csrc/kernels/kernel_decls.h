@@ -54,6 +54,7 @@ int argmax_partials(const float *part_val, const int32_t *part_idx, int32_t npar
 int tp_argmax_merge(const TpArgmaxRec *recs, int tp, int64_t B, int64_t *out_host, int64_t *out_dev, const unsigned int *err, int64_t *err_out,
                     hipStream_t s);
 
+bool stream_preferred(int64_t T, int64_t N);   // linear() streams the weights of such a product: few rows, or few outputs (linear.hip)
 int64_t stream_row_limit();    // rows up to which the weight-streaming kernels are preferred over the LDS-tiled GEMM (linear.hip)
 bool splitk_prefers_tiles(int64_t T, int64_t K, int64_t N);   // linear_splitk takes the LDS-tiled kernel (gemm_tiled_splitk) for this shape
 int linear_splitk(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, int64_t S,

@@ -398,7 +398,7 @@ int decode_splitk_slices(int64_t T, int64_t K, int64_t N) {
     while (S < 4 && tiles * S < 256 && K % (32 * S * 2) == 0 && K / (S * 2) >= 128) S *= 2;
     return (int)S;
 }
-static inline bool prefer_stream(int64_t T, int64_t N) {
+bool stream_preferred(int64_t T, int64_t N) {
     // up to 64 rows the weight-streaming kernel; beyond, the LDS-tiled kernel with 32- / 64-token tiles and the 4-buffer ring (r02,
     // ctx 256: bs 66 2.20 -> 1.83 ms/step, bs 96 2.48 -> 2.15, bs 128 2.82 -> 2.23).
     return T <= stream_row_limit() || T * N <= 192 * 1024;       // (qkv of 0.6B, 80 rows 9.1 / 7.9, 96 rows 10.0 / 7.9)
@@ -427,7 +427,7 @@ static int linear_routed(const half_bits *x, int64_t ldx, const half_bits *W, in
         }
     }
     if (gelu) *gelu = false;                               // (the tiled and the streaming kernel have no such epilogue)
-    if (!y_f32 && gemm_tiled_ok(T, K, N, ldx) && !prefer_stream(T, N)) return gemm_tiled(x, ldx, W, T, K, N, (half_bits *)y, s, Wt);
+    if (!y_f32 && gemm_tiled_ok(T, K, N, ldx) && !stream_preferred(T, N)) return gemm_tiled(x, ldx, W, T, K, N, (half_bits *)y, s, Wt);
     if (!y_f32 && linear_stream_ok(T, K, N, ldx)) return linear_stream(x, ldx, W, T, K, N, (half_bits *)y, s, Wt);   // large weights
     const half_t *xx = (const half_t *)x, *ww = (const half_t *)(Wt ? Wt : W);
     const int t = (int)T, k = (int)K, n = (int)N;
@@ -474,7 +474,7 @@ int linear_gelu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, 
     return linear_routed(x, ldx, W, T, K, N, y, false, s, nullptr, applied);
 }
 
-bool linear_resid_ok(int64_t T, int64_t K, int64_t N, int64_t ldx) { return gemm_tiled_ok(T, K, N, ldx) && !prefer_stream(T, N) && N % 8 == 0; }
+bool linear_resid_ok(int64_t T, int64_t K, int64_t N, int64_t ldx) { return gemm_tiled_ok(T, K, N, ldx) && !stream_preferred(T, N) && N % 8 == 0; }
 int linear_resid(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *h, hipStream_t s, const half_bits *Wt) {
     if (!linear_resid_ok(T, K, N, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "linear_resid: T=%ld K=%ld N=%ld", (long)T, (long)K, (long)N);
     const int64_t r = gemm256_ok(T, K, N, ldx) ? rows_on_256(T, K, N) : 0;
@@ -518,7 +518,7 @@ static int linear_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64
         return r == T ? 0 : gemm_tiled_silu_mul(x + r * ldx, ldx, W, T - r, K, I, out + r * I, s, gelu, Wt);
     }
     // (56 rows and more of weights that the large-weight kernel does not take: the two blocks of 32 rows each read x for every 16 columns; 64 rows, K = 1024, I = 3072 9.1 / 8.2, 48 rows 8.2 / 8.2)
-    if (gemm_tiled_ok(T, K, I, ldx) && I % 64 == 0 && (!prefer_stream(T, 2 * I) || (T >= 56 && T * I > 128 * 1024 && !linear_stream_silu_ok(T, K, I, ldx)))) return gemm_tiled_silu_mul(x, ldx, W, T, K, I, out, s, gelu, Wt);
+    if (gemm_tiled_ok(T, K, I, ldx) && I % 64 == 0 && (!stream_preferred(T, 2 * I) || (T >= 56 && T * I > 128 * 1024 && !linear_stream_silu_ok(T, K, I, ldx)))) return gemm_tiled_silu_mul(x, ldx, W, T, K, I, out, s, gelu, Wt);
     if (linear_stream_silu_ok(T, K, I, ldx)) return linear_stream_silu_mul(x, ldx, W, T, K, I, out, s, Wt, gelu);              // large weights
     const half_t *xx = (const half_t *)x, *ww = (const half_t *)(Wt ? Wt : W);
     LinEpi e{};
@@ -583,7 +583,7 @@ int linear_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, i
         if (int rc = gemm256_qkv_rope_store(x, ldx, W, r, K, H, KVH, D, positions, slots, cos_t, sin_t, qkv, k_cache, v_cache, s, kv_cache_only)) return rc;
         return r == T ? 0 : gemm_tiled_qkv_rope_store(x + r * ldx, ldx, W, T - r, K, H, KVH, D, positions + r, slots ? slots + r : nullptr, cos_t, sin_t, qkv + r * (H + 2 * KVH) * D, k_cache, v_cache, s, Wt, kv_cache_only);
     }
-    if (gemm_tiled_ok(T, K, (H + 2 * KVH) * D, ldx) && 128 % D == 0 && !prefer_stream(T, (H + 2 * KVH) * D))
+    if (gemm_tiled_ok(T, K, (H + 2 * KVH) * D, ldx) && 128 % D == 0 && !stream_preferred(T, (H + 2 * KVH) * D))
         return gemm_tiled_qkv_rope_store(x, ldx, W, T, K, H, KVH, D, positions, slots, cos_t, sin_t, qkv, k_cache, v_cache, s, Wt, kv_cache_only);
     if (linear_stream_rope_ok(T, K, H, KVH, D, ldx))                                                                  // large weights
         return linear_stream_qkv_rope_store(x, ldx, W, T, K, H, KVH, D, positions, slots, cos_t, sin_t, qkv, k_cache, v_cache, s, Wt);

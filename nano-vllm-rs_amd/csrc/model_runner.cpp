@@ -620,9 +620,9 @@ int nvr_model_runner::row_parallel_norm(const uint16_t *x, int64_t K, const uint
         S = 4;                                       // large weights: 64-column workgroups x 4 k-slices (linear_splitk)
     } else if (!comm.active() && tp == 1 && T > KD(stream_row_limit()) && T <= slab_rows && Hd <= 8192 && ((Hd + 127) / 128) * ((T + 127) / 128) <= 64 &&
                KD(gemm_tiled_splitk_ok(T, K, Hd, 4, K))) {
-        S = 4;                                       // 97..1024 rows, few 128x128 tiles: k-split of the tiled kernel (gemm_tiled_splitk;
-                                                     // bs = 256 / 512 decode 4.04 -> 3.67 / 6.18 -> 5.33 ms in r01; with the 32- / 64-token
-                                                     // tiles of r02 it also wins from 97 rows on: same boundary as prefer_stream, linear.hip)
+        S = 4;                                       // 65..1024 rows, few 128x128 tiles: k-split of the tiled kernel (gemm_tiled_splitk;
+                                                     // bs = 256 / 512 decode 4.04 -> 3.67 / 6.18 -> 5.33 ms; with the 32- / 64-token tiles from
+                                                     // the streaming kernels' last row on)
     }
     if (S > 1) {
         RC(KD(linear_splitk(x, K, W, T, K, Hd, S, slabs, stream, Wt)));
@@ -636,7 +636,7 @@ int nvr_model_runner::row_parallel_norm(const uint16_t *x, int64_t K, const uint
     }
     // (the step's GEMM kernel by linear.hip's routing: 256-row tiles when its cost rule prefers them, else the 128-row kernel; the chunks call THAT kernel)
     const bool big = KD(gemm256_preferred(T, K, Hd, K));
-    if (comm.active() && comm_stream && tp_overlap && ((big && T >= 1024) || (!big && T >= 512 && T * Hd > 384 * 1024 && KD(gemm_tiled_ok(T, K, Hd, K))))) {   // (T * N <= 384 Ki: linear() streams the weights instead)
+    if (comm.active() && comm_stream && tp_overlap && ((big && T >= 1024) || (!big && T >= 512 && !KD(stream_preferred(T, Hd)) && KD(gemm_tiled_ok(T, K, Hd, K))))) {   // (where linear() does not stream the weights instead)
         // Prefill on tensor-parallel ranks (row g): the rows are cut into chunks (multiples of the 256-row GEMM tile, so every tile and every
         // row is computed exactly as in one piece: bit-identical), and the all-reduce of chunk i runs on the communication stream while the
         // compute stream works on the GEMM of chunk i+1; the residual add + RMSNorm of a chunk follows its reduce.  Host order

@@ -656,6 +656,46 @@ def test_tensor_parallel_prefill_exchange_overlaps_on_a_second_stream(tp, p2p, h
 
 
 @pytest.mark.gpu
+def test_prefill_exchange_overlaps_wherever_the_products_run_on_tiles():
+    """Steps of few outputs a row (rows x hidden between 192 Ki and 384 Ki) take the LDS tiles like larger ones, and their exchange is cut into chunks like theirs; the serial form's bits."""
+    import threading
+    sys.path.insert(0, ROOT)
+    import nvr_import
+    nvr = nvr_import.load()
+    mc = nvr.ModelConfig(vocab_size=256, hidden_size=256, intermediate_size=512, num_hidden_layers=2, num_attention_heads=8, num_key_value_heads=4, head_dim=64, max_position_embeddings=1024,
+                         tie_word_embeddings=1, seed=9)
+    prompts = [nvr.synthetic_tokens(n, 5, i, 256) for i, n in enumerate((700, 300))]
+
+    def run(overlap):
+        group, engines, out, errors = nvr.LocalGroup(2, p2p=True), [], [None, None], []
+        for r in range(2):
+            e = nvr.LLMEngine(nvr.Config(skip_block_size_check=1, tensor_parallel_size=2, tensor_parallel_rank=r, enforce_eager=1, max_num_seqs=2, max_num_batched_tokens=1024, max_model_len=768,
+                                         kvcache_block_size=64, num_kvcache_blocks=32), mc)
+            group.attach(e.model_runner)
+            e.model_runner.set_tp_prefill_overlap(overlap)
+            nvr.lib().nvr_seq_reset_id_counter()
+            for p in prompts:
+                e.add_request(p, nvr.SamplingParams(temperature=0.0, max_tokens=1, ignore_eos=True))
+            engines.append(e)
+
+        def drive(r):
+            try:
+                rec = engines[r].step()
+                out[r] = (rec["is_prefill"], rec["num_tokens"], engines[r].model_runner.last_overlap_chunks(), engines[r].model_runner.logits(2).copy())
+            except BaseException as ex:                                                 # noqa: BLE001
+                errors.append((r, ex))
+        threads = [threading.Thread(target=drive, args=(r,)) for r in range(2)]
+        for t in threads: t.start()
+        for t in threads: t.join(120)
+        assert not errors, errors
+        return out
+    a, b = run(1), run(0)
+    for x, y in zip(a, b):
+        assert x[:3] == (True, 1000, 3) and y[:3] == (True, 1000, 0), (x[:3], y[:3])
+        assert np.array_equal(x[3].view(np.uint32), y[3].view(np.uint32)), "overlapped and serial prefill exchange differ in bits"
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("async_on", [0, 1])
 def test_peer_that_never_arrives_fails_the_step_and_the_group_recovers(async_on):
     """Negative path of the one-shot collectives (kernels/comm_p2p.hip): rank 1 never enters a decode step that rank 0 runs.  Rank 0's
