@@ -664,7 +664,8 @@ int gemm_tiled_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *
     if (!gemm_tiled_ok(T, K, N, ldx) || D % 16 || 128 % D) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_qkv_rope_store: T=%ld K=%ld D=%ld", (long)T, (long)K, (long)D);
     TileEpi e{};
     e.pos = positions; e.slots = slots; e.cos_t = cos_t; e.sin_t = sin_t; e.kc = (half_t *)k_cache; e.vc = (half_t *)v_cache;
-    e.H = (int32_t)H; e.KVH = (int32_t)KVH; e.D = (int32_t)D; e.kv_cache_only = kv_cache_only;
+    e.H = (int32_t)H; e.KVH = (int32_t)KVH; e.D = (int32_t)D;
+    e.kv_cache_only = kv_cache_only && slots && k_cache && v_cache;
     if (int rc = gemm_tiled_prepare()) return rc;
     tiled_launch<TEPI_ROPE>((N / 16 + 7) / 8, 1, x, ldx, W, Wt, T, K, N, N, (half_t *)qkv, e, s);
     return tiled_check("gemm_tiled_qkv_rope_store");
