@@ -1132,9 +1132,28 @@ __global__ __launch_bounds__(256, 2) void retention_chunk_kernel(RetentionArgs a
             oc = __builtin_amdgcn_mfma_f32_16x16x4f32(pp[r], vf[r], oc, 0, 0, 0);
             od = __builtin_amdgcn_mfma_f32_16x16x4f32(pp[r + 1], vf[r + 1], od, 0, 0, 0);
         }
+        oc = oc + od;
+        // a later token's weight is a zero, which makes NaN of a value that is not finite: such columns are summed up to each token's own (a wave's columns of a chunk, seldom)
+        float z = (vf[0] * 0.f + vf[1] * 0.f) + (vf[2] * 0.f + vf[3] * 0.f);
+        if (__any(z != 0.f)) {
+            z += __shfl_xor(z, 16, 64); z += __shfl_xor(z, 32, 64);
+            f32x4 os = {0.f, 0.f, 0.f, 0.f};
+            for (int jg = 0; jg < 4; ++jg)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float v = __shfl(vf[r], jg * 16 + m, 64);
+#pragma unroll
+                    for (int y = 0; y < 4; ++y) {
+                        const float p = __shfl(pp[r], jg * 16 + 4 * g + y, 64);
+                        if (4 * jg + r <= 4 * g + y) os[y] = fmaf(p, v, os[y]);
+                    }
+                }
+#pragma unroll
+            for (int y = 0; y < 4; ++y) oc[y] = z != 0.f ? os[y] : oc[y];
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            if (4 * g + r < nb) a.o[(int64_t)(r0 + i0 + 4 * g + r) * a.H * Dv + (int64_t)h * Dv + cb + w * 16 + m] = fmaf(o[0][r], wo[r], oc[r] + od[r]);
+            if (4 * g + r < nb) a.o[(int64_t)(r0 + i0 + 4 * g + r) * a.H * Dv + (int64_t)h * Dv + cb + w * 16 + m] = fmaf(o[0][r], wo[r], oc[r]);
     }
 #pragma unroll
     for (int t = 0; t < ND; ++t)

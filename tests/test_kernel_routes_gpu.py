@@ -621,7 +621,7 @@ def test_retention_prompts_in_chunks_of_16_tokens(dim, vdim, lens):
             at[i] += n
             rows[i].append(out["s%d" % i])
     for i in range(3):
-        _compare_layer_rows(cfg, w, "bfloat16", [toks[i][:at[i]]], [np.concatenate(rows[i])[-4:]])
+        _compare_layer_rows(cfg, w, "bfloat16", [toks[i][:at[i]]], [np.concatenate(rows[i])])
 
 
 @pytest.mark.parametrize("dim,vdim", [(64, 128), (128, 64)])
@@ -646,6 +646,25 @@ def test_retention_of_a_short_portion_does_not_depend_on_its_neighbours(dim, vdi
         d.end("s")
         got.append(np.concatenate(rows).view(np.uint32))
     assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (128, 128)])
+@pytest.mark.parametrize("at", [1, 9, 15, 16, 30])
+def test_retention_values_that_are_not_finite_reach_no_earlier_token(dim, vdim, at):
+    """A token whose values overflow, inside a chunk and at its ends: every row in front of it has the bits that it has with an ordinary token in that place, every row from it on holds what the
+    recurrence has there too, no number."""
+    import rugudra_util as u
+    cfg = u.make_config([u.retention_layer(2, dim, vdim, decay=[0.9, 0.999], ff=None)], width=128, taps=3)
+    w = u.make_weights(cfg, seed=at)
+    w["embed"][:, 5], w["l0.canon1"][5], w["l0.mix.v"][:, 5] = 0.0, 0.0, 0.0
+    w["embed"][96, 5], w["l0.mix.v"][3, 5] = 8.0, 3e38                                # token 96 alone has a channel that takes one value column beyond the largest number
+    d = u.Driver(cfg, w, dtype="bfloat16", slots=1, pages=8, max_tokens=64, max_len=64)
+    toks = np.random.default_rng(at).integers(0, 96, 37)
+    want = d.run_alone(toks)
+    toks[at] = 96
+    got = d.run_alone(toks)
+    assert np.all(np.isfinite(want)) and np.array_equal(got[:at].view(np.uint32), want[:at].view(np.uint32))
+    assert not np.any(np.isfinite(got[at:]).all(axis=1))
 
 
 @pytest.mark.parametrize("taps", [2, 3, 4, 5])
