@@ -1314,6 +1314,8 @@ int norm_canon(const float *x, const Batch &b, int64_t W, float eps, int taps, f
                bool bf16, float *hist, int64_t slots, hipStream_t s) {
     if (b.T == 0) return 0;
     if (taps < 1) return nvr::fail(NVR_ERR_INVALID_ARG, "norm_canon: taps %d (at least 1)", taps);
+    // steps of one row per sequence: a workgroup per row, however many (it reads the convolution weights again for every row, from L2).  us, a few rows a workgroup / so, 4 taps: 1 / 16 / 64 / 256
+    // rows of 128 5.5 6.3 10.4 12.3 / 3.4 4.0 4.8 4.0, of 1024 7.0 8.1 13.9 14.9 / 3.5 3.7 4.0 5.2, of 2048 10.6 11.9 25.4 26.0 / 4.6 4.8 5.2 6.1, of 4096 19.4 21.0 45.7 46.9 / 5.6 6.1 6.6 8.5
     if (join_norm_canon_ok(b, W, taps, x, nullptr, hist)) return join_norm_canon(const_cast<float *>(x), nullptr, 0, 0.f, b, W, eps, taps, g1, w1, out1, g2, w2, out2, bf16, hist, slots, s);
     if (W % 4 == 0 && taps <= 8 && ((uintptr_t)x | (uintptr_t)hist) % 16 == 0) {
         // rows per workgroup: many for prompts (the convolution weights of a column are read once per workgroup), few for decode-sized steps (more workgroups)

@@ -388,7 +388,7 @@ int64_t stream_row_limit() { return 64; }
 // streaming split-k kernel walks the weights once per 32-row block (Qwen3-8B bs 64: o + down 92 us per layer against 46 us at bs 128 on the tiles;
 // up to 32 rows the streaming kernel stays ahead: Qwen3-8B bs 32 / 16 5.00 / 4.20 ms per step against 5.10 / 4.38 on 32-token tiles, 8 slices)
 bool splitk_prefers_tiles(int64_t T, int64_t K, int64_t N) { return T > stream_row_limit() || (T > 32 && N * K * 2 >= (24ll << 20)); }
-// ... and with 8 slices whatever the weights: 64 rows, N = 1024, K = 2048 / 3072 5.0 / 6.3 us as two blocks and 2 slices, 4.3 / 5.0 on the tiles
+// ... and with 8 slices whatever the weights: 64 rows, N = 1024, K = 2048 / 3072 5.3 / 6.6 us as two blocks and 2 slices, 4.4 / 5.5 on the tiles
 constexpr int64_t TILE_SLICES = 8;
 // k-slices of the N = hidden GEMMs of a decode-sized step (linear_splitk): reach ~256 workgroups with slices of >= 256 columns that are
 // multiples of 64
@@ -399,9 +399,11 @@ int decode_splitk_slices(int64_t T, int64_t K, int64_t N) {
     return (int)S;
 }
 bool stream_preferred(int64_t T, int64_t N) {
-    // up to 64 rows the weight-streaming kernel; beyond, the LDS-tiled kernel with 32- / 64-token tiles and the 4-buffer ring (r02,
-    // ctx 256: bs 66 2.20 -> 1.83 ms/step, bs 96 2.48 -> 2.15, bs 128 2.82 -> 2.23).
-    return T <= stream_row_limit() || T * N <= 192 * 1024;       // (qkv of 0.6B, 80 rows 9.1 / 7.9, 96 rows 10.0 / 7.9)
+    // up to 64 rows the weight-streaming kernel; beyond, the LDS-tiled kernel with 32- / 64-token tiles (ctx 256: bs 66 2.20 -> 1.83 ms/step, bs 96 2.48 -> 2.15, bs 128 2.82 -> 2.23) from
+    // 192 Ki outputs on.  us, streamed / tiles, widths of 256 to 4096 columns: K = 1024 7.0 / 7.0 at 200-240 Ki outputs, 9.3 / 7.0 at 290-380 Ki (80 rows of 4096 columns 9.1 / 7.9, 96 rows
+    // 10.0 / 7.9), K = 2048 12.2 / 11.2 and 17.2 / 11.3, K = 4096 21.7 / 20.5 and 31.5 / 21; K = 512 4.2-4.8 / 4.9 and 5.9 / 4.9: there the line could lie at 260 Ki, but one line keeps prompts of
+    // like sizes on one kernel.
+    return T <= stream_row_limit() || T * N <= 192 * 1024;
 }
 static inline int waves_for(int64_t K) { return K >= 2048 ? 16 : (K >= 1024 ? 8 : 4); }
 
@@ -517,8 +519,10 @@ static int linear_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64
         if (int rc = gelu ? gemm256_gelu_mul(x, ldx, W, r, K, I, out, s) : gemm256_silu_mul(x, ldx, W, r, K, I, out, s)) return rc;
         return r == T ? 0 : gemm_tiled_silu_mul(x + r * ldx, ldx, W, T - r, K, I, out + r * I, s, gelu, Wt);
     }
-    // (56 rows and more of weights that the large-weight kernel does not take: the two blocks of 32 rows each read x for every 16 columns; 64 rows, K = 1024, I = 3072 9.1 / 8.2, 48 rows 8.2 / 8.2)
-    if (gemm_tiled_ok(T, K, I, ldx) && I % 64 == 0 && (!stream_preferred(T, 2 * I) || (T >= 56 && T * I > 128 * 1024 && !linear_stream_silu_ok(T, K, I, ldx)))) return gemm_tiled_silu_mul(x, ldx, W, T, K, I, out, s, gelu, Wt);
+    // (56 rows and more of weights that the large-weight kernel does not take: the two blocks of 32 rows each read x for every 16 columns.  us of 56 / 64 rows, blocks | tiles: K = 512, I = 2304
+    // 5.2 5.4 | 5.3 5.9, 3840 6.1 6.3 | 6.2 6.3, 4864 7.6 7.8 | 6.4 6.4; K = 768, I = 2304 7.0 7.4 | 7.0 7.4, 3840 8.1 8.5 | 7.5 7.6; K = 1024, I = 2304 8.3 8.7 | 8.3 8.4, 3072 8.9 9.3 | 8.3 8.4,
+    // 4864 11.9 12.5 | 9.0 9.2; K = 2560, I = 3072 20.4 21.3 | 17.1 17.5, 4864 29.5 31.1 | 19.7 19.9)
+    if (gemm_tiled_ok(T, K, I, ldx) && I % 64 == 0 && (!stream_preferred(T, 2 * I) || (T >= 56 && T * I > (K >= 768 ? 128 : 256) * 1024 && !linear_stream_silu_ok(T, K, I, ldx)))) return gemm_tiled_silu_mul(x, ldx, W, T, K, I, out, s, gelu, Wt);
     if (linear_stream_silu_ok(T, K, I, ldx)) return linear_stream_silu_mul(x, ldx, W, T, K, I, out, s, Wt, gelu);              // large weights
     const half_t *xx = (const half_t *)x, *ww = (const half_t *)(Wt ? Wt : W);
     LinEpi e{};

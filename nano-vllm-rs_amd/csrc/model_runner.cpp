@@ -610,7 +610,11 @@ int nvr_model_runner::row_parallel_norm(const uint16_t *x, int64_t K, const uint
     }
     int64_t S = 1;
     if (!comm.active() && tp == 1 && T <= 64 && T <= KD(stream_row_limit()) && Hd <= 2048) {
-        S = T > 32 && 8 * T <= 4 * slab_rows && KD(gemm_tiled_splitk_ok(T, K, Hd, 8, K)) ? 8 : KD(decode_splitk_slices(T, K, Hd));
+        // 33..64 rows: eight slices on the tiles where a slice has three K-tiles and the row enough columns.  us of product + norm of 33 / 48 / 64 rows, as blocks of 32 rows with up to four slices |
+        // so: N = 512, K = 2048 5.8 5.8 5.9 | 6.3 6.6 6.5, K = 6144 8.4 8.5 8.7 | 9.1 9.6 9.6; N = 768, K = 1024 5.8 5.8 6.0 | 5.9 6.0 6.2, K = 1536 6.4 6.6 6.6 | 6.1 6.4 6.5; N = 1024,
+        // K = 1024 5.7 5.7 6.0 | 6.0 6.0 6.5, 1536 6.4 6.7 6.9 | 6.3 6.5 6.7, 2048 7.2 7.1 7.4 | 6.7 6.8 7.2, 3072 8.2 8.4 8.7 | 7.7 7.9 8.1; N = 1536, K = 1536 8.5 8.7 8.7 | 7.2 7.7 8.0;
+        // N = 2048, K = 1024 6.9 6.9 7.1 | 7.1 7.5 8.1, 1536 8.3 8.2 8.4 | 7.9 8.2 8.5, 2048 9.7 9.5 9.5 | 8.2 8.8 9.3, 6144 20.7 19.4 19.1 | 10.7 11.4 11.8
+        S = T > 32 && Hd >= 768 && K >= 1536 && 8 * T <= 4 * slab_rows && KD(gemm_tiled_splitk_ok(T, K, Hd, 8, K)) ? 8 : KD(decode_splitk_slices(T, K, Hd));
     } else if (!comm.active() && tp == 1 && T > 32 && T <= 64 && Hd <= 8192 && KD(splitk_prefers_tiles(T, K, Hd)) && 8 * T <= 4 * slab_rows &&
                KD(gemm_tiled_splitk_ok(T, K, Hd, 4, K))) {
         // 33..64 rows over large weights (Qwen3-8B bs 64): one 64-token tile per 128 weight rows, k split until ~256 workgroups stream the
