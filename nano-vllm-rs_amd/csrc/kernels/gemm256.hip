@@ -76,8 +76,8 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__
                                                       int tiles_x, int tiles_y, int CG) {
     extern __shared__ __attribute__((aligned(16))) char smem[];           // 2 x G_BUF
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    int r = lane & 15, q = lane >> 4;
-    int wn = wave >> 2, wm = wave & 3;
+    const int r = lane & 15, q = lane >> 4;
+    const int wn = wave >> 2, wm = wave & 3;
     const int grp = __builtin_amdgcn_readfirstlane(wave >> 2);
 
     // Persistent workgroup.  The K-tile stream runs ACROSS its tiles: K-tile g of the stream lives in buffer g & 1, and the
@@ -113,8 +113,8 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__
     // Address = tile base (scalar) + uniform row term of (half, i) (scalar) + ONE thread constant per operand: two 64-bit registers
     // instead of eight pointers that had to be rebuilt, with the RoPE row map's divisions, inside the last K-tile of every tile
     // (r03: that rebuild spilled ~80 registers to scratch in the RoPE variant — global-memory round trips in the K loop).
-    int r0 = tid >> 3, cch = ((tid & 7) ^ (r0 & 7)) * 8;                  // row inside a 64-row group, swizzled 16-byte chunk (elements)
-    int64_t a_thr = (int64_t)g_w_thr<EPI, RD>(r0) * K + cch, b_thr = (int64_t)r0 * ldx + cch;
+    const int r0 = tid >> 3, cch = ((tid & 7) ^ (r0 & 7)) * 8;            // row inside a 64-row group, swizzled 16-byte chunk (elements)
+    const int64_t a_thr = (int64_t)g_w_thr<EPI, RD>(r0) * K + cch, b_thr = (int64_t)r0 * ldx + cch;
     const half_t *wb = W, *xb = x;                                         // of the tile being STAGED (the next one during a tile's last K-tile)
     int rows_left = 0x3fffffff;                                            // T - 1 - m0 when the tile's row block is ragged
     int wrows_left = 0x3fffffff;                                           // LM head: N - 1 - bx * 256 when the tile's vocabulary block is ragged
