@@ -524,7 +524,7 @@ def test_prompt_attention_of_heads_of_128(G, KVH, bs, ctx, growth):
     NB = sum(-(-c // bs) for c in ctx)
     order, tables, at = rng.permutation(NB), [], 0
     k, v = np.zeros((NB * bs, KVH, D), F16), _bits(rng, (NB * bs, KVH, D), 1.0)
-    q, want = [], []
+    q, want, spread, square = [], [], [], []
     for c in ctx:
         t = order[at:at + -(-c // bs)]
         at += len(t)
@@ -540,13 +540,26 @@ def test_prompt_attention_of_heads_of_128(G, KVH, bs, ctx, growth):
         tables.append(t.astype(np.int32))
         q.append(qs)
         kk, vv, qq = (np.repeat(a[rows].astype(np.float64), G, 1) if a is not None else qs.astype(np.float64) for a in (k, v, None))
-        s = np.einsum("ihd,jhd->hij", qq, kk) * D ** -0.5
+        s = np.matmul(qq.transpose(1, 0, 2), kk.transpose(1, 2, 0)) * D ** -0.5
         s[:, np.arange(c)[None, :] > np.arange(c)[:, None]] = -np.inf
         p = np.exp(s - s.max(2, keepdims=True))
-        want.append(np.einsum("hij,jhd->ihd", p / p.sum(2, keepdims=True), vv))
+        p /= p.sum(2, keepdims=True)
+        w = np.matmul(p, vv.transpose(1, 0, 2)).transpose(1, 0, 2)
+        want.append(w)
+        sums = [np.matmul(a, b.transpose(1, 0, 2)) for a, b in ((p, vv * vv), (p * p, vv * vv), (p * p, vv))]
+        wh = w.transpose(1, 0, 2)
+        spread.append(np.sqrt(np.maximum(sums[0] - wh * wh, 0)).transpose(1, 0, 2))   # at least the sum of weight x |value - result| (weights add up to 1)
+        square.append(np.maximum(sums[1] - 2 * wh * sums[2] + wh * wh * np.sum(p * p, 2, keepdims=True), 0).transpose(1, 0, 2))      # the sum of (weight x (value - result))^2
     whole = _prefill(np.concatenate(q), ctx, ctx, k, v, tables, H, KVH, D, bs)
-    # a weight is rounded to 11 bits before it meets its value, and so is the result: 2^-11 of the sum of |weight x value| (at most the largest |value|, about 4.5) each, and the sums' 24 bits
-    assert np.max(np.abs(whole - np.concatenate(want))) <= 2 * 4.5 * 2.0 ** -11
+    # the result is rounded to 11 bits, and so is every weight before it meets its value and joins the row's sum: at most 2^-11 of |result| and of the sum of weight x |value - result|, and a
+    # twentieth for the 24 bits of scores and sums
+    w, spread, square, got = (np.concatenate(a).astype(np.float64).reshape(-1, D) for a in (want, spread, square, [whole]))
+    assert np.all(np.abs(got - w) <= 1.05 * 2.0 ** -11 * (np.abs(w) + spread) + 2.0 ** -25)
+    # a row's sum that is off moves the whole row by a factor.  Roundings are as often up as down: a deviation of at most 2^-11 / sqrt(3) each, those of the weights one for all columns of a row;
+    # the factor of all rows together within five deviations (and the 24 bits of a sum)
+    moved = np.sum((got - w) * w) / np.sum(w * w)
+    deviation = 2.0 ** -11 / np.sqrt(3) * np.sqrt(np.sum(np.sum(np.abs(w) * np.sqrt(square), 1) ** 2) + np.sum(w ** 4)) / np.sum(w * w)
+    assert abs(moved) <= 5 * deviation + 2.0 ** -20, (moved, deviation)
     at = 0
     for i, c in enumerate(ctx):
         for n in {1, min(c, 17), min(c, 70), c}:                                      # its last n tokens alone
