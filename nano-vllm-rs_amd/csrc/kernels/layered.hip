@@ -1,6 +1,7 @@
 // layered.hip — kernels of layer-list models (kernels/layered.h): f32 residual stream, scalar-gain RMS norm + causal convolution in front
 // of each sublayer, attention with distance penalty and sink, retention with f32 state, clamped gated feed-forward.  wave64, gfx950.
 #include <hip/hip_runtime.h>
+#include <type_traits>
 #include <math.h>
 #include <algorithm>
 #include "../common.h"
@@ -1003,12 +1004,6 @@ __global__ __launch_bounds__(256, 2) void retention_chunk_kernel(RetentionArgs a
     if (tid == 0) { double p = 1.0; const double dd = a.decay[h]; for (int i = 0; i < 17; ++i) { pw[i] = (float)p; pl[i] = (float)(p - (double)pw[i]); p *= dd; } }
     float *S = a.state + (((int64_t)b.slot[sq] * a.H + h) * D) * Dv + cb + w * 16 + m;
     f32x4 sa[ND];
-#pragma unroll
-    for (int t = 0; t < ND; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sa[t][r] = st > 0 ? S[(int64_t)(16 * t + 4 * g + r) * Dv] : 0.f;
-#pragma unroll
-    for (int t = 0; t < ND; ++t) asm volatile("" : "+v"(sa[t]));                   // (waited for here, not in the loop)
     // staged: 4 coordinates of the lower half and their partners of one token's q and k, 4 value columns of a token
     const int ti = tid / PT & 15, d0 = (tid % PT) * 4, vi = tid >> 4, vc = (tid & 15) * 4;
     const bool rot = D == 128 || tid < 16 * PT;
@@ -1048,6 +1043,16 @@ __global__ __launch_bounds__(256, 2) void retention_chunk_kernel(RetentionArgs a
 #pragma unroll
         for (int y = 0; y < 4; ++y) vt[(vc + y) * KS + vi] = ld_f(ve, y);
     };
+    // CAREFUL: a wave looks whether one of its 16 columns of a chunk holds a value that is not finite.  A later token's weight is a zero, which makes NaN of such a value for the tokens in front of
+    // it: those columns are summed up to each token's own.  (In the plain walk the check and its branch cost 6 us of 263: the state tells at the end, below.)
+    auto walk = [&](auto careful_c) {
+    constexpr bool CAREFUL = decltype(careful_c)::value;
+#pragma unroll
+    for (int t = 0; t < ND; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sa[t][r] = st > 0 ? S[(int64_t)(16 * t + 4 * g + r) * Dv] : 0.f;
+#pragma unroll
+    for (int t = 0; t < ND; ++t) asm volatile("" : "+v"(sa[t]));                   // (waited for here, not in the loop)
     request(0);
     put(rsm, 0);
     request(16);
@@ -1133,28 +1138,39 @@ __global__ __launch_bounds__(256, 2) void retention_chunk_kernel(RetentionArgs a
             od = __builtin_amdgcn_mfma_f32_16x16x4f32(pp[r + 1], vf[r + 1], od, 0, 0, 0);
         }
         oc = oc + od;
-        // a later token's weight is a zero, which makes NaN of a value that is not finite: such columns are summed up to each token's own (a wave's columns of a chunk, seldom)
-        float z = (vf[0] * 0.f + vf[1] * 0.f) + (vf[2] * 0.f + vf[3] * 0.f);
-        if (__any(z != 0.f)) {
-            z += __shfl_xor(z, 16, 64); z += __shfl_xor(z, 32, 64);
-            f32x4 os = {0.f, 0.f, 0.f, 0.f};
-            for (int jg = 0; jg < 4; ++jg)
+        if constexpr (CAREFUL) {
+            float z = (vf[0] * 0.f + vf[1] * 0.f) + (vf[2] * 0.f + vf[3] * 0.f);   // not 0: one of the four is not finite
+            if (__any(z != 0.f)) {
+                z += __shfl_xor(z, 16, 64); z += __shfl_xor(z, 32, 64);
+                f32x4 os = {0.f, 0.f, 0.f, 0.f};
+                for (int jg = 0; jg < 4; ++jg)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float v = __shfl(vf[r], jg * 16 + m, 64);
+                    for (int r = 0; r < 4; ++r) {
+                        const float v = __shfl(vf[r], jg * 16 + m, 64);
 #pragma unroll
-                    for (int y = 0; y < 4; ++y) {
-                        const float p = __shfl(pp[r], jg * 16 + 4 * g + y, 64);
-                        if (4 * jg + r <= 4 * g + y) os[y] = fmaf(p, v, os[y]);
+                        for (int y = 0; y < 4; ++y) {
+                            const float p = __shfl(pp[r], jg * 16 + 4 * g + y, 64);
+                            if (4 * jg + r <= 4 * g + y) os[y] = fmaf(p, v, os[y]);
+                        }
                     }
-                }
 #pragma unroll
-            for (int y = 0; y < 4; ++y) oc[y] = z != 0.f ? os[y] : oc[y];
+                for (int y = 0; y < 4; ++y) oc[y] = z != 0.f ? os[y] : oc[y];
+            }
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r)
             if (4 * g + r < nb) a.o[(int64_t)(r0 + i0 + 4 * g + r) * a.H * Dv + (int64_t)h * Dv + cb + w * 16 + m] = fmaf(o[0][r], wo[r], oc[r]);
     }
+    };
+    walk(std::false_type{});
+    // a value that is not finite leaves a state that is not (a product with a zero is a NaN, and no decay takes either away): the sequence is walked again from the state in memory, every output
+    // written again
+    float z = 0.f;
+#pragma unroll
+    for (int t = 0; t < ND; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z = fmaf(sa[t][r], 0.f, z);
+    if (__syncthreads_or(z != 0.f)) walk(std::true_type{});
 #pragma unroll
     for (int t = 0; t < ND; ++t)
 #pragma unroll
