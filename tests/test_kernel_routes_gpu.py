@@ -450,6 +450,31 @@ def test_tile_products_of_few_k_tiles_and_ragged_edges(T, K, N):
         assert np.all(np.abs(s.astype(np.float64).sum(0) - ref) <= bound)
 
 
+@pytest.mark.parametrize("T,K,N", [(33, 1536, 768), (48, 2048, 1040), (64, 512, 784), (64, 3072, 2048)])
+def test_products_of_33_to_64_rows_in_eight_slices(T, K, N):
+    """The o / down products of such steps on the tiles, eight slices of one to six K-tiles: the slabs' sum against 64 bits, the tiled copy's bits, and the residual add + norm over eight slabs."""
+    rng, l, S = np.random.default_rng(T + K), nvr.lib(), 8
+    x, W, h, w = _bits(rng, (T, K), 0.5), _bits(rng, (N, K), 0.1), _bits(rng, (T, N), 1.0), _bits(rng, (N,), 0.1) + F16(1)
+    d_x, d_W = dev(x), dev(W)
+    d_T, sa, sb = _copy_of(d_W, N, K), nvr.DeviceBuffer(S * T * N * 4), nvr.DeviceBuffer(S * T * N * 4)
+    nvr.check(l.nvr_linear_splitk(d_x.ptr, K, d_W.ptr, T, K, N, S, sa.ptr, None))
+    nvr.check(l.nvr_linear_splitk_tiled(d_x.ptr, K, d_W.ptr, d_T.ptr, T, K, N, S, sb.ptr, None))
+    s = sa.to_numpy((S, T, N), np.float32)
+    assert np.array_equal(s, sb.to_numpy((S, T, N), np.float32))
+    ref, bound = _product_bound(x, W)
+    assert np.all(np.abs(s.astype(np.float64).sum(0) - ref) <= bound)
+    d_h, d_w, d_o = dev(h), dev(w), nvr.DeviceBuffer(T * N * 2)
+    nvr.check(l.nvr_add_rmsnorm_slabs(d_h.ptr, sa.ptr, S, d_w.ptr, 1e-6, T, N, d_o.ptr, None))
+    total = s[0]
+    for z in range(1, S):
+        total = total + s[z]
+    want = (h.astype(np.float32) + total.astype(F16).astype(np.float32)).astype(F16)
+    assert np.array_equal(d_h.to_numpy((T, N), np.uint16), want.view(np.uint16))
+    v = want.astype(np.float64)
+    norm = (v / np.sqrt((v * v).mean(1, keepdims=True) + 1e-6)) * w.astype(np.float64)
+    assert np.all(np.abs(d_o.to_numpy((T, N), F16) - norm) <= np.abs(norm) * 1.01 * 2.0 ** -11 + 2.0 ** -25)
+
+
 @pytest.mark.parametrize("T,K,I", [(97, 128, 3072), (200, 64, 4160), (509, 1024, 3072), (384, 192, 3072), (700, 320, 2112)])
 def test_tile_gate_up_forms(T, K, I):
     """gate_up + SiLU on the tiles (128-row and 96-row ones): the tiled copy's bits, and every element within two roundings of the unit of the rounded products."""
