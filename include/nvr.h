@@ -565,11 +565,12 @@ NVR_API int nvr_linear_qkv_rope_store_tiled(const nvr_half *x, int64_t ldx, cons
                                             nvr_half *qkv, nvr_half *k_cache, nvr_half *v_cache, void *stream);
 NVR_API int nvr_lm_head_tiled(const nvr_half *x, int64_t ldx, const nvr_half *W, const nvr_half *Wt, int64_t T, int64_t K, int64_t N,
                               float *logits, float *part_val, int32_t *part_idx, int32_t *nparts, void *stream);
-/* k-slices S of nvr_linear_splitk for the N = hidden GEMMs of a decode-sized step (o_proj, down_proj): enough to reach ~256 workgroups */
+/* k-slices S of nvr_linear_splitk for the N = hidden GEMMs of a decode-sized step (o_proj, down_proj): enough to reach ~256 workgroups
+ * (the runner's steps of 33..64 rows over long k take eight, on the tiles) */
 NVR_API int nvr_decode_splitk_slices(int64_t T, int64_t K, int64_t N);
 /* h[T,N] <- fp16(h + fp16(x · Wᵀ)) with the residual add (qwen3.rs:382,389) in the epilogue of the
- * 256x256 MFMA GEMM; only for shapes that kernel takes (T >= 256, N % 256 == 0, K % 64 == 0 and preferred by the routing of nvr_linear:
- * NVR_ERR_UNSUPPORTED otherwise).  Bit-identical to nvr_linear into a scratch tensor followed by the add of nvr_add_rmsnorm. */
+ * 256x256 MFMA GEMM, all rows on it; only for shapes that kernel takes (T >= 256, N % 256 == 0, K % 64 == 0) and whose tiles fill most of
+ * the chip (NVR_ERR_UNSUPPORTED otherwise; which they are does not move with the routing of nvr_linear).  Bit-identical to nvr_linear into a scratch tensor followed by the add of nvr_add_rmsnorm. */
 NVR_API int nvr_linear_add_residual(const nvr_half *x, int64_t ldx, const nvr_half *W, int64_t T, int64_t K, int64_t N, nvr_half *h,
                                     void *stream);
 /* K12+K13 fused: out[T,I] = SiluAndMul(x · W_gate_upᵀ), W [2I,K] gate rows then up rows

@@ -517,9 +517,9 @@ __global__ __launch_bounds__(64 * FLASH_WAVES, 8 / FLASH_WAVES) void flash_prefi
 // (K runs one step ahead of V through the LDS ring).  The accumulators are rescaled at a step's start, behind the barrier, where the products on them have long ended, and only if a query of the
 // wave met a larger score.  Raising the maximum only past a margin (2^8 in the exponentials' unit) takes another 7 % off, but the largest weight is then no longer the 1 that has no rounding:
 // the attention's error against 64 bits grew by 2.5 %.
-// bfloat16, G = 2, us before (16 x 16 x 32 products, one after the other) / now: 32 prompts of 1024 tokens 201 / 184 a layer, one of 509 16.2 / 15.1, of 2048 49.0 / 45.5, of 8192 334 / 325; 100
-// steps of one workgroup per CU 143 / 134, of two 212 / 212: cycles fall, and with the matrix cores' load the clock, from 2.1 to 1.75 GHz.  Of 202 us of two per CU without rescaling: without the K
-// reads 171, the V reads 188, the exponentials 185, the LDS-DMA 183, products and the rest of the vector work alone 127.
+// bfloat16, G = 2, us before (16 x 16 x 32 products, one after the other) / now, launches alone: 32 prompts of 1024 tokens 201 / 184 a layer (in a step of float16 218 / 197), one of 509 16.2 /
+// 15.1, of 2048 49.0 / 45.5, of 8192 334 / 325; 100 steps of one workgroup per CU 143 / 134, of two 212 / 212: cycles fall, and with the matrix cores' load the clock, from 2.1 to 1.75 GHz.  Of 202
+// us of two per CU without rescaling: without the K reads 171, the V reads 188, the exponentials 185, the LDS-DMA 183, products and the rest of the vector work alone 127.
 // N products, each followed by READS LDS reads (those of the product AHEAD products later) and VALU vector instructions
 template <int N, int READS, int AHEAD, int VALU>
 __device__ __forceinline__ void sched_pattern() {

@@ -986,7 +986,7 @@ __global__ __launch_bounds__(256) void retention_block_kernel(RetentionArgs a, B
 // in LDS, and the one after is requested, before this one's last barrier: one barrier per chunk.  Powers of the decay: products in f64, rounded once, that of the
 // state's own as two f32 numbers.  A chunk's k v^T is summed before it joins the state, whose error against 64 bits is thereby
 // below the token-by-token sum's (1024 tokens of a unit normal: output 1.7e-7 of its size against 4.6e-7, state 1.6e-7 against 5.5e-7; 16 tokens 1.16e-7 against 1.24e-7).
-// 16 x 1024 tokens, 16 heads of 128 x 128: 266 us against 686 of the recurrence (150 us of matrix instructions; the rest is LDS, rotation and the waits of a chunk at two waves a SIMD);
+// 16 x 1024 tokens, 16 heads of 128 x 128: 268 us against 686 of the recurrence (150 us of matrix instructions; the rest is LDS, rotation and the waits of a chunk at two waves a SIMD);
 // one prompt of 1024: 163 against 352; 2 x 16 tokens, 64 heads of 128 x 64: 6.9 against 11.0.  Not a bit-for-bit cut: where a prompt's portions end moves the chunks' limits.  A sequence of
 // fewer rows than a chunk keeps the recurrence whatever else is in the step (RetentionArgs::below), so that its bits do not depend on its neighbours.
 constexpr int RET_CHUNK = 16;

@@ -704,7 +704,7 @@ kl::SinkAttnArgs LayeredModel::diff_args(const LayerW &w, const LayeredSpec::Lay
     return a;
 }
 
-// One position per sequence: up to four workgroups per compute unit share the keys.
+// One position per sequence: up to two workgroups per compute unit share the keys.
 int LayeredModel::decode_attention(nvr_model_runner &r, const kl::SinkAttnArgs &a, const StepPlan &p) {
     // shares of the keys: at most two workgroups on a compute unit, all resident at once.  More shares leave some units with three of them and most with two, and merge more partial rows (16
     // sequences of 1040 keys, 8 key/value heads: 4 shares 20.0 us, 5 26.3; of 2048 keys: 4 32.9, 8 40.6; 64 of 1040: 1 56.9, 2 64.7; 8 of 8192, 4 heads: 16 37, 32 47)
