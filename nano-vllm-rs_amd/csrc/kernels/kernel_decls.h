@@ -141,6 +141,7 @@ bool gemm256_lm_head_ok(int64_t T, int64_t K, int64_t N, int64_t ldx);
 int gemm256_lm_head(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, float *logits, float *part_val,
                     int32_t *part_idx, int32_t *nparts, hipStream_t s);
 bool gemm256_preferred(int64_t T, int64_t K, int64_t N, int64_t ldx);     // the 256x256 kernel is the faster one of the two for the whole shape
+bool gemm256_epilogue_preferred(int64_t T, int64_t K, int64_t N, int64_t ldx);   // ... for a product whose epilogue is a launch of its own on other tiles
 bool linear_add_residual_ok(int64_t T, int64_t K, int64_t N, int64_t ldx);   // the shapes nvr_linear_add_residual takes
 // h <- h + x.W^T (the product rounded first) of a prompt-sized step on the tiles that the shape takes
 bool linear_resid_ok(int64_t T, int64_t K, int64_t N, int64_t ldx);

@@ -377,12 +377,17 @@ static int64_t rows_on_256(int64_t T, int64_t K, int64_t N) {
     }
     return best;
 }
-// the shapes for which the 256x256 kernel was estimated the faster one when nvr_linear_add_residual was added: what it takes does not move with the tiles' speed
-bool linear_add_residual_ok(int64_t T, int64_t K, int64_t N, int64_t ldx) {
+// where the 256x256 kernel was estimated the faster one before both kernels' times were fitted anew: what nvr_linear_add_residual takes does not move with them
+static bool former_256(int64_t T, int64_t K, int64_t N) {
     const int64_t t256 = ((N + 255) / 256) * ((T + 255) / 256), t128 = ((N + 127) / 128) * ((T + 127) / 128);
     const double kk = (double)K / 1024.0, c128 = (t128 <= 256 ? 15.0 * kk : (double)((t128 + 511) / 512) * 21.0 * kk) + 5.0;
-    return gemm256_ok(T, K, N, ldx) && (double)((t256 + 255) / 256) * (17.0 * kk + 20.0) < c128;
+    return (double)((t256 + 255) / 256) * (17.0 * kk + 20.0) < c128;
 }
+bool linear_add_residual_ok(int64_t T, int64_t K, int64_t N, int64_t ldx) { return gemm256_ok(T, K, N, ldx) && former_256(T, K, N); }
+// a product with an epilogue that the 256x256 kernel alone has (GELU, max(y, 0)^2): elsewhere it is a launch of its own that reads and writes the rows again, so the line lies where either estimate
+// prefers the kernel.  us a layer with GELU, tiles and a launch of its own / so: 2064 rows of 4096 columns, K = 1024 145 / 140, 2304 rows 146 / 141; 8192 columns, K = 2048 2064 rows 294 / 299 (the
+// unrounded product's GELU all the same), 2560 rows 322 / 310
+bool gemm256_epilogue_preferred(int64_t T, int64_t K, int64_t N, int64_t ldx) { return gemm256_ok(T, K, N, ldx) && (prefer_256(T, K, N) || former_256(T, K, N)); }
 int64_t stream_row_limit() { return 64; }
 // split-k GEMMs of the N = hidden projections: LDS tiles beyond the streaming kernels' rows — and from 33 rows on over large weights, where the
 // streaming split-k kernel walks the weights once per 32-row block (Qwen3-8B bs 64: o + down 92 us per layer against 46 us at bs 128 on the tiles;
@@ -413,6 +418,9 @@ static int launch_check(const char *what) {
     return 0;
 }
 
+// outputs up to which a product with GELU stays on the streaming kernel: on tiles the product is rounded before GELU, by a launch of its own.  us a layer, tiles and that launch / so: 200 / 300 /
+// 384 rows of 1024 columns, K = 256 49.0 50.6 50.8 / 44.4 46.4 49.1, 100 / 192 rows of 2048, K = 512 53.9 55.5 / 49.9 53.2, 72 / 96 rows of 4096, K = 1024 68.5 69.5 / 67.0 68.9
+constexpr int64_t GELU_STREAM = 384 * 1024;
 // gelu (not null): in, whether y = gelu(x . W^T) is wanted; out, whether the kernel this shape takes has applied it
 static int linear_routed(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, void *y, bool y_f32, hipStream_t s, const half_bits *Wt, bool *gelu) {
     const bool act = gelu && *gelu;
@@ -422,14 +430,14 @@ static int linear_routed(const half_bits *x, int64_t ldx, const half_bits *W, in
     if (T == 0) return 0;
     // prompts: rows_on_256; up to 64 rows and for small T * N the weight-streaming kernel over blocks of 32 rows
     if (!y_f32 && gemm256_ok(T, K, N, ldx)) {
-        if (act) { if (prefer_256(T, K, N)) return gemm256_gelu(x, ldx, W, T, K, N, (half_bits *)y, s); }
+        if (act) { if (gemm256_epilogue_preferred(T, K, N, ldx)) return gemm256_gelu(x, ldx, W, T, K, N, (half_bits *)y, s); }
         else if (const int64_t r = rows_on_256(T, K, N)) {
             if (int rc = gemm256(x, ldx, W, r, K, N, (half_bits *)y, s)) return rc;
             return r == T ? 0 : gemm_tiled(x + r * ldx, ldx, W, T - r, K, N, (half_bits *)y + r * N, s, Wt);
         }
     }
     if (gelu) *gelu = false;                               // (the tiled and the streaming kernel have no such epilogue)
-    if (!y_f32 && gemm_tiled_ok(T, K, N, ldx) && !stream_preferred(T, N)) return gemm_tiled(x, ldx, W, T, K, N, (half_bits *)y, s, Wt);
+    if (!y_f32 && gemm_tiled_ok(T, K, N, ldx) && !stream_preferred(T, N) && !(act && T * N <= GELU_STREAM)) return gemm_tiled(x, ldx, W, T, K, N, (half_bits *)y, s, Wt);
     if (!y_f32 && linear_stream_ok(T, K, N, ldx)) return linear_stream(x, ldx, W, T, K, N, (half_bits *)y, s, Wt);   // large weights
     const half_t *xx = (const half_t *)x, *ww = (const half_t *)(Wt ? Wt : W);
     const int t = (int)T, k = (int)K, n = (int)N;

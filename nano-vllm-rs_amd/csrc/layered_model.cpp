@@ -1248,7 +1248,7 @@ int LayeredModel::forward_scaled(nvr_model_runner &r, const StepPlan &p) {
         }
         RC(kl::residual_join(j, bf16, s));
         if (L.has_mlp) {
-            if (bf16 && nvr::kb::gemm256_preferred(T, W, L.ff, W)) RC(nvr::kb::gemm256_relu2((const uint16_t *)a2, W, (const uint16_t *)w.up, T, W, L.ff, (uint16_t *)act, s));   // (the squared ReLU in the product's epilogue)
+            if (bf16 && nvr::kb::gemm256_epilogue_preferred(T, W, L.ff, W)) RC(nvr::kb::gemm256_relu2((const uint16_t *)a2, W, (const uint16_t *)w.up, T, W, L.ff, (uint16_t *)act, s));   // (the squared ReLU in the product's epilogue)
             else {
                 RC(gemm(r, a2, W, w.up, T, W, L.ff, gu));
                 RC(kl::relu_squared(gu, L.ff, T, L.ff, act, L.ff, bf16, s));

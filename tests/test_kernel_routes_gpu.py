@@ -662,6 +662,22 @@ def test_retention_prompts_in_chunks_of_16_tokens(dim, vdim, lens):
         _compare_layer_rows(cfg, w, "bfloat16", [toks[i][:at[i]]], [np.concatenate(rows[i])])
 
 
+@pytest.mark.parametrize("rows,width,ff", [(190, 256, 1024), (94, 512, 2048)])
+def test_products_with_gelu_in_their_epilogue_beside_a_few_more_rows(rows, width, ff):
+    """GELU of the unrounded product, in its epilogue, up to 384 Ki outputs: a prompt on either side of 192 Ki, where products without it change to the tiles (which would round before a GELU of
+    its own), has the same bits alone and beside a prompt of ten tokens."""
+    import kiduvik_util as k
+    import rugudra_util as u
+    cfg = k.make_config([k.diff(heads=4, kv_heads=2, dim=32, vdim=64, rot=16, mlp=k.dense(ff)) for _ in range(2)], width=width, vocab=96, side=0)
+    d = u.Driver(cfg, k.make_weights(cfg, seed=rows), dtype="bfloat16", page=64, pages=8, slots=2, max_tokens=256, max_len=256)
+    toks = np.random.default_rng(rows).integers(0, 96, rows + 10)
+    assert rows * ff <= 192 * 1024 < (rows + 10) * ff
+    alone = d.step([("a", toks[:rows])])["a"]
+    d.end("a")
+    beside = d.step([("a", toks[:rows]), ("b", toks[rows:])])["a"]
+    assert np.array_equal(alone.view(np.uint32), beside.view(np.uint32))
+
+
 @pytest.mark.parametrize("dim,vdim", [(64, 128), (128, 64)])
 @pytest.mark.parametrize("n", [1, 7, 15])
 def test_retention_of_a_short_portion_does_not_depend_on_its_neighbours(dim, vdim, n):
