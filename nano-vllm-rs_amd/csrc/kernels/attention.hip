@@ -40,8 +40,11 @@ struct AttnParams {
     float *part_o; float *part_ml;     // [nq, H, num_parts, D], [nq, H, num_parts, 2]
     half_t *out;                       // [nq, H, D]
     unsigned int *tickets;             // FUSE: one arrival counter per (query, kv head), zero between launches (the last arriver re-arms it)
-    const half_t *qn_w, *kn_w; float qk_eps; const int64_t *pos; const int32_t *slots; const float *cos_t, *sin_t;   // QKN (AttnArgs)
 };
+struct OwnRows { const half_t *qn_w, *kn_w; float qk_eps; const int64_t *pos; const int32_t *slots; const float *cos_t, *sin_t; };   // QKN (AttnArgs)
+struct AttnParamsOwn : AttnParams, OwnRows {};         // (a type of its own: the arguments of the other instances stay as short as they were)
+template <bool QKN> struct AttnParamsOf { using type = AttnParams; };
+template <> struct AttnParamsOf<true> { using type = AttnParamsOwn; };
 
 // One 8-element piece of a head of 128 held by 16 lanes (dc = lane % 16, elements dc * 8 ..): RMSNorm over the head and rotation as qknorm_rope_store_kernel does them — its sums' pairs, its
 // roundings, nothing contracted: the same bits.  g: the norm's weights of the piece, c / s: cosines and sines of pairs (dc % 8) * 8 ..
@@ -162,7 +165,8 @@ __device__ __forceinline__ half4_t merge_partitions(int np, LoadML load_ml, Load
 // (4.6 us a layer at a few rows, as much as this whole kernel over short contexts): the first waves form the G query heads and the key row, 16 lanes a head, while every wave's first keys are on
 // their way; all read them back from LDS.  The row of the last key is taken from there, not from the cache; the workgroup whose keys end with it stores it.
 template <int D, int G, bool PAGED, bool DIRECT_OUT, int U, int WAVES, bool NT, bool UB, bool FUSE = false, bool SHM = false, bool QKN = false>
-__global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(AttnParams p) {
+__global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnParamsOf<QKN>::type own) {
+    const AttnParams &p = own;                          // (a type that does not depend on the instance: hipcc drops the host stub otherwise)
     static_assert(!QKN || (D == 128 && PAGED && UB && !SHM && G < 4 * WAVES), "QKN: paged heads of 128");
     constexpr int LPR = D / 8;          // lanes per K/V row
     constexpr int RPI = 64 / LPR;       // rows per wave-instruction (= tokens per row group)
@@ -212,18 +216,20 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(AttnParams p) {
     }
     // QKN: head item wave * 4 + tg (G query heads, then the key head) of the step's row, and the value row's piece
     const half_t *own_row = QKN ? p.q + (int64_t)t * p.ldq : nullptr;
-    const int hi = wave * 4 + tg, own_slot = QKN && p.slots ? p.slots[t] : -1;
+    const int hi = wave * 4 + tg;
+    int own_slot = -1;
     const bool forms = QKN && wave * 4 <= G;                              // (uniform)
     half8_t hx, hg, own_k, own_v; float4_t hc[2], hs[2];
     __shared__ half8_t own_lds[QKN ? (G + 1) * 16 : 1];
     if constexpr (QKN) {
-        const int64_t at = p.pos[t] * (D / 2) + (dc & 7) * 8;
+        if (own.slots) own_slot = own.slots[t];
+        const int64_t at = own.pos[t] * (D / 2) + (dc & 7) * 8;
         if (forms) {
             const int hh = min(hi, G);
             hx = *reinterpret_cast<const half8_t *>(own_row + (hh < G ? g * G + hh : p.H + g) * D + dc * 8);
-            hg = *reinterpret_cast<const half8_t *>((hh < G ? p.qn_w : p.kn_w) + dc * 8);
+            hg = *reinterpret_cast<const half8_t *>((hh < G ? own.qn_w : own.kn_w) + dc * 8);
 #pragma unroll
-            for (int x = 0; x < 2; ++x) { hc[x] = *reinterpret_cast<const float4_t *>(p.cos_t + at + 4 * x); hs[x] = *reinterpret_cast<const float4_t *>(p.sin_t + at + 4 * x); }
+            for (int x = 0; x < 2; ++x) { hc[x] = *reinterpret_cast<const float4_t *>(own.cos_t + at + 4 * x); hs[x] = *reinterpret_cast<const float4_t *>(own.sin_t + at + 4 * x); }
         }
         own_v = *reinterpret_cast<const half8_t *>(own_row + (p.H + p.KVH + g) * D + dc * 8);
     }
@@ -338,29 +344,22 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(AttnParams p) {
         }
     };
 
-    half8_t kt[U], vt[U], kk[U], vv[U];
-    auto issue_round = [&](int tb) {
-        if (PAGED && UB) {
+    half8_t kt[U], vt[U];
+    if (R == 0) issue_remainder(kt, vt);
+    if constexpr (QKN) {
+        half8_t kk[U], vv[U];
+        auto issue_round = [&](int tb) {
             const int64_t base = block_base(tb);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const unsigned lo = (unsigned)((u * RPI + tg) * row_elems + dc * 8);
                 kk[u] = load_row16<NT>(p.k + base + lo); vv[u] = load_row16<NT>(p.v + base + lo);
             }
-        } else {
-            int64_t off[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) off[u] = lane_row(tb + u * RPI + tg);
-#pragma unroll
-            for (int u = 0; u < U; ++u) { kk[u] = load_row16<NT>(p.k + off[u]); vv[u] = load_row16<NT>(p.v + off[u]); }
-        }
-    };
-    if (R == 0) issue_remainder(kt, vt);
-    if constexpr (QKN) {
+        };
         if (R > 0) issue_round(p0 + wave * TPI);
         asm volatile("" ::: "memory");                                    // the requests stay in front of the norm
         if (forms) {
-            const half8_t o = norm_rotate_piece(hx, hg, hc, hs, p.qk_eps, dc);
+            const half8_t o = norm_rotate_piece(hx, hg, hc, hs, own.qk_eps, dc);
             if (hi <= G) own_lds[hi * 16 + dc] = o;
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                // (LDS alone: __syncthreads may wait for the keys as well)
@@ -378,25 +377,46 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(AttnParams p) {
             *reinterpret_cast<half8_t *>(const_cast<half_t *>(p.k) + dst) = own_k;
             *reinterpret_cast<half8_t *>(const_cast<half_t *>(p.v) + dst) = own_v;
         }
-    }
-    // QKN: the pieces of token ctx - 1 among rows tb + step * u + tg (clamped to the partition's last one: those lanes' weights are 0, but what they are multiplied with has to be a number)
-    auto take_own = [&](half8_t (&ka)[U], half8_t (&va)[U], int tb, int step) {
-        if (QKN && own_slot >= 0)
+        // the pieces of token ctx - 1 among rows tb + step * u + tg (clamped to the partition's last one: those lanes' weights are 0, but what they are multiplied with has to be a number)
+        auto take_own = [&](half8_t (&ka)[U], half8_t (&va)[U], int tb, int step) {
+            if (own_slot >= 0)
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (min(tb + step * u + tg, pend - 1) == ctx - 1) { ka[u] = own_k; va[u] = own_v; }
-    };
-    for (int r = 0; r < R; ++r) {
-        const int tb = p0 + (r * WAVES + wave) * TPI;
-        if (!QKN || r > 0) issue_round(tb);
-        if (r == R - 1) issue_remainder(kt, vt);
-        if (QKN && tb + TPI >= ctx) take_own(kk, vv, tb, RPI);
-        process(std::false_type{}, kk, vv, 0);
+                for (int u = 0; u < U; ++u)
+                    if (min(tb + step * u + tg, pend - 1) == ctx - 1) { ka[u] = own_k; va[u] = own_v; }
+        };
+        for (int r = 0; r < R; ++r) {
+            const int tb = p0 + (r * WAVES + wave) * TPI;
+            if (r > 0) issue_round(tb);
+            if (r == R - 1) issue_remainder(kt, vt);
+            if (tb + TPI >= ctx) take_own(kk, vv, tb, RPI);
+            process(std::false_type{}, kk, vv, 0);
+        }
+        if (gt0 < ng && p0 + (gt0 + (U - 1) * WAVES + 1) * RPI >= ctx) take_own(kt, vt, p0 + gt0 * RPI, WAVES * RPI);
+    } else {
+        // (a loop of its own: with its requests in the lambda above, hipcc forms the addresses otherwise, and a launch is slower: 24 x 700 keys 15.6 / 16.0 us, 32 x 2048 of 32 heads 45.8 / 46.1,
+        // 256 x 1024 161 / 162)
+        for (int r = 0; r < R; ++r) {
+            const int tb = p0 + (r * WAVES + wave) * TPI;
+            half8_t kk[U], vv[U];
+            if (PAGED && UB) {
+                const int64_t base = block_base(tb);
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const unsigned lo = (unsigned)((u * RPI + tg) * row_elems + dc * 8);
+                    kk[u] = load_row16<NT>(p.k + base + lo); vv[u] = load_row16<NT>(p.v + base + lo);
+                }
+            } else {
+                int64_t off[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) off[u] = lane_row(tb + u * RPI + tg);
+#pragma unroll
+                for (int u = 0; u < U; ++u) { kk[u] = load_row16<NT>(p.k + off[u]); vv[u] = load_row16<NT>(p.v + off[u]); }
+            }
+            if (r == R - 1) issue_remainder(kt, vt);
+            process(std::false_type{}, kk, vv, 0);
+        }
     }
-    if (gt0 < ng) {
-        if (QKN && p0 + (gt0 + (U - 1) * WAVES + 1) * RPI >= ctx) take_own(kt, vt, p0 + gt0 * RPI, WAVES * RPI);
-        process(std::true_type{}, kt, vt, p0 + gt0 * RPI);
-    }
+    if (gt0 < ng) process(std::true_type{}, kt, vt, p0 + gt0 * RPI);
 
     // bring the row-group slots of the wave to their common max and sum them, then merge the waves through LDS
     constexpr bool ONE = SHM && WAVES == 1;                               // one wave per workgroup: its sums ARE the partition's partial (the cross-wave
@@ -553,7 +573,8 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float *__restrict
 // 44.5 / 39.8; heads of 64, 4 kv heads, 66 of 4000 keys: groups of 8 111.4 / 98.3, of 4 74.1 / 60.5, of 2 63.0 / 45.4.
 // QKN (27 sequences of 64 .. 8100 keys: a step of Qwen3-0.6B 1950 -> 1922 us): as in attn_rows_kernel, the step's own rows come raw; a segment's query heads (and key row, where it holds the query's last key) are formed when it is opened, behind its first requests.
 template <int D, int G, int U, int WAVES, bool QKN = false>
-__global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, int nq, int nw) {
+__global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(typename AttnParamsOf<QKN>::type own, int nq, int nw) {
+    const AttnParams &p = own;
     static_assert(!QKN || (D == 128 && G < 4 * WAVES), "QKN: heads of 128");
     constexpr int LPR = D / 8, RPI = 64 / LPR, TPI = RPI * U, CH = TPI * WAVES;
     static_assert(G * D <= WAVES * 64 && G * (D / 4) <= WAVES * 64, "one pass over the (head, column) pairs");
@@ -642,7 +663,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
         bt = p.block_tables + (int64_t)t * p.max_blocks;
         bt_chunk = (p0 >> p.bs_shift) >> 6;
         int64_t own_pos = 0; int own_slot = -1;
-        if constexpr (QKN) { own_pos = p.pos[t]; own_slot = p.slots ? p.slots[t] : -1; }
+        if constexpr (QKN) { own_pos = own.pos[t]; own_slot = own.slots ? own.slots[t] : -1; }
         { const int idx = (bt_chunk << 6) + lane; bt_reg = idx < p.max_blocks ? bt[idx] : 0; asm volatile("" : "+v"(bt_reg)); }
         half8_t hx, hg; float4_t hc[2], hs[2];
         if constexpr (QKN) {
@@ -651,9 +672,9 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
                 const int hh = min(wave * 4 + tg, G);
                 const int64_t at = own_pos * (D / 2) + (dc & 7) * 8;
                 hx = *reinterpret_cast<const half8_t *>(row + (hh < G ? g * G + hh : p.H + g) * D + dc * 8);
-                hg = *reinterpret_cast<const half8_t *>((hh < G ? p.qn_w : p.kn_w) + dc * 8);
+                hg = *reinterpret_cast<const half8_t *>((hh < G ? own.qn_w : own.kn_w) + dc * 8);
 #pragma unroll
-                for (int x = 0; x < 2; ++x) { hc[x] = *reinterpret_cast<const float4_t *>(p.cos_t + at + 4 * x); hs[x] = *reinterpret_cast<const float4_t *>(p.sin_t + at + 4 * x); }
+                for (int x = 0; x < 2; ++x) { hc[x] = *reinterpret_cast<const float4_t *>(own.cos_t + at + 4 * x); hs[x] = *reinterpret_cast<const float4_t *>(own.sin_t + at + 4 * x); }
             }
             own_v = *reinterpret_cast<const half8_t *>(row + (p.H + p.KVH + g) * D + dc * 8);
         } else {
@@ -670,7 +691,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_share_kernel(AttnParams p, in
             asm volatile("" ::: "memory");
             half8_t *lds = own_lds[opened & 1];
             if (wave * 4 <= G) {
-                const half8_t o = norm_rotate_piece(hx, hg, hc, hs, p.qk_eps, dc);
+                const half8_t o = norm_rotate_piece(hx, hg, hc, hs, own.qk_eps, dc);
                 if (wave * 4 + tg <= G) lds[(wave * 4 + tg) * 16 + dc] = o;
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -858,12 +879,13 @@ size_t attn_workspace_bytes(int64_t nq, int64_t H, int64_t D, int64_t max_ctx) {
 }
 
 template <int D, int G, int U, int WAVES, bool NT>
-static void launch_cfg(const AttnParams &p, bool paged, bool direct, int64_t nwg, hipStream_t s, bool fuse = false, bool shm = false, bool qkn = false) {
+static void launch_cfg(const AttnParams &p, bool paged, bool direct, int64_t nwg, hipStream_t s, bool fuse = false, bool shm = false, const OwnRows *own = nullptr) {
     dim3 grid((unsigned)nwg), block(WAVES * 64);
     if constexpr (D == 128 && G <= 4 && WAVES >= 4 && NT)
-        if (qkn) {
-            if (direct) attn_rows_kernel<D, G, true, true, U, WAVES, NT, true, false, false, true><<<grid, block, 0, s>>>(p);
-            else attn_rows_kernel<D, G, true, false, U, WAVES, NT, true, true, false, true><<<grid, block, 0, s>>>(p);
+        if (own) {
+            const AttnParamsOwn po{p, *own};
+            if (direct) attn_rows_kernel<D, G, true, true, U, WAVES, NT, true, false, false, true><<<grid, block, 0, s>>>(po);
+            else attn_rows_kernel<D, G, true, false, U, WAVES, NT, true, true, false, true><<<grid, block, 0, s>>>(po);
             return;
         }
     constexpr int TPI = 64 / (D / 8) * U;
@@ -899,9 +921,7 @@ static int own_rows(const AttnArgs &a, hipStream_t s) {                    // wh
 static bool own_rows_aligned(const AttnArgs &a) {
     return a.qn_w && a.ldq % 8 == 0 && (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.qn_w | (uintptr_t)a.kn_w | (uintptr_t)a.cos_t | (uintptr_t)a.sin_t) & 15) == 0;
 }
-static void own_rows_params(AttnParams &p, const AttnArgs &a) {
-    p.qn_w = (const half_t *)a.qn_w; p.kn_w = (const half_t *)a.kn_w; p.qk_eps = a.qk_eps; p.pos = a.pos; p.slots = a.slots; p.cos_t = a.cos_t; p.sin_t = a.sin_t;
-}
+static OwnRows own_rows_params(const AttnArgs &a) { return OwnRows{(const half_t *)a.qn_w, (const half_t *)a.kn_w, a.qk_eps, a.pos, a.slots, a.cos_t, a.sin_t}; }
 
 template <int D, int G>
 static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
@@ -1001,8 +1021,7 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
             bool in_it = false;
             if constexpr (D == 128 && G <= 4)
                 if (own_rows_aligned(a)) {
-                    own_rows_params(p, a);
-                    attn_share_kernel<D, G, DU / 2, 8, true><<<dim3((unsigned)(shares * a.KVH)), dim3(512), 0, s>>>(p, (int)a.nq, shares);
+                    attn_share_kernel<D, G, DU / 2, 8, true><<<dim3((unsigned)(shares * a.KVH)), dim3(512), 0, s>>>(AttnParamsOwn{p, own_rows_params(a)}, (int)a.nq, shares);
                     in_it = true;
                 }
             if (!in_it) {
@@ -1036,21 +1055,21 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
     // 64 1674 / 1677, 128 2243 / 2249; 256 of 1024 keys 6069 / 6090)
     const int tpi = 64 / (D / 8) * (brief || waves == 4 ? DU : DU / 2);
     const bool qkn = D == 128 && G <= 4 && !shared && paged && pairs <= share_workgroups() && (waves == 8 || waves == 4) && (direct || fuse) && p.block_size % tpi == 0 && (p.num_parts == 1 || p.part_size % tpi == 0) && own_rows_aligned(a);
-    if (qkn) own_rows_params(p, a);
-    else if (int rc = own_rows(a, s)) return rc;
+    const OwnRows own_params = own_rows_params(a), *const own = qkn ? &own_params : nullptr;
+    if (!qkn) if (int rc = own_rows(a, s)) return rc;
     if (shared)
         if (int rc = flash_shared_prefix(a.q, a.ldq, a.k, a.v, a.block_tables, a.max_blocks, a.block_size, a.nq, a.H, a.KVH, a.D, a.scale,
                                          shared_part, sparts, np, p.part_o, p.part_ml, s, a.shared_rows, a.shared_count)) return rc;
     {
         if (brief) {
             const bool ub = p.block_size % (64 / (D / 8) * DU) == 0;
-            if (qkn) launch_cfg<D, G, DU, 8, true>(p, true, true, nwg, s, false, false, true);
+            if (qkn) launch_cfg<D, G, DU, 8, true>(p, true, true, nwg, s, false, false, own);
             else if (ub) attn_rows_kernel<D, G, true, true, DU, 8, true, true><<<dim3((unsigned)nwg), dim3(512), 0, s>>>(p);
             else attn_rows_kernel<D, G, true, true, DU, 8, true, false><<<dim3((unsigned)nwg), dim3(512), 0, s>>>(p);
-        } else if (waves == 8) launch_cfg<D, G, DU / 2, 8, true>(p, paged, direct, nwg, s, fuse, false, qkn);  // K/V streamed once: nt loads
+        } else if (waves == 8) launch_cfg<D, G, DU / 2, 8, true>(p, paged, direct, nwg, s, fuse, false, own);  // K/V streamed once: nt loads
         else if (paged && waves == 1) { if constexpr (G * (D / 4) <= 64) launch_cfg<D, G, DU, 1, true>(p, paged, direct, nwg, s, fuse, shm); }   // (U = 2: 3.18-3.20 against 3.14-3.17 ms per configs[4] step)
         else if (paged && waves == 2) { if constexpr (G * (D / 4) <= 128) launch_cfg<D, G, DU, 2, true>(p, paged, direct, nwg, s, fuse, shm); }
-        else if (paged) launch_cfg<D, G, DU, 4, true>(p, paged, direct, nwg, s, fuse, shm, qkn);
+        else if (paged) launch_cfg<D, G, DU, 4, true>(p, paged, direct, nwg, s, fuse, shm, own);
         else launch_cfg<D, G, DU, 4, false>(p, paged, direct, nwg, s);                     // prefill: rows re-read from L2
     }
     if (!direct && !fuse && !shm)
