@@ -107,7 +107,6 @@ struct RetentionArgs {
     // gated form, decay_exp: the decay is exp(-exp(az + abias)) instead of a power of the sigmoid.  bonus (gated form, [H][D] f32): the output is read BEFORE the update
     // and sees the current token through the bonus alone, o = (S_(t-1) + diag(bonus_h) k v^T)^T q, then S_t = diag(decay) S_(t-1) + k v^T
     bool decay_exp; const float *bonus;
-    int32_t below;                           // (set by retention(): > 0, the recurrence walks only the sequences of fewer rows of this step)
 };
 int retention(const RetentionArgs &a, const Batch &b, bool bf16, hipStream_t s);
 // out[t][h*Dv + c] = o[t][h][c] / rms(o[t][h][:]) * w[c] * silu(gate[t][h*Dv + c]); gate: rows of the operand type (stride ldg) from column gcol; w (one weight per

@@ -789,7 +789,10 @@ __global__ __launch_bounds__(256) void retention_seq_kernel(RetentionArgs a, Bat
 // barrier later they are summed over the 8 row groups.  Token order and arithmetic per token are those of the token-by-token kernel: the result does not depend
 // on where a prompt is cut.  Thread (c, part) owns rows part * RMAX .. part * RMAX + RMAX - 1 of column c.
 // GATED: the decay is per token and key channel, sigmoid(z + bias)^(1/tau) with z from rows of the operand type, and q is scaled by qscale (gated linear attention).
-template <int RMAX, class PT, int MODE>
+// SHORT: the sequences of fewer rows than a chunk of a step whose others retention_chunk_kernel walks (an instance of its own: the comparison alone cost the others 16.4 -> 17.2 us a decode step's
+// launch of 24 sequences)
+constexpr int RET_CHUNK = 16;
+template <int RMAX, class PT, int MODE, bool SHORT = false>
 __global__ __launch_bounds__(256) void retention_block_kernel(RetentionArgs a, Batch b) {
     constexpr bool GATED = MODE != 0, PRE = MODE == 2;
     constexpr int TB = 16;
@@ -801,7 +804,7 @@ __global__ __launch_bounds__(256) void retention_block_kernel(RetentionArgs a, B
     const int sq = blockIdx.x, h = blockIdx.y, cb = blockIdx.z * 32;
     const int cl = threadIdx.x & 31, c = cb + cl, part = threadIdx.x >> 5;
     const int r0 = b.cu[sq], n = b.cu[sq + 1] - r0, st = b.start[sq];
-    if (!GATED && a.below > 0 && n >= a.below) return;        // (walked by retention_chunk_kernel)
+    if (SHORT && n >= RET_CHUNK) return;
     const bool tok = !GATED && a.tok_gate != nullptr;
     const float dec = (GATED || tok) ? 0.f : a.decay[h];
     const int Dr = Dv - a.v_ones;
@@ -988,8 +991,7 @@ __global__ __launch_bounds__(256) void retention_block_kernel(RetentionArgs a, B
 // below the token-by-token sum's (1024 tokens of a unit normal: output 1.7e-7 of its size against 4.6e-7, state 1.6e-7 against 5.5e-7; 16 tokens 1.16e-7 against 1.24e-7).
 // 16 x 1024 tokens, 16 heads of 128 x 128: 268 us against 686 of the recurrence (150 us of matrix instructions; the rest is LDS, rotation and the waits of a chunk at two waves a SIMD);
 // one prompt of 1024: 163 against 352; 2 x 16 tokens, 64 heads of 128 x 64: 6.9 against 11.0.  Not a bit-for-bit cut: where a prompt's portions end moves the chunks' limits.  A sequence of
-// fewer rows than a chunk keeps the recurrence whatever else is in the step (RetentionArgs::below), so that its bits do not depend on its neighbours.
-constexpr int RET_CHUNK = 16;
+// fewer rows than a chunk keeps the recurrence whatever else is in the step, so that its bits do not depend on its neighbours.
 template <int D>
 __global__ __launch_bounds__(256, 2) void retention_chunk_kernel(RetentionArgs a, Batch b) {
     constexpr int ND = D / 16, QS = D + 4, KS = 20, HALF = D / 2, PT = D / 8;      // (row strides: the 16 lanes of a b128 read touch every bank once)
@@ -1486,28 +1488,31 @@ int retention(const RetentionArgs &a, const Batch &b, bool bf16, hipStream_t s) 
     } while (0)
     // sequences of a whole chunk of rows or more (from 16 rows the chunk form is the faster one at every size measured: 4.8 us against 7.9 at 2 x 16 tokens, 2 heads of 64 x 64; single
     // tokens keep the recurrence, which the state's bytes bound).  A sequence's form goes by its own rows: the shorter ones of such a step take the recurrence in a launch of their own
-    RetentionArgs few = a;
-    few.below = 0;
     if (bf16 && !gated && !a.tok_gate && a.v_ones == 0 && (a.D == 64 || a.D == 128) && a.rot_dims == a.D && a.Dv % 64 == 0 && b.max_rows >= RET_CHUNK && ((a.ld | a.qcol | a.kcol | a.vcol) & 3) == 0 &&
         ((uintptr_t)a.proj & 7) == 0 && (((uintptr_t)a.cos_t | (uintptr_t)a.sin_t) & 15) == 0) {
         const dim3 g((unsigned)b.B, (unsigned)a.H, (unsigned)(a.Dv / 64));
         const size_t lds = (2 * (32 * ((size_t)a.D + 4) + (a.D + 64) * 20) + 2 * 1024 + 40) * 4;
         if (a.D == 64) retention_chunk_kernel<64><<<g, dim3(256), lds, s>>>(a, b);
         else retention_chunk_kernel<128><<<g, dim3(256), lds, s>>>(a, b);
-        if (b.min_rows >= RET_CHUNK) return launched("retention");
-        few.below = RET_CHUNK;
+        if (b.min_rows < RET_CHUNK) {
+            const dim3 gs((unsigned)b.B, (unsigned)a.H, (unsigned)((a.Dv + 31) / 32));
+            const size_t ls = ((size_t)2 * 16 * a.D + 16 * 32 + 16 * 8 * 32 + 32 + 128) * 4;
+            if (a.D == 64) retention_block_kernel<8, bf16_t, 0, true><<<gs, dim3(256), ls, s>>>(a, b);
+            else retention_block_kernel<16, bf16_t, 0, true><<<gs, dim3(256), ls, s>>>(a, b);
+        }
+        return launched("retention");
     }
     const size_t lds = ((size_t)(gated ? 3 : 2) * 16 * a.D + 16 * 32 + 16 * 8 * 32 + 32 + 128) * 4;
     if (a.D <= 256 && lds <= 64 * 1024) {                 // (beyond: the token-by-token form, whose LDS does not grow with the key size)
         const dim3 grid((unsigned)b.B, (unsigned)a.H, (unsigned)(((a.tok_gate && a.v_ones == 1 ? a.Dv - 1 : a.Dv) + 31) / 32));   // (a single column of ones rides in the first block)
 #define NVR_RETB(R_)                                                                                 \
     do {                                                                                             \
-        if (gated && a.bonus) { if (bf16) retention_block_kernel<R_, bf16_t, 2><<<grid, dim3(256), lds, s>>>(few, b);   \
-                                else retention_block_kernel<R_, float, 2><<<grid, dim3(256), lds, s>>>(few, b); }       \
-        else if (gated) { if (bf16) retention_block_kernel<R_, bf16_t, 1><<<grid, dim3(256), lds, s>>>(few, b);   \
-                     else retention_block_kernel<R_, float, 1><<<grid, dim3(256), lds, s>>>(few, b); }       \
-        else if (bf16) retention_block_kernel<R_, bf16_t, 0><<<grid, dim3(256), lds, s>>>(few, b); \
-        else retention_block_kernel<R_, float, 0><<<grid, dim3(256), lds, s>>>(few, b);            \
+        if (gated && a.bonus) { if (bf16) retention_block_kernel<R_, bf16_t, 2><<<grid, dim3(256), lds, s>>>(a, b);   \
+                                else retention_block_kernel<R_, float, 2><<<grid, dim3(256), lds, s>>>(a, b); }       \
+        else if (gated) { if (bf16) retention_block_kernel<R_, bf16_t, 1><<<grid, dim3(256), lds, s>>>(a, b);   \
+                     else retention_block_kernel<R_, float, 1><<<grid, dim3(256), lds, s>>>(a, b); }       \
+        else if (bf16) retention_block_kernel<R_, bf16_t, 0><<<grid, dim3(256), lds, s>>>(a, b); \
+        else retention_block_kernel<R_, float, 0><<<grid, dim3(256), lds, s>>>(a, b);            \
     } while (0)
         if (rows <= 8) NVR_RETB(8);
         else if (rows <= 16) NVR_RETB(16);
