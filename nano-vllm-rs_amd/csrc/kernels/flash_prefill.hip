@@ -517,9 +517,10 @@ __global__ __launch_bounds__(64 * FLASH_WAVES, 8 / FLASH_WAVES) void flash_prefi
 // (K runs one step ahead of V through the LDS ring).  The accumulators are rescaled at a step's start, behind the barrier, where the products on them have long ended, and only if a query of the
 // wave met a larger score.  Raising the maximum only past a margin (2^8 in the exponentials' unit) takes another 7 % off, but the largest weight is then no longer the 1 that has no rounding:
 // the attention's error against 64 bits grew by 2.5 %.
-// bfloat16, G = 2, us before (16 x 16 x 32 products, one after the other) / now, launches alone: 32 prompts of 1024 tokens 201 / 184 a layer (in a step of float16 218 / 197), one of 509 16.2 /
-// 15.1, of 2048 49.0 / 45.5, of 8192 334 / 325; 100 steps of one workgroup per CU 143 / 134, of two 212 / 212: cycles fall, and with the matrix cores' load the clock, from 2.1 to 1.75 GHz.  Of 202
-// us of two per CU without rescaling: without the K reads 171, the V reads 188, the exponentials 185, the LDS-DMA 183, products and the rest of the vector work alone 127.
+// bfloat16, G = 2, us before (16 x 16 x 32 products, one after the other) / now, launches alone: 32 prompts of 1024 tokens 201 / 184 a layer (in a step of float16 218 / 197), one of 2048 49.0 /
+// 45.5, of 8192 334 / 325; one of 16, 64, 128, 300, 509 tokens through block tables 5.6 7.2 8.6 12.2 16.9 / 5.4 6.0 7.2 10.9 15.0; 100 steps of one workgroup per CU 143 / 134, of two 212 / 212:
+// cycles fall, and with the matrix cores' load the clock, from 2.1 to 1.75 GHz.  Of 202 us of two per CU without rescaling: without the K reads 171, the V reads 188, the exponentials 185, the
+// LDS-DMA 183, products and the rest of the vector work alone 127.
 // N products, each followed by READS LDS reads (those of the product AHEAD products later) and VALU vector instructions
 template <int N, int READS, int AHEAD, int VALU>
 __device__ __forceinline__ void sched_pattern() {
@@ -706,8 +707,10 @@ __global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
     scores(s0, s1);
     if (KT - 1 > tile.pos0) { mask(0, s0); mask(32, s1); }
     float mx = maximum(s0, s1);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();                                         // (K of step 2 takes the place of K of step 0)
+    if (nsteps > 2) {                                                     // (K of step 2 takes the place of K of step 0)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+    }
     int it = 0;
     for (; it + 1 < mysteps; ++it) {                                      // a step and the scores of the one behind it
         request(it);
@@ -747,11 +750,12 @@ __global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
         for (int k = 0; k < 4; ++k) { pf[k] = exponentials(k < 2 ? s0 : s1, k & 1, mc); add_up(pf[k]); }
 #pragma unroll
         for (int k = 0; k < 4; ++k) values(k, pf[k]);
-        close();
+        if (it + 1 < nsteps) close();
     }
     for (++it; it < nsteps; ++it) { request(it); close(); }               // steps of the tile's later queries
     l = xor32_partner_sum(l);
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    // w / l = w inv + w rest with inv two units below 1 / l: within half a unit of f32, two instructions a number, and an infinite w stays (rest > 0, both terms have its sign)
+    const float r1 = 1.0f / l, inv = l > 0.f ? __uint_as_float(__float_as_uint(r1) - 2) : 0.f, rest = l > 0.f ? fmaf(-inv, l, 1.0f) * r1 : 0.f;
     half_t *orow = p.out + (int64_t)qrow * p.ldo + (int64_t)head * D + h * 8;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
@@ -761,10 +765,7 @@ __global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
             union { half_t v[8]; unsigned u[4]; } x;
             union { half8_t v; unsigned u[4]; } y;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {                                  // (the quotient, corrected once: within half a unit of f32; an infinite one stays)
-                const float w = o[dt][e + j], d = w * inv, c = fmaf(fmaf(-d, l, w), inv, d);
-                x.v[j] = (half_t)(fabsf(d) < INFINITY ? c : d);
-            }
+            for (int j = 0; j < 8; ++j) { const float w = o[dt][e + j]; x.v[j] = (half_t)fmaf(w, inv, w * rest); }
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const auto sw = __builtin_amdgcn_permlane32_swap(x.u[j], x.u[2 + j], false, false);
