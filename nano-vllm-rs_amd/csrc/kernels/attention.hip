@@ -1019,8 +1019,11 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
             p.part0 = 0; p.kv0 = 0; p.kv0_rows = nullptr; p.tickets = a.tickets;
             const int shares = (int)std::max<int64_t>(1, cus / a.KVH);                      // one workgroup per CU
             bool in_it = false;
+            // (the step's own rows in this launch up to three pairs for two CUs: a share opens more segments beyond, and each waits for its norms.  Qwen3-0.6B with norms, us a step by a launch in
+            // front / here: 33 sequences of 32..700 keys 1436 / 1388, 40 of 64..4000 1960 / 1922, 48 of 64..2000 1834 / 1780, 56 of 64..2000 1926 / 1992, 64 of 64..3000 2317 / 2308, 80 of 32..700
+            // 1853 / 1890, 96 of 64..2000 2488 / 2514, 128 of 32..700 2244 / 2309, 200 of 32..1000 2730 / 2737)
             if constexpr (D == 128 && G <= 4)
-                if (own_rows_aligned(a)) {
+                if (own_rows_aligned(a) && 2 * pairs <= 3 * (int64_t)cus) {
                     attn_share_kernel<D, G, DU / 2, 8, true><<<dim3((unsigned)(shares * a.KVH)), dim3(512), 0, s>>>(AttnParamsOwn{p, own_rows_params(a)}, (int)a.nq, shares);
                     in_it = true;
                 }
