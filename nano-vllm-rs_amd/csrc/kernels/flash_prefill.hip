@@ -752,7 +752,7 @@ __global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
         for (int k = 0; k < 4; ++k) values(k, pf[k]);
         if (it + 1 < nsteps) close();
     }
-    for (++it; it < nsteps; ++it) { request(it); close(); }               // steps of the tile's later queries
+    for (++it; it + 1 < nsteps; ++it) { request(it); close(); }           // steps of the tile's later queries (the last one has nothing to request or to close)
     l = xor32_partner_sum(l);
     // w / l = w inv + w rest with inv two units below 1 / l: within half a unit of f32, two instructions a number, and an infinite w stays (rest > 0, both terms have its sign)
     const float r1 = 1.0f / l, inv = l > 0.f ? __uint_as_float(__float_as_uint(r1) - 2) : 0.f, rest = l > 0.f ? fmaf(-inv, l, 1.0f) * r1 : 0.f;
