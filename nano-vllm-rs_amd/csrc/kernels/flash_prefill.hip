@@ -518,7 +518,7 @@ __global__ __launch_bounds__(64 * FLASH_WAVES, 8 / FLASH_WAVES) void flash_prefi
 // wave met a larger score.  Raising the maximum only past a margin (2^8 in the exponentials' unit) takes another 7 % off, but the largest weight is then no longer the 1 that has no rounding:
 // the attention's error against 64 bits grew by 2.5 %.
 // bfloat16, G = 2, us before (16 x 16 x 32 products, one after the other) / now, launches alone: 32 prompts of 1024 tokens 201 / 184 a layer (in a step of float16 218 / 197), one of 2048 49.0 /
-// 45.5, of 8192 334 / 325; one of 16, 64, 128, 300, 509 tokens through block tables 5.6 7.2 8.6 12.2 16.9 / 5.4 6.0 7.2 10.9 15.0; 100 steps of one workgroup per CU 143 / 134, of two 212 / 212:
+// 45.5, of 8192 334 / 325; one of 16, 64, 128, 300, 509 tokens through block tables 5.9 7.5 8.8 12.3 17.2 / 5.7 6.2 7.4 11.1 15.4; 100 steps of one workgroup per CU 143 / 134, of two 212 / 212:
 // cycles fall, and with the matrix cores' load the clock, from 2.1 to 1.75 GHz.  Of 202 us of two per CU without rescaling: without the K reads 171, the V reads 188, the exponentials 185, the
 // LDS-DMA 183, products and the rest of the vector work alone 127.
 // N products, each followed by READS LDS reads (those of the product AHEAD products later) and VALU vector instructions
@@ -765,7 +765,12 @@ __global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
             union { half_t v[8]; unsigned u[4]; } x;
             union { half8_t v; unsigned u[4]; } y;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) { const float w = o[dt][e + j]; x.v[j] = (half_t)fmaf(w, inv, w * rest); }
+            for (int j = 0; j < 8; ++j) {
+                float w = o[dt][e + j];
+                w = fmaf(w, inv, w * rest);
+                asm("" : "+v"(w));                                         // (rounded to 32 bits first, as ever: hipcc would fuse the sum with the rounding to float16)
+                x.v[j] = (half_t)w;
+            }
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const auto sw = __builtin_amdgcn_permlane32_swap(x.u[j], x.u[2 + j], false, false);
