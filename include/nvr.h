@@ -594,6 +594,12 @@ NVR_API int nvr_qk_norm_rope_store_kv(nvr_half *qkv, const int64_t *positions, c
                                       int64_t H, int64_t KVH, int64_t D, const float *cos_t, const float *sin_t,
                                       const nvr_half *q_norm_w, const nvr_half *k_norm_w, float eps,
                                       nvr_half *k_cache, nvr_half *v_cache, void *stream);
+/* qkv = x · W_qkvᵀ and nvr_qk_norm_rope_store_kv on it in one launch (the bits of nvr_linear_tiled with that behind it), for heads of 128 and the row counts that nvr_linear multiplies on LDS
+ * tiles (NVR_ERR_UNSUPPORTED otherwise).  Wt: nvr_retile_weight mode 0 of W, or null; kv_cache_only: k and v rows go to the caches alone where they have a slot */
+NVR_API int nvr_linear_qkv_norm_rope_store(const nvr_half *x, int64_t ldx, const nvr_half *W, const nvr_half *Wt, int64_t T, int64_t K,
+                                           int64_t H, int64_t KVH, int64_t D, const int64_t *positions, const int32_t *slot_mapping,
+                                           const float *cos_t, const float *sin_t, const nvr_half *q_norm_w, const nvr_half *k_norm_w, float eps,
+                                           nvr_half *qkv, nvr_half *k_cache, nvr_half *v_cache, int kv_cache_only, void *stream);
 NVR_API int nvr_rope_table(int64_t D, int64_t max_pos, double theta, float *cos_dev, float *sin_dev); /* rotary_embedding.rs:74-119 */
 /* K9 decode paged attention, attention.rs:225-235,264-318 (A-8).  q rows have stride ldq
  * elements ([B, H, D] inside the packed qkv buffer).  workspace: nvr_paged_attn_workspace_bytes. */

@@ -389,6 +389,7 @@ extern "C" {
     pub fn nvr_linear_qkv_rope_store(x: *const u16, ldx: i64, W: *const u16, T: i64, K: i64, H: i64, KVH: i64, D: i64, positions: *const i64, slot_mapping: *const i32, cos_t: *const f32, sin_t: *const f32, qkv: *mut u16, k_cache: *mut u16, v_cache: *mut u16, stream: *mut c_void) -> c_int;
     pub fn nvr_rope_store_kv(qkv: *mut u16, positions: *const i64, slot_mapping: *const i32, T: i64, H: i64, KVH: i64, D: i64, cos_t: *const f32, sin_t: *const f32, k_cache: *mut u16, v_cache: *mut u16, stream: *mut c_void) -> c_int;
     pub fn nvr_qk_norm_rope_store_kv(qkv: *mut u16, positions: *const i64, slot_mapping: *const i32, T: i64, H: i64, KVH: i64, D: i64, cos_t: *const f32, sin_t: *const f32, q_norm_w: *const u16, k_norm_w: *const u16, eps: f32, k_cache: *mut u16, v_cache: *mut u16, stream: *mut c_void) -> c_int;
+    pub fn nvr_linear_qkv_norm_rope_store(x: *const u16, ldx: i64, W: *const u16, Wt: *const u16, T: i64, K: i64, H: i64, KVH: i64, D: i64, positions: *const i64, slot_mapping: *const i32, cos_t: *const f32, sin_t: *const f32, q_norm_w: *const u16, k_norm_w: *const u16, eps: f32, qkv: *mut u16, k_cache: *mut u16, v_cache: *mut u16, kv_cache_only: c_int, stream: *mut c_void) -> c_int;
     pub fn nvr_rope_table(D: i64, max_pos: i64, theta: f64, cos_dev: *mut f32, sin_dev: *mut f32) -> c_int;
     pub fn nvr_paged_attn_workspace_bytes(B: i64, H: i64, D: i64, max_context_len: i64) -> usize;
     pub fn nvr_paged_attn_decode(q: *const u16, ldq: i64, k_cache: *const u16, v_cache: *const u16, meta: *const nvr_attn_meta, H: i64, KVH: i64, D: i64, block_size: i64, scale: f32, out: *mut u16, workspace: *mut c_void, stream: *mut c_void) -> c_int;

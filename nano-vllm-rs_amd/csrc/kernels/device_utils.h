@@ -155,6 +155,28 @@ __device__ __forceinline__ float head_sum(float x) {
     return dpp_add<0xB1>(x);
 }
 
+// RMSNorm over a head of LPH * 16 columns held by LPH neighbouring lanes, lane j with columns j * 8 .. of either half (x1, x2; the norm's weights g1, g2).  The sums' pairs, divisions and roundings
+// of qknorm_rope_store_kernel, hence its bits.  x / rms: with y = 1 / rms rounded, q = x y and the residual r = x - q rms (exact), q + r y is the rounded quotient (Markstein, IBM Journal of
+// Research and Development 34, 1990, theorem 7.1) as long as nothing over- or underflows (r of numbers below 1e-30 may): 3 instructions a number instead of 10.
+template <int LPH>
+__device__ __forceinline__ void head_norm(half8_t &x1, half8_t &x2, half8_t g1, half8_t g2, float eps) {
+#pragma clang fp contract(off)
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) { const float a = (float)x1[e], b = (float)x2[e], aa = a * a, bb = b * b, ab = aa + bb; ss = ss + ab; }
+    ss = head_sum<LPH>(ss);
+    const float rms = sqrtf(ss / (float)(LPH * 16) + eps);
+    if (rms > 1e-15f && rms < 1e15f) {
+        const float y = __fdiv_rn(1.0f, rms);
+        auto quotient = [&](float x) { const float q = x * y; return __fmaf_rn(__fmaf_rn(-q, rms, x), y, q); };
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { x1[e] = to_half_rn(__fmul_rn(quotient((float)x1[e]), (float)g1[e])); x2[e] = to_half_rn(__fmul_rn(quotient((float)x2[e]), (float)g2[e])); }
+    } else {                                                                  // (NaN, infinities, zeros without eps)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { x1[e] = to_half_rn(__fmul_rn(__fdiv_rn((float)x1[e], rms), (float)g1[e])); x2[e] = to_half_rn(__fmul_rn(__fdiv_rn((float)x2[e], rms), (float)g2[e])); }
+    }
+}
+
 // lane-wise butterflies across the 16-lane rows of a wave on the gfx950 lane-swap instructions (no LDS traffic):
 // v_permlane16_swap exchanges the odd rows of one register with the even rows of another, v_permlane32_swap the
 // upper half of one with the lower half of the other; fed the same value twice, the two results are x and its

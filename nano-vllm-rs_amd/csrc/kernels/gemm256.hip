@@ -32,7 +32,8 @@
 
 namespace nvr { namespace NVR_DT_NS {
 
-enum { GEPI_F16 = 0, GEPI_RESID = 1, GEPI_SILU = 2, GEPI_ROPE = 3, GEPI_LMHEAD = 4, GEPI_RELU2 = 5, GEPI_GELU = 6, GEPI_GELU_ERF = 7 };   // GELU_ERF: y = gelu(x·Wᵀ) with the error function (from the unrounded product); RELU2: y = max(x·Wᵀ, 0)² (the product rounded to 16 bits first, as the unfused pair of launches does)
+enum { GEPI_F16 = 0, GEPI_RESID = 1, GEPI_SILU = 2, GEPI_ROPE = 3, GEPI_LMHEAD = 4, GEPI_RELU2 = 5, GEPI_GELU = 6, GEPI_GELU_ERF = 7, GEPI_QKN = 8 };   // GELU_ERF: y = gelu(x·Wᵀ) with the error function (from the unrounded product); RELU2: y = max(x·Wᵀ, 0)² (the product rounded to 16 bits first, as the unfused pair of launches does)
+constexpr bool g_rope(int epi) { return epi == GEPI_ROPE || epi == GEPI_QKN; }      // QKN: RMSNorm over the columns of every q and k head in front of the rotation
 constexpr bool g_glu(int epi) { return epi == GEPI_SILU || epi == GEPI_GELU; }      // gate and up rows in one tile, out = act(gate) * up (GELU: the tanh form)
 //   // RESID: y is the residual stream: y <- fp16(y + fp16(x·Wᵀ)) (qwen3.rs:382,389)
 // LMHEAD (r06): the LM head over >= 128 rows (ParallelLMHead::compute_logits, embed_head.rs:292-306, + the greedy branch of Sampler::forward,
@@ -46,6 +47,7 @@ struct G256Epi {
     int32_t H, KVH, D;
     int32_t kv_cache_only;             // GEPI_ROPE: k and v rows go to the caches only (the attention that follows reads them there)
     float *logits; float *pval; int32_t *pidx;   // GEPI_LMHEAD: f32 logits [T][N] (nullable), arg-max partials [tiles_x][T]
+    const half_t *qn_w, *kn_w; float qk_eps;     // GEPI_QKN: the norms' weights [D]
     const int32_t *row_w; int64_t w_stride; const int32_t *rows_used;      // (rows_used, on the device: rows behind it are nobody's; null: all T) GRP (rows grouped by expert): row block rb of 256 rows multiplies the matrix W + row_w[rb] * w_stride
 };
 
@@ -58,13 +60,13 @@ constexpr int G_BUF = 4 * G_HALF;                                         // A0 
 //   RoPE: head = bx*(256/D) + rho/hd2, row = head*D + hA*hd2 + rho%hd2  (hd2 = D/2 divides 64: rho/hd2 = r0/hd2 + i*(64/hd2))
 template <int EPI, int RD>
 __device__ __forceinline__ int g_w_thr(int r0) {
-    if (EPI == GEPI_ROPE) { constexpr int hd2 = RD / 2 > 0 ? RD / 2 : 1; return (r0 / hd2) * RD + r0 % hd2; }
+    if (g_rope(EPI)) { constexpr int hd2 = RD / 2 > 0 ? RD / 2 : 1; return (r0 / hd2) * RD + r0 % hd2; }
     return r0;
 }
 template <int EPI, int RD>
 __device__ __forceinline__ int g_w_uni(int hA, int i, int N) {
     if (g_glu(EPI)) return hA * N + i * 64;
-    if (EPI == GEPI_ROPE) return i * 128 + hA * (RD / 2);
+    if (g_rope(EPI)) return i * 128 + hA * (RD / 2);
     return hA * 128 + i * 64;
 }
 
@@ -192,7 +194,7 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__
     // start of their own tile they sat in front of that tile's first staging waits (s_waitcnt vmcnt is in issue order) and stalled
     // every tile's first K-tile by a memory round trip.
     auto request_rows = [&](int tile_, int slot) {
-        if (EPI == GEPI_ROPE && grp == 0) {
+        if (g_rope(EPI) && grp == 0) {
             int m = (tile_ / tiles_x) * 256 + wave * 64 + lane; if (m > T - 1) m = T - 1;
             char *dst = smem + 2 * G_BUF + slot * 2048 + wave * 256;
             __builtin_amdgcn_global_load_lds(epi.pos + m, (__attribute__((address_space(3))) void *)dst, 4, 0, 0);
@@ -219,8 +221,8 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__
 #define G256_W(NOMORE_) if (more) { G256_R_END(4) } else { G256_R_END(NOMORE_) }
 
     constexpr int OUTC = g_glu(EPI) ? 128 : 256;                  // output columns of a tile
-    const int64_t ldy = (EPI == GEPI_ROPE) ? (int64_t)(epi.H + 2 * epi.KVH) * RD : (int64_t)N;
-    constexpr int hd2 = (EPI == GEPI_ROPE) ? RD / 2 : 1;
+    const int64_t ldy = g_rope(EPI) ? (int64_t)(epi.H + 2 * epi.KVH) * RD : (int64_t)N;
+    constexpr int hd2 = g_rope(EPI) ? RD / 2 : 1;
 
     int tile_no = 0;
     for (int g = 0;; ) {
@@ -340,13 +342,14 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__
         // head), so the requests for the cos / sin rows leave right after a half's conversion and fly across its staging barrier.
         if (have_next) request_rows(next_tile, (tile_no + 1) & 1);
         const int *lds_pos = reinterpret_cast<const int *>(smem + 2 * G_BUF + (tile_no & 1) * 2048), *lds_slot = lds_pos + 256;
-        constexpr int hp = (EPI == GEPI_ROPE) ? RD / 16 : 1;               // 16-byte pieces per half head
-        const int pc = tid & 15, head_l = pc / hp, pcc = pc % hp;         // this thread's pair inside a row (16 pairs per 256 columns)
-        const int ch1 = head_l * 2 * hp + pcc, ch2 = ch1 + hp;
-        const int rhead = (EPI == GEPI_ROPE) ? bx * (256 / (RD > 0 ? RD : 256)) + head_l : 0;
-        const bool rot = (EPI == GEPI_ROPE) && rhead < epi.H + epi.KVH;   // q and k heads rotate, v heads pass through
-        int rslot[4];
-        float4_t cs[4][2], sn[4][2];
+        // A thread takes the same pair of pieces of every head of its rows: the heads share one set of cosines and sines (a thread per head and pair fetched them once for each
+        // head: for 256 x 256 outputs as many bytes as the outputs).
+        constexpr int hp = g_rope(EPI) ? RD / 16 : 1;                     // 16-byte pieces per half head = neighbouring lanes of a head's row
+        constexpr int RPP = 512 / hp, PASSES = g_rope(EPI) ? 128 / RPP : 1, HN = g_rope(EPI) ? 256 / RD : 1;      // rows per pass over a half, heads of a row
+        const int pcc = tid % hp, prow = tid / hp, head0 = bx * HN;
+        int rslot[PASSES];
+        float4_t cs[PASSES][2], sn[PASSES][2];
+        half8_t g1[HN], g2[HN];
         // plain / residual / RoPE epilogues: all 128 accumulator registers become 64 registers of packed fp16 at once (the values the
         // halves stage below), so that the second half's results do not sit in f32 under the first half's store phase: the RoPE
         // store phase holds 64 registers of cos / sin next to them, and a spill here is a global-memory round trip (scratch)
@@ -389,13 +392,13 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int ml = wm * 32 + j * 16 + r;                      // token row inside the half
-                if (EPI == GEPI_F16 || EPI == GEPI_RESID || EPI == GEPI_ROPE || EPI == GEPI_RELU2 || EPI == GEPI_GELU_ERF) {
+                if (EPI == GEPI_F16 || EPI == GEPI_RESID || g_rope(EPI) || EPI == GEPI_RELU2 || EPI == GEPI_GELU_ERF) {
 #pragma unroll
                     for (int a = 0; a < 2; ++a)
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
                             const int rho = wn * 64 + i * 16 + q * 4;     // local W row; RoPE: A0 / A1 hold the first / second halves of the heads
-                            const int colo = (EPI == GEPI_ROPE) ? (rho / hd2) * RD + a * hd2 + rho % hd2 : a * 128 + rho;
+                            const int colo = g_rope(EPI) ? (rho / hd2) * RD + a * hd2 + rho % hd2 : a * 128 + rho;
                             put(ml, colo, pk[a][i][hB][j]);
                         }
                 } else if (g_glu(EPI)) {
@@ -412,21 +415,28 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__
                     }
                 }
             }
-            if (EPI == GEPI_ROPE) {
+            if (g_rope(EPI)) {
 #pragma unroll
-                for (int kk = 0; kk < 4; ++kk) {
-                    const int row = hB * 128 + (tid >> 4) + kk * 32;
+                for (int kk = 0; kk < PASSES; ++kk) {
+                    const int row = hB * 128 + prow + kk * RPP;
                     const int pos = lds_pos[row];
                     rslot[kk] = epi.slots ? lds_slot[row] : -1;
 #pragma unroll
                     for (int hh = 0; hh < 2; ++hh) cs[kk][hh] = sn[kk][hh] = (float4_t){0.f, 0.f, 0.f, 0.f};     // (left open, they are carried from tile to tile: 24 registers over the K loop, whose staging addresses then sat in scratch — each wait for one was a wait for the whole ring; 32768 x 4096 x 1024: 319 -> 259 us)
-                    if (rot) {
+                    if (head0 < epi.H + epi.KVH) {                        // q and k heads rotate, v heads pass through
 #pragma unroll
                         for (int hh = 0; hh < 2; ++hh) {
                             cs[kk][hh] = *reinterpret_cast<const float4_t *>(epi.cos_t + (int64_t)pos * hd2 + pcc * 8 + hh * 4);
                             sn[kk][hh] = *reinterpret_cast<const float4_t *>(epi.sin_t + (int64_t)pos * hd2 + pcc * 8 + hh * 4);
                         }
                     }
+                }
+            }
+            if constexpr (EPI == GEPI_QKN) {
+#pragma unroll
+                for (int hh = 0; hh < HN; ++hh) {
+                    const half_t *w = head0 + hh < epi.H ? epi.qn_w : epi.kn_w;
+                    g1[hh] = *reinterpret_cast<const half8_t *>(w + pcc * 8); g2[hh] = *reinterpret_cast<const half8_t *>(w + (hp + pcc) * 8);
                 }
             }
             __syncthreads();
@@ -447,33 +457,38 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__
                 __syncthreads();
                 continue;
             }
-            if (EPI == GEPI_ROPE) {
+            if (g_rope(EPI)) {
 #pragma unroll
-                for (int kk = 0; kk < 4; ++kk) {
-                    const int row = (tid >> 4) + kk * 32, m = m0 + hB * 128 + row;
-                    const half8_t x1 = *reinterpret_cast<const half8_t *>(scratch + row * (OUTC * 2) + ((ch1 ^ (row & 15)) << 4));
-                    const half8_t x2 = *reinterpret_cast<const half8_t *>(scratch + row * (OUTC * 2) + ((ch2 ^ (row & 15)) << 4));
-                    half8_t o1 = x1, o2 = x2;
-                    if (rot) {
+                for (int kk = 0; kk < PASSES; ++kk) {
+                    const int row = prow + kk * RPP, m = m0 + hB * 128 + row;
 #pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            const float a = (float)x1[e], b = (float)x2[e], cc = cs[kk][e >> 2][e & 3], ss = sn[kk][e >> 2][e & 3];
-                            o1[e] = to_half_rn(mul_sub_unfused(a, cc, b, ss));
-                            o2[e] = to_half_rn(mul_add_unfused(b, cc, a, ss));
+                    for (int hh = 0; hh < HN; ++hh) {
+                        const int rhead = head0 + hh, ch1 = hh * 2 * hp + pcc, ch2 = ch1 + hp;
+                        const bool rot = rhead < epi.H + epi.KVH;
+                        half8_t x1 = *reinterpret_cast<const half8_t *>(scratch + row * (OUTC * 2) + ((ch1 ^ (row & 15)) << 4));
+                        half8_t x2 = *reinterpret_cast<const half8_t *>(scratch + row * (OUTC * 2) + ((ch2 ^ (row & 15)) << 4));
+                        half8_t o1 = x1, o2 = x2;
+                        if (rot) {
+                            if constexpr (EPI == GEPI_QKN) head_norm<hp>(x1, x2, g1[hh], g2[hh], epi.qk_eps);
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) {
+                                const float a = (float)x1[e], b = (float)x2[e], cc = cs[kk][e >> 2][e & 3], ss = sn[kk][e >> 2][e & 3];
+                                o1[e] = to_half_rn(mul_sub_unfused(a, cc, b, ss));
+                                o2[e] = to_half_rn(mul_add_unfused(b, cc, a, ss));
+                            }
                         }
-                    }
-                    if (m >= T) continue;
-                    half_t *yrow = y + (int64_t)m * ldy + bx * OUTC;
-                    if (rhead < epi.H || !epi.kv_cache_only) {
-                        *reinterpret_cast<half8_t *>(yrow + ch1 * 8) = o1;
-                        *reinterpret_cast<half8_t *>(yrow + ch2 * 8) = o2;
-                    }
-                    if (rhead >= epi.H && rslot[kk] >= 0) {
-                        const bool is_k = rhead < epi.H + epi.KVH;
-                        const int kvh = is_k ? rhead - epi.H : rhead - epi.H - epi.KVH;
-                        half_t *crow = (is_k ? epi.kc : epi.vc) + ((int64_t)rslot[kk] * epi.KVH + kvh) * RD;
-                        *reinterpret_cast<half8_t *>(crow + pcc * 8) = o1;
-                        *reinterpret_cast<half8_t *>(crow + (hp + pcc) * 8) = o2;
+                        if (m >= T) continue;
+                        half_t *yrow = y + (int64_t)m * ldy + bx * OUTC;
+                        if (rhead < epi.H || !epi.kv_cache_only) {
+                            *reinterpret_cast<half8_t *>(yrow + ch1 * 8) = o1;
+                            *reinterpret_cast<half8_t *>(yrow + ch2 * 8) = o2;
+                        }
+                        if (rhead >= epi.H && rslot[kk] >= 0) {
+                            const int kvh = rot ? rhead - epi.H : rhead - epi.H - epi.KVH;
+                            half_t *crow = (rot ? epi.kc : epi.vc) + ((int64_t)rslot[kk] * epi.KVH + kvh) * RD;
+                            *reinterpret_cast<half8_t *>(crow + pcc * 8) = o1;
+                            *reinterpret_cast<half8_t *>(crow + (hp + pcc) * 8) = o2;
+                        }
                     }
                 }
                 __syncthreads();
@@ -509,7 +524,7 @@ static int g256_prepare() {                                               // 128
                          reinterpret_cast<const void *>(&gemm256_kernel<GEPI_RESID>), reinterpret_cast<const void *>(&gemm256_kernel<GEPI_LMHEAD>),
                          reinterpret_cast<const void *>(&gemm256_kernel<GEPI_F16, 0, true>), reinterpret_cast<const void *>(&gemm256_kernel<GEPI_SILU, 0, true>),
                          reinterpret_cast<const void *>(&gemm256_kernel<GEPI_RELU2>), reinterpret_cast<const void *>(&gemm256_kernel<GEPI_GELU>),
-                         reinterpret_cast<const void *>(&gemm256_kernel<GEPI_GELU_ERF>)};
+                         reinterpret_cast<const void *>(&gemm256_kernel<GEPI_GELU_ERF>), reinterpret_cast<const void *>(&gemm256_kernel<GEPI_QKN, 128>)};
     for (const void *f : fns) {
         hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * G_BUF + 4096);
         if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "gemm256: hipFuncSetAttribute: %s", hipGetErrorString(e));
@@ -618,7 +633,8 @@ int gemm256_gelu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_
 }
 int gemm256_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D,
                            const int64_t *positions, const int32_t *slots, const float *cos_t, const float *sin_t, half_bits *qkv,
-                           half_bits *k_cache, half_bits *v_cache, hipStream_t s, bool kv_cache_only) {
+                           half_bits *k_cache, half_bits *v_cache, hipStream_t s, bool kv_cache_only, const QkNorm *norm) {
+    if (norm && D != 128) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm256_qkv_rope_store: head norms with D=%ld", (long)D);
     if (!gemm256_rope_ok(T, K, H, KVH, D, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm256_qkv_rope_store: T=%ld K=%ld D=%ld", (long)T, (long)K, (long)D);
     if (int rc = g256_prepare()) return rc;
     const int64_t N = (H + 2 * KVH) * D;
@@ -627,7 +643,11 @@ int gemm256_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, 
     e.H = (int32_t)H; e.KVH = (int32_t)KVH; e.D = (int32_t)D;
     e.kv_cache_only = (kv_cache_only && slots && k_cache && v_cache) ? 1 : 0;
     const int tx = (int)(N / 256), tt = tx * (int)((T + 255) / 256);
-    if (D == 128)
+    if (norm) {
+        e.qn_w = (const half_t *)norm->q_w; e.kn_w = (const half_t *)norm->k_w; e.qk_eps = norm->eps;
+        gemm256_kernel<GEPI_QKN, 128><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF + 4096, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
+                                                                                                  (int)N, (int)N, (half_t *)qkv, e, tx, tt / tx, g256_cg(tx, tt / tx, true));
+    } else if (D == 128)
         gemm256_kernel<GEPI_ROPE, 128><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF + 4096, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
                                                                                                   (int)N, (int)N, (half_t *)qkv, e, tx, tt / tx, g256_cg(tx, tt / tx, true));
     else

@@ -28,7 +28,7 @@
 
 namespace nvr { namespace NVR_DT_NS {
 
-enum { TEPI_F16 = 0, TEPI_SILU = 2, TEPI_ROPE = 3, TEPI_LMHEAD = 4, TEPI_SLAB = 5, TEPI_RESID = 6 };     // RESID: y <- y + x.W^T, the product rounded first
+enum { TEPI_F16 = 0, TEPI_SILU = 2, TEPI_ROPE = 3, TEPI_LMHEAD = 4, TEPI_SLAB = 5, TEPI_RESID = 6, TEPI_QKN = 7 };     // RESID: y <- y + x.W^T, the product rounded first; QKN: heads of 128, RMSNorm over the columns of every q and k head, rotation, store
 
 // Where a launch's tiles lie: nx column tiles (W rows) x ny token tiles x nz k-slices, numbered slice by slice, within a slice in strips of `width` column tiles, within a strip
 // token tile by token tile.  Workgroups are dealt to the 8 XCDs in turn and each XCD has an L2 of its own, so XCD c takes the c-th eighth of that line: a compact block of tiles,
@@ -58,6 +58,7 @@ struct TileEpi {
     // TEPI_SLAB: k-slice z owns k in [z*kslice, (z+1)*kslice) and writes its f32 partial tile to slabs[z][T][N]
     float *slabs; int64_t slab_stride; int32_t kslice;
     int32_t gelu;                          // TEPI_SILU: gelu (tanh form) instead of silu
+    const half_t *qn_w, *kn_w; float qk_eps;      // TEPI_QKN: the norms' weights
     TileMap map;
     int32_t tiled;                         // W is the copy [rows/16][K/32][16][32] (retile_weight; TEPI_ROPE: its 16-row tiles are the n-tiles)
 };
@@ -154,19 +155,22 @@ __global__ __launch_bounds__(256, 2) void gemm_tiled_kernel(const half_t *__rest
     // TEPI_ROPE: the epilogue's inputs arrive UNDER the K loop instead of as three dependent round trips behind it (position -> cos / sin row -> rotate; cache
     // slot -> store).  Positions and slots are requested here, in front of the first operand tile, the cos / sin pieces once the positions are in.  A wave's four
     // n-tiles need 128 consecutive bytes of each table per token; lanes q and q + 2 need the same ones, so each requests two n-tiles' pieces and they trade them.
-    constexpr bool ROPE = EPI == TEPI_ROPE;
+    // TEPI_QKN: a workgroup's columns are one head; behind the K loop a thread takes row j * 32 + tid / 8 and the pair of pieces tid % 8 (its positions, cosines, sines and norm weights are
+    // requested here in the same way).
+    constexpr bool QKN = EPI == TEPI_QKN, ROPE = EPI == TEPI_ROPE || QKN;
     int64_t rope_pos[MT];
     int rope_slot[MT];
     float4_t pre_cs[MT][2], pre_sn[MT][2];
-    const int tph = ROPE ? epi.D / 16 : 1, tsh = 31 - __clz(tph), heads = epi.H + 2 * epi.KVH;      // n-tiles per head: 1, 2, 4 or 8
-    const int rope_head = ROPE ? (at.x * 8 + wn * 4) >> tsh : 0;          // the head of the first of this wave's four n-tiles
+    const int tph = EPI == TEPI_ROPE ? epi.D / 16 : 1, tsh = 31 - __clz(tph), heads = epi.H + 2 * epi.KVH;      // n-tiles per head: 1, 2, 4 or 8
+    const int rope_head = QKN ? at.x : ROPE ? (at.x * 8 + wn * 4) >> tsh : 0;          // the head of the first of this wave's four n-tiles
     const bool rope_rot = ROPE && rope_head < epi.H + epi.KVH;
+    half8_t norm_w[2];
     if (ROPE) {
 #pragma unroll
         for (int j = 0; j < MT; ++j) {
             // (as inline asm: a compiler-visible load makes hipcc drain vmcnt(0) at its first use, operand tiles in flight included; the values are complete
             //  once the first operand tile is, which is younger — see the pin there)
-            const int m = m0 + wm * (16 * MT) + j * 16 + r, mc = m < T ? m : T - 1;
+            const int m = m0 + (QKN ? j * 32 + ((int)threadIdx.x >> 3) : wm * (16 * MT) + j * 16 + r), mc = m < T ? m : T - 1;
             const int64_t *src = epi.pos + mc;
             asm volatile("global_load_dwordx2 %0, %1, off" : "=v"(rope_pos[j]) : "v"(src) : "memory");
             const int32_t *ss = epi.slots ? epi.slots + mc : reinterpret_cast<const int32_t *>(src);      // (no branch: a value in flight would be copied at its end)
@@ -218,7 +222,22 @@ __global__ __launch_bounds__(256, 2) void gemm_tiled_kernel(const half_t *__rest
             if (!epi.slots) rope_slot[j] = -1;
         }
     }
-    if (rope_rot) {
+    constexpr int PRE = QKN && MT == 4 ? 2 : MT;                          // (registers: the 128-token tile's other two behind the K loop)
+    auto request_angles = [&](int j) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int64_t at_pos = rope_pos[j] * 64 + (threadIdx.x & 7) * 8 + u * 4;
+            pre_cs[j][u] = *reinterpret_cast<const float4_t *>(epi.cos_t + at_pos);
+            pre_sn[j][u] = *reinterpret_cast<const float4_t *>(epi.sin_t + at_pos);
+        }
+    };
+    if (QKN && rope_rot) {
+        const half_t *w = (rope_head < epi.H ? epi.qn_w : epi.kn_w) + (threadIdx.x & 7) * 8;
+        norm_w[0] = *reinterpret_cast<const half8_t *>(w); norm_w[1] = *reinterpret_cast<const half8_t *>(w + 64);
+#pragma unroll
+        for (int j = 0; j < PRE; ++j) request_angles(j);
+    }
+    if (!QKN && rope_rot) {
         const int half_d = epi.D / 2;
 #pragma unroll
         for (int j = 0; j < MT; ++j)
@@ -250,7 +269,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tiled_kernel(const half_t *__rest
         first_half();
         // K-tile kt + 1 has landed once at most the 4 + MT requests per thread of each of the NS - 2 younger K-tiles are outstanding (the cos / sin requests of a rotating
         // TEPI_ROPE wave are younger than K-tiles 1 .. NS - 1 and may stay in flight with them)
-        if (rope_rot && kt + 1 < NS) wait_requests<(NS - 2) * (4 + MT) + 4 * MT>();
+        if (rope_rot && kt + 1 < NS) wait_requests<(NS - 2) * (4 + MT) + 4 * PRE + (QKN ? 2 : 0)>();
         else wait_requests<(NS - 2) * (4 + MT)>();
         __builtin_amdgcn_s_barrier();                                     // every thread's pieces of K-tile kt + 1 are in, and every wave has read K-tile kt: its slot is free
         __builtin_amdgcn_sched_barrier(0);
@@ -313,6 +332,51 @@ __global__ __launch_bounds__(256, 2) void gemm_tiled_kernel(const half_t *__rest
             if (v > bv || (v == bv && i2 < bi)) { bv = v; bi = i2; }
             epi.pval[(int64_t)at.x * T + m0 + threadIdx.x] = bv;
             epi.pidx[(int64_t)at.x * T + m0 + threadIdx.x] = bi;
+        }
+        return;
+    }
+    if constexpr (QKN) {
+        // the products, rounded, as [token][16 pieces ^ token & 15] over the operand buffers; then every row's norm, rotation and stores (head_norm: 8 lanes a row)
+        if (PRE < MT && rope_rot) {
+#pragma unroll
+            for (int j = PRE; j < MT; ++j) request_angles(j);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const int ml = wm * (16 * MT) + j * 16 + r;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int col = wn * 64 + i * 16 + q * 4;
+                *reinterpret_cast<half4_t *>(smem + ml * 256 + ((((col >> 3) ^ (ml & 15)) << 4) | ((col & 4) << 1))) =
+                    (half4_t){(half_t)acc[i][j][0], (half_t)acc[i][j][1], (half_t)acc[i][j][2], (half_t)acc[i][j][3]};
+            }
+        }
+        __syncthreads();
+        const int pc = threadIdx.x & 7;
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const int ml = j * 32 + ((int)threadIdx.x >> 3), m = m0 + ml;
+            half8_t x1 = *reinterpret_cast<const half8_t *>(smem + ml * 256 + ((pc ^ (ml & 15)) << 4));
+            half8_t x2 = *reinterpret_cast<const half8_t *>(smem + ml * 256 + (((8 + pc) ^ (ml & 15)) << 4));
+            if (rope_rot) {
+                head_norm<8>(x1, x2, norm_w[0], norm_w[1], epi.qk_eps);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float a = (float)x1[e], b = (float)x2[e], cc = pre_cs[j][e >> 2][e & 3], sn = pre_sn[j][e >> 2][e & 3];
+                    x1[e] = to_half_rn(mul_sub_unfused(a, cc, b, sn));
+                    x2[e] = to_half_rn(mul_add_unfused(b, cc, a, sn));
+                }
+            }
+            if (m >= T) continue;
+            if (rope_head < epi.H || !epi.kv_cache_only) {
+                half_t *row = y + (int64_t)m * N + rope_head * 128 + pc * 8;
+                *reinterpret_cast<half8_t *>(row) = x1; *reinterpret_cast<half8_t *>(row + 64) = x2;
+            }
+            if (rope_head >= epi.H && rope_slot[j] >= 0) {
+                half_t *row = (rope_rot ? epi.kc : epi.vc) + ((int64_t)rope_slot[j] * epi.KVH + rope_head - epi.H - (rope_rot ? 0 : epi.KVH)) * 128 + pc * 8;
+                *reinterpret_cast<half8_t *>(row) = x1; *reinterpret_cast<half8_t *>(row + 64) = x2;
+            }
         }
         return;
     }
@@ -589,7 +653,7 @@ int gemm_tiled_prepare() {
     { hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tiled_kernel<EPI_, NS_, MT_>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(NS_ * BYTES_)); \
       if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "gemm_tiled: LDS opt-in failed: %s", hipGetErrorString(e)); }
 #define NVR_TILED_ATTR(EPI_) NVR_TILED_ATTR1(EPI_, 3, 4, kStageBytes) NVR_TILED_ATTR1(EPI_, 4, 2, kStageBytes64) NVR_TILED_ATTR1(EPI_, 3, 2, kStageBytes64) NVR_TILED_ATTR1(EPI_, 4, 1, kStageBytes32)
-    NVR_TILED_ATTR(TEPI_F16) NVR_TILED_ATTR(TEPI_SILU) NVR_TILED_ATTR(TEPI_ROPE) NVR_TILED_ATTR(TEPI_LMHEAD) NVR_TILED_ATTR(TEPI_SLAB) NVR_TILED_ATTR(TEPI_RESID)
+    NVR_TILED_ATTR(TEPI_F16) NVR_TILED_ATTR(TEPI_SILU) NVR_TILED_ATTR(TEPI_ROPE) NVR_TILED_ATTR(TEPI_LMHEAD) NVR_TILED_ATTR(TEPI_SLAB) NVR_TILED_ATTR(TEPI_RESID) NVR_TILED_ATTR(TEPI_QKN)
 #undef NVR_TILED_ATTR
 #undef NVR_TILED_ATTR1
     if (hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tiled_silu96_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, RING96 * S96_BUF) != hipSuccess)
@@ -659,15 +723,19 @@ int gemm_tiled_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int
 }
 int gemm_tiled_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D,
                               const int64_t *positions, const int32_t *slots, const float *cos_t, const float *sin_t, half_bits *qkv,
-                              half_bits *k_cache, half_bits *v_cache, hipStream_t s, const half_bits *Wt, bool kv_cache_only) {
+                              half_bits *k_cache, half_bits *v_cache, hipStream_t s, const half_bits *Wt, bool kv_cache_only, const QkNorm *norm) {
     const int64_t N = (H + 2 * KVH) * D;
+    if (norm && D != 128) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_qkv_rope_store: head norms with D=%ld", (long)D);
     if (!gemm_tiled_ok(T, K, N, ldx) || D % 16 || 128 % D) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_qkv_rope_store: T=%ld K=%ld D=%ld", (long)T, (long)K, (long)D);
     TileEpi e{};
     e.pos = positions; e.slots = slots; e.cos_t = cos_t; e.sin_t = sin_t; e.kc = (half_t *)k_cache; e.vc = (half_t *)v_cache;
     e.H = (int32_t)H; e.KVH = (int32_t)KVH; e.D = (int32_t)D;
     e.kv_cache_only = kv_cache_only && slots && k_cache && v_cache;
     if (int rc = gemm_tiled_prepare()) return rc;
-    tiled_launch<TEPI_ROPE>((N / 16 + 7) / 8, 1, x, ldx, W, Wt, T, K, N, N, (half_t *)qkv, e, s);
+    if (norm) {
+        e.qn_w = (const half_t *)norm->q_w; e.kn_w = (const half_t *)norm->k_w; e.qk_eps = norm->eps;
+        tiled_launch<TEPI_QKN>(N / BN, 1, x, ldx, W, Wt, T, K, N, N, (half_t *)qkv, e, s);
+    } else tiled_launch<TEPI_ROPE>((N / 16 + 7) / 8, 1, x, ldx, W, Wt, T, K, N, N, (half_t *)qkv, e, s);
     return tiled_check("gemm_tiled_qkv_rope_store");
 }
 

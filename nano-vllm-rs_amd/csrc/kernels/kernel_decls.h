@@ -87,6 +87,11 @@ int linear_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, i
                           int64_t KVH, int64_t D, const int64_t *positions, const int32_t *slots, const float *cos_t,
                           const float *sin_t, half_bits *qkv, half_bits *k_cache, half_bits *v_cache, hipStream_t s,
                           const half_bits *Wt = nullptr, bool kv_cache_only = false);
+// The same with the head norms, for the shapes that linear() multiplies on LDS tiles and heads of 128: each output has the bits of linear() with rope_store_kv behind it.  Wt: mode 0
+bool linear_qkv_norm_rope_store_ok(int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D, int64_t ldx);
+int linear_qkv_norm_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D, const int64_t *positions, const int32_t *slots,
+                               const float *cos_t, const float *sin_t, half_bits *qkv, half_bits *k_cache, half_bits *v_cache, const QkNorm &norm, hipStream_t s,
+                               const half_bits *Wt = nullptr, bool kv_cache_only = false);
 // kv_cache_only: the caller's attention reads K / V from the caches only, so the k and v columns of qkv need not be written (the 256^2
 // prefill kernel then skips those stores: a third of its output bytes; the other routes write them anyway)
 
@@ -123,7 +128,8 @@ int gemm_tiled_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int
                         hipStream_t s, bool gelu = false, const half_bits *Wt = nullptr);
 int gemm_tiled_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH,
                               int64_t D, const int64_t *positions, const int32_t *slots, const float *cos_t, const float *sin_t,
-                              half_bits *qkv, half_bits *k_cache, half_bits *v_cache, hipStream_t s, const half_bits *Wt = nullptr, bool kv_cache_only = false);
+                              half_bits *qkv, half_bits *k_cache, half_bits *v_cache, hipStream_t s, const half_bits *Wt = nullptr, bool kv_cache_only = false,
+                              const QkNorm *norm = nullptr);   // norm: Wt in the plain order of rows (retile_weight mode 0)
 
 // 256x256x64 eight-wave MFMA GEMM (T >= 256, N % 256 == 0 / I % 128 == 0 / whole heads per 256 rows): same results
 // layout and epilogues; preferred over gemm_tiled when its shape test passes
@@ -150,7 +156,7 @@ int gemm256_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_
 int gemm256_gelu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s);
 int gemm256_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D,
                            const int64_t *positions, const int32_t *slots, const float *cos_t, const float *sin_t, half_bits *qkv,
-                           half_bits *k_cache, half_bits *v_cache, hipStream_t s, bool kv_cache_only = false);
+                           half_bits *k_cache, half_bits *v_cache, hipStream_t s, bool kv_cache_only = false, const QkNorm *norm = nullptr);
 
 size_t attn_workspace_bytes(int64_t nq, int64_t H, int64_t D, int64_t max_ctx);
 int64_t attn_brief_context(int64_t nq, int64_t H, int64_t KVH);   // contexts up to it (0: none) have a decode attention of their own: worth a captured step of their own

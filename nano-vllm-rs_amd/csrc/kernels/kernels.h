@@ -55,6 +55,9 @@ struct AttnArgs {
     const int64_t *pos; const int32_t *slots; const float *cos_t, *sin_t;
 };
 
+// RMSNorm over the columns of every q and k head in front of the rotation: weights [D] each
+struct QkNorm { const half_bits *q_w, *k_w; float eps; };
+
 // MFMA flash prefill attention.  A tile = up to 64/G consecutive query positions of one sequence.
 struct FlashTile { int32_t q_row0, nq, pos0, kv_ref; };   // first q row, #queries, absolute position of the first query,
                                                           // contiguous: first key row of the sequence / paged: block-table row

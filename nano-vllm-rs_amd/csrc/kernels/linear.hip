@@ -620,6 +620,20 @@ int linear_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, i
     return launch_check("linear_qkv_rope_store");
 }
 
+// As linear() routes the plain product: a last norm's launch behind it read and wrote every row once more (509 rows of 16 + 8 + 8 heads 4.2 us, 3815 rows 14.6, 3062 rows of 32 + 8 + 8 18.7).
+bool linear_qkv_norm_rope_store_ok(int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D, int64_t ldx) {
+    const int64_t N = (H + 2 * KVH) * D;
+    return D == 128 && K % 32 == 0 && gemm_tiled_ok(T, K, N, ldx) && ((gemm256_rope_ok(T, K, H, KVH, D, ldx) && rows_on_256(T, K, N) > 0) || !stream_preferred(T, N));
+}
+int linear_qkv_norm_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D, const int64_t *positions, const int32_t *slots,
+                               const float *cos_t, const float *sin_t, half_bits *qkv, half_bits *k_cache, half_bits *v_cache, const QkNorm &norm, hipStream_t s, const half_bits *Wt, bool kv_cache_only) {
+    const uintptr_t at = (uintptr_t)qkv | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)norm.q_w | (uintptr_t)norm.k_w | (uintptr_t)cos_t | (uintptr_t)sin_t;
+    if (!linear_qkv_norm_rope_store_ok(T, K, H, KVH, D, ldx) || (at & 15)) return nvr::fail(NVR_ERR_UNSUPPORTED, "linear_qkv_norm_rope_store: T=%ld K=%ld D=%ld", (long)T, (long)K, (long)D);
+    const int64_t N = (H + 2 * KVH) * D, r = gemm256_rope_ok(T, K, H, KVH, D, ldx) ? rows_on_256(T, K, N) : 0;
+    if (r > 0) if (int rc = gemm256_qkv_rope_store(x, ldx, W, r, K, H, KVH, D, positions, slots, cos_t, sin_t, qkv, k_cache, v_cache, s, kv_cache_only, &norm)) return rc;
+    return r == T ? 0 : gemm_tiled_qkv_rope_store(x + r * ldx, ldx, W, T - r, K, H, KVH, D, positions + r, slots ? slots + r : nullptr, cos_t, sin_t, qkv + r * N, k_cache, v_cache, s, Wt, kv_cache_only, &norm);
+}
+
 // ---- products of a decode step of few rows whose workgroups form RMSNorm(h + slabs) themselves (linear_skinny_kernel, NORM)
 // (three and four rows: from the width on at which the products behind a launch of its own split k over the same eight waves, so that the step's bits are theirs)
 bool norm_linear_ok(int64_t T, int64_t K, int64_t S) { return T >= 1 && T <= NORM_ROWS && (T <= 2 || waves_for(K) == 8) && K % 256 == 0 && T * K <= NORM_ELEMS && (S == 2 || S == 4); }

@@ -848,6 +848,12 @@ int nvr_model_runner::forward_prefill_two(int64_t T, int64_t B) {
     return NVR_OK;
 }
 
+// Whether the qkv product of a step of T rows norms, rotates and stores them (models with q / k norms): on LDS tiles; a decode step's only where the attention does not form them itself (at most
+// three (row, kv head) pairs for two CUs).
+bool nvr_model_runner::qkv_norms_rows(int64_t T, bool is_prefill) const {
+    return mc.qk_norm && !mc.use_bias && KD(linear_qkv_norm_rope_store_ok(T, Hd, H, KVH, D, Hd)) && (is_prefill || 2 * T * KVH > 3 * (int64_t)num_cus);
+}
+
 // Qwen3Model::forward, src/models/qwen3.rs:487-505; layer wiring :372-392; attention :208-240; MLP :305-314.
 int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max_ctx) {
     hipStream_t st = stream;
@@ -874,11 +880,16 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
         const k::NormIn before{hc, slabs, T * Hd, (int32_t)owed, w.ln1, mc.rms_norm_eps, hn};
         if (l == 0 && !embed_norm) RC(KD(rmsnorm(h, w.ln1, mc.rms_norm_eps, T, Hd, n, st)));   // later layers: see down_proj
         if (mc.qk_norm || mc.use_bias) {         // A-27: the head norms sit between the projection and RoPE: plain GEMM, then one
+            if (qkv_norms_rows(T, is_prefill)) {
+                RC(KD(linear_qkv_norm_rope_store(n, Hd, w.qkv, T, Hd, H, KVH, D, pos, slots, cos_t, sin_t, qkv, k_cache(l), v_cache(l), k::QkNorm{w.q_norm, w.k_norm, mc.rms_norm_eps}, st, qkv_t,
+                                                 is_prefill && n_tiles > 0 && (prefill_paged || prefill_kv_cache))));
+            } else {
             if (owed) { RC(KD(norm_linear(before, w.qkv, T, Hd, QKV, qkv, st, qkv_t))); std::swap(hc, hn); }
             else RC(KD(linear(n, Hd, w.qkv, T, Hd, QKV, qkv, false, st, qkv_t)));                  // norm + RoPE + KV-store launch
             if (mc.use_bias) RC(KD(add_bias(qkv, w.qkv_b, T, QKV, st)));                            // A-30: the bias precedes the norms and RoPE (qwen3.rs:208-222)
             if (is_prefill || !mc.qk_norm)                                                          // (a decode step's rows are normed, rotated and stored by its attention)
                 RC(KD(rope_store_kv(qkv, pos, slots, T, H, KVH, D, cos_t, sin_t, k_cache(l), v_cache(l), st, w.q_norm, w.k_norm, mc.rms_norm_eps)));
+            }
         } else if (owed) {
             RC(KD(norm_linear_qkv_rope_store(before, w.qkv, T, Hd, H, KVH, D, pos, slots, cos_t, sin_t, qkv, k_cache(l), v_cache(l), st, qkv_t)));
             std::swap(hc, hn);
@@ -910,7 +921,7 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
             a.block_size = (int32_t)block_size; a.workspace = attn_ws; a.workspace_bytes = attn_ws_bytes; a.tickets = attn_tickets;
             a.shared_len = (int32_t)decode_shared_len;
             a.ragged = decode_ragged;
-            if (mc.qk_norm) { a.qn_w = w.q_norm; a.kn_w = w.k_norm; a.qk_eps = mc.rms_norm_eps; a.pos = pos; a.slots = slots; a.cos_t = cos_t; a.sin_t = sin_t; }
+            if (mc.qk_norm && !qkv_norms_rows(T, false)) { a.qn_w = w.q_norm; a.kn_w = w.k_norm; a.qk_eps = mc.rms_norm_eps; a.pos = pos; a.slots = slots; a.cos_t = cos_t; a.sin_t = sin_t; }
             if (decode_shared_len > 0 && decode_shared_rows < T) {     // a group inside the batch: per-row kv0, member rows, member count
                 a.shared_kv0 = (const int32_t *)(in_dev + off_dec + dof_skv0); a.shared_rows = (const int32_t *)(in_dev + off_dec + dof_srows);
                 a.shared_count = (const int32_t *)(in_dev + off_dec + dof_scount);
@@ -1011,15 +1022,16 @@ int nvr_model_runner::execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill
         // (gemm256 skips the k / v columns of the qkv buffer: -9 % on that GEMM).  If every sequence's blocks are consecutive (blocks come off
         // the free list in order until it has been recycled) token p of a sequence sits at cache row table[0] * bs + p and the kernel runs in
         // its contiguous form (-1.7 ms of a 32 x 1024 prefill); otherwise it walks the block tables like a prefill behind a cached prefix
-        // (-0.5 ms).  q/k-norm models keep the qkv buffer (their norm + RoPE launch writes both anyway).
-        prefill_kv_cache = flash_ok && !prefill_paged && !mc.qk_norm && !mc.use_bias;
+        // (-0.5 ms).  q/k-norm models keep the qkv buffer where a launch of its own norms, rotates and stores the rows (it writes both anyway).
+        const bool rows_stored = !mc.use_bias && (!mc.qk_norm || qkv_norms_rows(total, true));      // by the qkv product, in the caches alone where the attention reads them there
+        prefill_kv_cache = flash_ok && !prefill_paged && rows_stored;
         for (size_t b = 0; b < nseq && prefill_kv_cache; ++b) {
             const nvr_seq &sq = *seqs[b];
             const size_t nb = std::min(sq.block_table.size(), (size_t)(((int64_t)sq.len() + bs - 1) / bs));
             for (size_t j = 1; j < nb; ++j)
                 if (sq.block_table[j] != sq.block_table[j - 1] + 1) { prefill_kv_cache = false; break; }
         }
-        if (flash_ok && !prefill_paged && !mc.qk_norm && !mc.use_bias && !prefill_kv_cache) prefill_paged = true;
+        if (flash_ok && !prefill_paged && rows_stored && !prefill_kv_cache) prefill_paged = true;
         const int qb = flash_ok ? KD(flash_tile_positions((int)H, (int)KVH)) : 1;
         {   // the step's arrays back to back at the start of the arena (sized by THIS step's token count): one upload instead of seven
             size_t o = 0;

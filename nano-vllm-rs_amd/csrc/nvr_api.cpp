@@ -653,6 +653,13 @@ int nvr_qk_norm_rope_store_kv(nvr_half *qkv, const int64_t *pos, const int32_t *
     if (g_ops_f32) return nvr::kf::rope_store_kv(FP(qkv), pos, slots, T, H, KVH, D, c, sn, FP(kc), FP(vc), FP(qw), FP(kw), eps, (hipStream_t)s);
     return KO(rope_store_kv(qkv, pos, slots, T, H, KVH, D, c, sn, kc, vc, (hipStream_t)s, qw, kw, eps));
 }
+int nvr_linear_qkv_norm_rope_store(const nvr_half *x, int64_t ldx, const nvr_half *W, const nvr_half *Wt, int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D, const int64_t *pos,
+                                   const int32_t *slots, const float *c, const float *sn, const nvr_half *qw, const nvr_half *kw, float eps, nvr_half *qkv, nvr_half *kc, nvr_half *vc,
+                                   int kv_cache_only, void *s) {
+    NO_F32("nvr_linear_qkv_norm_rope_store");
+    if (!qw || !kw) return nvr::fail(NVR_ERR_INVALID_ARG, "nvr_linear_qkv_norm_rope_store: norm weights are null");
+    return KO(linear_qkv_norm_rope_store(x, ldx, W, T, K, H, KVH, D, pos, slots, c, sn, qkv, kc, vc, k::QkNorm{qw, kw, eps}, (hipStream_t)s, Wt, kv_cache_only != 0));
+}
 int nvr_rope_table(int64_t D, int64_t max_pos, double theta, float *cos_dev, float *sin_dev) {   // rotary_embedding.rs:74-119 (A-14)
     NVR_GUARD_BEGIN
     const int64_t half = D / 2;

@@ -101,6 +101,63 @@ def test_qk_norm_forms(T, H, KVH, D, shift):
     assert not kc[~seen].any() and not vc[~seen].any()
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("T,K,H,KVH", [(65, 1024, 16, 8), (97, 256, 16, 4), (200, 512, 8, 4), (509, 1024, 16, 8), (1000, 128, 16, 8), (1100, 1024, 5, 3), (2304, 256, 16, 8), (3062, 1024, 32, 8)])
+def test_qkv_product_with_head_norms(T, K, H, KVH, dtype):
+    """nvr_linear_qkv_norm_rope_store has the bits of nvr_linear_tiled with nvr_qk_norm_rope_store_kv behind it: tiles of 32, 64 and 128 rows, 256-row tiles, both in one product, ragged last
+    tiles, a tile of q and k heads; rows without a slot, of zeros, with an infinity, of the largest numbers; k and v rows in the caches alone leave their columns of qkv as they were."""
+    D, N, bf = 128, (H + 2 * KVH) * 128, dtype == "bfloat16"
+    rng = np.random.default_rng(T * 7 + K)
+
+    def bits(a):
+        a = np.ascontiguousarray(a, np.float32)
+        if not bf:
+            return a.astype(F16).view(np.uint16)
+        u = a.view(np.uint32)
+        return ((u + 0x7fff + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    x[3] = 0
+    x[5, 0] = np.inf
+    x[7] *= 1e4 if bf else 30.0
+    x[T - 1] *= 1e-3
+    xb, Wb = bits(x), bits(rng.standard_normal((N, K)) * K ** -0.5)
+    qw, kw = bits(1 + 0.3 * rng.standard_normal(D)), bits(1 + 0.3 * rng.standard_normal(D))
+    pos = rng.integers(0, 400, T).astype(np.int64)
+    slots = rng.permutation(2 * T)[:T].astype(np.int32)
+    slots[[2, T - 2]] = -1
+    cos, sin = oracle.rope_table(D, 512, 1e6)
+    l = nvr.lib()
+    d_x, d_W, d_qw, d_kw, d_pos, d_slots, d_cos, d_sin = (dev(a) for a in (xb, Wb, qw, kw, pos, slots, cos, sin))
+    d_Wt = nvr.DeviceBuffer(N * K * 2)
+    nvr.check(l.nvr_ops_set_dtype(dtype.encode()))
+    try:
+        nvr.check(l.nvr_retile_weight(d_W.ptr, d_Wt.ptr, N, K, 0, H, KVH, D, None))
+        out = []
+        for form in range(4):                                              # two launches; one; one from W alone; one with k and v in the caches alone
+            y, kc, vc = dev(np.full((T, N), 0x7b7b, np.uint16)), nvr.DeviceBuffer(2 * T * KVH * D * 2), nvr.DeviceBuffer(2 * T * KVH * D * 2)
+            kc.zero(); vc.zero()
+            if form == 0:
+                nvr.check(l.nvr_linear_tiled(d_x.ptr, K, d_W.ptr, d_Wt.ptr, T, K, N, y.ptr, 0, None))
+                nvr.check(l.nvr_qk_norm_rope_store_kv(y.ptr, d_pos.ptr, d_slots.ptr, T, H, KVH, D, d_cos.ptr, d_sin.ptr, d_qw.ptr, d_kw.ptr, 1e-6, kc.ptr, vc.ptr, None))
+            else:
+                nvr.check(l.nvr_linear_qkv_norm_rope_store(d_x.ptr, K, d_W.ptr, None if form == 2 else d_Wt.ptr, T, K, H, KVH, D, d_pos.ptr, d_slots.ptr, d_cos.ptr, d_sin.ptr, d_qw.ptr, d_kw.ptr, 1e-6,
+                                                           y.ptr, kc.ptr, vc.ptr, int(form == 3), None))
+            nvr.check(l.nvr_device_synchronize())
+            out.append((y.to_numpy((T, N), np.uint16), kc.to_numpy((2 * T, KVH * D), np.uint16), vc.to_numpy((2 * T, KVH * D), np.uint16)))
+        assert l.nvr_linear_qkv_norm_rope_store(d_x.ptr, K, d_W.ptr, None, 32, K, H, KVH, D, d_pos.ptr, d_slots.ptr, d_cos.ptr, d_sin.ptr, d_qw.ptr, d_kw.ptr, 1e-6, y.ptr, kc.ptr, vc.ptr, 0, None) == -10
+    finally:
+        nvr.check(l.nvr_ops_set_dtype(b"float16"))
+    want = out[0]
+    nan = 0x7f80 if bf else 0x7c00                                         # (a NaN is a NaN, whatever its bits)
+    canon = [[np.where((a & 0x7fff) > nan, 0x7fff, a) for a in o] for o in out]
+    for form in (1, 2):
+        for a, b in zip(canon[form], canon[0]):
+            assert np.array_equal(a, b), form
+    assert np.array_equal(canon[3][0][:, :H * D], canon[0][0][:, :H * D]) and (out[3][0][:, H * D:] == 0x7b7b).all()
+    assert np.array_equal(canon[3][1], canon[0][1]) and np.array_equal(canon[3][2], canon[0][2])
+    assert (want[1].any(1) | want[2].any(1)).sum() <= T - 2 and np.isfinite(x).sum() == x.size - 1
+
+
 @pytest.mark.parametrize("B,V", [(1, 65536), (1, 65535), (3, 151936), (1, 65539), (128, 65540), (129, 65540), (300, 64)])
 def test_greedy_rows_cut_into_parts(B, V):
     """The greedy choice of f32 logits rows: cut into parts over the grid (few long rows) or one workgroup per row (short rows, or many of them), through a
