@@ -32,9 +32,9 @@
 
 namespace nvr { namespace NVR_DT_NS {
 
-enum { GEPI_F16 = 0, GEPI_RESID = 1, GEPI_SILU = 2, GEPI_ROPE = 3, GEPI_LMHEAD = 4, GEPI_RELU2 = 5, GEPI_GELU = 6, GEPI_GELU_ERF = 7, GEPI_QKN = 8 };   // GELU_ERF: y = gelu(x·Wᵀ) with the error function (from the unrounded product); RELU2: y = max(x·Wᵀ, 0)² (the product rounded to 16 bits first, as the unfused pair of launches does)
+enum { GEPI_F16 = 0, GEPI_RESID = 1, GEPI_SILU = 2, GEPI_ROPE = 3, GEPI_LMHEAD = 4, GEPI_RELU2 = 5, GEPI_GELU = 6, GEPI_GELU_ERF = 7, GEPI_QKN = 8, GEPI_CLAMP = 9 };   // GELU_ERF: y = gelu(x·Wᵀ) with the error function (from the unrounded product); RELU2: y = max(x·Wᵀ, 0)² (the product rounded to 16 bits first, as the unfused pair of launches does)
 constexpr bool g_rope(int epi) { return epi == GEPI_ROPE || epi == GEPI_QKN; }      // QKN: RMSNorm over the columns of every q and k head in front of the rotation
-constexpr bool g_glu(int epi) { return epi == GEPI_SILU || epi == GEPI_GELU; }      // gate and up rows in one tile, out = act(gate) * up (GELU: the tanh form)
+constexpr bool g_glu(int epi) { return epi == GEPI_SILU || epi == GEPI_GELU || epi == GEPI_CLAMP; }      // gate and up rows in one tile, out = act(gate) * up (GELU: the tanh form; CLAMP: clamped_unit_fast, rows of y ldo apart)
 //   // RESID: y is the residual stream: y <- fp16(y + fp16(x·Wᵀ)) (qwen3.rs:382,389)
 // LMHEAD (r06): the LM head over >= 128 rows (ParallelLMHead::compute_logits, embed_head.rs:292-306, + the greedy branch of Sampler::forward,
 // sampler.rs:109-112): W = the [V, hidden] head, nothing is written as fp16 — every tile leaves (max, lowest vocabulary index) of its 256
@@ -48,6 +48,7 @@ struct G256Epi {
     int32_t kv_cache_only;             // GEPI_ROPE: k and v rows go to the caches only (the attention that follows reads them there)
     float *logits; float *pval; int32_t *pidx;   // GEPI_LMHEAD: f32 logits [T][N] (nullable), arg-max partials [tiles_x][T]
     const half_t *qn_w, *kn_w; float qk_eps;     // GEPI_QKN: the norms' weights [D]
+    float limit, alpha; int64_t ldo;             // GEPI_CLAMP
     const int32_t *row_w; int64_t w_stride; const int32_t *rows_used;      // (rows_used, on the device: rows behind it are nobody's; null: all T) GRP (rows grouped by expert): row block rb of 256 rows multiplies the matrix W + row_w[rb] * w_stride
 };
 
@@ -221,7 +222,7 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__
 #define G256_W(NOMORE_) if (more) { G256_R_END(4) } else { G256_R_END(NOMORE_) }
 
     constexpr int OUTC = g_glu(EPI) ? 128 : 256;                  // output columns of a tile
-    const int64_t ldy = g_rope(EPI) ? (int64_t)(epi.H + 2 * epi.KVH) * RD : (int64_t)N;
+    const int64_t ldy = g_rope(EPI) ? (int64_t)(epi.H + 2 * epi.KVH) * RD : EPI == GEPI_CLAMP ? epi.ldo : (int64_t)N;
     constexpr int hd2 = g_rope(EPI) ? RD / 2 : 1;
 
     int tile_no = 0;
@@ -408,8 +409,11 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
                             const float gf = (float)to_half_rn(acc[0][i][hB][j][e]), uf = (float)to_half_rn(acc[1][i][hB][j][e]);
-                            const float sg = gate_factor(gf, EPI == GEPI_GELU);
-                            h[e] = to_half_rn(__fmul_rn(__fmul_rn(gf, sg), uf));
+                            if constexpr (EPI == GEPI_CLAMP) h[e] = to_half_rn(clamped_unit_fast(gf, uf, epi.limit, epi.alpha));
+                            else {
+                                const float sg = gate_factor(gf, EPI == GEPI_GELU);
+                                h[e] = to_half_rn(__fmul_rn(__fmul_rn(gf, sg), uf));
+                            }
                         }
                         put(ml, wn * 64 + i * 16 + q * 4, h);
                     }
@@ -524,7 +528,8 @@ static int g256_prepare() {                                               // 128
                          reinterpret_cast<const void *>(&gemm256_kernel<GEPI_RESID>), reinterpret_cast<const void *>(&gemm256_kernel<GEPI_LMHEAD>),
                          reinterpret_cast<const void *>(&gemm256_kernel<GEPI_F16, 0, true>), reinterpret_cast<const void *>(&gemm256_kernel<GEPI_SILU, 0, true>),
                          reinterpret_cast<const void *>(&gemm256_kernel<GEPI_RELU2>), reinterpret_cast<const void *>(&gemm256_kernel<GEPI_GELU>),
-                         reinterpret_cast<const void *>(&gemm256_kernel<GEPI_GELU_ERF>), reinterpret_cast<const void *>(&gemm256_kernel<GEPI_QKN, 128>)};
+                         reinterpret_cast<const void *>(&gemm256_kernel<GEPI_GELU_ERF>), reinterpret_cast<const void *>(&gemm256_kernel<GEPI_QKN, 128>),
+                         reinterpret_cast<const void *>(&gemm256_kernel<GEPI_CLAMP>)};
     for (const void *f : fns) {
         hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * G_BUF + 4096);
         if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "gemm256: hipFuncSetAttribute: %s", hipGetErrorString(e));
@@ -630,6 +635,16 @@ int gemm256_gelu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_
     gemm256_kernel<GEPI_GELU><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
                                                                                          (int)I, (int)(2 * I), (half_t *)out, G256Epi{}, tx, tt / tx, g256_cg(tx, tt / tx, false));
     return g256_check("gemm256_gelu_mul");
+}
+// the clamped gated unit, rows of out ldo apart
+int gemm256_clamped_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, float limit, float alpha, half_bits *out, int64_t ldo, hipStream_t s) {
+    if (!gemm256_silu_ok(T, K, I, ldx) || ldo % 8 || ldo < I) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm256_clamped_glu: T=%ld K=%ld I=%ld", (long)T, (long)K, (long)I);
+    if (int rc = g256_prepare()) return rc;
+    G256Epi e{}; e.limit = limit; e.alpha = alpha; e.ldo = ldo;
+    const int tx = (int)(I / 128), tt = tx * (int)((T + 255) / 256);
+    gemm256_kernel<GEPI_CLAMP><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
+                                                                                          (int)I, (int)(2 * I), (half_t *)out, e, tx, tt / tx, g256_cg(tx, tt / tx, false));
+    return g256_check("gemm256_clamped_glu");
 }
 int gemm256_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D,
                            const int64_t *positions, const int32_t *slots, const float *cos_t, const float *sin_t, half_bits *qkv,

@@ -28,7 +28,7 @@
 
 namespace nvr { namespace NVR_DT_NS {
 
-enum { TEPI_F16 = 0, TEPI_SILU = 2, TEPI_ROPE = 3, TEPI_LMHEAD = 4, TEPI_SLAB = 5, TEPI_RESID = 6, TEPI_QKN = 7 };     // RESID: y <- y + x.W^T, the product rounded first; QKN: heads of 128, RMSNorm over the columns of every q and k head, rotation, store
+enum { TEPI_F16 = 0, TEPI_SILU = 2, TEPI_ROPE = 3, TEPI_LMHEAD = 4, TEPI_SLAB = 5, TEPI_RESID = 6, TEPI_QKN = 7, TEPI_CLAMP = 8 };     // RESID: y <- y + x.W^T, the product rounded first; QKN: heads of 128, RMSNorm over the columns of every q and k head, rotation, store
 
 // Where a launch's tiles lie: nx column tiles (W rows) x ny token tiles x nz k-slices, numbered slice by slice, within a slice in strips of `width` column tiles, within a strip
 // token tile by token tile.  Workgroups are dealt to the 8 XCDs in turn and each XCD has an L2 of its own, so XCD c takes the c-th eighth of that line: a compact block of tiles,
@@ -59,6 +59,7 @@ struct TileEpi {
     float *slabs; int64_t slab_stride; int32_t kslice;
     int32_t gelu;                          // TEPI_SILU: gelu (tanh form) instead of silu
     const half_t *qn_w, *kn_w; float qk_eps;      // TEPI_QKN: the norms' weights
+    float limit, alpha; int64_t ldo;              // TEPI_CLAMP
     TileMap map;
     int32_t tiled;                         // W is the copy [rows/16][K/32][16][32] (retile_weight; TEPI_ROPE: its 16-row tiles are the n-tiles)
 };
@@ -83,10 +84,12 @@ __device__ __forceinline__ void wait_ring(int younger) {
     }
 }
 
+constexpr bool t_glu(int epi) { return epi == TEPI_SILU || epi == TEPI_CLAMP; }      // gate and up rows in one tile (CLAMP: clamped_unit_fast, rows of y ldo apart)
+
 // W row of local row r (0..15) of the workgroup's 16-row n-tile `t` (0..7)
 template <int EPI>
 __device__ __forceinline__ int tile_w_row(int bx, int t, int r, int N, const TileEpi &e) {
-    if (EPI == TEPI_SILU) {                       // N == I; the workgroup owns 64 output columns
+    if (t_glu(EPI)) {                             // N == I; the workgroup owns 64 output columns
         const int wn = t >> 2, nt = t & 3;
         return (nt >> 1) * N + bx * 64 + wn * 32 + (nt & 1) * 16 + r;
     }
@@ -101,7 +104,7 @@ __device__ __forceinline__ int tile_w_row(int bx, int t, int r, int N, const Til
 // the same n-tile in the tiled copy
 template <int EPI>
 __device__ __forceinline__ int tile_w_block(int bx, int t, int N) {
-    if (EPI == TEPI_SILU) return ((t & 3) >> 1) * (N >> 4) + bx * 4 + (t >> 2) * 2 + (t & 1);
+    if (t_glu(EPI)) return ((t & 3) >> 1) * (N >> 4) + bx * 4 + (t >> 2) * 2 + (t & 1);
     return bx * 8 + t;
 }
 
@@ -420,20 +423,23 @@ __global__ __launch_bounds__(256, 2) void gemm_tiled_kernel(const half_t *__rest
                 }
                 if (m < T && n < N) *reinterpret_cast<half8_t *>(y + (int64_t)m * N + n) = v8;
             }
-        } else if (EPI == TEPI_SILU) {
+        } else if (t_glu(EPI)) {
             half4_t h[2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {                                 // tiles i (gate) and i+2 (up), same 16 columns
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float gf = (float)to_half_rn(acc[i][j][e]), uf = (float)to_half_rn(acc[i + 2][j][e]);
-                    const float sg = gate_factor(gf, epi.gelu);
-                    h[i][e] = to_half_rn(__fmul_rn(__fmul_rn(gf, sg), uf));
+                    if constexpr (EPI == TEPI_CLAMP) h[i][e] = to_half_rn(clamped_unit_fast(gf, uf, epi.limit, epi.alpha));
+                    else {
+                        const float sg = gate_factor(gf, epi.gelu);
+                        h[i][e] = to_half_rn(__fmul_rn(__fmul_rn(gf, sg), uf));
+                    }
                 }
             }
             const half8_t v8 = pair8(h[0], h[1]);
             const int n = at.x * 64 + wn * 32 + col_in_pair;
-            if (m < T && n < N) *reinterpret_cast<half8_t *>(y + (int64_t)m * N + n) = v8;
+            if (m < T && n < N) *reinterpret_cast<half8_t *>(y + (int64_t)m * (EPI == TEPI_CLAMP ? epi.ldo : (int64_t)N) + n) = v8;
         } else {                                                          // TEPI_ROPE
             const int half_d = epi.D / 2;
             const int64_t ldy = (int64_t)heads * epi.D;
@@ -653,7 +659,7 @@ int gemm_tiled_prepare() {
     { hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tiled_kernel<EPI_, NS_, MT_>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(NS_ * BYTES_)); \
       if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "gemm_tiled: LDS opt-in failed: %s", hipGetErrorString(e)); }
 #define NVR_TILED_ATTR(EPI_) NVR_TILED_ATTR1(EPI_, 3, 4, kStageBytes) NVR_TILED_ATTR1(EPI_, 4, 2, kStageBytes64) NVR_TILED_ATTR1(EPI_, 3, 2, kStageBytes64) NVR_TILED_ATTR1(EPI_, 4, 1, kStageBytes32)
-    NVR_TILED_ATTR(TEPI_F16) NVR_TILED_ATTR(TEPI_SILU) NVR_TILED_ATTR(TEPI_ROPE) NVR_TILED_ATTR(TEPI_LMHEAD) NVR_TILED_ATTR(TEPI_SLAB) NVR_TILED_ATTR(TEPI_RESID) NVR_TILED_ATTR(TEPI_QKN)
+    NVR_TILED_ATTR(TEPI_F16) NVR_TILED_ATTR(TEPI_SILU) NVR_TILED_ATTR(TEPI_ROPE) NVR_TILED_ATTR(TEPI_LMHEAD) NVR_TILED_ATTR(TEPI_SLAB) NVR_TILED_ATTR(TEPI_RESID) NVR_TILED_ATTR(TEPI_QKN) NVR_TILED_ATTR(TEPI_CLAMP)
 #undef NVR_TILED_ATTR
 #undef NVR_TILED_ATTR1
     if (hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_tiled_silu96_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, RING96 * S96_BUF) != hipSuccess)
@@ -720,6 +726,13 @@ int gemm_tiled_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int
     TileEpi e{}; e.gelu = gelu ? 1 : 0;
     tiled_launch<TEPI_SILU>(I / 64, 1, x, ldx, W, Wt, T, K, I, 2 * I, (half_t *)out, e, s);
     return tiled_check("gemm_tiled_silu_mul");
+}
+int gemm_tiled_clamped_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, float limit, float alpha, half_bits *out, int64_t ldo, hipStream_t s) {
+    if (!gemm_tiled_ok(T, K, I, ldx) || I % 64 || ldo % 8 || ldo < I) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_clamped_glu: T=%ld K=%ld I=%ld", (long)T, (long)K, (long)I);
+    if (int rc = gemm_tiled_prepare()) return rc;
+    TileEpi e{}; e.limit = limit; e.alpha = alpha; e.ldo = ldo;
+    tiled_launch<TEPI_CLAMP>(I / 64, 1, x, ldx, W, nullptr, T, K, I, 2 * I, (half_t *)out, e, s);
+    return tiled_check("gemm_tiled_clamped_glu");
 }
 int gemm_tiled_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D,
                               const int64_t *positions, const int32_t *slots, const float *cos_t, const float *sin_t, half_bits *qkv,

@@ -560,14 +560,23 @@ int linear_gelu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t
 }
 
 // gate_up GEMM + the clamped gated unit of a layer list: W [2I, K] (gate rows, then up rows), out [T, ldo].  Few rows, whose product the weight-row kernel takes: the unit
-// is a launch of its own otherwise, and a launch behind a launch is about 5 us whatever it holds (16 rows of 1024, I = 3072: 11.3 -> 6.3 us together).  More rows run the tiles' kernels, which
-// store each product once and whose 16384-row unit is a copy at the memory's rate.
+// is a launch of its own otherwise, and a launch behind a launch is about 5 us whatever it holds (16 rows of 1024, I = 3072: 11.3 -> 6.3 us together).  Shapes of the LDS tiles, routed as linear()
+// routes the plain product: the unit by itself reads both halves of every row again and the product writes twice the columns (16384 rows of 1024, I = 3072: 201 + 59 us -> 168).
+static bool clamped_glu_on_tiles(int64_t T, int64_t K, int64_t I, int64_t ldx) {
+    return K % 32 == 0 && I % 64 == 0 && gemm_tiled_ok(T, K, I, ldx) && ((gemm256_silu_ok(T, K, I, ldx) && rows_on_256(T, K, 2 * I) > 0) || !stream_preferred(T, 2 * I));
+}
 bool linear_clamped_glu_ok(const half_bits *x, int64_t ldx, int64_t T, int64_t K, int64_t I, const half_bits *out, int64_t ldo) {
+    if (((uintptr_t)x | (uintptr_t)out) % 16 == 0 && ldo % 8 == 0 && ldo >= I && clamped_glu_on_tiles(T, K, I, ldx)) return true;
     return T <= 32 && K % 32 == 0 && I % 16 == 0 && ldx % 8 == 0 && ldo % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)out % 8 == 0 && !linear_stream_silu_ok(T, K, I, ldx);
 }
 int linear_clamped_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, float limit, float alpha, half_bits *out, int64_t ldo, hipStream_t s) {
     if (!linear_clamped_glu_ok(x, ldx, T, K, I, out, ldo)) return nvr::fail(NVR_ERR_UNSUPPORTED, "linear_clamped_glu: T=%ld K=%ld I=%ld", (long)T, (long)K, (long)I);
     if (T == 0) return 0;
+    if (T > 32) {
+        const int64_t r = gemm256_silu_ok(T, K, I, ldx) ? rows_on_256(T, K, 2 * I) : 0;
+        if (r > 0) if (int rc = gemm256_clamped_glu(x, ldx, W, r, K, I, limit, alpha, out, ldo, s)) return rc;
+        return r == T ? 0 : gemm_tiled_clamped_glu(x + r * ldx, ldx, W, T - r, K, I, limit, alpha, out + r * ldo, ldo, s);
+    }
     LinEpiClamp e{};
     e.limit = limit; e.alpha = alpha; e.ldy = ldo;
     const unsigned gx = (unsigned)(I / 16);

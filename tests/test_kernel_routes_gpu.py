@@ -465,6 +465,19 @@ def test_layer_list_gated_head_norm_and_clamped_unit(dtype, heads, vdim, ff, bat
     _compare_layer_rows(cfg, w, dtype, base, [np.concatenate([g["s%d" % i] for g in got]) for i in range(batch)])
 
 
+@pytest.mark.parametrize("width,ff,batch,tokens", [(64, 2112, 3, 24), (64, 2112, 9, 34), (128, 2176, 5, 140), (1024, 3072, 24, 96)])
+def test_layer_list_clamped_unit_on_tiles(width, ff, batch, tokens):
+    """The clamped unit in the epilogue of 32-, 64-, 128- and 256-row tiles, against the float64 restatement: prompts of slightly different lengths in one step, every row of it."""
+    import rugudra_util as u
+    cfg = u.make_config([u.retention_layer(2, 32, 32, ff=ff), u.attention_layer(2, 1, 64, 64, ff=ff)], width=width, taps=4)
+    w = u.make_weights(cfg, seed=ff + width)
+    d = u.Driver(cfg, w, dtype="bfloat16", slots=batch, pages=batch * (tokens // 16 + 2), max_tokens=batch * (tokens + 2), max_len=256)
+    rng = np.random.default_rng(batch)
+    base = [rng.integers(0, 97, tokens + i) for i in range(3)]
+    got = d.step([("s%d" % i, base[i % 3]) for i in range(batch)])
+    _compare_layer_rows(cfg, w, "bfloat16", base, [got["s%d" % i] for i in range(batch)])
+
+
 def _bits(rng, shape, std):
     """float16 numbers of a deviation."""
     return (rng.standard_normal(shape) * std).astype(F16)
