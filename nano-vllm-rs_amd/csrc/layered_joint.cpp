@@ -340,7 +340,7 @@ int LayeredModel::forward_joint(nvr_model_runner &r, const StepPlan &p) {
     }
     kl::GroupNormArgs n{}; n.in = x; n.ldi = W; n.in_f32 = true; n.rows = p.d_want; n.rows_n = R; n.W = W; n.groups = 1; n.eps = eps; n.w = wfinal; n.out = xsel; n.ldo = W;
     RC(kl::group_norm(n, bf16, s));
-    return gemm(r, xsel, W, head, R, W, spec.vocab, r.logits, true);
+    return head_product(r, R);
 }
 
 }  // namespace nvr

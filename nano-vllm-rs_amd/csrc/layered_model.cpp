@@ -219,6 +219,11 @@ int LayeredModel::init(nvr_model_runner &r) {
     // sampling (Sampler::sample, sampler.rs:71-218: the runner's own samplers read r.logits)
     NVR_HIP_CHECK(hipMalloc((void **)&r.d_tok, (size_t)r.max_seqs * 8)); NVR_HIP_CHECK(hipMalloc((void **)&r.d_maxval, (size_t)r.max_seqs * 4));
     NVR_HIP_CHECK(hipHostMalloc((void **)&r.h_tok, (size_t)r.max_seqs * 8, hipHostMallocDefault));
+    if (hipHostGetDevicePointer((void **)&r.h_tok_dev, r.h_tok, 0) != hipSuccess) { r.h_tok_dev = nullptr; (void)hipGetLastError(); }
+    if (bf16) {                                                           // arg-max partials of the head's product (head_parts)
+        const size_t n = std::max<size_t>((size_t)nvr::k::LM_HEAD_MAX_PARTS * 32, (size_t)((V + 127) / 128) * (size_t)r.max_seqs);
+        NVR_HIP_CHECK(hipMalloc((void **)&r.d_lm_pval, n * 4)); NVR_HIP_CHECK(hipMalloc((void **)&r.d_lm_pidx, n * 4));
+    }
     NVR_HIP_CHECK(hipMalloc((void **)&r.d_temp, (size_t)r.max_seqs * 4)); NVR_HIP_CHECK(hipMalloc((void **)&r.d_topk, (size_t)r.max_seqs * 8));
     NVR_HIP_CHECK(hipMalloc((void **)&r.d_topp, (size_t)r.max_seqs * 4)); NVR_HIP_CHECK(hipMalloc((void **)&r.d_keys, (size_t)r.max_seqs * 8));
     NVR_HIP_CHECK(hipHostMalloc((void **)&r.samp_host, (size_t)r.max_seqs * 24, hipHostMallocDefault));
@@ -300,6 +305,19 @@ int LayeredModel::gemm(nvr_model_runner &r, const void *a, int64_t lda, const vo
     if (!bf16) return nvr::kf::linear((const float *)a, lda, (const float *)w, T, K, N, nullptr, (float *)y, r.stream);
     if (K % 32 == 0 && N % 16 == 0 && lda % 8 == 0) return nvr::kb::linear((const uint16_t *)a, lda, (const uint16_t *)w, T, K, N, y, y_f32, r.stream);
     return kl::gemm_any(a, lda, w, T, K, N, y, y_f32, true, r.stream);
+}
+
+// arg-max partials the head's product of R rows leaves (0: none, its rows are searched by a launch of their own)
+int64_t LayeredModel::head_parts(const nvr_model_runner &r, int64_t R) const {
+    return bf16 && R <= r.max_seqs ? nvr::kb::lm_head_parts(R, spec.width, spec.vocab, spec.width) : 0;
+}
+// logits of the R rows of xsel.  On the dense graph's LM head where it takes the shape: its weights stream at the memory's rate (16 rows, 32768 x 1024, us: the plain product 19.6, so 16.8), and
+// the greedy choice is made over its partials (6.4 -> 3.2), written to the host's buffer without a copy behind it
+int LayeredModel::head_product(nvr_model_runner &r, int64_t R) {
+    const int64_t W = spec.width;
+    if (head_parts(r, R) == 0) return gemm(r, xsel, W, head, R, W, spec.vocab, r.logits, true);
+    int32_t parts = 0;
+    return nvr::kb::lm_head((const uint16_t *)xsel, W, (const uint16_t *)head, R, W, spec.vocab, r.logits, r.d_lm_pval, r.d_lm_pidx, &parts, r.stream, true);
 }
 
 // One step over a batch of chunks: sequence i contributes its tokens [chunk_start, chunk_start + chunk_len).  want: rows of the step (in batch
@@ -434,6 +452,7 @@ int LayeredModel::execute(nvr_model_runner &r, nvr_seq *const *seqs, size_t nseq
         RC(forward(r, plan));
     for (size_t i = 0; i < nseq; ++i) slot_par[(size_t)seqs[i]->state_slot] ^= 1;
     r.last_rows = R; r.last_tokens = T;
+    r.lm_parts = (int32_t)head_parts(r, (int64_t)R);
     return NVR_OK;
 }
 
@@ -536,7 +555,7 @@ int LayeredModel::forward(nvr_model_runner &r, const StepPlan &p) {
     }
     if (owed) RC(kl::axpy_parts(x, parts, (int)owed, bf16, (float)spec.residual_mult, T * W, s));
     RC(kl::norm_rows(x, d_want, (int64_t)R, W, eps, gfinal, xsel, bf16, s));
-    return gemm(r, xsel, W, head, (int64_t)R, W, spec.vocab, r.logits, true);
+    return head_product(r, (int64_t)R);
 }
 
 // ===================================================================================================================================================
@@ -1020,7 +1039,7 @@ int LayeredModel::forward_sequential(nvr_model_runner &r, const StepPlan &p) {
     }
     kl::GroupNormArgs n{}; n.in = x; n.ldi = W; n.in_f32 = true; n.rows = p.d_want; n.rows_n = R; n.W = W; n.groups = groups; n.eps = eps; n.w = wfinal; n.out = xsel; n.ldo = W;
     RC(kl::group_norm(n, bf16, s));
-    return gemm(r, xsel, W, head, R, W, spec.vocab, r.logits, true);
+    return head_product(r, R);
 }
 
 // ===================================================================================================================================================
@@ -1260,7 +1279,7 @@ int LayeredModel::forward_scaled(nvr_model_runner &r, const StepPlan &p) {
     }
     kl::GroupNormArgs n{}; n.in = x; n.ldi = W; n.in_f32 = true; n.rows = p.d_want; n.rows_n = R; n.W = W; n.groups = 1; n.eps = eps; n.w = wfinal; n.out = xsel; n.ldo = W;
     RC(kl::group_norm(n, bf16, s));
-    RC(gemm(r, xsel, W, head, R, W, spec.vocab, r.logits, true));
+    RC(head_product(r, R));
     if (spec.logit_scale != 1.0) RC(kl::scale_f32(r.logits, R * spec.vocab, (float)spec.logit_scale, s));
     return NVR_OK;
 }

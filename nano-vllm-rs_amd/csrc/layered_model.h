@@ -233,6 +233,8 @@ private:
     int load_streams(nvr_model_runner &r, const std::string &name, int dtype, const int64_t *shape, int ndim, const void *data);
     int forward_streams(nvr_model_runner &r, const StepPlan &p);
     template <class T> int own(T **p, size_t bytes);
+    int64_t head_parts(const nvr_model_runner &r, int64_t R) const;
+    int head_product(nvr_model_runner &r, int64_t R);
     int gemm(nvr_model_runner &r, const void *a, int64_t lda, const void *w, int64_t T, int64_t K, int64_t N, void *y, bool y_f32 = false);
     int put(nvr_model_runner &r, void *dst, int64_t dst_ld, int64_t rows, int64_t cols, int dtype, const void *src, bool as_operand);
 };

@@ -262,7 +262,7 @@ int LayeredModel::forward_streams(nvr_model_runner &r, const StepPlan &p) {
         }
         if (L.has_mlp) { RC(join(i, 1)); st.place = nullptr; st.y = tmp; }
     }
-    return gemm(r, xsel, W, head, R, W, spec.vocab, r.logits, true);
+    return head_product(r, R);
 }
 
 }  // namespace nvr

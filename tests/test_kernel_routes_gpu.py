@@ -478,6 +478,31 @@ def test_layer_list_clamped_unit_on_tiles(width, ff, batch, tokens):
     _compare_layer_rows(cfg, w, "bfloat16", base, [got["s%d" % i] for i in range(batch)])
 
 
+@pytest.mark.parametrize("batch", [1, 16, 17, 32, 33, 130])
+@pytest.mark.parametrize("vocab", [112, 100, 4112])
+def test_layer_list_head_and_greedy_choice(vocab, batch):
+    """Logits and greedy choice of a layer list whose head runs on the dense graph's (widths and vocabularies it takes, 1 .. 130 rows) or as a plain product (a vocabulary of 100), first step and
+    replays: logits against the float64 restatement, tokens the first maximum of the logits."""
+    import rugudra_util as u
+    cfg = u.make_config([u.retention_layer(2, 32, 32, ff=64)], width=256, taps=2)
+    cfg["vocab"] = vocab
+    w = u.make_weights(cfg, seed=vocab)
+    d = u.Driver(cfg, w, dtype="bfloat16", slots=batch, pages=batch * 2, max_tokens=max(64, 9 * batch), max_len=64)
+    rng = np.random.default_rng(vocab)
+    base = [rng.integers(0, vocab, 6 + i) for i in range(min(batch, 3))]
+    names = ["s%d" % i for i in range(batch)]
+    d.step([(n, base[i % 3][:-3]) for i, n in enumerate(names)])
+    rows = [[] for _ in names]
+    for k in range(3):
+        logits = d.step([(n, base[i % 3][len(base[i % 3]) - 3 + k:][:1]) for i, n in enumerate(names)])
+        seqs = [d.live[n] for n in names]
+        tokens = d.runner.sample_tokens(seqs)
+        for i, n in enumerate(names):
+            assert tokens[i] == int(np.argmax(logits[n][-1])), (i, k)
+            rows[i].append(logits[n])
+    _compare_layer_rows(cfg, w, "bfloat16", base, [np.concatenate(r) for r in rows])
+
+
 def _bits(rng, shape, std):
     """float16 numbers of a deviation."""
     return (rng.standard_normal(shape) * std).astype(F16)
