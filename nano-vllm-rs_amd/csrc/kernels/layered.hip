@@ -129,12 +129,15 @@ __global__ __launch_bounds__(256) void norm_canon_kernel(const float *__restrict
 // The same for widths that are multiples of 4 and up to 8 taps, RB rows per workgroup and nothing staged in LDS: the waves first reduce the rows the group
 // needs (its own and the taps-1 before them) to 1 / rms each, then every thread walks its columns four at a time and gathers, per output row, the taps inputs
 // from the step's rows (L1 / L2 hits: a row is read by up to taps neighbours), the slot's history, or zero.
-template <class OT, int RB>
-__global__ __launch_bounds__(256) void norm_canon_rows_kernel(const float *__restrict__ x, Batch b, int W, float eps, int taps, float g1, const float *__restrict__ w1,
+// TAPS: the taps where they are 2, 3 or 4 (0: a general number).  A thread then keeps the TAPS - 1 rows behind its columns in registers, each normed once, and its weights come in 16-byte pieces:
+// every row is read once more instead of TAPS times (16384 rows of 1024, 4 taps: 66.8 -> 38.6 us, 3.5 TB/s of its 134 MB).
+template <class OT, int RB, int TAPS>
+__global__ __launch_bounds__(256) void norm_canon_rows_kernel(const float *__restrict__ x, Batch b, int W, float eps, int taps_rt, float g1, const float *__restrict__ w1,
                                                               OT *__restrict__ out1, float g2, const float *__restrict__ w2, OT *__restrict__ out2,
                                                               float *__restrict__ hist, int64_t slots) {
     __shared__ float rinv[RB + 8];
     __shared__ int rs_i[RB], rs_n[RB], rs_st[RB], rs_par[RB]; __shared__ int64_t rs_slot[RB];
+    const int taps = TAPS ? TAPS : taps_rt;
     const int t0 = blockIdx.x * RB, hrows = taps - 1;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int k = wave; k < RB + hrows; k += 4) {
@@ -151,6 +154,66 @@ __global__ __launch_bounds__(256) void norm_canon_rows_kernel(const float *__res
         rs_i[threadIdx.x] = t - c0; rs_n[threadIdx.x] = b.cu[sq + 1] - c0; rs_st[threadIdx.x] = b.start[sq]; rs_par[threadIdx.x] = b.par[sq]; rs_slot[threadIdx.x] = b.slot[sq];
     }
     __syncthreads();
+    if constexpr (TAPS != 0) {
+        for (int c4 = threadIdx.x * 4; c4 < W; c4 += 1024) {
+            float wa[4 * TAPS], wb[4 * TAPS];
+#pragma unroll
+            for (int j = 0; j < TAPS; ++j) {
+                *reinterpret_cast<float4 *>(wa + 4 * j) = *reinterpret_cast<const float4 *>(w1 + (int64_t)c4 * TAPS + 4 * j);
+                if (out2) *reinterpret_cast<float4 *>(wb + 4 * j) = *reinterpret_cast<const float4 *>(w2 + (int64_t)c4 * TAPS + 4 * j);
+            }
+            float4 u[TAPS];                                                   // u[d]: the row d back, normed
+            auto row = [&](int t) { return *reinterpret_cast<const float4 *>(x + (int64_t)min(max(t, 0), b.T - 1) * W + c4); };
+            auto normed = [&](float4 v, float ri) { return float4{v.x * ri, v.y * ri, v.z * ri, v.w * ri}; };
+            float4 ahead[4];                                                  // requested four rows before they are used
+#pragma unroll
+            for (int k = 0; k < TAPS - 1; ++k) u[TAPS - 2 - k] = row(t0 - (TAPS - 1) + k);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) ahead[k] = row(t0 + k);
+#pragma unroll
+            for (int k = 0; k < TAPS - 1; ++k) if (t0 - (TAPS - 1) + k >= 0) u[TAPS - 2 - k] = normed(u[TAPS - 2 - k], rinv[k]);
+#pragma unroll
+            for (int r = 0; r < RB; ++r) {
+                const int t = t0 + r;
+                if (t >= b.T) break;
+                const int i = __builtin_amdgcn_readfirstlane(rs_i[r]);
+                const bool last = i == __builtin_amdgcn_readfirstlane(rs_n[r]) - 1;
+#pragma unroll
+                for (int d = TAPS - 1; d > 0; --d) u[d] = u[d - 1];
+                u[0] = normed(ahead[r & 3], rinv[r + hrows]);
+                if (r + 4 < RB) ahead[r & 3] = row(t + 4);
+                float4 w[TAPS];
+#pragma unroll
+                for (int d = 0; d < TAPS; ++d) w[d] = u[d];
+                if (i < TAPS - 1) {                                           // rows in front of the chunk: the slot's history, or zero before position 0
+                    const float *hin = hist + ((int64_t)rs_par[r] * slots + rs_slot[r]) * hrows * W;
+#pragma unroll
+                    for (int d = 1; d < TAPS; ++d)
+                        if (i - d < 0) w[d] = rs_st[r] + i - d >= 0 ? *reinterpret_cast<const float4 *>(hin + (int64_t)(hrows + (i - d)) * W + c4) : float4{0.f, 0.f, 0.f, 0.f};
+                }
+                float a1[4] = {0.f, 0.f, 0.f, 0.f}, a2[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int j = 0; j < TAPS; ++j) {
+                    const float4 v = w[TAPS - 1 - j];
+                    const float uu[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                    for (int y = 0; y < 4; ++y) { a1[y] = fmaf(wa[y * TAPS + j], __fmul_rn(g1, uu[y]), a1[y]); if (out2) a2[y] = fmaf(wb[y * TAPS + j], __fmul_rn(g2, uu[y]), a2[y]); }
+                }
+                if (last) {
+                    float *hout = hist + ((int64_t)(rs_par[r] ^ 1) * slots + rs_slot[r]) * hrows * W;
+#pragma unroll
+                    for (int d = 0; d < TAPS - 1; ++d) *reinterpret_cast<float4 *>(hout + (int64_t)(hrows - 1 - d) * W + c4) = w[d];
+                }
+                const float u0[4] = {w[0].x, w[0].y, w[0].z, w[0].w};
+                float o1[4], o2[4];
+#pragma unroll
+                for (int y = 0; y < 4; ++y) { o1[y] = fmaf(g1, u0[y], a1[y]); o2[y] = fmaf(g2, u0[y], a2[y]); }      // (spelled out: hipcc would contract some of the unrolled rows only)
+                st4_f(out1, (int64_t)t * W + c4, o1);
+                if (out2) st4_f(out2, (int64_t)t * W + c4, o2);
+            }
+        }
+        return;
+    }
     for (int c4 = threadIdx.x * 4; c4 < W; c4 += 1024) {
         float wa[4][8], wb[4][8];
 #pragma unroll
@@ -193,6 +256,14 @@ __global__ __launch_bounds__(256) void norm_canon_rows_kernel(const float *__res
     }
 }
 
+template <class OT, int RB>
+void norm_canon_rows_launch(dim3 grid, const float *x, const Batch &b, int W, float eps, int taps, float g1, const float *w1, void *out1, float g2, const float *w2, void *out2, float *hist,
+                            int64_t slots, hipStream_t s) {
+    const bool al = ((uintptr_t)w1 | (uintptr_t)w2) % 16 == 0;
+    auto k = !al ? norm_canon_rows_kernel<OT, RB, 0> : taps == 2 ? norm_canon_rows_kernel<OT, RB, 2> : taps == 3 ? norm_canon_rows_kernel<OT, RB, 3> : taps == 4 ? norm_canon_rows_kernel<OT, RB, 4>
+                 : norm_canon_rows_kernel<OT, RB, 0>;
+    k<<<grid, dim3(256), 0, s>>>(x, b, W, eps, taps, g1, w1, (OT *)out1, g2, w2, (OT *)out2, hist, slots);
+}
 // The join behind the last sublayer and norm_canon of one-row chunks (decode steps) in one launch: x <- x + mult * y where y is the operand type's rounding of the sum of
 // `parts` partial products [parts][T][W] (linear_splitk: added in their order), then the norm, the convolution over the slot's history and the history of the next step.  One
 // row per workgroup, NI 4-column pieces per thread, everything requested before the first sum: the launch is one trip to memory, as each of the two was (16 rows of 1024: 4.6 + 10.6 -> 5.0 us).
@@ -1203,19 +1274,21 @@ __device__ __forceinline__ void ld4_f(const bf16_t *p, float (&v)[4]) {
 }
 // The same for head widths that are multiples of 4, up to 256 * NP: one wave per (row, head), four columns per lane and piece, the head, its gate and its gain requested before the
 // sum and kept in registers.  The general form above walks its heads one behind the other and goes to memory twice for each, two bytes at a time: decode steps are bound by that chain
-// (16 rows of 8 heads x 256 columns, bfloat16: 8.75 -> 4.96 us, as long as an empty launch behind another); 16384 rows move at the memory's rate either way (102 -> 101 us)
-template <class OT, int NP>
+// (16 rows of 8 heads x 256 columns, bfloat16: 8.75 -> 4.96 us, as long as an empty launch behind another); 16384 rows 102 -> 101 us
+// LPH: lanes of a head, a wave or (widths up to 128, whose columns would leave the other half of it idle) half of one: 16384 rows of 16 heads x 128 98.8 -> 55.9 us (4.8 TB/s of its 268 MB), 16
+// rows as long as before
+template <class OT, int NP, int LPH>
 __global__ __launch_bounds__(256) void head_norm_gate4_kernel(const float *__restrict__ o, const OT *__restrict__ gate, int64_t ldg, int H, int Dv, float eps,
                                                               const float *__restrict__ w, OT *__restrict__ out, int64_t ldo, int w_heads) {
-    const unsigned groups = (unsigned)(H + 3) >> 2;                            // grid: rows x groups of four heads
+    constexpr int HPB = 256 / LPH;
+    const unsigned groups = (unsigned)(H + HPB - 1) / HPB;                     // grid: rows x groups of HPB heads
     const int64_t t = blockIdx.x / groups;
-    const int h = (int)(blockIdx.x % groups) * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (h >= H) return;
+    const int hh = (int)(blockIdx.x % groups) * HPB + (int)(threadIdx.x / LPH), h = min(hh, H - 1), lane = threadIdx.x % LPH;      // (clamped: a wave's halves sum together)
     const int64_t i = t * H + h;
     float v[NP][4], g[NP][4], k[NP][4], ss = 0.f;
 #pragma unroll
     for (int q = 0; q < NP; ++q) {
-        const int c = q * 256 + lane * 4;
+        const int c = q * (LPH * 4) + lane * 4;
         if (c >= Dv) continue;
         ld4_f(o + i * Dv + c, v[q]);
         ld4_f(gate + t * ldg + (int64_t)h * Dv + c, g[q]);
@@ -1223,12 +1296,16 @@ __global__ __launch_bounds__(256) void head_norm_gate4_kernel(const float *__res
         else k[q][0] = k[q][1] = k[q][2] = k[q][3] = 1.0f;
         ss += (v[q][0] * v[q][0] + v[q][1] * v[q][1]) + (v[q][2] * v[q][2] + v[q][3] * v[q][3]);
     }
-    ss = wave_sum(ss);
+    if constexpr (LPH == 64) ss = wave_sum(ss);
+    else {
+#pragma unroll
+        for (int o = 16; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+    }
     const float r = 1.0f / sqrtf(ss / (float)Dv + eps);
 #pragma unroll
     for (int q = 0; q < NP; ++q) {
-        const int c = q * 256 + lane * 4;
-        if (c >= Dv) continue;
+        const int c = q * (LPH * 4) + lane * 4;
+        if (c >= Dv || hh >= H) continue;
         float y[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) y[e] = v[q][e] * r * k[q][e] * (g[q][e] / (1.0f + expf(-g[q][e])));
@@ -1278,6 +1355,47 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const float *__restrict_
     ss = block_sum<256>(ss, red);
     const float rs = 1.0f / sqrtf(ss / (float)W + eps);
     for (int c = threadIdx.x; c < W; c += 256) st_f(out, r * W + c, xr[c] * rs * g);
+}
+
+// the same rows of x + m * (sum of the partial products, rounded): the join behind the last layer rides on the final norm.  NI 4-column pieces per thread, everything requested before the first sum
+// (16 rows of 1024 in 4 parts: two launches 5.0 + 4.8 us, so 5.0)
+template <class OT, int NI>
+__global__ __launch_bounds__(256) void join_norm_rows_kernel(const float *__restrict__ x, const float *__restrict__ parts, int nparts, float m, const int32_t *__restrict__ rows, int64_t stride, int W,
+                                                             float eps, float g, OT *__restrict__ out) {
+    __shared__ float red[4];
+    const int64_t r = blockIdx.x, at = (int64_t)rows[r] * W;
+    float4 v[NI], p[NI][8];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int c = (threadIdx.x + i * 256) * 4;
+        if (c >= W) continue;
+        v[i] = *reinterpret_cast<const float4 *>(x + at + c);
+#pragma unroll
+        for (int z = 0; z < 8; ++z) if (z < nparts) p[i][z] = *reinterpret_cast<const float4 *>(parts + z * stride + at + c);
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int c = (threadIdx.x + i * 256) * 4;
+        if (c >= W) continue;
+        float4 y = p[i][0];
+#pragma unroll
+        for (int z = 1; z < 8; ++z) if (z < nparts) { y.x += p[i][z].x; y.y += p[i][z].y; y.z += p[i][z].z; y.w += p[i][z].w; }
+        const float yr[4] = {y.x, y.y, y.z, y.w};
+        OT ro[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st_f(ro, e, yr[e]);
+        v[i].x += m * ld_f(ro, 0); v[i].y += m * ld_f(ro, 1); v[i].z += m * ld_f(ro, 2); v[i].w += m * ld_f(ro, 3);
+        ss += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+    }
+    ss = block_sum<256>(ss, red);
+    const float rs = 1.0f / sqrtf(ss / (float)W + eps);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int c = (threadIdx.x + i * 256) * 4;
+        const float o[4] = {v[i].x * rs * g, v[i].y * rs * g, v[i].z * rs * g, v[i].w * rs * g};
+        if (c < W) st4_f(out, r * W + c, o);
+    }
 }
 
 template <class ET, class YT>
@@ -1340,8 +1458,8 @@ int norm_canon(const float *x, const Batch &b, int64_t W, float eps, int taps, f
 #define NVR_NC(RB_)                                                                                                                                       \
     do {                                                                                                                                                  \
         const dim3 grid((unsigned)((b.T + RB_ - 1) / RB_));                                                                                               \
-        if (bf16) norm_canon_rows_kernel<bf16_t, RB_><<<grid, dim3(256), 0, s>>>(x, b, (int)W, eps, taps, g1, w1, (bf16_t *)out1, g2, w2, (bf16_t *)out2, hist, slots); \
-        else norm_canon_rows_kernel<float, RB_><<<grid, dim3(256), 0, s>>>(x, b, (int)W, eps, taps, g1, w1, (float *)out1, g2, w2, (float *)out2, hist, slots);        \
+        if (bf16) norm_canon_rows_launch<bf16_t, RB_>(grid, x, b, (int)W, eps, taps, g1, w1, out1, g2, w2, out2, hist, slots, s);                                          \
+        else norm_canon_rows_launch<float, RB_>(grid, x, b, (int)W, eps, taps, g1, w1, out1, g2, w2, out2, hist, slots, s);                                                \
     } while (0)
         if (b.T >= 4096) NVR_NC(16); else if (b.T >= 64) NVR_NC(4); else NVR_NC(1);
 #undef NVR_NC
@@ -1534,13 +1652,13 @@ int head_norm_gate(const float *o, const void *gate, int64_t ldg, int64_t gcol, 
     const int64_t es = bf16 ? 2 : 4;
     if (Dv % 4 == 0 && Dv <= 1024 && ldg % 4 == 0 && gcol % 4 == 0 && ldo % 4 == 0 && ((uintptr_t)gate | (uintptr_t)out) % (4 * es) == 0 && ((uintptr_t)o | (uintptr_t)w) % 16 == 0 &&
         T * ((H + 3) / 4) <= 0x7fffffff) {
-        const dim3 wide((unsigned)(T * ((H + 3) / 4)));
-#define NVR_HNG(NP_)                                                                                                                                                                        \
+#define NVR_HNG(NP_, LPH_)                                                                                                                                                                  \
     do {                                                                                                                                                                                    \
-        if (bf16) head_norm_gate4_kernel<bf16_t, NP_><<<wide, dim3(256), 0, s>>>(o, (const bf16_t *)gate + gcol, ldg, (int)H, (int)Dv, eps, w, (bf16_t *)out, ldo, w_heads ? 1 : 0);         \
-        else head_norm_gate4_kernel<float, NP_><<<wide, dim3(256), 0, s>>>(o, (const float *)gate + gcol, ldg, (int)H, (int)Dv, eps, w, (float *)out, ldo, w_heads ? 1 : 0);                 \
+        const dim3 wide((unsigned)(T * ((H + 256 / LPH_ - 1) / (256 / LPH_))));                                                                                                             \
+        if (bf16) head_norm_gate4_kernel<bf16_t, NP_, LPH_><<<wide, dim3(256), 0, s>>>(o, (const bf16_t *)gate + gcol, ldg, (int)H, (int)Dv, eps, w, (bf16_t *)out, ldo, w_heads ? 1 : 0);   \
+        else head_norm_gate4_kernel<float, NP_, LPH_><<<wide, dim3(256), 0, s>>>(o, (const float *)gate + gcol, ldg, (int)H, (int)Dv, eps, w, (float *)out, ldo, w_heads ? 1 : 0);           \
     } while (0)
-        if (Dv <= 256) NVR_HNG(1); else if (Dv <= 512) NVR_HNG(2); else NVR_HNG(4);
+        if (Dv <= 128) NVR_HNG(1, 32); else if (Dv <= 256) NVR_HNG(1, 64); else if (Dv <= 512) NVR_HNG(2, 64); else NVR_HNG(4, 64);
 #undef NVR_HNG
         return launched("head_norm_gate");
     }
@@ -1569,6 +1687,21 @@ int axpy(float *x, const void *y, bool bf16, float mult, int64_t n, hipStream_t 
     return launched("axpy");
 }
 
+bool join_norm_rows_ok(const float *x, const float *parts, int nparts, int64_t W, const void *out) {
+    return nparts >= 1 && nparts <= 8 && W % 4 == 0 && W <= 4096 && ((uintptr_t)x | (uintptr_t)parts | (uintptr_t)out) % 16 == 0;
+}
+int join_norm_rows(const float *x, const float *parts, int nparts, float mult, const int32_t *rows, int64_t R, int64_t T, int64_t W, float eps, float g, void *out, bool bf16, hipStream_t s) {
+    if (R == 0) return 0;
+    if (!join_norm_rows_ok(x, parts, nparts, W, out)) return nvr::fail(NVR_ERR_UNSUPPORTED, "join_norm_rows: %d partial products, width %ld", nparts, (long)W);
+#define NVR_JNR(NI_)                                                                                                                                                        \
+    do {                                                                                                                                                                    \
+        if (bf16) join_norm_rows_kernel<bf16_t, NI_><<<dim3((unsigned)R), dim3(256), 0, s>>>(x, parts, nparts, mult, rows, T * W, (int)W, eps, g, (bf16_t *)out);           \
+        else join_norm_rows_kernel<float, NI_><<<dim3((unsigned)R), dim3(256), 0, s>>>(x, parts, nparts, mult, rows, T * W, (int)W, eps, g, (float *)out);                  \
+    } while (0)
+    if (W <= 1024) NVR_JNR(1); else if (W <= 2048) NVR_JNR(2); else NVR_JNR(4);
+#undef NVR_JNR
+    return launched("join_norm_rows");
+}
 int norm_rows(const float *x, const int32_t *rows, int64_t R, int64_t W, float eps, float g, void *out, bool bf16, hipStream_t s) {
     if (R == 0) return 0;
     if (bf16) norm_rows_kernel<bf16_t><<<dim3((unsigned)R), dim3(256), 0, s>>>(x, rows, (int)W, eps, g, (bf16_t *)out);

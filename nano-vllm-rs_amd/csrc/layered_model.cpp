@@ -553,6 +553,10 @@ int LayeredModel::forward(nvr_model_runner &r, const StepPlan &p) {
             RC(kl::axpy(x, tmp, bf16, (float)spec.residual_mult, T * W, s));
         }
     }
+    if (owed && kl::join_norm_rows_ok(x, parts, (int)owed, W, xsel)) {                                             // (nothing reads the stream behind the last layer)
+        RC(kl::join_norm_rows(x, parts, (int)owed, (float)spec.residual_mult, d_want, (int64_t)R, T, W, eps, gfinal, xsel, bf16, s));
+        return head_product(r, (int64_t)R);
+    }
     if (owed) RC(kl::axpy_parts(x, parts, (int)owed, bf16, (float)spec.residual_mult, T * W, s));
     RC(kl::norm_rows(x, d_want, (int64_t)R, W, eps, gfinal, xsel, bf16, s));
     return head_product(r, (int64_t)R);

@@ -478,6 +478,24 @@ def test_layer_list_clamped_unit_on_tiles(width, ff, batch, tokens):
     _compare_layer_rows(cfg, w, "bfloat16", base, [got["s%d" % i] for i in range(batch)])
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("taps,width,batch", [(2, 64, 130), (3, 1028, 3), (4, 64, 130), (4, 1088, 9), (5, 64, 130)])
+def test_layer_list_norm_and_convolution_rows(dtype, taps, width, batch):
+    """Norm and convolution of chunks of many rows by 16, 4 and one row per workgroup, with the rows behind kept in registers (2 to 4 taps) and not: sequences that begin, end and go on in the
+    middle of a workgroup's rows, chunks shorter than the taps, a second chunk behind the history of the first; against the float64 restatement."""
+    import rugudra_util as u
+    cfg = u.make_config([u.retention_layer(3, 32, 36, ff=48)], width=width, taps=taps)
+    w = u.make_weights(cfg, seed=taps + width)
+    d = u.Driver(cfg, w, dtype=dtype, slots=batch, pages=batch * 6, max_tokens=batch * 48, max_len=128)
+    rng = np.random.default_rng(taps)
+    base = [rng.integers(0, 97, n) for n in (33, 46, 37)]
+    cuts = [(0, c, len(t)) for c, t in zip((32, 1, 34), base)]
+    got = [[], []]
+    for k in range(2):
+        got[k] = d.step([("s%d" % i, base[i % 3][cuts[i % 3][k]:cuts[i % 3][k + 1]]) for i in range(batch)])
+    _compare_layer_rows(cfg, w, dtype, base, [np.concatenate([g["s%d" % i] for g in got]) for i in range(batch)])
+
+
 @pytest.mark.parametrize("batch", [1, 16, 17, 32, 33, 130])
 @pytest.mark.parametrize("vocab", [112, 100, 4112])
 def test_layer_list_head_and_greedy_choice(vocab, batch):
