@@ -878,6 +878,222 @@ size_t attn_workspace_bytes(int64_t nq, int64_t H, int64_t D, int64_t max_ctx) {
     return (size_t)(nq * H * max_parts * (D + 2) * sizeof(float));
 }
 
+// ---- a batch behind one shared prefix, in one launch --------------------------------------------------------------
+// A workgroup takes the G query heads of a kv head for NS sequences: its eight waves walk the shared keys in chunks of 32 on the matrix cores, every query row of the workgroup on one column
+// (S^T = K Q^T, O^T += V^T P^T, both operands through a wave's own LDS image: fragments straight from the pages would be 16 rows x 64 bytes a request, whose lanes' addresses take four times as long), then 8 / NS waves walk each sequence's own keys as attn_rows_kernel
+// does; all of a row's partials meet in LDS.  Against a launch for the shared keys and one for the own ones (flash_shared_prefix, SHM) there is one start-up, no partials in memory, and no merge of
+// them: a workgroup reads the shared keys again (from its XCD's L2), which is what bounds the launch beside the own keys: 512 bytes a key and workgroup at 82 GB/s.
+// The weights of shared keys are rounded to 16 bits for the product as there, their sum is that of the rounded weights; own keys' weights stay in f32.
+constexpr int PRE_CH = 32, PRE_VS = 128 * 2 + 32, PRE_OS = 128 + 4;        // keys of a chunk; bytes of an image row, f32 numbers of a partial row (conflict-free strides)
+template <int G, int NS>
+constexpr size_t prefix_lds() { return std::max<size_t>((size_t)8 * PRE_CH * PRE_VS, ((size_t)8 * G * NS + 8 * G) * PRE_OS * 4); }
+template <int G, int NS>
+__global__ __launch_bounds__(512) void attn_prefix_kernel(AttnParams p, int nq, int shared_len) {
+    constexpr int D = 128, R = G * NS, WPS = 8 / NS, U = 4;
+    static_assert(R <= 16 && 8 % NS == 0, "the rows of a workgroup are columns of one product");
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    __shared__ float sh_ml[8][R][2], own_ml[8][G][2];
+    const int g = blockIdx.x % p.KVH, t0 = (blockIdx.x / p.KVH) * NS;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lm = lane & 15, lq = lane >> 4;
+    const float scale2 = p.scale * 1.44269504088896340736f;
+    const int row_elems = p.KVH * D;
+    // this wave's sequence: its block table from the shared keys on, its length, its queries for the own keys (lm: the lane's 16-byte piece, lq: its row of a group of four)
+    const int ts = min(t0 + wave / WPS, nq - 1), wsub = wave % WPS;
+    const int32_t *bt = p.block_tables + (int64_t)ts * p.max_blocks;
+    const int b0 = shared_len >> p.bs_shift;
+    int bt_base = b0, bt_reg = bt[min(b0 + lane, p.max_blocks - 1)];
+    const int ctx = p.ctx_lens[ts];
+    half2_t qv[G][4];
+    {
+        const half_t *q = p.q + (int64_t)ts * p.ldq + (int64_t)g * G * D + lm * 8;
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            const half8_t h = *reinterpret_cast<const half8_t *>(q + i * D);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) qv[i][j] = (half2_t){h[2 * j], h[2 * j + 1]};
+        }
+    }
+    half8_t qf[4];                                                            // column lm of the products: row lm of the workgroup (the columns behind the last repeat it)
+    {
+        const int r = min(lm, R - 1), t = min(t0 + r / G, nq - 1);
+        const half_t *q = p.q + (int64_t)t * p.ldq + (int64_t)(g * G + r % G) * D + lq * 8;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) qf[ks] = *reinterpret_cast<const half8_t *>(q + ks * 32);
+    }
+    auto block_row = [&](int tok) -> int64_t {                                // cache row of a key of this sequence's own blocks (uniform)
+        const int bi = tok >> p.bs_shift;
+        if (bi >= bt_base + 64) { bt_base = bi; bt_reg = bt[min(bi + lane, p.max_blocks - 1)]; }
+        return (int64_t)__builtin_amdgcn_readlane(bt_reg, bi - bt_base) * p.block_size + (tok & (p.block_size - 1));
+    };
+    const int ngroups = (max(ctx - shared_len, 0) + 3) >> 2;                  // groups of four own keys, dealt to the sequence's waves in turn
+    half8_t kk[U], vv[U];
+    auto request_own = [&](int first) {                                       // groups first, first + WPS, ..
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int tok = shared_len + (min(first + u * WPS, ngroups - 1) << 2);
+            const int64_t at = (block_row(tok) + min(lq, ctx - 1 - tok)) * row_elems + g * D + lm * 8;
+            kk[u] = load_row16<true>(p.k + at); vv[u] = load_row16<true>(p.v + at);
+        }
+    };
+    if (wsub < ngroups) request_own(wsub);
+    // ---- shared keys
+    char *img = smem + wave * PRE_CH * PRE_VS;
+    float m = -INFINITY, l = 0.f;
+    float4_t o[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) o[t] = (float4_t){0.f, 0.f, 0.f, 0.f};
+    half8_t kx[8], vx[8];                                                     // a chunk as it comes from the pages: row 4 i + lq, 16-byte piece lm
+    auto request_shared = [&](int x) {
+        const int base = x * PRE_CH;
+        const int64_t row0 = (int64_t)p.block_tables[base >> p.bs_shift] * p.block_size + (base & (p.block_size - 1));
+        const int64_t at = (row0 + lq) * row_elems + g * D + lm * 8;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) kx[u] = *reinterpret_cast<const half8_t *>(p.k + at + u * 4 * row_elems);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) vx[u] = *reinterpret_cast<const half8_t *>(p.v + at + u * 4 * row_elems);
+    };
+    const int chunks = shared_len / PRE_CH;
+    if (wave < chunks) request_shared(wave);
+    for (int x = wave; x < chunks; x += 8) {
+        half8_t kf[2][4];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) { const int row = 4 * u + lq; *reinterpret_cast<half8_t *>(img + row * 256 + ((lm ^ (row & 15)) << 4)) = kx[u]; }
+        asm volatile("" ::: "memory");                                        // (a wave's LDS requests are served in order: what is written is read behind it, and written again behind that)
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) kf[mt][ks] = *reinterpret_cast<const half8_t *>(img + (mt * 16 + lm) * 256 + (((ks * 4 + lq) ^ lm) << 4));
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int u = 0; u < 8; ++u) *reinterpret_cast<half8_t *>(img + (4 * u + lq) * PRE_VS + lm * 16) = vx[u];
+        asm volatile("" ::: "memory");
+        if (x + 8 < chunks) request_shared(x + 8);
+        float4_t s[2];
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+            s[mt] = (float4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) s[mt] = mfma16(kf[mt][ks], qf[ks], s[mt]);
+        }
+        float mx = -INFINITY;                                                 // scores of row lm: keys base + mt * 16 + lq * 4 + e
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { s[mt][e] *= scale2; mx = fmaxf(mx, s[mt][e]); }
+        mx = xor32_partner_max(xor16_partner_max(mx));
+        const float mn = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f(m - mn);
+        const bool moved = mn != m;
+        m = mn;
+        half8_t pf;
+        float rs = 0.f;
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { const half_t w = (half_t)__builtin_amdgcn_exp2f(s[mt][e] - mn); rs += (float)w; pf[mt * 4 + e] = w; }
+        l = fmaf(l, alpha, rs);
+        if (__any(moved)) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) o[t] *= alpha;
+        }
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const char *at = img + (lq * 4 + (lm >> 2)) * PRE_VS + t * 32 + (lm & 3) * 8;
+            const half4_t a0 = lds_read_tr16(at), a1 = lds_read_tr16(at + 16 * PRE_VS);
+            o[t] = mfma16(__builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7), pf, o[t]);
+        }
+        asm volatile("" ::: "memory");
+    }
+    // ---- own keys
+    float om[G], ol[G], acc[G][8];
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+        om[i] = -INFINITY; ol[i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[i][j] = 0.f;
+    }
+    for (int first = wsub; first < ngroups; first += WPS * U) {
+        float sc[U][G];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool valid = first + u * WPS < ngroups && shared_len + ((first + u * WPS) << 2) + lq < ctx;
+#pragma unroll
+            for (int i = 0; i < G; ++i) {
+                float d = 0.f;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) d = dot2((half2_t){kk[u][2 * j], kk[u][2 * j + 1]}, qv[i][j], d);
+                sc[u][i] = valid ? row_sum<16>(d) * scale2 : -INFINITY;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+            float mx = sc[0][i];
+#pragma unroll
+            for (int u = 1; u < U; ++u) mx = fmaxf(mx, sc[u][i]);
+            const float mn = fmaxf(om[i], mx), ms = mn == -INFINITY ? 0.f : mn, alpha = __builtin_amdgcn_exp2f(om[i] - ms);
+            om[i] = mn;
+            float ps = 0.f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[i][j] *= alpha;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const float pr = __builtin_amdgcn_exp2f(sc[u][i] - ms);
+                ps += pr;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc[i][j] = fmaf(pr, (float)vv[u][j], acc[i][j]);
+            }
+            ol[i] = fmaf(ol[i], alpha, ps);
+        }
+        if (first + WPS * U < ngroups) request_own(first + WPS * U);
+    }
+    // ---- partials of every row: [wave][row] of the shared keys, [wave][head] of the own ones
+    l = xor32_partner_sum(xor16_partner_sum(l));
+    __syncthreads();                                                          // every wave is done with its image
+    float *sh_o = reinterpret_cast<float *>(smem), *own_o = sh_o + 8 * R * PRE_OS;
+    if (lm < R) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) *reinterpret_cast<float4_t *>(sh_o + (wave * R + lm) * PRE_OS + t * 16 + lq * 4) = o[t];
+        if (lq == 0) { sh_ml[wave][lm][0] = m; sh_ml[wave][lm][1] = l; }
+    }
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+        const float M = xor32_partner_max(xor16_partner_max(om[i])), w = om[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(om[i] - M);
+        const float L = xor32_partner_sum(xor16_partner_sum(ol[i] * w));
+        float4_t a[2];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[j >> 2][j & 3] = xor32_partner_sum(xor16_partner_sum(acc[i][j] * w));
+        if (lq == 0) {
+            float *at = own_o + (wave * G + i) * PRE_OS + lm * 8;
+            *reinterpret_cast<float4_t *>(at) = a[0]; *reinterpret_cast<float4_t *>(at + 4) = a[1];
+            if (lm == 0) { own_ml[wave][i][0] = M; own_ml[wave][i][1] = L; }
+        }
+    }
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < R * (D / 4); idx += 512) {
+        const int r = idx / (D / 4), c = (idx % (D / 4)) * 4, sq = r / G, i = r % G;
+        if (t0 + sq >= nq) continue;
+        float M = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) M = fmaxf(M, sh_ml[w][r][0]);
+#pragma unroll
+        for (int w = 0; w < WPS; ++w) M = fmaxf(M, own_ml[sq * WPS + w][i][0]);
+        float4_t v = {0.f, 0.f, 0.f, 0.f};
+        float L = 0.f;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) {
+            const float f = __builtin_amdgcn_exp2f(sh_ml[w][r][0] - M);      // (a wave without a chunk: 2^-inf = 0)
+            v += *reinterpret_cast<const float4_t *>(sh_o + (w * R + r) * PRE_OS + c) * f;
+            L = fmaf(sh_ml[w][r][1], f, L);
+        }
+#pragma unroll
+        for (int w = 0; w < WPS; ++w) {
+            const float f = __builtin_amdgcn_exp2f(own_ml[sq * WPS + w][i][0] - M);
+            v += *reinterpret_cast<const float4_t *>(own_o + ((sq * WPS + w) * G + i) * PRE_OS + c) * f;
+            L = fmaf(own_ml[sq * WPS + w][i][1], f, L);
+        }
+        *reinterpret_cast<half4_t *>(p.out + ((int64_t)(t0 + sq) * p.H + g * G + i) * D + c) = (half4_t){(half_t)(v[0] / L), (half_t)(v[1] / L), (half_t)(v[2] / L), (half_t)(v[3] / L)};
+    }
+}
+
 template <int D, int G, int U, int WAVES, bool NT>
 static void launch_cfg(const AttnParams &p, bool paged, bool direct, int64_t nwg, hipStream_t s, bool fuse = false, bool shm = false, const OwnRows *own = nullptr) {
     dim3 grid((unsigned)nwg), block(WAVES * 64);
@@ -922,6 +1138,28 @@ static bool own_rows_aligned(const AttnArgs &a) {
     return a.qn_w && a.ldq % 8 == 0 && (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.qn_w | (uintptr_t)a.kn_w | (uintptr_t)a.cos_t | (uintptr_t)a.sin_t) & 15) == 0;
 }
 static OwnRows own_rows_params(const AttnArgs &a) { return OwnRows{(const half_t *)a.qn_w, (const half_t *)a.kn_w, a.qk_eps, a.pos, a.slots, a.cos_t, a.sin_t}; }
+
+// A whole batch behind its prefix, up to as many sequences a workgroup as give every CU one, and as long as reading the shared keys for each workgroup costs less than the second launch: each 256 keys
+// are 1.6 us more (0.5-0.85 in the launch of their own).  us a layer, two launches / one, 75 own keys, groups of 2: 33 sequences behind 256 / 512 / 1024 / 2048 keys 13.4 14.7 16.3 19.3 / 11.0 12.6 15.8
+// 21.9; 64 16.0 17.3 19.4 22.8 / 11.7 13.4 16.8 23.5; 128 19.7 21.8 24.3 25.5 / 14.7 16.6 19.6 26.1; 256 27.4 29.2 30.5 33.4 / 22.2 24.1 27.3 34.0.
+static bool prefix_in_one_launch(const AttnArgs &a, int64_t pairs) {
+    const int G = a.H / a.KVH;
+    return !a.shared_rows && a.shared_len <= 1536 && (a.block_size & (a.block_size - 1)) == 0 && a.block_size % 64 == 0 && pairs <= (int64_t)share_workgroups() * (G <= 2 ? 8 : 4) && a.ldq % 8 == 0 &&
+           (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.out) & 15) == 0;
+}
+template <int G, int NS>
+static int launch_prefix(const AttnParams &p, int nq, int shared_len, hipStream_t s) {
+    static bool done = false;                                                 // (more than 64 KiB of LDS are opted in once; a flag that several threads may set alike)
+    if (!done) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_prefix_kernel<G, NS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)prefix_lds<G, NS>());
+        if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "attention (shared prefix): LDS opt-in failed: %s", hipGetErrorString(e));
+        done = true;
+    }
+    attn_prefix_kernel<G, NS><<<dim3((unsigned)((nq + NS - 1) / NS * p.KVH)), dim3(512), prefix_lds<G, NS>(), s>>>(p, nq, shared_len);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "attention (shared prefix) launch failed: %s", hipGetErrorString(e));
+    return 0;
+}
 
 template <int D, int G>
 static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
@@ -1036,6 +1274,15 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
             return 0;
         }
     }
+    if constexpr (D == 128 && G <= 4)
+        if (shared && prefix_in_one_launch(a, pairs)) {
+            if (int rc = own_rows(a, s)) return rc;
+            const int64_t ns = (pairs + share_workgroups() - 1) / share_workgroups();     // sequences of a workgroup: one workgroup per CU
+            if (ns <= 1) return launch_prefix<G, 1>(p, a.nq, a.shared_len, s);
+            if (ns <= 2) return launch_prefix<G, 2>(p, a.nq, a.shared_len, s);
+            if (ns <= 4) return launch_prefix<G, 4>(p, a.nq, a.shared_len, s);
+            if constexpr (G <= 2) return launch_prefix<G, 8>(p, a.nq, a.shared_len, s);
+        }
     const bool direct = np <= 1;
     if (!direct && a.workspace_bytes && (size_t)a.nq * a.H * np * (D + 2) * sizeof(float) > a.workspace_bytes)
         return nvr::fail(NVR_ERR_INVALID_ARG, "attention: %d partitions of %d queries x %d heads need %zu workspace bytes, %zu given",

@@ -448,6 +448,45 @@ def test_brief_decode_attention_against_partitions(B, G, KVH, D, bs, ctx, bound)
     assert np.all(np.abs(a - b) <= 2 * np.maximum(np.spacing(np.abs(b).astype(F16)).astype(np.float32), 2.0 ** -14 / 8)), np.abs(a - b).max()
 
 
+@pytest.mark.parametrize("B,G,KVH,bs,P,own", [
+    (3, 2, 8, 64, 1, [4300, 10, 0]),                                                       # own blocks past the 64 a wave holds; one sequence a workgroup, waves without a chunk of the prefix
+    (32, 1, 8, 128, 3, [(5 * i) % 40 for i in range(32)]),
+    (33, 2, 8, 256, 2, [1 + 8 * i for i in range(33)]),                                     # two sequences a workgroup, the last one alone
+    (65, 4, 8, 64, 7, [(17 * i) % 150 for i in range(65)]),                                 # four, 16 rows
+    (101, 4, 8, 128, 12, [3] * 101),                                                       # the longest prefix of the one launch
+    (131, 2, 8, 64, 5, [(29 * i) % 90 for i in range(131)]),                                # eight
+    (256, 1, 8, 64, 24, [64 + i % 3 for i in range(256)]),
+    (2047, 2, 1, 64, 1, [i % 7 for i in range(2047)]),                                     # one kv head
+    (129, 4, 8, 64, 2, [40] * 129), (40, 2, 8, 64, 25, [9] * 40),                           # beside the rule: more workgroups than CUs, a longer prefix
+])
+def test_shared_prefix_decode_attention_in_one_launch(B, G, KVH, bs, P, own):
+    """Shared and own keys of a batch in one launch (1, 2, 4 and 8 sequences a workgroup, groups of 1, 2 and 4) against the plain kernel on the same inputs: f32 sums in another order, the prefix's
+    weights rounded to float16, one rounding (3 ulps, as the two launches' test)."""
+    l, D, H = nvr.lib(), 128, G * KVH
+    rng = np.random.default_rng(B + P)
+    S, blocks = P * bs, [(o + bs - 1) // bs for o in own]
+    mb, pool = P + max(blocks) + 1, P + sum(blocks)
+    perm, at = rng.permutation(pool), P
+    bt = np.full((B, mb), -1, np.int32)
+    for b in range(B):
+        bt[b, :P] = perm[:P]
+        bt[b, P:P + blocks[b]] = perm[at:at + blocks[b]]
+        at += blocks[b]
+    q = rng.standard_normal((B, H, D)).astype(F16)
+    k, v = (rng.standard_normal((pool, bs, KVH, D)).astype(F16) for _ in range(2))
+    k[perm[P - 1], -1] = 3 * q[0].reshape(KVH, G, D)[:, 0]                 # a prefix whose last key outweighs the rest for some rows
+    d_q, d_k, d_v, d_bt, d_ctx = dev(q), dev(k), dev(v), dev(bt), dev(np.asarray([S + o for o in own], np.int32))
+    meta = nvr.AttnMetaC()
+    meta.context_lens, meta.block_tables, meta.max_blocks, meta.batch, meta.max_context_len = d_ctx.ptr, d_bt.ptr, mb, B, S + max(own)
+    ws = nvr.DeviceBuffer(l.nvr_paged_attn_workspace_bytes(B, H, D, S + max(own) + bs))
+    a, b = nvr.DeviceBuffer(B * H * D * 2), nvr.DeviceBuffer(B * H * D * 2)
+    nvr.check(l.nvr_fill_const(b.ptr, B * H * D, C.c_float(float("nan")), None))
+    nvr.check(l.nvr_paged_attn_decode(d_q.ptr, H * D, d_k.ptr, d_v.ptr, C.byref(meta), H, KVH, D, bs, D ** -0.5, a.ptr, ws.ptr, None))
+    nvr.check(l.nvr_paged_attn_decode_shared(d_q.ptr, H * D, d_k.ptr, d_v.ptr, C.byref(meta), H, KVH, D, bs, D ** -0.5, S, None, None, None, b.ptr, ws.ptr, None))
+    x, y = a.to_numpy((B, H, D), F16).astype(np.float32), b.to_numpy((B, H, D), F16).astype(np.float32)
+    assert np.all(np.abs(x - y) <= 1e-3 + 3 * 2.0 ** -10 * np.abs(x)), np.abs(x - y).max()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("heads,vdim,ff,batch", [(1, 30, 48, 1), (3, 32, 48, 16), (5, 4, 64, 17), (2, 64, 2064, 32), (4, 96, 40, 33)])
 def test_layer_list_gated_head_norm_and_clamped_unit(dtype, heads, vdim, ff, batch):
