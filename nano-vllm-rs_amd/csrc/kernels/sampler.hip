@@ -103,7 +103,9 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float *__restric
     const int row = blockIdx.x;
     const float *x = logits + (int64_t)row * V;
     float *w = ws + (int64_t)row * V;
-    const float temp = temperature[row];
+    const float temp = temperature[row], row_p = top_p ? top_p[row] : -1.0f;      // (together: see sample_rows_kernel)
+    const long long row_k = top_k ? top_k[row] : 0;
+    const uint64_t rkey = keys ? keys[row] : 0ull;
     const bool greedy = (temp == 0.0f);                                // sampler.rs:78-81
 
     if (!greedy) {
@@ -112,7 +114,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float *__restric
         __syncthreads();
 
         // ---- top-k, sampler.rs:115-148 --------------------------------------------------------
-        long long k = top_k ? top_k[row] : 0;
+        long long k = row_k;
         if (k > 0 && k < V) {
             auto key = [&](int i) { return ordered_key(w[i]); };
             unsigned int prefix = 0, mask = 0, need = (unsigned int)k, cnt_eq = 0;
@@ -138,7 +140,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float *__restric
         }
 
         // ---- top-p, sampler.rs:151-188 --------------------------------------------------------
-        const float p = top_p ? top_p[row] : -1.0f;
+        const float p = row_p;
         if (p >= 0.0f) {
             float lm = -INFINITY;
             for (int i = threadIdx.x; i < V; i += kThreads) lm = fmaxf(lm, w[i]);
@@ -192,7 +194,6 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float *__restric
     }
 
     // ---- Gumbel-max (or plain argmax when greedy), sampler.rs:109-112,191-203 ----------------------
-    const uint64_t rkey = keys ? keys[row] : 0ull;
     float bv = -INFINITY; int bi = 0x7fffffff;
     for (int i = threadIdx.x; i < V; i += kThreads) {
         float v;
@@ -299,7 +300,10 @@ __global__ __launch_bounds__(kThreads) void sample_rows_kernel(const float *__re
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int base = part * chunk, end = min(V, base + chunk);
     const float *x = logits + (int64_t)row * V;
-    const float temp = temperature[row];
+    // (a row's numbers together: where the caller leaves them in host memory, they are one trip over the bus)
+    const float temp = temperature[row], row_p = top_p ? top_p[row] : -1.0f;
+    const long long row_k = top_k ? top_k[row] : 0;
+    const uint64_t rkey = keys ? keys[row] : 0ull;
     const bool greedy = (temp == 0.0f);                                // sampler.rs:78-81
     unsigned int epoch = 0;
 
@@ -373,7 +377,7 @@ __global__ __launch_bounds__(kThreads) void sample_rows_kernel(const float *__re
 
     if (!greedy) {
         // ---- top-k, sampler.rs:115-148: 4-pass radix select of the k-th largest key ------------------
-        const long long k = top_k ? top_k[row] : 0;
+        const long long k = row_k;
         if (k > 0 && k < V) {
             auto key = [&](int j) { return ordered_key(w[j]); };
             unsigned int prefix = 0, mask = 0, need = (unsigned int)k, cnt_eq = 0;
@@ -412,7 +416,7 @@ __global__ __launch_bounds__(kThreads) void sample_rows_kernel(const float *__re
         }
 
         // ---- top-p, sampler.rs:151-188 ------------------------------------------------------------------
-        const float p = top_p ? top_p[row] : -1.0f;
+        const float p = row_p;
         if (p >= 0.0f) {
             float lm = -INFINITY;
 #pragma unroll
@@ -516,7 +520,6 @@ __global__ __launch_bounds__(kThreads) void sample_rows_kernel(const float *__re
     }
 
     // ---- Gumbel-max (or plain argmax when greedy), sampler.rs:109-112,191-203 ----------------------
-    const uint64_t rkey = keys ? keys[row] : 0ull;
     unsigned long long best = 0;                                       // (ordered value << 32) | ~index; 0 = nothing kept
 #pragma unroll
     for (int j = 0; j < EPT; ++j) {

@@ -224,9 +224,8 @@ int LayeredModel::init(nvr_model_runner &r) {
         const size_t n = std::max<size_t>((size_t)nvr::k::LM_HEAD_MAX_PARTS * 32, (size_t)((V + 127) / 128) * (size_t)r.max_seqs);
         NVR_HIP_CHECK(hipMalloc((void **)&r.d_lm_pval, n * 4)); NVR_HIP_CHECK(hipMalloc((void **)&r.d_lm_pidx, n * 4));
     }
-    NVR_HIP_CHECK(hipMalloc((void **)&r.d_temp, (size_t)r.max_seqs * 4)); NVR_HIP_CHECK(hipMalloc((void **)&r.d_topk, (size_t)r.max_seqs * 8));
-    NVR_HIP_CHECK(hipMalloc((void **)&r.d_topp, (size_t)r.max_seqs * 4)); NVR_HIP_CHECK(hipMalloc((void **)&r.d_keys, (size_t)r.max_seqs * 8));
     NVR_HIP_CHECK(hipHostMalloc((void **)&r.samp_host, (size_t)r.max_seqs * 24, hipHostMallocDefault));
+    NVR_HIP_CHECK(hipHostGetDevicePointer((void **)&r.samp_dev, r.samp_host, 0));
     NVR_HIP_CHECK(hipMalloc(&r.sample_ws, nvr::kb::sample_workspace_bytes(r.max_seqs, V)));
     NVR_HIP_CHECK(hipDeviceSynchronize());
     return NVR_OK;

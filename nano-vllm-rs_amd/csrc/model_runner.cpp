@@ -45,7 +45,7 @@ nvr_model_runner::~nvr_model_runner() {
                              void *ts[] = {l.qkv_t, l.o_t, l.gate_up_t, l.down_t, l.q_norm, l.k_norm, l.qkv_b, l.o_b, l.gate_up_b, l.down_b}; for (void *t : ts) if (t) hipFree(t); }
     if (lm_head_t) hipFree(lm_head_t);
     void *ptrs[] = {embed, mc.tie_word_embeddings ? nullptr : lm_head, norm, cos_t, sin_t, kv_pool, h, n, qkv, attn,
-                    proj, gu, act, nlast, logits, attn_ws, slabs, in_dev, d_tok, d_maxval, d_temp, d_topk, d_topp, d_keys,
+                    proj, gu, act, nlast, logits, attn_ws, slabs, in_dev, d_tok, d_maxval,
                     sample_ws, d_gather_val, d_gather_idx, d_gather_logits, d_full_logits, sample_ws_full, d_lm_pval, d_lm_pidx, d_rec, d_gather_rec, f32_gather, f32_h2};
     for (void *p : ptrs) if (p) hipFree(p);
     if (in_host) hipHostFree(in_host);
@@ -187,8 +187,8 @@ int nvr_model_runner::init() {                                       // ModelRun
             RC(dmalloc(&lm_snap[i], em * max_seqs * Hd));                   // the LM head's input rows of the step with this parity (present_step)
         }
     }
-    RC(dmalloc(&d_temp, max_seqs)); RC(dmalloc(&d_topk, max_seqs)); RC(dmalloc(&d_topp, max_seqs)); RC(dmalloc(&d_keys, max_seqs));
     NVR_HIP_CHECK(hipHostMalloc((void **)&samp_host, max_seqs * 24, hipHostMallocDefault));
+    NVR_HIP_CHECK(hipHostGetDevicePointer((void **)&samp_dev, samp_host, 0));
     NVR_HIP_CHECK(hipMalloc(&sample_ws, KD(sample_workspace_bytes(max_seqs, Vl))));
     RC(dmalloc(&d_gather_val, tp * max_seqs)); RC(dmalloc(&d_gather_idx, tp * max_seqs));   // (max, argmax) pairs of every rank
     if (tp > 1) { RC(dmalloc(&d_rec, max_seqs)); RC(dmalloc(&d_gather_rec, tp * max_seqs)); }
@@ -1543,11 +1543,16 @@ int nvr_model_runner::sample(nvr_seq *const *seqs, size_t nseq, int64_t *out) {
             tpv[i] = (sp.has_top_p && sp.top_p < 1.0f) ? sp.top_p : -1.0f;
             ky[i] = nvr_sample_key(cfg.sample_seed, seqs[i]->seq_id, seqs[i]->num_completion_tokens());   // A-20
         }
-        NVR_HIP_CHECK(hipMemcpyAsync(d_temp, t, B * 4, hipMemcpyHostToDevice, stream));
-        NVR_HIP_CHECK(hipMemcpyAsync(d_topk, tk, B * 8, hipMemcpyHostToDevice, stream));
-        NVR_HIP_CHECK(hipMemcpyAsync(d_topp, tpv, B * 4, hipMemcpyHostToDevice, stream));
-        NVR_HIP_CHECK(hipMemcpyAsync(d_keys, ky, B * 8, hipMemcpyHostToDevice, stream));
-        RC(KD(sample(lg, B, Vs, d_temp, d_topk, d_topp, d_keys, d_tok, ws, stream, false)));
+        // the sampler reads its few numbers a row where the host wrote them, and writes the tokens where the host reads them (the call waits for it): four uploads and a copy back were 4.7 us each,
+        // more than the two trips
+        const char *const dev = samp_dev;
+        RC(KD(sample(lg, B, Vs, (const float *)(dev + max_seqs * 16), (const int64_t *)dev, (const float *)(dev + max_seqs * 20), (const uint64_t *)(dev + max_seqs * 8), h_tok_dev ? h_tok_dev : d_tok, ws,
+                     stream, false)));
+        if (h_tok_dev) {
+            NVR_HIP_CHECK(hipStreamSynchronize(stream));
+            std::memcpy(out, h_tok, B * 8);
+            return NVR_OK;
+        }
     }
     NVR_HIP_CHECK(hipMemcpyAsync(h_tok, d_tok, B * 8, hipMemcpyDeviceToHost, stream));      // to_vec1 :152
     NVR_HIP_CHECK(hipStreamSynchronize(stream));
