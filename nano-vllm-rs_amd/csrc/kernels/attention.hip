@@ -43,8 +43,11 @@ struct AttnParams {
 };
 struct OwnRows { const half_t *qn_w, *kn_w; float qk_eps; const int64_t *pos; const int32_t *slots; const float *cos_t, *sin_t; };   // QKN (AttnArgs)
 struct AttnParamsOwn : AttnParams, OwnRows {};         // (a type of its own: the arguments of the other instances stay as short as they were)
-template <bool QKN> struct AttnParamsOf { using type = AttnParams; };
-template <> struct AttnParamsOf<true> { using type = AttnParamsOwn; };
+struct OutRows { const half_t *w; float *slabs; int64_t stride; int32_t N; };       // OUTP: the output product's weights [N][H D] and its slabs, one per kv head, `stride` elements apart
+struct AttnParamsOut : AttnParams, OwnRows, OutRows {};
+template <bool QKN, bool OUTP = false> struct AttnParamsOf { using type = AttnParams; };
+template <> struct AttnParamsOf<true, false> { using type = AttnParamsOwn; };
+template <bool QKN> struct AttnParamsOf<QKN, true> { using type = AttnParamsOut; };
 
 // One 8-element piece of a head of 128 held by 16 lanes (dc = lane % 16, elements dc * 8 ..): RMSNorm over the head and rotation as qknorm_rope_store_kernel does them — its sums' pairs, its
 // roundings, nothing contracted: the same bits.  g: the norm's weights of the piece, c / s: cosines and sines of pairs (dc % 8) * 8 ..
@@ -164,10 +167,16 @@ __device__ __forceinline__ half4_t merge_partitions(int np, LoadML load_ml, Load
 // QKN (heads of 128, UB): the step's own rows come raw — RMSNorm over q and k heads, rotation and the store of the new key and value row ride here instead of a launch of their own in front
 // (4.6 us a layer at a few rows, as much as this whole kernel over short contexts): the first waves form the G query heads and the key row, 16 lanes a head, while every wave's first keys are on
 // their way; all read them back from LDS.  The row of the last key is taken from there, not from the cache; the workgroup whose keys end with it stores it.
-template <int D, int G, bool PAGED, bool DIRECT_OUT, int U, int WAVES, bool NT, bool UB, bool FUSE = false, bool SHM = false, bool QKN = false>
-__global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnParamsOf<QKN>::type own) {
+// OUTP (one workgroup's worth of keys per pair, few queries): the output product rides here.  blockIdx.y = OUT_ROWS of its rows: the workgroups of a pair all form the pair's G heads (its keys come from
+// one XCD's L2, where the pairs' workgroups meet) and multiply them, rounded as the launch between the two rounded them, with their rows of the G D columns of W that belong to the pair, requested behind
+// the first keys; the pair's sums go to slab g, added up by the norm that reads the slabs.  Launches bound such a step: one sequence of 128 keys, 16 heads, 1024 columns, attention 6.9 and product
+// 4.1 us, so 6.5 (attn_out_rides).
+constexpr int OUT_ROWS = 64;
+template <int D, int G, bool PAGED, bool DIRECT_OUT, int U, int WAVES, bool NT, bool UB, bool FUSE = false, bool SHM = false, bool QKN = false, bool OUTP = false>
+__global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnParamsOf<QKN, OUTP>::type own) {
     const AttnParams &p = own;                          // (a type that does not depend on the instance: hipcc drops the host stub otherwise)
     static_assert(!QKN || (D == 128 && PAGED && UB && !SHM && G < 4 * WAVES), "QKN: paged heads of 128");
+    static_assert(!OUTP || (PAGED && DIRECT_OUT && WAVES == 8 && G * D <= 512), "OUTP: a wave takes eight rows of up to 64 pieces of the product");
     constexpr int LPR = D / 8;          // lanes per K/V row
     constexpr int RPI = 64 / LPR;       // rows per wave-instruction (= tokens per row group)
     constexpr int TPI = RPI * U;        // tokens per chunk
@@ -346,7 +355,44 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnPara
 
     half8_t kt[U], vt[U];
     if (R == 0) issue_remainder(kt, vt);
-    if constexpr (QKN) {
+    // OUTP: LW lanes hold a row's G D columns, a wave's 64 / LW groups of lanes OL consecutive rows each
+    constexpr int LW = OUTP ? G * D / 8 : 64, OL = LW / 8;
+    half8_t ow[OUTP ? OL : 1];
+    const int on = blockIdx.y * OUT_ROWS + wave * 8 + lane / LW * OL;
+    auto request_out = [&]() {
+        if constexpr (OUTP) {
+            const half_t *w = own.w + (int64_t)on * (p.H * D) + g * (G * D) + lane % LW * 8;
+#pragma unroll
+            for (int u = 0; u < OL; ++u) ow[u] = *reinterpret_cast<const half8_t *>(w + (int64_t)u * (p.H * D));
+        }
+    };
+    if constexpr (OUTP && !QKN) {
+        half8_t kk[U], vv[U];
+        auto issue_round = [&](int tb) {
+            if constexpr (UB) {
+                const int64_t base = block_base(tb);
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const unsigned lo = (unsigned)((u * RPI + tg) * row_elems + dc * 8);
+                    kk[u] = load_row16<NT>(p.k + base + lo); vv[u] = load_row16<NT>(p.v + base + lo);
+                }
+            } else {
+                int64_t off[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) off[u] = lane_row(tb + u * RPI + tg);
+#pragma unroll
+                for (int u = 0; u < U; ++u) { kk[u] = load_row16<NT>(p.k + off[u]); vv[u] = load_row16<NT>(p.v + off[u]); }
+            }
+        };
+        if (R > 0) issue_round(p0 + wave * TPI);
+        asm volatile("" ::: "memory");
+        request_out();
+        for (int r = 0; r < R; ++r) {
+            if (r > 0) issue_round(p0 + (r * WAVES + wave) * TPI);
+            if (r == R - 1) issue_remainder(kt, vt);
+            process(std::false_type{}, kk, vv, 0);
+        }
+    } else if constexpr (QKN) {
         half8_t kk[U], vv[U];
         auto issue_round = [&](int tb) {
             const int64_t base = block_base(tb);
@@ -358,6 +404,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnPara
         };
         if (R > 0) issue_round(p0 + wave * TPI);
         asm volatile("" ::: "memory");                                    // the requests stay in front of the norm
+        request_out();
         if (forms) {
             const half8_t o = norm_rotate_piece(hx, hg, hc, hs, own.qk_eps, dc);
             if (hi <= G) own_lds[hi * 16 + dc] = o;
@@ -372,7 +419,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnPara
             for (int j = 0; j < 4; ++j) qv[i][j] = (half2_t){h[2 * j], h[2 * j + 1]};
         }
         own_k = own_lds[G * 16 + dc];
-        if (wave == WAVES - 1 && tg == 0 && own_slot >= 0 && pend == ctx && p0 < ctx) {
+        if (wave == WAVES - 1 && tg == 0 && own_slot >= 0 && pend == ctx && p0 < ctx && (!OUTP || blockIdx.y == 0)) {
             const int64_t dst = ((int64_t)own_slot * p.KVH + g) * D + dc * 8;
             *reinterpret_cast<half8_t *>(const_cast<half_t *>(p.k) + dst) = own_k;
             *reinterpret_cast<half8_t *>(const_cast<half_t *>(p.v) + dst) = own_v;
@@ -450,6 +497,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnPara
     const auto rs_o = __builtin_amdgcn_make_buffer_rsrc(DIRECT_OUT ? nullptr : p.part_o + pair0 * D, 0, DIRECT_OUT ? 0 : (int)(G * p.num_parts * D * 4), 0x00020000);
     const auto rs_ml = __builtin_amdgcn_make_buffer_rsrc(DIRECT_OUT ? nullptr : p.part_ml + pair0 * 2, 0, DIRECT_OUT ? 0 : (int)(G * p.num_parts * 2 * 4), 0x00020000);
     constexpr int AUX = FUSE ? 16 : 0;                                    // sc1: write-through, so the hand-off needs no release fence
+    __shared__ __attribute__((aligned(16))) half_t heads[OUTP ? G * D : 8];
     if constexpr (!ONE)
     for (int idx = threadIdx.x; idx < G * D; idx += WAVES * 64) {
         const int i = idx / D, d = idx % D;
@@ -469,7 +517,9 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnPara
             L = mul_then_add(wgt, sm_ml[w2][i][1], L);
         }
         const int h = g * G + i;
-        if (DIRECT_OUT) {
+        if constexpr (OUTP) {
+            heads[idx] = (half_t)(L > 0.f ? o / L : 0.f);
+        } else if (DIRECT_OUT) {
             p.out[((int64_t)t * p.H + h) * D + d] = (half_t)(L > 0.f ? o / L : 0.f);
         } else if (SHM) {
             shm_o[i][d] = o;
@@ -479,6 +529,26 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnPara
             __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o), rs_o, (slot * D + d) * 4, 0, AUX);
             if (d == 0) { __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(M), rs_ml, slot * 8, 0, AUX);
                           __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(L), rs_ml, slot * 8 + 4, 0, AUX); }
+        }
+    }
+    if constexpr (OUTP) {
+        __syncthreads();
+        const half8_t x = *reinterpret_cast<const half8_t *>(heads + lane % LW * 8);
+        float y[OL];
+#pragma unroll
+        for (int u = 0; u < OL; ++u) {
+            float d = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) d = dot2((half2_t){x[2 * j], x[2 * j + 1]}, (half2_t){ow[u][2 * j], ow[u][2 * j + 1]}, d);
+            d = row_sum<LW < 16 ? LW : 16>(d);
+            if (LW >= 32) d = xor16_partner_sum(d);
+            if (LW >= 64) d = xor32_partner_sum(d);
+            y[u] = d;
+        }
+        if (lane % LW == 0) {
+            float *const to = own.slabs + g * own.stride + (int64_t)t * own.N + on;
+#pragma unroll
+            for (int u = 0; u < OL; ++u) to[u] = y[u];
         }
     }
     if constexpr (!DIRECT_OUT) {
@@ -1161,8 +1231,48 @@ static int launch_prefix(const AttnParams &p, int nq, int shared_len, hipStream_
     return 0;
 }
 
+// Whether a decode step's attention takes the output product along (OUTP): no more workgroups than CUs (two on a CU wait for each other's registers: 4 sequences of 128 keys 767 / 835 us a step), and
+// contexts of up to two rounds of keys, since every workgroup of a pair walks all of them.  Qwen3-0.6B, us a step, two launches / one: 1 sequence of 40 keys 660 / 627, 128 694 / 645, 200 707 / 673,
+// 255 700 / 656, 400 710 / 711; 2 sequences of 40 694 / 656, 128 716 / 674, 255 741 / 693, 400 757 / 751; with q / k norms 1 of 128 674 / 637, 300 701 / 701, 2 of 128 729 / 692, 300 762 / 765.
+bool attn_out_rides(int64_t nq, int64_t H, int64_t KVH, int64_t D, int64_t N, int64_t max_ctx) {
+    if (KVH <= 0 || H % KVH || max_ctx > 256 || nq * KVH * (N / OUT_ROWS) > share_workgroups()) return false;
+    const int64_t G = H / KVH;
+    return (D == 64 || D == 128) && (G == 1 || G == 2 || G == 4) && (KVH == 2 || KVH == 4 || KVH == 8) && N % OUT_ROWS == 0;
+}
+template <int D, int G>
+static int launch_attn_out(const AttnArgs &a, hipStream_t s) {
+    constexpr int U = D == 128 ? 4 : 2, TPI = 64 / (D / 8) * U;
+    if (!attn_out_rides(a.nq, a.H, a.KVH, D, a.out_n, a.max_ctx) || a.shared_len > 0 || a.seq_of_q || ((uintptr_t)a.out_w & 15))
+        return nvr::fail(NVR_ERR_INVALID_ARG, "attention + output product: %d queries, %d / %d heads of %d, %d columns, contexts up to %d", a.nq, a.H, a.KVH, D, a.out_n, a.max_ctx);
+    AttnParamsOut p{};
+    p.q = (const half_t *)a.q; p.ldq = a.ldq; p.k = (const half_t *)a.k; p.v = (const half_t *)a.v;
+    p.ctx_lens = a.ctx_lens; p.block_tables = a.block_tables; p.max_blocks = a.max_blocks; p.block_size = a.block_size;
+    p.bs_shift = (a.block_size > 0 && (a.block_size & (a.block_size - 1)) == 0) ? __builtin_ctz(a.block_size) : -1;
+    p.H = a.H; p.KVH = a.KVH; p.scale = a.scale; p.part_size = 0x3fffffff; p.num_parts = 1;
+    p.w = (const half_t *)a.out_w; p.slabs = a.out_slabs; p.stride = (int64_t)a.nq * a.out_n; p.N = a.out_n;
+    const dim3 grid((unsigned)(a.nq * a.KVH), (unsigned)(a.out_n / OUT_ROWS));
+    const bool ub = a.block_size % TPI == 0;
+    bool in_it = false;
+    if constexpr (D == 128)
+        if (ub && own_rows_aligned(a)) {
+            static_cast<OwnRows &>(p) = own_rows_params(a);
+            attn_rows_kernel<D, G, true, true, U, 8, false, true, false, false, true, true><<<grid, dim3(512), 0, s>>>(p);
+            in_it = true;
+        }
+    if (!in_it) {
+        if (int rc = own_rows(a, s)) return rc;
+        if (ub) attn_rows_kernel<D, G, true, true, U, 8, false, true, false, false, false, true><<<grid, dim3(512), 0, s>>>(p);
+        else attn_rows_kernel<D, G, true, true, U, 8, false, false, false, false, false, true><<<grid, dim3(512), 0, s>>>(p);
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "attention + output product launch failed: %s", hipGetErrorString(e));
+    return 0;
+}
+
 template <int D, int G>
 static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
+    if constexpr (G <= 4)
+        if (paged && a.out_w) return launch_attn_out<D, G>(a, s);
     AttnParams p{};
     p.q = (const half_t *)a.q; p.ldq = a.ldq; p.k = (const half_t *)a.k; p.v = (const half_t *)a.v; p.ldkv = a.ldkv;
     p.ctx_lens = a.ctx_lens; p.seq_of_q = a.seq_of_q; p.kv_base = a.kv_base; p.block_tables = a.block_tables;

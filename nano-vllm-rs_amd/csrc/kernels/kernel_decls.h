@@ -161,6 +161,7 @@ int gemm256_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, 
                            half_bits *k_cache, half_bits *v_cache, hipStream_t s, bool kv_cache_only = false, const QkNorm *norm = nullptr);
 
 size_t attn_workspace_bytes(int64_t nq, int64_t H, int64_t D, int64_t max_ctx);
+bool attn_out_rides(int64_t nq, int64_t H, int64_t KVH, int64_t D, int64_t N, int64_t max_ctx);   // whether a decode step's attention takes the output product of N rows along (AttnArgs::out_w)
 int64_t attn_brief_context(int64_t nq, int64_t H, int64_t KVH);   // contexts up to it (0: none) have a decode attention of their own: worth a captured step of their own
 int attention(const AttnArgs &a, bool paged, hipStream_t s);
 

@@ -53,6 +53,9 @@ struct AttnArgs {
     // norms' weights): the attention does that first, in its own launch where its kernel can (attention.hip: QKN), else by that launch in front
     const half_bits *qn_w, *kn_w; float qk_eps;
     const int64_t *pos; const int32_t *slots; const float *cos_t, *sin_t;
+    // paged decode, out_w not null (attn_out_rides): the output product x . out_w^T (out_w [out_n, H D]) in the same launch; `out` is not written, but out_slabs [KVH][nq][out_n], the heads of a kv head in a
+    // slab of their own
+    const half_bits *out_w; int32_t out_n; float *out_slabs;
 };
 
 // RMSNorm over the columns of every q and k head in front of the rotation: weights [D] each

@@ -50,9 +50,10 @@ struct LinEpi {
 // What single instances need beyond it stays out of the others' arguments
 struct LinEpiNorm : LinEpi { NormIn norm; };                       // NORM instances: x is formed by the workgroup itself
 struct LinEpiClamp : LinEpi { float limit, alpha; int64_t ldy; };  // EPI_CLAMP: min(g, limit) sigmoid(alpha min(g, limit)) (clamp(u, +-limit) + 1); row stride of y
-template <int EPI, bool NORM> struct LinArgs { using type = LinEpi; };
-template <int EPI> struct LinArgs<EPI, true> { using type = LinEpiNorm; };
-template <> struct LinArgs<EPI_CLAMP, false> { using type = LinEpiClamp; };
+// NORM: slabs that an instance has room for (0: it takes its rows as they are)
+template <int EPI, int NORM> struct LinArgs { using type = LinEpiNorm; };
+template <int EPI> struct LinArgs<EPI, 0> { using type = LinEpi; };
+template <> struct LinArgs<EPI_CLAMP, 0> { using type = LinEpiClamp; };
 
 // W row handled by local row r (0..15) of n-tile i of workgroup bx
 template <int EPI>
@@ -71,7 +72,7 @@ __device__ __forceinline__ int w_row(int bx, int i, int NT, int r, int N, const 
 // the slabs, 16-bit residual add, 16-bit normalised row), formed by every workgroup in LDS while its first weight pieces are on the way, so that the add + norm launch in front of
 // the product disappears; workgroup 0 writes the new residual rows to norm.h_out, a second buffer, since the others still read the old ones.
 constexpr int NORM_ELEMS = 4096;
-template <int NT, int MT, int WAVES, int EPI, bool NORM = false>
+template <int NT, int MT, int WAVES, int EPI, int NORM = 0>
 __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t *__restrict__ x, int64_t ldx,
                                                                    const half_t *__restrict__ W, int T, int K, int N,
                                                                    void *__restrict__ y, typename LinArgs<EPI, NORM>::type epi) {
@@ -122,7 +123,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
         }
     };
     constexpr int KS = 32 * WAVES;
-    constexpr bool AHEAD = NORM || EPI == EPI_ROPE;
+    constexpr bool AHEAD = NORM > 0 || EPI == EPI_ROPE;
     half8_t a_first[U][NT], b_first[U][MT];                  // AHEAD: the first pieces of the weights (and rows)
     auto first_request = [&]() {
 #pragma unroll
@@ -130,21 +131,21 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
             const int kk = min(wave * 32 + u * KS, K - 32);
 #pragma unroll
             for (int i = 0; i < NT; ++i) a_first[u][i] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(wrow[i] + (int64_t)kk * kmul));
-            if constexpr (!NORM)
+            if constexpr (NORM == 0)
 #pragma unroll
                 for (int j = 0; j < MT; ++j) b_first[u][j] = *reinterpret_cast<const half8_t *>(xrow[j] + kk);
         }
         asm volatile("" ::: "memory");
     };
-    if constexpr (AHEAD && !NORM) { first_request(); rope_request(); }
-    if constexpr (NORM) {
+    if constexpr (AHEAD && NORM == 0) { first_request(); rope_request(); }
+    if constexpr (NORM > 0) {
         static_assert(MT == 1, "one row block");
         constexpr int NI = NORM_ELEMS / 4 / (WAVES * 64);     // 4-column pieces per thread
         __shared__ float ss_w[NI * WAVES];                    // sums of squares of 64 neighbouring pieces (K is a multiple of 256: inside one row)
         half_t *xs = reinterpret_cast<half_t *>(norm_lds);
         const NormIn &nm = epi.norm;
         const int per_row = K / 4, total = T * per_row;
-        half4_t hv[NI], gv[NI]; float4_t sv[NI][4];
+        half4_t hv[NI], gv[NI]; float4_t sv[NI][NORM];
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const int idx = i * (WAVES * 64) + (int)threadIdx.x;
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
                 const int64_t o = (int64_t)row * K + c;
                 hv[i] = *reinterpret_cast<const half4_t *>((const half_t *)nm.h_in + o); gv[i] = *reinterpret_cast<const half4_t *>((const half_t *)nm.w + c);
 #pragma unroll
-                for (int z = 0; z < 4; ++z) sv[i][z] = z < nm.S ? *reinterpret_cast<const float4_t *>(nm.slabs + z * nm.stride + o) : (float4_t){0.f, 0.f, 0.f, 0.f};
+                for (int z = 0; z < NORM; ++z) sv[i][z] = z < nm.S ? *reinterpret_cast<const float4_t *>(nm.slabs + z * nm.stride + o) : (float4_t){0.f, 0.f, 0.f, 0.f};
             }
         }
         asm volatile("" ::: "memory");
@@ -166,7 +167,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
                 float ss = 0.f;
                 float4_t a = sv[i][0];
 #pragma unroll
-                for (int z = 1; z < 4; ++z) a += sv[i][z];
+                for (int z = 1; z < NORM; ++z) a += sv[i][z];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     hv[i][e] = to_half_rn((float)hv[i][e] + (float)to_half_rn(a[e]));
@@ -219,7 +220,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
                 }
 #pragma unroll
                 for (int j = 0; j < MT; ++j) {
-                    if (AHEAD && !NORM && k == kbeg + wave * 32) b[u][j] = b_first[u][j];
+                    if (AHEAD && NORM == 0 && k == kbeg + wave * 32) b[u][j] = b_first[u][j];
                     else b[u][j] = *reinterpret_cast<const half8_t *>(xrow[j] + kk);
                 }
             } else {
@@ -340,7 +341,7 @@ __global__ __launch_bounds__(WAVES * 64) void linear_skinny_kernel(const half_t 
 }
 
 template <int NT, int MT, int WAVES, int EPI>
-static void launch(const half_t *x, int64_t ldx, const half_t *W, int T, int K, int N, void *y, const typename LinArgs<EPI, false>::type &e,
+static void launch(const half_t *x, int64_t ldx, const half_t *W, int T, int K, int N, void *y, const typename LinArgs<EPI, 0>::type &e,
                    unsigned gx, hipStream_t s, unsigned gz = 1) {
     dim3 grid(gx, (unsigned)((T + 16 * MT - 1) / (16 * MT)), gz);
     linear_skinny_kernel<NT, MT, WAVES, EPI><<<grid, dim3(WAVES * 64), 0, s>>>(x, ldx, W, T, K, N, y, e);
@@ -645,14 +646,20 @@ int linear_qkv_norm_rope_store(const half_bits *x, int64_t ldx, const half_bits 
 
 // ---- products of a decode step of few rows whose workgroups form RMSNorm(h + slabs) themselves (linear_skinny_kernel, NORM)
 // (three and four rows: from the width on at which the products behind a launch of its own split k over the same eight waves, so that the step's bits are theirs)
-bool norm_linear_ok(int64_t T, int64_t K, int64_t S) { return T >= 1 && T <= NORM_ROWS && (T <= 2 || waves_for(K) == 8) && K % 256 == 0 && T * K <= NORM_ELEMS && (S == 2 || S == 4); }
+bool norm_linear_ok(int64_t T, int64_t K, int64_t S) { return T >= 1 && T <= NORM_ROWS && (T <= 2 || waves_for(K) == 8) && K % 256 == 0 && T * K <= NORM_ELEMS && (S == 2 || S == 4 || S == 8); }
 template <int NT, int EPI>
 static int norm_launch(const NormIn &nm, const half_bits *W, int64_t T, int64_t K, int64_t N, void *y, const LinEpi &le, int64_t gx, bool tiled, hipStream_t s, const char *what) {
     if (!norm_linear_ok(T, K, nm.S)) return nvr::fail(NVR_ERR_UNSUPPORTED, "%s: T=%ld K=%ld, %d slabs", what, (long)T, (long)K, nm.S);
     LinEpiNorm e{};
     static_cast<LinEpi &>(e) = le;
     e.norm = nm; e.tiled = tiled;
-    linear_skinny_kernel<NT, 1, 8, EPI, true><<<dim3((unsigned)gx), dim3(512), (size_t)(T * (K + 8) * 2), s>>>(nullptr, 0, (const half_t *)W, (int)T, (int)K, (int)N, y, e);
+    if constexpr (EPI == EPI_SILU)
+        if (nm.S > 4) {                                                   // (the slabs that an attention with the output product in it leaves, one per kv head)
+            linear_skinny_kernel<NT, 1, 8, EPI, 8><<<dim3((unsigned)gx), dim3(512), (size_t)(T * (K + 8) * 2), s>>>(nullptr, 0, (const half_t *)W, (int)T, (int)K, (int)N, y, e);
+            return launch_check(what);
+        }
+    if (nm.S > 4) return nvr::fail(NVR_ERR_UNSUPPORTED, "%s: %d slabs", what, nm.S);
+    linear_skinny_kernel<NT, 1, 8, EPI, 4><<<dim3((unsigned)gx), dim3(512), (size_t)(T * (K + 8) * 2), s>>>(nullptr, 0, (const half_t *)W, (int)T, (int)K, (int)N, y, e);
     return launch_check(what);
 }
 // which products of these shapes take the weight-streaming kernel above at so few rows (large weights have a kernel of their own)

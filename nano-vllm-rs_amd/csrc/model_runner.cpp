@@ -872,6 +872,8 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
     const int64_t S_o = KD(decode_splitk_slices(T, H * D, Hd)), S_d = KD(decode_splitk_slices(T, I, Hd));
     const bool ride = !is_prefill && !comm.active() && tp == 1 && !mc.use_bias && Hd <= 2048 && KD(norm_linear_silu_ok(T, Hd, I, S_o)) && 
                       (mc.qk_norm ? KD(norm_linear_plain_ok(T, Hd, QKV, S_d)) : KD(norm_linear_rope_ok(T, Hd, H, KVH, D, S_d)));
+    // ... and of few and short contexts the output product rides on the attention, a slab per kv head
+    const bool out_rides = ride && decode_shared_len == 0 && KD(attn_out_rides(T, H, KVH, D, Hd, max_ctx)) && KD(norm_linear_silu_ok(T, Hd, I, KVH)) && KVH * T <= 4 * slab_rows;
     uint16_t *hc = h, *hn = proj;
     int64_t owed = 0;
     for (int64_t l = 0; l < L; ++l) {
@@ -926,11 +928,12 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
                 a.shared_kv0 = (const int32_t *)(in_dev + off_dec + dof_skv0); a.shared_rows = (const int32_t *)(in_dev + off_dec + dof_srows);
                 a.shared_count = (const int32_t *)(in_dev + off_dec + dof_scount);
             }
+            if (out_rides) { a.out_w = w.o; a.out_n = (int32_t)Hd; a.out_slabs = slabs; }
             RC(KD(attention(a, true, st)));
         }
         if (ride) {
-            RC(KD(linear_splitk(attn, H * D, w.o, T, H * D, Hd, S_o, slabs, st, tl ? w.o_t : nullptr)));
-            RC(KD(norm_linear_silu_mul(k::NormIn{hc, slabs, T * Hd, (int32_t)S_o, w.ln2, mc.rms_norm_eps, hn}, w.gate_up, T, Hd, I, act, st, tl ? w.gate_up_t : nullptr)));
+            if (!out_rides) RC(KD(linear_splitk(attn, H * D, w.o, T, H * D, Hd, S_o, slabs, st, tl ? w.o_t : nullptr)));
+            RC(KD(norm_linear_silu_mul(k::NormIn{hc, slabs, T * Hd, (int32_t)(out_rides ? KVH : S_o), w.ln2, mc.rms_norm_eps, hn}, w.gate_up, T, Hd, I, act, st, tl ? w.gate_up_t : nullptr)));
             std::swap(hc, hn);
             RC(KD(linear_splitk(act, I, w.down, T, I, Hd, S_d, slabs, st, tl ? w.down_t : nullptr)));
             owed = S_d;
