@@ -479,7 +479,12 @@ int LayeredModel::forward(nvr_model_runner &r, const StepPlan &p) {
             RC(kl::norm_canon(x, b, W, eps, (int)spec.taps, w.g1, w.canon1, a1, w.g2, w.canon2, L.has_mlp ? a2 : nullptr, bf16, st.hist, slots, s));
         }
         owed = 0;
-        RC(gemm(r, a1, W, w.mix, T, W, w.nmix, proj));
+        // mixer and feed-forward read the stream of the layer in front: in steps of few rows their first products share a launch
+        uint16_t *const glu = (uint16_t *)((char *)cat + (size_t)(w.mixcols * esz));
+        const bool paired = bf16 && L.has_mlp && nvr::kb::linear_beside_clamped_glu_ok((const uint16_t *)a2, W, T, W, w.nmix, L.ff, glu, w.kcat);
+        if (paired) RC(nvr::kb::linear_beside_clamped_glu((const uint16_t *)a1, (const uint16_t *)a2, W, (const uint16_t *)w.mix, (const uint16_t *)w.gu, T, W, w.nmix, L.ff, (float)L.limit, 1.702f,
+                                                          (uint16_t *)proj, glu, w.kcat, s));
+        else RC(gemm(r, a1, W, w.mix, T, W, w.nmix, proj));
         if (L.mixer == LayeredSpec::ATTENTION) {
             kl::SinkAttnArgs a{};
             a.q = (const char *)proj + (size_t)(w.qcol * esz); a.ldq = w.nmix; a.kc = st.kc; a.vc = st.vc; a.r1 = w.r1; a.r2 = w.r2; a.sink = w.sink;
@@ -532,8 +537,7 @@ int LayeredModel::forward(nvr_model_runner &r, const StepPlan &p) {
             RC(kl::retention(a, b, bf16, s));
             RC(kl::head_norm_gate(ret_o, proj, w.nmix, w.gcol, T, L.heads, L.vdim, eps, nullptr, cat, w.kcat, bf16, s));
         }
-        if (L.has_mlp) {
-            uint16_t *const glu = (uint16_t *)((char *)cat + (size_t)(w.mixcols * esz));
+        if (L.has_mlp && !paired) {
             if (bf16 && nvr::kb::linear_clamped_glu_ok((const uint16_t *)a2, W, T, W, L.ff, glu, w.kcat))
                 RC(nvr::kb::linear_clamped_glu((const uint16_t *)a2, W, (const uint16_t *)w.gu, T, W, L.ff, (float)L.limit, 1.702f, glu, w.kcat, s));
             else {

@@ -991,3 +991,19 @@ def test_decode_attention_takes_the_output_product_along(hidden, heads, kv, dim,
         prompts = [oracle.fill_tokens(n, 3, i, mcfg.vocab_size).tolist() for i, n in enumerate(lengths)]
         sps = [dict(temperature=0.0, max_tokens=9, ignore_eos=True)] * len(lengths)
         assert _run_pair(mcfg, ecfg, prompts, sps, dtype=dtype)["decode_steps"] >= 8
+
+
+@pytest.mark.parametrize("width,heads,ff,batch", [(64, 2, 80, 1), (256, 2, 96, 16), (256, 2, 96, 17), (1024, 2, 208, 32), (64, 16, 2064, 17), (1024, 16, 2048, 32)])
+def test_layer_list_decode_steps_of_two_products_in_one_launch(width, heads, ff, batch):
+    """Decode steps of a layer list whose mixer's product and clamped unit share a launch: four and eight waves, one and two row tiles to a workgroup, last tiles of one row and full ones, in both kinds
+    of layers — a first step and replays, against the float64 restatement."""
+    import rugudra_util as u
+    cfg = u.make_config([u.retention_layer(heads, 32, 32, ff=ff), u.attention_layer(heads, 1 if heads < 16 else heads, 64, 64, ff=ff)], width=width, taps=2)
+    w = u.make_weights(cfg, seed=ff + width)
+    d = u.Driver(cfg, w, dtype="bfloat16", slots=batch, pages=batch * 2, max_tokens=9 * batch, max_len=64)
+    rng = np.random.default_rng(width)
+    base = [rng.integers(0, 97, 6 + i) for i in range(min(batch, 3))]
+    names = ["s%d" % i for i in range(batch)]
+    d.step([(n, base[i % 3][:-3]) for i, n in enumerate(names)])
+    steps = [d.step([(n, base[i % 3][len(base[i % 3]) - 3 + k:][:1]) for i, n in enumerate(names)]) for k in range(3)]
+    _compare_layer_rows(cfg, w, "bfloat16", base, [np.concatenate([s[n] for s in steps]) for n in names])
