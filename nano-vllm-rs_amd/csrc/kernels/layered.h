@@ -109,6 +109,9 @@ struct RetentionArgs {
     bool decay_exp; const float *bonus;
 };
 int retention(const RetentionArgs &a, const Batch &b, bool bf16, hipStream_t s);
+// retention and head_norm_gate (no gain) of a step of one token per sequence in one launch: a.o is not written, out [T, ldo] receives what head_norm_gate leaves, with its bits
+bool retention_step_ok(const RetentionArgs &a, const Batch &b, const void *gate, int64_t ldg, int64_t gcol, const void *out, int64_t ldo, bool bf16);
+int retention_step(const RetentionArgs &a, const Batch &b, const void *gate, int64_t ldg, int64_t gcol, float eps, void *out, int64_t ldo, hipStream_t s);
 // out[t][h*Dv + c] = o[t][h][c] / rms(o[t][h][:]) * w[c] * silu(gate[t][h*Dv + c]); gate: rows of the operand type (stride ldg) from column gcol; w (one weight per
 // value column, shared by the heads) may be null; w_heads: w holds a weight per head and column ([H * Dv])
 int head_norm_gate(const float *o, const void *gate, int64_t ldg, int64_t gcol, int64_t T, int64_t H, int64_t Dv, float eps, const float *w, void *out, int64_t ldo,

@@ -1313,6 +1313,65 @@ __global__ __launch_bounds__(256) void head_norm_gate4_kernel(const float *__res
     }
 }
 
+// One token per sequence of the plain decaying form, bfloat16 rows, with the gated norm of the head behind it: a workgroup per (sequence, head) holds the head's whole state, 8 parts of R rows, four columns
+// a thread, so that a row of the state is read and written in 16-byte pieces, all of them requested at once (retention_block_kernel: 4 bytes a lane, a workgroup per 32 columns), and the head's sum
+// of squares needs no other workgroup.  Arithmetic and order are those of retention_block_kernel and head_norm_gate4_kernel, their fused multiply-adds spelled out: a token's bits do not depend on
+// which of them its step takes.  MEASURED_RET
+template <int R, int CG>                                                   // D = 8 R key rows, Dv = 4 CG value columns
+__global__ __launch_bounds__(8 * CG) void retention_step_kernel(RetentionArgs a, Batch b, const bf16_t *__restrict__ gate, int64_t ldg, float eps, bf16_t *__restrict__ out, int64_t ldo) {
+    constexpr int D = 8 * R, Dv = 4 * CG, half = D / 2, NT = 8 * CG;
+    __shared__ __attribute__((aligned(16))) float qs[D], ks[D], partial[8][Dv];
+    const int sq = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, part = tid / CG, c = tid % CG * 4;
+    const int st = b.start[sq];
+    float *const S = a.state + (((int64_t)b.slot[sq] * a.H + h) * D + part * R) * Dv + c;
+    const bf16_t *const row = (const bf16_t *)a.proj + (int64_t)sq * a.ld;
+    const float dec = a.decay[h];
+    float v[4], g[4] = {0.f, 0.f, 0.f, 0.f};
+    ld4_f(row + a.vcol + (int64_t)h * Dv + c, v);
+    if (tid < CG) ld4_f(gate + (int64_t)sq * ldg + (int64_t)h * Dv + c, g);
+    float4 s[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) s[r] = *reinterpret_cast<const float4 *>(S + (int64_t)r * Dv);
+    for (int i = tid; i < D; i += NT) {                                     // pair i % half of q (the first half of the threads) or k
+        const bool key = i >= half;
+        const int j = key ? i - half : i;
+        const bf16_t *const x = row + (key ? a.kcol : a.qcol) + (int64_t)h * D;
+        const float u = ld_f(x, j), w = ld_f(x, j + half), cs = a.cos_t[(int64_t)st * half + j], sn = a.sin_t[(int64_t)st * half + j];
+        const float lo = fmaf(u, cs, -(w * sn)), hi = fmaf(w, cs, u * sn);
+        if (key) { ks[j] = lo * a.kscale; ks[j + half] = hi * a.kscale; } else { qs[j] = lo; qs[j + half] = hi; }
+    }
+    __syncthreads();
+    float o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const float k = ks[part * R + r], q = qs[part * R + r];
+        float *const e = reinterpret_cast<float *>(&s[r]);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            e[x] = fmaf(dec, st > 0 ? e[x] : 0.f, k * v[x]);
+            o[x] = fmaf(e[x], q, o[x]);
+        }
+        *reinterpret_cast<float4 *>(S + (int64_t)r * Dv) = s[r];
+    }
+    *reinterpret_cast<float4 *>(&partial[part][c]) = float4{o[0], o[1], o[2], o[3]};
+    __syncthreads();
+    if (tid < CG) {
+        float y[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = 0; p < 8; ++p) {
+            const float4 z = *reinterpret_cast<const float4 *>(&partial[p][c]);
+            y[0] += z.x; y[1] += z.y; y[2] += z.z; y[3] += z.w;
+        }
+        float ss = fmaf(y[0], y[0], y[1] * y[1]) + fmaf(y[2], y[2], y[3] * y[3]);
+#pragma unroll
+        for (int x = CG / 2; x > 0; x >>= 1) ss += __shfl_xor(ss, x, 64);
+        const float r = 1.0f / sqrtf(ss / (float)Dv + eps);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = y[e] * r * 1.0f * (g[e] / (1.0f + expf(-g[e])));
+        st4_f(out, (int64_t)sq * ldo + (int64_t)h * Dv + c, y);
+    }
+}
+
 template <class OT>
 __global__ __launch_bounds__(256) void clamped_glu_kernel(const OT *__restrict__ gu, int64_t T, int64_t F, float limit, float alpha, OT *__restrict__ out, int64_t ldo) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -1644,6 +1703,25 @@ int retention(const RetentionArgs &a, const Batch &b, bool bf16, hipStream_t s) 
     else NVR_RET(64);
 #undef NVR_RET
     return launched("retention");
+}
+
+bool retention_step_ok(const RetentionArgs &a, const Batch &b, const void *gate, int64_t ldg, int64_t gcol, const void *out, int64_t ldo, bool bf16) {
+    return bf16 && b.max_rows == 1 && b.T == b.B && a.az == nullptr && a.tok_gate == nullptr && a.decay != nullptr && a.v_ones == 0 && a.qk_share <= 1 && (a.D == 64 || a.D == 128) && a.rot_dims == a.D &&
+           (a.Dv == 64 || a.Dv == 128) && ((a.ld | a.vcol | ldg | gcol | ldo) & 3) == 0 && (((uintptr_t)a.proj | (uintptr_t)gate | (uintptr_t)out) & 7) == 0 && ((uintptr_t)a.state & 15) == 0;
+}
+int retention_step(const RetentionArgs &a, const Batch &b, const void *gate, int64_t ldg, int64_t gcol, float eps, void *out, int64_t ldo, hipStream_t s) {
+    if (!retention_step_ok(a, b, gate, ldg, gcol, out, ldo, true)) return nvr::fail(NVR_ERR_UNSUPPORTED, "retention_step: D=%d Dv=%d", a.D, a.Dv);
+    if (b.T == 0) return 0;
+    const dim3 grid((unsigned)b.B, (unsigned)a.H);
+    const bf16_t *const g = (const bf16_t *)gate + gcol;
+    if (a.D == 64) {
+        if (a.Dv == 64) retention_step_kernel<8, 16><<<grid, dim3(128), 0, s>>>(a, b, g, ldg, eps, (bf16_t *)out, ldo);
+        else retention_step_kernel<8, 32><<<grid, dim3(256), 0, s>>>(a, b, g, ldg, eps, (bf16_t *)out, ldo);
+    } else {
+        if (a.Dv == 64) retention_step_kernel<16, 16><<<grid, dim3(128), 0, s>>>(a, b, g, ldg, eps, (bf16_t *)out, ldo);
+        else retention_step_kernel<16, 32><<<grid, dim3(256), 0, s>>>(a, b, g, ldg, eps, (bf16_t *)out, ldo);
+    }
+    return launched("retention_step");
 }
 
 int head_norm_gate(const float *o, const void *gate, int64_t ldg, int64_t gcol, int64_t T, int64_t H, int64_t Dv, float eps, const float *w, void *out, int64_t ldo,

@@ -534,8 +534,12 @@ int LayeredModel::forward(nvr_model_runner &r, const StepPlan &p) {
             a.proj = proj; a.ld = w.nmix; a.qcol = w.qcol; a.kcol = w.kcol; a.vcol = w.vcol; a.decay = w.decay; a.cos_t = w.freq; a.sin_t = w.sin_t; a.rot_dims = (int32_t)L.rot_dims;
             a.az = nullptr; a.ldz = 0; a.abias = nullptr; a.inv_tau = 1.f; a.qscale = 1.f;
             a.kscale = 1.0f / std::sqrt((float)L.dim); a.H = (int32_t)L.heads; a.D = (int32_t)L.dim; a.Dv = (int32_t)L.vdim; a.state = st.state; a.o = ret_o;
-            RC(kl::retention(a, b, bf16, s));
-            RC(kl::head_norm_gate(ret_o, proj, w.nmix, w.gcol, T, L.heads, L.vdim, eps, nullptr, cat, w.kcat, bf16, s));
+            if (kl::retention_step_ok(a, b, proj, w.nmix, w.gcol, cat, w.kcat, bf16))
+                RC(kl::retention_step(a, b, proj, w.nmix, w.gcol, eps, cat, w.kcat, s));
+            else {
+                RC(kl::retention(a, b, bf16, s));
+                RC(kl::head_norm_gate(ret_o, proj, w.nmix, w.gcol, T, L.heads, L.vdim, eps, nullptr, cat, w.kcat, bf16, s));
+            }
         }
         if (L.has_mlp && !paired) {
             if (bf16 && nvr::kb::linear_clamped_glu_ok((const uint16_t *)a2, W, T, W, L.ff, glu, w.kcat))

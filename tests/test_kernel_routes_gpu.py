@@ -1007,3 +1007,27 @@ def test_layer_list_decode_steps_of_two_products_in_one_launch(width, heads, ff,
     d.step([(n, base[i % 3][:-3]) for i, n in enumerate(names)])
     steps = [d.step([(n, base[i % 3][len(base[i % 3]) - 3 + k:][:1]) for i, n in enumerate(names)]) for k in range(3)]
     _compare_layer_rows(cfg, w, "bfloat16", base, [np.concatenate([s[n] for s in steps]) for n in names])
+
+
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (64, 128), (128, 64), (128, 128)])
+def test_retention_of_single_tokens_norms_and_gates_its_heads(dim, vdim):
+    """Steps of one token per sequence, whose retention norms and gates its heads itself, against the same tokens in steps beside a portion of several rows (launches of their own): bit for bit, from a
+    sequence's first token (no state yet, in a slot that another sequence left) on, first steps and replays."""
+    import rugudra_util as u
+    cfg = u.make_config([u.retention_layer(3, dim, vdim, decay=[0.3, 0.95, 0.9995], ff=None)], width=128, taps=3)
+    w = u.make_weights(cfg, seed=dim + vdim)
+    d = u.Driver(cfg, w, dtype="bfloat16", slots=3, pages=24, max_tokens=64, max_len=64)
+    rng = np.random.default_rng(vdim)
+    toks, other = [rng.integers(0, 97, 6) for _ in range(2)], rng.integers(0, 97, 3)
+    got = []
+    for beside in (False, True):
+        rows = []
+        for k in range(6):
+            step = d.step([("s%d" % i, toks[i][k:k + 1]) for i in range(2)] + ([("o", other)] if beside else []))
+            rows += [step["s0"], step["s1"]]
+            if beside:
+                d.end("o")
+        for i in range(2):
+            d.end("s%d" % i)
+        got.append(np.concatenate(rows).view(np.uint32))
+    assert np.array_equal(got[0], got[1])
