@@ -370,7 +370,7 @@ int LayeredModel::execute(nvr_model_runner &r, nvr_seq *const *seqs, size_t nseq
         o_ftiles[k] = carve(cnt * sizeof(nvr::kt::FlashTile)); n_ftiles[k] = (int32_t)cnt;
     }
     if (off > in_bytes) return fail(NVR_ERR_INVARIANT, "execute_model: step inputs of %zu bytes exceed the arena", off);
-    NVR_HIP_CHECK(hipStreamSynchronize(r.stream));                       // in_host is written again: the upload of a step whose results nobody has read may still wait behind the step in front of it
+    if (!r.inputs_read) NVR_HIP_CHECK(hipStreamSynchronize(r.stream));   // in_host is written again: the upload of a step whose results nobody has read may still wait behind the step in front of it
     for (size_t k = 0; k < flash_kinds.size(); ++k) {
         const int64_t pw = flash_kinds[k].positions;
         nvr::kt::FlashTile *tl = (nvr::kt::FlashTile *)(in_host + o_ftiles[k]);
@@ -405,6 +405,7 @@ int LayeredModel::execute(nvr_model_runner &r, nvr_seq *const *seqs, size_t nseq
     }
     cu[nseq] = (int32_t)t;
     if (want) for (size_t i = 0; i < R; ++i) { if (want[i] < 0 || want[i] >= T) return fail(NVR_ERR_INVALID_ARG, "execute_model: logits row %d of a step of %ld rows", want[i], (long)T); wnt[i] = want[i]; }
+    r.inputs_read = false;
     NVR_HIP_CHECK(hipMemcpyAsync(in_dev, in_host, off, hipMemcpyHostToDevice, r.stream));
     kl::Batch b{};
     b.ids = (const int64_t *)(in_dev + o_ids); b.row_seq = (const int32_t *)(in_dev + o_rs); b.cu = (const int32_t *)(in_dev + o_cu);

@@ -148,6 +148,9 @@ private:
                                                          // rides on the consumer GEMV (the workgroups of that launch still read the first while one of them writes)
     float *f32_gather = nullptr; int64_t f32_gather_rows = 0;   // float32 tensor-parallel ranks: every rank's partial sums [tp][f32_gather_rows][hidden], a piece of the step's rows at a time
     int row_parallel_norm(const uint16_t *x, int64_t K, const uint16_t *W, const uint16_t *Wt, int64_t T, const uint16_t *wn, const uint16_t *bias = nullptr);
+    bool inputs_read = false;                            // the last step's tokens have been seen: the upload of its inputs is behind it
+    void await_tokens(int64_t B);
+    int take_tokens(int64_t B, int64_t *out);
     int64_t *h_tok_dev = nullptr;                        // device-visible address of the pinned token buffer h_tok
     int64_t slab_rows = 64;           // rows the split-k slab buffers hold (row_parallel_norm)
     // sharing group of a decode batch (0 = none / too small: plain paged attention); fills kv0[nseq], rows[nseq], *count of the arena
