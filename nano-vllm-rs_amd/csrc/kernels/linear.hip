@@ -431,7 +431,7 @@ static void launch(const half_t *x, int64_t ldx, const half_t *W, int T, int K, 
 
 // 256x256 kernel or 128x128 kernel?  Fitted to both over 22 token counts (100..8192) x the projections of Qwen3-0.6B and Qwen3-8B, weights from HBM.  A round of <= 256 tiles of the
 // 256x256 kernel takes 18.5 K/1024 + 8 us however few there are (K = 1024 25 us, 2048 39, 4096 81, 12288 235).  The 128x128 kernel takes 9.4 K/1024 + 3.5 us while its tiles fit one per CU
-// (13.3 / 22 / 42 / 118), beyond that 8 K/1024 + 1.2 per 256 tiles, a last part of a round counted half (768 tiles 31, 1152 45, 2048 73 at K = 1024).  us of both, 256 / 128: qkv of 0.6B 27.1 /
+// (13.3 / 22 / 42 / 118), beyond that 8 K/1024 + 1.2 per 256 tiles (768 tiles 31, 1152 45, 2048 73 at K = 1024).  us of both, 256 / 128: qkv of 0.6B 27.1 /
 // 20.4 at 2048 tokens, 27.4 / 29.4 at 2560, 49.8 / 45.6 at 4672; o_proj 44.8 / 34.4 at 8192; 8B qkv 84.6 / 64.7 at 1280, 82.9 / 100.1 at 1536, 166 / 153 at 3062.  N = W rows
 static double cost_256(int64_t T, int64_t K, int64_t N) {
     const int64_t tiles = ((N + 255) / 256) * ((T + 255) / 256);
@@ -440,7 +440,10 @@ static double cost_256(int64_t T, int64_t K, int64_t N) {
 static double cost_128(int64_t T, int64_t K, int64_t N) {
     const int64_t tiles = ((N + 127) / 128) * ((T + 127) / 128);
     const double kk = (double)K / 1024.0, rounds = (double)tiles / 256.0;
-    return tiles <= 256 ? 9.4 * kk + 3.5 : 0.5 * (rounds + (double)((tiles + 255) / 256)) * (8.0 * kk + 1.2) + 2.0;
+    if (tiles <= 256) return 9.4 * kk + 3.5;
+    // (two workgroups share a CU: up to 512 tiles a last part of a round is one of the two; what begins a third round lasts a whole one.  us of a Qwen3-0.6B prompt, a last part of any round counted
+    // half / so: 1408 tokens 3703 / 3650, 2176 4944 / 4675, 2304 5022 / 4766; 8B, 2900 tokens 39160 / 38850)
+    return (tiles <= 512 ? 0.5 * (rounds + (double)((tiles + 255) / 256)) : (double)((tiles + 255) / 256)) * (8.0 * kk + 1.2) + 2.0;
 }
 static inline bool prefer_256(int64_t T, int64_t K, int64_t N) { return cost_256(T, K, N) < cost_128(T, K, N); }
 bool gemm256_preferred(int64_t T, int64_t K, int64_t N, int64_t ldx) { return gemm256_ok(T, K, N, ldx) && prefer_256(T, K, N); }
