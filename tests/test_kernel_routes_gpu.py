@@ -602,6 +602,22 @@ def test_tile_products_of_few_k_tiles_and_ragged_edges(T, K, N):
         assert np.all(np.abs(s.astype(np.float64).sum(0) - ref) <= bound)
 
 
+@pytest.mark.parametrize("T,K,N,S", [(20, 1024, 16384, 4), (3, 1056, 12288, 1), (32, 2592, 6144, 1), (17, 3616, 4096, 1), (1, 6144, 4096, 2)])
+def test_split_products_of_large_weights(T, K, N, S):
+    """Slabs of weights of 24 MiB and more, 1 to 15 steps of a wave (one to eight sets of two steps; last sets of one step; waves of one step less than others), one and two row tiles: against 64 bits, and
+    the tiled copy's bits."""
+    rng, l = np.random.default_rng(T + K), nvr.lib()
+    x, W = _bits(rng, (T, K), 0.5), _bits(rng, (N, K), 0.1)
+    d_x, d_W = dev(x), dev(W)
+    d_T, sa, sb = _copy_of(d_W, N, K), nvr.DeviceBuffer(S * T * N * 4), nvr.DeviceBuffer(S * T * N * 4)
+    nvr.check(l.nvr_linear_splitk(d_x.ptr, K, d_W.ptr, T, K, N, S, sa.ptr, None))
+    nvr.check(l.nvr_linear_splitk_tiled(d_x.ptr, K, d_W.ptr, d_T.ptr, T, K, N, S, sb.ptr, None))
+    s = sa.to_numpy((S, T, N), np.float32)
+    assert np.array_equal(s, sb.to_numpy((S, T, N), np.float32))
+    ref, bound = _product_bound(x, W)
+    assert np.all(np.abs(s.astype(np.float64).sum(0) - ref) <= bound)
+
+
 @pytest.mark.parametrize("T,K,N", [(33, 1536, 768), (48, 2048, 1040), (64, 512, 784), (64, 3072, 2048)])
 def test_products_of_33_to_64_rows_in_eight_slices(T, K, N):
     """The o / down products of such steps on the tiles, eight slices of one to six K-tiles: the slabs' sum against 64 bits, the tiled copy's bits, and the residual add + norm over eight slabs."""
