@@ -167,13 +167,13 @@ __device__ __forceinline__ half4_t merge_partitions(int np, LoadML load_ml, Load
 // QKN (heads of 128, UB): the step's own rows come raw — RMSNorm over q and k heads, rotation and the store of the new key and value row ride here instead of a launch of their own in front
 // (4.6 us a layer at a few rows, as much as this whole kernel over short contexts): the first waves form the G query heads and the key row, 16 lanes a head, while every wave's first keys are on
 // their way; all read them back from LDS.  The row of the last key is taken from there, not from the cache; the workgroup whose keys end with it stores it.
-// OUTP (one workgroup's worth of keys per pair, few queries): the output product rides here.  blockIdx.y = OUT_ROWS of its rows: the workgroups of a pair all form the pair's G heads (its keys come from
+// OUTP (one workgroup's worth of keys per pair, few queries): the output product rides here.  blockIdx.y = OUTP (64 or 128) of its rows: the workgroups of a pair all form the pair's G heads (its keys come from
 // one XCD's L2, where the pairs' workgroups meet) and multiply them, rounded as the launch between the two rounded them, with their rows of the G D columns of W that belong to the pair, requested behind
 // the first keys; the pair's sums go to slab g, added up by the norm that reads the slabs.  Launches bound such a step: one sequence of 128 keys, 16 heads, 1024 columns, attention 6.9 and product
 // 4.1 us, so 6.5 (attn_out_rides).
-constexpr int OUT_ROWS = 64;
-template <int D, int G, bool PAGED, bool DIRECT_OUT, int U, int WAVES, bool NT, bool UB, bool FUSE = false, bool SHM = false, bool QKN = false, bool OUTP = false>
-__global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnParamsOf<QKN, OUTP>::type own) {
+constexpr int OUT_ROWS = 64;                              // (128 where 64 would put two workgroups on a CU)
+template <int D, int G, bool PAGED, bool DIRECT_OUT, int U, int WAVES, bool NT, bool UB, bool FUSE = false, bool SHM = false, bool QKN = false, int OUTP = 0>
+__global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnParamsOf<QKN, (OUTP > 0)>::type own) {
     const AttnParams &p = own;                          // (a type that does not depend on the instance: hipcc drops the host stub otherwise)
     static_assert(!QKN || (D == 128 && PAGED && UB && !SHM && G < 4 * WAVES), "QKN: paged heads of 128");
     static_assert(!OUTP || (PAGED && DIRECT_OUT && WAVES == 8 && G * D <= 512), "OUTP: a wave takes eight rows of up to 64 pieces of the product");
@@ -356,17 +356,17 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnPara
     half8_t kt[U], vt[U];
     if (R == 0) issue_remainder(kt, vt);
     // OUTP: LW lanes hold a row's G D columns, a wave's 64 / LW groups of lanes OL consecutive rows each
-    constexpr int LW = OUTP ? G * D / 8 : 64, OL = LW / 8;
+    constexpr int LW = OUTP ? G * D / 8 : 64, OL = OUTP == 128 ? LW / 4 : LW / 8;
     half8_t ow[OUTP ? OL : 1];
-    const int on = blockIdx.y * OUT_ROWS + wave * 8 + lane / LW * OL;
+    const int on = blockIdx.y * OUTP + wave * (OUTP / 8) + lane / LW * OL;
     auto request_out = [&]() {
-        if constexpr (OUTP) {
+        if constexpr (OUTP > 0) {
             const half_t *w = own.w + (int64_t)on * (p.H * D) + g * (G * D) + lane % LW * 8;
 #pragma unroll
             for (int u = 0; u < OL; ++u) ow[u] = *reinterpret_cast<const half8_t *>(w + (int64_t)u * (p.H * D));
         }
     };
-    if constexpr (OUTP && !QKN) {
+    if constexpr (OUTP > 0 && !QKN) {
         half8_t kk[U], vv[U];
         auto issue_round = [&](int tb) {
             if constexpr (UB) {
@@ -517,7 +517,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnPara
             L = mul_then_add(wgt, sm_ml[w2][i][1], L);
         }
         const int h = g * G + i;
-        if constexpr (OUTP) {
+        if constexpr (OUTP > 0) {
             heads[idx] = (half_t)(L > 0.f ? o / L : 0.f);
         } else if (DIRECT_OUT) {
             p.out[((int64_t)t * p.H + h) * D + d] = (half_t)(L > 0.f ? o / L : 0.f);
@@ -531,7 +531,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_rows_kernel(typename AttnPara
                           __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(L), rs_ml, slot * 8 + 4, 0, AUX); }
         }
     }
-    if constexpr (OUTP) {
+    if constexpr (OUTP > 0) {
         __syncthreads();
         const half8_t x = *reinterpret_cast<const half8_t *>(heads + lane % LW * 8);
         float y[OL];
@@ -1231,17 +1231,39 @@ static int launch_prefix(const AttnParams &p, int nq, int shared_len, hipStream_
     return 0;
 }
 
-// Whether a decode step's attention takes the output product along (OUTP): no more workgroups than CUs (two on a CU wait for each other's registers: 4 sequences of 128 keys 767 / 835 us a step), and
+// Whether a decode step's attention takes the output product along (OUTP): no more workgroups than CUs (two on a CU wait for each other's registers: 4 sequences of 128 keys 767 / 835 us a step), which 128 rows a workgroup
+// allow twice as many sequences as 64, and
 // contexts of up to two rounds of keys, since every workgroup of a pair walks all of them.  Qwen3-0.6B, us a step, two launches / one: 1 sequence of 40 keys 660 / 627, 128 694 / 645, 200 707 / 673,
-// 255 700 / 656, 400 710 / 711; 2 sequences of 40 694 / 656, 128 716 / 674, 255 741 / 693, 400 757 / 751; with q / k norms 1 of 128 674 / 637, 300 701 / 701, 2 of 128 729 / 692, 300 762 / 765.
+// 255 700 / 656, 400 710 / 711; 2 sequences of 40 694 / 656, 128 716 / 674, 255 741 / 693, 400 757 / 751; 3 of 128 727 / 696, 4 762 / 734; with q / k norms 1 of 128 674 / 637, 300 701 / 701, 2 of 128 729 / 692, 300 762 / 765, 4 of 255 797 / 761.
 bool attn_out_rides(int64_t nq, int64_t H, int64_t KVH, int64_t D, int64_t N, int64_t max_ctx) {
-    if (KVH <= 0 || H % KVH || max_ctx > 256 || nq * KVH * (N / OUT_ROWS) > share_workgroups()) return false;
+    if (KVH <= 0 || H % KVH || max_ctx > 256 || nq > 4 || nq * KVH * (N / (N % 128 ? 64 : 128)) > share_workgroups()) return false;
     const int64_t G = H / KVH;
     return (D == 64 || D == 128) && (G == 1 || G == 2 || G == 4) && (KVH == 2 || KVH == 4 || KVH == 8) && N % OUT_ROWS == 0;
 }
+template <int D, int G, int R>
+static int launch_attn_out_rows(const AttnArgs &a, AttnParamsOut &p, hipStream_t s) {
+    constexpr int U = D == 128 ? 4 : 2, TPI = 64 / (D / 8) * U;
+    const dim3 grid((unsigned)(a.nq * a.KVH), (unsigned)(a.out_n / R));
+    const bool ub = a.block_size % TPI == 0;
+    bool in_it = false;
+    if constexpr (D == 128)
+        if (ub && own_rows_aligned(a)) {
+            static_cast<OwnRows &>(p) = own_rows_params(a);
+            attn_rows_kernel<D, G, true, true, U, 8, false, true, false, false, true, R><<<grid, dim3(512), 0, s>>>(p);
+            in_it = true;
+        }
+    if (!in_it) {
+        if (int rc = own_rows(a, s)) return rc;
+        if (ub) attn_rows_kernel<D, G, true, true, U, 8, false, true, false, false, false, R><<<grid, dim3(512), 0, s>>>(p);
+        else attn_rows_kernel<D, G, true, true, U, 8, false, false, false, false, false, R><<<grid, dim3(512), 0, s>>>(p);
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "attention + output product launch failed: %s", hipGetErrorString(e));
+    return 0;
+}
+
 template <int D, int G>
 static int launch_attn_out(const AttnArgs &a, hipStream_t s) {
-    constexpr int U = D == 128 ? 4 : 2, TPI = 64 / (D / 8) * U;
     if (!attn_out_rides(a.nq, a.H, a.KVH, D, a.out_n, a.max_ctx) || a.shared_len > 0 || a.seq_of_q || ((uintptr_t)a.out_w & 15))
         return nvr::fail(NVR_ERR_INVALID_ARG, "attention + output product: %d queries, %d / %d heads of %d, %d columns, contexts up to %d", a.nq, a.H, a.KVH, D, a.out_n, a.max_ctx);
     AttnParamsOut p{};
@@ -1250,23 +1272,9 @@ static int launch_attn_out(const AttnArgs &a, hipStream_t s) {
     p.bs_shift = (a.block_size > 0 && (a.block_size & (a.block_size - 1)) == 0) ? __builtin_ctz(a.block_size) : -1;
     p.H = a.H; p.KVH = a.KVH; p.scale = a.scale; p.part_size = 0x3fffffff; p.num_parts = 1;
     p.w = (const half_t *)a.out_w; p.slabs = a.out_slabs; p.stride = (int64_t)a.nq * a.out_n; p.N = a.out_n;
-    const dim3 grid((unsigned)(a.nq * a.KVH), (unsigned)(a.out_n / OUT_ROWS));
-    const bool ub = a.block_size % TPI == 0;
-    bool in_it = false;
-    if constexpr (D == 128)
-        if (ub && own_rows_aligned(a)) {
-            static_cast<OwnRows &>(p) = own_rows_params(a);
-            attn_rows_kernel<D, G, true, true, U, 8, false, true, false, false, true, true><<<grid, dim3(512), 0, s>>>(p);
-            in_it = true;
-        }
-    if (!in_it) {
-        if (int rc = own_rows(a, s)) return rc;
-        if (ub) attn_rows_kernel<D, G, true, true, U, 8, false, true, false, false, false, true><<<grid, dim3(512), 0, s>>>(p);
-        else attn_rows_kernel<D, G, true, true, U, 8, false, false, false, false, false, true><<<grid, dim3(512), 0, s>>>(p);
-    }
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "attention + output product launch failed: %s", hipGetErrorString(e));
-    return 0;
+    const int64_t pairs = (int64_t)a.nq * a.KVH;
+    if (pairs * (a.out_n / OUT_ROWS) > share_workgroups() && a.out_n % 128 == 0) return launch_attn_out_rows<D, G, 128>(a, p, s);
+    return launch_attn_out_rows<D, G, 64>(a, p, s);
 }
 
 template <int D, int G>

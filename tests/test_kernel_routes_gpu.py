@@ -994,16 +994,16 @@ def test_work_balanced_decode_attention_forms_its_own_rows(heads, dtype):
 
 
 @pytest.mark.parametrize("hidden,heads,kv,dim,qk_norm,dtype", [(256, 4, 4, 64, False, "float16"), (512, 8, 2, 64, False, "bfloat16"), (512, 16, 8, 128, False, "float16"), (512, 8, 8, 128, True, "bfloat16"),
-                                                               (256, 8, 2, 128, True, "float16")])
+                                                               (256, 8, 2, 128, True, "float16"), (1024, 16, 8, 128, False, "float16"), (1024, 8, 8, 128, True, "bfloat16")])
 @pytest.mark.parametrize("page", [16, 20])
 def test_decode_attention_takes_the_output_product_along(hidden, heads, kv, dim, qk_norm, dtype, page):
-    """One and two sequences whose attention multiplies its heads with the output product's columns itself: groups of one, two and four heads, slabs of two, four and eight kv heads, pages of whole
+    """One to four sequences (64 and 128 rows of the product a workgroup) whose attention multiplies its heads with the output product's columns itself: groups of one, two and four heads, slabs of two, four and eight kv heads, pages of whole
     chunks of keys and others, contexts on both sides of a round of keys (128) and of the 256 beyond which the product is a launch of its own — logits against the oracle, step by step."""
     from oracle import model_oracle as mo
     from test_engine_gpu import _run_pair
     mcfg = mo.small(hidden_size=hidden, num_hidden_layers=2, intermediate_size=512, head_dim=dim, num_attention_heads=heads, num_key_value_heads=kv, qk_norm=qk_norm, seed=heads, init_std=0.02)
-    ecfg = dict(max_num_seqs=2, max_num_batched_tokens=512, max_model_len=300, kvcache_block_size=page, num_kvcache_blocks=48)
-    for lengths in ([122], [251], [1, 126]):
+    ecfg = dict(max_num_seqs=4, max_num_batched_tokens=512, max_model_len=300, kvcache_block_size=page, num_kvcache_blocks=64)
+    for lengths in ([122], [251], [1, 126]) + (([30, 121, 1, 9], [5, 124, 17]) if hidden == 1024 else ()):
         prompts = [oracle.fill_tokens(n, 3, i, mcfg.vocab_size).tolist() for i, n in enumerate(lengths)]
         sps = [dict(temperature=0.0, max_tokens=9, ignore_eos=True)] * len(lengths)
         assert _run_pair(mcfg, ecfg, prompts, sps, dtype=dtype)["decode_steps"] >= 8
