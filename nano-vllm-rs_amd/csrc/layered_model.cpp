@@ -452,7 +452,9 @@ int LayeredModel::execute(nvr_model_runner &r, nvr_seq *const *seqs, size_t nseq
         RC(forward(r, plan));
     for (size_t i = 0; i < nseq; ++i) slot_par[(size_t)seqs[i]->state_slot] ^= 1;
     r.last_rows = R; r.last_tokens = T;
-    r.lm_parts = (int32_t)head_parts(r, (int64_t)R);
+    // the greedy choice is the first maximum of the logits as they are reported.  A scale behind the product (forward_scaled) turns their order round (a negative one), makes all of them equal (0) or
+    // rounds two neighbours to one number: the partials of the unscaled products are no use then, argmax_parts reads the scaled rows
+    r.lm_parts = spec.logit_scale == 1.0 ? (int32_t)head_parts(r, (int64_t)R) : 0;
     return NVR_OK;
 }
 

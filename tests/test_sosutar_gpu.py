@@ -285,6 +285,27 @@ def test_greedy_generation_through_the_scheduler(chunked):
             assert row.max() - row[full[k + 1]] <= 3 * TOL["float32"] * spread, f"request {sid}: token {k + 1} is not the greedy choice"
 
 
+@pytest.mark.parametrize("vocab, batch", [(112, 1), (4112, 17), (272, 33)])
+@pytest.mark.parametrize("scale", [-0.5, 0.0, 3.0, 1.0])
+def test_greedy_choice_is_the_first_maximum_of_the_scaled_logits(scale, vocab, batch):
+    """Widths and vocabularies whose head leaves arg-max partials of its unscaled products: the token is the first maximum of the logits that the step reports, whatever the scale makes of their order
+    (a negative one turns it round, 0 makes all of them equal, 3 rounds some neighbours to one number: head rows in pairs whose logits differ in the last place)."""
+    cfg = make_config([mlstm_layer()], vocab=vocab, width=256, logit_scale=scale)
+    w = make_weights(cfg, seed=31)
+    w["head"][0::2, 0] = 0
+    w["head"][1::2] = w["head"][0::2]
+    w["head"][1::2, 0] = 2.0 ** -23                                        # (logits of the greedy choice are 2 .. 4: their last place is 2^-22)
+    d = Driver(cfg, w, "bfloat16", slots=batch, pages=2 * batch, max_tokens=8 * batch, max_len=32)
+    rng = np.random.default_rng(vocab)
+    names = ["s%d" % i for i in range(batch)]
+    d.step([(n, rng.integers(0, vocab, 4)) for n in names])
+    for _ in range(3):
+        logits = d.step([(n, rng.integers(0, vocab, 1)) for n in names])
+        tokens = d.runner.sample_tokens([d.live[n] for n in names])
+        for n, t in zip(names, tokens):
+            assert t == int(np.argmax(logits[n][0])), (n, t, int(np.argmax(logits[n][0])))
+
+
 # ------------------------------------------------------------------------------------------------ designs and schedules drawn at random
 def random_design(seed):
     rng = np.random.default_rng(seed)
