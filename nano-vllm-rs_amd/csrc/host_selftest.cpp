@@ -13,6 +13,7 @@
 #include "common.h"
 #include "scheduler.h"
 #include "tokenizer.h"
+#include "kernels/slab_walk.h"
 
 namespace {
 struct Rng {                                                     // splitmix64
@@ -149,6 +150,27 @@ void tokenizer_trace(uint64_t seed) {
         for (size_t i = 0; i < back.size(); ++i) CHECK(back[i] == ids[i]);
     }
 }
+// every request of every wave of a split product that linear_slab_kernel takes lies inside its slice, and the waves' steps are the slice's columns, each once; no wave of it has less than two sets
+void slab_walks() {
+    size_t taken = 0;
+    for (int K = 32; K <= 16384; K += 32)
+        for (int S = 1; S <= K / 32; ++S) {
+            const int kslice = K / S;
+            if (K % (32 * S) || !nvr::slab_takes(kslice)) continue;
+            ++taken;
+            std::vector<int> seen((size_t)K / 32, 0);
+            CHECK(nvr::slab_steps(kslice) % nvr::SLAB_SET == 0 && nvr::slab_steps(kslice) >= 2 * nvr::SLAB_SET);
+            for (int z = 0; z < S; ++z)
+                for (int wave = 0; wave < nvr::SLAB_WAVES; ++wave)
+                    for (int step = 0; step < nvr::slab_steps(kslice); ++step) {
+                        const int k = nvr::slab_column(kslice, z, wave) + step * nvr::SLAB_STEP;
+                        CHECK(k >= z * kslice && k + 32 <= (z + 1) * kslice && k + 32 <= K);
+                        ++seen[(size_t)k / 32];
+                    }
+            for (int n : seen) CHECK(n == 1);
+        }
+    CHECK(taken > 0 && !nvr::slab_takes(32) && !nvr::slab_takes(128) && !nvr::slab_takes(1280) && nvr::slab_takes(1024) && nvr::slab_takes(3072));
+}
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -156,6 +178,7 @@ int main(int argc, char **argv) {
     for (uint64_t s = 0; s < 40; ++s) { scheduler_trace(base * 1000 + s, false); scheduler_trace(base * 2000 + s, true); }
     for (uint64_t s = 0; s < 6; ++s) block_manager_trace(base * 3000 + s);
     tokenizer_trace(base * 4000);
+    slab_walks();
     std::printf("host_selftest ok (seed %llu)\n", (unsigned long long)base);
     return 0;
 }

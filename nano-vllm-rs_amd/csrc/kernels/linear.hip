@@ -26,6 +26,7 @@
 #include <cstdlib>
 #include "kernels.h"
 #include "device_utils.h"
+#include "slab_walk.h"
 #include "../common.h"
 
 namespace nvr { namespace NVR_DT_NS {
@@ -424,17 +425,15 @@ __global__ __launch_bounds__(WAVES * 64) void linear_beside_unit_kernel(const ha
 
 // The split-k products of large weights (linear_splitk: 64 columns a workgroup, eight waves, slab blockIdx.z): what linear_skinny_kernel<4, MT, 8, EPI_SLAB> computes, with its sums' order.  A wave has
 // several rounds of requests there (12 steps of 32 k at K = 12288 in four slices), and each round waited for the one in front of it; here three sets of two steps take turns, two of them on their way
-// while the third is multiplied.  Qwen3-8B, us a
-// step, linear_skinny_kernel / so: 32 sequences of 2048 keys 5087 / 5051, 24 of 300 3740 / 3714, up to 16 sequences the same; a request behind the last step in the place of a condition costs 5 %.
+// while the third is multiplied.  Slices: slab_takes.  Qwen3-8B, us a step, linear_skinny_kernel / so: 32 sequences of 2048 keys 5087 / 5051, 24 of 300 3740 / 3714, up to 16 sequences the same.
 template <int MT>
 __global__ __launch_bounds__(512) void linear_slab_kernel(const half_t *__restrict__ x, int64_t ldx, const half_t *__restrict__ W, int T, int K, int N, float *__restrict__ y, int kslice, int64_t slab_stride,
                                                           int tiled) {
-    constexpr int NT = 4, WAVES = 8, U = 2, KS = 32 * WAVES;
+    constexpr int NT = 4, WAVES = SLAB_WAVES, U = SLAB_SET;
     __shared__ float4_t part[WAVES][NT * MT][64];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
-    const int m0 = blockIdx.y * (16 * MT), k0 = (int)blockIdx.z * kslice + wave * 32;
-    const int steps = max(0, (min(K, ((int)blockIdx.z + 1) * kslice) - k0 + KS - 1) / KS);      // of this wave
-    const int64_t step = tiled ? (int64_t)(KS / 32) * 512 : KS;
+    const int m0 = blockIdx.y * (16 * MT), k0 = slab_column(kslice, (int)blockIdx.z, wave), sets = slab_steps(kslice) / U;
+    const int64_t step = tiled ? (int64_t)(SLAB_STEP / 32) * 512 : SLAB_STEP;
     const half_t *wrow[NT], *xrow[MT];
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
@@ -449,41 +448,41 @@ __global__ __launch_bounds__(512) void linear_slab_kernel(const half_t *__restri
 #pragma unroll
         for (int j = 0; j < MT; ++j) acc[i][j] = (float4_t){0.f, 0.f, 0.f, 0.f};
     struct Set { half8_t a[U][NT], b[U][MT]; } s0, s1, s2 = {};
-    auto request = [&](Set &s, int at) {
+    auto request = [&](Set &s, int set) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int k = max(0, min(at + u, steps - 1));
+            const int k = set * U + u;
 #pragma unroll
             for (int i = 0; i < NT; ++i) s.a[u][i] = __builtin_nontemporal_load(reinterpret_cast<const half8_t *>(wrow[i] + k * step));
 #pragma unroll
-            for (int j = 0; j < MT; ++j) s.b[u][j] = *reinterpret_cast<const half8_t *>(xrow[j] + (int64_t)k * KS);
+            for (int j = 0; j < MT; ++j) s.b[u][j] = *reinterpret_cast<const half8_t *>(xrow[j] + (int64_t)k * SLAB_STEP);
         }
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto multiply = [&](const Set &s, int at) {
+    auto multiply = [&](const Set &s) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (at + u < steps)                                           // (uniform over the wave)
 #pragma unroll
-                for (int i = 0; i < NT; ++i)
+            for (int i = 0; i < NT; ++i)
 #pragma unroll
-                    for (int j = 0; j < MT; ++j) acc[i][j] = mfma16(s.a[u][i], s.b[u][j], acc[i][j]);
+                for (int j = 0; j < MT; ++j) acc[i][j] = mfma16(s.a[u][i], s.b[u][j], acc[i][j]);
         __builtin_amdgcn_sched_barrier(0);
     };
-    const int sets = (steps + U - 1) / U;
-    request(s0, 0); request(s1, U);
+    request(s0, 0); request(s1, 1);                                       // (two sets at least)
     int i = 0;                                                            // sets i and i + 1 are on their way
     for (; i + 5 <= sets; i += 3) {
-        request(s2, (i + 2) * U); multiply(s0, i * U);
-        request(s0, (i + 3) * U); multiply(s1, (i + 1) * U);
-        request(s1, (i + 4) * U); multiply(s2, (i + 2) * U);
+        request(s2, i + 2); multiply(s0);
+        request(s0, i + 3); multiply(s1);
+        request(s1, i + 4); multiply(s2);
     }
-    if (i + 2 < sets) request(s2, (i + 2) * U);
-    multiply(s0, i * U);
-    if (i + 3 < sets) request(s0, (i + 3) * U);
-    multiply(s1, (i + 1) * U); multiply(s2, (i + 2) * U);
-    if (i + 3 < sets) multiply(s0, (i + 3) * U);
+    const int left = sets - i;                                            // 2, 3 or 4
+    if (left > 2) request(s2, i + 2);
+    multiply(s0);
+    if (left > 3) request(s0, i + 3);
+    multiply(s1);
+    if (left > 2) multiply(s2);
+    if (left > 3) multiply(s0);
 #pragma unroll
     for (int i = 0; i < NT; ++i)
 #pragma unroll
@@ -670,6 +669,11 @@ int linear_splitk(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T
         // large weights (Qwen3-8B o/down: N = 4096): 64 output columns per workgroup so that an x fragment feeds four weight
         // tiles (x costs half the weight bytes instead of twice), 8 waves; with S = 4: 10.8 / 29.5 us vs 15.5 / 45 us for the
         // 16-column kernel at K = 4096 / 12288 (scratch/splitk_8b.py)
+        if (!slab_takes(e.kslice)) {
+            if (T <= 16) launch<4, 1, 8, EPI_SLAB>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K, (int)N, slabs, e, (unsigned)(N / 64), s, (unsigned)S);
+            else launch<4, 2, 8, EPI_SLAB>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K, (int)N, slabs, e, (unsigned)(N / 64), s, (unsigned)S);
+            return launch_check("linear_splitk");
+        }
         const int mt = T <= 16 ? 1 : 2;
         const dim3 grid((unsigned)(N / 64), (unsigned)((T + 16 * mt - 1) / (16 * mt)), (unsigned)S);
         if (mt == 1) linear_slab_kernel<1><<<grid, dim3(512), 0, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K, (int)N, slabs, e.kslice, e.slab_stride, e.tiled);

@@ -602,10 +602,12 @@ def test_tile_products_of_few_k_tiles_and_ragged_edges(T, K, N):
         assert np.all(np.abs(s.astype(np.float64).sum(0) - ref) <= bound)
 
 
-@pytest.mark.parametrize("T,K,N,S", [(20, 1024, 16384, 4), (3, 1056, 12288, 1), (32, 2592, 6144, 1), (17, 3616, 4096, 1), (1, 6144, 4096, 2)])
+@pytest.mark.parametrize("T,K,N,S", [(20, 1024, 16384, 4), (3, 1056, 12288, 1), (32, 2592, 6144, 1), (17, 3616, 4096, 1), (1, 6144, 4096, 2),
+                                     (20, 1024, 12288, 8), (4, 1152, 12288, 9), (7, 128, 98304, 1), (32, 96, 131072, 3),
+                                     (16, 4096, 4096, 4), (31, 3072, 4096, 2), (2, 2048, 8192, 1), (32, 5120, 4096, 2), (17, 3584, 4096, 1), (5, 4096, 3200, 1)])
 def test_split_products_of_large_weights(T, K, N, S):
-    """Slabs of weights of 24 MiB and more, 1 to 15 steps of a wave (one to eight sets of two steps; last sets of one step; waves of one step less than others), one and two row tiles: against 64 bits, and
-    the tiled copy's bits."""
+    """Slabs of weights of 24 MiB and more, no step to 16 steps of a wave (slices of 32 to 224 columns, odd steps, waves of one step less than others; two to eight whole sets of two), one and two row tiles:
+    against 64 bits, and the tiled copy's bits."""
     rng, l = np.random.default_rng(T + K), nvr.lib()
     x, W = _bits(rng, (T, K), 0.5), _bits(rng, (N, K), 0.1)
     d_x, d_W = dev(x), dev(W)
