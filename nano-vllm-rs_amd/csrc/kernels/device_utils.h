@@ -58,10 +58,10 @@ __device__ __forceinline__ float dot2(half2_t a, half2_t b, float c) {
 __device__ __forceinline__ float sigmoid_fast(float x) { return __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
 // what the gate g of a gated feed-forward is multiplied by: silu(g) = g sigmoid(g); the tanh form of gelu, g (1 + tanh(sqrt(2/pi) (g + 0.044715 g^3))) / 2 = g sigmoid(2 sqrt(2/pi) (g + 0.044715 g^3))
 __device__ __forceinline__ float gate_factor(float g, bool gelu) { return sigmoid_fast(gelu ? 1.5957691216057308f * (g + 0.044715f * g * g * g) : g); }
-// the clamped gated unit of the layer lists, min(g, limit) sigmoid(alpha min(g, limit)) (clamp(u, +-limit) + 1), in the same instructions
-__device__ __forceinline__ float clamped_unit_fast(float g, float u, float limit, float alpha) {
-    g = fminf(g, limit);
-    return g * sigmoid_fast(alpha * g) * (fminf(fmaxf(u, -limit), limit) + 1.0f);
+// the clamped gated unit of the layer lists, min(g, limit) sigmoid(alpha min(g, limit)) (clamp(u, +-limit) + 1), as every kernel of theirs has it: a row's unit does not depend on the size of its step
+__device__ __forceinline__ float clamped_unit(float g, float u, float limit, float alpha) {
+    g = fminf(g, limit); u = fminf(fmaxf(u, -limit), limit);
+    return g / (1.0f + expf(-alpha * g)) * (u + 1.0f);
 }
 // gelu with the error function, z Phi(z), for results that are rounded to 16 bits: erfc by the rational approximation 7.1.26 of Abramowitz and Stegun, Handbook of Mathematical
 // Functions (absolute error below 1.5e-7), one v_rcp and one v_exp; z Phi(z) = max(z, 0) - |z| erfc(|z| / sqrt 2) / 2

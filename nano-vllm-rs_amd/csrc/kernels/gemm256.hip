@@ -34,7 +34,7 @@ namespace nvr { namespace NVR_DT_NS {
 
 enum { GEPI_F16 = 0, GEPI_RESID = 1, GEPI_SILU = 2, GEPI_ROPE = 3, GEPI_LMHEAD = 4, GEPI_RELU2 = 5, GEPI_GELU = 6, GEPI_GELU_ERF = 7, GEPI_QKN = 8, GEPI_CLAMP = 9 };   // GELU_ERF: y = gelu(x·Wᵀ) with the error function (from the unrounded product); RELU2: y = max(x·Wᵀ, 0)² (the product rounded to 16 bits first, as the unfused pair of launches does)
 constexpr bool g_rope(int epi) { return epi == GEPI_ROPE || epi == GEPI_QKN; }      // QKN: RMSNorm over the columns of every q and k head in front of the rotation
-constexpr bool g_glu(int epi) { return epi == GEPI_SILU || epi == GEPI_GELU || epi == GEPI_CLAMP; }      // gate and up rows in one tile, out = act(gate) * up (GELU: the tanh form; CLAMP: clamped_unit_fast, rows of y ldo apart)
+constexpr bool g_glu(int epi) { return epi == GEPI_SILU || epi == GEPI_GELU || epi == GEPI_CLAMP; }      // gate and up rows in one tile, out = act(gate) * up (GELU: the tanh form; CLAMP: clamped_unit, rows of y ldo apart)
 //   // RESID: y is the residual stream: y <- fp16(y + fp16(x·Wᵀ)) (qwen3.rs:382,389)
 // LMHEAD (r06): the LM head over >= 128 rows (ParallelLMHead::compute_logits, embed_head.rs:292-306, + the greedy branch of Sampler::forward,
 // sampler.rs:109-112): W = the [V, hidden] head, nothing is written as fp16 — every tile leaves (max, lowest vocabulary index) of its 256
@@ -409,7 +409,7 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
                             const float gf = (float)to_half_rn(acc[0][i][hB][j][e]), uf = (float)to_half_rn(acc[1][i][hB][j][e]);
-                            if constexpr (EPI == GEPI_CLAMP) h[e] = to_half_rn(clamped_unit_fast(gf, uf, epi.limit, epi.alpha));
+                            if constexpr (EPI == GEPI_CLAMP) h[e] = to_half_rn(clamped_unit(gf, uf, epi.limit, epi.alpha));
                             else {
                                 const float sg = gate_factor(gf, EPI == GEPI_GELU);
                                 h[e] = to_half_rn(__fmul_rn(__fmul_rn(gf, sg), uf));

@@ -84,7 +84,7 @@ __device__ __forceinline__ void wait_ring(int younger) {
     }
 }
 
-constexpr bool t_glu(int epi) { return epi == TEPI_SILU || epi == TEPI_CLAMP; }      // gate and up rows in one tile (CLAMP: clamped_unit_fast, rows of y ldo apart)
+constexpr bool t_glu(int epi) { return epi == TEPI_SILU || epi == TEPI_CLAMP; }      // gate and up rows in one tile (CLAMP: clamped_unit, rows of y ldo apart)
 
 // W row of local row r (0..15) of the workgroup's 16-row n-tile `t` (0..7)
 template <int EPI>
@@ -430,7 +430,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tiled_kernel(const half_t *__rest
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float gf = (float)to_half_rn(acc[i][j][e]), uf = (float)to_half_rn(acc[i + 2][j][e]);
-                    if constexpr (EPI == TEPI_CLAMP) h[i][e] = to_half_rn(clamped_unit_fast(gf, uf, epi.limit, epi.alpha));
+                    if constexpr (EPI == TEPI_CLAMP) h[i][e] = to_half_rn(clamped_unit(gf, uf, epi.limit, epi.alpha));
                     else {
                         const float sg = gate_factor(gf, epi.gelu);
                         h[i][e] = to_half_rn(__fmul_rn(__fmul_rn(gf, sg), uf));

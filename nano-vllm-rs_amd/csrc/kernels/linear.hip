@@ -729,7 +729,8 @@ int linear_gelu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t
 
 // gate_up GEMM + the clamped gated unit of a layer list: W [2I, K] (gate rows, then up rows), out [T, ldo].  Few rows, whose product the weight-row kernel takes: the unit
 // is a launch of its own otherwise, and a launch behind a launch is about 5 us whatever it holds (16 rows of 1024, I = 3072: 11.3 -> 6.3 us together).  Shapes of the LDS tiles, routed as linear()
-// routes the plain product: the unit by itself reads both halves of every row again and the product writes twice the columns (16384 rows of 1024, I = 3072: 201 + 59 us -> 168).
+// routes the plain product: the unit by itself reads both halves of every row again and the product writes twice the columns (16384 rows of 1024, I = 3072: 201 + 59 us -> 192; with
+// the unit on v_rcp and the fast exponential 168, but then a row's unit would depend on the size of its step, and be off by a few last places of f32 more).
 static bool clamped_glu_on_tiles(int64_t T, int64_t K, int64_t I, int64_t ldx) {
     return K % 32 == 0 && I % 64 == 0 && gemm_tiled_ok(T, K, I, ldx) && ((gemm256_silu_ok(T, K, I, ldx) && rows_on_256(T, K, 2 * I) > 0) || !stream_preferred(T, 2 * I));
 }

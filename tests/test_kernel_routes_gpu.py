@@ -517,6 +517,36 @@ def test_layer_list_clamped_unit_on_tiles(width, ff, batch, tokens):
     _compare_layer_rows(cfg, w, "bfloat16", base, [got["s%d" % i] for i in range(batch)])
 
 
+@pytest.mark.parametrize("width,ff,batch,tokens", [(64, 2112, 9, 34), (256, 2176, 3, 300), (1024, 3072, 40, 100)])
+def test_layer_list_clamped_unit_does_not_depend_on_the_step(width, ff, batch, tokens):
+    """A row's clamped unit in a prompt step (on 32- to 256-row tiles) and in portions of up to 32 rows: bit for bit.  Every product of the model has one term (the mixer's output none), so that the
+    order of its sums does not matter; half of the stream's columns hold the token's embedding, the others the unit and nothing else, scaled until its smallest values (gates down to -12) count."""
+    import rugudra_util as u
+    half, limit = width // 2, 7.0
+    cfg = u.make_config([u.retention_layer(2, 32, 32, ff=ff, limit=limit)], width=width, taps=2, embedding_scale=1.0, residual_mult=1.0)
+    w = u.make_weights(cfg, seed=width)
+    rng = np.random.default_rng(ff)
+    w["embed"][:, half:] = 0
+    w["l0.mix.o"][:] = 0
+    for name, scale in (("l0.mlp.gate", 4.0), ("l0.mlp.up", 2.0)):
+        w[name][:] = 0
+        w[name][np.arange(ff), rng.integers(0, half, ff)] = scale * rng.choice([-1.0, 1.0], ff)
+    w["l0.mlp.down"][:] = 0
+    w["l0.mlp.down"][np.arange(half, width), rng.permutation(ff)[:half]] = 2.0 ** 20
+    w["head"][:] = 0
+    w["head"][np.arange(97), half + np.arange(97) * 7 % half] = 1
+    base = [rng.integers(0, 97, tokens) for _ in range(batch)]
+    rows = []
+    for portion in (tokens, 32):
+        d = u.Driver(cfg, w, dtype="bfloat16", slots=batch, pages=batch * (tokens // 16 + 2), max_tokens=batch * tokens, max_len=512)
+        if portion == tokens:
+            got = d.step([("s%d" % i, t) for i, t in enumerate(base)])
+            rows.append(np.concatenate([got["s%d" % i] for i in range(batch)]))
+        else:
+            rows.append(np.concatenate([d.run_alone(t, cuts=[portion]) for t in base]))
+    assert np.abs(rows[0]).max() > 0 and np.array_equal(rows[0].view(np.uint32), rows[1].view(np.uint32)), (rows[0] != rows[1]).mean()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("taps,width,batch", [(2, 64, 130), (3, 1028, 3), (4, 64, 130), (4, 1088, 9), (5, 64, 130)])
 def test_layer_list_norm_and_convolution_rows(dtype, taps, width, batch):
