@@ -1051,7 +1051,7 @@ __global__ __launch_bounds__(512) void attn_prefix_kernel(AttnParams p, int nq, 
 #pragma unroll
             for (int e = 0; e < 4; ++e) { s[mt][e] *= scale2; mx = fmaxf(mx, s[mt][e]); }
         mx = xor32_partner_max(xor16_partner_max(mx));
-        const float mn = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f(m - mn);
+        const float mn = fmaxf(m, mx), ms = mn == -INFINITY ? 0.f : mn, alpha = __builtin_amdgcn_exp2f(m - ms);      // (only keys of score -inf so far: weights of 0)
         const bool moved = mn != m;
         m = mn;
         half8_t pf;
@@ -1059,7 +1059,7 @@ __global__ __launch_bounds__(512) void attn_prefix_kernel(AttnParams p, int nq, 
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) { const half_t w = (half_t)__builtin_amdgcn_exp2f(s[mt][e] - mn); rs += (float)w; pf[mt * 4 + e] = w; }
+            for (int e = 0; e < 4; ++e) { const half_t w = (half_t)__builtin_amdgcn_exp2f(s[mt][e] - ms); rs += (float)w; pf[mt * 4 + e] = w; }
         l = fmaf(l, alpha, rs);
         if (__any(moved)) {
 #pragma unroll
@@ -1160,7 +1160,10 @@ __global__ __launch_bounds__(512) void attn_prefix_kernel(AttnParams p, int nq, 
             v += *reinterpret_cast<const float4_t *>(own_o + ((sq * WPS + w) * G + i) * PRE_OS + c) * f;
             L = fmaf(own_ml[sq * WPS + w][i][1], f, L);
         }
-        *reinterpret_cast<half4_t *>(p.out + ((int64_t)(t0 + sq) * p.H + g * G + i) * D + c) = (half4_t){(half_t)(v[0] / L), (half_t)(v[1] / L), (half_t)(v[2] / L), (half_t)(v[3] / L)};
+        half4_t hv;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) hv[e] = (half_t)(L > 0.f ? v[e] / L : 0.f);      // (as merge_partitions: no key of a finite score, or NaN among them)
+        *reinterpret_cast<half4_t *>(p.out + ((int64_t)(t0 + sq) * p.H + g * G + i) * D + c) = hv;
     }
 }
 

@@ -487,6 +487,54 @@ def test_shared_prefix_decode_attention_in_one_launch(B, G, KVH, bs, P, own):
     assert np.all(np.abs(x - y) <= 1e-3 + 3 * 2.0 ** -10 * np.abs(x)), np.abs(x - y).max()
 
 
+@pytest.mark.parametrize("B,G,KVH,P", [(33, 2, 8, 5), (64, 4, 8, 9), (40, 1, 8, 4), (150, 2, 8, 8)])
+@pytest.mark.parametrize("masked", ["first", "one_wave", "prefix", "everything", "nan_query"])
+def test_shared_prefix_decode_attention_with_infinities(B, G, KVH, P, masked):
+    """Keys of score -inf among the shared ones (the first 32, all of one wave's chunks, the whole prefix; everything: zeros, as the other decode kernels leave), and a query of NaN (zeros) beside others
+    that must not notice: against 64 bits, with the bound of the test above for the rounding of the prefix's weights and of the result."""
+    l, D, H, bs = nvr.lib(), 128, G * KVH, 64
+    rng = np.random.default_rng(B + P)
+    S, own = P * bs, [(7 * i) % 60 + 1 for i in range(B)]
+    pool = P + B
+    bt = np.zeros((B, P + 1), np.int32)
+    bt[:, :P], bt[:, P] = np.arange(P), P + np.arange(B)
+    q = rng.standard_normal((B, H, D)).astype(F16)
+    q[..., 0] = 1
+    k, v = (rng.standard_normal((pool, bs, KVH, D)).astype(F16) for _ in range(2))
+    keys = k.reshape(pool * bs, KVH, D)
+    if masked == "first":
+        keys[:32, :, 0] = -np.inf
+    elif masked == "one_wave":
+        for x in range(3, S // 32, 8):
+            keys[x * 32:x * 32 + 32, :, 0] = -np.inf
+    elif masked == "prefix":
+        keys[:S, :, 0] = -np.inf
+    elif masked == "everything":
+        keys[..., 0] = -np.inf
+    want = np.zeros((B, H, D))
+    for b in range(B):
+        rows = np.concatenate([np.arange(S), (P + b) * bs + np.arange(own[b])])
+        kb, vb = keys[rows].astype(np.float64), v.reshape(pool * bs, KVH, D)[rows].astype(np.float64)
+        for g in range(KVH):
+            sc = q[b, g * G:(g + 1) * G].astype(np.float64) @ kb[:, g].T * D ** -0.5
+            m = sc.max(1, keepdims=True)
+            if np.isfinite(m).all():
+                w = np.exp(sc - m)
+                want[b, g * G:(g + 1) * G] = w / w.sum(1, keepdims=True) @ vb[:, g]
+    if masked == "nan_query":
+        q[1, 0] = np.nan
+        want[1, 0] = 0
+    d_q, d_k, d_v, d_bt, d_ctx = dev(q), dev(k), dev(v), dev(bt), dev(np.asarray([S + o for o in own], np.int32))
+    meta = nvr.AttnMetaC()
+    meta.context_lens, meta.block_tables, meta.max_blocks, meta.batch, meta.max_context_len = d_ctx.ptr, d_bt.ptr, P + 1, B, S + max(own)
+    ws = nvr.DeviceBuffer(l.nvr_paged_attn_workspace_bytes(B, H, D, S + bs))
+    out = nvr.DeviceBuffer(B * H * D * 2)
+    nvr.check(l.nvr_fill_const(out.ptr, B * H * D, C.c_float(float("nan")), None))
+    nvr.check(l.nvr_paged_attn_decode_shared(d_q.ptr, H * D, d_k.ptr, d_v.ptr, C.byref(meta), H, KVH, D, bs, D ** -0.5, S, None, None, None, out.ptr, ws.ptr, None))
+    got = out.to_numpy((B, H, D), F16).astype(np.float64)
+    assert np.all(np.abs(got - want) <= 1e-3 + 3 * 2.0 ** -10 * np.abs(want)), np.nanmax(np.abs(got - want))
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("heads,vdim,ff,batch", [(1, 30, 48, 1), (3, 32, 48, 16), (5, 4, 64, 17), (2, 64, 2064, 32), (4, 96, 40, 33)])
 def test_layer_list_gated_head_norm_and_clamped_unit(dtype, heads, vdim, ff, batch):
