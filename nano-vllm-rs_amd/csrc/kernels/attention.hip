@@ -1212,13 +1212,29 @@ static bool own_rows_aligned(const AttnArgs &a) {
 }
 static OwnRows own_rows_params(const AttnArgs &a) { return OwnRows{(const half_t *)a.qn_w, (const half_t *)a.kn_w, a.qk_eps, a.pos, a.slots, a.cos_t, a.sin_t}; }
 
-// A whole batch behind its prefix, up to as many sequences a workgroup as give every CU one, and as long as reading the shared keys for each workgroup costs less than the second launch: each 256 keys
-// are 1.6 us more (0.5-0.85 in the launch of their own).  us a layer, two launches / one, 75 own keys, groups of 2: 33 sequences behind 256 / 512 / 1024 / 2048 keys 13.4 14.7 16.3 19.3 / 11.0 12.6 15.8
-// 21.9; 64 16.0 17.3 19.4 22.8 / 11.7 13.4 16.8 23.5; 128 19.7 21.8 24.3 25.5 / 14.7 16.6 19.6 26.1; 256 27.4 29.2 30.5 33.4 / 22.2 24.1 27.3 34.0.
-static bool prefix_in_one_launch(const AttnArgs &a, int64_t pairs) {
-    const int G = a.H / a.KVH;
-    return !a.shared_rows && a.shared_len <= 1536 && (a.block_size & (a.block_size - 1)) == 0 && a.block_size % 64 == 0 && pairs <= (int64_t)share_workgroups() * (G <= 2 ? 8 : 4) && a.ldq % 8 == 0 &&
-           (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.out) & 15) == 0;
+// A whole batch behind its prefix in one launch or two.  One: as many sequences a workgroup (NS: 1, 2, 4 or 8) as give every CU one workgroup.  It saves the second launch (5 us) and has no partials in
+// memory, but every workgroup reads the shared keys (256 of them 1.6 us, 0.5-0.85 in the launch of their own), and a sequence's own keys are walked by 8 / NS waves, where the two launches give each pair four and
+// cut long ones over the idle CUs: the longest sequence is waited for.  So the bound on its own keys goes by NS, a little further where all are long (then the bytes count on either side), half as far
+// (NS 4 and 8: three quarters) beyond 512 shared keys: over 2520 shapes the choice is 0.5 % above the better of the two, one launch throughout 14.6 %, two 14.4 %.  us a launch, two / one, groups of 2 of 8 kv heads behind 512 keys; all of so many own keys; one of them among 15:
+//   16 sequences (NS 1) 256 own 19.0 / 15.0, 512 21.1 / 19.6, 1000 behind 256 23.9 / 29.7; one of 2000 behind 256 27.6 / 48.4
+//   33 (NS 2) 64 14.5 / 11.2, 192 18.5 / 17.2, 256 20.4 / 20.2; one of 192 14.6 / 14.9, of 256 15.7 / 17.5
+//   64 (NS 2) 64 16.8 / 11.8, 256 25.6 / 21.3; one of 192 16.3 / 15.2, of 256 17.2 / 17.6, of 2000 behind 256 47 / 87
+//   65 (NS 4) 64 17.3 / 14.0, 128 21.1 / 19.8, 192 24.8 / 25.8; one of 96 16.4 / 14.8, of 128 16.1 / 17.3, of 256 17.2 / 27.5
+//   128 (NS 4) 64 20.0 / 14.6, 192 31.4 / 27.1; one of 128 17.4 / 17.4, of 192 17.7 / 22.5
+//   129 (NS 8) 64 20.7 / 19.7, 128 27.0 / 31.5; one of 64 18.5 / 17.2, of 96 18.6 / 22.0
+//   256 (NS 8) 64 25.4 / 21.1, 128 35.2 / 33.8; one of 64 19.2 / 17.5, of 96 19.5 / 22.2
+// and behind 1024: 33 of 96 17.2 / 16.5, of 192 18.8 / 20.3; 128 of 64 21.3 / 17.9, one of 128 19.2 / 20.1.  Below 32 pairs the launch of the shared keys is cut over idle CUs too: 2 sequences of 2 kv
+// heads behind 512, 75 own 11.4 / 9.3, 250 11.8 / 12.8, behind 1024, 75 own 12.4 / 13.0.
+int32_t attn_prefix_launches(int64_t nq, int64_t H, int64_t KVH, int64_t shared_len, int64_t longest, int64_t mean) {
+    const int64_t G = H / std::max<int64_t>(KVH, 1), pairs = nq * KVH, cus = share_workgroups(), prefix = pairs < 32 ? 2 * shared_len : shared_len;
+    if (prefix > 1024 || pairs > cus * (G <= 2 ? 8 : 4)) return 2;
+    const int64_t bound = pairs <= cus ? (pairs < 96 ? 256 : 384) : pairs <= 2 * cus ? std::min<int64_t>(192 + mean / 2, 256) : pairs <= 4 * cus ? 96 + mean / 2 : 64;
+    return longest <= (prefix <= 512 ? bound : pairs <= 2 * cus ? bound / 2 : bound * 3 / 4) ? 1 : 2;
+}
+static bool prefix_in_one_launch(const AttnArgs &a) {
+    return !a.shared_rows && (a.block_size & (a.block_size - 1)) == 0 && a.block_size % 64 == 0 && a.ldq % 8 == 0 && (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.out) & 15) == 0 &&
+           (int64_t)a.nq * a.KVH <= (int64_t)share_workgroups() * (a.H / a.KVH <= 2 ? 8 : 4) &&
+           (a.prefix_launches ? a.prefix_launches : attn_prefix_launches(a.nq, a.H, a.KVH, a.shared_len, a.max_ctx - a.shared_len, 0)) == 1;
 }
 template <int G, int NS>
 static int launch_prefix(const AttnParams &p, int nq, int shared_len, hipStream_t s) {
@@ -1396,7 +1412,7 @@ static int launch_attn(const AttnArgs &a, bool paged, hipStream_t s) {
         }
     }
     if constexpr (D == 128 && G <= 4)
-        if (shared && prefix_in_one_launch(a, pairs)) {
+        if (shared && prefix_in_one_launch(a)) {
             if (int rc = own_rows(a, s)) return rc;
             const int64_t ns = (pairs + share_workgroups() - 1) / share_workgroups();     // sequences of a workgroup: one workgroup per CU
             if (ns <= 1) return launch_prefix<G, 1>(p, a.nq, a.shared_len, s);

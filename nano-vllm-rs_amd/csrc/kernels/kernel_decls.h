@@ -166,6 +166,8 @@ int gemm256_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, 
 
 size_t attn_workspace_bytes(int64_t nq, int64_t H, int64_t D, int64_t max_ctx);
 bool attn_out_rides(int64_t nq, int64_t H, int64_t KVH, int64_t D, int64_t N, int64_t max_ctx);   // whether a decode step's attention takes the output product of N rows along (AttnArgs::out_w)
+// launches (1 or 2) of the attention behind a prefix of shared_len tokens of the whole batch: longest, mean: keys that its sequences have behind it
+int32_t attn_prefix_launches(int64_t nq, int64_t H, int64_t KVH, int64_t shared_len, int64_t longest, int64_t mean);
 int64_t attn_brief_context(int64_t nq, int64_t H, int64_t KVH);   // contexts up to it (0: none) have a decode attention of their own: worth a captured step of their own
 int attention(const AttnArgs &a, bool paged, hipStream_t s);
 

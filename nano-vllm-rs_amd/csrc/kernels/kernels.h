@@ -49,6 +49,8 @@ struct AttnArgs {
     // paged decode with `tickets`: the caller knows the contexts are RAGGED (their sum is well below nq * max_ctx) and asks for the work-balanced form
     // (attn_share_kernel: one workgroup per CU over equal shares of all keys) wherever it can run — not only where the pair count asks for it
     bool ragged;
+    // behind a prefix that the whole batch shares: launches that the caller wants (1 or 2, attn_prefix_launches: it knows the contexts themselves, not only their bound); 0: chosen by max_ctx
+    int32_t prefix_launches;
     // paged decode, qn_w not null: the step's own rows in q's buffer ([H q heads][KVH k heads][KVH v heads] per row, stride ldq) are not normed, rotated and stored yet (rope_store_kv with the two
     // norms' weights): the attention does that first, in its own launch where its kernel can (attention.hip: QKN), else by that launch in front
     const half_bits *qn_w, *kn_w; float qk_eps;

@@ -743,7 +743,8 @@ int64_t nvr_model_runner::shared_prefix_plan(nvr_seq *const *seqs, size_t nseq, 
     return S;
 }
 
-// a captured decode step is a function of (batch size, context bucket, shared-prefix length, whole batch or a group of it, logits wanted)
+// a captured decode step is a function of (batch size, context bucket, shared-prefix length, whole batch or a group of it, logits wanted) and of the form of its attention: the work-balanced one,
+// or behind a prefix of the whole batch two launches instead of one (a step is never both)
 static inline uint64_t graph_key(bool want_logits, size_t nseq, int64_t bucket, int64_t shared_len, bool group, bool ragged) {
     return ((uint64_t)want_logits << 63) | ((uint64_t)group << 62) | ((uint64_t)ragged << 61) | ((uint64_t)nseq << 44) | ((uint64_t)(shared_len / 64) << 24) | (uint64_t)(bucket / 256);   // (0: the brief contexts in front of the first 256)
 }
@@ -762,6 +763,11 @@ bool nvr_model_runner::ragged_batch(size_t nseq, int64_t sum_ctx, int64_t max_ct
     // not below six units per CU in all: the step is then launch-bound and the per-pair launch's shorter ramp wins (12 sequences of 20..1500 keys: 1.08
     // against 1.24 ms per step; 8 of 64..8192 keys — 2040 units — 1.65 -> 1.33 the other way)
     return pairs <= 1024 && max_ctx * (int64_t)nseq * 100 >= sum_ctx * 130 && units >= 6 * cus;
+}
+// A decode batch that shares a prefix as a whole: by the contexts of the step itself, not by the bound it is captured for (each form has a captured step of its own)
+int32_t nvr_model_runner::prefix_launches(size_t nseq, int64_t sum_ctx, int64_t max_ctx) const {
+    if (f32 || decode_shared_len <= 0 || decode_shared_rows < (int64_t)nseq) return 0;
+    return KD(attn_prefix_launches((int64_t)nseq, H, KVH, decode_shared_len, max_ctx - decode_shared_len, sum_ctx / (int64_t)nseq - decode_shared_len));
 }
 
 // Prefill on tensor-parallel ranks as TWO micro-batches of whole sequences (row g, nvr_runner_set_tp_prefill_overlap(r, 2)): rows [0, mb_rows)
@@ -924,6 +930,7 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
             a.block_size = (int32_t)block_size; a.workspace = attn_ws; a.workspace_bytes = attn_ws_bytes; a.tickets = attn_tickets;
             a.shared_len = (int32_t)decode_shared_len;
             a.ragged = decode_ragged;
+            a.prefix_launches = decode_prefix_launches;
             if (mc.qk_norm && !qkv_norms_rows(T, false)) { a.qn_w = w.q_norm; a.kn_w = w.k_norm; a.qk_eps = mc.rms_norm_eps; a.pos = pos; a.slots = slots; a.cos_t = cos_t; a.sin_t = sin_t; }
             if (decode_shared_len > 0 && decode_shared_rows < T) {     // a group inside the batch: per-row kv0, member rows, member count
                 a.shared_kv0 = (const int32_t *)(in_dev + off_dec + dof_skv0); a.shared_rows = (const int32_t *)(in_dev + off_dec + dof_srows);
@@ -1161,6 +1168,7 @@ int nvr_model_runner::execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill
         decode_shared_len = shared_prefix_plan(seqs, nseq, (int32_t *)(hd + dof_skv0), (int32_t *)(hd + dof_srows), (int32_t *)(hd + dof_scount),
                                                &decode_shared_rows);
         decode_ragged = ragged_batch(nseq, sum_ctx, (cfg.enforce_eager || graphs_disabled) ? max_ctx : (max_ctx + 255) / 256 * 256);
+        decode_prefix_launches = prefix_launches(nseq, sum_ctx, max_ctx);
     }
     // one H2D per array actually used this step (K19)
     auto up = [&](size_t off, size_t bytes) { return hipMemcpyAsync(in_dev + off, in_host + off, bytes, hipMemcpyHostToDevice, stream); };
@@ -1197,7 +1205,7 @@ int nvr_model_runner::execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill
 
     // decode: replay a hipGraph captured per (batch size, context bucket) — execute_with_cuda_graph :303-326
     const int64_t bucket = context_bucket(nseq, max_ctx);
-    const uint64_t key = graph_key(want_logits, nseq, bucket, decode_shared_len, decode_shared_len > 0 && decode_shared_rows < (int64_t)nseq, decode_ragged);
+    const uint64_t key = graph_key(want_logits, nseq, bucket, decode_shared_len, decode_shared_len > 0 && decode_shared_rows < (int64_t)nseq, decode_ragged || decode_prefix_launches == 2);
     auto it = graphs.find(key);
     if (it == graphs.end()) {
         if (graphs.size() >= (size_t)env.max_graphs) {   // a long-lived engine sees many (batch size, bucket) pairs: bound the cache
@@ -1257,6 +1265,7 @@ int nvr_model_runner::execute_decode_ahead(nvr_seq *const *seqs, size_t nseq, in
     decode_shared_len = shared_prefix_plan(seqs, nseq, (int32_t *)(hd + dof_skv0), (int32_t *)(hd + dof_srows), (int32_t *)(hd + dof_scount),
                                            &decode_shared_rows);
     decode_ragged = ragged_batch(nseq, sum_ctx, (cfg.enforce_eager || graphs_disabled) ? max_ctx : (max_ctx + 255) / 256 * 256);
+    decode_prefix_launches = prefix_launches(nseq, sum_ctx, max_ctx);
     NVR_HIP_CHECK(hipMemcpyAsync(in_dev + off_dec + dof_pos, hd + dof_pos, dof_bt + nseq * max_blocks_per_seq * 4 - dof_pos, hipMemcpyHostToDevice, stream));
     last_rows = nseq; last_prefill = false; last_tokens = (int64_t)nseq;
     lm_parts = KD(lm_head_parts((int64_t)nseq, Hd, Vl, Hd));
@@ -1265,7 +1274,7 @@ int nvr_model_runner::execute_decode_ahead(nvr_seq *const *seqs, size_t nseq, in
     const int64_t T = (int64_t)nseq;
     if (cfg.enforce_eager || graphs_disabled) return forward(T, T, false, max_ctx);
     const int64_t bucket = context_bucket(nseq, max_ctx);
-    const uint64_t key = graph_key(want_logits, nseq, bucket, decode_shared_len, decode_shared_len > 0 && decode_shared_rows < (int64_t)nseq, decode_ragged);
+    const uint64_t key = graph_key(want_logits, nseq, bucket, decode_shared_len, decode_shared_len > 0 && decode_shared_rows < (int64_t)nseq, decode_ragged || decode_prefix_launches == 2);
     auto it = graphs.find(key);
     if (it == graphs.end()) {
         // flushing the cache needs an idle stream, and the current step is still running: decline — the engine rolls the

@@ -82,9 +82,11 @@ struct nvr_model_runner {
     std::map<uint64_t, hipGraphExec_t> graphs;
     size_t last_rows = 0; bool last_prefill = false; int64_t last_tokens = 0;
     int64_t decode_shared_len = 0;                       // the last decode step: tokens its sharing group holds in the same leading blocks
+    int32_t decode_prefix_launches = 0;                  // the last decode step: launches of its attention where the whole batch shares a prefix (attn_prefix_launches), else 0
     bool decode_ragged = false;                          // the decode step's contexts are ragged enough for the work-balanced attention launch (ragged_batch)
     bool qkv_norms_rows(int64_t T, bool is_prefill) const;
     bool ragged_batch(size_t nseq, int64_t sum_ctx, int64_t max_ctx) const;
+    int32_t prefix_launches(size_t nseq, int64_t sum_ctx, int64_t max_ctx) const;
     int64_t decode_shared_rows = 0;                      // ... and how many of the step's sequences belong to that group (== batch: all)
     nvr::Comm comm;
     bool graphs_disabled = false;   // set when capture with RCCL nodes fails: fall back to eager launches

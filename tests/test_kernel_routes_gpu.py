@@ -458,6 +458,10 @@ def test_brief_decode_attention_against_partitions(B, G, KVH, D, bs, ctx, bound)
     (256, 1, 8, 64, 24, [64 + i % 3 for i in range(256)]),
     (2047, 2, 1, 64, 1, [i % 7 for i in range(2047)]),                                     # one kv head
     (129, 4, 8, 64, 2, [40] * 129), (40, 2, 8, 64, 25, [9] * 40),                           # beside the rule: more workgroups than CUs, a longer prefix
+    (2, 2, 8, 64, 4, [256, 0]), (2, 2, 8, 64, 4, [257, 1]), (12, 4, 8, 128, 4, [384] + [5] * 11), (12, 4, 8, 128, 4, [385] + [5] * 11),     # both sides of the rule: one sequence a workgroup
+    (33, 2, 8, 64, 8, [192] + [31] * 32), (64, 4, 8, 64, 16, [1 + (3 * i) % 96 for i in range(64)]), (64, 1, 8, 64, 16, [97] * 64),          # two
+    (65, 4, 8, 64, 7, [(17 * i) % 97 for i in range(65)]), (127, 2, 8, 256, 4, [48] * 127), (66, 2, 8, 64, 2, [97] * 66),                   # four
+    (131, 2, 8, 64, 5, [(29 * i) % 65 for i in range(131)]), (255, 1, 8, 64, 16, [32] * 255), (255, 1, 8, 64, 16, [33] * 255),              # eight
 ])
 def test_shared_prefix_decode_attention_in_one_launch(B, G, KVH, bs, P, own):
     """Shared and own keys of a batch in one launch (1, 2, 4 and 8 sequences a workgroup, groups of 1, 2 and 4) against the plain kernel on the same inputs: f32 sums in another order, the prefix's
@@ -1087,6 +1091,20 @@ def test_decode_attention_takes_the_output_product_along(hidden, heads, kv, dim,
         prompts = [oracle.fill_tokens(n, 3, i, mcfg.vocab_size).tolist() for i, n in enumerate(lengths)]
         sps = [dict(temperature=0.0, max_tokens=9, ignore_eos=True)] * len(lengths)
         assert _run_pair(mcfg, ecfg, prompts, sps, dtype=dtype)["decode_steps"] >= 8
+
+
+@pytest.mark.parametrize("eager", [False, True])
+def test_decode_behind_a_shared_prefix_while_own_contexts_grow(eager):
+    """Three requests behind 512 tokens whose longest passes 128 tokens of its own on the way: one launch before, two behind it, each form a captured step of its own — logits against the oracle, step
+    by step."""
+    from oracle import model_oracle as mo
+    from test_engine_gpu import _run_pair
+    mcfg = mo.small(seed=9, hidden_size=512, num_attention_heads=4, num_key_value_heads=2, head_dim=128, intermediate_size=768, num_hidden_layers=2)
+    ecfg = dict(max_num_seqs=4, max_num_batched_tokens=2048, max_model_len=768, kvcache_block_size=64, num_kvcache_blocks=60)
+    system = oracle.fill_tokens(512, 4, 7, mcfg.vocab_size).tolist()
+    prompts = [system + oracle.fill_tokens(n, 4, 100 + n, mcfg.vocab_size).tolist() for n in (120, 3, 60)]
+    r = _run_pair(mcfg, ecfg, prompts, [dict(temperature=0.0, max_tokens=20, ignore_eos=True)] * 3, product_kw=dict(shared_prefix_min_seqs=2), **(dict(enforce_eager=True) if eager else {}))
+    assert r["decode_steps"] >= 19 and r["near_ties"] <= 2, r
 
 
 @pytest.mark.parametrize("width,heads,ff,batch", [(64, 2, 80, 1), (256, 2, 96, 16), (256, 2, 96, 17), (1024, 2, 208, 32), (64, 16, 2064, 17), (1024, 16, 2048, 32)])
