@@ -17,6 +17,7 @@
 //    itself; otherwise f32 partials go to a workspace and a second tiny kernel merges them.
 //  * all G = H/KVH query heads of a kv head are processed together so K/V are read once.
 #include <algorithm>
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <type_traits>
@@ -1236,14 +1237,24 @@ static bool prefix_in_one_launch(const AttnArgs &a) {
            (int64_t)a.nq * a.KVH <= (int64_t)share_workgroups() * (a.H / a.KVH <= 2 ? 8 : 4) &&
            (a.prefix_launches ? a.prefix_launches : attn_prefix_launches(a.nq, a.H, a.KVH, a.shared_len, a.max_ctx - a.shared_len, 0)) == 1;
 }
+// (more than 64 KiB of LDS are opted in for each instance, at runner creation: a captured decode step may be a runner's first call of one)
+int attn_prepare() {
+    static std::atomic<bool> done{false};
+    if (done.load(std::memory_order_acquire)) return 0;
+#define NVR_PREFIX_ATTR(G_, NS_)                                                                                                                                                                  \
+    {                                                                                                                                                                                             \
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_prefix_kernel<G_, NS_>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)prefix_lds<G_, NS_>());            \
+        if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "attention (shared prefix): LDS opt-in failed: %s", hipGetErrorString(e));                                                             \
+    }
+    NVR_PREFIX_ATTR(1, 1) NVR_PREFIX_ATTR(1, 2) NVR_PREFIX_ATTR(1, 4) NVR_PREFIX_ATTR(1, 8) NVR_PREFIX_ATTR(2, 1) NVR_PREFIX_ATTR(2, 2) NVR_PREFIX_ATTR(2, 4) NVR_PREFIX_ATTR(2, 8)
+    NVR_PREFIX_ATTR(4, 1) NVR_PREFIX_ATTR(4, 2) NVR_PREFIX_ATTR(4, 4)
+#undef NVR_PREFIX_ATTR
+    done.store(true, std::memory_order_release);
+    return 0;
+}
 template <int G, int NS>
 static int launch_prefix(const AttnParams &p, int nq, int shared_len, hipStream_t s) {
-    static bool done = false;                                                 // (more than 64 KiB of LDS are opted in once; a flag that several threads may set alike)
-    if (!done) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_prefix_kernel<G, NS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)prefix_lds<G, NS>());
-        if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "attention (shared prefix): LDS opt-in failed: %s", hipGetErrorString(e));
-        done = true;
-    }
+    if (int rc = attn_prepare()) return rc;                                   // (callers without a runner)
     attn_prefix_kernel<G, NS><<<dim3((unsigned)((nq + NS - 1) / NS * p.KVH)), dim3(512), prefix_lds<G, NS>(), s>>>(p, nq, shared_len);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "attention (shared prefix) launch failed: %s", hipGetErrorString(e));

@@ -169,6 +169,7 @@ bool attn_out_rides(int64_t nq, int64_t H, int64_t KVH, int64_t D, int64_t N, in
 // launches (1 or 2) of the attention behind a prefix of shared_len tokens of the whole batch: longest, mean: keys that its sequences have behind it
 int32_t attn_prefix_launches(int64_t nq, int64_t H, int64_t KVH, int64_t shared_len, int64_t longest, int64_t mean);
 int64_t attn_brief_context(int64_t nq, int64_t H, int64_t KVH);   // contexts up to it (0: none) have a decode attention of their own: worth a captured step of their own
+int attn_prepare();                                                         // LDS opt-in of the shared-prefix instances (call outside captures)
 int attention(const AttnArgs &a, bool paged, hipStream_t s);
 
 bool flash_prefill_ok(int D, int H, int KVH);

@@ -139,6 +139,7 @@ int nvr_model_runner::init() {                                       // ModelRun
     comm.force = env.tp_force_comm; comm.timeout_ms = env.p2p_timeout_ms; comm.p2p_fenced = env.p2p_fenced;
     RC(KD(linear_stream_prepare()));
     RC(KD(gemm_tiled_prepare()));
+    RC(KD(attn_prepare()));
     lazy_logits = env.lazy_logits && !f32;
     {   // arg-max partials [parts][rows]: <= LM_HEAD_MAX_PARTS x 32 rows (lm_head_kernel), or one per 128 vocabulary columns x all rows
         const size_t pe = std::max<size_t>((size_t)k::LM_HEAD_MAX_PARTS * 32, (size_t)((Vl + 127) / 128) * (size_t)max_seqs);
