@@ -47,10 +47,14 @@ struct G256Epi {
     int32_t H, KVH, D;
     int32_t kv_cache_only;             // GEPI_ROPE: k and v rows go to the caches only (the attention that follows reads them there)
     float *logits; float *pval; int32_t *pidx;   // GEPI_LMHEAD: f32 logits [T][N] (nullable), arg-max partials [tiles_x][T]
-    const half_t *qn_w, *kn_w; float qk_eps;     // GEPI_QKN: the norms' weights [D]
-    float limit, alpha; int64_t ldo;             // GEPI_CLAMP
     const int32_t *row_w; int64_t w_stride; const int32_t *rows_used;      // (rows_used, on the device: rows behind it are nobody's; null: all T) GRP (rows grouped by expert): row block rb of 256 rows multiplies the matrix W + row_w[rb] * w_stride
 };
+// What single instances need beyond it stays out of the others' arguments
+struct G256EpiNorm : G256Epi { const half_t *qn_w, *kn_w; float qk_eps; };      // GEPI_QKN: the norms' weights [D]
+struct G256EpiClamp : G256Epi { float limit, alpha; int64_t ldo; };             // GEPI_CLAMP
+template <int EPI> struct G256Args { using type = G256Epi; };
+template <> struct G256Args<GEPI_QKN> { using type = G256EpiNorm; };
+template <> struct G256Args<GEPI_CLAMP> { using type = G256EpiClamp; };
 
 constexpr int G_BK = 64, G_HT = 128, G_HALF = G_HT * G_BK * 2;          // 16 KiB per half-tile
 constexpr int G_BUF = 4 * G_HALF;                                         // A0 A1 B0 B1
@@ -75,7 +79,7 @@ __device__ __forceinline__ int g_w_uni(int hA, int i, int N) {
 // fold to shifts, and the scalar registers they needed in the K loop are what pushed that variant into SGPR -> VGPR spills
 template <int EPI, int RD = 0, bool GRP = false>
 __global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__ x, int64_t ldx, const half_t *__restrict__ W,
-                                                      int T, int K, int N, int NW, half_t *__restrict__ y, G256Epi epi,
+                                                      int T, int K, int N, int NW, half_t *__restrict__ y, typename G256Args<EPI>::type epi,
                                                       int tiles_x, int tiles_y, int CG) {
     extern __shared__ __attribute__((aligned(16))) char smem[];           // 2 x G_BUF
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -222,7 +226,8 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__
 #define G256_W(NOMORE_) if (more) { G256_R_END(4) } else { G256_R_END(NOMORE_) }
 
     constexpr int OUTC = g_glu(EPI) ? 128 : 256;                  // output columns of a tile
-    const int64_t ldy = g_rope(EPI) ? (int64_t)(epi.H + 2 * epi.KVH) * RD : EPI == GEPI_CLAMP ? epi.ldo : (int64_t)N;
+    int64_t ldy = g_rope(EPI) ? (int64_t)(epi.H + 2 * epi.KVH) * RD : (int64_t)N;
+    if constexpr (EPI == GEPI_CLAMP) ldy = epi.ldo;
     constexpr int hd2 = g_rope(EPI) ? RD / 2 : 1;
 
     int tile_no = 0;
@@ -640,7 +645,7 @@ int gemm256_gelu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_
 int gemm256_clamped_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, float limit, float alpha, half_bits *out, int64_t ldo, hipStream_t s) {
     if (!gemm256_silu_ok(T, K, I, ldx) || ldo % 8 || ldo < I) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm256_clamped_glu: T=%ld K=%ld I=%ld", (long)T, (long)K, (long)I);
     if (int rc = g256_prepare()) return rc;
-    G256Epi e{}; e.limit = limit; e.alpha = alpha; e.ldo = ldo;
+    G256EpiClamp e{}; e.limit = limit; e.alpha = alpha; e.ldo = ldo;
     const int tx = (int)(I / 128), tt = tx * (int)((T + 255) / 256);
     gemm256_kernel<GEPI_CLAMP><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
                                                                                           (int)I, (int)(2 * I), (half_t *)out, e, tx, tt / tx, g256_cg(tx, tt / tx, false));
@@ -653,7 +658,7 @@ int gemm256_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, 
     if (!gemm256_rope_ok(T, K, H, KVH, D, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm256_qkv_rope_store: T=%ld K=%ld D=%ld", (long)T, (long)K, (long)D);
     if (int rc = g256_prepare()) return rc;
     const int64_t N = (H + 2 * KVH) * D;
-    G256Epi e{};
+    G256EpiNorm e{};
     e.pos = positions; e.slots = slots; e.cos_t = cos_t; e.sin_t = sin_t; e.kc = (half_t *)k_cache; e.vc = (half_t *)v_cache;
     e.H = (int32_t)H; e.KVH = (int32_t)KVH; e.D = (int32_t)D;
     e.kv_cache_only = (kv_cache_only && slots && k_cache && v_cache) ? 1 : 0;

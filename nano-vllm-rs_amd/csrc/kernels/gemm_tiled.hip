@@ -58,11 +58,16 @@ struct TileEpi {
     // TEPI_SLAB: k-slice z owns k in [z*kslice, (z+1)*kslice) and writes its f32 partial tile to slabs[z][T][N]
     float *slabs; int64_t slab_stride; int32_t kslice;
     int32_t gelu;                          // TEPI_SILU: gelu (tanh form) instead of silu
-    const half_t *qn_w, *kn_w; float qk_eps;      // TEPI_QKN: the norms' weights
-    float limit, alpha; int64_t ldo;              // TEPI_CLAMP
     TileMap map;
     int32_t tiled;                         // W is the copy [rows/16][K/32][16][32] (retile_weight; TEPI_ROPE: its 16-row tiles are the n-tiles)
 };
+// What single instances need beyond it stays out of the others' arguments (Qwen3-0.6B in float16, us a step with / without the three numbers and two pointers in all of them: 33 sequences of 64..200
+// keys 1336 / 1320, 48 of 64..300 1475 / 1461, 64 of 300 1631 / 1615)
+struct TileEpiNorm : TileEpi { const half_t *qn_w, *kn_w; float qk_eps; };      // TEPI_QKN: the norms' weights
+struct TileEpiClamp : TileEpi { float limit, alpha; int64_t ldo; };             // TEPI_CLAMP
+template <int EPI> struct TileArgs { using type = TileEpi; };
+template <> struct TileArgs<TEPI_QKN> { using type = TileEpiNorm; };
+template <> struct TileArgs<TEPI_CLAMP> { using type = TileEpiClamp; };
 
 constexpr int BM = 128, BN = 128, BK = 64;
 constexpr int RING96 = 3;                                                 // K-tiles in the LDS ring of the 96-row kernel
@@ -113,7 +118,7 @@ __device__ __forceinline__ int tile_w_block(int bx, int t, int N) {
 template <int EPI, int NS, int MT = 4>
 __global__ __launch_bounds__(256, 2) void gemm_tiled_kernel(const half_t *__restrict__ x, int64_t ldx,
                                                          const half_t *__restrict__ W, int T, int K, int N, int NW,
-                                                         half_t *__restrict__ y, TileEpi epi) {
+                                                         half_t *__restrict__ y, typename TileArgs<EPI>::type epi) {
     // one LDS array (cdna guide §5 item 4a): [NS buffers][A 16 KiB | B 16 or 8 KiB]
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int BMt = 32 * MT;                                          // tokens per workgroup
@@ -234,12 +239,13 @@ __global__ __launch_bounds__(256, 2) void gemm_tiled_kernel(const half_t *__rest
             pre_sn[j][u] = *reinterpret_cast<const float4_t *>(epi.sin_t + at_pos);
         }
     };
-    if (QKN && rope_rot) {
-        const half_t *w = (rope_head < epi.H ? epi.qn_w : epi.kn_w) + (threadIdx.x & 7) * 8;
-        norm_w[0] = *reinterpret_cast<const half8_t *>(w); norm_w[1] = *reinterpret_cast<const half8_t *>(w + 64);
+    if constexpr (QKN)
+        if (rope_rot) {
+            const half_t *w = (rope_head < epi.H ? epi.qn_w : epi.kn_w) + (threadIdx.x & 7) * 8;
+            norm_w[0] = *reinterpret_cast<const half8_t *>(w); norm_w[1] = *reinterpret_cast<const half8_t *>(w + 64);
 #pragma unroll
-        for (int j = 0; j < PRE; ++j) request_angles(j);
-    }
+            for (int j = 0; j < PRE; ++j) request_angles(j);
+        }
     if (!QKN && rope_rot) {
         const int half_d = epi.D / 2;
 #pragma unroll
@@ -439,7 +445,9 @@ __global__ __launch_bounds__(256, 2) void gemm_tiled_kernel(const half_t *__rest
             }
             const half8_t v8 = pair8(h[0], h[1]);
             const int n = at.x * 64 + wn * 32 + col_in_pair;
-            if (m < T && n < N) *reinterpret_cast<half8_t *>(y + (int64_t)m * (EPI == TEPI_CLAMP ? epi.ldo : (int64_t)N) + n) = v8;
+            int64_t ldo = N;
+            if constexpr (EPI == TEPI_CLAMP) ldo = epi.ldo;
+            if (m < T && n < N) *reinterpret_cast<half8_t *>(y + (int64_t)m * ldo + n) = v8;
         } else {                                                          // TEPI_ROPE
             const int half_d = epi.D / 2;
             const int64_t ldy = (int64_t)heads * epi.D;
@@ -638,7 +646,7 @@ constexpr size_t kStageBytes32 = (BN + 32) * BK * 2;                     // MT =
 // K-tiles in flight: two of the 128-token tiles when two workgroups share a CU (64 KiB each), three when one is alone on it; three or (a long K loop, one workgroup per CU) four of the 64-token
 // tiles, four of the 32-token tiles.  More are slower: 512 tokens x 4096 columns 8.2 us with three, 8.3 with four, 8.7 with six (a launch's LDS takes time to be given out).
 template <int EPI>
-static void tiled_launch(int64_t nx, int64_t nz, const half_bits *x_, int64_t ldx, const half_bits *W_, const half_bits *Wt, int64_t T, int64_t K, int64_t N, int64_t NW, half_t *y, TileEpi e, hipStream_t s) {
+static void tiled_launch(int64_t nx, int64_t nz, const half_bits *x_, int64_t ldx, const half_bits *W_, const half_bits *Wt, int64_t T, int64_t K, int64_t N, int64_t NW, half_t *y, typename TileArgs<EPI>::type e, hipStream_t s) {
     const half_t *x = (const half_t *)x_, *W = (const half_t *)(Wt ? Wt : W_);
     e.tiled = Wt != nullptr;
     const int mt = tiled_mt(T, nx * nz);
@@ -730,7 +738,7 @@ int gemm_tiled_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int
 int gemm_tiled_clamped_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, float limit, float alpha, half_bits *out, int64_t ldo, hipStream_t s) {
     if (!gemm_tiled_ok(T, K, I, ldx) || I % 64 || ldo % 8 || ldo < I) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_clamped_glu: T=%ld K=%ld I=%ld", (long)T, (long)K, (long)I);
     if (int rc = gemm_tiled_prepare()) return rc;
-    TileEpi e{}; e.limit = limit; e.alpha = alpha; e.ldo = ldo;
+    TileEpiClamp e{}; e.limit = limit; e.alpha = alpha; e.ldo = ldo;
     tiled_launch<TEPI_CLAMP>(I / 64, 1, x, ldx, W, nullptr, T, K, I, 2 * I, (half_t *)out, e, s);
     return tiled_check("gemm_tiled_clamped_glu");
 }
@@ -740,7 +748,7 @@ int gemm_tiled_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *
     const int64_t N = (H + 2 * KVH) * D;
     if (norm && D != 128) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_qkv_rope_store: head norms with D=%ld", (long)D);
     if (!gemm_tiled_ok(T, K, N, ldx) || D % 16 || 128 % D) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_qkv_rope_store: T=%ld K=%ld D=%ld", (long)T, (long)K, (long)D);
-    TileEpi e{};
+    TileEpiNorm e{};
     e.pos = positions; e.slots = slots; e.cos_t = cos_t; e.sin_t = sin_t; e.kc = (half_t *)k_cache; e.vc = (half_t *)v_cache;
     e.H = (int32_t)H; e.KVH = (int32_t)KVH; e.D = (int32_t)D;
     e.kv_cache_only = kv_cache_only && slots && k_cache && v_cache;
