@@ -837,26 +837,28 @@ int linear_qkv_norm_rope_store(const half_bits *x, int64_t ldx, const half_bits 
 
 // ---- products of a decode step of few rows whose workgroups form RMSNorm(h + slabs) themselves (linear_skinny_kernel, NORM)
 // (three and four rows: from the width on at which the products behind a launch of its own split k over the same eight waves, so that the step's bits are theirs)
-bool norm_linear_ok(int64_t T, int64_t K, int64_t S) { return T >= 1 && T <= NORM_ROWS && (T <= 2 || waves_for(K) == 8) && K % 256 == 0 && T * K <= NORM_ELEMS && (S == 2 || S == 4 || S == 8); }
+// (slabs: 2 or 4 of a split product; in front of the gate and up product also 8, one per kv head, of an attention with the output product in it)
+static bool norm_linear_ok(int64_t T, int64_t K, int64_t S, int64_t most) {
+    return T >= 1 && T <= NORM_ROWS && (T <= 2 || waves_for(K) == 8) && K % 256 == 0 && T * K <= NORM_ELEMS && (S == 2 || S == 4 || S == 8) && S <= most;
+}
 template <int NT, int EPI>
 static int norm_launch(const NormIn &nm, const half_bits *W, int64_t T, int64_t K, int64_t N, void *y, const LinEpi &le, int64_t gx, bool tiled, hipStream_t s, const char *what) {
-    if (!norm_linear_ok(T, K, nm.S)) return nvr::fail(NVR_ERR_UNSUPPORTED, "%s: T=%ld K=%ld, %d slabs", what, (long)T, (long)K, nm.S);
+    if (!norm_linear_ok(T, K, nm.S, EPI == EPI_SILU ? 8 : 4)) return nvr::fail(NVR_ERR_UNSUPPORTED, "%s: T=%ld K=%ld, %d slabs", what, (long)T, (long)K, nm.S);
     LinEpiNorm e{};
     static_cast<LinEpi &>(e) = le;
     e.norm = nm; e.tiled = tiled;
     if constexpr (EPI == EPI_SILU)
-        if (nm.S > 4) {                                                   // (the slabs that an attention with the output product in it leaves, one per kv head)
+        if (nm.S > 4) {
             linear_skinny_kernel<NT, 1, 8, EPI, 8><<<dim3((unsigned)gx), dim3(512), (size_t)(T * (K + 8) * 2), s>>>(nullptr, 0, (const half_t *)W, (int)T, (int)K, (int)N, y, e);
             return launch_check(what);
         }
-    if (nm.S > 4) return nvr::fail(NVR_ERR_UNSUPPORTED, "%s: %d slabs", what, nm.S);
     linear_skinny_kernel<NT, 1, 8, EPI, 4><<<dim3((unsigned)gx), dim3(512), (size_t)(T * (K + 8) * 2), s>>>(nullptr, 0, (const half_t *)W, (int)T, (int)K, (int)N, y, e);
     return launch_check(what);
 }
 // which products of these shapes take the weight-streaming kernel above at so few rows (large weights have a kernel of their own)
-bool norm_linear_plain_ok(int64_t T, int64_t K, int64_t N, int64_t S) { return norm_linear_ok(T, K, S) && N % 16 == 0 && !linear_stream_ok(T, K, N, K); }
-bool norm_linear_silu_ok(int64_t T, int64_t K, int64_t I, int64_t S) { return norm_linear_ok(T, K, S) && I % 16 == 0 && !linear_stream_silu_ok(T, K, I, K); }
-bool norm_linear_rope_ok(int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D, int64_t S) { return norm_linear_ok(T, K, S) && D % 16 == 0 && !linear_stream_rope_ok(T, K, H, KVH, D, K); }
+bool norm_linear_plain_ok(int64_t T, int64_t K, int64_t N, int64_t S) { return norm_linear_ok(T, K, S, 4) && N % 16 == 0 && !linear_stream_ok(T, K, N, K); }
+bool norm_linear_silu_ok(int64_t T, int64_t K, int64_t I, int64_t S) { return norm_linear_ok(T, K, S, 8) && I % 16 == 0 && !linear_stream_silu_ok(T, K, I, K); }
+bool norm_linear_rope_ok(int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D, int64_t S) { return norm_linear_ok(T, K, S, 4) && D % 16 == 0 && !linear_stream_rope_ok(T, K, H, KVH, D, K); }
 int norm_linear(const NormIn &nm, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *y, hipStream_t s, const half_bits *Wt) {
     return norm_launch<1, EPI_F16>(nm, Wt ? Wt : W, T, K, N, y, LinEpi{}, N / 16, Wt != nullptr, s, "norm + linear");
 }
