@@ -81,12 +81,12 @@ int linear_gelu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, 
 // gate / up products with gelu (tanh form) in silu's place
 int linear_gelu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s);
 // gate_up with the clamped gated unit of a layer list in the epilogue, rows of out ldo apart (up to 32 rows, and the shapes that linear() multiplies on LDS tiles)
-// ... beside a plain product y = x . W^T of N columns and the same K, in one launch (the bits of the two)
-bool linear_beside_clamped_glu_ok(const half_bits *x2, int64_t ldx, int64_t T, int64_t K, int64_t N, int64_t I, const half_bits *out, int64_t ldo);
-int linear_beside_clamped_glu(const half_bits *x, const half_bits *x2, int64_t ldx, const half_bits *W, const half_bits *W2, int64_t T, int64_t K, int64_t N, int64_t I, float limit, float alpha, half_bits *y,
-                              half_bits *out, int64_t ldo, hipStream_t s);
 bool linear_clamped_glu_ok(const half_bits *x, int64_t ldx, int64_t T, int64_t K, int64_t I, const half_bits *out, int64_t ldo);
 int linear_clamped_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, float limit, float alpha, half_bits *out, int64_t ldo, hipStream_t s);
+// ... beside a plain product y = x . W^T of N columns and the same K, in one launch (the bits of the two)
+bool linear_beside_clamped_glu_ok(const half_bits *x, const half_bits *x2, int64_t ldx, int64_t T, int64_t K, int64_t N, int64_t I, const half_bits *y, const half_bits *out, int64_t ldo);
+int linear_beside_clamped_glu(const half_bits *x, const half_bits *x2, int64_t ldx, const half_bits *W, const half_bits *W2, int64_t T, int64_t K, int64_t N, int64_t I, float limit, float alpha, half_bits *y,
+                              half_bits *out, int64_t ldo, hipStream_t s);
 int linear_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H,
                           int64_t KVH, int64_t D, const int64_t *positions, const int32_t *slots, const float *cos_t,
                           const float *sin_t, half_bits *qkv, half_bits *k_cache, half_bits *v_cache, hipStream_t s,

@@ -765,14 +765,14 @@ int linear_clamped_glu(const half_bits *x, int64_t ldx, const half_bits *W, int6
 // linear_clamped_glu().  A launch of 5-7 us a layer is
 // saved: us a request batch of a 4-layer list (width 1024, I = 3072), two launches / one: 1 request of 64 + 32 tokens 5009 / 4598, 8 of 100 + 32 5774 / 5380, 16 of 1024 + 32 10334 / 9920, 24 of 100 + 32
 // 7405 / 7025.
-bool linear_beside_clamped_glu_ok(const half_bits *x2, int64_t ldx, int64_t T, int64_t K, int64_t N, int64_t I, const half_bits *out, int64_t ldo) {
-    if (T < 1 || T > 32 || K % 32 || N % 16 || ldx % 8 || waves_for(K) == 16 || !linear_clamped_glu_ok(x2, ldx, T, K, I, out, ldo)) return false;
+bool linear_beside_clamped_glu_ok(const half_bits *x, const half_bits *x2, int64_t ldx, int64_t T, int64_t K, int64_t N, int64_t I, const half_bits *y, const half_bits *out, int64_t ldo) {
+    if (((uintptr_t)x & 15) || ((uintptr_t)y & 7) || T < 1 || T > 32 || K % 32 || N % 16 || ldx % 8 || waves_for(K) == 16 || !linear_clamped_glu_ok(x2, ldx, T, K, I, out, ldo)) return false;
     if ((N / 64) * (T <= 16 ? 1 : (T + 31) / 32) >= 1024 || linear_stream_ok(T, K, N, ldx) || gemm256_ok(T, K, N, ldx)) return false;
     return (T <= 16 || N / 16 < 128) == (T <= 16 || I / 16 < 128);
 }
 int linear_beside_clamped_glu(const half_bits *x, const half_bits *x2, int64_t ldx, const half_bits *W, const half_bits *W2, int64_t T, int64_t K, int64_t N, int64_t I, float limit, float alpha, half_bits *y,
                               half_bits *out, int64_t ldo, hipStream_t s) {
-    if (!linear_beside_clamped_glu_ok(x2, ldx, T, K, N, I, out, ldo) || ((uintptr_t)x & 15) || ((uintptr_t)y & 7))
+    if (!linear_beside_clamped_glu_ok(x, x2, ldx, T, K, N, I, y, out, ldo))
         return nvr::fail(NVR_ERR_UNSUPPORTED, "linear beside linear_clamped_glu: T=%ld K=%ld N=%ld I=%ld", (long)T, (long)K, (long)N, (long)I);
     const bool mt1 = T <= 16 || I / 16 < 128;
     const dim3 grid((unsigned)(I / 16 + N / 16), (unsigned)((T + (mt1 ? 15 : 31)) / (mt1 ? 16 : 32)));

@@ -484,7 +484,7 @@ int LayeredModel::forward(nvr_model_runner &r, const StepPlan &p) {
         owed = 0;
         // mixer and feed-forward read the stream of the layer in front: in steps of few rows their first products share a launch
         uint16_t *const glu = (uint16_t *)((char *)cat + (size_t)(w.mixcols * esz));
-        const bool paired = bf16 && L.has_mlp && nvr::kb::linear_beside_clamped_glu_ok((const uint16_t *)a2, W, T, W, w.nmix, L.ff, glu, w.kcat);
+        const bool paired = bf16 && L.has_mlp && nvr::kb::linear_beside_clamped_glu_ok((const uint16_t *)a1, (const uint16_t *)a2, W, T, W, w.nmix, L.ff, (const uint16_t *)proj, glu, w.kcat);
         if (paired) RC(nvr::kb::linear_beside_clamped_glu((const uint16_t *)a1, (const uint16_t *)a2, W, (const uint16_t *)w.mix, (const uint16_t *)w.gu, T, W, w.nmix, L.ff, (float)L.limit, 1.702f,
                                                           (uint16_t *)proj, glu, w.kcat, s));
         else RC(gemm(r, a1, W, w.mix, T, W, w.nmix, proj));
