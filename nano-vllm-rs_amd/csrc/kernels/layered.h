@@ -130,10 +130,10 @@ int join_norm_canon(float *x, const float *parts, int nparts, float mult, const 
                     void *out2, bool bf16, float *hist, int64_t slots, hipStream_t s);
 
 // out[r] = x[rows[r]] / sqrt(mean^2 + eps) * g, in the operand type
+int norm_rows(const float *x, const int32_t *rows, int64_t R, int64_t W, float eps, float g, void *out, bool bf16, hipStream_t s);
 // norm_rows of x + mult * (the sum of nparts partial products [T][W], rounded to the model's type): axpy_parts and norm_rows, the stream left as it was
 bool join_norm_rows_ok(const float *x, const float *parts, int nparts, int64_t W, const void *out);
 int join_norm_rows(const float *x, const float *parts, int nparts, float mult, const int32_t *rows, int64_t R, int64_t T, int64_t W, float eps, float g, void *out, bool bf16, hipStream_t s);
-int norm_rows(const float *x, const int32_t *rows, int64_t R, int64_t W, float eps, float g, void *out, bool bf16, hipStream_t s);
 
 // y[T][N] (f32, or the operand type) = a[T][K] . w[N][K]^T for shapes the tiled GEMMs do not take (any T, K, N)
 int gemm_any(const void *a, int64_t lda, const void *w, int64_t T, int64_t K, int64_t N, void *y, bool y_f32, bool bf16, hipStream_t s);

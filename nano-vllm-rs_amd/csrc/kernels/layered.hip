@@ -1707,7 +1707,8 @@ int retention(const RetentionArgs &a, const Batch &b, bool bf16, hipStream_t s) 
 }
 
 bool retention_step_ok(const RetentionArgs &a, const Batch &b, const void *gate, int64_t ldg, int64_t gcol, const void *out, int64_t ldo, bool bf16) {
-    return bf16 && b.max_rows == 1 && b.T == b.B && a.az == nullptr && a.tok_gate == nullptr && a.decay != nullptr && a.v_ones == 0 && a.qk_share <= 1 && (a.D == 64 || a.D == 128) && a.rot_dims == a.D &&
+    // (the plain decaying form: abias, inv_tau, qscale and decay_exp belong to the gated ones, as in retention(), which refuses a bonus here)
+    return bf16 && b.max_rows == 1 && b.T == b.B && a.az == nullptr && a.tok_gate == nullptr && a.bonus == nullptr && a.decay != nullptr && a.v_ones == 0 && a.qk_share <= 1 && (a.D == 64 || a.D == 128) && a.rot_dims == a.D &&
            (a.Dv == 64 || a.Dv == 128) && ((a.ld | a.vcol | ldg | gcol | ldo) & 3) == 0 && (((uintptr_t)a.proj | (uintptr_t)gate | (uintptr_t)out) & 7) == 0 && ((uintptr_t)a.state & 15) == 0;
 }
 int retention_step(const RetentionArgs &a, const Batch &b, const void *gate, int64_t ldg, int64_t gcol, float eps, void *out, int64_t ldo, hipStream_t s) {
