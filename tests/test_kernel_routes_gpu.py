@@ -702,6 +702,22 @@ def test_split_products_of_large_weights(T, K, N, S):
     assert np.all(np.abs(s.astype(np.float64).sum(0) - ref) <= bound)
 
 
+@pytest.mark.parametrize("T,kslice,N,S", [(3, 1024, 12288, 1), (20, 1536, 4096, 2), (32, 3072, 4096, 1), (16, 2048, 8192, 1)])
+def test_split_products_have_one_order_of_sums(T, kslice, N, S):
+    """Slices that linear_slab_kernel takes, and the same with 32 columns of zeros in x behind each, which it leaves to linear_skinny_kernel: bit for bit (the first wave adds zeros to its sums)."""
+    rng, l = np.random.default_rng(T + kslice), nvr.lib()
+    out = []
+    x, W = _bits(rng, (T, S, kslice), 0.5), _bits(rng, (N, S, kslice), 0.1)
+    for pad in (0, 32):
+        K = S * (kslice + pad)
+        xp = np.concatenate([x, np.zeros((T, S, pad), F16)], 2).reshape(T, K)
+        Wp = np.concatenate([W, np.ones((N, S, pad), F16)], 2).reshape(N, K)
+        d_x, d_W, d_s = dev(xp), dev(Wp), nvr.DeviceBuffer(S * T * N * 4)
+        nvr.check(l.nvr_linear_splitk(d_x.ptr, K, d_W.ptr, T, K, N, S, d_s.ptr, None))
+        out.append(d_s.to_numpy((S, T, N), np.float32))
+    assert np.array_equal(out[0], out[1])
+
+
 @pytest.mark.parametrize("T,K,N", [(33, 1536, 768), (48, 2048, 1040), (64, 512, 784), (64, 3072, 2048)])
 def test_products_of_33_to_64_rows_in_eight_slices(T, K, N):
     """The o / down products of such steps on the tiles, eight slices of one to six K-tiles: the slabs' sum against 64 bits, the tiled copy's bits, and the residual add + norm over eight slabs."""
@@ -1121,6 +1137,24 @@ def test_layer_list_decode_steps_of_two_products_in_one_launch(width, heads, ff,
     d.step([(n, base[i % 3][:-3]) for i, n in enumerate(names)])
     steps = [d.step([(n, base[i % 3][len(base[i % 3]) - 3 + k:][:1]) for i, n in enumerate(names)]) for k in range(3)]
     _compare_layer_rows(cfg, w, "bfloat16", base, [np.concatenate([s[n] for s in steps]) for n in names])
+
+
+@pytest.mark.parametrize("width,ff", [(256, 208), (1024, 1024)])
+def test_layer_list_two_products_in_one_launch_have_the_bits_of_two(width, ff):
+    """Decode steps of 16 sequences, whose two first products share a launch, and of 32 (a wide mixer beside a narrow feed-forward: two launches, of two and one row tiles to a workgroup): the 16
+    sequences that both hold come out bit for bit."""
+    import rugudra_util as u
+    cfg = u.make_config([u.retention_layer(16, 32, 32, ff=ff), u.retention_layer(16, 32, 32, ff=ff)], width=width, taps=2)
+    w = u.make_weights(cfg, seed=ff + width)
+    toks = np.random.default_rng(width).integers(0, 97, (32, 6))
+    got = []
+    for batch in (16, 32):
+        d = u.Driver(cfg, w, dtype="bfloat16", slots=batch, pages=2 * batch, max_tokens=4 * batch, max_len=64)
+        for first in range(0, batch, 16):                                  # (the prompts in steps of the same size)
+            d.step([("s%d" % i, toks[i][:3]) for i in range(first, first + 16)])
+        steps = [d.step([("s%d" % i, toks[i][k:k + 1]) for i in range(batch)]) for k in range(3, 6)]
+        got.append(np.concatenate([s["s%d" % i] for s in steps for i in range(16)]).view(np.uint32))
+    assert np.array_equal(got[0], got[1]), (got[0] != got[1]).mean()
 
 
 @pytest.mark.parametrize("dim,vdim", [(64, 64), (64, 128), (128, 64), (128, 128)])
