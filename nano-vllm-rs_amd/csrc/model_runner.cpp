@@ -1493,8 +1493,8 @@ int nvr_model_runner::ensure_logits() {
 }
 
 // Tokens that the last kernel of a step writes to the pinned buffer: marked as missing in front of its launch, then watched.  Everything in front of that kernel has ended when they appear, and the host
-// goes on as soon as they do; a stream that is waited for wakes it later.  us, waited for / watched: one sequence of 128
-// keys 640 / 630 a step, 16 requests of 1024 + 32 tokens of a layer list 9729 / 9541, one of 64 + 32 4315 / 4050, a float32 request of 128 + 48 43670 / 43140.  What takes longer than the watch, or never comes, is the stream's to report.
+// goes on as soon as they do; a stream that is waited for wakes it later.  us, waited for / watched: one sequence of 128 keys 678 / 672 a step (640 / 630 stepped again and again), 16 requests of 1024 + 32
+// tokens of a layer list 9717 / 9574, one of 64 + 32 4315 / 4050, a float32 request of 128 + 48 44260 / 43670.  What takes longer than the watch, or never comes, is the stream's to report.
 void nvr_model_runner::await_tokens(int64_t B) {
     for (int64_t i = 0; i < B; ++i) h_tok[i] = INT64_MIN;
 }
