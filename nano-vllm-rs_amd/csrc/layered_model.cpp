@@ -405,7 +405,7 @@ int LayeredModel::execute(nvr_model_runner &r, nvr_seq *const *seqs, size_t nseq
     }
     cu[nseq] = (int32_t)t;
     if (want) for (size_t i = 0; i < R; ++i) { if (want[i] < 0 || want[i] >= T) return fail(NVR_ERR_INVALID_ARG, "execute_model: logits row %d of a step of %ld rows", want[i], (long)T); wnt[i] = want[i]; }
-    r.inputs_read = false;
+    r.inputs_read = r.step_replayed = false;
     NVR_HIP_CHECK(hipMemcpyAsync(in_dev, in_host, off, hipMemcpyHostToDevice, r.stream));
     kl::Batch b{};
     b.ids = (const int64_t *)(in_dev + o_ids); b.row_seq = (const int32_t *)(in_dev + o_rs); b.cu = (const int32_t *)(in_dev + o_cu);
@@ -446,6 +446,7 @@ int LayeredModel::execute(nvr_model_runner &r, nvr_seq *const *seqs, size_t nseq
                 it->second = ge;
             }
             NVR_HIP_CHECK(hipGraphLaunch(it->second, r.stream));
+            r.step_replayed = true;
             ++graph_replays;
         }
     } else

@@ -151,6 +151,7 @@ private:
     float *f32_gather = nullptr; int64_t f32_gather_rows = 0;   // float32 tensor-parallel ranks: every rank's partial sums [tp][f32_gather_rows][hidden], a piece of the step's rows at a time
     int row_parallel_norm(const uint16_t *x, int64_t K, const uint16_t *W, const uint16_t *Wt, int64_t T, const uint16_t *wn, const uint16_t *bias = nullptr);
     bool inputs_read = false;                            // the last step's tokens have been seen: the upload of its inputs is behind it
+    bool step_replayed = false;                          // the last step was one graph launch (take_tokens)
     void await_tokens(int64_t B);
     int take_tokens(int64_t B, int64_t *out);
     int64_t *h_tok_dev = nullptr;                        // device-visible address of the pinned token buffer h_tok
