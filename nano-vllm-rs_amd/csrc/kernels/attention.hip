@@ -1262,12 +1262,13 @@ static int launch_prefix(const AttnParams &p, int nq, int shared_len, hipStream_
 }
 
 // Whether a decode step's attention takes the output product along (OUTP): no more workgroups than CUs (two on a CU wait for each other's registers: 4 sequences of 128 keys 767 / 835 us a step), which 128 rows a workgroup
-// allow twice as many sequences as 64, and
-// contexts of up to two rounds of keys, since every workgroup of a pair walks all of them.  Qwen3-0.6B, us a step, two launches / one: 1 sequence of 128 keys that is new to the caches 699 / 672; the same
-// sequences stepped again and again, whose keys and weights the last-level cache holds in part: 1 of 40 keys 660 / 627, 128 694 / 645, 200 707 / 673,
-// 255 700 / 656, 400 710 / 711; 2 sequences of 40 694 / 656, 128 716 / 674, 255 741 / 693, 400 757 / 751; 3 of 128 727 / 696, 4 762 / 734; with q / k norms 1 of 128 674 / 637, 300 701 / 701, 2 of 128 729 / 692, 300 762 / 765, 4 of 255 797 / 761.
+// allow twice as many sequences as 64, and contexts of up to two rounds of keys, since every workgroup of a pair walks all of them; four sequences, which each have 128 rows' workgroups, of one round only.
+// Qwen3-0.6B, us a step whose keys are new to the caches, two launches / one, float16: 1 sequence of 40 keys 667 / 630, 128 699 / 672, 200 708 / 699, 254 743 / 731; 2 of 40 701 / 662, 128 723 / 706,
+// 254 771 / 770; 3 of 128 746 / 730, 254 796 / 796; 4 of 40 743 / 729, 128 772 / 766, 254 822 / 834; with q / k norms (bfloat16) 1 of 40 677 / 643, 200 711 / 693, 254 733 / 724; 2 of 40 723 / 693, 128
+// 736 / 716, 254 781 / 787; 3 of 128 749 / 736, 254 794 / 794; 4 of 40 771 / 754, 128 783 / 779, 254 832 / 839.  (The same step again and again, whose keys the last-level cache holds, gains more:
+// 1 of 128 694 / 645, 4 of 255 with norms 797 / 761.)
 bool attn_out_rides(int64_t nq, int64_t H, int64_t KVH, int64_t D, int64_t N, int64_t max_ctx) {
-    if (KVH <= 0 || H % KVH || max_ctx > 256 || nq > 4 || nq * KVH * (N / (N % 128 ? 64 : 128)) > share_workgroups()) return false;
+    if (KVH <= 0 || H % KVH || nq > 4 || max_ctx > (nq < 4 ? 256 : attn_brief_context(nq, H, KVH)) || nq * KVH * (N / (N % 128 ? 64 : 128)) > share_workgroups()) return false;
     const int64_t G = H / KVH;
     return (D == 64 || D == 128) && (G == 1 || G == 2 || G == 4) && (KVH == 2 || KVH == 4 || KVH == 8) && N % OUT_ROWS == 0;
 }

@@ -1110,6 +1110,19 @@ def test_decode_attention_takes_the_output_product_along(hidden, heads, kv, dim,
 
 
 @pytest.mark.parametrize("eager", [False, True])
+def test_decode_of_four_sequences_whose_output_product_leaves_the_attention(eager):
+    """Four sequences whose longest context passes the 136 keys up to which their attention multiplies its heads with the output product's columns, replayed steps and eager ones — logits against the
+    oracle, step by step."""
+    from oracle import model_oracle as mo
+    from test_engine_gpu import _run_pair
+    mcfg = mo.small(hidden_size=1024, num_hidden_layers=2, intermediate_size=512, head_dim=128, num_attention_heads=16, num_key_value_heads=8, seed=4, init_std=0.02)
+    ecfg = dict(max_num_seqs=4, max_num_batched_tokens=512, max_model_len=300, kvcache_block_size=64, num_kvcache_blocks=32)
+    prompts = [oracle.fill_tokens(n, 3, i, mcfg.vocab_size).tolist() for i, n in enumerate((130, 5, 60, 1))]
+    r = _run_pair(mcfg, ecfg, prompts, [dict(temperature=0.0, max_tokens=12, ignore_eos=True)] * 4, **(dict(enforce_eager=True) if eager else {}))
+    assert r["decode_steps"] >= 11
+
+
+@pytest.mark.parametrize("eager", [False, True])
 def test_decode_behind_a_shared_prefix_while_own_contexts_grow(eager):
     """Three requests behind 512 tokens whose longest passes 128 tokens of its own on the way: one launch before, two behind it, each form a captured step of its own — logits against the oracle, step
     by step."""
