@@ -1237,21 +1237,6 @@ static bool prefix_in_one_launch(const AttnArgs &a) {
            (int64_t)a.nq * a.KVH <= (int64_t)share_workgroups() * (a.H / a.KVH <= 2 ? 8 : 4) &&
            (a.prefix_launches ? a.prefix_launches : attn_prefix_launches(a.nq, a.H, a.KVH, a.shared_len, a.max_ctx - a.shared_len, 0)) == 1;
 }
-// (more than 64 KiB of LDS are opted in for each instance, at runner creation: a captured decode step may be a runner's first call of one)
-int attn_prepare() {
-    static std::atomic<bool> done{false};
-    if (done.load(std::memory_order_acquire)) return 0;
-#define NVR_PREFIX_ATTR(G_, NS_)                                                                                                                                                                  \
-    {                                                                                                                                                                                             \
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_prefix_kernel<G_, NS_>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)prefix_lds<G_, NS_>());            \
-        if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "attention (shared prefix): LDS opt-in failed: %s", hipGetErrorString(e));                                                             \
-    }
-    NVR_PREFIX_ATTR(1, 1) NVR_PREFIX_ATTR(1, 2) NVR_PREFIX_ATTR(1, 4) NVR_PREFIX_ATTR(1, 8) NVR_PREFIX_ATTR(2, 1) NVR_PREFIX_ATTR(2, 2) NVR_PREFIX_ATTR(2, 4) NVR_PREFIX_ATTR(2, 8)
-    NVR_PREFIX_ATTR(4, 1) NVR_PREFIX_ATTR(4, 2) NVR_PREFIX_ATTR(4, 4)
-#undef NVR_PREFIX_ATTR
-    done.store(true, std::memory_order_release);
-    return 0;
-}
 template <int G, int NS>
 static int launch_prefix(const AttnParams &p, int nq, int shared_len, hipStream_t s) {
     if (int rc = attn_prepare()) return rc;                                   // (callers without a runner)
@@ -1490,6 +1475,23 @@ int attention(const AttnArgs &a, bool paged, hipStream_t s) {
 #undef NVR_ATTN_CASE
     return nvr::fail(NVR_ERR_UNSUPPORTED, "attention: unsupported head_dim=%d / group=%d (D in {64,128}, G in {1,2,4,8})",
                      a.D, G);
+}
+
+// (more than 64 KiB of LDS are opted in for each instance, in front of a runner's first step of this form: the step may be captured.  Not at the runner's creation: with the opt-in there a step of one
+// sequence of 128 keys, which has none of these kernels, took 672 us instead of 661)
+int attn_prepare() {
+    static std::atomic<bool> done{false};
+    if (done.load(std::memory_order_acquire)) return 0;
+#define NVR_PREFIX_ATTR(G_, NS_)                                                                                                                                                                  \
+    {                                                                                                                                                                                             \
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_prefix_kernel<G_, NS_>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)prefix_lds<G_, NS_>());            \
+        if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "attention (shared prefix): LDS opt-in failed: %s", hipGetErrorString(e));                                                             \
+    }
+    NVR_PREFIX_ATTR(1, 1) NVR_PREFIX_ATTR(1, 2) NVR_PREFIX_ATTR(1, 4) NVR_PREFIX_ATTR(1, 8) NVR_PREFIX_ATTR(2, 1) NVR_PREFIX_ATTR(2, 2) NVR_PREFIX_ATTR(2, 4) NVR_PREFIX_ATTR(2, 8)
+    NVR_PREFIX_ATTR(4, 1) NVR_PREFIX_ATTR(4, 2) NVR_PREFIX_ATTR(4, 4)
+#undef NVR_PREFIX_ATTR
+    done.store(true, std::memory_order_release);
+    return 0;
 }
 
 }}  // namespace nvr::k / nvr::kb (NVR_DT_NS)

@@ -139,7 +139,6 @@ int nvr_model_runner::init() {                                       // ModelRun
     comm.force = env.tp_force_comm; comm.timeout_ms = env.p2p_timeout_ms; comm.p2p_fenced = env.p2p_fenced;
     RC(KD(linear_stream_prepare()));
     RC(KD(gemm_tiled_prepare()));
-    RC(KD(attn_prepare()));
     lazy_logits = env.lazy_logits && !f32;
     {   // arg-max partials [parts][rows]: <= LM_HEAD_MAX_PARTS x 32 rows (lm_head_kernel), or one per 128 vocabulary columns x all rows
         const size_t pe = std::max<size_t>((size_t)k::LM_HEAD_MAX_PARTS * 32, (size_t)((Vl + 127) / 128) * (size_t)max_seqs);
@@ -1170,6 +1169,7 @@ int nvr_model_runner::execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill
                                                &decode_shared_rows);
         decode_ragged = ragged_batch(nseq, sum_ctx, (cfg.enforce_eager || graphs_disabled) ? max_ctx : (max_ctx + 255) / 256 * 256);
         decode_prefix_launches = prefix_launches(nseq, sum_ctx, max_ctx);
+        if (decode_prefix_launches == 1) RC(KD(attn_prepare()));      // (in front of a capture)
     }
     // one H2D per array actually used this step (K19)
     auto up = [&](size_t off, size_t bytes) { return hipMemcpyAsync(in_dev + off, in_host + off, bytes, hipMemcpyHostToDevice, stream); };
@@ -1268,6 +1268,7 @@ int nvr_model_runner::execute_decode_ahead(nvr_seq *const *seqs, size_t nseq, in
                                            &decode_shared_rows);
     decode_ragged = ragged_batch(nseq, sum_ctx, (cfg.enforce_eager || graphs_disabled) ? max_ctx : (max_ctx + 255) / 256 * 256);
     decode_prefix_launches = prefix_launches(nseq, sum_ctx, max_ctx);
+    if (decode_prefix_launches == 1) RC(KD(attn_prepare()));
     NVR_HIP_CHECK(hipMemcpyAsync(in_dev + off_dec + dof_pos, hd + dof_pos, dof_bt + nseq * max_blocks_per_seq * 4 - dof_pos, hipMemcpyHostToDevice, stream));
     last_rows = nseq; last_prefill = false; last_tokens = (int64_t)nseq;
     lm_parts = KD(lm_head_parts((int64_t)nseq, Hd, Vl, Hd));
