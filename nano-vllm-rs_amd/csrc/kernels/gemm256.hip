@@ -3,28 +3,23 @@
 // reference call sites as in linear.hip (linear.rs:354-356,228-239,437-439; activation.rs:46-63;
 // rotary_embedding.rs:23-48; attention.rs:150-174).  Bound: MFMA (880.8 MFLOP per prefill token).
 //
-// Structure (after cdna_hip_programming.md "The 256² 8-phase template"; the half-tile / phase assignment is this file's):
-//   * workgroup = 8 waves (2 along n x 4 along m) = 256 W rows (A operand) x 256 tokens (B operand), BK = 64.
+// Structure:
+//   * workgroup = 4 waves (2 along n x 2 along m), one per SIMD with all of its 512 registers, = 256 W rows (A operand) x 256 tokens (B operand), BK = 64.
 //     Each operand tile is two HALF-TILES of 128 rows (16 KiB: [row][8 chunks of 16 B], chunk' = chunk ^ (row & 7),
 //     conflict-free for the 4 x 16 lane groups of ds_read_b128).  LDS = 2 K-tile buffers x {A0, A1, B0, B1} = 128 KiB.
-//   * a wave owns 64 rows of EACH A half and 32 rows of EACH B half, so its 128 x 64 output splits into four
-//     quadrants (A half, B half) of 16 MFMAs (v_mfma_f32_16x16x32_f16, 4 n-tiles x 2 m-tiles x 2 k-steps) — one
-//     quadrant per PHASE, and each phase needs only the half-tiles named below.
-//   * a K-tile is four phases; every phase = R { ds_read the fragments it is missing; global_load_lds ONE half-tile of the NEXT
-//     K-tile (2 x 16 B per thread) into the other buffer; s_waitcnt vmcnt(4); s_barrier } + M { 16 MFMAs; s_barrier }, the two wave
-//     groups one barrier interval apart (reads and LDS-DMA issue of one overlap MFMAs of the other; r03: the requests moved from
-//     M to R, where the wave only waits for the other group's MFMAs: -2..3 % per K-tile):
-//         phase 0: quadrant (A0,B0)  reads A0 (8 fragments) + B0 (4)   stages A0'
-//         phase 1: quadrant (A0,B1)  reads B1 (4)                      stages B0'
-//         phase 2: quadrant (A1,B1)  reads A1 (8)                      stages B1'
-//         phase 3: quadrant (A1,B0)  reads B0 again (4)                stages A1'
-//     vmcnt(4) leaves the two youngest half-tiles in flight; every half-tile has two phases to land before the
-//     barrier in front of its first reader (RAW: own loads counted, then the barrier), and it is written into the
-//     buffer whose last reader finished a whole K-tile earlier (WAR).  The loads never drain to 0 in the loop.
-//   * row maps put epilogue partners in ONE lane: SiLU — A0 = gate rows, A1 = up rows of the same 128 columns; RoPE —
-//     A0 = first halves, A1 = second halves of the same heads.
-//   * epilogue: results are staged in LDS (the operand buffers are dead) per 128-token half and written as 16-byte
-//     pieces of contiguous rows.
+//   * a wave owns 64 rows of EACH half, so its 128 x 128 output (256 accumulation registers) splits into four quadrants (A half, B half) of 32 MFMAs
+//     (v_mfma_f32_16x16x32_f16, 4 n-tiles x 4 m-tiles x 2 k-steps): one quadrant per PHASE.  A fragment read from LDS feeds eight products (eight waves of 128 x 64: 5.3, with 1.5 times the LDS reads).
+//   * fragments of all four half-tiles fit in registers (128), so a phase brings in the half-tile that the NEXT one (A0: the one after) adds, and requests (LDS-DMA, 4 x 16 B per thread) a half-tile of
+//     the K-tile after next into a slot whose last reader is a barrier back:
+//         phase 0: quadrant (A0,B0)  reads B1        requests A0''        phase 2: quadrant (A1,B1)  reads A0'       requests B1''
+//         phase 1: quadrant (A0,B1)  reads A1        requests B0''        phase 3: quadrant (A1,B0)  reads B0'       requests A1''
+//     ending with s_waitcnt vmcnt(20) (the five youngest half-tiles stay in flight: a request has five phases of 512 clocks to land) and ONE barrier.
+//   * results leave straight from the accumulators as 16-byte pieces: the W rows of a half-tile are laid into LDS in the order that gives a lane eight neighbouring columns, and epilogue partners are
+//     in ONE lane (SiLU: A0 = gate rows, A1 = up rows of the same 128 columns; RoPE: A0 = first halves, A1 = second halves of the same heads).  No barrier, and the next tile's requests are under way.
+// What bounds it: power.  With operands of zeros a K-tile takes 1.05 us at 2.4 GHz however many CUs run (2520 clocks: 128 products of 17 and the ~120 other instructions of a wave, which nothing overlaps), with
+// random ones 1.07 us on 32 CUs and 1.45 on 256: the clock falls to what the part's power allows.  us, eight waves of 128 x 64 with 8 barriers a K-tile and results through LDS / so: 4096 x 12288 x 4096
+// (T K N) 294 / 281, 32768 x 3072 x 1024 + residual 183 / 162, 32768 x 2048 x 1024 113 / 101, 32768 x 1024 x 4096 231 / 221, gate and up of 3072 columns 362 / 347, of 12288 at 3062 x 4096 478 / 451,
+// qkv with RoPE and store 270 / 250, with head norms 299 / 280.  (One barrier a K-tile with all requests behind it: the same rate alone, but 15 % less where the operands come from memory.)
 #include <cstdlib>
 #include "kernels.h"
 #include "device_utils.h"
@@ -58,471 +53,406 @@ template <> struct G256Args<GEPI_CLAMP> { using type = G256EpiClamp; };
 
 constexpr int G_BK = 64, G_HT = 128, G_HALF = G_HT * G_BK * 2;          // 16 KiB per half-tile
 constexpr int G_BUF = 4 * G_HALF;                                         // A0 A1 B0 B1
+constexpr int G_THREADS = 256;
 
-// W row behind local row rho = r0 + 64 i (r0 = 0..63, i = 0, 1) of A half hA of workgroup column bx, split into the part that depends
-// on the thread (r0), the part that is uniform in the workgroup (hA, i) and the tile's column term (bx x 256 rows; SiLU: bx x 128):
-//   plain / residual: bx*256 + hA*128 + rho          SiLU (N == I): hA*N + bx*128 + rho
-//   RoPE: head = bx*(256/D) + rho/hd2, row = head*D + hA*hd2 + rho%hd2  (hd2 = D/2 divides 64: rho/hd2 = r0/hd2 + i*(64/hd2))
-template <int EPI, int RD>
-__device__ __forceinline__ int g_w_thr(int r0) {
-    if (g_rope(EPI)) { constexpr int hd2 = RD / 2 > 0 ? RD / 2 : 1; return (r0 / hd2) * RD + r0 % hd2; }
-    return r0;
-}
-template <int EPI, int RD>
-__device__ __forceinline__ int g_w_uni(int hA, int i, int N) {
-    if (g_glu(EPI)) return hA * N + i * 64;
-    if (g_rope(EPI)) return i * 128 + hA * (RD / 2);
-    return hA * 128 + i * 64;
+// 1 KiB of an operand into LDS: 16 bytes a lane from base + off, lane-linear at the byte that M0 holds (set an instruction before, by the hardware's rule).  Inline asm: hipcc drains the
+// builtin in front of LDS reads that it cannot tell apart from it; the requests are counted by hand.  Nothing else in this kernel uses M0.
+__device__ __forceinline__ void g_dma(unsigned off, const char *base) { asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base) : "memory"); }
+
+// 4 bytes a lane from a pointer each
+__device__ __forceinline__ void g_dma4(unsigned lds, const void *src) {
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, off\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "s"(lds), "v"(src) : "memory");
 }
 
-// RD: head_dim of the RoPE variant as a compile-time constant (64 or 128; 0 for the other epilogues): its row map and pair geometry
-// fold to shifts, and the scalar registers they needed in the K loop are what pushed that variant into SGPR -> VGPR spills
+// c += a . b (FIRST: c = a . b) with the accumulators held where they are: the 256 of a lane fill the accumulation registers, and hipcc, which gives every product a destination of its own, would
+// move them about (200 copies in a K-tile of 128 products).  Hazards that hipcc does not see behind inline asm: an accumulator is never written but by a product (a tile's first ones take no addend:
+// nothing has to be zeroed either), and G256_SETTLE stands in front of the first ordinary read.
+template <bool FIRST>
+__device__ __forceinline__ void g_mma(half8_t a, half8_t b, float4_t &c) {
+#ifdef NVR_BF16
+    if constexpr (FIRST) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
+    else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+#else
+    if constexpr (FIRST) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
+    else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+#endif
+}
+
 template <int EPI, int RD = 0, bool GRP = false>
-__global__ __launch_bounds__(512) void gemm256_kernel(const half_t *__restrict__ x, int64_t ldx, const half_t *__restrict__ W,
+__global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__restrict__ x, int64_t ldx, const half_t *__restrict__ W,
                                                       int T, int K, int N, int NW, half_t *__restrict__ y, typename G256Args<EPI>::type epi,
-                                                      int tiles_x, int tiles_y, int CG) {
-    extern __shared__ __attribute__((aligned(16))) char smem[];           // 2 x G_BUF
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+                                                      int tiles_x, int tiles_y, int PW) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];           // 2 x G_BUF, then what an epilogue needs
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int r = lane & 15, q = lane >> 4;
-    const int wn = wave >> 2, wm = wave & 3;
-    const int grp = __builtin_amdgcn_readfirstlane(wave >> 2);
+    const int wn = wave >> 1, wm = wave & 1;
 
     // Persistent workgroup.  The K-tile stream runs ACROSS its tiles: K-tile g of the stream lives in buffer g & 1, and the
-    // last K-tile of a tile already stages K-tile 0 of the next tile, so those loads fly during the epilogue.
-    // Tile order is XCD-aware (workgroup w runs on XCD w % 8, each XCD has its own 4 MiB L2): the 8 XCDs form CG column
-    // groups x 8/CG row groups; an XCD owns the columns of its group (its W slice stays L2-resident) and every
-    // (8/CG)-th row block, and its workgroups walk that set column-fastest, so the workgroups that share an x row block
-    // run on ONE XCD at the same time: x is fetched from HBM CG times instead of once per XCD that happens to see it.
-    const int tiles_total = tiles_x * (GRP && epi.rows_used ? min(tiles_y, (*epi.rows_used + 255) / 256) : tiles_y);     // (row blocks are the slow index of the tile order)
-    int xcd_step = 0, u = 0, nbx = 0, bx0 = 0, rg = 0, RG = 1, n_u = 0;
-    if (CG > 0) {
-        const int c = blockIdx.x & 7;
-        RG = 8 / CG; nbx = tiles_x / CG; bx0 = (c % CG) * nbx; rg = c / CG;
-        n_u = nbx * ((tiles_y - rg + RG - 1) / RG);                       // tiles of this XCD
-        u = blockIdx.x >> 3; xcd_step = gridDim.x >> 3;
-    }
-    // LM head: W (the [V, hidden] head: 311 MB on Qwen3-0.6B) is the stream and x (T rows) sits in every L2, so the tiles_y row blocks of ONE
-    // column tile run at the same time on the SAME XCD (workgroups w, w + 8, ...: index uu -> XCD uu & 7, slot uu >> 3; tiles_y consecutive
-    // slots share a column tile): its 512 KiB of W rows are fetched from HBM once and found in that XCD's L2 by the others.  The index space is
-    // padded to whole groups of 8 column tiles; the holes (only in the last group) end a workgroup's walk.
-    auto lm_bx = [&](int uu) { return ((uu >> 3) / tiles_y) * 8 + (uu & 7); };
+    // last two K-tiles of a tile already stage K-tiles 0 and 1 of the next one, so those loads fly during the epilogue.
+    // Tile order: column panels of PW tiles, each walked row block by row block; the line of tiles is cut into eight equal pieces, one per XCD (workgroup w runs on XCD w % 8, each XCD has its own
+    // 4 MiB L2).  The 32 workgroups of an XCD are then at about PW columns x 32 / PW row blocks at any time, and fetch PW + 32 / PW half-megabyte slices of either operand for a K-tile instead of
+    // the 18 or 33 of a plain order (us, one box each: 4096 x 12288 x 4096 278 -> 272; 32768 x 1024 x 4096 230 -> 221; 32768 x 2048 x 1024 112 -> 103).
+    const int rows_y = GRP && epi.rows_used ? min(tiles_y, (__builtin_amdgcn_readfirstlane(*epi.rows_used) + 255) / 256) : tiles_y, tiles_total = tiles_x * rows_y;
+    const int xcd = blockIdx.x & 7, step = gridDim.x >> 3, u_end = tiles_total / 8 * (xcd + 1) + min(xcd + 1, tiles_total % 8);
+    int u = tiles_total / 8 * xcd + min(xcd, tiles_total % 8) + (int)(blockIdx.x >> 3);
+    if (u >= u_end) return;
+    struct Tile { int bx, by; };
     auto tile_of = [&](int uu) {
-        if (EPI == GEPI_LMHEAD) return ((uu >> 3) % tiles_y) * tiles_x + lm_bx(uu);
-        return CG > 0 ? (rg + RG * (uu / nbx)) * tiles_x + bx0 + uu % nbx : uu;
+        const int panel = uu / (PW * rows_y), rem = uu - panel * (PW * rows_y), width = min(PW, tiles_x - panel * PW), by = rem / width;
+        return Tile{panel * PW + rem - by * width, by};
     };
-    auto have = [&](int uu) {
-        if (EPI == GEPI_LMHEAD) return uu < ((tiles_x + 7) / 8) * 8 * tiles_y && lm_bx(uu) < tiles_x;
-        return CG > 0 ? uu < n_u : uu < tiles_total;
-    };
-    if (CG <= 0) { u = blockIdx.x; xcd_step = gridDim.x; }
-    if (!have(u)) return;
-    // staging sources: thread copies pieces idx = i*512 + tid (i = 0,1) of each half-tile: row = idx/8 = r0 + 64 i, LDS slot idx%8.
-    // Address = tile base (scalar) + uniform row term of (half, i) (scalar) + ONE thread constant per operand: two 64-bit registers
-    // instead of eight pointers that had to be rebuilt, with the RoPE row map's divisions, inside the last K-tile of every tile
-    // (r03: that rebuild spilled ~80 registers to scratch in the RoPE variant — global-memory round trips in the K loop).
-    const int r0 = tid >> 3, cch = ((tid & 7) ^ (r0 & 7)) * 8;            // row inside a 64-row group, swizzled 16-byte chunk (elements)
-    const int64_t a_thr = (int64_t)g_w_thr<EPI, RD>(r0) * K + cch, b_thr = (int64_t)r0 * ldx + cch;
-    const half_t *wb = W, *xb = x;                                         // of the tile being STAGED (the next one during a tile's last K-tile)
-    int rows_left = 0x3fffffff;                                            // T - 1 - m0 when the tile's row block is ragged
-    int wrows_left = 0x3fffffff;                                           // LM head: N - 1 - bx * 256 when the tile's vocabulary block is ragged
-    auto set_sources = [&](int tile) {
-        const int bx = tile % tiles_x, m0 = (tile / tiles_x) * 256;
-        wb = W + (int64_t)bx * (g_glu(EPI) ? 128 : 256) * K;
-        if (GRP) wb += (int64_t)epi.row_w[tile / tiles_x] * epi.w_stride;
-        xb = x + (int64_t)m0 * ldx;
-        rows_left = m0 + 256 > T ? T - 1 - m0 : 0x3fffffff;
-        if (EPI == GEPI_LMHEAD) wrows_left = bx * 256 + 256 > N ? N - 1 - bx * 256 : 0x3fffffff;
-    };
-    // half-tile ids: 0 = A0, 1 = A1, 2 = B0, 3 = B1; kt = K-tile index inside the (current or next) tile, g = stream index
-    auto stage = [&](int ht, int kt, int g) {
-        char *dst = smem + (g & 1) * G_BUF + ht * G_HALF;
-        const int k0 = kt * G_BK;
+
+    constexpr int hd2 = g_rope(EPI) ? RD / 2 : 1;
+    constexpr int OUTC = g_glu(EPI) ? 128 : 256;                          // output columns of a tile
+    // Staging: a request is 32 rows (8 lanes a row) of a half-tile; LDS row rho = r0 + 32 i.  W row behind LDS row rho of A half hA: the 32 rows of a group lie in the order in which the
+    // accumulators of two neighbouring 16-row tiles give a lane eight neighbouring columns (LDS row 16 b + 4 a + e holds row 8 a + 4 b + e), so that results leave as 16-byte pieces straight from
+    // the registers; groups by column: plain bx*256 + hA*128 + ..   gate / up: hA*N + bx*128 + ..   RoPE: half hA of the tile's 256 / D heads, group by group; of two heads of 128 a wave gets the
+    // same 32 columns of both (GEPI_ROPE: one set of sines serves the two; loading them for each head took 13 us of 259 at 32768 x 1024 x 4096) or one head whole (GEPI_QKN: its norm is then the wave's own).
+    const int r0 = tid >> 3, pr = ((r0 & 15) >> 2) * 8 + (r0 >> 4) * 4 + (r0 & 3);
+    const unsigned cch = (unsigned)(((tid & 7) ^ (r0 & 7)) * 16);         // swizzled 16-byte chunk of the row
+    constexpr int PH = EPI == GEPI_QKN ? 2 : 1;                           // 32-column groups that a wave has of a half head
+    auto w_row = [&](int i) { return !g_rope(EPI) ? i * 32 + pr : RD == 64 ? i * 64 + pr : PH == 2 ? (i >> 1) * 128 + (i & 1) * 32 + pr : (i & 1) * 128 + (i >> 1) * 32 + pr; };
+    const int64_t half_w = (int64_t)(g_glu(EPI) ? N : g_rope(EPI) ? hd2 : 128) * K;      // from an A half's rows to the other's
+    unsigned va[EPI == GEPI_LMHEAD ? 8 : 4], vb[8];                       // byte offsets of the thread's pieces from the tile's rows
+    const char *pa0 = nullptr, *pa1 = nullptr, *pb = nullptr;             // next K-tile to request
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const half_t *src;
-            if (ht < 2) {
-                src = wb + (int64_t)g_w_uni<EPI, RD>(ht & 1, i, N) * K + a_thr + k0;
-                if (EPI == GEPI_LMHEAD && wrows_left != 0x3fffffff && (ht & 1) * 128 + i * 64 + r0 > wrows_left) src = wb + (int64_t)wrows_left * K + cch + k0;   // clamp
-            } else {
-                const int rowu = (ht & 1) * 128 + i * 64;
-                src = xb + (int64_t)rowu * ldx + b_thr + k0;
-                if (rows_left != 0x3fffffff && rowu + r0 > rows_left) src = xb + (int64_t)rows_left * ldx + cch + k0;   // ragged last row block: clamp
-            }
-            __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void *)(dst + (i * 512 + wave * 64) * 16), 16, 0, 0);
+    for (int i = 0; i < 4; ++i) va[i] = (unsigned)w_row(i) * (unsigned)K * 2u + cch;
+    auto set_sources = [&](Tile t) {
+        const int bx = t.bx, m0 = t.by * 256;
+        const half_t *wb = W + (int64_t)bx * OUTC * K;
+        if (GRP) wb += (int64_t)__builtin_amdgcn_readfirstlane(epi.row_w[t.by]) * epi.w_stride;
+        pa0 = (const char *)wb;
+        pa1 = (const char *)(wb + half_w);
+        pb = (const char *)(x + (int64_t)m0 * ldx);
+        const int rows_left = T - 1 - m0;                                 // ragged last row block: its last row again
+#pragma unroll
+        for (int i = 0; i < 8; ++i) vb[i] = (unsigned)min(i * 32 + r0, rows_left) * (unsigned)ldx * 2u + cch;
+        if constexpr (EPI == GEPI_LMHEAD) {                               // (a ragged vocabulary block likewise; both halves count from its first row)
+            pa1 = pa0;
+            const int wrows_left = N - 1 - bx * 256;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) va[i] = (unsigned)min(i * 32 + pr, wrows_left) * (unsigned)K * 2u + cch;
+        }
+    };
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)smem, lds_w = lds0 + (unsigned)wave * 1024u;
+    // piece i = 0..3 of half-tile ht (0 = A0, 1 = A1, 2 = B0, 3 = B1)
+    auto aim = [&](int ht, int i, unsigned lds) { asm volatile("s_add_u32 m0, %0, %1" ::"s"(lds), "i"(ht * G_HALF + i * 4096) : "scc"); };
+    auto request = [&](int ht, int i) {
+        if (ht < 2) g_dma(va[EPI == GEPI_LMHEAD ? ht * 4 + i : i], ht ? pa1 : pa0);
+        else g_dma(vb[(ht - 2) * 4 + i], pb);
+    };
+    auto request_all = [&](int g) {                                       // a whole K-tile, in the order of the phases: A0, B0, B1, A1
+#pragma unroll
+        for (int n = 0; n < 16; ++n) {
+            const int ht = n < 4 ? 0 : n < 8 ? 2 : n < 12 ? 3 : 1;
+            aim(ht, n & 3, lds_w + (unsigned)((g & 1) * G_BUF));
+            asm volatile("s_nop 0");
+            request(ht, n & 3);
+        }
+    };
+    // RoPE: positions (low dwords of the int64 entries) and cache slots of a tile's 256 token rows travel to LDS behind the K-tile ring by LDS-DMA, 4 bytes per lane (64 rows a wave), into one
+    // of two 2 KiB slots by tile parity, one tile ahead.
+    auto request_rows = [&](Tile t, int slot) {
+        if (g_rope(EPI)) {
+            int m = t.by * 256 + wave * 64 + lane; if (m > T - 1) m = T - 1;
+            const unsigned dst = lds0 + (unsigned)(2 * G_BUF + slot * 2048 + wave * 256);
+            g_dma4(dst, epi.pos + m);
+            if (epi.slots) g_dma4(dst + 1024, epi.slots + m);
         }
     };
 
-    float4_t acc[2][4][2][2];                                             // [A half][n-tile][B half][m-tile]
-    half8_t af[4][2], bf[2][2];                                           // [tile][k-step]
-    auto read_a = [&](const char *buf, int hA) {
-        const char *base = buf + hA * G_HALF;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = wn * 64 + i * 16 + r;
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-                af[i][ks] = *reinterpret_cast<const half8_t *>(base + (row * 8 + ((ks * 4 + q) ^ (row & 7))) * 16);
-        }
+    float4_t acc[2][4][2][4];                                             // [A half][n-tile][B half][m-tile]
+    half8_t fa[2][4][2], fb[2][4][2];                                     // [half][tile][k-step]
+    const int sw = (q ^ (r & 7)) * 16;
+    const int a_lane = (wn * 64 + r) * 128 + sw, b_lane = 2 * G_HALF + (wm * 64 + r) * 128 + sw;
+    auto read = [&](half8_t (&f)[4][2], int e, int half, int lane_at, int g) {      // fragment e of the 8 of half-tile `half` of an operand: tile e / 2, k-step e & 1 (chunk + 4, i.e. ^ 64)
+        f[e >> 1][e & 1] = *reinterpret_cast<const half8_t *>(smem + (g & 1) * G_BUF + half * G_HALF + (e >> 1) * 2048 + (lane_at ^ ((e & 1) * 64)));
     };
-    auto read_b = [&](const char *buf, int hB) {
-        const char *base = buf + (2 + hB) * G_HALF;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int row = wm * 32 + j * 16 + r;
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-                bf[j][ks] = *reinterpret_cast<const half8_t *>(base + (row * 8 + ((ks * 4 + q) ^ (row & 7))) * 16);
-        }
-    };
-    auto mma = [&](float4_t (&c)[4][2][2], int hB) {                      // c = acc[hA]
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    c[i][hB][j] = mfma16(af[i][ks], bf[j][ks], c[i][hB][j]);
-    };
+    // One phase: the 32 products of quadrant (A half HA, B half HB) of a K-tile, B's fragments outermost.  A product leaves its wave room for three instructions: the 8 fragments of the half-tile that
+    // the phase brings into registers (F of READ_G, one behind every fourth product, or behind the products of the B fragment that they replace) and the four pieces of the half-tile that it
+    // requests (two instructions each) go between them.  Own requests that the next phase reads have landed (all but the youngest five half-tiles), own reads of the phase before are back, barrier.
+#define G256_PHASE(HA_, HB_, F_, FH_, LANE_, READ_G_, RHT_, VM_, FIRST_)                                                                          \
+    _Pragma("unroll") for (int n = 0; n < 32; ++n) {                                                                                       \
+        constexpr bool behind = (RHT_) == 1;                              /* phase 3 */                                                    \
+        if (!behind && n % 3 == 0 && n < 24) read(F_[FH_], n / 3, FH_, LANE_, READ_G_);                                                    \
+        if (behind && n >= 8 && n % 8 == 0) { read(F_[FH_], n / 4 - 2, FH_, LANE_, READ_G_); }                                             \
+        if (behind && n >= 8 && n % 8 == 1) { read(F_[FH_], n / 4 - 1, FH_, LANE_, READ_G_); }                                             \
+        if (n % 8 == 4) aim(RHT_, n / 8, req_lds);                                                                                         \
+        if (n % 8 == 5) request(RHT_, n / 8);                                                                                              \
+        __builtin_amdgcn_sched_barrier(0);                                                                                                 \
+        if ((FIRST_) && !(n & 4)) g_mma<true>(fa[HA_][n & 3][0], fb[HB_][n >> 3][0], acc[HA_][n & 3][HB_][n >> 3]);                        \
+        else g_mma<false>(fa[HA_][n & 3][(n >> 2) & 1], fb[HB_][n >> 3][(n >> 2) & 1], acc[HA_][n & 3][HB_][n >> 3]);                      \
+        __builtin_amdgcn_sched_barrier(0);                                                                                                 \
+    }                                                                                                                                      \
+    if ((RHT_) == 1) { read(F_[FH_], 6, FH_, LANE_, READ_G_); read(F_[FH_], 7, FH_, LANE_, READ_G_); }                                     \
+    asm volatile("" ::: "memory");                                                                                                         \
+    __builtin_amdgcn_s_waitcnt(((VM_) & 15) | 0x70 | ((RHT_) == 1 ? 2 << 8 : 0) | ((VM_) >> 4) << 14);                                     \
+    __builtin_amdgcn_s_barrier();                                                                                                          \
+    asm volatile("" ::: "memory");
+#define G256_KTILE(VM_, FIRST_)                                                                                                                    \
+    {                                                                                                                                      \
+        const unsigned req_lds = lds_w + (unsigned)((g & 1) * G_BUF);                                                                      \
+        G256_PHASE(0, 0, fb, 1, b_lane, g, 0, VM_, FIRST_)                                                                                         \
+        G256_PHASE(0, 1, fa, 1, a_lane, g, 2, VM_, FIRST_)                                                                                         \
+        G256_PHASE(1, 1, fa, 0, a_lane, g + 1, 3, VM_, FIRST_)                                                                                     \
+        G256_PHASE(1, 0, fb, 0, b_lane, g + 1, 1, VM_, FIRST_)                                                                                     \
+        advance();                                                                                                                         \
+        ++g;                                                                                                                               \
+    }
+#define G256_SETTLE(A_, I_)                                               /* (wait states between a product and an ordinary read of its result, which hipcc does not count behind inline asm) */    \
+    asm volatile("s_nop 15\n\ts_nop 3" : "+a"(acc[A_][I_][0][0]), "+a"(acc[A_][I_][0][1]), "+a"(acc[A_][I_][0][2]), "+a"(acc[A_][I_][0][3]), "+a"(acc[A_][I_][1][0]), "+a"(acc[A_][I_][1][1]),    \
+                 "+a"(acc[A_][I_][1][2]), "+a"(acc[A_][I_][1][3]));
 
-    // The two wave groups (waves 0-3 and 4-7: one wave of each per SIMD) run ONE barrier interval apart, and a phase is
-    // two intervals — R {ds_read, stage one half-tile, s_waitcnt vmcnt, barrier} and M {16 MFMAs, barrier} — so that on every
-    // SIMD the fragment reads and the LDS-DMA issue of one wave (~100 clocks a piece) overlap the MFMAs of the other.  Group 1
-    // takes one extra barrier before each tile's K loop, group 0 one after it.  Hazards with the stagger: a half-tile staged in
-    // R(p) is first read in R(p+3); every wave counts its own loads at the end of R(p+2) (vmcnt(4): all but the two youngest
-    // half-tiles, those of R(p+1) and R(p+2); the epilogue's stores count too, which only makes the wait stricter), i.e. group
-    // 0 in interval 2p+4 and group 1 in 2p+5, and the earliest reader (group 0, R(p+3)) runs in interval 2p+6.  A half-tile is
-    // restaged no earlier than the interval after its last ds_read by either group has returned (group 1's R(3) reads B0 while
-    // group 0's R(0) of the next K-tile stages A0; B0 is restaged two intervals later).
-    // RoPE: positions (low dwords of the int64 entries) and cache slots of a tile's 256 token rows travel to LDS behind the K-tile ring
-    // by LDS-DMA, 4 bytes per lane (waves 0-3: 64 rows each), into one of two 2 KiB slots by tile parity.  They are requested one tile
-    // AHEAD, at the start of the previous tile's epilogue (whose first barrier drains the wave's requests anyway): asked for at the
-    // start of their own tile they sat in front of that tile's first staging waits (s_waitcnt vmcnt is in issue order) and stalled
-    // every tile's first K-tile by a memory round trip.
-    auto request_rows = [&](int tile_, int slot) {
-        if (g_rope(EPI) && grp == 0) {
-            int m = (tile_ / tiles_x) * 256 + wave * 64 + lane; if (m > T - 1) m = T - 1;
-            char *dst = smem + 2 * G_BUF + slot * 2048 + wave * 256;
-            __builtin_amdgcn_global_load_lds(epi.pos + m, (__attribute__((address_space(3))) void *)dst, 4, 0, 0);
-            if (epi.slots) __builtin_amdgcn_global_load_lds(epi.slots + m, (__attribute__((address_space(3))) void *)(dst + 1024), 4, 0, 0);
-        }
-    };
     const int KT = K / G_BK;
-    int tile = tile_of(u);
+    Tile tile = tile_of(u);
+    int su = u, skt = 0;                               // su, skt: tile and K-tile that the next requests are for
+    auto advance = [&]() {
+        pa0 += 2 * G_BK; pa1 += 2 * G_BK; pb += 2 * G_BK;
+        if (++skt == KT) {
+            skt = 0;
+            if (su + step < u_end) { su += step; set_sources(tile_of(su)); }
+            else { pa0 -= 2 * (int64_t)K; pa1 -= 2 * (int64_t)K; pb -= 2 * (int64_t)K; }      // (nothing left: the last tile's first K-tiles again, which nobody reads)
+        }
+    };
     set_sources(tile);
     request_rows(tile, 0);
-    stage(0, 0, 0); stage(2, 0, 0); stage(3, 0, 0); stage(1, 0, 0);       // A0, B0, B1, A1 of the first K-tile
-    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    request_all(0);
+    advance();
+    request_all(1);
+    advance();
+    asm volatile("s_waitcnt vmcnt(20)" ::: "memory");                     // (the rows and) A0, B0 and B1 of K-tile 0
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int e = 0; e < 8; ++e) { read(fa[0], e, 0, a_lane, 0); read(fb[0], e, 0, b_lane, 0); }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();                                         // (phase 0 refills A0)
+    asm volatile("" ::: "memory");
 
-#define G256_R_END(N_)                                                                                                \
-    asm volatile("s_waitcnt vmcnt(" #N_ ")" ::: "memory");                                                            \
-    __builtin_amdgcn_s_barrier();
-#define G256_M(C_, HB_)                                                                                               \
-    __builtin_amdgcn_s_setprio(1);                                                                                    \
-    mma(C_, HB_);                                                                                                     \
-    __builtin_amdgcn_s_setprio(0);                                                                                    \
-    __builtin_amdgcn_s_barrier();
-#define G256_S(HT_) if (more) stage(HT_, skt, g + 1);
-#define G256_W(NOMORE_) if (more) { G256_R_END(4) } else { G256_R_END(NOMORE_) }
+    const int64_t ldy = [&]() -> int64_t { if constexpr (EPI == GEPI_CLAMP) return epi.ldo; else return g_rope(EPI) ? (int64_t)(epi.H + 2 * epi.KVH) * RD : (int64_t)N; }();
 
-    constexpr int OUTC = g_glu(EPI) ? 128 : 256;                  // output columns of a tile
-    int64_t ldy = g_rope(EPI) ? (int64_t)(epi.H + 2 * epi.KVH) * RD : (int64_t)N;
-    if constexpr (EPI == GEPI_CLAMP) ldy = epi.ldo;
-    constexpr int hd2 = g_rope(EPI) ? RD / 2 : 1;
-
+    // Stores that a whole tile's epilogue leaves behind every request that is under way then: the first K-tile of the next tile need not wait for them (they are counted in order with the requests;
+    // 32768 x 1024 x 4096: 231 -> 223 us).  RoPE's stores may be left out (slots), the LM head's are not told.
+    constexpr int SLACK = g_rope(EPI) || EPI == GEPI_LMHEAD ? 0 : g_glu(EPI) ? 16 : 32;
+    bool whole = false;                                                   // the tile before this one was a whole one
     int tile_no = 0;
     for (int g = 0;; ) {
-        if (grp == 1) __builtin_amdgcn_s_barrier();                       // stagger
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int b = 0; b < 2; ++b)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) acc[a][i][b][j] = (float4_t){0.f, 0.f, 0.f, 0.f};
-        const bool have_next = have(u + xcd_step);
-        const int next_tile = have_next ? tile_of(u + xcd_step) : 0;
-        for (int kt = 0; kt < KT; ++kt, ++g) {
-            const char *buf = smem + (g & 1) * G_BUF;
-            const bool last = kt == KT - 1;
-            const bool more = !last || have_next;
-            if (last && more) set_sources(next_tile);                     // from here on the staging feeds the next tile
-            const int skt = last ? 0 : kt + 1;
-            // phase 0: (A0, B0)
-            read_b(buf, 0); read_a(buf, 0);
-            G256_S(0)
-            G256_W(2)
-            G256_M(acc[0], 0)
-            // phase 1: (A0, B1)
-            read_b(buf, 1);
-            G256_S(2)
-            G256_W(0)
-            G256_M(acc[0], 1)
-            // phase 2: (A1, B1)
-            read_a(buf, 1);
-            G256_S(3)
-            G256_W(0)
-            G256_M(acc[1], 1)
-            // phase 3: (A1, B0)
-            read_b(buf, 0);
-            G256_S(1)
-            G256_W(0)
-            G256_M(acc[1], 0)
-        }
-        if (grp == 0) __builtin_amdgcn_s_barrier();                       // re-align the groups
+        const bool have_next = u + step < u_end;
+        if (SLACK > 0 && whole) G256_KTILE(20 + SLACK, true)
+        else G256_KTILE(20, true)
+        for (int kt = 1; kt < KT; ++kt) G256_KTILE(20, false)
+        whole = tile.by * 256 + 256 <= T;
+        G256_SETTLE(0, 0) G256_SETTLE(0, 1) G256_SETTLE(0, 2) G256_SETTLE(0, 3) G256_SETTLE(1, 0) G256_SETTLE(1, 1) G256_SETTLE(1, 2) G256_SETTLE(1, 3)
 
-
-        // ---- epilogue of `tile`: the buffer of the K-tile just consumed is dead: per 128-token half hB, stage
-        // [token][column] there (16-byte chunks XOR-swizzled by the row) and write 16-byte pieces of contiguous rows,
-        // while the next tile's first K-tile lands in the other buffer.
-        {   // (scope: the epilogue works on shadow copies of the thread coordinates, see etid)
-        char *scratch = smem + ((g - 1) & 1) * G_BUF;
-        const int bx = tile % tiles_x, m0 = (tile / tiles_x) * 256;
-        // The thread coordinates of the epilogue come from a value the compiler cannot see through: otherwise it hoists the epilogue's
-        // address arithmetic (LDS offsets of the 16 puts and the read-back pieces, row / column terms of the stores: ~70 registers of
-        // loop invariants) out of the persistent tile loop, where they cannot all stay in registers next to the K loop's 176 — they
-        // were spilled to scratch at kernel start and reloaded in every epilogue, one global-memory round trip after the other
-        // (RoPE variant, r03: 72-89 spilled registers).  Recomputing them per tile is ~100 VALU instructions.
-        int etid = tid;
-        asm volatile("" : "+v"(etid));
-        const int tid = etid, wave = tid >> 6, lane = tid & 63, r = lane & 15, q = lane >> 4, wn = wave >> 2, wm = wave & 3;
-        (void)wave; (void)lane;
-        if (EPI == GEPI_LMHEAD) {
-            // C layout of an MFMA: lane (r, q) holds 4 consecutive vocabulary entries (W rows q*4 .. q*4+3 of the 16-row tile) of token r.
+        // ---- epilogue of `tile`, straight from the accumulators: lane (r, q) has of token row m0 + hB*128 + wm*64 + j*16 + r the eight columns q*8 .. of every 32-column group wn*2 + p of either
+        // A half (tiles 2p and 2p + 1).  No LDS, no barrier: the requests of the next tile's first two K-tiles are under way.
+        {
+        const int bx = tile.bx, m0 = tile.by * 256;
+        // (the thread coordinates come from a value that the compiler cannot see through: otherwise it hoists the epilogue's address arithmetic out of the tile loop, where it has no registers)
+        int elane = lane;
+        asm volatile("" : "+v"(elane));
+        const int r = elane & 15, q = elane >> 4;
+        const int mrow = wm * 64 + r;                                     // + hB*128 + j*16
+        auto eight = [&](int a, int p, int b, int j) {
+            const float4_t lo = acc[a][2 * p][b][j], hi = acc[a][2 * p + 1][b][j];
+            return (half8_t){(half_t)lo[0], (half_t)lo[1], (half_t)lo[2], (half_t)lo[3], (half_t)hi[0], (half_t)hi[1], (half_t)hi[2], (half_t)hi[3]};
+        };
+        if constexpr (EPI == GEPI_LMHEAD) {
             // Per token row: (max, lowest index) over this lane's 32 entries in ascending column order (strict >: the first maximum stays),
             // then over the 4 lanes of the token (larger value, else lower index), then over the two wave columns through LDS.
-            float *sv = reinterpret_cast<float *>(scratch); int *si = reinterpret_cast<int *>(scratch + 1024);
-            const int n_base = bx * 256 + wn * 64 + q * 4;
-            float bestv[2][2]; int besti[2][2];
+            float *sv = reinterpret_cast<float *>(smem + 2 * G_BUF); int *si = reinterpret_cast<int *>(smem + 2 * G_BUF + 1024);
+            int lim = N - (bx * 256 + wn * 64 + q * 8);                   // vocabulary entries from the lane's first one on (opaque: no row of compares is kept over the K loop)
+            int nv = N, tv = T;
+            asm volatile("" : "+v"(lim), "+v"(nv), "+v"(tv));
+            const int n_base = nv - lim;
+            float bestv[2][4]; int besti[2][4];
 #pragma unroll
             for (int b = 0; b < 2; ++b)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const int ml = b * 128 + wm * 32 + j * 16 + r, m = m0 + ml;
+                for (int j = 0; j < 4; ++j) {
+                    const int ml = b * 128 + mrow + j * 16, m = m0 + ml;
                     float bv = -INFINITY; int bi = 0x7fffffff;
+                    float *lrow = epi.logits + (int64_t)m * nv + n_base;
+                    const int out = epi.logits && m < tv ? lim : 0;
 #pragma unroll
                     for (int a = 0; a < 2; ++a)
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            const int c0 = n_base + a * 128 + i * 16;
+                            const int c0 = a * 128 + (i >> 1) * 32 + (i & 1) * 4;
                             const float4_t v = acc[a][i][b][j];
-                            if (epi.logits && m < T && c0 < N) *reinterpret_cast<float4_t *>(epi.logits + (int64_t)m * N + c0) = v;
+                            if (c0 < out) *reinterpret_cast<float4_t *>(lrow + c0) = v;
 #pragma unroll
-                            for (int e = 0; e < 4; ++e)
-                                if (c0 + e < N && v[e] > bv) { bv = v[e]; bi = c0 + e; }
+                            for (int e = 0; e < 4; ++e) {
+                                const bool more = (c0 + e < lim) & (v[e] > bv);
+                                bv = more ? v[e] : bv; bi = more ? n_base + c0 + e : bi;
+                            }
                         }
 #pragma unroll
                     for (int o = 16; o < 64; o <<= 1) {
                         const float v2 = __shfl_xor(bv, o, 64); const int i2 = __shfl_xor(bi, o, 64);
-                        if (v2 > bv || (v2 == bv && i2 < bi)) { bv = v2; bi = i2; }
+                        const bool other = (v2 > bv) | ((v2 == bv) & (i2 < bi));
+                        bv = other ? v2 : bv; bi = other ? i2 : bi;
                     }
                     bestv[b][j] = bv; besti[b][j] = bi;
                     if (wn == 1 && q == 0) { sv[ml] = bv; si[ml] = bi; }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             __syncthreads();
             if (wn == 0 && q == 0) {
 #pragma unroll
                 for (int b = 0; b < 2; ++b)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const int ml = b * 128 + wm * 32 + j * 16 + r, m = m0 + ml;
+                    for (int j = 0; j < 4; ++j) {
+                        const int ml = b * 128 + mrow + j * 16, m = m0 + ml;
                         float bv = bestv[b][j]; int bi = besti[b][j];
                         const float v2 = sv[ml]; const int i2 = si[ml];
                         if (v2 > bv || (v2 == bv && i2 < bi)) { bv = v2; bi = i2; }
-                        if (m < T) { epi.pval[(int64_t)bx * T + m] = bv; epi.pidx[(int64_t)bx * T + m] = bi; }
+                        if (m < tv) { epi.pval[(int64_t)bx * tv + m] = bv; epi.pidx[(int64_t)bx * tv + m] = bi; }
                     }
             }
-            __syncthreads();                                              // the next tile's second K-tile is staged into this buffer
-        }
-        auto put = [&](int ml, int col, half4_t h) {                      // 4 consecutive columns (col % 4 == 0) of token row ml
-            *reinterpret_cast<half4_t *>(scratch + ml * (OUTC * 2) + ((((col >> 3) ^ (ml & 15)) << 4) | ((col & 4) << 1))) = h;
-        };
-        // RoPE (r03): the accumulators are staged as plain fp16 like GEPI_F16 and the rotation happens in the STORE phase, on pairs of
-        // 16-byte pieces (x1 = 8 columns of a head's first half, x2 = the same columns of its second half) read back from the LDS
-        // image: there the accumulators of the half are dead, so the cos / sin values of a thread's four pairs (16 x 16 B) are
-        // requested as ONE batch behind the staging barrier.  Rotating at the accumulators needed them one by one in front of each
-        // use (each waited for with vmcnt(0) while LDS-DMA was pending) inside 256 registers with spills: 23 k of a tile's 93 k
-        // cycles (profiles/r03_prefill_gemm_epilogue.txt).  Same arithmetic on the same fp16-rounded GEMM outputs: bit-identical.
-        // The tile's 256 positions and cache slots were brought into LDS by LDS-DMA when the tile started (below the tile loop's
-        // head), so the requests for the cos / sin rows leave right after a half's conversion and fly across its staging barrier.
-        if (have_next) request_rows(next_tile, (tile_no + 1) & 1);
-        const int *lds_pos = reinterpret_cast<const int *>(smem + 2 * G_BUF + (tile_no & 1) * 2048), *lds_slot = lds_pos + 256;
-        // A thread takes the same pair of pieces of every head of its rows: the heads share one set of cosines and sines (a thread per head and pair fetched them once for each
-        // head: for 256 x 256 outputs as many bytes as the outputs).
-        constexpr int hp = g_rope(EPI) ? RD / 16 : 1;                     // 16-byte pieces per half head = neighbouring lanes of a head's row
-        constexpr int RPP = 512 / hp, PASSES = g_rope(EPI) ? 128 / RPP : 1, HN = g_rope(EPI) ? 256 / RD : 1;      // rows per pass over a half, heads of a row
-        const int pcc = tid % hp, prow = tid / hp, head0 = bx * HN;
-        int rslot[PASSES];
-        float4_t cs[PASSES][2], sn[PASSES][2];
-        half8_t g1[HN], g2[HN];
-        // plain / residual / RoPE epilogues: all 128 accumulator registers become 64 registers of packed fp16 at once (the values the
-        // halves stage below), so that the second half's results do not sit in f32 under the first half's store phase: the RoPE
-        // store phase holds 64 registers of cos / sin next to them, and a spill here is a global-memory round trip (scratch)
-        half4_t pk[2][4][2][2];
-        if (!g_glu(EPI) && EPI != GEPI_LMHEAD) {
+            __syncthreads();                                              // (the next tile's partials go to the same place)
+        } else if constexpr (g_rope(EPI)) {
+            // Partners are in one lane: columns c .. c + 7 of a head's first half (A half 0) and the same ones of its second half (A half 1).  The products are rounded to 16 bits, then rotated.
+            if (have_next) request_rows(tile_of(u + step), (tile_no + 1) & 1);
+            const int *lds_pos = reinterpret_cast<const int *>(smem + 2 * G_BUF + (tile_no & 1) * 2048), *lds_slot = lds_pos + 256;
+            const int head0 = bx * (256 / RD) + (RD == 64 ? wn * 2 : PH == 2 ? wn : 0);      // head of the wave's group p: head0 + (PH == 2 ? 0 : p)
+            half8_t g1[2], g2[2];
+            if constexpr (EPI == GEPI_QKN) {
+                const half_t *w = head0 < epi.H ? epi.qn_w : epi.kn_w;
 #pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int b = 0; b < 2; ++b)
-#pragma unroll
-                        for (int j = 0; j < 2; ++j) {
-                            float4_t v = acc[a][i][b][j];
-                            if (EPI == GEPI_RELU2) {
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) { const float r = fmaxf((float)(half_t)v[e], 0.f); v[e] = r * r; }
-                            }
-                            if (EPI == GEPI_GELU_ERF) {
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) v[e] = gelu_erf_fast(v[e]);
-                            }
-                            pk[a][i][b][j] = (half4_t){(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
-                        }
-        }
-#pragma unroll
-        for (int hB = 0; hB < (EPI == GEPI_LMHEAD ? 0 : 2); ++hB) {
-            // GEPI_RESID: the residual pieces this thread will add to are requested first; their latency runs under the conversion
-            // of the accumulators, the LDS staging and the barrier
-            constexpr int RPC = (EPI == GEPI_RESID) ? (128 * (OUTC / 8)) / 512 : 1;
-            half8_t hres[RPC];
-            if (EPI == GEPI_RESID) {
-#pragma unroll
-                for (int kk = 0; kk < RPC; ++kk) {
-                    const int pidx = tid + kk * 512, row = pidx / (OUTC / 8), ch = pidx % (OUTC / 8);
-                    const int m = m0 + hB * 128 + row, col = bx * OUTC + ch * 8;
-                    hres[kk] = (m < T && col < ldy) ? *reinterpret_cast<const half8_t *>(y + (int64_t)m * ldy + col) : (half8_t)(half_t)0;
-                }
+                for (int p = 0; p < 2; ++p) { g1[p] = *reinterpret_cast<const half8_t *>(w + p * 32 + q * 8); g2[p] = *reinterpret_cast<const half8_t *>(w + 64 + p * 32 + q * 8); }
             }
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int ml = wm * 32 + j * 16 + r;                      // token row inside the half
-                if (EPI == GEPI_F16 || EPI == GEPI_RESID || g_rope(EPI) || EPI == GEPI_RELU2 || EPI == GEPI_GELU_ERF) {
-#pragma unroll
-                    for (int a = 0; a < 2; ++a)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int rho = wn * 64 + i * 16 + q * 4;     // local W row; RoPE: A0 / A1 hold the first / second halves of the heads
-                            const int colo = g_rope(EPI) ? (rho / hd2) * RD + a * hd2 + rho % hd2 : a * 128 + rho;
-                            put(ml, colo, pk[a][i][hB][j]);
-                        }
-                } else if (g_glu(EPI)) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        half4_t h;
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const float gf = (float)to_half_rn(acc[0][i][hB][j][e]), uf = (float)to_half_rn(acc[1][i][hB][j][e]);
-                            if constexpr (EPI == GEPI_CLAMP) h[e] = to_half_rn(clamped_unit(gf, uf, epi.limit, epi.alpha));
-                            else {
-                                const float sg = gate_factor(gf, EPI == GEPI_GELU);
-                                h[e] = to_half_rn(__fmul_rn(__fmul_rn(gf, sg), uf));
-                            }
-                        }
-                        put(ml, wn * 64 + i * 16 + q * 4, h);
-                    }
+            const int cc0 = (RD == 128 && PH == 1 ? wn * 32 : 0) + q * 8; // column in the half head (PH == 2: + p*32)
+            // rows of the caches and of y, from o1 (first half) and o2 (second half) of group p
+            auto leave = [&](int t, int p, bool rot, half8_t o1, half8_t o2) {
+                const int ml = (t >> 2) * 128 + mrow + (t & 3) * 16, m = m0 + ml, head = head0 + (PH == 2 ? 0 : p), c = (PH == 2 ? p * 32 : 0) + cc0;
+                if (m >= T) return;
+                if (head < epi.H || !epi.kv_cache_only) {
+                    half_t *yrow = y + (int64_t)m * ldy + (int64_t)head * RD + c;
+                    *reinterpret_cast<half8_t *>(yrow) = o1;
+                    *reinterpret_cast<half8_t *>(yrow + hd2) = o2;
                 }
-            }
-            if (g_rope(EPI)) {
+                if (head >= epi.H) {
+                    const int slot = epi.slots ? lds_slot[ml] : -1;
+                    if (slot < 0) return;
+                    half_t *crow = (rot ? epi.kc : epi.vc) + ((int64_t)slot * epi.KVH + (rot ? head - epi.H : head - epi.H - epi.KVH)) * RD + c;
+                    *reinterpret_cast<half8_t *>(crow) = o1;
+                    *reinterpret_cast<half8_t *>(crow + hd2) = o2;
+                }
+            };
+            if (head0 < epi.H + epi.KVH) {                                // q and k heads rotate, v heads pass through
+                constexpr int AHEAD = 4 - PH;                             // sines of a token tile's rows, requested three (QKN: two) tiles ahead
+                float4_t cs[AHEAD][PH][2], sn[AHEAD][PH][2];
+                auto sines = [&](int t) {
+                    const int64_t at = (int64_t)lds_pos[(t >> 2) * 128 + mrow + (t & 3) * 16] * hd2 + cc0;
 #pragma unroll
-                for (int kk = 0; kk < PASSES; ++kk) {
-                    const int row = hB * 128 + prow + kk * RPP;
-                    const int pos = lds_pos[row];
-                    rslot[kk] = epi.slots ? lds_slot[row] : -1;
-#pragma unroll
-                    for (int hh = 0; hh < 2; ++hh) cs[kk][hh] = sn[kk][hh] = (float4_t){0.f, 0.f, 0.f, 0.f};     // (left open, they are carried from tile to tile: 24 registers over the K loop, whose staging addresses then sat in scratch — each wait for one was a wait for the whole ring; 32768 x 4096 x 1024: 319 -> 259 us)
-                    if (head0 < epi.H + epi.KVH) {                        // q and k heads rotate, v heads pass through
+                    for (int p = 0; p < PH; ++p)
 #pragma unroll
                         for (int hh = 0; hh < 2; ++hh) {
-                            cs[kk][hh] = *reinterpret_cast<const float4_t *>(epi.cos_t + (int64_t)pos * hd2 + pcc * 8 + hh * 4);
-                            sn[kk][hh] = *reinterpret_cast<const float4_t *>(epi.sin_t + (int64_t)pos * hd2 + pcc * 8 + hh * 4);
+                            cs[t % AHEAD][p][hh] = *reinterpret_cast<const float4_t *>(epi.cos_t + at + p * 32 + hh * 4);
+                            sn[t % AHEAD][p][hh] = *reinterpret_cast<const float4_t *>(epi.sin_t + at + p * 32 + hh * 4);
                         }
-                    }
-                }
-            }
-            if constexpr (EPI == GEPI_QKN) {
+                };
+                #pragma unroll
+                for (int t = 0; t < AHEAD; ++t) sines(t);
 #pragma unroll
-                for (int hh = 0; hh < HN; ++hh) {
-                    const half_t *w = head0 + hh < epi.H ? epi.qn_w : epi.kn_w;
-                    g1[hh] = *reinterpret_cast<const half8_t *>(w + pcc * 8); g2[hh] = *reinterpret_cast<const half8_t *>(w + (hp + pcc) * 8);
-                }
-            }
-            __syncthreads();
-            constexpr int CPR = OUTC / 8;                                 // 16-byte pieces per row
-            if (EPI == GEPI_RESID) {
-                // h <- fp16(h + fp16(acc)): the rounding points of add_rmsnorm's add
+                for (int t = 0; t < 8; ++t) {
+                    const int b = t >> 2, j = t & 3;
+                    half8_t x1[2], x2[2];
 #pragma unroll
-                for (int kk = 0; kk < (128 * CPR) / 512; ++kk) {
-                    const int pidx = tid + kk * 512, row = pidx / CPR, ch = pidx % CPR;
-                    const int m = m0 + hB * 128 + row, col = bx * OUTC + ch * 8;
-                    if (m >= T || col >= ldy) continue;
-                    const half8_t v8 = *reinterpret_cast<const half8_t *>(scratch + row * (OUTC * 2) + ((ch ^ (row & 15)) << 4));
-                    half8_t o8;
+                    for (int p = 0; p < 2; ++p) { x1[p] = eight(0, p, b, j); x2[p] = eight(1, p, b, j); }
+                    if constexpr (EPI == GEPI_QKN) head_norm_pieces(x1, x2, g1, g2, epi.qk_eps);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) o8[e] = to_half_rn((float)hres[kk][e] + (float)v8[e]);
-                    *reinterpret_cast<half8_t *>(y + (int64_t)m * ldy + col) = o8;
-                }
-                __syncthreads();
-                continue;
-            }
-            if (g_rope(EPI)) {
-#pragma unroll
-                for (int kk = 0; kk < PASSES; ++kk) {
-                    const int row = prow + kk * RPP, m = m0 + hB * 128 + row;
-#pragma unroll
-                    for (int hh = 0; hh < HN; ++hh) {
-                        const int rhead = head0 + hh, ch1 = hh * 2 * hp + pcc, ch2 = ch1 + hp;
-                        const bool rot = rhead < epi.H + epi.KVH;
-                        half8_t x1 = *reinterpret_cast<const half8_t *>(scratch + row * (OUTC * 2) + ((ch1 ^ (row & 15)) << 4));
-                        half8_t x2 = *reinterpret_cast<const half8_t *>(scratch + row * (OUTC * 2) + ((ch2 ^ (row & 15)) << 4));
-                        half8_t o1 = x1, o2 = x2;
+                    for (int p = 0; p < 2; ++p) {
+                        const bool rot = PH == 2 || head0 + p < epi.H + epi.KVH;
+                        half8_t o1 = x1[p], o2 = x2[p];
                         if (rot) {
-                            if constexpr (EPI == GEPI_QKN) head_norm<hp>(x1, x2, g1[hh], g2[hh], epi.qk_eps);
 #pragma unroll
                             for (int e = 0; e < 8; ++e) {
-                                const float a = (float)x1[e], b = (float)x2[e], cc = cs[kk][e >> 2][e & 3], ss = sn[kk][e >> 2][e & 3];
-                                o1[e] = to_half_rn(mul_sub_unfused(a, cc, b, ss));
-                                o2[e] = to_half_rn(mul_add_unfused(b, cc, a, ss));
+                                const float f1 = (float)x1[p][e], f2 = (float)x2[p][e], cc = cs[t % AHEAD][PH == 2 ? p : 0][e >> 2][e & 3], ss = sn[t % AHEAD][PH == 2 ? p : 0][e >> 2][e & 3];
+                                o1[e] = to_half_rn(mul_sub_unfused(f1, cc, f2, ss));
+                                o2[e] = to_half_rn(mul_add_unfused(f2, cc, f1, ss));
                             }
                         }
-                        if (m >= T) continue;
-                        half_t *yrow = y + (int64_t)m * ldy + bx * OUTC;
-                        if (rhead < epi.H || !epi.kv_cache_only) {
-                            *reinterpret_cast<half8_t *>(yrow + ch1 * 8) = o1;
-                            *reinterpret_cast<half8_t *>(yrow + ch2 * 8) = o2;
-                        }
-                        if (rhead >= epi.H && rslot[kk] >= 0) {
-                            const int kvh = rot ? rhead - epi.H : rhead - epi.H - epi.KVH;
-                            half_t *crow = (rot ? epi.kc : epi.vc) + ((int64_t)rslot[kk] * epi.KVH + kvh) * RD;
-                            *reinterpret_cast<half8_t *>(crow + pcc * 8) = o1;
-                            *reinterpret_cast<half8_t *>(crow + (hp + pcc) * 8) = o2;
-                        }
+                        leave(t, p, rot, o1, o2);
                     }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (t + AHEAD < 8) sines(t + AHEAD);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                __syncthreads();
-                continue;
+            } else {
+#pragma unroll
+                for (int t = 0; t < 8; ++t)
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) leave(t, p, false, eight(0, p, t >> 2, t & 3), eight(1, p, t >> 2, t & 3));
+            }
+        } else {
+            constexpr int NA = g_glu(EPI) ? 1 : 2;
+            half_t *yt = y + (int64_t)m0 * ldy + (int64_t)bx * OUTC + wn * 64;
+            const unsigned lane_off = (unsigned)(mrow * ldy) + q * 8;
+            half8_t res[EPI == GEPI_RESID ? 8 : 1][2][2];                 // RESID: the rows that are added to, requested four token tiles ahead
+            auto residual = [&](int t) {
+                const int b = t >> 2, j = t & 3;
+                const bool in = m0 + b * 128 + mrow + j * 16 < T;
+#pragma unroll
+                for (int a = 0; a < 2; ++a)
+#pragma unroll
+                    for (int p = 0; p < 2; ++p)
+                        res[EPI == GEPI_RESID ? t : 0][a][p] = in ? *reinterpret_cast<const half8_t *>(yt + (int64_t)(b * 128 + j * 16) * ldy + lane_off + a * 128 + p * 32) : (half8_t)(half_t)0;
+            };
+            if (EPI == GEPI_RESID) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) residual(t);
             }
 #pragma unroll
-            for (int kk = 0; kk < (128 * CPR) / 512; ++kk) {
-                const int pidx = tid + kk * 512;
-                const int row = pidx / CPR, ch = pidx % CPR;
-                const int m = m0 + hB * 128 + row, col = bx * OUTC + ch * 8;
-                if (m >= T || col >= ldy) continue;
-                const half8_t v8 = *reinterpret_cast<const half8_t *>(scratch + row * (OUTC * 2) + ((ch ^ (row & 15)) << 4));
-                *reinterpret_cast<half8_t *>(y + (int64_t)m * ldy + col) = v8;
+            for (int t = 0; t < 8; ++t) {
+                const int b = t >> 2, j = t & 3;
+                if (EPI == GEPI_RESID && t < 4) residual(t + 4);
+                const bool in = m0 + b * 128 + mrow + j * 16 < T;
+                half_t *yrow = yt + (int64_t)(b * 128 + j * 16) * ldy + lane_off;
+#pragma unroll
+                for (int a = 0; a < NA; ++a)
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) {
+                        half8_t o;
+                        if constexpr (g_glu(EPI)) {
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) {
+                                const float gf = (float)to_half_rn(acc[0][2 * p + (e >> 2)][b][j][e & 3]), uf = (float)to_half_rn(acc[1][2 * p + (e >> 2)][b][j][e & 3]);
+                                if constexpr (EPI == GEPI_CLAMP) o[e] = to_half_rn(clamped_unit(gf, uf, epi.limit, epi.alpha));
+                                else {
+                                    const float sg = gate_factor(gf, EPI == GEPI_GELU);
+                                    o[e] = to_half_rn(__fmul_rn(__fmul_rn(gf, sg), uf));
+                                }
+                            }
+                        } else if constexpr (EPI == GEPI_RELU2) {
+                            const half8_t v = eight(a, p, b, j);
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) { const float f = fmaxf((float)v[e], 0.f); o[e] = (half_t)(f * f); }
+                        } else if constexpr (EPI == GEPI_GELU_ERF) {
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) o[e] = (half_t)gelu_erf_fast(acc[a][2 * p + (e >> 2)][b][j][e & 3]);
+                        } else if constexpr (EPI == GEPI_RESID) {
+                            // h <- fp16(h + fp16(acc)): the rounding points of add_rmsnorm's add
+                            const half8_t v = eight(a, p, b, j);
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) o[e] = to_half_rn((float)res[t][a][p][e] + (float)v[e]);
+                        } else o = eight(a, p, b, j);
+                        if (in) *reinterpret_cast<half8_t *>(yrow + a * 128 + p * 32) = o;
+                    }
             }
-            __syncthreads();
         }
         }   // epilogue scope
         ++tile_no;
         if (!have_next) break;
-        tile = next_tile; u += xcd_step;
+        u += step;
+        tile = tile_of(u);
     }
-#undef G256_R_END
-#undef G256_M
-#undef G256_S
-#undef G256_W
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                      // (requests behind the last tile: the LDS is given back only now)
+#undef G256_PHASE
+#undef G256_KTILE
+#undef G256_SETTLE
 }
 
 static int g256_prepare() {                                               // 128 KiB of dynamic LDS: opt-in once
@@ -542,15 +472,8 @@ static int g256_prepare() {                                               // 128
     done = true;
     return 0;
 }
-static int g256_grid(int tiles) { return tiles < 256 ? tiles : 256; }   // one persistent workgroup per CU (128 KiB of LDS each)
-// column groups CG for the XCD-aware tile order (0 = plain order).  Measured at T = 32768 (scratch/gemm_prefill_bench.py,
-// +-5 % run to run): the plain GEMMs and SiLU do not care (CG 0/1/2/4 within noise; CG = 8 loses 8 % at N = 6144), the
-// RoPE + KV-store epilogue gains 12 % with CG = 1 (an XCD writes whole output rows and cache rows at a time).
-static int g256_cg(int tiles_x, int tiles_y, bool rope) {
-    int cg = rope ? 1 : 0;
-    if (cg && (tiles_x % cg || tiles_y < 8 / cg || tiles_x * tiles_y < 256)) cg = 0;
-    return cg;
-}
+static int g256_grid(int tiles) { return tiles < 256 ? (tiles + 7) / 8 * 8 : 256; }   // one persistent workgroup per CU (128 KiB of LDS each), as many on every XCD
+static int g256_panel(int tiles_x) { const int panels = (tiles_x + 7) / 8; return (tiles_x + panels - 1) / panels; }   // columns of a panel: 8, or the next smaller number that makes the panels alike
 static int g256_check(const char *what) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "%s launch failed: %s", what, hipGetErrorString(e));
@@ -572,8 +495,8 @@ int gemm256(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int6
     if (!gemm256_ok(T, K, N, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm256: T=%ld K=%ld N=%ld", (long)T, (long)K, (long)N);
     if (int rc = g256_prepare()) return rc;
     const int tx = (int)(N / 256), tt = tx * (int)((T + 255) / 256);
-    gemm256_kernel<GEPI_F16><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
-                                                                                        (int)N, (int)N, (half_t *)y, G256Epi{}, tx, tt / tx, g256_cg(tx, tt / tx, false));
+    gemm256_kernel<GEPI_F16><<<dim3((unsigned)g256_grid(tt)), dim3(G_THREADS), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
+                                                                                        (int)N, (int)N, (half_t *)y, G256Epi{}, tx, tt / tx, g256_panel(tx));
     return g256_check("gemm256");
 }
 // y = max(x . W^T, 0)^2: a dense feed-forward's up product with its squared ReLU in the epilogue
@@ -581,8 +504,8 @@ int gemm256_relu2(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T
     if (!gemm256_ok(T, K, N, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm256_relu2: T=%ld K=%ld N=%ld", (long)T, (long)K, (long)N);
     if (int rc = g256_prepare()) return rc;
     const int tx = (int)(N / 256), tt = tx * (int)((T + 255) / 256);
-    gemm256_kernel<GEPI_RELU2><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
-                                                                                          (int)N, (int)N, (half_t *)y, G256Epi{}, tx, tt / tx, g256_cg(tx, tt / tx, false));
+    gemm256_kernel<GEPI_RELU2><<<dim3((unsigned)g256_grid(tt)), dim3(G_THREADS), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
+                                                                                          (int)N, (int)N, (half_t *)y, G256Epi{}, tx, tt / tx, g256_panel(tx));
     return g256_check("gemm256_relu2");
 }
 // y = gelu(x . W^T) with the error function, of the unrounded product
@@ -590,8 +513,8 @@ int gemm256_gelu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T,
     if (!gemm256_ok(T, K, N, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm256_gelu: T=%ld K=%ld N=%ld", (long)T, (long)K, (long)N);
     if (int rc = g256_prepare()) return rc;
     const int tx = (int)(N / 256), tt = tx * (int)((T + 255) / 256);
-    gemm256_kernel<GEPI_GELU_ERF><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
-                                                                                             (int)N, (int)N, (half_t *)y, G256Epi{}, tx, tt / tx, g256_cg(tx, tt / tx, false));
+    gemm256_kernel<GEPI_GELU_ERF><<<dim3((unsigned)g256_grid(tt)), dim3(G_THREADS), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
+                                                                                             (int)N, (int)N, (half_t *)y, G256Epi{}, tx, tt / tx, g256_panel(tx));
     return g256_check("gemm256_gelu");
 }
 // Rows grouped by expert (a mixture of experts over many tokens): T is a multiple of 256 and row block rb multiplies the matrix W + row_w[rb] * w_stride
@@ -601,8 +524,8 @@ int gemm256_grouped(const half_bits *x, int64_t ldx, const half_bits *W, int64_t
     if (int rc = g256_prepare()) return rc;
     G256Epi e{}; e.row_w = row_w; e.w_stride = w_stride; e.rows_used = rows_used;
     const int tx = (int)(N / 256), tt = tx * (int)(T / 256);
-    gemm256_kernel<GEPI_F16, 0, true><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K, (int)N, (int)N, (half_t *)y, e, tx,
-                                                                                                  tt / tx, 0);
+    gemm256_kernel<GEPI_F16, 0, true><<<dim3((unsigned)g256_grid(tt)), dim3(G_THREADS), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K, (int)N, (int)N, (half_t *)y, e, tx,
+                                                                                                  tt / tx, g256_panel(tx));
     return g256_check("gemm256_grouped");
 }
 int gemm256_grouped_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t w_stride, const int32_t *row_w, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s, const int32_t *rows_used) {
@@ -610,8 +533,8 @@ int gemm256_grouped_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W
     if (int rc = g256_prepare()) return rc;
     G256Epi e{}; e.row_w = row_w; e.w_stride = w_stride; e.rows_used = rows_used;
     const int tx = (int)(I / 128), tt = tx * (int)(T / 256);
-    gemm256_kernel<GEPI_SILU, 0, true><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K, (int)I, (int)(2 * I), (half_t *)out, e,
-                                                                                                   tx, tt / tx, 0);
+    gemm256_kernel<GEPI_SILU, 0, true><<<dim3((unsigned)g256_grid(tt)), dim3(G_THREADS), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K, (int)I, (int)(2 * I), (half_t *)out, e,
+                                                                                                   tx, tt / tx, g256_panel(tx));
     return g256_check("gemm256_grouped_silu_mul");
 }
 // h[T,N] <- fp16(h + fp16(x·Wᵀ)): the row-parallel GEMM with the residual add of qwen3.rs:382,389 in its epilogue (prefill steps on one
@@ -620,16 +543,16 @@ int gemm256_resid(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T
     if (!gemm256_ok(T, K, N, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm256_resid: T=%ld K=%ld N=%ld", (long)T, (long)K, (long)N);
     if (int rc = g256_prepare()) return rc;
     const int tx = (int)(N / 256), tt = tx * (int)((T + 255) / 256);
-    gemm256_kernel<GEPI_RESID><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
-                                                                                          (int)N, (int)N, (half_t *)h, G256Epi{}, tx, tt / tx, g256_cg(tx, tt / tx, false));
+    gemm256_kernel<GEPI_RESID><<<dim3((unsigned)g256_grid(tt)), dim3(G_THREADS), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
+                                                                                          (int)N, (int)N, (half_t *)h, G256Epi{}, tx, tt / tx, g256_panel(tx));
     return g256_check("gemm256_resid");
 }
 int gemm256_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s) {
     if (!gemm256_silu_ok(T, K, I, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm256_silu_mul: T=%ld K=%ld I=%ld", (long)T, (long)K, (long)I);
     if (int rc = g256_prepare()) return rc;
     const int tx = (int)(I / 128), tt = tx * (int)((T + 255) / 256);
-    gemm256_kernel<GEPI_SILU><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
-                                                                                         (int)I, (int)(2 * I), (half_t *)out, G256Epi{}, tx, tt / tx, g256_cg(tx, tt / tx, false));
+    gemm256_kernel<GEPI_SILU><<<dim3((unsigned)g256_grid(tt)), dim3(G_THREADS), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
+                                                                                         (int)I, (int)(2 * I), (half_t *)out, G256Epi{}, tx, tt / tx, g256_panel(tx));
     return g256_check("gemm256_silu_mul");
 }
 // out = gelu(gate) * up with the tanh form of gelu
@@ -637,8 +560,8 @@ int gemm256_gelu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_
     if (!gemm256_silu_ok(T, K, I, ldx)) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm256_gelu_mul: T=%ld K=%ld I=%ld", (long)T, (long)K, (long)I);
     if (int rc = g256_prepare()) return rc;
     const int tx = (int)(I / 128), tt = tx * (int)((T + 255) / 256);
-    gemm256_kernel<GEPI_GELU><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
-                                                                                         (int)I, (int)(2 * I), (half_t *)out, G256Epi{}, tx, tt / tx, g256_cg(tx, tt / tx, false));
+    gemm256_kernel<GEPI_GELU><<<dim3((unsigned)g256_grid(tt)), dim3(G_THREADS), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
+                                                                                         (int)I, (int)(2 * I), (half_t *)out, G256Epi{}, tx, tt / tx, g256_panel(tx));
     return g256_check("gemm256_gelu_mul");
 }
 // the clamped gated unit, rows of out ldo apart
@@ -647,8 +570,8 @@ int gemm256_clamped_glu(const half_bits *x, int64_t ldx, const half_bits *W, int
     if (int rc = g256_prepare()) return rc;
     G256EpiClamp e{}; e.limit = limit; e.alpha = alpha; e.ldo = ldo;
     const int tx = (int)(I / 128), tt = tx * (int)((T + 255) / 256);
-    gemm256_kernel<GEPI_CLAMP><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
-                                                                                          (int)I, (int)(2 * I), (half_t *)out, e, tx, tt / tx, g256_cg(tx, tt / tx, false));
+    gemm256_kernel<GEPI_CLAMP><<<dim3((unsigned)g256_grid(tt)), dim3(G_THREADS), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
+                                                                                          (int)I, (int)(2 * I), (half_t *)out, e, tx, tt / tx, g256_panel(tx));
     return g256_check("gemm256_clamped_glu");
 }
 int gemm256_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t H, int64_t KVH, int64_t D,
@@ -665,14 +588,14 @@ int gemm256_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, 
     const int tx = (int)(N / 256), tt = tx * (int)((T + 255) / 256);
     if (norm) {
         e.qn_w = (const half_t *)norm->q_w; e.kn_w = (const half_t *)norm->k_w; e.qk_eps = norm->eps;
-        gemm256_kernel<GEPI_QKN, 128><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF + 4096, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
-                                                                                                  (int)N, (int)N, (half_t *)qkv, e, tx, tt / tx, g256_cg(tx, tt / tx, true));
+        gemm256_kernel<GEPI_QKN, 128><<<dim3((unsigned)g256_grid(tt)), dim3(G_THREADS), 2 * G_BUF + 4096, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
+                                                                                                  (int)N, (int)N, (half_t *)qkv, e, tx, tt / tx, g256_panel(tx));
     } else if (D == 128)
-        gemm256_kernel<GEPI_ROPE, 128><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF + 4096, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
-                                                                                                  (int)N, (int)N, (half_t *)qkv, e, tx, tt / tx, g256_cg(tx, tt / tx, true));
+        gemm256_kernel<GEPI_ROPE, 128><<<dim3((unsigned)g256_grid(tt)), dim3(G_THREADS), 2 * G_BUF + 4096, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
+                                                                                                  (int)N, (int)N, (half_t *)qkv, e, tx, tt / tx, g256_panel(tx));
     else
-        gemm256_kernel<GEPI_ROPE, 64><<<dim3((unsigned)g256_grid(tt)), dim3(512), 2 * G_BUF + 4096, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
-                                                                                                 (int)N, (int)N, (half_t *)qkv, e, tx, tt / tx, g256_cg(tx, tt / tx, true));
+        gemm256_kernel<GEPI_ROPE, 64><<<dim3((unsigned)g256_grid(tt)), dim3(G_THREADS), 2 * G_BUF + 4096, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
+                                                                                                 (int)N, (int)N, (half_t *)qkv, e, tx, tt / tx, g256_panel(tx));
     return g256_check("gemm256_qkv_rope_store");
 }
 
@@ -691,9 +614,8 @@ int gemm256_lm_head(const half_bits *x, int64_t ldx, const half_bits *W, int64_t
     e.logits = logits; e.pval = part_val; e.pidx = part_idx;
     const int tx = (int)((N + 255) / 256), tt = tx * (int)((T + 255) / 256);
     *nparts = tx;
-    const int padded = (tx + 7) / 8 * 8 * (tt / tx);                        // index space of the XCD-paired tile order (kernel: lm_bx)
-    gemm256_kernel<GEPI_LMHEAD><<<dim3((unsigned)g256_grid(padded)), dim3(512), 2 * G_BUF, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
-                                                                                           (int)N, (int)N, nullptr, e, tx, tt / tx, 0);
+    gemm256_kernel<GEPI_LMHEAD><<<dim3((unsigned)g256_grid(tt)), dim3(G_THREADS), 2 * G_BUF + 2048, s>>>((const half_t *)x, ldx, (const half_t *)W, (int)T, (int)K,
+                                                                                           (int)N, (int)N, nullptr, e, tx, tt / tx, g256_panel(tx));
     return g256_check("gemm256_lm_head");
 }
 
