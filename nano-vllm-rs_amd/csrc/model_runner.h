@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 #include <map>
 #include <vector>
+#include "host_copy.h"
 #include "sequence.h"
 #include "comm.h"
 #include "common.h"
@@ -96,6 +97,7 @@ struct nvr_model_runner {
     int set_p2p_fenced(bool on);           // switch the one-shot collectives' protocol (captured decode graphs hold the old one: dropped)
 
     ~nvr_model_runner();
+    nvr::HostCopy host_copy;                              // logits into a program's own memory
     int init();
     int execute(nvr_seq *const *seqs, size_t nseq, bool is_prefill, bool logits_asked = false);   // logits_asked: the caller reads the f32 logits of every row
     // a full (un-sharded) checkpoint tensor by its HF / reference name -> this rank's slice of the packed

@@ -175,12 +175,17 @@ nvr_block_manager_t *nvr_sched_block_manager(nvr_scheduler_t *sc) { return sc->i
 size_t nvr_sched_take_finished(nvr_scheduler_t *sc, nvr_seq_t **out, size_t cap) { return sc->impl.take_finished(out, cap); }
 
 // ------------------------------------------------------------------ ModelRunner
+// runners whose logits can be large have what copies them ready
+static int host_copy_for(nvr_model_runner &r) {
+    if ((size_t)r.max_seqs * r.Vl * sizeof(float) >= nvr::HostCopy::LEAST) NVR_HIP_CHECK(r.host_copy.prepare());
+    return NVR_OK;
+}
 nvr_model_runner_t *nvr_runner_create(const nvr_config *cfg, const nvr_model_config *mc) {
     NVR_GUARD_BEGIN
     if (nvr_config_validate(cfg) || nvr_config_runnable(cfg)) return nullptr;
     nvr_model_runner *r = new nvr_model_runner();
     r->cfg = *cfg; r->mc = *mc;
-    if (r->init() != NVR_OK) { delete r; return nullptr; }
+    if (r->init() != NVR_OK || host_copy_for(*r) != NVR_OK) { delete r; return nullptr; }
     return r;
     NVR_GUARD_END(nullptr)
 }
@@ -194,7 +199,7 @@ nvr_model_runner_t *nvr_runner_create_spec(const nvr_config *cfg, const nvr_mode
     r->cfg = *cfg;
     r->layered.reset(new nvr::LayeredModel());
     r->layered->spec = spec->layered;
-    if (r->init() != NVR_OK) { delete r; return nullptr; }
+    if (r->init() != NVR_OK || host_copy_for(*r) != NVR_OK) { delete r; return nullptr; }
     return r;
     NVR_GUARD_END(nullptr)
 }
@@ -230,7 +235,12 @@ int nvr_runner_copy_logits(nvr_model_runner_t *r, float *host_out, size_t rows) 
     NVR_HIP_CHECK(hipSetDevice(r->device));
     if (int rc = r->ensure_logits()) return rc;
     if (r->tp > 1) { if (int rc = r->comm.p2p_check_error(r->stream)) return rc; }
-    NVR_HIP_CHECK(hipMemcpyAsync(host_out, r->logits, rows * r->Vl * sizeof(float), hipMemcpyDeviceToHost, r->stream));
+    const size_t bytes = rows * r->Vl * sizeof(float);
+    if (r->host_copy.takes(host_out, bytes)) {
+        NVR_HIP_CHECK(r->host_copy.run(r->device, r->stream, host_out, r->logits, bytes));
+        return NVR_OK;
+    }
+    NVR_HIP_CHECK(hipMemcpyAsync(host_out, r->logits, bytes, hipMemcpyDeviceToHost, r->stream));
     NVR_HIP_CHECK(hipStreamSynchronize(r->stream));
     return NVR_OK;
 }
