@@ -19,7 +19,7 @@
 // What bounds it: power.  With operands of zeros a K-tile takes 1.05 us at 2.4 GHz however many CUs run (2520 clocks: 128 products of 17 and the ~120 other instructions of a wave, which nothing overlaps), with
 // random ones 1.07 us on 32 CUs and 1.45 on 256: the clock falls to what the part's power allows.  us, eight waves of 128 x 64 with 8 barriers a K-tile and results through LDS / so: 4096 x 12288 x 4096
 // (T K N) 294 / 281, 32768 x 3072 x 1024 + residual 183 / 162, 32768 x 2048 x 1024 113 / 101, 32768 x 1024 x 4096 231 / 221, gate and up of 3072 columns 362 / 347, of 12288 at 3062 x 4096 478 / 451,
-// qkv with RoPE and store 270 / 250, with head norms 299 / 280.  (One barrier a K-tile with all requests behind it: the same rate alone, but 15 % less where the operands come from memory.)
+// qkv with RoPE and store 273 / 257, with head norms 297 / 287.  (One barrier a K-tile with all requests behind it: the same rate alone, but 15 % less where the operands come from memory.)
 #include <cstdlib>
 #include "kernels.h"
 #include "device_utils.h"
@@ -63,20 +63,6 @@ __device__ __forceinline__ void g_dma(unsigned off, const char *base) { asm vola
 __device__ __forceinline__ void g_dma4(unsigned lds, const void *src) {
     unsigned keep;
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, off\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "s"(lds), "v"(src) : "memory");
-}
-
-// c += a . b (FIRST: c = a . b) with the accumulators held where they are: the 256 of a lane fill the accumulation registers, and hipcc, which gives every product a destination of its own, would
-// move them about (200 copies in a K-tile of 128 products).  Hazards that hipcc does not see behind inline asm: an accumulator is never written but by a product (a tile's first ones take no addend:
-// nothing has to be zeroed either), and G256_SETTLE stands in front of the first ordinary read.
-template <bool FIRST>
-__device__ __forceinline__ void g_mma(half8_t a, half8_t b, float4_t &c) {
-#ifdef NVR_BF16
-    if constexpr (FIRST) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
-    else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-#else
-    if constexpr (FIRST) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
-    else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-#endif
 }
 
 template <int EPI, int RD = 0, bool GRP = false>
@@ -172,7 +158,7 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
     // One phase: the 32 products of quadrant (A half HA, B half HB) of a K-tile, B's fragments outermost.  A product leaves its wave room for three instructions: the 8 fragments of the half-tile that
     // the phase brings into registers (F of READ_G, one behind every fourth product, or behind the products of the B fragment that they replace) and the four pieces of the half-tile that it
     // requests (two instructions each) go between them.  Own requests that the next phase reads have landed (all but the youngest five half-tiles), own reads of the phase before are back, barrier.
-#define G256_PHASE(HA_, HB_, F_, FH_, LANE_, READ_G_, RHT_, VM_, FIRST_)                                                                          \
+#define G256_PHASE(HA_, HB_, F_, FH_, LANE_, READ_G_, RHT_, VM_)                                                                          \
     _Pragma("unroll") for (int n = 0; n < 32; ++n) {                                                                                       \
         constexpr bool behind = (RHT_) == 1;                              /* phase 3 */                                                    \
         if (!behind && n % 3 == 0 && n < 24) read(F_[FH_], n / 3, FH_, LANE_, READ_G_);                                                    \
@@ -181,8 +167,7 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
         if (n % 8 == 4) aim(RHT_, n / 8, req_lds);                                                                                         \
         if (n % 8 == 5) request(RHT_, n / 8);                                                                                              \
         __builtin_amdgcn_sched_barrier(0);                                                                                                 \
-        if ((FIRST_) && !(n & 4)) g_mma<true>(fa[HA_][n & 3][0], fb[HB_][n >> 3][0], acc[HA_][n & 3][HB_][n >> 3]);                        \
-        else g_mma<false>(fa[HA_][n & 3][(n >> 2) & 1], fb[HB_][n >> 3][(n >> 2) & 1], acc[HA_][n & 3][HB_][n >> 3]);                      \
+        acc[HA_][n & 3][HB_][n >> 3] = mfma16(fa[HA_][n & 3][(n >> 2) & 1], fb[HB_][n >> 3][(n >> 2) & 1], acc[HA_][n & 3][HB_][n >> 3]);  \
         __builtin_amdgcn_sched_barrier(0);                                                                                                 \
     }                                                                                                                                      \
     if ((RHT_) == 1) { read(F_[FH_], 6, FH_, LANE_, READ_G_); read(F_[FH_], 7, FH_, LANE_, READ_G_); }                                     \
@@ -190,19 +175,16 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
     __builtin_amdgcn_s_waitcnt(((VM_) & 15) | 0x70 | ((RHT_) == 1 ? 2 << 8 : 0) | ((VM_) >> 4) << 14);                                     \
     __builtin_amdgcn_s_barrier();                                                                                                          \
     asm volatile("" ::: "memory");
-#define G256_KTILE(VM_, FIRST_)                                                                                                                    \
+#define G256_KTILE(VM_)                                                                                                                    \
     {                                                                                                                                      \
         const unsigned req_lds = lds_w + (unsigned)((g & 1) * G_BUF);                                                                      \
-        G256_PHASE(0, 0, fb, 1, b_lane, g, 0, VM_, FIRST_)                                                                                         \
-        G256_PHASE(0, 1, fa, 1, a_lane, g, 2, VM_, FIRST_)                                                                                         \
-        G256_PHASE(1, 1, fa, 0, a_lane, g + 1, 3, VM_, FIRST_)                                                                                     \
-        G256_PHASE(1, 0, fb, 0, b_lane, g + 1, 1, VM_, FIRST_)                                                                                     \
+        G256_PHASE(0, 0, fb, 1, b_lane, g, 0, VM_)                                                                                         \
+        G256_PHASE(0, 1, fa, 1, a_lane, g, 2, VM_)                                                                                         \
+        G256_PHASE(1, 1, fa, 0, a_lane, g + 1, 3, VM_)                                                                                     \
+        G256_PHASE(1, 0, fb, 0, b_lane, g + 1, 1, VM_)                                                                                     \
         advance();                                                                                                                         \
         ++g;                                                                                                                               \
     }
-#define G256_SETTLE(A_, I_)                                               /* (wait states between a product and an ordinary read of its result, which hipcc does not count behind inline asm) */    \
-    asm volatile("s_nop 15\n\ts_nop 3" : "+a"(acc[A_][I_][0][0]), "+a"(acc[A_][I_][0][1]), "+a"(acc[A_][I_][0][2]), "+a"(acc[A_][I_][0][3]), "+a"(acc[A_][I_][1][0]), "+a"(acc[A_][I_][1][1]),    \
-                 "+a"(acc[A_][I_][1][2]), "+a"(acc[A_][I_][1][3]));
 
     const int KT = K / G_BK;
     Tile tile = tile_of(u);
@@ -239,12 +221,24 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
     int tile_no = 0;
     for (int g = 0;; ) {
         const bool have_next = u + step < u_end;
-        if (SLACK > 0 && whole) G256_KTILE(20 + SLACK, true)
-        else G256_KTILE(20, true)
-        for (int kt = 1; kt < KT; ++kt) G256_KTILE(20, false)
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[a][i][b][j] = (float4_t){0.f, 0.f, 0.f, 0.f};
+        // (in accumulation registers from here on: 256 is all there are, and any temporary among them has hipcc move accumulators about within the loop; a tile's first products without an addend need such)
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                asm volatile("" : "+a"(acc[a][i][0][0]), "+a"(acc[a][i][0][1]), "+a"(acc[a][i][0][2]), "+a"(acc[a][i][0][3]), "+a"(acc[a][i][1][0]), "+a"(acc[a][i][1][1]), "+a"(acc[a][i][1][2]), "+a"(acc[a][i][1][3]));
+        int kt = 0;
+        if (SLACK > 0 && whole) { G256_KTILE(20 + SLACK) ++kt; }
+        do G256_KTILE(20) while (++kt < KT);                              // (two K-tiles at least)
         whole = tile.by * 256 + 256 <= T;
-        G256_SETTLE(0, 0) G256_SETTLE(0, 1) G256_SETTLE(0, 2) G256_SETTLE(0, 3) G256_SETTLE(1, 0) G256_SETTLE(1, 1) G256_SETTLE(1, 2) G256_SETTLE(1, 3)
-
         // ---- epilogue of `tile`, straight from the accumulators: lane (r, q) has of token row m0 + hB*128 + wm*64 + j*16 + r the eight columns q*8 .. of every 32-column group wn*2 + p of either
         // A half (tiles 2p and 2p + 1).  No LDS, no barrier: the requests of the next tile's first two K-tiles are under way.
         {
@@ -254,6 +248,10 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
         asm volatile("" : "+v"(elane));
         const int r = elane & 15, q = elane >> 4;
         const int mrow = wm * 64 + r;                                     // + hB*128 + j*16
+        // (the accumulators of a token tile stay in accumulation registers up to here: hipcc would bring all 256 over in front of the epilogue, and spill)
+        auto hold = [&](int b, int j) {
+            asm volatile("" : "+a"(acc[0][0][b][j]), "+a"(acc[0][1][b][j]), "+a"(acc[0][2][b][j]), "+a"(acc[0][3][b][j]), "+a"(acc[1][0][b][j]), "+a"(acc[1][1][b][j]), "+a"(acc[1][2][b][j]), "+a"(acc[1][3][b][j]));
+        };
         auto eight = [&](int a, int p, int b, int j) {
             const float4_t lo = acc[a][2 * p][b][j], hi = acc[a][2 * p + 1][b][j];
             return (half8_t){(half_t)lo[0], (half_t)lo[1], (half_t)lo[2], (half_t)lo[3], (half_t)hi[0], (half_t)hi[1], (half_t)hi[2], (half_t)hi[3]};
@@ -272,6 +270,7 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int ml = b * 128 + mrow + j * 16, m = m0 + ml;
+                    hold(b, j);
                     float bv = -INFINITY; int bi = 0x7fffffff;
                     float *lrow = epi.logits + (int64_t)m * nv + n_base;
                     const int out = epi.logits && m < tv ? lim : 0;
@@ -383,9 +382,10 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
                 }
             } else {
 #pragma unroll
-                for (int t = 0; t < 8; ++t)
+                for (int t = 0; t < 8; ++t) {
 #pragma unroll
                     for (int p = 0; p < 2; ++p) leave(t, p, false, eight(0, p, t >> 2, t & 3), eight(1, p, t >> 2, t & 3));
+                }
             }
         } else {
             constexpr int NA = g_glu(EPI) ? 1 : 2;
@@ -409,6 +409,7 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
             for (int t = 0; t < 8; ++t) {
                 const int b = t >> 2, j = t & 3;
                 if (EPI == GEPI_RESID && t < 4) residual(t + 4);
+                hold(b, j);
                 const bool in = m0 + b * 128 + mrow + j * 16 < T;
                 half_t *yrow = yt + (int64_t)(b * 128 + j * 16) * ldy + lane_off;
 #pragma unroll
@@ -441,6 +442,7 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
                         } else o = eight(a, p, b, j);
                         if (in) *reinterpret_cast<half8_t *>(yrow + a * 128 + p * 32) = o;
                     }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
         }   // epilogue scope
@@ -452,7 +454,6 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                      // (requests behind the last tile: the LDS is given back only now)
 #undef G256_PHASE
 #undef G256_KTILE
-#undef G256_SETTLE
 }
 
 static int g256_prepare() {                                               // 128 KiB of dynamic LDS: opt-in once
