@@ -163,19 +163,23 @@ __device__ __forceinline__ float head_sum(float x) {
 // RMSNorm over a head of LPH * 16 columns held by LPH neighbouring lanes, lane j with columns j * 8 .. of either half (x1, x2; the norm's weights g1, g2).  The sums' pairs, divisions and roundings
 // of qknorm_rope_store_kernel, hence its bits.  x / rms: with y = 1 / rms rounded, q = x y and the residual r = x - q rms (exact), q + r y is the rounded quotient (Markstein, IBM Journal of
 // Research and Development 34, 1990, theorem 7.1) as long as nothing over- or underflows (r of numbers below 1e-30 may): 3 instructions a number instead of 10.
-// (head_scale: what is behind the sum of the squares ss)
-template <int LPH>
-__device__ __forceinline__ void head_scale(half8_t &x1, half8_t &x2, half8_t g1, half8_t g2, float ss, float eps) {
+// (head_scale: what is behind the sum of the squares ss, for N pairs of pieces of the head)
+template <int LPH, int N>
+__device__ __forceinline__ void head_scale(half8_t (&x1)[N], half8_t (&x2)[N], const half8_t (&g1)[N], const half8_t (&g2)[N], float ss, float eps) {
 #pragma clang fp contract(off)
     const float rms = sqrtf(ss / (float)(LPH * 16) + eps);
     if (rms > 1e-15f && rms < 1e15f) {
         const float y = __fdiv_rn(1.0f, rms);
         auto quotient = [&](float x) { const float q = x * y; return __fmaf_rn(__fmaf_rn(-q, rms, x), y, q); };
 #pragma unroll
-        for (int e = 0; e < 8; ++e) { x1[e] = to_half_rn(__fmul_rn(quotient((float)x1[e]), (float)g1[e])); x2[e] = to_half_rn(__fmul_rn(quotient((float)x2[e]), (float)g2[e])); }
+        for (int n = 0; n < N; ++n)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { x1[n][e] = to_half_rn(__fmul_rn(quotient((float)x1[n][e]), (float)g1[n][e])); x2[n][e] = to_half_rn(__fmul_rn(quotient((float)x2[n][e]), (float)g2[n][e])); }
     } else {                                                                  // (NaN, infinities, zeros without eps)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) { x1[e] = to_half_rn(__fmul_rn(__fdiv_rn((float)x1[e], rms), (float)g1[e])); x2[e] = to_half_rn(__fmul_rn(__fdiv_rn((float)x2[e], rms), (float)g2[e])); }
+        for (int n = 0; n < N; ++n)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { x1[n][e] = to_half_rn(__fmul_rn(__fdiv_rn((float)x1[n][e], rms), (float)g1[n][e])); x2[n][e] = to_half_rn(__fmul_rn(__fdiv_rn((float)x2[n][e], rms), (float)g2[n][e])); }
     }
 }
 template <int LPH>
@@ -184,7 +188,10 @@ __device__ __forceinline__ void head_norm(half8_t &x1, half8_t &x2, half8_t g1, 
     float ss = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) { const float a = (float)x1[e], b = (float)x2[e], aa = a * a, bb = b * b, ab = aa + bb; ss = ss + ab; }
-    head_scale<LPH>(x1, x2, g1, g2, head_sum<LPH>(ss), eps);
+    half8_t a1[1] = {x1}, a2[1] = {x2};
+    const half8_t b1[1] = {g1}, b2[1] = {g2};
+    head_scale<LPH>(a1, a2, b1, b2, head_sum<LPH>(ss), eps);
+    x1 = a1[0]; x2 = a2[0];
 }
 
 // (xor-16 and xor-32 partner sums: below)
@@ -201,9 +208,7 @@ __device__ __forceinline__ void head_norm_pieces(half8_t (&x1)[2], half8_t (&x2)
         for (int e = 0; e < 8; ++e) { const float a = (float)x1[p][e], b = (float)x2[p][e], aa = a * a, bb = b * b, ab = aa + bb; ss = ss + ab; }
         sp[p] = ss;
     }
-    const float ss = xor16_partner_sum(xor32_partner_sum(sp[0] + sp[1]));
-#pragma unroll
-    for (int p = 0; p < 2; ++p) head_scale<8>(x1[p], x2[p], g1[p], g2[p], ss, eps);
+    head_scale<8>(x1, x2, g1, g2, xor16_partner_sum(xor32_partner_sum(sp[0] + sp[1])), eps);
 }
 
 // lane-wise butterflies across the 16-lane rows of a wave on the gfx950 lane-swap instructions (no LDS traffic):

@@ -19,7 +19,7 @@
 // What bounds it: power.  With operands of zeros a K-tile takes 1.05 us at 2.4 GHz however many CUs run (2520 clocks: 128 products of 17 and the ~120 other instructions of a wave, which nothing overlaps), with
 // random ones 1.07 us on 32 CUs and 1.45 on 256: the clock falls to what the part's power allows.  us, eight waves of 128 x 64 with 8 barriers a K-tile and results through LDS / so: 4096 x 12288 x 4096
 // (T K N) 294 / 281, 32768 x 3072 x 1024 + residual 183 / 162, 32768 x 2048 x 1024 113 / 101, 32768 x 1024 x 4096 231 / 221, gate and up of 3072 columns 362 / 347, of 12288 at 3062 x 4096 478 / 451,
-// qkv with RoPE and store 273 / 257, with head norms 297 / 287.  (One barrier a K-tile with all requests behind it: the same rate alone, but 15 % less where the operands come from memory.)
+// qkv with RoPE and store 265 / 245, with head norms 298 / 274, of 3815 rows 36.8 / 35.7.  (One barrier a K-tile with all requests behind it: the same rate alone, but 15 % less where the operands come from memory.)
 #include <cstdlib>
 #include "kernels.h"
 #include "device_utils.h"
@@ -158,14 +158,14 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
     // One phase: the 32 products of quadrant (A half HA, B half HB) of a K-tile, B's fragments outermost.  A product leaves its wave room for three instructions: the 8 fragments of the half-tile that
     // the phase brings into registers (F of READ_G, one behind every fourth product, or behind the products of the B fragment that they replace) and the four pieces of the half-tile that it
     // requests (two instructions each) go between them.  Own requests that the next phase reads have landed (all but the youngest five half-tiles), own reads of the phase before are back, barrier.
-#define G256_PHASE(HA_, HB_, F_, FH_, LANE_, READ_G_, RHT_, VM_)                                                                          \
+#define G256_PHASE(HA_, HB_, F_, FH_, LANE_, READ_G_, RHT_, VM_, REQ_)                                                                          \
     _Pragma("unroll") for (int n = 0; n < 32; ++n) {                                                                                       \
         constexpr bool behind = (RHT_) == 1;                              /* phase 3 */                                                    \
         if (!behind && n % 3 == 0 && n < 24) read(F_[FH_], n / 3, FH_, LANE_, READ_G_);                                                    \
         if (behind && n >= 8 && n % 8 == 0) { read(F_[FH_], n / 4 - 2, FH_, LANE_, READ_G_); }                                             \
         if (behind && n >= 8 && n % 8 == 1) { read(F_[FH_], n / 4 - 1, FH_, LANE_, READ_G_); }                                             \
-        if (n % 8 == 4) aim(RHT_, n / 8, req_lds);                                                                                         \
-        if (n % 8 == 5) request(RHT_, n / 8);                                                                                              \
+        if ((REQ_) && n % 8 == 4) aim(RHT_, n / 8, req_lds);                                                                               \
+        if ((REQ_) && n % 8 == 5) request(RHT_, n / 8);                                                                                              \
         __builtin_amdgcn_sched_barrier(0);                                                                                                 \
         acc[HA_][n & 3][HB_][n >> 3] = mfma16(fa[HA_][n & 3][(n >> 2) & 1], fb[HB_][n >> 3][(n >> 2) & 1], acc[HA_][n & 3][HB_][n >> 3]);  \
         __builtin_amdgcn_sched_barrier(0);                                                                                                 \
@@ -175,14 +175,15 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
     __builtin_amdgcn_s_waitcnt(((VM_) & 15) | 0x70 | ((RHT_) == 1 ? 2 << 8 : 0) | ((VM_) >> 4) << 14);                                     \
     __builtin_amdgcn_s_barrier();                                                                                                          \
     asm volatile("" ::: "memory");
-#define G256_KTILE(VM_)                                                                                                                    \
+#define G256_KTILE(V0_, V1_, V2_, V3_, REQ_)                                                                                                \
     {                                                                                                                                      \
         const unsigned req_lds = lds_w + (unsigned)((g & 1) * G_BUF);                                                                      \
-        G256_PHASE(0, 0, fb, 1, b_lane, g, 0, VM_)                                                                                         \
-        G256_PHASE(0, 1, fa, 1, a_lane, g, 2, VM_)                                                                                         \
-        G256_PHASE(1, 1, fa, 0, a_lane, g + 1, 3, VM_)                                                                                     \
-        G256_PHASE(1, 0, fb, 0, b_lane, g + 1, 1, VM_)                                                                                     \
-        advance();                                                                                                                         \
+        (void)req_lds;                                                                                                                     \
+        G256_PHASE(0, 0, fb, 1, b_lane, g, 0, V0_, REQ_)                                                                                   \
+        G256_PHASE(0, 1, fa, 1, a_lane, g, 2, V1_, REQ_)                                                                                   \
+        G256_PHASE(1, 1, fa, 0, a_lane, g + 1, 3, V2_, REQ_)                                                                               \
+        G256_PHASE(1, 0, fb, 0, b_lane, g + 1, 1, V3_, REQ_)                                                                               \
+        if (REQ_) advance();                                                                                                               \
         ++g;                                                                                                                               \
     }
 
@@ -194,7 +195,6 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
         if (++skt == KT) {
             skt = 0;
             if (su + step < u_end) { su += step; set_sources(tile_of(su)); }
-            else { pa0 -= 2 * (int64_t)K; pa1 -= 2 * (int64_t)K; pb -= 2 * (int64_t)K; }      // (nothing left: the last tile's first K-tiles again, which nobody reads)
         }
     };
     set_sources(tile);
@@ -235,9 +235,14 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 asm volatile("" : "+a"(acc[a][i][0][0]), "+a"(acc[a][i][0][1]), "+a"(acc[a][i][0][2]), "+a"(acc[a][i][0][3]), "+a"(acc[a][i][1][0]), "+a"(acc[a][i][1][1]), "+a"(acc[a][i][1][2]), "+a"(acc[a][i][1][3]));
-        int kt = 0;
-        if (SLACK > 0 && whole) { G256_KTILE(20 + SLACK) ++kt; }
-        do G256_KTILE(20) while (++kt < KT);                              // (two K-tiles at least)
+        // (a workgroup's last two K-tiles request nothing: what is still under way is counted down)
+        int kt = have_next ? KT : KT - 2;
+        if (SLACK > 0 && whole && kt > 0) { G256_KTILE(20 + SLACK, 20 + SLACK, 20 + SLACK, 20 + SLACK, true) --kt; }
+        for (; kt > 0; --kt) G256_KTILE(20, 20, 20, 20, true)
+        if (!have_next) {
+            G256_KTILE(16, 12, 8, 4, false)
+            G256_KTILE(0, 0, 0, 0, false)
+        }
         whole = tile.by * 256 + 256 <= T;
         // ---- epilogue of `tile`, straight from the accumulators: lane (r, q) has of token row m0 + hB*128 + wm*64 + j*16 + r the eight columns q*8 .. of every 32-column group wn*2 + p of either
         // A half (tiles 2p and 2p + 1).  No LDS, no barrier: the requests of the next tile's first two K-tiles are under way.
@@ -353,7 +358,7 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
                             sn[t % AHEAD][p][hh] = *reinterpret_cast<const float4_t *>(epi.sin_t + at + p * 32 + hh * 4);
                         }
                 };
-                #pragma unroll
+#pragma unroll
                 for (int t = 0; t < AHEAD; ++t) sines(t);
 #pragma unroll
                 for (int t = 0; t < 8; ++t) {
@@ -451,7 +456,6 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
         u += step;
         tile = tile_of(u);
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                      // (requests behind the last tile: the LDS is given back only now)
 #undef G256_PHASE
 #undef G256_KTILE
 }
