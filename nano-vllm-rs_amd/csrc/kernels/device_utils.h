@@ -28,6 +28,24 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 
 constexpr int kWave = 64;
 
+// Workgroup `block` (its number in the launch: XCD block % 8) of those from `first` to `end`, a multiple of 8 of them, requests its share of its XCD's runs (Ahead)
+template <int THREADS, class A>
+__device__ __forceinline__ void request_ahead(const A &a, unsigned block, unsigned first, unsigned end) {
+    const unsigned xcd = block & 7, per = (end - first) >> 3, unit = (unsigned)a.unit;
+    const unsigned total = a.units > (int)xcd ? ((unsigned)a.units - xcd + 7) / 8 * unit : 0;      // pieces of this XCD's units
+    const float4_t *p = reinterpret_cast<const float4_t *>(a.w);
+    for (unsigned f = ((block - first) >> 3) * (8 * THREADS) + threadIdx.x; f < total; f += per * (8 * THREADS)) {
+        float4_t v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const unsigned c = min(f + e * THREADS, total - 1), u = c / unit;
+            v[e] = p[(uint64_t)(u * 8 + xcd) * unit + (c - u * unit)];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) asm volatile("" : : "v"(v[e]));
+    }
+}
+
 // D = A(16 x 32) . B(32 x 16) + C on the matrix cores, f32 accumulate (v_mfma_f32_16x16x32_f16 / _bf16)
 __device__ __forceinline__ float4_t mfma16(half8_t a, half8_t b, float4_t c) {
 #ifdef NVR_BF16

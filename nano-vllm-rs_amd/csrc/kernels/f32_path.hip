@@ -857,12 +857,20 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnArgsF a, int paged) 
 // 2002 / 3000 / 4922 now); prompts of 128 rows 38 / 19, 509 268 / 129, 1024 873 / 401
 // PAGED 2: pages of a power of two tokens (1 << shift): a shift and a mask per key where the general form divides twice, some 40 instructions each in front of every request
 // (one sequence of 150 keys 7.4 -> 7.0 us a launch)
+// The memory is idle meanwhile, and most CUs: AHEAD_WGS workgroups behind the rows' own bring weights of the launches behind this one (a.ahead) into the L2 caches.  A launch that reads 4 / 8 / 12 / 24 MB
+// from there takes 1.8 us whatever their number, 2.4 / 3.0 / 3.7 / 5.7 from HBM, and from another XCD's L2 what it takes from HBM.
+constexpr int AHEAD_WGS = 96;
 template <int NF, int NW, int PAGED>
 __global__ __launch_bounds__(64 * NW) void attention_rows_kernel(AttnArgsF a, int shift) {
     constexpr int D = 64 * NF, KB = NF <= 2 ? 4 : 2;                     // keys a group requests at a time
     constexpr int STEP = 16, ROUND = KB * STEP, NEXT = NW == 8 ? 2 * ROUND : ROUND;   // groups of four waves; keys of their round; from a wave's round to its next one
     __shared__ __attribute__((aligned(16))) float part[8][D];
     __shared__ float pm[8], pl[8];
+    if (blockIdx.y >= (unsigned)a.H) {                                   // behind the query rows' workgroups
+        const unsigned block = blockIdx.x + gridDim.x * blockIdx.y, first = gridDim.x * a.H, end = first + ((gridDim.x * gridDim.y - first) & ~7u);
+        if (block < end) { request_ahead<64 * NW>(a.ahead[0], block, first, end); request_ahead<64 * NW>(a.ahead[1], block, first, end); }
+        return;
+    }
     const int t = blockIdx.x, hd = blockIdx.y, g = hd / (a.H / a.KVH);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, group = (wave & 3) * 4 + (lane >> 4);
     const int first = NW == 8 ? (wave >> 2) * ROUND : 0;                 // the wave's first round
@@ -991,12 +999,13 @@ int attention(const AttnArgsF &a, bool paged, hipStream_t s) {
     if (a.D > 256 || a.D % 4) return nvr::fail(NVR_ERR_UNSUPPORTED, "f32 attention: head_dim %d (multiples of 4 up to 256)", a.D);
     const size_t lds = ((size_t)a.max_ctx + 5 * (size_t)a.D + 8) * 4;
     if (lds > 160 * 1024) return nvr::fail(NVR_ERR_UNSUPPORTED, "f32 attention: context %d does not fit the score buffer (%zu bytes of LDS)", a.max_ctx, lds);
-    const dim3 grid((unsigned)a.nq, (unsigned)a.H);
+    dim3 grid((unsigned)a.nq, (unsigned)a.H);
     // rows in 16-byte pieces: a multiple of 16 of them per head, everything aligned to them; eight waves share a query row's keys while there are less than two rows of workgroups per CU (eight
     // waves in place of four cost a step of 64 prompt rows 2.76 against 2.61 ms, four in place of eight a sequence of 4096 keys 3.62 against 3.04); the same bits either way
     const bool pieces = a.D % 64 == 0 && a.ldq % 4 == 0 && (paged || a.ldkv % 4 == 0) && (((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) & 15) == 0;
     if (pieces) {
         const bool few = (int64_t)a.nq * a.H < 512;
+        if (a.ahead[0].units || a.ahead[1].units) grid.y += (AHEAD_WGS + a.nq - 1) / a.nq;
         const int shift = paged && (a.block_size & (a.block_size - 1)) == 0 ? __builtin_ctz((unsigned)a.block_size) : -1;
 #define NVR_ARW(NF_, NW_) do { if (shift >= 0) attention_rows_kernel<NF_, NW_, 2><<<grid, dim3(64 * NW_), 0, s>>>(a, shift); \
                                else if (paged) attention_rows_kernel<NF_, NW_, 1><<<grid, dim3(64 * NW_), 0, s>>>(a, 0); \

@@ -17,6 +17,10 @@ constexpr int LM_HEAD_MAX_PARTS = 2048;
 
 struct TpArgmaxRec { float val; int32_t pad; int64_t idx; };           // 16 B: a rank's (max, global arg-max) of one row
 
+// Weights that launches behind this one read: `units` runs of `unit` pieces of 16 bytes, run u by workgroups of XCD u % 8.  Workgroups behind a launch's own may bring them into those XCDs' L2 caches
+// (device_utils.h: request_ahead), which keep them from launch to launch.
+struct Ahead { const void *w; int32_t units, unit; };
+
 // the input of a product that forms RMSNorm(h_in + sum of S slabs, `stride` elements apart) * w itself (linear.hip: NORM); h_out receives the new residual rows
 struct NormIn { const half_bits *h_in; const float *slabs; int64_t stride; int32_t S; const half_bits *w; float eps; half_bits *h_out; };
 
@@ -97,6 +101,7 @@ struct AttnArgsF {
     const int32_t *ctx_lens, *seq_of_q, *kv_base, *block_tables; int32_t max_blocks, block_size;
     int32_t nq, H, KVH, D; float scale; int32_t max_ctx;
     float *out;                                   // [nq, H, D]
+    Ahead ahead[2];                               // brought into the L2 caches beside the attention (units 0: nothing)
 };
 
 }}  // namespace nvr::kt

@@ -316,6 +316,18 @@ int nvr_model_runner::row_parallel_norm_f32(int64_t T, const float *wn, int64_t 
     return NVR_OK;
 }
 
+// What a decode step's attention brings into the L2 caches (AttnArgsF::ahead) for the two launches behind it: the output product's rows and the gate half of the next one's, four rows a workgroup of the
+// GEMVs.  While both are sure to be there when they are read: 24 of the caches' 32 MiB, keys and values of 10 MiB.  Qwen3-0.6B, us a step, without / so: one sequence of 20 / 500 / 1000 / 2000 keys
+// 809 1067 1322 1808 / 797 1039 1315 1821, two of 150 / 1000 1007 1481 / 966 1486, four of 150 / 500 1203 1431 / 1185 1440, eight of 60 / 150 / 300 1673 1728 1843 / 1671 1707 1838; a request of 128 tokens and
+// its 48 answers 43.7 / 41.7 ms, the output product's rows alone 42.5.  What launches without idle memory bring takes them longer than it saves behind them: the down projection's rows on the gated
+// unit and the next layer's on the down projection + 2.5 ms; the 16-bit steps' weights on the norms in front of them (32 sequences of 1024 keys 1436 / 1553, 4 MiB of them 1452).
+void nvr_model_runner::ahead_f32(nvr::kt::AttnArgsF &a, const Layer &w) const {
+    const int64_t o = Hd * H * D * 4, gate = I * Hd * 4, most = 24ll << 20;
+    if (Hd % 4 || I % 4 || o > most || (int64_t)a.nq * a.max_ctx * KVH * D * 8 > 10ll << 20) return;
+    a.ahead[0] = {w.o, (int32_t)(Hd / 4), (int32_t)(H * D)};
+    if (o + gate <= most) a.ahead[1] = {w.gate_up, (int32_t)(I / 4), (int32_t)Hd};
+}
+
 // the f32 graph (Qwen3Model::forward, qwen3.rs:487-505; layer wiring :372-392): one launch per op, eager
 int nvr_model_runner::forward_f32(int64_t T, int64_t B, bool is_prefill, int64_t max_ctx) {
     namespace kf = nvr::kf;
@@ -355,6 +367,7 @@ int nvr_model_runner::forward_f32(int64_t T, int64_t B, bool is_prefill, int64_t
             a.k = F(k_cache(l)); a.v = F(v_cache(l)); a.block_tables = dd_bt; a.max_blocks = (int32_t)max_blocks_per_seq; a.block_size = (int32_t)block_size;
             if (is_prefill) a.seq_of_q = d_kvbase;
         }
+        if (ride && !is_prefill) ahead_f32(a, w);
         RC(kf::attention(a, paged, st));
         const bool cut = !ride && !comm.active() && tp == 1 && !mc.use_bias;
         int64_t S;

@@ -147,6 +147,7 @@ private:
     int forward_f32(int64_t T, int64_t B, bool is_prefill, int64_t max_ctx);
     int64_t context_bucket(size_t nseq, int64_t max_ctx) const;
     int row_parallel_norm_f32(int64_t T, const float *wn, int64_t parts = 1);
+    void ahead_f32(nvr::kt::AttnArgsF &a, const Layer &w) const;
     int row_parallel_f32(const float *x, int64_t K, const float *W, const float *bias, int64_t T, bool cut, int64_t *parts);
     float *f32_h2 = nullptr;                             // float32, one rank: second residual-stream buffer [8][hidden] of the decode-sized steps whose add + norm
                                                          // rides on the consumer GEMV (the workgroups of that launch still read the first while one of them writes)

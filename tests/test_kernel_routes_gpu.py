@@ -1037,6 +1037,38 @@ def test_float32_decode_rows_form_their_norm_from_columns_in_registers(hidden):
             assert ta == tb and np.array_equal(la, lb)
 
 
+@pytest.mark.parametrize("hidden,inter,kv,dim,rows,length", [(16, 20, 1, 64, 1, 9), (28, 36, 1, 128, 3, 9),      # less than one run of four rows per XCD, and seven or nine of them
+                                                             (64, 30, 1, 64, 8, 5),                            # columns that are no multiple of four
+                                                             (1024, 3072, 4, 128, 1, 40), (1024, 1028, 2, 192, 7, 20),
+                                                             (2048, 4096, 1, 256, 2, 12),                      # the gate half does not fit beside the output product's rows
+                                                             (64, 64, 2, 256, 6, 420)])                        # keys and values that leave the caches no room
+def test_float32_decode_attention_brings_weights_into_the_caches(hidden, inter, kv, dim, rows, length):
+    """float32 decode steps whose attention launch holds workgroups that request the next products' weights: the runner that keeps the launches apart, which brings nothing, bit for bit (the requests
+    leave nothing behind), with and without graphs."""
+    import os
+    model = nvr.ModelConfig(vocab_size=400, hidden_size=hidden, intermediate_size=inter, num_hidden_layers=2, num_attention_heads=2 * kv, num_key_value_heads=kv, head_dim=dim,
+                            max_position_embeddings=512, tie_word_embeddings=1, seed=hidden)
+    got = []
+    for fused, eager in (("0", 0), ("1", 0), ("1", 1)):
+        os.environ["NVR_F32_FUSED_NORM"] = fused
+        try:
+            eng = nvr.LLMEngine(nvr.Config(skip_block_size_check=1, dtype="float32", enforce_eager=eager, max_num_seqs=rows, max_num_batched_tokens=4096, max_model_len=480, kvcache_block_size=16,
+                                           num_kvcache_blocks=30 * rows), model)
+        finally:
+            os.environ.pop("NVR_F32_FUSED_NORM", None)
+        for i in range(rows):
+            eng.add_request(nvr.synthetic_tokens(length + i, 5, i, 400), nvr.SamplingParams(temperature=0.0, max_tokens=4, ignore_eos=True))
+        out = []
+        while not eng.is_finished():
+            rec = eng.step()
+            out.append((rec["tokens"], eng.model_runner.logits(rec["num_seqs"]).copy().view(np.uint32)))
+        got.append(out)
+    for other in got[1:]:
+        assert len(other) == len(got[0]) >= 4
+        for (ta, la), (tb, lb) in zip(got[0], other):
+            assert ta == tb and np.array_equal(la, lb)
+
+
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("hidden,qk_norm", [(256, False), (768, True), (1024, False), (1280, False)])
 def test_decode_steps_of_one_to_five_rows(hidden, qk_norm, dtype):
