@@ -46,8 +46,14 @@ struct FlashParams {
     int32_t window, keep_first;                  // PEN and DIFF instantiations: > 0, a query sees only the keys less than `window` positions back (and the first keep_first keys)
     const float *gate_bias; float softcap; int32_t chunk;   // GATE instantiations (FlashArgs): sigmoid weights with a bias per head, capped scores, chunks of positions
     const float *lambda; float out_scale, eps; const half_t *head_gate; int64_t ldhg;   // DIFF instantiations (FlashArgs)
+    int32_t ntiles; Ahead ahead;                 // flash_plain_kernel: tiles, behind whose workgroups others bring weights into the L2 caches
 };
 
+
+// Steps whose tiles leave AHEAD_WGS and more of the CUs idle: that many workgroups bring FlashArgs::ahead into the L2 caches meanwhile.  Qwen3-0.6B in bfloat16, its gated unit's 12 MiB, us a step without / so:
+// 100 tokens 1252 / 1241, 160 1344 / 1316, 250 1488 / 1426, 320 1679 / 1620, 509 1846 / 1818, 640 2246 / 2216, 800 2505 / 2432, 1000 2716 / 2685, 1280 3294 / 3248, 1600 (for more tiles than that) 3685 / 3686;
+// 8 of 30 1365 / 1321; one of 4000, 3200 of them cached, 4228 / 4126.  48 workgroups: short prompts wait for them (8 of 60 1629 / 1685, 96 1592); 192 the same as 96 to 1 % slower.
+constexpr int AHEAD_WGS = 96;
 
 template <int D>
 __device__ __forceinline__ int v_swz(int row) { return D == 128 ? ((row & 7) << 1) : (((row >> 1) & 3) << 1); }
@@ -536,6 +542,7 @@ template <int G, bool PAGED, bool UB>
 __global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
     constexpr int D = 128, NT = 256, KT = 64, CPR = D / 8, PIECES = KT * CPR / NT, IMG = KT * D * 2;      // IMG: bytes of a K or V image of one step
     static_assert(FLASH_WAVES == 4, "four waves share a tile");
+    if (blockIdx.x >= (unsigned)(p.ntiles * p.KVH)) { request_ahead<NT>(p.ahead, blockIdx.x, p.ntiles * p.KVH, gridDim.x); return; }
     __shared__ __attribute__((aligned(16))) char smem[4 * IMG];           // K of even / odd steps, V of even / odd steps
     const int g = blockIdx.x % p.KVH;
     const FlashTile tile = p.tiles[blockIdx.x / p.KVH];
@@ -812,7 +819,9 @@ int flash_prefill(const FlashArgs &a, bool paged, hipStream_t s) {
     const int G = a.H / a.KVH;
     dim3 grid((unsigned)((int64_t)a.ntiles * a.KVH)), block(64 * FLASH_WAVES);
     const bool ub = paged && p.bs_shift >= 0 && a.block_size % NVR_FLASH_KT == 0;
+    p.ntiles = a.ntiles;
     if (a.D == 128 && !diff && !gate && !pen) {
+        if (a.ahead.units && grid.x <= 256 - AHEAD_WGS) { p.ahead = a.ahead; grid.x += AHEAD_WGS; }
 #define NVR_FLASH_PLAIN(GG)                                                                           \
     if (G == GG) {                                                                                    \
         if (ub) flash_plain_kernel<GG, true, true><<<grid, block, 0, s>>>(p);                         \

@@ -720,16 +720,24 @@ int gemm_tiled_resid(const half_bits *x, int64_t ldx, const half_bits *W, int64_
     tiled_launch<TEPI_RESID>((N + BN - 1) / BN, 1, x, ldx, W, Wt, T, K, N, N, (half_t *)h, TileEpi{}, s);
     return tiled_check("gemm_tiled_resid");
 }
+// 96-row tiles when they put a workgroup on (nearly) every CU where the 128-row tiles leave a quarter of them idle (T = 512, I = 3072: 256 against 192; T = 321..384: 192 against 144)
+static bool on_96_rows(int64_t T, int64_t I) {
+    const int64_t ty = (T + BM - 1) / BM, w128 = (I / 64) * ty, w96 = (I / 48) * ty;
+    return I % 48 == 0 && tiled_mt(T, I / 64) == 4 && w96 <= 256 && w96 > w128 && w128 * 8 <= w96 * 7;
+}
+// the weights of gemm_tiled_silu_mul by the XCD that reads them: workgroup x of the 96-row tiles takes 48 gate and 48 up rows; of the others an XCD takes an eighth of both where that is a strip
+Ahead gemm_tiled_silu_ahead(const half_bits *W, int64_t T, int64_t K, int64_t I) {
+    if (on_96_rows(T, I)) return (I / 48) % 8 ? Ahead{} : Ahead{W, (int32_t)(2 * I / 48), (int32_t)(48 * K / 8)};
+    const int64_t nx = I / 64, mt = tiled_mt(T, nx);
+    if (nx % 8 || tile_map(nx, (T + 32 * mt - 1) / (32 * mt), 1, 32 * mt).width * 8 != nx) return {};
+    return {W, 16, (int32_t)(I / 8 * K / 8)};
+}
 int gemm_tiled_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out, hipStream_t s, bool gelu, const half_bits *Wt) {
     if (!gemm_tiled_ok(T, K, I, ldx) || I % 64) return nvr::fail(NVR_ERR_UNSUPPORTED, "gemm_tiled_silu_mul: T=%ld K=%ld I=%ld", (long)T, (long)K, (long)I);
     if (int rc = gemm_tiled_prepare()) return rc;
-    {   // 96-row tiles when they put a workgroup on (nearly) every CU where the 128-row tiles leave a quarter of them idle (T = 512, I = 3072: 256 against 192;
-        // T = 321..384: 192 against 144)
-        const int64_t ty = (T + BM - 1) / BM, w128 = (I / 64) * ty, w96 = (I / 48) * ty;
-        if (!gelu && I % 48 == 0 && tiled_mt(T, I / 64) == 4 && w96 <= 256 && w96 > w128 && w128 * 8 <= w96 * 7) {
-            gemm_tiled_silu96_kernel<<<dim3((unsigned)(I / 48), (unsigned)ty), dim3(256), RING96 * S96_BUF, s>>>((const half_t *)x, ldx, (const half_t *)(Wt ? Wt : W), (int)T, (int)K, (int)I, (half_t *)out, Wt != nullptr);
-            return tiled_check("gemm_tiled_silu_mul (96-row tiles)");
-        }
+    if (!gelu && on_96_rows(T, I)) {
+        gemm_tiled_silu96_kernel<<<dim3((unsigned)(I / 48), (unsigned)((T + BM - 1) / BM)), dim3(256), RING96 * S96_BUF, s>>>((const half_t *)x, ldx, (const half_t *)(Wt ? Wt : W), (int)T, (int)K, (int)I, (half_t *)out, Wt != nullptr);
+        return tiled_check("gemm_tiled_silu_mul (96-row tiles)");
     }
     TileEpi e{}; e.gelu = gelu ? 1 : 0;
     tiled_launch<TEPI_SILU>(I / 64, 1, x, ldx, W, Wt, T, K, I, 2 * I, (half_t *)out, e, s);

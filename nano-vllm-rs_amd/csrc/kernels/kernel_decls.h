@@ -76,6 +76,8 @@ int add_rmsnorm_slabs(half_bits *h, const float *slabs, int64_t S, const half_bi
 // qkv -> RoPE(q,k) + KV store, W [(H+2KVH)D, K] -> qkv [T,(H+2KVH)D] (roped q,k; v) and cache rows at slots
 int linear_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I,
                     half_bits *out, hipStream_t s, const half_bits *Wt = nullptr);
+// linear_silu_mul's weights (Wt where its kernel reads those) by the XCD that reads them, where they fit into the L2 caches and one XCD reads each of them; else nothing
+Ahead linear_silu_ahead(const half_bits *W, int64_t T, int64_t K, int64_t I, const half_bits *Wt = nullptr);
 // y = gelu(x . W^T), the form with the error function, where the kernel of this shape has it in its epilogue (*applied), else y = x . W^T
 int linear_gelu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *y, bool *applied, hipStream_t s);
 // gate / up products with gelu (tanh form) in silu's place
@@ -128,6 +130,7 @@ int gemm_tiled_lm_head(const half_bits *x, int64_t ldx, const half_bits *W, int6
 bool gemm_tiled_ok(int64_t T, int64_t K, int64_t N, int64_t ldx);
 int gemm_tiled(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *y, hipStream_t s, const half_bits *Wt = nullptr);
 int gemm_tiled_resid(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t N, half_bits *h, hipStream_t s, const half_bits *Wt = nullptr);   // h <- h + x.W^T, the product rounded first
+Ahead gemm_tiled_silu_ahead(const half_bits *W, int64_t T, int64_t K, int64_t I);
 int gemm_tiled_silu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, half_bits *out,
                         hipStream_t s, bool gelu = false, const half_bits *Wt = nullptr);
 int gemm_tiled_clamped_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I, float limit, float alpha, half_bits *out, int64_t ldo, hipStream_t s);

@@ -71,6 +71,7 @@ struct QkNorm { const half_bits *q_w, *k_w; float eps; };
 struct FlashTile { int32_t q_row0, nq, pos0, kv_ref; };   // first q row, #queries, absolute position of the first query,
                                                           // contiguous: first key row of the sequence / paged: block-table row
 struct FlashArgs {
+    Ahead ahead;                                           // brought into the L2 caches beside the attention where it leaves CUs idle (units 0: nothing)
     const half_bits *q; int64_t ldq;
     const half_bits *k, *v; int64_t ldkv;                  // contiguous rows (stride ldkv) or paged caches [NB, bs, KVH, D]
     const int32_t *block_tables; int32_t max_blocks, block_size;

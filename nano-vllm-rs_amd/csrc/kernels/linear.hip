@@ -685,6 +685,18 @@ int linear_splitk(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T
     return launch_check("linear_splitk");
 }
 
+// 56 rows and more of weights that the large-weight kernel does not take: the two blocks of 32 rows each read x for every 16 columns.  us of 56 / 64 rows, blocks | tiles: K = 512, I = 2304
+// 5.2 5.4 | 5.3 5.9, 3840 6.1 6.3 | 6.2 6.3, 4864 7.6 7.8 | 6.4 6.4; K = 768, I = 2304 7.0 7.4 | 7.0 7.4, 3840 8.1 8.5 | 7.5 7.6; K = 1024, I = 2304 8.3 8.7 | 8.3 8.4, 3072 8.9 9.3 | 8.3 8.4,
+// 4864 11.9 12.5 | 9.0 9.2; K = 2560, I = 3072 20.4 21.3 | 17.1 17.5, 4864 29.5 31.1 | 19.7 19.9
+static bool glu_on_tiles(int64_t T, int64_t K, int64_t I, int64_t ldx) {
+    return gemm_tiled_ok(T, K, I, ldx) && I % 64 == 0 && (!stream_preferred(T, 2 * I) || (T >= 56 && T * I > (K >= 768 ? 128 : 256) * 1024 && !linear_stream_silu_ok(T, K, I, ldx)));
+}
+Ahead linear_silu_ahead(const half_bits *W, int64_t T, int64_t K, int64_t I, const half_bits *Wt) {
+    if (2 * I * K * 2 > 24ll << 20 || K % 32 || I % 128) return {};
+    if (gemm256_silu_ok(T, K, I, K) && rows_on_256(T, K, 2 * I) > 0) return {};
+    return glu_on_tiles(T, K, I, K) ? gemm_tiled_silu_ahead(Wt ? Wt : W, T, K, I) : Ahead{};
+}
+
 // gate_up GEMM + SiluAndMul: W [2I, K] (gate rows then up rows), out [T, I]
 static int linear_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64_t T, int64_t K, int64_t I,
                       half_bits *out, hipStream_t s, const half_bits *Wt, bool gelu) {
@@ -695,10 +707,7 @@ static int linear_glu(const half_bits *x, int64_t ldx, const half_bits *W, int64
         if (int rc = gelu ? gemm256_gelu_mul(x, ldx, W, r, K, I, out, s) : gemm256_silu_mul(x, ldx, W, r, K, I, out, s)) return rc;
         return r == T ? 0 : gemm_tiled_silu_mul(x + r * ldx, ldx, W, T - r, K, I, out + r * I, s, gelu, Wt);
     }
-    // (56 rows and more of weights that the large-weight kernel does not take: the two blocks of 32 rows each read x for every 16 columns.  us of 56 / 64 rows, blocks | tiles: K = 512, I = 2304
-    // 5.2 5.4 | 5.3 5.9, 3840 6.1 6.3 | 6.2 6.3, 4864 7.6 7.8 | 6.4 6.4; K = 768, I = 2304 7.0 7.4 | 7.0 7.4, 3840 8.1 8.5 | 7.5 7.6; K = 1024, I = 2304 8.3 8.7 | 8.3 8.4, 3072 8.9 9.3 | 8.3 8.4,
-    // 4864 11.9 12.5 | 9.0 9.2; K = 2560, I = 3072 20.4 21.3 | 17.1 17.5, 4864 29.5 31.1 | 19.7 19.9)
-    if (gemm_tiled_ok(T, K, I, ldx) && I % 64 == 0 && (!stream_preferred(T, 2 * I) || (T >= 56 && T * I > (K >= 768 ? 128 : 256) * 1024 && !linear_stream_silu_ok(T, K, I, ldx)))) return gemm_tiled_silu_mul(x, ldx, W, T, K, I, out, s, gelu, Wt);
+    if (glu_on_tiles(T, K, I, ldx)) return gemm_tiled_silu_mul(x, ldx, W, T, K, I, out, s, gelu, Wt);
     if (linear_stream_silu_ok(T, K, I, ldx)) return linear_stream_silu_mul(x, ldx, W, T, K, I, out, s, Wt, gelu);              // large weights
     const half_t *xx = (const half_t *)x, *ww = (const half_t *)(Wt ? Wt : W);
     LinEpi e{};

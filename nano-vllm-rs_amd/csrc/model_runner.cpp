@@ -934,6 +934,7 @@ int nvr_model_runner::forward(int64_t T, int64_t B, bool is_prefill, int64_t max
             } else { f.k = qkv + H * D; f.v = qkv + (H + KVH) * D; f.ldkv = QKV; }
             f.tiles = (const k::FlashTile *)(in_dev + off_tiles); f.ntiles = (int32_t)n_tiles;
             f.H = (int32_t)H; f.KVH = (int32_t)KVH; f.D = (int32_t)D; f.scale = scale; f.out = attn;
+            if (!comm.active() && !mc.use_bias) f.ahead = KD(linear_silu_ahead(w.gate_up, T, Hd, I, tl ? w.gate_up_t : nullptr));
             RC(KD(flash_prefill(f, prefill_paged, st)));
         } else if (is_prefill) {                                     // head shapes outside the MFMA kernel: row kernel
             a.k = qkv + H * D; a.v = qkv + (H + KVH) * D; a.ldkv = QKV; a.kv_base = d_kvbase; a.workspace = nullptr;

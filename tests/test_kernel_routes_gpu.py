@@ -1070,6 +1070,21 @@ def test_float32_decode_attention_brings_weights_into_the_caches(hidden, inter, 
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("inter,lengths", [(3072, [65]), (3072, [330]),            # strips of an eighth; tiles of 96 rows
+                                           (2304, [400]), (2112, [130, 7]),        # 48 of them in a row; columns in no eighths, which bring nothing
+                                           (512, [200]), (512, [1216]), (512, [1217])])   # 152 workgroups of attention, and 160
+def test_prompt_attention_brings_weights_into_the_caches(inter, lengths, dtype):
+    """Prompt steps whose attention launch holds workgroups that request the gated unit's weights, at the ends of the rule: the prompts' logits and those of the token behind them against the oracle, at the
+    engine's tolerance for the type."""
+    from oracle import model_oracle as mo
+    from test_engine_gpu import _run_pair
+    mcfg = mo.small(hidden_size=256, num_hidden_layers=2, intermediate_size=inter, head_dim=128, num_attention_heads=16, num_key_value_heads=8, max_position_embeddings=2048, seed=inter, init_std=0.02)
+    ecfg = dict(max_num_seqs=2, max_num_batched_tokens=1280, max_model_len=1280, kvcache_block_size=16, num_kvcache_blocks=160)
+    prompts = [oracle.fill_tokens(n, 3, i, mcfg.vocab_size).tolist() for i, n in enumerate(lengths)]
+    _run_pair(mcfg, ecfg, prompts, [dict(temperature=0.0, max_tokens=2, ignore_eos=True) for _ in lengths], dtype=dtype)
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("hidden,qk_norm", [(256, False), (768, True), (1024, False), (1280, False)])
 def test_decode_steps_of_one_to_five_rows(hidden, qk_norm, dtype):
     """A batch that shrinks from five rows to one: the add + norm formed by the consuming products (up to four rows of 1024 numbers, three of 1280; a wave count of row pieces that is and is not a
