@@ -46,13 +46,16 @@ struct FlashParams {
     int32_t window, keep_first;                  // PEN and DIFF instantiations: > 0, a query sees only the keys less than `window` positions back (and the first keep_first keys)
     const float *gate_bias; float softcap; int32_t chunk;   // GATE instantiations (FlashArgs): sigmoid weights with a bias per head, capped scores, chunks of positions
     const float *lambda; float out_scale, eps; const half_t *head_gate; int64_t ldhg;   // DIFF instantiations (FlashArgs)
-    int32_t ntiles; Ahead ahead;                 // flash_plain_kernel: tiles, behind whose workgroups others bring weights into the L2 caches
 };
+struct FlashParamsAhead : FlashParams { int32_t ntiles; Ahead ahead; };      // AHEAD instantiations of flash_plain_kernel
+template <bool AHEAD> struct FlashParamsOf { using type = FlashParams; };
+template <> struct FlashParamsOf<true> { using type = FlashParamsAhead; };
 
 
 // Steps whose tiles leave AHEAD_WGS and more of the CUs idle: that many workgroups bring FlashArgs::ahead into the L2 caches meanwhile.  Qwen3-0.6B in bfloat16, its gated unit's 12 MiB, us a step without / so:
 // 100 tokens 1252 / 1241, 160 1344 / 1316, 250 1488 / 1426, 320 1679 / 1620, 509 1846 / 1818, 640 2246 / 2216, 800 2505 / 2432, 1000 2716 / 2685, 1280 3294 / 3248, 1600 (for more tiles than that) 3685 / 3686;
 // 8 of 30 1365 / 1321; one of 4000, 3200 of them cached, 4228 / 4126.  48 workgroups: short prompts wait for them (8 of 60 1629 / 1685, 96 1592); 192 the same as 96 to 1 % slower.
+// (Instances of their own: the branch in the others cost steps without it 0.7 % of the launch, 181.0 / 182.3 us at 3815 rows behind 11400 cached.)
 constexpr int AHEAD_WGS = 96;
 
 template <int D>
@@ -538,11 +541,12 @@ __device__ __forceinline__ void sched_pattern() {
         __builtin_amdgcn_sched_group_barrier(0x2, VALU, 0);
     }
 }
-template <int G, bool PAGED, bool UB>
-__global__ __launch_bounds__(256, 2) void flash_plain_kernel(FlashParams p) {
+template <int G, bool PAGED, bool UB, bool AHEAD = false>
+__global__ __launch_bounds__(256, 2) void flash_plain_kernel(typename FlashParamsOf<AHEAD>::type own) {
+    const FlashParams &p = own;
     constexpr int D = 128, NT = 256, KT = 64, CPR = D / 8, PIECES = KT * CPR / NT, IMG = KT * D * 2;      // IMG: bytes of a K or V image of one step
     static_assert(FLASH_WAVES == 4, "four waves share a tile");
-    if (blockIdx.x >= (unsigned)(p.ntiles * p.KVH)) { request_ahead<NT>(p.ahead, blockIdx.x, p.ntiles * p.KVH, gridDim.x); return; }
+    if constexpr (AHEAD) if (blockIdx.x >= (unsigned)(own.ntiles * p.KVH)) { request_ahead<NT>(own.ahead, blockIdx.x, own.ntiles * p.KVH, gridDim.x); return; }
     __shared__ __attribute__((aligned(16))) char smem[4 * IMG];           // K of even / odd steps, V of even / odd steps
     const int g = blockIdx.x % p.KVH;
     const FlashTile tile = p.tiles[blockIdx.x / p.KVH];
@@ -819,16 +823,21 @@ int flash_prefill(const FlashArgs &a, bool paged, hipStream_t s) {
     const int G = a.H / a.KVH;
     dim3 grid((unsigned)((int64_t)a.ntiles * a.KVH)), block(64 * FLASH_WAVES);
     const bool ub = paged && p.bs_shift >= 0 && a.block_size % NVR_FLASH_KT == 0;
-    p.ntiles = a.ntiles;
     if (a.D == 128 && !diff && !gate && !pen) {
-        if (a.ahead.units && grid.x <= 256 - AHEAD_WGS) { p.ahead = a.ahead; grid.x += AHEAD_WGS; }
+        const bool ahead = a.ahead.units && grid.x <= 256 - AHEAD_WGS;
+        FlashParamsAhead pa{};
+        static_cast<FlashParams &>(pa) = p; pa.ntiles = a.ntiles; pa.ahead = a.ahead;
+        if (ahead) grid.x += AHEAD_WGS;
 #define NVR_FLASH_PLAIN(GG)                                                                           \
     if (G == GG) {                                                                                    \
-        if (ub) flash_plain_kernel<GG, true, true><<<grid, block, 0, s>>>(p);                         \
+        if (ahead && ub) flash_plain_kernel<GG, true, true, true><<<grid, block, 0, s>>>(pa);         \
+        else if (ahead && paged) flash_plain_kernel<GG, true, false, true><<<grid, block, 0, s>>>(pa); \
+        else if (ahead) flash_plain_kernel<GG, false, false, true><<<grid, block, 0, s>>>(pa);        \
+        else if (ub) flash_plain_kernel<GG, true, true><<<grid, block, 0, s>>>(p);                    \
         else if (paged) flash_plain_kernel<GG, true, false><<<grid, block, 0, s>>>(p);                \
         else flash_plain_kernel<GG, false, false><<<grid, block, 0, s>>>(p);                          \
     }
-        NVR_FLASH_PLAIN(1) NVR_FLASH_PLAIN(2) NVR_FLASH_PLAIN(4)
+    NVR_FLASH_PLAIN(1) NVR_FLASH_PLAIN(2) NVR_FLASH_PLAIN(4)
 #undef NVR_FLASH_PLAIN
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return nvr::fail(NVR_ERR_HIP, "flash_prefill launch failed: %s", hipGetErrorString(e));
