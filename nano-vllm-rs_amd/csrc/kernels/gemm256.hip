@@ -1,7 +1,7 @@
-// gemm256.hip — 256x256x64 eight-wave MFMA GEMM for the prefill regime (T >= 256 tokens): y[T,N] = x[T,K]·W[N,K]^T,
+// gemm256.hip — 256x256x64 four-wave MFMA GEMM for the prefill regime (T >= 256 tokens): y[T,N] = x[T,K]·W[N,K]^T,
 // with the three epilogues of the decode kernels (plain fp16, gate_up -> SiluAndMul, qkv -> RoPE + KV store).
 // reference call sites as in linear.hip (linear.rs:354-356,228-239,437-439; activation.rs:46-63;
-// rotary_embedding.rs:23-48; attention.rs:150-174).  Bound: MFMA (880.8 MFLOP per prefill token).
+// rotary_embedding.rs:23-48; attention.rs:150-174).  Bound: MFMA (880.8 MFLOP per prefill token of Qwen3-0.6B).
 //
 // Structure:
 //   * workgroup = 4 waves (2 along n x 2 along m), one per SIMD with all of its 512 registers, = 256 W rows (A operand) x 256 tokens (B operand), BK = 64.

@@ -504,9 +504,10 @@ static void launch(const half_t *x, int64_t ldx, const half_t *W, int T, int K, 
     linear_skinny_kernel<NT, MT, WAVES, EPI><<<grid, dim3(WAVES * 64), 0, s>>>(x, ldx, W, T, K, N, y, e);
 }
 
-// 256x256 kernel or 128x128 kernel?  Fitted to both over 22 token counts (100..8192) x the projections of Qwen3-0.6B and Qwen3-8B, weights from HBM.  A round of <= 256 tiles of the
-// 256x256 kernel takes 18.5 K/1024 + 8 us however few there are (K = 1024 25 us, 2048 39, 4096 81, 12288 235).  The 128x128 kernel takes 9.4 K/1024 + 3.5 us while its tiles fit one per CU
-// (13.3 / 22 / 42 / 118), beyond that 8 K/1024 + 1.2 per 256 tiles (768 tiles 31, 1152 45, 2048 73 at K = 1024).  us of both, 256 / 128: qkv of 0.6B 27.1 /
+// 256x256 kernel or 128x128 kernel?  Fitted to both over 22 token counts (100..8192) x the projections of Qwen3-0.6B and Qwen3-8B, weights from HBM.  The 128x128 kernel takes 9.4 K/1024 + 3.5 us
+// while its tiles fit one per CU (K = 1024 13.3 us, 2048 22, 4096 42, 12288 118), beyond that 8 K/1024 + 1.2 per 256 tiles (768 tiles 31, 1152 45, 2048 73 at K = 1024).  The line for the 256x256
+// kernel, 18.5 K/1024 + 8 us for a round of <= 256 tiles however few there are, is that of a form with eight waves; with four a round of n tiles takes (17.5 + 6 max(0, n - 128) / 128) K/1024 + 1.5 and a
+// launch 5.5.  Rows dealt by that fit would take less than 3 % less at a few sizes (and none at most), so a step's rows stay where they were.  us of the two with the former, 256 / 128: qkv of 0.6B 27.1 /
 // 20.4 at 2048 tokens, 27.4 / 29.4 at 2560, 49.8 / 45.6 at 4672; o_proj 44.8 / 34.4 at 8192; 8B qkv 84.6 / 64.7 at 1280, 82.9 / 100.1 at 1536, 166 / 153 at 3062.  N = W rows
 static double cost_256(int64_t T, int64_t K, int64_t N) {
     const int64_t tiles = ((N + 255) / 256) * ((T + 255) / 256);
