@@ -17,19 +17,18 @@ class HostCopy {
 public:
     static constexpr size_t PIECE = 1 << 20, LEAST = 8 << 20;              // (LEAST: below, the runtime's own copy is as fast)
     static constexpr int LANES = 4;
-    ~HostCopy() {
-        for (Lane &l : lanes)
-            for (int i = 0; i < 2; ++i) if (l.landed[i]) (void)hipEventDestroy(l.landed[i]);
-        if (pinned) (void)hipHostFree(pinned);
-    }
-    hipError_t prepare() {                                                 // once, on the device's thread; not within a capture
-        if (pinned) return hipSuccess;
-        if (hipError_t e = hipHostMalloc((void **)&pinned, PIECE * 2 * LANES, hipHostMallocDefault)) return e;
+    ~HostCopy() { release(); }
+    // Once, on the device's thread; not within a capture.  Where the pieces or an event are not to be had nothing is kept, and the runtime copies (takes)
+    void prepare() {
+        if (pinned) return;
+        hipError_t e = hipHostMalloc((void **)&pinned, PIECE * 2 * LANES, hipHostMallocDefault);
+        if (e != hipSuccess) pinned = nullptr;
         for (int t = 0; t < LANES; ++t) {
-            lanes[t].at = pinned + (size_t)t * 2 * PIECE;
-            for (int i = 0; i < 2; ++i) if (hipError_t e = hipEventCreateWithFlags(&lanes[t].landed[i], hipEventDisableTiming)) return e;
+            lanes[t].at = pinned ? pinned + (size_t)t * 2 * PIECE : nullptr;
+            for (int i = 0; i < 2 && e == hipSuccess; ++i)
+                if ((e = hipEventCreateWithFlags(&lanes[t].landed[i], hipEventDisableTiming)) != hipSuccess) lanes[t].landed[i] = nullptr;
         }
-        return hipSuccess;
+        if (e != hipSuccess) { release(); (void)hipGetLastError(); }
     }
     // whether `to` is memory that this copies to: neither the runtime's own (pinned, managed or device memory, which it copies to at the link's rate) nor too little
     bool takes(const void *to, size_t bytes) const {
@@ -60,6 +59,12 @@ private:
     struct Lane { char *at = nullptr; hipEvent_t landed[2] = {}; } lanes[LANES];
     char *pinned = nullptr;
     std::mutex busy;
+    void release() {
+        for (Lane &l : lanes)
+            for (hipEvent_t &e : l.landed) if (e) { (void)hipEventDestroy(e); e = nullptr; }
+        if (pinned) (void)hipHostFree(pinned);
+        pinned = nullptr;
+    }
     hipError_t lane(int t, int device, hipStream_t stream, char *to, const char *from, size_t bytes) {
         const Lane &l = lanes[t];
         if (hipError_t e = hipSetDevice(device)) return e;

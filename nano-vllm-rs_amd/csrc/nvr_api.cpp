@@ -175,17 +175,17 @@ nvr_block_manager_t *nvr_sched_block_manager(nvr_scheduler_t *sc) { return sc->i
 size_t nvr_sched_take_finished(nvr_scheduler_t *sc, nvr_seq_t **out, size_t cap) { return sc->impl.take_finished(out, cap); }
 
 // ------------------------------------------------------------------ ModelRunner
-// runners whose logits can be large have what copies them ready
-static int host_copy_for(nvr_model_runner &r) {
-    if ((size_t)r.max_seqs * r.Vl * sizeof(float) >= nvr::HostCopy::LEAST) NVR_HIP_CHECK(r.host_copy.prepare());
-    return NVR_OK;
+// runners whose logits can be large have what copies them ready (or, where it is not to be had, the runtime's copy)
+static void prepare_host_copy(nvr_model_runner &r) {
+    if ((size_t)r.max_seqs * r.Vl * sizeof(float) >= nvr::HostCopy::LEAST) r.host_copy.prepare();
 }
 nvr_model_runner_t *nvr_runner_create(const nvr_config *cfg, const nvr_model_config *mc) {
     NVR_GUARD_BEGIN
     if (nvr_config_validate(cfg) || nvr_config_runnable(cfg)) return nullptr;
     nvr_model_runner *r = new nvr_model_runner();
     r->cfg = *cfg; r->mc = *mc;
-    if (r->init() != NVR_OK || host_copy_for(*r) != NVR_OK) { delete r; return nullptr; }
+    if (r->init() != NVR_OK) { delete r; return nullptr; }
+    prepare_host_copy(*r);
     return r;
     NVR_GUARD_END(nullptr)
 }
@@ -199,7 +199,8 @@ nvr_model_runner_t *nvr_runner_create_spec(const nvr_config *cfg, const nvr_mode
     r->cfg = *cfg;
     r->layered.reset(new nvr::LayeredModel());
     r->layered->spec = spec->layered;
-    if (r->init() != NVR_OK || host_copy_for(*r) != NVR_OK) { delete r; return nullptr; }
+    if (r->init() != NVR_OK) { delete r; return nullptr; }
+    prepare_host_copy(*r);
     return r;
     NVR_GUARD_END(nullptr)
 }

@@ -1,4 +1,7 @@
 """GPU test (-m gpu): logits into a program's own memory, by the runtime's copy and by several threads (csrc/host_copy.h)."""
+import ctypes as C
+import threading
+
 import numpy as np
 import pytest
 
@@ -27,3 +30,23 @@ def test_logits_arrive_whole_in_any_memory_and_number_of_pieces():
     device.zero()
     nvr.check(nvr.lib().nvr_runner_copy_logits(runner.h, device.ptr, batch))
     assert np.array_equal(device.to_numpy(want.shape, np.float32), want)
+    hip = nvr.lib()                                           # (finds the runtime that it has loaded)
+    pinned = C.c_void_p()
+    assert hip.hipHostMalloc(C.byref(pinned), C.c_size_t(want.nbytes), 0) == 0
+    try:
+        held = np.frombuffer((C.c_char * want.nbytes).from_address(pinned.value), np.float32).reshape(want.shape)
+        held[:] = 0
+        nvr.check(nvr.lib().nvr_runner_copy_logits(runner.h, pinned, batch))
+        assert np.array_equal(held, want)
+    finally:
+        assert hip.hipHostFree(pinned) == 0
+    got = [[], []]                                            # two callers at once: they take turns
+    def caller(mine):
+        for _ in range(4):
+            mine.append(runner.logits(batch))
+    threads = [threading.Thread(target=caller, args=(mine,)) for mine in got]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert [len(mine) for mine in got] == [4, 4] and all(np.array_equal(one, want) for mine in got for one in mine)
