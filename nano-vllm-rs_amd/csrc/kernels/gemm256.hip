@@ -56,14 +56,13 @@ constexpr int G_BUF = 4 * G_HALF;                                         // A0 
 constexpr int G_THREADS = 256;
 
 // 1 KiB of an operand into LDS: 16 bytes a lane from base + off, lane-linear at the byte that M0 holds (set an instruction before, by the hardware's rule).  Inline asm: hipcc drains the
-// builtin in front of LDS reads that it cannot tell apart from it; the requests are counted by hand.  Nothing else in this kernel uses M0.
-__device__ __forceinline__ void g_dma(unsigned off, const char *base) { asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base) : "memory"); }
+// builtin in front of LDS reads that it cannot tell apart from it; the requests are counted by hand.  M0 travels from g_aim to g_dma as a value of the compiler's own, which keeps the register free
+// between the two.
+__device__ __forceinline__ unsigned g_aim(unsigned lds, int piece) { unsigned at; asm volatile("s_add_u32 %0, %1, %2" : "={m0}"(at) : "s"(lds), "i"(piece) : "scc"); return at; }
+__device__ __forceinline__ void g_dma(unsigned at, unsigned off, const char *base) { asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(at) : "memory"); }
 
 // 4 bytes a lane from a pointer each
-__device__ __forceinline__ void g_dma4(unsigned lds, const void *src) {
-    unsigned keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, off\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "s"(lds), "v"(src) : "memory");
-}
+__device__ __forceinline__ void g_dma4(unsigned lds, const void *src) { asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "{m0}"(lds) : "memory"); }
 
 template <int EPI, int RD = 0, bool GRP = false>
 __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__restrict__ x, int64_t ldx, const half_t *__restrict__ W,
@@ -123,18 +122,18 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
     };
     const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)smem, lds_w = lds0 + (unsigned)wave * 1024u;
     // piece i = 0..3 of half-tile ht (0 = A0, 1 = A1, 2 = B0, 3 = B1)
-    auto aim = [&](int ht, int i, unsigned lds) { asm volatile("s_add_u32 m0, %0, %1" ::"s"(lds), "i"(ht * G_HALF + i * 4096) : "scc"); };
-    auto request = [&](int ht, int i) {
-        if (ht < 2) g_dma(va[EPI == GEPI_LMHEAD ? ht * 4 + i : i], ht ? pa1 : pa0);
-        else g_dma(vb[(ht - 2) * 4 + i], pb);
+    auto aim = [&](int ht, int i, unsigned lds) { return g_aim(lds, ht * G_HALF + i * 4096); };
+    auto request = [&](int ht, int i, unsigned at) {
+        if (ht < 2) g_dma(at, va[EPI == GEPI_LMHEAD ? ht * 4 + i : i], ht ? pa1 : pa0);
+        else g_dma(at, vb[(ht - 2) * 4 + i], pb);
     };
     auto request_all = [&](int g) {                                       // a whole K-tile, in the order of the phases: A0, B0, B1, A1
 #pragma unroll
         for (int n = 0; n < 16; ++n) {
             const int ht = n < 4 ? 0 : n < 8 ? 2 : n < 12 ? 3 : 1;
-            aim(ht, n & 3, lds_w + (unsigned)((g & 1) * G_BUF));
+            const unsigned at = aim(ht, n & 3, lds_w + (unsigned)((g & 1) * G_BUF));
             asm volatile("s_nop 0");
-            request(ht, n & 3);
+            request(ht, n & 3, at);
         }
     };
     // RoPE: positions (low dwords of the int64 entries) and cache slots of a tile's 256 token rows travel to LDS behind the K-tile ring by LDS-DMA, 4 bytes per lane (64 rows a wave), into one
@@ -159,13 +158,14 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
     // the phase brings into registers (F of READ_G, one behind every fourth product, or behind the products of the B fragment that they replace) and the four pieces of the half-tile that it
     // requests (two instructions each) go between them.  Own requests that the next phase reads have landed (all but the youngest five half-tiles), own reads of the phase before are back, barrier.
 #define G256_PHASE(HA_, HB_, F_, FH_, LANE_, READ_G_, RHT_, VM_, REQ_)                                                                          \
+    unsigned at_##RHT_ = 0;                                                                                                                \
     _Pragma("unroll") for (int n = 0; n < 32; ++n) {                                                                                       \
         constexpr bool behind = (RHT_) == 1;                              /* phase 3 */                                                    \
         if (!behind && n % 3 == 0 && n < 24) read(F_[FH_], n / 3, FH_, LANE_, READ_G_);                                                    \
         if (behind && n >= 8 && n % 8 == 0) { read(F_[FH_], n / 4 - 2, FH_, LANE_, READ_G_); }                                             \
         if (behind && n >= 8 && n % 8 == 1) { read(F_[FH_], n / 4 - 1, FH_, LANE_, READ_G_); }                                             \
-        if ((REQ_) && n % 8 == 4) aim(RHT_, n / 8, req_lds);                                                                               \
-        if ((REQ_) && n % 8 == 5) request(RHT_, n / 8);                                                                                              \
+        if ((REQ_) && n % 8 == 4) at_##RHT_ = aim(RHT_, n / 8, req_lds);                                                                              \
+        if ((REQ_) && n % 8 == 5) request(RHT_, n / 8, at_##RHT_);                                                                                            \
         __builtin_amdgcn_sched_barrier(0);                                                                                                 \
         acc[HA_][n & 3][HB_][n >> 3] = mfma16(fa[HA_][n & 3][(n >> 2) & 1], fb[HB_][n >> 3][(n >> 2) & 1], acc[HA_][n & 3][HB_][n >> 3]);  \
         __builtin_amdgcn_sched_barrier(0);                                                                                                 \

@@ -35,3 +35,35 @@ def test_inline_assembly_holds_no_vector_arithmetic(path):
             if i.split()[0] in ("s_mov_b32", "s_add_u32") and i.split()[1] == "m0,":       # a request into LDS reads m0 one wait state behind its write at the earliest
                 following = instructions[at + 1:at + 2]
                 assert not following or not following[0].startswith("global_load_lds"), "%s:%d: %s" % (path, line, i)
+
+
+def _whole(text):
+    """Every asm statement with its operands."""
+    for m in re.finditer(r'\basm\s*(?:volatile\s*)?\(', text):
+        depth, at, quoted = 1, m.end(), False
+        while depth:
+            c = text[at]
+            if quoted and c == "\\":
+                at += 1
+            elif c == '"':
+                quoted = not quoted
+            elif not quoted:
+                depth += {"(": 1, ")": -1}.get(c, 0)
+            at += 1
+        yield text.count("\n", 0, m.start()) + 1, text[m.start():at]
+
+
+@pytest.mark.parametrize("path", KERNELS, ids=[os.path.basename(p) for p in KERNELS])
+def test_inline_assembly_tells_the_compiler_of_m0(path):
+    """A request into LDS takes its place from M0: the statement sets M0 itself and puts back what it held, or M0 goes in and out as an operand, so that the compiler keeps nothing else there."""
+    with open(path) as f:
+        text = f.read()
+    for line, statement in _whole(text):
+        instructions = next(i for _, i in _statements(statement))
+        writes = [at for at, i in enumerate(instructions) if re.match(r"s_\w+ m0,", i)]
+        if writes and not re.search(r'"(=\{m0\}|m0)"', statement):
+            kept = [i.split()[1].rstrip(",") for i in instructions[:writes[0]] if re.match(r"s_mov_b32 %\d+, m0$", i)]
+            assert kept and instructions[writes[-1]] == "s_mov_b32 m0, " + kept[0], "%s:%d: M0 written" % (path, line)
+        for at, i in enumerate(instructions):
+            if i.startswith("global_load_lds"):
+                assert '"{m0}"' in statement or (writes and writes[0] < at), "%s:%d: M0 read" % (path, line)
