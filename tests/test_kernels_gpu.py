@@ -737,7 +737,7 @@ def test_decode_gemms_over_large_weights(T):
 
 
 def test_prefill_gemm_large_repeatable():
-    """The 256x256 eight-wave kernel keeps LDS-DMA loads in flight across barriers: screen it for races — many runs
+    """The 256x256 kernel keeps LDS-DMA loads in flight across barriers: screen it for races — many runs
     of a many-workgroup shape must be bit-identical to each other and match the oracle on sampled rows."""
     rng = np.random.default_rng(41)
     T, K, N = 8192, 1024, 2048                            # 8 x 32 = 256 tiles: routed to the 256x256 kernel (> 128 tiles)
@@ -752,7 +752,7 @@ def test_prefill_gemm_large_repeatable():
         else: assert np.array_equal(got, first), rep
     rows = rng.choice(T, 256, replace=False)
     assert_close_f16(first.view(F16)[rows], oracle.round_f16(oracle.linear(x[rows], W)), ulps=1, atol=2e-4, what="gemm256")
-    # same screen for the SiLU epilogue on a persistent grid with more tiles than workgroups (T=8192, I=1024: 8 x 32 tiles x ...)
+    # same screen for the SiLU epilogue (T=8192, I=1024: 8 x 32 tiles, one for every workgroup; more tiles than workgroups: tests/test_gemm256.py)
     T2, I = 8192, 1024
     x2, x2b = h16(rng.standard_normal((T2, K)))
     W2, W2b = h16(rng.standard_normal((2 * I, K)) * 0.05)
