@@ -569,9 +569,9 @@ def test_layer_list_clamped_unit_on_tiles(width, ff, batch, tokens):
     _compare_layer_rows(cfg, w, "bfloat16", base, [got["s%d" % i] for i in range(batch)])
 
 
-@pytest.mark.parametrize("width,ff,batch,tokens", [(64, 2112, 9, 34), (256, 2176, 3, 300), (1024, 3072, 40, 100)])
+@pytest.mark.parametrize("width,ff,batch,tokens", [(64, 2112, 9, 34), (256, 2176, 3, 300), (1024, 3072, 40, 100), (256, 2176, 22, 303)])      # (the last two: 384 and 459 tiles of 256 rows)
 def test_layer_list_clamped_unit_does_not_depend_on_the_step(width, ff, batch, tokens):
-    """A row's clamped unit in a prompt step (on 32- to 256-row tiles) and in portions of up to 32 rows: bit for bit.  Every product of the model has one term (the mixer's output none), so that the
+    """A row's clamped unit in a prompt step (on 32- to 256-row tiles, one and several of them a workgroup) and in portions of up to 32 rows: bit for bit.  Every product of the model has one term (the mixer's output none), so that the
     order of its sums does not matter; half of the stream's columns hold the token's embedding, the others the unit and nothing else, scaled until its smallest values (gates down to -12) count."""
     import rugudra_util as u
     half, limit = width // 2, 7.0
@@ -1069,17 +1069,21 @@ def test_float32_decode_attention_brings_weights_into_the_caches(hidden, inter, 
             assert ta == tb and np.array_equal(la, lb)
 
 
+# Prompts whose attention brings the gated unit's weights, 256 columns: an eighth of them to an XCD, or 48 rows of them in turn for tiles of 96 rows (what tests/test_weights_ahead.py looks at)
+AHEAD_PROMPTS = [(3072, [65]), (3072, [330]), (2304, [512]), (2112, [130, 7]),     # (2112: columns in no eighths, which bring nothing)
+                 (512, [200]), (3072, [1216]), (3072, [1217]), (3072, [1281])]     # 152 workgroups of attention, 160, and 168, which bring nothing
+AHEAD_96_ROWS = {(sum(lengths), inter): sum(lengths) in (330, 512) for inter, lengths in AHEAD_PROMPTS}
+
+
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
-@pytest.mark.parametrize("inter,lengths", [(3072, [65]), (3072, [330]),            # strips of an eighth; tiles of 96 rows
-                                           (2304, [400]), (2112, [130, 7]),        # 48 of them in a row; columns in no eighths, which bring nothing
-                                           (512, [200]), (512, [1216]), (512, [1217])])   # 152 workgroups of attention, and 160
+@pytest.mark.parametrize("inter,lengths", AHEAD_PROMPTS)
 def test_prompt_attention_brings_weights_into_the_caches(inter, lengths, dtype):
     """Prompt steps whose attention launch holds workgroups that request the gated unit's weights, at the ends of the rule: the prompts' logits and those of the token behind them against the oracle, at the
     engine's tolerance for the type."""
     from oracle import model_oracle as mo
     from test_engine_gpu import _run_pair
     mcfg = mo.small(hidden_size=256, num_hidden_layers=2, intermediate_size=inter, head_dim=128, num_attention_heads=16, num_key_value_heads=8, max_position_embeddings=2048, seed=inter, init_std=0.02)
-    ecfg = dict(max_num_seqs=2, max_num_batched_tokens=1280, max_model_len=1280, kvcache_block_size=16, num_kvcache_blocks=160)
+    ecfg = dict(max_num_seqs=2, max_num_batched_tokens=1344, max_model_len=1344, kvcache_block_size=16, num_kvcache_blocks=160)
     prompts = [oracle.fill_tokens(n, 3, i, mcfg.vocab_size).tolist() for i, n in enumerate(lengths)]
     _run_pair(mcfg, ecfg, prompts, [dict(temperature=0.0, max_tokens=2, ignore_eos=True) for _ in lengths], dtype=dtype)
 
