@@ -21,6 +21,7 @@
 // (T K N) 294 / 281, 32768 x 3072 x 1024 + residual 183 / 162, 32768 x 2048 x 1024 113 / 101, 32768 x 1024 x 4096 231 / 221, gate and up of 3072 columns 362 / 347, of 12288 at 3062 x 4096 478 / 451,
 // qkv with RoPE and store 265 / 245, with head norms 298 / 274, of 3815 rows 36.8 / 35.7.  (One barrier a K-tile with all requests behind it: the same rate alone, but 15 % less where the operands come from memory.)
 #include <cstdlib>
+#include <type_traits>
 #include "kernels.h"
 #include "device_utils.h"
 #include "../common.h"
@@ -264,6 +265,8 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
         if constexpr (EPI == GEPI_LMHEAD) {
             // Per token row: (max, lowest index) over this lane's 32 entries in ascending column order (strict >: the first maximum stays),
             // then over the 4 lanes of the token (larger value, else lower index), then over the two wave columns through LDS.
+            // A wave has its SIMD to itself, so nothing runs beside this: three instructions an entry, the bound in the vocabulary's last tile alone and the lane's first column behind the loop (with
+            // both in it, us without logits at N = 151936, K = 1024, with / so: 192 rows 112 / 107, 256 97 / 91, 512 150 / 144, 2048 530 / 505; K = 4096, 256 rows 316 / 309)
             float *sv = reinterpret_cast<float *>(smem + 2 * G_BUF); int *si = reinterpret_cast<int *>(smem + 2 * G_BUF + 1024);
             int lim = N - (bx * 256 + wn * 64 + q * 8);                   // vocabulary entries from the lane's first one on (opaque: no row of compares is kept over the K loop)
             int nv = N, tv = T;
@@ -277,21 +280,32 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm256_kernel(const half_t *__r
                     const int ml = b * 128 + mrow + j * 16, m = m0 + ml;
                     hold(b, j);
                     float bv = -INFINITY; int bi = 0x7fffffff;
-                    float *lrow = epi.logits + (int64_t)m * nv + n_base;
-                    const int out = epi.logits && m < tv ? lim : 0;
+                    if (epi.logits) {
+                        float *lrow = epi.logits + (int64_t)m * nv + n_base;
+                        const int out = m < tv ? lim : 0;
 #pragma unroll
-                    for (int a = 0; a < 2; ++a)
+                        for (int a = 0; a < 2; ++a)
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int c0 = a * 128 + (i >> 1) * 32 + (i & 1) * 4;
-                            const float4_t v = acc[a][i][b][j];
-                            if (c0 < out) *reinterpret_cast<float4_t *>(lrow + c0) = v;
+                            for (int i = 0; i < 4; ++i)
+                                if (const int c0 = a * 128 + (i >> 1) * 32 + (i & 1) * 4; c0 < out) *reinterpret_cast<float4_t *>(lrow + c0) = acc[a][i][b][j];
+                    }
+                    auto largest = [&](auto ragged) {
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                const bool more = (c0 + e < lim) & (v[e] > bv);
-                                bv = more ? v[e] : bv; bi = more ? n_base + c0 + e : bi;
+                        for (int a = 0; a < 2; ++a)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                const int c0 = a * 128 + (i >> 1) * 32 + (i & 1) * 4;
+                                const float4_t v = acc[a][i][b][j];
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) {
+                                    const bool more = (!decltype(ragged)::value || c0 + e < lim) && v[e] > bv;
+                                    bv = more ? v[e] : bv; bi = more ? c0 + e : bi;
+                                }
                             }
-                        }
+                    };
+                    if (bx * 256 + 256 <= N) largest(std::false_type{});
+                    else largest(std::true_type{});
+                    if (bi != 0x7fffffff) bi += n_base;
 #pragma unroll
                     for (int o = 16; o < 64; o <<= 1) {
                         const float v2 = __shfl_xor(bv, o, 64); const int i2 = __shfl_xor(bi, o, 64);
@@ -606,7 +620,7 @@ int gemm256_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *W, 
 
 // LM head over >= G256_LM_MIN_T (192) rows (large decode batches: 512 sequences — and many-sequence prefills): f32 logits on demand,
 // one (max, lowest index) partial per 256-column tile and row; N any multiple of 16
-constexpr int64_t G256_LM_MIN_T = 192;     // (measured: 128x128 tiles 78 us at 128 rows, 136 us at 255; these tiles 102 us up to 256 rows)
+constexpr int64_t G256_LM_MIN_T = 192;     // (us without logits, K = 1024, N = 151936: 128x128 tiles 78 at 128 rows, 129 at 160..192, 132 at 256; these tiles 90..107 at 192..256; K = 4096: 270, 470, 483; 298..309)
 bool gemm256_lm_head_ok(int64_t T, int64_t K, int64_t N, int64_t ldx) {
     return g256_enabled() && T >= G256_LM_MIN_T && T <= 65536 && K % G_BK == 0 && K >= 2 * G_BK && N % 16 == 0 && N >= 256 && ldx % 8 == 0 &&
            (N + 255) / 256 <= LM_HEAD_MAX_PARTS && N < (1ll << 31) && ((N + 255) / 256) * ((T + 255) / 256) < (1ll << 30);

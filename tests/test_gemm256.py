@@ -34,14 +34,21 @@ def test_head_at_the_edges_of_its_pipeline(T, K, N):
     nvr = nvr_import.load()
     rng = np.random.default_rng(T)
     x, W = (rng.standard_normal((T, K), dtype=np.float32)).astype(np.float16), (rng.standard_normal((N, K), dtype=np.float32) * np.float32(0.05)).astype(np.float16)
+    x[5], x[7] = 0, np.nan                                  # a row of equal logits, and one of no number
     d_x, d_W, d_y = nvr.DeviceBuffer.from_numpy(x), nvr.DeviceBuffer.from_numpy(W), nvr.DeviceBuffer(T * N * 4)
     parts = C.c_int32(0)
     d_pv, d_pi = nvr.DeviceBuffer(2048 * T * 4), nvr.DeviceBuffer(2048 * T * 4)
     nvr.check(nvr.lib().nvr_lm_head(d_x.ptr, K, d_W.ptr, T, K, N, d_y.ptr, d_pv.ptr, d_pi.ptr, C.byref(parts), None))
     assert parts.value == (N + 255) // 256
     got, want = d_y.to_numpy((T, N), np.float32), x.astype(np.float64) @ W.astype(np.float64).T
+    assert np.isnan(got[7]).all()
+    got[7], want[7] = 0, 0
     assert np.all(np.abs(got - want) <= K * 2.0 ** -24 * 0.25 * K ** 0.5 + 1e-6)
     value, index = d_pv.to_numpy((parts.value, T), np.float32), d_pi.to_numpy((parts.value, T), np.int32)
+    first = np.arange(parts.value, dtype=np.int32) * 256
+    assert np.array_equal(index[:, 5], first) and not value[:, 5].any()                  # (the first of equal ones)
+    assert np.all(value[:, 7] == -np.inf) and np.all(index[:, 7] == 0x7fffffff)          # (no entry is larger than the lowest value)
+    value[:, 7], index[:, 7] = 0, first
     best = value.argmax(0)
     assert np.array_equal(index[best, np.arange(T)], got.argmax(1)) and np.array_equal(value.max(0), got.max(1))
 
