@@ -46,7 +46,7 @@ public:
         int started = 1;
         try {
             threads.reserve(LANES - 1);
-            for (; started < LANES; ++started) threads.emplace_back([=, &rc, this, t = started] { rc[t] = lane(t, device, stream, (char *)to, (const char *)from, bytes); });
+            for (; started < LANES; ++started) threads.emplace_back([this, &rc, device, stream, to, from, bytes, t = started] { rc[t] = lane(t, device, stream, (char *)to, (const char *)from, bytes); });
         } catch (...) {}                                                   // (no thread to be had: the caller takes their pieces too)
         rc[0] = lane(0, device, stream, (char *)to, (const char *)from, bytes);
         for (int t = started; t < LANES; ++t) rc[t] = lane(t, device, stream, (char *)to, (const char *)from, bytes);

@@ -19,7 +19,10 @@
 // What bounds it: power.  With operands of zeros a K-tile takes 1.05 us at 2.4 GHz however many CUs run (2520 clocks: 128 products of 17 and the ~120 other instructions of a wave, which nothing overlaps), with
 // random ones 1.07 us on 32 CUs and 1.45 on 256: the clock falls to what the part's power allows.  us, eight waves of 128 x 64 with 8 barriers a K-tile and results through LDS / so: 4096 x 12288 x 4096
 // (T K N) 294 / 281, 32768 x 3072 x 1024 + residual 183 / 162, 32768 x 2048 x 1024 113 / 101, 32768 x 1024 x 4096 231 / 221, gate and up of 3072 columns 362 / 347, of 12288 at 3062 x 4096 478 / 451,
-// qkv with RoPE and store 265 / 245, with head norms 298 / 274, of 3815 rows 36.8 / 35.7.  (One barrier a K-tile with all requests behind it: the same rate alone, but 15 % less where the operands come from memory.)
+// qkv with RoPE and store 265 / 245, with head norms 298 / 274, of 3815 rows 36.8 / 35.7; rows grouped by expert, 32768 of 1024 to 768 and back 101 + 53 / 89 + 48, 2048 26 + 19.5 / 25 + 20.  A wave without
+// another beside it pays for its epilogue's arithmetic in full: single rounds of 144..256 tiles with K <= 1024 whose epilogue computes much take 1 to 4 % more (with head norms, 160 tiles 32.1 / 33.4;
+// heads of 64 31.3 / 32.0; the clamped unit at K = 512 21.7 / 22.6).  Registers: 476 to 512 of 512 a lane; the head norms' instance keeps one more in scratch memory (a store and a load a tile), the
+// head's 29 scalar ones in lanes of a vector register, the others nothing.  (One barrier a K-tile with all requests behind it: the same rate alone, but 15 % less where the operands come from memory.)
 #include <cstdlib>
 #include <type_traits>
 #include "kernels.h"

@@ -139,7 +139,7 @@ int gemm_tiled_qkv_rope_store(const half_bits *x, int64_t ldx, const half_bits *
                               half_bits *qkv, half_bits *k_cache, half_bits *v_cache, hipStream_t s, const half_bits *Wt = nullptr, bool kv_cache_only = false,
                               const QkNorm *norm = nullptr);   // norm: Wt in the plain order of rows (retile_weight mode 0)
 
-// 256x256x64 eight-wave MFMA GEMM (T >= 256, N % 256 == 0 / I % 128 == 0 / whole heads per 256 rows): same results
+// 256x256x64 four-wave MFMA GEMM (T >= 256, N % 256 == 0 / I % 128 == 0 / whole heads per 256 rows): same results
 // layout and epilogues; preferred over gemm_tiled when its shape test passes
 bool gemm256_ok(int64_t T, int64_t K, int64_t N, int64_t ldx);
 bool gemm256_silu_ok(int64_t T, int64_t K, int64_t I, int64_t ldx);

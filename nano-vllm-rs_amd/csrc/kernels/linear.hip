@@ -504,11 +504,12 @@ static void launch(const half_t *x, int64_t ldx, const half_t *W, int T, int K, 
     linear_skinny_kernel<NT, MT, WAVES, EPI><<<grid, dim3(WAVES * 64), 0, s>>>(x, ldx, W, T, K, N, y, e);
 }
 
-// 256x256 kernel or 128x128 kernel?  Fitted to both over 22 token counts (100..8192) x the projections of Qwen3-0.6B and Qwen3-8B, weights from HBM.  The 128x128 kernel takes 9.4 K/1024 + 3.5 us
-// while its tiles fit one per CU (K = 1024 13.3 us, 2048 22, 4096 42, 12288 118), beyond that 8 K/1024 + 1.2 per 256 tiles (768 tiles 31, 1152 45, 2048 73 at K = 1024).  The line for the 256x256
-// kernel, 18.5 K/1024 + 8 us for a round of <= 256 tiles however few there are, is that of a form with eight waves; with four a round of n tiles takes (17.5 + 6 max(0, n - 128) / 128) K/1024 + 1.5 and a
-// launch 5.5.  Rows dealt by that fit would take less than 3 % less at a few sizes (and none at most), so a step's rows stay where they were.  us of the two with the former, 256 / 128: qkv of 0.6B 27.1 /
-// 20.4 at 2048 tokens, 27.4 / 29.4 at 2560, 49.8 / 45.6 at 4672; o_proj 44.8 / 34.4 at 8192; 8B qkv 84.6 / 64.7 at 1280, 82.9 / 100.1 at 1536, 166 / 153 at 3062.  N = W rows
+// 256x256 kernel or 128x128 kernel?  The 128x128 kernel takes 9.4 K/1024 + 3.5 us while its tiles fit one per CU (K = 1024 13.3 us, 2048 22, 4096 42, 12288 118), beyond that 8 K/1024 + 1.2 per 256
+// tiles (768 tiles 31, 1152 45, 2048 73 at K = 1024).  The line for the 256x256 kernel is a round of its tiles for a round of its time, whatever their number.  The kernel itself takes less for a round
+// of few tiles, but so do the 128-row tiles that compete for it: over 424 sizes (512..8192 rows by 128, the projections of Qwen3-0.6B and Qwen3-8B, weights from HBM) the rows that these lines deal take within
+// 1 % of the best dealing at all but 3, those of a line that follows a round's tiles ((17.5 + 6 max(0, n - 128) / 128) K/1024 + 1.5, a launch 5.5) at all but 15, and 0.06 % and 0.12 % over the best in
+// all (gate and up of 0.6B, 6272..6528 rows: 76.3..76.8 us so, 79.8..80.5 by that line; 3328 rows 48.9 and 47.4).  us of the two kernels, 256 / 128: qkv of 0.6B 25.4 / 19.8 at 2048 tokens, 25.9 / 28.9 at
+// 2560, 49.4 / 45.6 at 4608; o_proj 44.4 / 36.8 at 8192; 8B qkv 76.1 / 65.0 at 1280, 78.9 / 104 at 1536, 166 / 163 at 3072.  N = W rows
 static double cost_256(int64_t T, int64_t K, int64_t N) {
     const int64_t tiles = ((N + 255) / 256) * ((T + 255) / 256);
     return (double)((tiles + 255) / 256) * (18.5 * (double)K / 1024.0 + 8.0);
@@ -525,8 +526,8 @@ static inline bool prefer_256(int64_t T, int64_t K, int64_t N) { return cost_256
 bool gemm256_preferred(int64_t T, int64_t K, int64_t N, int64_t ldx) { return gemm256_ok(T, K, N, ldx) && prefer_256(T, K, N); }
 // Rows [0, r) of a product on 256x256 tiles and the others on 128x128 ones (0: all on the latter, T: all on the former).  A last round of 256x256 tiles costs as much as a full one however few
 // they are, so the rows that do not fill one go to the small tiles where that is estimated 4 % cheaper: both kernels sum a row's products in the same order, and a row has the same bits on either.
-// us, the better kernel for all rows / split: 8B qkv 154.9 / 130.3 at 3062 rows, o_proj 154.1 / 134.4 at 4672, down_proj 453.7 / 377.2 at 4672, 484.6 / 393.1 at 5120; 0.6B gate_up 45.9 / 42.2 at
-// 3062, qkv 43.1 / 38.8 at 4300, 44.7 / 43.5 at 4672, o_proj 76.5 / 64.8 at 17000.
+// us, the better kernel for all rows / split: 8B qkv 163 / 137 at 3072 rows, o_proj 168 / 136 at 4608, down_proj 482 / 380 at 4608, 489 / 416 at 5120; 0.6B gate_up 46.8 / 42.0 at 3072, qkv 44.1 / 38.8
+// at 4352, 45.6 / 40.2 at 4608, o_proj 78.6 / 62.8 at 17000.
 static int64_t rows_on_256(int64_t T, int64_t K, int64_t N) {
     const double c256 = cost_256(T, K, N), c128 = cost_128(T, K, N);
     int64_t best = c256 < c128 ? T : 0;
@@ -547,8 +548,8 @@ static bool former_256(int64_t T, int64_t K, int64_t N) {
 }
 bool linear_add_residual_ok(int64_t T, int64_t K, int64_t N, int64_t ldx) { return gemm256_ok(T, K, N, ldx) && former_256(T, K, N); }
 // a product with an epilogue that the 256x256 kernel alone has (GELU, max(y, 0)^2): elsewhere it is a launch of its own that reads and writes the rows again, so the line lies where either estimate
-// prefers the kernel.  us a layer with GELU, tiles and a launch of its own / so: 2064 rows of 4096 columns, K = 1024 145 / 140, 2304 rows 146 / 141; 8192 columns, K = 2048 2064 rows 294 / 299 (the
-// unrounded product's GELU all the same), 2560 rows 322 / 310
+// prefers the kernel.  us of product and GELU, tiles and a launch of its own / so: 4096 columns, K = 1024 1800 rows 32.3 / 32.6, 2064 40.6 / 31.9, 2304 40.5 / 30.8; 8192 columns, K = 2048 2064 rows
+// 97.8 / 92.6, 2560 109 / 95.1
 bool gemm256_epilogue_preferred(int64_t T, int64_t K, int64_t N, int64_t ldx) { return gemm256_ok(T, K, N, ldx) && (prefer_256(T, K, N) || former_256(T, K, N)); }
 int64_t stream_row_limit() { return 64; }
 // split-k GEMMs of the N = hidden projections: LDS tiles beyond the streaming kernels' rows — and from 33 rows on over large weights, where the
@@ -739,8 +740,8 @@ int linear_gelu_mul(const half_bits *x, int64_t ldx, const half_bits *W, int64_t
 
 // gate_up GEMM + the clamped gated unit of a layer list: W [2I, K] (gate rows, then up rows), out [T, ldo].  Few rows, whose product the weight-row kernel takes: the unit
 // is a launch of its own otherwise, and a launch behind a launch is about 5 us whatever it holds (16 rows of 1024, I = 3072: 11.3 -> 6.3 us together).  Shapes of the LDS tiles, routed as linear()
-// routes the plain product: the unit by itself reads both halves of every row again and the product writes twice the columns (16384 rows of 1024, I = 3072: 201 + 59 us -> 192; with
-// the unit on v_rcp and the fast exponential 168, but then a row's unit would depend on the size of its step, and be off by a few last places of f32 more).
+// routes the plain product: the unit by itself reads both halves of every row again and the product writes twice the columns (1024 wide, I = 3072: 16384 rows 178 + 63 us -> 195, 4096 52 + 17 -> 67;
+// the unit on v_rcp and the fast exponential was 24 us faster at 16384, but then a row's unit would depend on the size of its step, and be off by a few last places of f32 more).
 static bool clamped_glu_on_tiles(int64_t T, int64_t K, int64_t I, int64_t ldx) {
     return K % 32 == 0 && I % 64 == 0 && gemm_tiled_ok(T, K, I, ldx) && ((gemm256_silu_ok(T, K, I, ldx) && rows_on_256(T, K, 2 * I) > 0) || !stream_preferred(T, 2 * I));
 }
