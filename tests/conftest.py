@@ -25,6 +25,12 @@ import gc
 import pytest
 
 
+def pytest_collection_finish(session):
+    """What the imports and the collected tests hold (hundreds of thousands of objects that live to the end) stays out of the collections between the tests below."""
+    gc.collect()
+    gc.freeze()
+
+
 @pytest.fixture(autouse=True)
 def _no_collector_inside_a_test():
     """Engines of earlier tests that are still waiting for the cycle collector are destroyed HERE, between tests, and the collector stays
