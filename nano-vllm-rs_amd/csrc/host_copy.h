@@ -12,7 +12,7 @@ namespace nvr {
 // The runtime copies to pageable memory through one staging buffer and one thread, which also takes the page faults of an array that was just allocated: 39 MB of logits of 64 sequences 3.9 ms, of
 // which the link needs 0.8.  Here LANES threads (the caller and three that live for the call) each bring every LANES-th piece into two pinned pieces in turn, on the stream that the array is made on,
 // and copy one to its place while the other lands: 1.5 ms.  (A stream for each thread is no faster, and its first use takes a millisecond.)  Nothing outlives a call but the pinned pieces (8 MiB a
-// runner); calls on one object take turns.
+// runner, a millisecond of the eleven that it takes to be made); calls on one object take turns.
 class HostCopy {
 public:
     static constexpr size_t PIECE = 1 << 20, LEAST = 8 << 20;              // (LEAST: below, the runtime's own copy is as fast)
